@@ -471,8 +471,9 @@ static TinyNNStatus conv2d_run(
         MG_REQUIRE(nr_elem(flt->layout) == conv_mfma_packed_bytes(g), TinyNN_ERROR_INVALID_LAYOUT,
                    "conv2d: packed filter has %zu bytes, expected %zu", nr_elem(flt->layout),
                    conv_mfma_packed_bytes(g));
-        MG_REQUIRE(aligned4(src->ptr) && aligned4(dst->ptr) && aligned16(flt->ptr) &&
-                           (!b || aligned4(b)),
+        // (FullyConnected over a K that is no multiple of 4: its kernels take any address)
+        MG_REQUIRE(aligned16(flt->ptr) &&
+                           ((g.ic & 3) || (aligned4(src->ptr) && aligned4(dst->ptr) && (!b || aligned4(b)))),
                    TinyNN_ERROR_INVALID_LAYOUT, "conv2d: misaligned operand");
         return conv_mfma_launch(g, src->ptr, flt->ptr, b, dst->ptr, workspace);
     }

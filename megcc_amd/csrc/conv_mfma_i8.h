@@ -145,6 +145,29 @@ __device__ __forceinline__ void dma_buffer_b128(v4u rsrc, unsigned voffset, unsi
                  : "memory");
 }
 
+// 16 bytes at any address (the unaligned access the hardware does anyway)
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+// FullyConnected rows that start at any byte: `v` was read `d` bytes before the place it was wanted from,
+// because that place is less than 16 bytes from the end of the tensor (or beyond it). Bytes d .. 15 of v
+// move down, zeros follow.
+__device__ __forceinline__ v4i fc_tail_piece(v4i v, unsigned d) {
+    const unsigned w = d >> 2, b = (d & 3) * 8;
+    const unsigned x[4] = {(unsigned)v[0], (unsigned)v[1], (unsigned)v[2], (unsigned)v[3]};
+    v4i r;
+#pragma unroll
+    for (unsigned i = 0; i < 4; ++i) {
+        unsigned lo = 0, hi = 0;
+#pragma unroll
+        for (unsigned k = 0; k < 4; ++k) {
+            lo = i + w == k ? x[k] : lo;
+            hi = i + 1 + w == k ? x[k] : hi;
+        }
+        r[i] = (int)(b ? (lo >> b) | (hi << (32 - b)) : lo);
+    }
+    return r;
+}
+
 struct PipeConfig {
     int bm, bn, ks, blocks_per_cu, threads, a_bytes;
     int nbuf;            // LDS stage buffers

@@ -324,6 +324,8 @@ static int conv_mfma_split(const ConvGeom& g) {
 }
 
 size_t conv_mfma_workspace_bytes(const ConvGeom& g) {
+    if (g.fmt == MEGCC_FMT_NCHW && (g.ic & 3))
+        return 0;  // (fc_any_k: no partial sums in memory)
     const int s = conv_mfma_split(g);
     const long P = (long)g.n * g.oh * g.ow;
     return s > 1 ? (size_t)s * P * ((g.oc + 3) & ~3) * sizeof(int32_t) : 0;
@@ -434,12 +436,23 @@ static TilePlan plan_tiles_uncached(const ConvGeom& g, int bn, long range_len, i
 
 static bool pick_dma(const ConvGeom& g, bool b128_ok, PipeConfig* pc, TilePlan* t, long* range_len, int* picked);
 
+bool fc_gevm_q8_supported(const ConvGeom& g);
+bool fc_tile_supported(const ConvGeom& g);
+TinyNNStatus fc_tile_launch(
+        const ConvGeom& g, const void* src, const void* packed, const void* bias, void* dst);
+// FullyConnected over any K: the kernels that take rows starting at any byte
+static bool fc_any_k(const ConvGeom& g) {
+    return fc_gevm_q8_supported(g) || fc_tile_supported(g);
+}
+
 bool conv_mfma_supported(const ConvGeom& g) {
     if (g.groups != 1)
         return false;
     bool fc = is_fc(g);
     if (!(g.fmt == MEGCC_FMT_NCHW44 || fc))
         return false;
+    if (fc && (g.ic & 3))  // rows that are no whole channel groups: kernels of their own
+        return fc_any_k(g);
     if (g.ic & 3)
         return false;
     if (g.fmt == MEGCC_FMT_NCHW44 && (g.oc & 3))
@@ -515,7 +528,6 @@ TinyNNStatus fc_stream_launch(
 bool fc_one_supported(const ConvGeom& g, const void* src);
 TinyNNStatus fc_one_launch(
         const ConvGeom& g, const void* src, const void* packed, const void* bias, void* dst);
-bool fc_gevm_q8_supported(const ConvGeom& g);
 TinyNNStatus fc_gevm_q8_launch(
         const ConvGeom& g, const void* src, const void* packed, const void* bias, void* dst);
 bool conv_pw_stream_supported(const ConvGeom& g);
@@ -592,6 +604,11 @@ TinyNNStatus conv_mfma_launch(
     if (is_fc(g) && fc_one_supported(g, src) && !few_long && !options().no_fcone && !options().no_fcs) {
         return fc_one_launch(g, src, packed, bias, dst);
     }
+    // rows that are no whole 128-byte blocks at 16-byte addresses
+    if (is_fc(g) && fc_tile_supported(g) && ((g.ic & 3) || (((g.ic & 127) || ((uintptr_t)src & 15)) && !options().no_fcs)))
+        return fc_tile_launch(g, src, packed, bias, dst);  // (notes its own variant)
+    MG_REQUIRE(!is_fc(g) || (g.ic & 3) == 0, TinyNN_ERROR_NO_IMPLEMENT,
+               "conv_mfma: no kernel left for a FullyConnected over K=%d (switched off)", g.ic);
     MfmaParams q = {};
     PipeConfig pc;
     const bool b128_ok = ((uintptr_t)src & 15) == 0 && !options().no_fcb;
@@ -599,6 +616,12 @@ TinyNNStatus conv_mfma_launch(
     TilePlan t;
     int picked = -1;  // variant of the LDS-direct kernel
     const bool pipe = pick_dma(g, b128_ok, &pc, &t, &range_len, &picked);
+    // FullyConnected: the LDS-direct kernel's 256 x 256 tiles win from half a chip of them on (2048 x 4096
+    // x 4096, 128 tiles: 43.7 us against 46.6; 4096 x 2048 x 1024, 64 tiles: 21.5 against 21.2; 2048 x 1024
+    // x 1000, 32 tiles: 14.8 against 8.6; 200 x 1024 x 1000: 13.0 on the one-stage kernel against 6.6)
+    if (is_fc(g) && g.n > 64 && fc_tile_supported(g) && !options().no_fcs &&
+        !(pipe && (long)((g.n + 255) / 256) * ((g.oc + 255) / 256) >= num_cus() / 2))
+        return fc_tile_launch(g, src, packed, bias, dst);
     if (!pipe) {
         range_len = 0;
         t = plan_tiles(g, BN);

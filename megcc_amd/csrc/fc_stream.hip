@@ -163,6 +163,7 @@ struct FcOneParams {
     const int32_t* bias;
     int8_t* dst;  // [M][OC]
     int M, K, OC, OCP, act;
+    unsigned last16;  // offset of the last 16 bytes of src
     float s_src, s_flt, s_dst;
 };
 
@@ -285,15 +286,17 @@ __global__ void __launch_bounds__(64 * FO_WAVES) fc_one_kernel(FcOneParams q) {
 // behind an earlier one, and it then waits for ALL of them before the first use: each prefetch
 // became a round trip of its own. Here a wave with fewer blocks than NB, or none, fetches a block it
 // has a right to read again and multiplies it with zeros; rows beyond M read row M - 1 and are
-// zeroed on their way into LDS.
-template <int NB>
+// zeroed on their way into LDS. ANYK: K is no multiple of 128 or the rows start at any byte - the last
+// block's surplus bytes meet the packed filter's zeros, and a piece that would run past the end of the
+// tensor is read 16 bytes before it and shifted into place (fc_tile.hip says more).
+template <int NB, bool ANYK>
 __global__ void __launch_bounds__(64 * FO_WAVES) fc_one32_kernel(FcOneParams q) {
     __shared__ int32_t red[FO_WAVES][16][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, kg = lane >> 5;
     const int oct = blockIdx.x, oc = oct * 32 + col;
     const int row0 = blockIdx.y * 32;
-    const int blocks = q.K >> 7;
+    const int blocks = ANYK ? (q.K + 127) >> 7 : q.K >> 7;
     const int myb = wave < blocks ? (blocks - wave + FO_WAVES - 1) / FO_WAVES : 0;  // <= NB
     const int wv = myb ? wave : 0;
     const size_t astep = (size_t)q.OCP * KROW;
@@ -307,7 +310,8 @@ __global__ void __launch_bounds__(64 * FO_WAVES) fc_one32_kernel(FcOneParams q) 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int row = min(row0 + i * 8 + srow, q.M - 1);
-            areg[b][i] = *(const v4i*)(q.src + (size_t)row * q.K + (wv + FO_WAVES * bc) * 128 + apc * 16);
+            const unsigned off = (unsigned)row * (unsigned)q.K + (unsigned)((wv + FO_WAVES * bc) * 128 + apc * 16);
+            areg[b][i] = ANYK ? (v4i)*(const v4i_any*)(q.src + min(off, q.last16)) : *(const v4i*)(q.src + off);
         }
     }
 #pragma unroll
@@ -329,6 +333,12 @@ __global__ void __launch_bounds__(64 * FO_WAVES) fc_one32_kernel(FcOneParams q) 
         for (int i = 0; i < 4; ++i) {
             const bool ok = row0 + i * 8 + srow < q.M && b < myb;
             v4i v = areg[b][i];
+            if (ANYK) {
+                const unsigned off = (unsigned)min(row0 + i * 8 + srow, q.M - 1) * (unsigned)q.K +
+                                     (unsigned)((wv + FO_WAVES * (b < myb ? b : 0)) * 128 + apc * 16);
+                if (off > q.last16)
+                    v = fc_tail_piece(v, off - q.last16);
+            }
             v.x = ok ? v.x : 0, v.y = ok ? v.y : 0, v.z = ok ? v.z : 0, v.w = ok ? v.w : 0;
             *(v4i*)(stage + (i * 8 + srow) * 128 + ((apc ^ srow) << 4)) = v;  // (a wave's LDS operations execute in order)
         }
@@ -365,7 +375,7 @@ __global__ void __launch_bounds__(64 * FO_WAVES) fc_one32_kernel(FcOneParams q) 
     }
     int8_t* o = q.dst + (size_t)row * q.OC + ocb;
     if ((q.OC & 3) == 0) {
-        *(uint32_t*)o = pack4(r[0], r[1], r[2], r[3]);
+        *(u32_any*)o = pack4(r[0], r[1], r[2], r[3]);
     } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -374,10 +384,19 @@ __global__ void __launch_bounds__(64 * FO_WAVES) fc_one32_kernel(FcOneParams q) 
     }
 }
 
-// M <= 64 rows, K a multiple of 128, 16-byte aligned activations
+// rows of whole 128-byte blocks at 16-byte addresses
+static bool fc_one_whole(const ConvGeom& g, const void* src) {
+    return (g.ic & 127) == 0 && ((uintptr_t)src & 15) == 0;
+}
+// two workgroups of 32 rows per channel tile instead of one of 64 (fc_one_launch)
+static bool fc_one_rows32(const ConvGeom& g) {
+    return g.n <= 32 || (g.oc + 31) / 32 * 2 <= num_cus();
+}
+// M <= 64 rows; any K up to 4096 in tiles of 32 rows, a longer one or tiles of 64 rows if K is a multiple
+// of 128 and the activations are 16-byte aligned
 bool fc_one_supported(const ConvGeom& g, const void* src) {
-    return g.n >= 1 && g.n <= 64 && g.ic >= 128 && (g.ic & 127) == 0 && ((uintptr_t)src & 15) == 0 &&
-           g.oc >= 1;
+    return g.n >= 1 && g.n <= 64 && g.oc >= 1 && (long)g.n * g.ic >= 16 &&
+           (fc_one_whole(g, src) ? g.ic >= 128 : g.ic <= 4096 && fc_one_rows32(g));
 }
 
 TinyNNStatus fc_one_launch(
@@ -392,6 +411,7 @@ TinyNNStatus fc_one_launch(
     q.OC = g.oc;
     q.OCP = (g.oc + OC_PAD - 1) / OC_PAD * OC_PAD;
     q.act = g.act;
+    q.last16 = (unsigned)((long)g.n * g.ic - 16);
     q.s_src = g.s_src;
     q.s_flt = g.s_flt;
     q.s_dst = g.s_dst;
@@ -400,16 +420,16 @@ TinyNNStatus fc_one_launch(
     // CU - what a CU pulls through its L2 port (its share of the weights + the activations of its
     // rows) bounds the kernel: 64 x 4096 x 4096 8.1 -> 6.6 us. (With a multiple of 8 channel tiles the
     // two are on the same XCD: the weights still leave HBM once.)
-    const bool rows32 = g.n <= 32 || oc_tiles * 2 <= num_cus();
-    const int nb = rows32 && g.ic <= 4096 ? (g.ic / 128 + FO_WAVES - 1) / FO_WAVES : 0;  // blocks per wave
-    note_kernel("fc_one", rows32 ? 32 : 64, nb);
+    const bool rows32 = fc_one_rows32(g), any = !fc_one_whole(g, src);
+    const int nb = rows32 && g.ic <= 4096 ? ((g.ic + 127) / 128 + FO_WAVES - 1) / FO_WAVES : 0;  // blocks per wave
+    note_kernel("fc_one", rows32 ? 32 : 64, nb, any ? 1 : -1);
     const dim3 grid32(oc_tiles, (g.n + 31) / 32), block(64 * FO_WAVES);
     if (nb == 1)
-        hipLaunchKernelGGL(fc_one32_kernel<1>, grid32, block, 0, stream(), q);
+        hipLaunchKernelGGL((any ? fc_one32_kernel<1, true> : fc_one32_kernel<1, false>), grid32, block, 0, stream(), q);
     else if (nb == 2)
-        hipLaunchKernelGGL(fc_one32_kernel<2>, grid32, block, 0, stream(), q);
+        hipLaunchKernelGGL((any ? fc_one32_kernel<2, true> : fc_one32_kernel<2, false>), grid32, block, 0, stream(), q);
     else if (nb >= 3)
-        hipLaunchKernelGGL(fc_one32_kernel<4>, grid32, block, 0, stream(), q);
+        hipLaunchKernelGGL((any ? fc_one32_kernel<4, true> : fc_one32_kernel<4, false>), grid32, block, 0, stream(), q);
     else if (rows32)
         hipLaunchKernelGGL(fc_one_kernel<1>, dim3(oc_tiles, (g.n + 31) / 32), dim3(64 * FO_WAVES), 0, stream(), q);
     else

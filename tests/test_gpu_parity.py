@@ -356,6 +356,28 @@ def test_matches_oracle(case):
     compare(got, want, repr(case))
 
 
+FC_ANY_K = [
+    # FullyConnected whose rows are no whole 128-byte blocks: (rows, K, N) at the edges of the kernels' tiles,
+    # rows at any byte, the last 16 bytes of the tensor inside and at the start of a piece, K below a piece
+    ("fc_gevm_q8", 1, 3, 10), ("fc_gevm_q8", 4, 491, 65),
+    ("fc_one", 5, 17, 33), ("fc_one", 33, 1001, 64), ("fc_one", 64, 4095, 129), ("fc_one", 24, 2052, 31),
+    ("fc_tile:64,1", 65, 5, 9), ("fc_tile:64,2", 65, 129, 67), ("fc_tile:64,4", 70, 2958, 70),
+    ("fc_tile:64,4", 225, 515, 361), ("fc_tile:64,2", 1100, 1123, 1001), ("fc_tile:64,1", 1500, 260, 1540),
+    ("fc_tile:128,1", 2049, 67, 2050), ("fc_tile:128,1", 2048, 259, 2052),
+]
+
+
+@pytest.mark.parametrize("kernel,m,k,n", FC_ANY_K)
+@pytest.mark.parametrize("act", [A.IDENTITY, A.RELU, A.H_SWISH])
+def test_fully_connected_over_any_k(kernel, m, k, n, act):
+    port.set_threads(8)
+    case = ConvCase(A.FMT_NCHW, A.DENSE, m, k, 1, 1, n, 1, 1, 0, act, scales=(0.01, 0.01, 0.01 * unsat(k) / 0.02))
+    arrays = case.gen(seed=17)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().replace("_xo", "").startswith(kernel), runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
 F32_NCHW44 = [
     # f32 channel-wise layers in NCHW44 (the reference's GI_chanwise kernels: 3x3 / 5x5, stride 1 / 2):
     # tiles of 4 x 64 pixels - extents below, at and above a tile, padding 0 .. k/2 + 1, every activation
