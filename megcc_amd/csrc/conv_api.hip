@@ -12,6 +12,7 @@
 
 #include "common.h"
 #include "conv_geom.h"
+#include "gemm_f32_ks.h"
 
 namespace mg {
 bool conv_mfma_supported(const ConvGeom& g);
@@ -565,6 +566,8 @@ static TinyNNStatus conv2d_run(
         nchw44_views(g.n, g.oc, g.oh, g.ow, &view, &dense);
         return strided_copy(dst_nchw, view, dst->ptr, dense, 4, "conv2d (f32 NCHW -> NCHW44)");
     }
+    if (f32 && !options().no_f32small && conv_f32_ks_supported(g))
+        return conv_f32_ks_launch(g, src->ptr, flt->ptr, b, dst->ptr);  // (notes its own variant)
     if (f32 && conv_f32_small_supported(g) && !options().no_f32small) {
         note_kernel("conv_f32_small");
         return conv_f32_small_launch(g, src->ptr, flt->ptr, b, dst->ptr);

@@ -19,6 +19,9 @@
 #include "gevm_f32.h"
 #include "conv_geom.h"
 #include "epilogue.h"
+#ifndef MG_HOST_AUDIT  // (a host build that runs this file's own kernels thread by thread)
+#include "gemm_f32_ks.h"
+#endif
 
 namespace mg {
 
@@ -578,6 +581,11 @@ extern "C" TinyNNStatus megcc_gfx950_matmul(
             return gevm_f32_launch(v);
         }
     }
+#ifndef MG_HOST_AUDIT
+    const GevmArgs ks = {q.A, q.B, q.C, q.M, q.N, q.K, q.a_rs, q.a_cs, q.b_rs, q.b_cs, q.ldc};
+    if (gemm_f32_ks_supported(ks))
+        return gemm_f32_ks_launch(ks, ta, tb);
+#endif
     gemm_plan_split(q, ws);
     // 64 x 256 tiles when they still give every CU a workgroup
     const bool skinny = q.M <= 64 && (long)((q.N + 255) / 256) * q.split >= 128;

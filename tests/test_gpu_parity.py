@@ -378,6 +378,31 @@ def test_fully_connected_over_any_k(kernel, m, k, n, act):
     compare(got, case.run_port(arrays), repr(case))
 
 
+F32_SHARED_K = [
+    # few output tiles, K shared by the waves of a workgroup: extents at and around the 32 / 64 tiles, K below
+    # one step of 8, with and without a rest, and long enough for whole lines per wave
+    *[MatMulCase(m, k, n, trans_a=ta, trans_b=tb) for m, k, n in ((5, 3, 7), (33, 8, 31), (64, 1031, 32), (300, 4100, 70))
+      for ta in (False, True) for tb in (False, True)],
+    MatMulCase(513, 100, 1100), MatMulCase(513, 100, 1100, trans_b=True), MatMulCase(1000, 1500, 1000, trans_b=True),
+    ConvCase(A.FMT_NCHW, A.DENSE, 1, 1, 5, 6, 1, 1, 1, 0, A.IDENTITY, dtype="f32"),
+    ConvCase(A.FMT_NCHW, A.DENSE, 3, 37, 13, 9, 33, 1, 2, 0, A.RELU, dtype="f32"),
+    ConvCase(A.FMT_NCHW, A.DENSE, 2, 16, 11, 17, 31, 3, 2, 1, A.H_SWISH, dtype="f32"),
+    ConvCase(A.FMT_NCHW, A.DENSE, 2, 5, 20, 14, 40, 5, 1, 2, A.SIGMOID, dtype="f32", bias=False),
+    ConvCase(A.FMT_NCHW, A.DENSE, 2, 9, 16, 15, 12, 3, 1, 2, A.RELU, dtype="f32", dilate=2),
+    ConvCase(A.FMT_NCHW, A.DENSE, 5, 126, 31, 30, 100, 3, 1, 0, A.IDENTITY, dtype="f32"),
+    ConvCase(A.FMT_NCHW, A.DENSE, 1, 455, 7, 7, 64, 3, 1, 1, A.RELU, dtype="f32"),
+]
+
+
+@pytest.mark.parametrize("case", F32_SHARED_K, ids=[repr(c) for c in F32_SHARED_K])
+def test_f32_products_whose_waves_share_k(case):
+    port.set_threads(8)
+    arrays = case.gen(seed=19)
+    got = run_gpu(case, arrays)
+    assert "gemm_ks" in runtime.last_kernel() or runtime.last_kernel().startswith("gemm_f32_ks"), runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
 F32_NCHW44 = [
     # f32 channel-wise layers in NCHW44 (the reference's GI_chanwise kernels: 3x3 / 5x5, stride 1 / 2):
     # tiles of 4 x 64 pixels - extents below, at and above a tile, padding 0 .. k/2 + 1, every activation
