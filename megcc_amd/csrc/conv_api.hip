@@ -52,6 +52,11 @@ TinyNNStatus conv_pw_dw_launch(
         const ConvGeom& pw, const ConvGeom& dw, const void* src, const void* packed, const void* pw_bias,
         const void* dw_flt, const void* dw_bias, void* dst);
 
+bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dst);
+TinyNNStatus conv_dw_pw_launch(
+        const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dflt, const void* dbias, const void* packed,
+        const void* pbias, void* dst);
+
 // A filter that went through megcc_gfx950_conv2d_init is a 1-d byte tensor.
 static bool is_packed_filter(const Tensor* flt) {
     return flt->layout.nr_dim == 1;
@@ -849,3 +854,63 @@ extern "C" TinyNNStatus megcc_gfx950_pw_dw(
             pw, dw, t.src->ptr, t.packed->ptr, t.pw_bias ? t.pw_bias->ptr : nullptr, t.dw_flt->ptr,
             t.dw_bias ? t.dw_bias->ptr : nullptr, t.dst->ptr);
 }
+
+// ---- channel-wise 3x3 -> pointwise 1x1 as one operator (model runtime only) ------------------------
+// inputs: source, channel-wise filter [, bias], packed pointwise filter [, bias]; attr.mid_scale is the scale
+// of the tensor in between. check_only: TinyNN_SUCCESS when the kernel takes the pair.
+namespace mg {
+TinyNNStatus dw_pw_run(
+        const MegccPwDwAttr* a, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, bool check_only) {
+    const char* who = "dw_pw";
+    MG_REQUIRE(a && inputs && outputs && nr_output == 1 && outputs[0] &&
+                       nr_input == 3 + (a->pw.with_bias ? 1 : 0) + (a->dw.with_bias ? 1 : 0),
+               TinyNN_ERROR_NULL_PTR, "%s: operands", who);
+    for (int i = 0; i < nr_input; ++i)
+        MG_REQUIRE(inputs[i], TinyNN_ERROR_NULL_PTR, "%s: input %d", who, i);
+    int k = 0;
+    const Tensor* src = inputs[k++];
+    const Tensor* dflt = inputs[k++];
+    const Tensor* dbias = a->dw.with_bias ? inputs[k++] : nullptr;
+    const Tensor* packed = inputs[k++];
+    const Tensor* pbias = a->pw.with_bias ? inputs[k++] : nullptr;
+    Tensor* dst = outputs[0];
+    MG_REQUIRE(is_q8(src) && is_q8(dflt) && is_q8(packed) && is_q8(dst) && (!dbias || is_q32(dbias)) && (!pbias || is_q32(pbias)) &&
+                       a->dw.format == MEGCC_FMT_NCHW44 && a->dw.sparse == MEGCC_SPARSE_GROUP && a->pw.format == MEGCC_FMT_NCHW44 &&
+                       a->pw.sparse == MEGCC_SPARSE_DENSE && is_packed_filter(packed) && !is_packed_filter(dflt) && a->mid_scale > 0.f,
+               TinyNN_ERROR_INVALID_LAYOUT, "%s: operand types", who);
+    ConvGeom dw, pw;
+    TinyNNStatus st = make_geom(&a->dw, src, dflt, nullptr, false, 0, &dw);
+    if (st != TinyNN_SUCCESS)
+        return st;
+    dw.s_dst = a->mid_scale;
+    Tensor mid = {};
+    mid.dtype.type_enum = TinyNN_QINT8;
+    mid.dtype.param.scale = a->mid_scale;
+    mid.layout.nr_dim = 5;
+    const uint32_t md[5] = {(uint32_t)dw.n, (uint32_t)(dw.oc / 4), (uint32_t)dw.oh, (uint32_t)dw.ow, 4u};
+    int stride = 1;
+    for (int i = 4; i >= 0; --i) {
+        mid.layout.dims[i] = md[i];
+        mid.layout.stride[i] = stride;
+        stride *= (int)md[i];
+    }
+    st = make_geom(&a->pw, &mid, packed, dst, true, 0, &pw);
+    if (st != TinyNN_SUCCESS)
+        return st;
+    for (const Tensor* b : {dbias, pbias}) {
+        if (!b)
+            continue;
+        const ConvGeom& g = b == dbias ? dw : pw;
+        const float d = g.s_src * g.s_flt - b->dtype.param.scale;
+        MG_REQUIRE(nr_elem(b->layout) == (size_t)g.oc && is_contiguous(b->layout) && aligned4(b->ptr) && (d < 0 ? -d : d) < 1e-5f,
+                   TinyNN_ERROR_INVALID_LAYOUT, "%s: bias", who);
+    }
+    MG_REQUIRE(conv_dw_pw_supported(dw, pw, src->ptr, dst->ptr) && conv_mfma_supported(pw) &&
+                       nr_elem(packed->layout) == conv_mfma_packed_bytes(pw) && aligned16(packed->ptr) && aligned4(dflt->ptr),
+               TinyNN_ERROR_NO_IMPLEMENT, "%s: shape, activation or alignment the kernel does not take", who);
+    if (check_only)
+        return TinyNN_SUCCESS;
+    return conv_dw_pw_launch(
+            dw, pw, src->ptr, dflt->ptr, dbias ? dbias->ptr : nullptr, packed->ptr, pbias ? pbias->ptr : nullptr, dst->ptr);
+}
+}  // namespace mg

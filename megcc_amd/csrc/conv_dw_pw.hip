@@ -1,0 +1,593 @@
+// Channel-wise 3x3 (pad 1, stride 1 or 2) and the pointwise 1x1 convolution of its result as ONE kernel,
+// qsi8 NCHW44: the block a MobileNet is made of. Run as two kernels the tensor between them goes out and
+// comes back - a third of the bytes of the whole network - and every block pays a second launch. Here
+// it stays in LDS:
+//   A workgroup of 8 waves walks over tiles of T = 64 SUB output pixels (slots: groups of 4 pixels of a
+//   row; a row's last group may hang over). Per tile
+//   1. channel-wise: a job is 16 channels (4 plane sets) x 64 pixels. The multiply-adds are products with
+//      banded matrices on the matrix cores, as in dwconv_mfma.hip but on v_mfma_i32_16x16x64_i8: a column
+//      is a group of 4 output pixels, the rows are 4 pixels x 4 channels, and K is 3 input rows (one quarter
+//      of the lanes each) x the group's own 4 pixels as they lie in memory - one aligned 16-byte load per
+//      lane, no byte loaded twice. (K = 16 pixels of ONE row, three products, loaded each piece four times:
+//      the L1's data path was busy 67 % of the kernel.) The pixels left and right of the group come from the
+//      neighbouring columns, two row shifts (DPP) and a v_mfma_i32_16x16x32_i8; those of the first and last
+//      column by one dword load. With stride 2 the group has 8 pixels, two products and the one on its left.
+//      A lane ends up with the 4 channels of one pixel: one dword, no shuffles. Four plane sets make the 16
+//      consecutive channels of a pixel the next product wants: one ds_write_b128. With up to 128 channels a
+//      wave has one job per tile and keeps its banded matrices in registers, else they are rebuilt per job
+//      from the filter in LDS by v_perm.
+//   2. pointwise: rows = output channels (the packed filter, in registers for the workgroup's life where it
+//      fits 8 chunks per wave, else streamed from L2 a few chunks ahead), columns = 32 pixels, the operand
+//      one conflict-free ds_read_b128 per 32 channels; 4 consecutive accumulators are a dword of the result.
+//   The next job's 12 loads fly while a job is requantised, the next tile's first ones while the pointwise
+//   product runs; two tile buffers, one barrier per tile.
+// Both requantisations are the exact ones of epilogue.h, so the result is bit for bit the two kernels'.
+// Bound: HBM on the large maps, the vector ALU's requantisation and the filter's way from L2 on the small
+// ones. Measured (N=64, us, one kernel / two): 32x112x112->64 22.5 / 33.8, 64 s2 -> 128 18.4 / 26.6,
+// 128x56x56->128 19.6 / 29.5, 256x28x28->256 15.7 / 23.0, 512x14x14->512 11.4 / 22.3; N=256: 87 / 119 and 34 / 49.
+#include <map>
+#include <mutex>
+
+#include "common.h"
+#include "conv_geom.h"
+#include "conv_mfma_i8.h"
+#include "epilogue.h"
+
+namespace mg {
+
+static constexpr int DP_THREADS = 512;
+typedef unsigned dp_v2u __attribute__((ext_vector_type(2)));
+
+struct DwPwParams {
+    const uint32_t* src;
+    const uint32_t* dflt;    // [C/4][3][3] dwords of 4 channel bytes
+    const int32_t* dbias;    // or NULL
+    const int8_t* wp;        // packed pointwise filter [C/32][OCP][32], halves swapped when (oc >> 3) & 1
+    const int32_t* pbias;    // or NULL
+    uint32_t* dst;
+    int src_bytes, dst_bytes;
+    int ih, iw, oh, ow, OC, OCP;
+    int plane;               // bytes of an input plane set
+    int xg, groups, tiles;   // groups of 4 pixels per row, in all; tiles of 16 SUB groups
+    int slices;              // workgroups that share a tile's output channels
+    FastDiv d_xg, d_oh;
+    RequantPack dq, pq;
+    float dc, pc;            // estimates for the tables (mode 0)
+    RequantTable dtable, ptable;
+};
+
+// 16 accumulators of one column -> 4 dwords (each 4 consecutive registers)
+// The empty volatile statements keep each form inside its branch: the compiler otherwise computes one of
+// them ahead of the branch and throws it away, 80 instructions of 120.
+template <int ACT, int N>
+__device__ __forceinline__ void dp_requant(int (&a)[N], uint32_t (&out)[N / 4], const RequantPack& q, float c, const int* table) {
+    auto here = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            asm volatile("" : "+v"(a[i]));
+    };
+    if (q.mode == 1) {  // (uniform)
+        here();
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i)
+            out[i] = requant_pack4<1, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+    } else if (q.mode == 2) {
+        here();
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i)
+            out[i] = requant_pack4<2, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+    } else {
+        here();
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i) {
+            int r[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                r[e] = requant_conv_table<ACT>(a[4 * i + e], c, table);
+            out[i] = pack4_perm(r[0], r[1], r[2], r[3]);
+        }
+    }
+}
+
+// LDS bytes of an instantiation
+template <int KC, int SUB>
+constexpr int dp_lds(int oc) {
+    const int C = 32 * KC;
+    return 2 * (64 * SUB) * C + C * 16 + C * 4 + oc * 4 + 2 * 4 * REQUANT_TABLE_ENTRIES;
+}
+
+// S: stride; KC: 32-channel chunks; SUB: 64-pixel parts of a tile; MT, NT: 32-channel and 32-pixel tiles per
+// wave of the pointwise product; RAG: IW % 4 (the input pixel right of a row's end is in its last piece)
+// DACT, PACT: activations of the two layers (IDENTITY / RELU)
+template <int S, int KC, int SUB, int MT, int NT, int RAG, int DACT, int PACT>
+__global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q) {
+    constexpr int C = 32 * KC, NQ = 2 * KC, T = 64 * SUB;
+    constexpr int JW = NQ * SUB / 8;                 // channel-wise jobs per wave and tile
+    constexpr int WP = T / (32 * NT), WO = 8 / WP;   // waves along the pixels, along the channels
+    constexpr bool KEEP_D = JW == 1 && S == 1, KEEP_P = KC * MT <= 8;
+    // chunks of the pointwise filter in flight (not KEEP_P): as many as the registers hold without spilling
+    constexpr int RING = KC >= 32 ? 2 : KC == 16 && S == 2 ? 4 : 8;
+    static_assert(JW >= 1 && WP >= 1 && WO >= 1 && WP * WO == 8, "8 waves");
+    extern __shared__ __attribute__((aligned(16))) int8_t dp_lds_mem[];
+    int8_t* const mid = dp_lds_mem;                             // [2][NQ][T] 16-byte pieces
+    int* const wl = (int*)(mid + 2 * T * C);                    // [C][4]: per channel the filter's 3 rows
+    int* const db = wl + C * 4;                                 // [C] bias
+    int* const pb = db + C;                                     // [OC slice] bias
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ocs = WO * 32 * MT;                               // channels of a slice
+    int* const dtbl = pb + ocs;
+    int* const ptbl = dtbl + REQUANT_TABLE_ENTRIES;
+
+    // workgroup -> (slice, run of tiles); each XCD gets a contiguous stretch of the runs
+    const int nb = gridDim.x;
+    const int lb = (nb & 7) == 0 ? (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    const int slice = lb % q.slices, wi = lb / q.slices, nw = nb / q.slices;
+    const int run_q = q.tiles / nw, run_r = q.tiles - run_q * nw;
+    const int t_begin = wi * run_q + min(wi, run_r), t_end = t_begin + run_q + (wi < run_r ? 1 : 0);
+
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)q.src, 0, q.src_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)q.dst, 0, q.dst_bytes, 0x00020000);
+    const unsigned OOB = 0x80000000u;
+    const int colq = lane & 15, kg4 = lane >> 4;   // channel-wise: column, quarter of K / pixel of the group
+    const int col = lane & 31, kg = lane >> 5;     // pointwise: column, half of K
+
+    // what a lane (column colq, input row kg4) reads of a job: byte offsets in plane set 0
+    struct Rows {
+        unsigned off, offb;   // the group's pixels (S = 2: offb the second four)
+        unsigned eoff;        // first / last column: the pixel left / right of the columns
+        unsigned lmask, rmask;
+        bool edge, edgeb;     // RAG: the piece (second piece) holds the pixel right of the row's end
+    };
+    auto rows_of = [&](int tile, int u) __attribute__((always_inline)) -> Rows {
+        const int g = tile * (16 * SUB) + u * 16 + colq;
+        const int rg = (int)fdiv(g, q.d_xg), x0 = (g - rg * q.xg) * 4;
+        const int n = (int)fdiv(rg, q.d_oh), y = rg - n * q.oh;
+        const int ix = S * x0, iy = S * y - 1 + kg4;
+        const bool ok = g < q.groups && tile < t_end && kg4 < 3 && (unsigned)iy < (unsigned)q.ih;
+        const unsigned o = (unsigned)(n * (C / 4) * q.plane + (iy * q.iw + ix) * 4);
+        Rows r;
+        r.off = ok ? o : OOB;
+        r.offb = ok && ix + 4 < q.iw ? o + 16 : OOB;
+        const bool l = x0 > 0, rt = ix + 4 < q.iw;
+        r.lmask = l ? ~0u : 0u;
+        r.rmask = rt ? ~0u : 0u;
+        r.eoff = ok && colq == 0 && l ? o - 4 : S == 1 && ok && colq == 15 && rt ? o + 16 : OOB;
+        r.edge = RAG != 0 && ix + 4 > q.iw;
+        r.edgeb = RAG != 0 && ix + 4 <= q.iw && ix + 8 > q.iw;
+        return r;
+    };
+    v4i B[4][S];
+    unsigned E[4];
+    auto request = [&](const Rows& r, int quad) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int pl = (quad * 4 + p) * q.plane;
+            B[p][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)r.off, pl, 0));
+            if (S == 2)
+                B[p][S - 1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)r.offb, pl, 0));
+            E[p] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)r.eoff, pl, 0);
+        }
+    };
+    // job i of this wave: channels 16 quad .. + 15, pixels 64 u .. + 63 of the tile
+    auto quad_of = [&](int i) { return (wave + 8 * i) % NQ; };
+    auto sub_of = [&](int i) { return (wave + 8 * i) / NQ; };
+    Rows rows = rows_of(t_begin, sub_of(0)), cur;
+    request(rows, quad_of(0));
+
+    // ---- set-up: filters, biases, tables -----------------------------------------------------------
+    // (all loads of a thread before its first store: a round trip for the whole set-up, not one per turn)
+    constexpr int WI = (C * 4 + DP_THREADS - 1) / DP_THREADS, BI = (C + DP_THREADS - 1) / DP_THREADS;
+    constexpr int PI = (WO * 32 * MT + DP_THREADS - 1) / DP_THREADS;
+    uint32_t wv[WI][3];
+    int dbv[BI], pbv[PI];
+#pragma unroll
+    for (int k = 0; k < WI; ++k) {
+        const int i = min(tid + k * DP_THREADS, C * 4 - 1);
+        const uint32_t* w = q.dflt + ((i >> 4) * 3 + min(i & 3, 2)) * 3;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            wv[k][j] = w[j];
+    }
+#pragma unroll
+    for (int k = 0; k < BI; ++k)
+        dbv[k] = q.dbias ? q.dbias[min(tid + k * DP_THREADS, C - 1)] : 0;
+#pragma unroll
+    for (int k = 0; k < PI; ++k)
+        pbv[k] = q.pbias ? q.pbias[min(slice * ocs + tid + k * DP_THREADS, q.OC - 1)] : 0;
+#pragma unroll
+    for (int k = 0; k < WI; ++k) {
+        const int i = tid + k * DP_THREADS, dy = i & 3, sh = 8 * ((i >> 2) & 3);
+        const uint32_t v = ((wv[k][0] >> sh) & 0xff) | (((wv[k][1] >> sh) & 0xff) << 8) | (((wv[k][2] >> sh) & 0xff) << 16);
+        if (i < C * 4)
+            wl[i] = dy < 3 ? (int)v : 0;  // (a fourth row of zeros)
+    }
+#pragma unroll
+    for (int k = 0; k < BI; ++k)
+        if (tid + k * DP_THREADS < C)
+            db[tid + k * DP_THREADS] = dbv[k];
+#pragma unroll
+    for (int k = 0; k < PI; ++k)
+        if (tid + k * DP_THREADS < ocs)
+            pb[tid + k * DP_THREADS] = pbv[k];
+    if (tid < REQUANT_TABLE_ENTRIES) {
+        if (q.dq.mode == 0)
+            dtbl[tid] = q.dtable.t[tid];
+    } else if (q.pq.mode == 0) {
+        ptbl[tid - REQUANT_TABLE_ENTRIES] = q.ptable.t[tid - REQUANT_TABLE_ENTRIES];
+    }
+    // byte selectors of the banded matrices: row = (pixel colq >> 2, channel colq & 3) of the group, input row kg4;
+    // the group's input pixel k meets it through filter column k + 1 - S px
+    const int px = colq >> 2, sh = 8 * (colq & 3);
+    auto selector = [&](int fw) { return (unsigned)fw < 3u ? (0x0c0c0c0cu & ~(0xffu << sh)) | ((unsigned)fw << sh) : 0x0c0c0c0cu; };
+    unsigned sel[4 * S], sell = selector(-S * px), selr = selector(5 - px);  // (left: k = -1, right: k = 4)
+#pragma unroll
+    for (int k = 0; k < 4 * S; ++k)
+        sel[k] = selector(k + 1 - S * px);
+    // pointwise filter rows of this wave
+    const int wo = wave % WO, wpx = wave / WO;
+    const int oc_wave = slice * ocs + wo * (32 * MT);
+    const int8_t* prow[MT];
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi) {
+        const int oc = min(oc_wave + mi * 32, q.OCP - 32) + col;
+        prow[mi] = q.wp + (size_t)oc * KROW + (((kg ^ (oc >> 3)) & 1) << 4);
+    }
+    const size_t cstep = (size_t)q.OCP * KROW;
+    v4i P[KEEP_P ? KC : RING][MT];
+    if (KEEP_P) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+#pragma unroll
+            for (int mi = 0; mi < MT; ++mi)
+                P[KEEP_P ? c : 0][mi] = *(const v4i*)(prow[mi] + c * cstep);
+    }
+    __syncthreads();
+    struct Band {
+        v4i m[S];
+        dp_v2u e;  // left, right
+    };
+    auto band_filter = [&](int quad, int p) { return (unsigned)wl[((quad * 4 + p) * 4 + (colq & 3)) * 4 + kg4]; };
+    auto band_half = [&](unsigned w, int h) __attribute__((always_inline)) {
+        v4i m;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            m[k] = (int)__builtin_amdgcn_perm(0u, w, sel[4 * h + k]);
+        return m;
+    };
+    auto band_edges = [&](unsigned w) __attribute__((always_inline)) {
+        return dp_v2u{__builtin_amdgcn_perm(0u, w, sell), S == 1 ? __builtin_amdgcn_perm(0u, w, selr) : 0u};
+    };
+    Band A[KEEP_D ? 4 : 1];
+    if (KEEP_D) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const unsigned w = band_filter(quad_of(0), p);
+#pragma unroll
+            for (int h = 0; h < S; ++h)
+                A[KEEP_D ? p : 0].m[h] = band_half(w, h);
+            A[KEEP_D ? p : 0].e = band_edges(w);
+        }
+    }
+
+    // (nothing in flight from here: the loop's own waits are then exact)
+    wait_vmcnt<0>();
+    for (int t = t_begin, buf = 0; t < t_end; ++t, buf ^= 1) {
+        // the pointwise filter's first chunks fly while the channel-wise stage runs
+        if (!KEEP_P) {
+#pragma unroll
+            for (int c = 0; c < RING; ++c)
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi)
+                    P[c][mi] = *(const v4i*)(prow[mi] + c * cstep);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        int8_t* const m = mid + buf * (T * C);
+        // ---- channel-wise ----------------------------------------------------------------------------
+#pragma unroll
+        for (int i = 0; i < JW; ++i) {
+            const int quad = quad_of(i), u = sub_of(i);
+            v4i acc[4];
+            if (i == 0)
+                cur = rows;
+            // the pixels left and right of each column's group
+            unsigned L[4], R[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                L[p] = E[p];
+                R[p] = E[p];
+            }
+            // (one block: a DPP read needs two cycles behind a vector write of its source)
+            asm volatile(
+                    "s_nop 1\n\t"
+                    "v_and_b32_dpp %0, %4, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                    "v_and_b32_dpp %1, %5, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                    "v_and_b32_dpp %2, %6, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                    "v_and_b32_dpp %3, %7, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                    "s_nop 1"
+                    : "+v"(L[0]), "+v"(L[1]), "+v"(L[2]), "+v"(L[3])
+                    : "v"(B[0][S - 1][3]), "v"(B[1][S - 1][3]), "v"(B[2][S - 1][3]), "v"(B[3][S - 1][3]), "v"(cur.lmask));
+            if (S == 1)
+                asm volatile(
+                        "s_nop 1\n\t"
+                        "v_and_b32_dpp %0, %4, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                        "v_and_b32_dpp %1, %5, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                        "v_and_b32_dpp %2, %6, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                        "v_and_b32_dpp %3, %7, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                        "s_nop 1"
+                        : "+v"(R[0]), "+v"(R[1]), "+v"(R[2]), "+v"(R[3])
+                        : "v"(B[0][0][0]), "v"(B[1][0][0]), "v"(B[2][0][0]), "v"(B[3][0][0]), "v"(cur.rmask));
+            // The short products of all four plane sets first: a long one that follows ITS short one directly has
+            // read sums that were not there yet (channels 0 and 1 of the last pixels), behind three others it never
+            // does.
+            unsigned w[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                acc[p] = *(const v4i*)(db + quad * 16 + p * 4);
+                if (!KEEP_D)
+                    w[p] = band_filter(quad, p);
+            }
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const dp_v2u al = KEEP_D ? A[KEEP_D ? p : 0].e : band_edges(w[p]), bl = {L[p], S == 1 ? R[p] : L[p]};
+                acc[p] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                        __builtin_bit_cast(long, al), __builtin_bit_cast(long, bl), acc[p], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int h = 0; h < S; ++h)
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    v4i b = B[p][h];
+                    if (RAG)
+                        b[RAG] = (h == 0 ? cur.edge : cur.edgeb) ? 0 : b[RAG];
+                    acc[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                            KEEP_D ? A[KEEP_D ? p : 0].m[h] : band_half(w[p], h), b, acc[p], 0, 0, 0);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            // the operands are consumed: the next job's loads fly while this one is requantised
+            // (several jobs a tile: tiles of 64 pixels, the same rows for all of them)
+            static_assert(JW == 1 || SUB == 1, "");
+            if (KEEP_P || i + 1 < JW) {
+                if (i + 1 == JW)
+                    rows = rows_of(t + 1, sub_of(0));
+                request(rows, quad_of(i + 1 < JW ? i + 1 : 0));
+            }
+            int a[16];
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    a[p * 4 + e] = acc[p][e];
+            uint32_t d[4];
+            dp_requant<DACT>(a, d, q.dq, q.dc, dtbl);
+            *(v4i*)(m + (quad * T + u * 64 + colq * 4 + kg4) * 16) = v4i{(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
+        }
+        lds_barrier();
+        // ---- pointwise -------------------------------------------------------------------------------
+        // where a column's results go. (Stores are issued whether or not the place exists: what is under no
+        // condition the compiler can count, and the next tile then waits for its loads, not for these stores.)
+        struct Where {
+            unsigned base;
+            bool ok;
+        };
+        auto where = [&](int ni) __attribute__((always_inline)) -> Where {
+            const int s = (wpx * NT + ni) * 32 + col;
+            const int g = t * (16 * SUB) + (s >> 2);
+            const int rg = (int)fdiv(g, q.d_xg), x = (g - rg * q.xg) * 4 + (s & 3);
+            const int n = (int)fdiv(rg, q.d_oh), y = rg - n * q.oh;
+            Where w;
+            w.ok = g < q.groups && x < q.ow;
+            w.base = (unsigned)((n * (q.OC >> 2) * q.oh + y) * q.ow + x) * 4u;
+            return w;
+        };
+        const unsigned ostep = (unsigned)(q.oh * q.ow) * 4u;
+        auto bias_of = [&](int mi, v16i& acc) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                const v4i bv = *(const v4i*)(pb + wo * (32 * MT) + mi * 32 + e4 * 8 + kg * 4);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    acc[e4 * 4 + k] = bv[k];
+            }
+        };
+        auto finish = [&](int mi, const Where& w, const v16i& acc) __attribute__((always_inline)) {
+            int a[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                a[e] = acc[e];
+            uint32_t d[4];
+            dp_requant<PACT>(a, d, q.pq, q.pc, ptbl);
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                const int oc4 = ((oc_wave + mi * 32) >> 2) + e4 * 2 + kg;
+                __builtin_amdgcn_raw_buffer_store_b32(d[e4], rd, (int)(oc4 * 4 < q.OC && w.ok ? w.base + (unsigned)oc4 * ostep : OOB), 0, 0);
+            }
+        };
+        auto operand = [&](int c, int ni) __attribute__((always_inline)) {
+            return *(const v4i*)(m + ((2 * c + kg) * T + (wpx * NT + ni) * 32 + col) * 16);
+        };
+        if constexpr (KEEP_P) {
+            // one 32 x 32 tile after the other: 16 accumulators live, four waves to a SIMD
+#pragma unroll
+            for (int ni = 0; ni < NT; ++ni) {
+                const Where w = where(ni);
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi) {
+                    v16i acc;
+                    bias_of(mi, acc);
+#pragma unroll
+                    for (int c = 0; c < KC; ++c)
+                        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(P[c][mi], operand(c, ni), acc, 0, 0, 0);
+                    finish(mi, w, acc);
+                }
+            }
+        } else {
+            v16i acc[MT][NT];
+#pragma unroll
+            for (int mi = 0; mi < MT; ++mi) {
+                bias_of(mi, acc[mi][0]);
+#pragma unroll
+                for (int ni = 1; ni < NT; ++ni)
+                    acc[mi][ni] = acc[mi][0];
+            }
+            static_for<KC>([&](auto cc) {
+                constexpr int c = decltype(cc)::value, slot = c % RING;
+#pragma unroll
+                for (int ni = 0; ni < NT; ++ni) {
+                    const v4i b = operand(c, ni);
+#pragma unroll
+                    for (int mi = 0; mi < MT; ++mi)
+                        acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(P[slot][mi], b, acc[mi][ni], 0, 0, 0);
+                }
+                if (c + RING < KC) {
+#pragma unroll
+                    for (int mi = 0; mi < MT; ++mi)
+                        P[slot][mi] = *(const v4i*)(prow[mi] + (c + RING) * cstep);
+                }
+                // the next tile's first job, behind the last chunk of the filter: loads come back in the order they
+                // were issued, and one asked for after these would wait for them
+                if (c + (RING < KC ? RING : KC) == KC) {
+                    rows = rows_of(t + 1, sub_of(0));
+                    request(rows, quad_of(0));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+#pragma unroll
+            for (int ni = 0; ni < NT; ++ni) {
+                const Where w = where(ni);
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi)
+                    finish(mi, w, acc[mi][ni]);
+            }
+        }
+    }
+}
+
+// the instantiation for C channels and OC: SUB, MT, NT
+struct DpShape {
+    int kc, sub, mt, nt;
+};
+static bool dp_shape(int c, int oc, DpShape* s) {
+    switch (c) {
+        case 32: *s = {1, 4, 2, 1}; break;                        // 64 channels a slice
+        case 64: *s = {2, 2, 2, 1}; break;                        // 128
+        case 128: *s = oc <= 128 ? DpShape{4, 1, 1, 1} : DpShape{4, 1, 1, 2}; break;  // 128 / 256
+        case 256: *s = oc <= 256 ? DpShape{8, 1, 1, 2} : DpShape{8, 1, 2, 2}; break;  // 256 / 512
+        case 512: *s = {16, 1, 2, 2}; break;                      // 512
+        case 1024: *s = {32, 1, 2, 2}; break;
+        default: return false;
+    }
+    return true;
+}
+
+bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dst) {
+    DpShape s;
+    return dw.fmt == MEGCC_FMT_NCHW44 && dw.groups == dw.ic && dw.ic == dw.oc && dw.fh == 3 && dw.fw == 3 && dw.ph == 1 &&
+           dw.pw == 1 && dw.dh == 1 && dw.dw == 1 && dw.sh == dw.sw && (dw.sh == 1 || dw.sh == 2) &&
+           pw.fmt == MEGCC_FMT_NCHW44 && pw.groups == 1 && pw.fh == 1 && pw.fw == 1 && pw.sh == 1 && pw.sw == 1 && pw.ph == 0 &&
+           pw.pw == 0 && pw.ic == dw.oc && (pw.oc & 31) == 0 && dp_shape(dw.ic, pw.oc, &s) &&
+           dw.act == MEGCC_NONLINE_RELU &&
+           (pw.act == MEGCC_NONLINE_IDENTITY || pw.act == MEGCC_NONLINE_RELU) &&
+           requant_table_ok(dw.s_src, dw.s_flt, dw.s_dst) && requant_table_ok(pw.s_src, pw.s_flt, pw.s_dst) &&
+           ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 3) == 0 && (long)dw.n * dw.ic * dw.ih * dw.iw < (1L << 31) &&
+           (long)pw.n * pw.oc * pw.oh * pw.ow < (1L << 31) && (long)dw.ih * dw.iw < (1L << 24) && dw.oh > 0 && dw.ow > 0;
+}
+
+template <int S, int KC, int SUB, int MT, int NT>
+static const void* dp_kernel(int rag, int dact, int pact) {
+    // (MobileNets use RELU behind both layers; a RELU-less pointwise layer is the linear bottleneck)
+#define MG_DP_ACT(R_)                                                                                                   \
+    (dact == MEGCC_NONLINE_RELU                                                                                          \
+             ? (pact == MEGCC_NONLINE_RELU ? (const void*)conv_dw_pw_kernel<S, KC, SUB, MT, NT, R_, MEGCC_NONLINE_RELU, MEGCC_NONLINE_RELU>        \
+                                           : (const void*)conv_dw_pw_kernel<S, KC, SUB, MT, NT, R_, MEGCC_NONLINE_RELU, MEGCC_NONLINE_IDENTITY>)   \
+             : nullptr)
+    return rag == 0 ? MG_DP_ACT(0) : rag == 1 ? MG_DP_ACT(1) : rag == 2 ? MG_DP_ACT(2) : MG_DP_ACT(3);
+#undef MG_DP_ACT
+}
+
+// workgroups of `kern` one CU holds at a time; 0 where it cannot have its LDS. Asked for once per kernel (its LDS
+// size goes with it).
+static int dp_resident(const void* kern, size_t lds) {
+    static std::map<const void*, int> cache;
+    static std::mutex lock;
+    std::lock_guard<std::mutex> guard(lock);
+    auto it = cache.find(kern);
+    if (it != cache.end())
+        return it->second;
+    int n = 0;
+    if (lds > 48 * 1024 && hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, DP_THREADS, lds) != hipSuccess || n < 1)
+        n = 1;
+    return cache[kern] = n;
+}
+
+TinyNNStatus conv_dw_pw_launch(
+        const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dflt, const void* dbias, const void* packed,
+        const void* pbias, void* dst) {
+    DwPwParams q = {};
+    DpShape s;
+    MG_REQUIRE(dp_shape(dw.ic, pw.oc, &s), TinyNN_ERROR_NO_IMPLEMENT, "conv_dw_pw: %d channels", dw.ic);
+    q.src = (const uint32_t*)src;
+    q.dflt = (const uint32_t*)dflt;
+    q.dbias = (const int32_t*)dbias;
+    q.wp = (const int8_t*)packed;
+    q.pbias = (const int32_t*)pbias;
+    q.dst = (uint32_t*)dst;
+    q.src_bytes = (int)((long)dw.n * dw.ic * dw.ih * dw.iw);
+    q.dst_bytes = (int)((long)pw.n * pw.oc * pw.oh * pw.ow);
+    q.ih = dw.ih, q.iw = dw.iw, q.oh = dw.oh, q.ow = dw.ow;
+    q.OC = pw.oc;
+    q.OCP = (pw.oc + OC_PAD - 1) / OC_PAD * OC_PAD;
+    q.plane = dw.ih * dw.iw * 4;
+    q.xg = (dw.ow + 3) / 4;
+    q.groups = dw.n * dw.oh * q.xg;
+    q.tiles = (q.groups + 16 * s.sub - 1) / (16 * s.sub);
+    const int wo = 8 / (64 * s.sub / (32 * s.nt)), ocs = wo * 32 * s.mt;
+    q.slices = (pw.oc + ocs - 1) / ocs;
+    q.d_xg = make_fastdiv(q.xg);
+    q.d_oh = make_fastdiv(q.oh);
+    q.dq = requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
+    q.pq = requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
+    q.dc = make_requant_fast(dw.s_src, dw.s_flt, dw.s_dst).c;
+    q.pc = make_requant_fast(pw.s_src, pw.s_flt, pw.s_dst).c;
+    if (q.dq.mode == 0)
+        q.dtable = requant_table_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
+    if (q.pq.mode == 0)
+        q.ptable = requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
+    const int rag = dw.iw & 3;
+    const void* kern = nullptr;
+    size_t lds = 0;
+#define MG_DP(KC_, SUB_, MT_, NT_)                                                                                   \
+    if (s.kc == KC_ && s.mt == MT_ && s.nt == NT_) {                                                                   \
+        kern = dw.sh == 1 ? dp_kernel<1, KC_, SUB_, MT_, NT_>(rag, dw.act, pw.act) : dp_kernel<2, KC_, SUB_, MT_, NT_>(rag, dw.act, pw.act); \
+        lds = (size_t)dp_lds<KC_, SUB_>(ocs);                                                                          \
+    }
+    MG_DP(1, 4, 2, 1)
+    MG_DP(2, 2, 2, 1)
+    MG_DP(4, 1, 1, 1)
+    MG_DP(4, 1, 1, 2)
+    MG_DP(8, 1, 1, 2)
+    MG_DP(8, 1, 2, 2)
+    MG_DP(16, 1, 2, 2)
+    MG_DP(32, 1, 2, 2)
+#undef MG_DP
+    MG_REQUIRE(kern, TinyNN_ERROR_NO_IMPLEMENT, "conv_dw_pw: no instance");
+    const int resident = dp_resident(kern, lds);
+    MG_REQUIRE(resident > 0, TinyNN_ERROR_RUNTIME, "conv_dw_pw: %d bytes of LDS", (int)lds);
+    // as many workgroups as are resident, each with a run of tiles
+    long runs = (long)num_cus() * resident / q.slices;
+    if (runs < 1)
+        runs = 1;
+    if (runs > q.tiles)
+        runs = q.tiles;
+    note_kernel("conv_dw_pw", dw.ic / 32, dw.sh, q.slices);
+    note_requant_affine(q.dq.mode != 0 && q.pq.mode != 0);
+    void* args[] = {&q};
+    hipError_t e = hipLaunchKernel(kern, dim3((unsigned)(runs * q.slices)), dim3(DP_THREADS), args, lds, stream());
+    MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_dw_pw: %s", hipGetErrorString(e));
+    return check_launch("conv_dw_pw");
+}
+
+}  // namespace mg

@@ -235,6 +235,41 @@ __device__ __forceinline__ int requant_conv_affine(int acc, float c, float d) {
     return m < LO ? LO : (m > 127 ? 127 : m);
 }
 
+// ---- four outputs at a time: scale, round, saturate and pack in one conversion ---------------------
+// v_cvt_pk_u8_f32 rounds to nearest (ties to even), saturates to 0..255 and puts the byte where it
+// belongs, which makes the floor, the clamp and the byte shuffling of the forms above unnecessary: 3
+// instructions per output and 1 / 2 per four of them. In RELU's case the byte is 2 out (+ 1): 0..255 covers
+// 0..127.5, and the one bit that is dropped afterwards turns the rounding into a floor; in IDENTITY's it
+// is out + 128. The value converted is
+//     mode 1: fma((float)a, c, d)              mode 2: fma(((float)a * s1) * s2, c, d)
+// - mode 2 repeats the reference's own first two roundings (or one of them: s2 = 1) and finds constants
+// where mode 1 has none (many input channels: c is small, and so is the room between the steps). All of
+// it is non-decreasing in a, so it equals the reference on all of int32 iff it does on both sides of each
+// of its steps: the host search (requant_table.hip) checks exactly that. Scales with exact ties whose
+// roundings land on either side have no such constants (mode 0) and keep the table.
+struct RequantPack {
+    float s1, s2, c, d;
+    int mode;
+};
+RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst);
+
+#ifndef MG_HOST_AUDIT  // (the conversion has no host form)
+// MODE, ACT compile-time; channels (or pixels) 0..3 of one dword
+template <int MODE, int ACT>
+__device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3, const RequantPack& q) {
+    const int a[4] = {a0, a1, a2, a3};
+    uint32_t r = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float x = (float)a[i];
+        if (MODE == 2)
+            x = x * q.s1 * q.s2;
+        r = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(x, q.c, q.d), i, r);
+    }
+    return ACT == MEGCC_NONLINE_RELU ? (r >> 1) & 0x7f7f7f7fu : r ^ 0x80808080u;
+}
+#endif
+
 // host side: the estimate above is valid (else kernels use the literal sequence per element)
 static inline bool requant_table_ok(float s_src, float s_flt, float s_dst) {
     const RequantFast q = make_requant_fast(s_src, s_flt, s_dst);

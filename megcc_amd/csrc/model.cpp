@@ -50,6 +50,7 @@ struct ModelOpr {
     void* processed_mem = nullptr;
     Workspace ws;
     int first_index = -1;  // index in Model::oprs of the (first) operator this schedule entry stands for
+    bool dw_pw = false;    // a channel-wise + pointwise pair as one kernel (desc.attr.pw_dw, no kind of its own)
 };
 
 struct Model {
@@ -179,13 +180,19 @@ bool plan_memory(Model* m) {
     // channel-wise layer's result: that source stays alive one operator longer, as it would in a
     // plan made for the one operator.
     std::vector<int> keep_until(m->tensors.size(), -1);
-    for (size_t i = 0; !options().no_fuse_pwdw && i + 1 < m->oprs.size(); ++i) {
+    for (size_t i = 0; i + 1 < m->oprs.size(); ++i) {
         const ModelOpr *o0 = m->oprs[i], *o1 = m->oprs[i + 1];
         if (o0->desc.kind != MEGCC_KERN_CONV || o1->desc.kind != MEGCC_KERN_CONV || o0->in.empty() ||
             o1->in.empty() || o0->out.size() != 1 || o1->in[0] != o0->out[0])
             continue;
         const MegccConvAttr &a = o0->desc.attr.conv, &b = o1->desc.attr.conv;
-        if (a.format == MEGCC_FMT_NCHW44 && a.sparse == MEGCC_SPARSE_DENSE && a.kernel_h == 1 && a.kernel_w == 1 &&
+        // The same for a channel-wise layer in front of a pointwise one (conv_dw_pw.hip). Not under
+        // "nopipeline", which keeps the plan to the operators as they are.
+        if (!options().no_fuse_dwpw && !options().no_pipeline && a.format == MEGCC_FMT_NCHW44 && a.sparse == MEGCC_SPARSE_GROUP &&
+            a.kernel_h == 3 && a.kernel_w == 3 && b.format == MEGCC_FMT_NCHW44 && b.sparse == MEGCC_SPARSE_DENSE && b.kernel_h == 1 &&
+            b.kernel_w == 1 && b.stride_h == 1 && b.stride_w == 1)
+            keep_until[root_of(m, o0->in[0])] = (int)i + 1;
+        if (!options().no_fuse_pwdw && a.format == MEGCC_FMT_NCHW44 && a.sparse == MEGCC_SPARSE_DENSE && a.kernel_h == 1 && a.kernel_w == 1 &&
             a.stride_h == 1 && a.stride_w == 1 && a.pad_h == 0 && a.pad_w == 0 && b.format == MEGCC_FMT_NCHW44 &&
             b.sparse == MEGCC_SPARSE_GROUP && b.kernel_h == 3 && b.kernel_w == 3 && b.pad_h == 1 && b.pad_w == 1) {
             // ... where the one kernel can win at all: shapes it takes, and no more images than give
@@ -253,6 +260,15 @@ static bool shares_bytes(const Tensor& a, const Tensor& b) {
         return false;
     return a0 < b0 + bn && b0 < a0 + an;
 }
+// one entry of the schedule
+static TinyNNStatus call_opr(Model* m, ModelOpr* o) {
+    if (o->dw_pw)
+        return dw_pw_run(&o->desc.attr.pw_dw, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(),
+                         (int)o->out_ptrs.size(), false);
+    return megcc_gfx950_call(
+            &o->desc, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(), (int)o->out_ptrs.size(), &o->ws,
+            &m->opt);
+}
 // Milliseconds `iters` back-to-back rounds of the operators in `ops` take on the library stream
 // (after one untimed round), or a negative value when a launch fails or an operand has no memory.
 static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters) {
@@ -266,9 +282,7 @@ static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters) {
     }
     auto round = [&]() {
         for (ModelOpr* o : ops)
-            if (megcc_gfx950_call(
-                        &o->desc, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(),
-                        (int)o->out_ptrs.size(), &o->ws, &m->opt) != TinyNN_SUCCESS)
+            if (call_opr(m, o) != TinyNN_SUCCESS)
                 return false;
         return true;
     };
@@ -361,6 +375,46 @@ static void build_schedule(Model* m, bool allow_pw_dw = true) {
                 delete f;
             }
         }
+        // A channel-wise 3x3 convolution and the pointwise convolution of its result: one kernel
+        // (conv_dw_pw.hip) when nothing else reads the tensor in between and it measures faster.
+        if (!options().no_fuse_dwpw && i + 1 < n && o0->desc.kind == MEGCC_KERN_CONV && !o0->has_processed && o0->out.size() == 1 &&
+            o0->desc.attr.conv.sparse == MEGCC_SPARSE_GROUP && o0->in.size() == (o0->desc.attr.conv.with_bias ? 3u : 2u)) {
+            ModelOpr* o1 = m->oprs[i + 1];
+            if (o1->desc.kind == MEGCC_KERN_CONV && o1->has_processed && o1->out.size() == 1 && o1->in[0] == o0->out[0] &&
+                o1->in.size() == (o1->desc.attr.conv.with_bias ? 3u : 2u) && temp(o0->out[0], 1)) {
+                ModelOpr* f = new ModelOpr();
+                f->first_index = i;
+                f->dw_pw = true;
+                memset(&f->desc, 0, sizeof(f->desc));
+                f->desc.attr.pw_dw.dw = o0->desc.attr.conv;
+                f->desc.attr.pw_dw.pw = o1->desc.attr.conv;
+                f->desc.attr.pw_dw.mid_scale = m->tensors[o0->out[0]]->t.dtype.param.scale;
+                f->symbol = "depthwise 3x3 + pointwise 1x1 (fused)";
+                memset(&f->ws, 0, sizeof(f->ws));
+                f->in = o0->in;
+                f->in_ptrs = o0->in_ptrs;
+                for (size_t k = 1; k < o1->in.size(); ++k) {
+                    f->in.push_back(o1->in[k]);
+                    f->in_ptrs.push_back(o1->in_ptrs[k]);
+                }
+                f->out = o1->out;
+                f->out_ptrs = o1->out_ptrs;
+                bool take = !shares_bytes(*f->in_ptrs[0], *f->out_ptrs[0]) &&
+                            dw_pw_run(&f->desc.attr.pw_dw, f->in_ptrs.data(), (int)f->in_ptrs.size(), f->out_ptrs.data(),
+                                      (int)f->out_ptrs.size(), true) == TinyNN_SUCCESS;
+                if (take && !options().fuse_dwpw) {
+                    const float one = time_oprs(m, {f}, 10), two = time_oprs(m, {o0, o1}, 10);
+                    take = one > 0.f && two > 0.f && one < 0.97f * two;
+                }
+                if (take) {
+                    m->fused.push_back(f);
+                    m->schedule.push_back(f);
+                    i += 1;
+                    continue;
+                }
+                delete f;
+            }
+        }
         // A pointwise convolution and the channel-wise 3x3 convolution of its result, on images small
         // enough for a workgroup to hold one: one kernel (megcc_gfx950_pw_dw) when nothing else reads
         // the tensor in between.
@@ -399,7 +453,7 @@ static void build_schedule(Model* m, bool allow_pw_dw = true) {
                 // contents do not matter before the first forward) and the faster one is kept. The
                 // switch "fusepwdw" takes the one kernel without measuring.
                 if (take && !options().fuse_pwdw) {
-                    const float one = time_oprs(m, {f}, 20), two = time_oprs(m, {o0, o1}, 20);
+                    const float one = time_oprs(m, {f}, 10), two = time_oprs(m, {o0, o1}, 10);
                     take = one > 0.f && two > 0.f && one < 0.97f * two;
                 }
                 if (take) {
@@ -625,9 +679,7 @@ static TinyNNStatus forward_eager(Model* m, bool overlap = false, hipEvent_t don
         } else if (idx < tb && m->tail_pending && m->waits_tail[(size_t)idx]) {
             join_tail(m);
         }
-        st = megcc_gfx950_call(
-                &o->desc, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(),
-                (int)o->out_ptrs.size(), &o->ws, &m->opt);
+        st = call_opr(m, o);
     }
     if (tb >= 0) {
         set_stream_override(nullptr, false);
@@ -1039,8 +1091,12 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
     // as two; batch 32 the other way round): the whole forward is timed both ways and the faster
     // schedule kept.
     bool has_pair = false;
-    for (const ModelOpr* o : m->schedule)
+    bool has_dw_pw = false;  // (a pair that saves work, not only a launch: judged well enough one by one)
+    for (const ModelOpr* o : m->schedule) {
         has_pair = has_pair || o->desc.kind == MEGCC_KERN_PW_DW;
+        has_dw_pw = has_dw_pw || o->dw_pw;
+    }
+    has_pair = has_pair && !has_dw_pw;
     if (with > 0.f && has_pair && !options().fuse_pwdw) {
         const std::vector<ModelOpr*> fused_schedule = m->schedule;
         const int fused_tb = m->tail_begin;

@@ -128,6 +128,111 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
         }
     }
     std::lock_guard<std::mutex> guard(lock);
+    if (cache.size() >= 4096)
+        cache.clear();
+    return cache[key] = found;
+}
+
+// host evaluation of requant_pack4 for one output
+static int pack_eval(int a, int act, const RequantPack& q) {
+    float x = (float)a;
+    if (q.mode == 2)
+        x = x * q.s1 * q.s2;
+    const float r = rintf(fmaf(x, q.c, q.d));  // (round to nearest even: the host's default mode)
+    const int u = r < 0.f ? 0 : r > 255.f ? 255 : (int)r;
+    return act == MEGCC_NONLINE_RELU ? u >> 1 : u - 128;
+}
+
+RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
+    static std::mutex lock;
+    static std::map<std::tuple<int, uint32_t, uint32_t, uint32_t>, RequantPack> cache;
+    const RequantPack none = {0.f, 0.f, 0.f, 0.f, 0};
+    if ((act != MEGCC_NONLINE_IDENTITY && act != MEGCC_NONLINE_RELU) || !requant_table_ok(s_src, s_flt, s_dst) ||
+        options().no_affine)
+        return none;
+    auto bits = [](float f) {
+        uint32_t u;
+        memcpy(&u, &f, 4);
+        return u;
+    };
+    const auto key = std::make_tuple(act, bits(s_src), bits(s_flt), bits(s_dst));
+    {
+        std::lock_guard<std::mutex> guard(lock);
+        auto it = cache.find(key);
+        if (it != cache.end())
+            return it->second;
+    }
+    const RequantTable& T = requant_table_for(act, s_src, s_flt, s_dst);
+    const bool relu = act == MEGCC_NONLINE_RELU;
+    auto literal = [&](int a) {
+        return relu ? requant_conv<MEGCC_NONLINE_RELU>(a, s_src, s_flt, s_dst)
+                    : requant_conv<MEGCC_NONLINE_IDENTITY>(a, s_src, s_flt, s_dst);
+    };
+    // both sides of every step of F, and the ends of the accumulator range
+    struct Point {
+        int a, y;
+    };
+    std::vector<Point> pts;
+    pts.push_back({INT32_MIN, literal(INT32_MIN)});
+    pts.push_back({INT32_MAX, literal(INT32_MAX)});
+    for (int i = 0; i < REQUANT_TABLE_ENTRIES - 1; ++i) {
+        const int t = T.t[i];
+        if (t == INT32_MIN)
+            continue;  // F never drops below this level
+        pts.push_back({t, literal(t)});
+        if (t < INT32_MAX)
+            pts.push_back({t + 1, literal(t + 1)});
+    }
+    // the forms in order of cost: no product in front, one, two
+    struct Form {
+        int mode;
+        float s1, s2, c0;
+    };
+    const float unit = relu ? 2.f : 1.f;
+    const Form forms[] = {{1, 1.f, 1.f, make_requant_fast(s_src, s_flt, s_dst).c * unit},
+                          {2, s_src, 1.f, s_flt / s_dst * unit},
+                          {2, s_src, s_flt, 1.f / s_dst * unit}};
+    RequantPack found = none;
+    std::vector<float> x(pts.size());
+    for (const Form& f : forms) {
+        for (size_t i = 0; i < pts.size(); ++i)
+            x[i] = f.mode == 2 ? (float)pts[i].a * f.s1 * f.s2 : (float)pts[i].a;
+        for (int k = 0; k <= 48 && !found.mode; ++k) {
+            // c = c0 moved (k + 1) / 2 ulps up (k odd) or down (k even)
+            float c = f.c0;
+            for (int s = 0; s < (k + 1) / 2; ++s)
+                c = nextafterf(c, (k & 1) ? INFINITY : 0.f);
+            double dlo = -1e30, dhi = 1e30;
+            for (size_t i = 0; i < pts.size(); ++i) {
+                const double prod = (double)x[i] * (double)c;
+                const int y = pts[i].y;
+                // RELU: 2 y <= rint <= 2 y + 1; IDENTITY: rint == y + 128
+                const double lo = relu ? 2.0 * y - 0.5 : y + 127.5, hi = relu ? 2.0 * y + 1.5 : y + 128.5;
+                if (y > (relu ? 0 : -128) && lo - prod > dlo)
+                    dlo = lo - prod;
+                if (y < 127 && hi - prod < dhi)
+                    dhi = hi - prod;
+            }
+            if (!(dlo <= dhi))
+                continue;
+            static const double kPos[] = {0.5, 0.375, 0.625, 0.25, 0.75, 0.125, 0.875};
+            for (double pos : kPos) {
+                const RequantPack q = {f.s1, f.s2, c, (float)(dlo + (dhi - dlo) * pos), f.mode};
+                bool ok = true;
+                for (size_t i = 0; i < pts.size() && ok; ++i)
+                    ok = pack_eval(pts[i].a, act, q) == pts[i].y;
+                if (ok) {
+                    found = q;
+                    break;
+                }
+            }
+        }
+        if (found.mode)
+            break;
+    }
+    std::lock_guard<std::mutex> guard(lock);
+    if (cache.size() >= 4096)
+        cache.clear();
     return cache[key] = found;
 }
 

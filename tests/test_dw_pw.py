@@ -1,0 +1,71 @@
+"""A channel-wise 3x3 convolution and the pointwise 1x1 convolution of its result as one kernel (the model
+runtime's conv_dw_pw), against the oracle's two convolutions run one after the other, bit for bit."""
+import numpy as np
+import pytest
+
+from cases import ConvCase
+from megcc_amd import abi, runtime
+from megcc_amd import abi as A
+from oracle import port
+
+pytestmark = pytest.mark.gpu
+
+TIES = (0.02, 0.01, 0.05)            # exact ties: both layers requantise by table
+GENERIC = (0.0213, 0.0097, 0.0371)
+
+PAIRS = [
+    # (n, c, oc, h, w, stride, pointwise act, scales): every channel count with a kernel of its own at the extents of
+    # MobileNets, then rows whose last group of 4 pixels hangs over by 1, 2, 3, tiles that cross images, fewer
+    # pixels than a tile, one row, output channels that leave part of the last slice empty
+    (1, 32, 64, 112, 112, 1, A.RELU, GENERIC), (1, 64, 128, 112, 112, 2, A.RELU, TIES),
+    (2, 128, 128, 56, 56, 1, A.RELU, GENERIC), (2, 128, 256, 56, 56, 2, A.RELU, GENERIC),
+    (3, 256, 256, 28, 28, 1, A.RELU, TIES), (3, 256, 512, 28, 28, 2, A.RELU, GENERIC),
+    (5, 512, 512, 14, 14, 1, A.RELU, GENERIC), (5, 512, 1024, 14, 14, 2, A.RELU, TIES),
+    (7, 1024, 1024, 7, 7, 1, A.RELU, GENERIC), (64, 512, 512, 14, 14, 1, A.RELU, GENERIC),
+    (2, 32, 64, 9, 5, 1, A.IDENTITY, TIES), (2, 32, 96, 6, 13, 2, A.RELU, GENERIC), (3, 64, 160, 5, 7, 1, A.RELU, GENERIC),
+    (3, 64, 32, 7, 6, 2, A.IDENTITY, GENERIC), (1, 128, 64, 1, 3, 1, A.RELU, TIES), (2, 128, 160, 11, 9, 2, A.RELU, GENERIC),
+    (1, 256, 96, 2, 2, 1, A.IDENTITY, GENERIC), (2, 256, 320, 10, 15, 2, A.RELU, TIES), (1, 512, 544, 3, 31, 1, A.RELU, GENERIC),
+    (1, 1024, 64, 4, 5, 2, A.RELU, TIES), (1, 1024, 1056, 5, 6, 1, A.IDENTITY, GENERIC), (40, 32, 64, 33, 17, 1, A.RELU, TIES),
+]
+
+
+@pytest.mark.parametrize("cfg", PAIRS, ids=lambda c: "n%d_c%d_oc%d_%dx%d_s%d_a%d_%s" % (c[:7] + ("ties" if c[7] is TIES else "gen",)))
+def test_pair_in_one_kernel(cfg):
+    n, c, oc, h, w, stride, act, scales = cfg
+    port.set_threads(8)
+    dw = ConvCase(A.FMT_NCHW44, A.GROUP, n, c, h, w, c, 3, stride, 1, A.RELU, scales=scales, flt_range=(-30, 30))
+    s2 = (scales[2], scales[1], scales[2] if scales is TIES else scales[2] * scales[1] * 4.0e3 * c ** 0.5 / 36.0)
+    pw = ConvCase(A.FMT_NCHW44, A.DENSE, n, c, dw.oh, dw.ow, oc, 1, 1, 0, act, scales=s2)
+    a0, a1 = dw.gen(51), pw.gen(52)
+    a1["src"] = dw.run_port(a0)
+    want = pw.run_port(a1)
+    assert len(np.unique(want)) > 20
+    bias_scale = lambda k: float(np.float32(k.scales[0]) * np.float32(k.scales[1]))
+    for fused in (True, False):
+        runtime.set_option("fusedwpw", int(fused))
+        runtime.set_option("nofusedwpw", int(not fused))
+        try:
+            m = runtime.Model()
+            x = m.tensor("x", dw.src_shape(), abi.QINT8, dw.scales[0])
+            m.mark_input(x)
+            t = x
+            for k, case, arrays in (("dw", dw, a0), ("pw", pw, a1)):
+                y = m.tensor(k, case.dst_shape(), abi.QINT8, case.scales[2])
+                m.opr(case.symbol(), [t, m.weight(k + ".w", arrays["flt"], abi.QINT8, case.scales[1]),
+                                      m.weight(k + ".b", arrays["bias"], abi.QINT32, bias_scale(case))], [y])
+                t = y
+            m.mark_output(t)
+            m.finalize()
+        finally:
+            runtime.set_option("fusedwpw", 0)
+            runtime.set_option("nofusedwpw", 0)
+        assert m.nr_kernel == (1 if fused else 2)
+        m.set_input(x, a0["src"])
+        for _ in range(2):
+            m.forward()
+        got = m.get(t)
+        print(runtime.last_kernel())
+        assert runtime.last_kernel().startswith("conv_dw_pw") == fused, runtime.last_kernel()
+        bad = int((got != want).sum())
+        assert bad == 0, "%s: %d of %d differ" % ("one kernel" if fused else "two kernels", bad, got.size)
+        m.close()
