@@ -21,6 +21,7 @@
 #include "epilogue.h"
 #ifndef MG_HOST_AUDIT  // (a host build that runs this file's own kernels thread by thread)
 #include "gemm_f32_ks.h"
+#include "gemm_f32_split.h"
 #endif
 
 namespace mg {
@@ -583,6 +584,8 @@ extern "C" TinyNNStatus megcc_gfx950_matmul(
     }
 #ifndef MG_HOST_AUDIT
     const GevmArgs ks = {q.A, q.B, q.C, q.M, q.N, q.K, q.a_rs, q.a_cs, q.b_rs, q.b_cs, q.ldc};
+    if (gemm_f32_split_supported(ks))
+        return gemm_f32_split_launch(ks, ta, tb);
     if (gemm_f32_ks_supported(ks))
         return gemm_f32_ks_launch(ks, ta, tb);
 #endif

@@ -6,6 +6,8 @@
 
 namespace mg {
 
+// estimated cycles of the busiest CU
+double gemm_f32_ks_cycles(const GevmArgs& v);
 bool gemm_f32_ks_supported(const GevmArgs& v);
 TinyNNStatus gemm_f32_ks_launch(const GevmArgs& v, int ta, int tb);
 bool conv_f32_ks_supported(const ConvGeom& g);

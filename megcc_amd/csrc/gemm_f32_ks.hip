@@ -370,6 +370,10 @@ static KsPlan conv_plan(const ConvGeom& g) {
     return ks_plan(g.oc, (long)g.n * g.oh * g.ow, (long)g.ic * g.fh * g.fw, true, false, true);
 }
 
+double gemm_f32_ks_cycles(const GevmArgs& v) {
+    return matmul_plan(v).cost;
+}
+
 bool gemm_f32_ks_supported(const GevmArgs& v) {
     const long as = 4 * ((long)(v.M - 1) * v.a_rs + (long)(v.K - 1) * v.a_cs + 1);
     const long bs = 4 * ((long)(v.K - 1) * v.b_rs + (long)(v.N - 1) * v.b_cs + 1);

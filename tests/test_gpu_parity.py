@@ -403,6 +403,57 @@ def test_f32_products_whose_waves_share_k(case):
     compare(got, case.run_port(arrays), repr(case))
 
 
+def _product(case, arrays):
+    """the product in 64 bits"""
+    a, b = (arrays[k].astype(np.float64) for k in ("a", "b"))
+    return (a.T if case.trans_a else a) @ (b.T if case.trans_b else b)
+
+
+F32_SPLIT = [MatMulCase(m, k, n, trans_a=ta, trans_b=tb)
+             # rows and columns beyond whole tiles; K of two stages, of a chain of eight and around it, with and without a rest,
+             # either side of the 512 where the small products get a sum of their own
+             for m, k, n in ((2900, 33, 3001), (2900, 145, 3001), (2040, 512, 1999), (1930, 531, 1925))
+             for ta in (False, True) for tb in (False, True)]
+
+
+@pytest.mark.parametrize("case", F32_SPLIT, ids=[repr(c) for c in F32_SPLIT])
+def test_f32_product_on_the_bf16_instructions(case):
+    """as accurate as f32: K roundings of 2^-24 of the magnitudes' sum bound an f32 sum in any order; three parts of 8
+    bits (and the products that are left out: 2^-25) stay inside it"""
+    arrays = case.gen(seed=23)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().startswith("gemm_f32_split"), runtime.last_kernel()
+    bound = _product(case, {k: np.abs(v) for k, v in arrays.items()}) * (case.k * 2.0 ** -24)
+    assert np.all(np.abs(got - _product(case, arrays)) <= bound)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3e38, 2.0 ** 60, 1e-38, 2.0 ** -103, 0.0])
+@pytest.mark.parametrize("k", [112, 600])
+def test_f32_product_of_values_bf16_parts_cannot_hold(k, value):
+    """a row of A and a column of B at the value: the tiles that meet them come out as of an f32 product, all others
+    as without them"""
+    case = MatMulCase(2560, k, 2560)
+    arrays = case.gen(seed=29)
+    plain = run_gpu(case, arrays)
+    arrays["a"][130, 5:] = value
+    arrays["b"][7:, 1000] = value
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().startswith("gemm_f32_split"), runtime.last_kernel()
+    rows, cols = np.arange(2560) != 130, np.arange(2560) != 1000
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = _product(case, arrays)
+        bound = _product(case, {n: np.abs(v) for n, v in arrays.items()}) * k * (2.0 ** -24) + k * 2.0 ** -126  # (and underflow)
+        for part in ((130, cols), (rows, 1000), (130, 1000)):
+            g, w, b = got[part], want[part], bound[part]
+            # (sums near the end of the f32 range may leave it on the way)
+            inside = np.isfinite(w) & (b * 2.0 ** 24 < 2.0 ** 127)
+            assert np.all(np.abs(g - w)[inside] <= b[inside])
+            if not np.isfinite(value):
+                assert np.array_equal(np.isnan(g), np.isnan(w)) and np.array_equal(g[np.isinf(w)], w[np.isinf(w)])
+    far = (np.arange(2560) // 128 != 130 // 128)[:, None] & (np.arange(2560) // 128 != 1000 // 128)[None]
+    assert np.array_equal(got[far], plain[far])
+
+
 F32_NCHW44 = [
     # f32 channel-wise layers in NCHW44 (the reference's GI_chanwise kernels: 3x3 / 5x5, stride 1 / 2):
     # tiles of 4 x 64 pixels - extents below, at and above a tile, padding 0 .. k/2 + 1, every activation
