@@ -1,6 +1,6 @@
 // Dense qsi8 NCHW44 convolution of any filter size, stride and dilation on the 4-way int8 dot
-// product (v_dot4_i32_i8): the implementation of what the matrix-core kernels do not take - more
-// than 9 taps (5x5, 7x7), or a filter that did not go through the init step. Same loop nest and
+// product (v_dot4_i32_i8): the implementation for a filter that did not go through the init step (the
+// matrix-core kernels read a packed one). Same loop nest and
 // epilogue as BareMetal/ConvKernel.cpp:305-344,374-380 on src [N,C/4,H,W,4] and filter
 // [OC/4,IC/4,FH,FW,4 ic,4 oc] (:58-64,95-99).
 //   * a thread owns one output pixel x OCB groups of 4 output channels; a pixel's 4 input channels

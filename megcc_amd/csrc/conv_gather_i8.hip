@@ -1,0 +1,303 @@
+// qsi8 dense NCHW44 convolution of any filter size, stride and dilation on the matrix cores
+// (v_mfma_i32_32x32x32_i8) without staging: for the layers the LDS-direct kernel (conv_mfma_i8_dma.hip) has no
+// variant for or leaves part of the chip idle on.
+//
+// What bounded those layers was the one-stage kernel's chain - gather a stage, barrier, multiply it with nothing in
+// flight - on a handful of 128-pixel tiles, and for more than 9 taps the dot-product kernel's 12 vector instructions
+// per 16 multiply-adds. Here nothing goes through LDS on the way in:
+//   * a step is one tap of 32 input channels = one MFMA per 32 x 32 outputs. The filter operand of 32 channels is one
+//     contiguous KB of the packed filter; the activation operand of 32 pixels is four dwords per lane, pixel = lane,
+//     32 lanes on consecutive pixels of one channel group's plane;
+//   * a tap outside the image turns the lane's offset into one beyond the tensor, which a buffer load answers with
+//     zero; channel groups beyond the last meet zero filter rows, and offsets beyond the tensor read zero too. Steps
+//     beyond a wave's share read zero the same way, so no load is under a condition. The whole offset is in the
+//     lane's register: the range check sees all of it;
+//   * RING steps are in flight per wave;
+//   * the waves of a workgroup share K (KW groups) and the pixels (the rest): small layers split K so that every CU
+//     has work; the groups' int32 sums meet in LDS, each group finishing its share of the tile.
+// Bound by the loads' way through the CU's address and data path (64 x 64 outputs a wave: 64 cycles of it a step for
+// 32 of its matrix units) on large layers and by the chain of steps of one wave on small ones. Measured (us, before:
+// the one-stage kernel of conv_mfma_i8.hip, beyond 9 taps conv_dot4.hip): 6 x 88 -> 148 57 x 43 stride 2 14.6 -> 7.1, 4 x
+// 24 -> 68 98 x 98 stride 2 14.8 -> 5.7, 1 x 356 -> 52 68 x 81 21.2 -> 8.5, 1 x 256 -> 256 28 x 28 8.0 -> 5.7, 47 x 104 -> 48 89 x 89 95.8 -> 51.2, 58 x
+// 264 -> 320 70 x 70 stride 2 216 -> 183; 5x5: 1 x 120 -> 280 19 x 19 134 -> 6.7, 60 x 28 -> 20 63 x 63 137 -> 21.7.
+// Reference loop: BareMetal/ConvKernel.cpp:305-344.
+#include "conv_mfma_i8.h"
+
+namespace mg {
+
+struct GatherParams {
+    const int8_t* src;
+    const int8_t* wp;     // packed filter [chunk][tap][OCP][32], 16-byte halves swapped when (oc >> 3) & 1
+    const int32_t* bias;  // [OC] or NULL
+    int8_t* dst;
+    unsigned src_bytes, wp_bytes;
+    int P, OC, steps, taps, kw;  // steps = chunks * taps
+    unsigned step_bytes;         // of the packed filter
+    unsigned plane, image, row;  // bytes of the source
+    int IH, IW, OHW, OW, FW, SH, SW, PH, PW, DH, DW;
+    FastDiv dOHW, dOW, dTaps, dFW;
+    int act;
+    float s_src, s_flt, s_dst;
+    float c, aff_c, aff_d;  // scale of the table's estimate; the fused multiply-add (aff_d 0: none, the table)
+    RequantTable table;
+};
+
+// Entry i of the table, straight from the kernel-argument segment (conv_mfma_i8.h: kernarg_rq_table)
+__device__ __forceinline__ int gather_table(int i) {
+    typedef const __attribute__((address_space(4))) char* kptr;
+    const kptr base = (kptr)__builtin_amdgcn_kernarg_segment_ptr();
+    return *(const __attribute__((address_space(4))) int*)(base + offsetof(GatherParams, table) + 4 * i);
+}
+
+// ACT: an activation whose outputs the threshold table describes, or -1 (the literal sequence of q.act)
+static constexpr int GATHER_WAVES = 4;  // of a workgroup
+
+template <int MT, int NT, int ACT>
+__global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(GatherParams q) {
+    constexpr int RING = 4;
+    extern __shared__ __attribute__((aligned(16))) int gather_lds[];
+    if (ACT >= 0) {
+        if (threadIdx.x < REQUANT_TABLE_ENTRIES)
+            gather_lds[threadIdx.x] = gather_table(threadIdx.x);
+        __syncthreads();
+    }
+    int* const parts = gather_lds + REQUANT_TABLE_ENTRIES;
+    const int lane = threadIdx.x & 63, col = lane & 31, kg = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int kw = q.kw, pw = waves / kw;           // groups that share K, waves side by side in pixels
+    const int grp = wave / pw, sub = wave - grp * pw;
+    const int oc0 = blockIdx.y * (32 * MT), p0 = (blockIdx.x * pw + sub) * (32 * NT);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)q.src, 0, (int)q.src_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)q.wp, 0, (int)q.wp_bytes, 0x00020000);
+
+    unsigned pix[NT];
+    int ih0[NT], iw0[NT], img[NT], rem[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int p = min(p0 + 32 * j + col, q.P - 1);
+        img[j] = (int)fdiv(p, q.dOHW);
+        rem[j] = p - img[j] * q.OHW;
+        const int oh = (int)fdiv(rem[j], q.dOW), ow = rem[j] - oh * q.OW;
+        ih0[j] = oh * q.SH - q.PH;
+        iw0[j] = ow * q.SW - q.PW;
+        pix[j] = (unsigned)img[j] * q.image + (unsigned)kg * 4u * q.plane + (unsigned)ih0[j] * q.row + (unsigned)iw0[j] * 4u;
+    }
+    unsigned aoff[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int oc = oc0 + 32 * i + col;  // (below OCP, a multiple of every tile height)
+        aoff[i] = (unsigned)oc * KROW + (((kg ^ (oc >> 3)) & 1) << 4);
+    }
+    v4i A[RING][MT], B[RING][NT];
+    auto load = [&](int s, v4i (&a)[MT], v4i (&b)[NT]) __attribute__((always_inline)) {
+        const bool over = s >= q.steps;
+        const int sc = over ? q.steps - 1 : s;
+        const int chunk = (int)fdiv(sc, q.dTaps), tap = sc - chunk * q.taps;
+        const int fh = (int)fdiv(tap, q.dFW), fw = tap - fh * q.FW;
+        const int dy = fh * q.DH, dx = fw * q.DW;
+        const unsigned off = (unsigned)chunk * 8u * q.plane + (unsigned)dy * q.row + (unsigned)dx * 4u;
+        const int bottom = over ? 0 : q.IH;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            a[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(aoff[i] + (unsigned)sc * q.step_bytes), 0, 0));
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const bool in = (unsigned)(ih0[j] + dy) < (unsigned)bottom && (unsigned)(iw0[j] + dx) < (unsigned)q.IW;
+            const unsigned o = in ? pix[j] + off : 0x80000000u;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                b[j][c] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)(o + (unsigned)c * q.plane), 0, 0);
+        }
+    };
+    v16i acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                acc[i][j][e] = 0;
+    // group g takes steps g, g + kw, ...
+    const int mine = (q.steps - grp + kw - 1) / kw;
+#pragma unroll
+    for (int r = 0; r < RING; ++r)
+        load(grp + r * kw, A[r], B[r]);
+    for (int t = 0; t < mine; t += RING) {
+#pragma unroll
+        for (int r = 0; r < RING; ++r) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[r][i], B[r][j], acc[i][j], 0, 0, 0);
+            load(grp + (t + r + RING) * kw, A[r], B[r]);
+        }
+    }
+    // [group][wave of it][quad][lane]: a quad is 4 neighbouring channels of the lane's pixel
+    constexpr int QUADS = MT * NT * 4;
+    if (kw > 1) {
+#pragma unroll
+        for (int x = 0; x < QUADS; ++x)
+            if ((x & (kw - 1)) != grp) {
+                const v16i& t = acc[x / (NT * 4)][x / 4 % NT];
+                *(v4i*)(parts + ((wave * QUADS + x) * 64 + lane) * 4) =
+                        v4i{t[x % 4 * 4], t[x % 4 * 4 + 1], t[x % 4 * 4 + 2], t[x % 4 * 4 + 3]};
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int x = 0; x < QUADS; ++x) {
+        if ((x & (kw - 1)) != grp)
+            continue;
+        const int i = x / (NT * 4), j = x / 4 % NT, e4 = x % 4;
+        int s[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            s[e] = acc[i][j][e4 * 4 + e];
+        for (int g = 0; g < kw; ++g) {
+            if (g == grp)
+                continue;
+            const v4i o = *(const v4i*)(parts + (((g * pw + sub) * QUADS + x) * 64 + lane) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s[e] += o[e];
+        }
+        const int oc = oc0 + 32 * i + 8 * e4 + 4 * kg;
+        // (the bias of a lane without an output: some other channel's)
+        int bv[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            bv[e] = q.bias ? q.bias[min(oc, q.OC - 4) + e] : 0;
+        if (oc >= q.OC || p0 + 32 * j + col >= q.P)
+            continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            s[e] += bv[e];
+        int r[4];
+        if constexpr (ACT == MEGCC_NONLINE_IDENTITY || ACT == MEGCC_NONLINE_RELU) {
+            if (q.aff_d != 0.f) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    r[e] = requant_conv_affine<ACT>(s[e], q.aff_c, q.aff_d);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    r[e] = requant_conv_table<ACT>(s[e], q.c, gather_lds);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (ACT < 0)
+                    r[e] = requant_conv_rt(q.act, s[e], q.s_src, q.s_flt, q.s_dst);
+                else
+                    r[e] = requant_conv_table<ACT>(s[e], q.c, gather_lds);
+            }
+        }
+        ((uint32_t*)q.dst)[((size_t)img[j] * (q.OC >> 2) + (oc >> 2)) * q.OHW + rem[j]] = pack4_perm(r[0], r[1], r[2], r[3]);
+    }
+}
+
+size_t conv_mfma_packed_bytes(const ConvGeom& g);
+
+bool conv_gather_i8_supported(const ConvGeom& g) {
+    const long P = (long)g.n * g.oh * g.ow, src = (long)g.n * g.ic * g.ih * g.iw;
+    return g.fmt == MEGCC_FMT_NCHW44 && g.groups == 1 && (g.ic & 3) == 0 && (g.oc & 3) == 0 && g.ic >= 4 && g.oc >= 4 &&
+           g.fh >= 1 && g.fw >= 1 && P >= 1 && P < (1L << 31) - 512 && src < (1L << 31) &&
+           // offsets before the first pixel and behind the last stay clear of the tensor's when they wrap
+           (long)g.ih * g.iw * 4 * 12 < (1L << 31) && (long)g.fh * g.dh < (1L << 20) && (long)g.fw * g.dw < (1L << 20) &&
+           (long)conv_mfma_packed_bytes(g) < (1L << 31) - 65536 && (long)((g.ic + 31) / 32) * g.fh * g.fw < (1L << 22) &&
+           (g.oc + 31) / 32 < 65536;
+}
+
+// The layers this kernel takes from the LDS-direct one (its variant `picked`). Measured over 3x3 and 5x5 layers of
+// 32 .. 512 channels, 7 x 7 .. 56 x 56, batch 1 .. 32 (us there / here):
+//   * the small-layer variants 6 and 7, one 32-channel tile a workgroup: when there is less than a 32 x 32 tile for
+//     every CU, and K is long enough to share (256 -> 256 28 x 28 8.0 / 5.6, 128 -> 128
+//     28 x 28 5.5 / 4.8; with 64 channels 4.7 / 4.7, with two tiles a CU 8.2 / 11.0);
+//   * the variants 8 and 9, a filter row a stage: when the tiles leave SIMDs without one (128 -> 128 28 x 28 N=8 20.2 /
+//     14.6, 64 -> 64 28 x 28 N=16 10.1 / 9.6; with more, 20.3 / 24.2), 9 when there are half as many (164 -> 60 18 x 17
+//     stride 2 N=56 29.2 / 21.9, 64 -> 64 56 x 56 stride 2 N=16 12.5 / 13.3). Layers of 48 channels and fewer would gain
+//     too (32 -> 32 28 x 28 N=16 6.9 / 5.1) but are what the row-split kernel is tested with.
+bool conv_gather_i8_wins(const ConvGeom& g, int picked) {
+    const long tiles = (((long)g.n * g.oh * g.ow + 31) / 32) * ((g.oc + 31) / 32);
+    if (picked == 6 || picked == 7)
+        return tiles < num_cus() && (long)((g.ic + 31) / 32) * g.fh * g.fw >= 36;
+    return (picked == 8 || picked == 9) && g.ic > 48 && tiles < (picked == 8 ? 4L : 2L) * num_cus();
+}
+
+TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const void* packed, const void* bias, void* dst) {
+    GatherParams q = {};
+    q.src = (const int8_t*)src;
+    q.wp = (const int8_t*)packed;
+    q.bias = (const int32_t*)bias;
+    q.dst = (int8_t*)dst;
+    q.src_bytes = (unsigned)((long)g.n * g.ic * g.ih * g.iw);
+    q.wp_bytes = (unsigned)conv_mfma_packed_bytes(g);
+    q.OHW = g.oh * g.ow;
+    q.OW = g.ow;
+    q.P = g.n * q.OHW;
+    q.OC = g.oc;
+    q.taps = g.fh * g.fw;
+    q.steps = (g.ic + 31) / 32 * q.taps;
+    q.step_bytes = (unsigned)((g.oc + OC_PAD - 1) / OC_PAD * OC_PAD * KROW);
+    q.plane = (unsigned)(g.ih * g.iw) * 4u;
+    q.image = (unsigned)(g.ic / 4) * q.plane;
+    q.row = (unsigned)g.iw * 4u;
+    q.IH = g.ih, q.IW = g.iw, q.FW = g.fw;
+    q.SH = g.sh, q.SW = g.sw, q.PH = g.ph, q.PW = g.pw, q.DH = g.dh, q.DW = g.dw;
+    q.dOHW = make_fastdiv(q.OHW);
+    q.dOW = make_fastdiv(g.ow);
+    q.dTaps = make_fastdiv(q.taps);
+    q.dFW = make_fastdiv(g.fw);
+    q.act = g.act;
+    q.s_src = g.s_src;
+    q.s_flt = g.s_flt;
+    q.s_dst = g.s_dst;
+    q.c = make_requant_fast(g.s_src, g.s_flt, g.s_dst).c;
+    const bool table = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
+    if (table)
+        q.table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+    // 64 x 64 outputs a wave where that gives every SIMD one, else less. 32 x 32: four groups share a long K however many
+    // tiles there are (7 x 124 -> 240 29 x 23 11.4 us with one, 10.4 with four; 256 -> 256 28 x 28 5.6 with four, 6.0
+    // with eight), a shorter one while SIMDs are idle (24 x 56 -> 16 66 x 66 stride 2 6.9 with two, 7.3 with four; 3 x 20 ->
+    // 404 42 x 32 6.5 with one, 7.9 with four). 64 x 64: two share a long K where a SIMD has under four waves, to
+    // even out the last round (10 x 452 -> 108 75 x 91 77.5 with one, 68.1 with two).
+    int mt = g.oc > 32 ? 2 : 1, nt = 2, kw = 1;
+    const long full = 4L * num_cus();
+    auto tiles = [&] { return (long)((q.P + 32 * nt - 1) / (32 * nt)) * ((g.oc + 32 * mt - 1) / (32 * mt)); };
+    if (tiles() < full)
+        nt = 1;
+    if (tiles() < full)
+        mt = 1;
+    if (mt * nt == 1) {
+        while (kw < 4 && q.steps >= 8 * kw && (tiles() * kw < full || q.steps >= 27))
+            kw *= 2;
+    } else if (mt * nt == 4 && q.steps >= 72 && tiles() < 4 * full) {
+        kw = 2;
+    }
+    constexpr int waves = GATHER_WAVES;
+#define MG_GATHER_A(MT_, NT_)                                                                          \
+    (!table                              ? conv_gather_i8_kernel<MT_, NT_, -1>                         \
+     : g.act == MEGCC_NONLINE_IDENTITY   ? conv_gather_i8_kernel<MT_, NT_, MEGCC_NONLINE_IDENTITY>     \
+     : g.act == MEGCC_NONLINE_RELU       ? conv_gather_i8_kernel<MT_, NT_, MEGCC_NONLINE_RELU>         \
+                                         : conv_gather_i8_kernel<MT_, NT_, MEGCC_NONLINE_H_SWISH>)
+    void (*kern)(GatherParams) = mt == 2 ? (nt == 2 ? MG_GATHER_A(2, 2) : MG_GATHER_A(2, 1))
+                                         : (nt == 2 ? MG_GATHER_A(1, 2) : MG_GATHER_A(1, 1));
+#undef MG_GATHER_A
+    const int pw = waves / kw;
+    const dim3 grid((unsigned)((q.P + 32 * nt * pw - 1) / (32 * nt * pw)), (unsigned)((g.oc + 32 * mt - 1) / (32 * mt)));
+    q.kw = kw;
+    note_kernel("conv_mfma_i8_gather", 32 * mt, 32 * nt, kw);
+    const RequantAffine aff = requant_affine_pick(table, g.act, g.s_src, g.s_flt, g.s_dst);
+    q.aff_c = aff.c;
+    q.aff_d = aff.d;
+    const size_t lds = REQUANT_TABLE_ENTRIES * 4 + (kw > 1 ? (size_t)waves * mt * nt * 4096 : 0);
+    if (lds > 48 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_gather_i8: LDS attribute: %s", hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(kern, grid, dim3(64 * waves), lds, stream(), q);
+    return check_launch("conv_gather_i8");
+}
+
+}  // namespace mg

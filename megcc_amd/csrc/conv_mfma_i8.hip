@@ -326,6 +326,8 @@ static int conv_mfma_split(const ConvGeom& g) {
 size_t conv_mfma_workspace_bytes(const ConvGeom& g) {
     if (g.fmt == MEGCC_FMT_NCHW && (g.ic & 3))
         return 0;  // (fc_any_k: no partial sums in memory)
+    if (g.fh * g.fw > MAX_TAPS_STAGE)
+        return 0;  // (no kernel of theirs splits K over workgroups)
     const int s = conv_mfma_split(g);
     const long P = (long)g.n * g.oh * g.ow;
     return s > 1 ? (size_t)s * P * ((g.oc + 3) & ~3) * sizeof(int32_t) : 0;
@@ -445,6 +447,8 @@ static bool fc_any_k(const ConvGeom& g) {
     return fc_gevm_q8_supported(g) || fc_tile_supported(g);
 }
 
+bool conv_gather_i8_supported(const ConvGeom& g);
+
 bool conv_mfma_supported(const ConvGeom& g) {
     if (g.groups != 1)
         return false;
@@ -458,8 +462,10 @@ bool conv_mfma_supported(const ConvGeom& g) {
     if (g.fmt == MEGCC_FMT_NCHW44 && (g.oc & 3))
         return false;
     if (g.fh * g.fw > MAX_TAPS_STAGE) {
-        // only the row-split variants of the LDS-direct kernel (no one-stage fallback: that kernel
-        // keeps every tap of a chunk in LDS and registers)
+        if (conv_gather_i8_supported(g))
+            return true;
+        // otherwise only the row-split variants of the LDS-direct kernel (no one-stage fallback: that
+        // kernel keeps every tap of a chunk in LDS and registers)
         PipeConfig pc;
         TilePlan t;
         long range_len = 0;
@@ -585,6 +591,10 @@ static bool pick_dma(const ConvGeom& g, bool b128_ok, PipeConfig* pc, TilePlan* 
     return pipe;
 }
 
+bool conv_gather_i8_wins(const ConvGeom& g, int picked);
+TinyNNStatus conv_gather_i8_launch(
+        const ConvGeom& g, const void* src, const void* packed, const void* bias, void* dst);
+
 TinyNNStatus conv_mfma_launch(
         const ConvGeom& g, const void* src, const void* packed, const void* bias, void* dst,
         const Workspace* ws) {
@@ -616,6 +626,11 @@ TinyNNStatus conv_mfma_launch(
     TilePlan t;
     int picked = -1;  // variant of the LDS-direct kernel
     const bool pipe = pick_dma(g, b128_ok, &pc, &t, &range_len, &picked);
+    // what no variant takes ran on the one-stage kernel below or, beyond 9 taps, on conv_dot4.hip: operands
+    // straight to registers are 1.2 to 30 times as fast on every layer measured
+    if ((!pipe || conv_gather_i8_wins(g, picked)) && conv_gather_i8_supported(g) &&
+        (!options().no_small || g.fh * g.fw > MAX_TAPS_STAGE))
+        return conv_gather_i8_launch(g, src, packed, bias, dst);  // (notes its own variant)
     // FullyConnected: the LDS-direct kernel's 256 x 256 tiles win from half a chip of them on (2048 x 4096
     // x 4096, 128 tiles: 43.7 us against 46.6; 4096 x 2048 x 1024, 64 tiles: 21.5 against 21.2; 2048 x 1024
     // x 1000, 32 tiles: 14.8 against 8.6; 200 x 1024 x 1000: 13.0 on the one-stage kernel against 6.6)

@@ -454,6 +454,37 @@ def test_f32_product_of_values_bf16_parts_cannot_hold(k, value):
     assert np.array_equal(got[far], plain[far])
 
 
+def _gather_cases():
+    def c(n, ic, ih, iw, oc, k, s, pad, act=A.RELU, **kw):
+        return ConvCase(A.FMT_NCHW44, A.DENSE, n, ic, ih, iw, oc, k, s, pad, act, **kw,
+                        scales=(0.02, 0.01, unsat(ic * k * k) * (40 if act == A.SIGMOID else 1)))
+    return [
+        # channels below, at and beyond a chunk of 32, pixels that are no whole tiles, padding 0 .. k, every activation
+        c(1, 4, 5, 6, 4, 3, 2, 1), c(3, 36, 13, 9, 36, 3, 2, 0, A.IDENTITY), c(2, 20, 11, 17, 68, 3, 2, 3, A.H_SWISH),
+        c(2, 52, 19, 14, 32, 3, 2, 1, A.SIGMOID), c(1, 8, 9, 9, 12, 3, 1, 2, bias=False, dilate=2),
+        # more than 9 taps
+        c(1, 4, 7, 7, 8, 5, 1, 2), c(2, 100, 19, 23, 44, 5, 2, 2, A.IDENTITY), c(1, 24, 15, 12, 28, 7, 1, 6, A.H_SWISH),
+        c(1, 64, 9, 8, 64, 5, 1, 4, dilate=2),
+        # K shared by 1 .. 4 waves: few tiles and a long K, many tiles and a short one
+        c(1, 512, 7, 7, 64, 3, 1, 1), c(1, 256, 28, 28, 256, 3, 1, 1), c(6, 88, 57, 43, 148, 3, 2, 1),
+        c(5, 132, 39, 40, 260, 3, 2, 1, A.H_SWISH),
+        # 64 outputs a wave in pixels, in channels, in both
+        c(20, 16, 63, 63, 20, 5, 1, 2), c(1, 20, 99, 106, 220, 3, 1, 2, dilate=2), c(21, 24, 111, 113, 72, 3, 2, 1, A.IDENTITY),
+    ]
+
+
+GATHER = _gather_cases()
+
+
+@pytest.mark.parametrize("case", GATHER, ids=[repr(c) for c in GATHER])
+def test_dense_layers_without_staging(case):
+    port.set_threads(16)
+    arrays = case.gen(seed=37)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().startswith("conv_mfma_i8_gather"), runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
 F32_NCHW44 = [
     # f32 channel-wise layers in NCHW44 (the reference's GI_chanwise kernels: 3x3 / 5x5, stride 1 / 2):
     # tiles of 4 x 64 pixels - extents below, at and above a tile, padding 0 .. k/2 + 1, every activation
