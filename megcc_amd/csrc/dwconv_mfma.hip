@@ -89,6 +89,8 @@ typedef unsigned dw_v4u __attribute__((ext_vector_type(4)));
 // are the halves of four pooling windows whose other halves the lane 32 further on holds: after the
 // vertical maximum the same two v_permlane32_swap that prepare the 16-byte stores of the plain
 // kernel hand each lane both halves of two windows; it stores 2 pixels of the final tensor.
+// Bound by the vector ALU beside memory: 267 vector instructions a tile (312 with a rounding of nine
+// instructions, a branch around each pixel's load and store): N=64 C=512 112x112 167 -> 150 us = 4.1 TB/s.
 
 // S: stride (only 1 is instantiated: with stride 2 the layer reads four bytes per byte written and
 // the v_dot4 kernel of dwconv.hip already runs at the rate of a copy - measured 7.8 us against
@@ -135,6 +137,8 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
 
     const __amdgpu_buffer_rsrc_t rd =
             __builtin_amdgcn_make_buffer_rsrc((void*)q.dst, 0, q.dst_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t ro =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(FUSE ? q.other : q.src), 0, FUSE ? q.dst_bytes : 0, 0x00020000);
     // where a lane's results go: byte offset of its 4 pixels in output row y, pixels left in the
     // row (<= 0: nothing to store), rows left in the image
     struct Where {
@@ -182,9 +186,16 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
             const int px0 = (x0 >> 1) + 2 * kg;
             w.pidx = (pset * q.poh + py) * q.pow + px0;
             w.pleft = col_ok && py < q.poh ? q.pow - px0 : 0;
+            // (rows of an even length: the lane's two pixels exist together and are one load and one store)
+            if ((q.pow & 1) == 0) {
+                const dwm_v2u v = __builtin_amdgcn_raw_buffer_load_b64(ro, w.pleft > 0 ? w.pidx * 4 : OOB, 0, 0);
+                w.b4[0] = v[0];
+                w.b4[1] = v[1];
+            } else {
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
-                w.b4[k] = w.pleft > k ? q.other[w.pidx + k] : 0u;
+                for (int k = 0; k < 2; ++k)
+                    w.b4[k] = __builtin_amdgcn_raw_buffer_load_b32(ro, w.pleft > k ? (w.pidx + k) * 4 : OOB, 0, 0);
+            }
         }
         return w;
     };
@@ -311,9 +322,9 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
                     pooled[1][c] = max(sbyte(s13[0], c), sbyte(s13[1], c));
                 }
             }
+            dwm_v2u out;
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
-                const bool ok = cur.pleft > k;
                 const uint32_t b4 = cur.b4[k];
                 int r4[4];
 #pragma unroll
@@ -323,8 +334,14 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
                     const float sum = v0 + v1;
                     r4[c] = fp32_to_int8((FUSE == 2 ? (sum > 0 ? sum : 0) : sum) * q.sdiv);
                 }
-                if (ok)
-                    q.dst[cur.pidx + k] = pack4_perm(r4[0], r4[1], r4[2], r4[3]);
+                out[k] = pack4_perm(r4[0], r4[1], r4[2], r4[3]);
+            }
+            if ((q.pow & 1) == 0) {
+                __builtin_amdgcn_raw_buffer_store_b64(out, rd, cur.pleft > 0 ? cur.pidx * 4 : OOB, 0, 0);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    __builtin_amdgcn_raw_buffer_store_b32(out[k], rd, cur.pleft > k ? (cur.pidx + k) * 4 : OOB, 0, 0);
             }
             continue;
         }
