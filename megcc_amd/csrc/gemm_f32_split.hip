@@ -283,14 +283,14 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
 }
 
 // Against the kernel for few tiles (gemm_f32_ks.hip) on its scale of cycles of the busiest CU: a tile that has a
-// CU to itself takes 106 a step of K, two that share one 205, and 12000 to start and store. Both sides
-// measured (us): 2048^3 101 here / 139 there, 1536^3 68 / 100, 1824 x 2002 x 2524 147 / 166, 735 x 3147 x
-// 3000 143 / 144; 512 x 4096 x 4096 (128 tiles: half the CUs) 183 / 136, 1024 x 1000 x 2048 49 / 46, 640 x 2000 x
-// 1900 92 / 51 stay there.
+// CU to itself counts 118 a step of K, two that share one 205, and 12000 to start and store. Both sides
+// measured (us): 2048^3 110 here / 139 there, 1536^3 69 / 100, 1824 x 2002 x 2524 152 / 166; 735 x 3147 x 3000 152 /
+// 144, 512 x 4096 x 4096 (128 tiles: half the CUs) 183 / 136, 1024 x 1000 x 2048 49 / 46, 640 x 2000 x 1900 92 / 51
+// stay there.
 static bool split_wins(const GevmArgs& v) {
     const long tiles = ((long)(v.M + SP_T - 1) / SP_T) * ((v.N + SP_T - 1) / SP_T);
     const long per_cu = (tiles + num_cus() - 1) / num_cus();
-    return 12000.0 + (double)v.K * (205.0 * (double)(per_cu / 2) + 106.0 * (double)(per_cu & 1)) < gemm_f32_ks_cycles(v);
+    return 12000.0 + (double)v.K * (205.0 * (double)(per_cu / 2) + 118.0 * (double)(per_cu & 1)) < gemm_f32_ks_cycles(v);
 }
 
 static unsigned side_bytes(long rows, long row, long k, long K) {
