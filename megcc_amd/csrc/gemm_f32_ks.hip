@@ -18,10 +18,11 @@
 //     offset into an out-of-range one with one shift and one and-or.
 //   * The last K % 8 values are one more step of one wave, fetched element by element at the start and
 //     masked on both sides (a row's neighbour may hold anything, Inf included).
-// Sums: every wave's chain is K / waves long (shorter than the tiled kernel's 512-step chains); the waves'
-// sums are added in wave order. Fp32MatMulM4N12.cpp:9-158, Fp32Im2col.cpp:88-218 are the loops replaced.
+// Sums: a wave closes its running sums every 64 values of K into a second set of registers; the waves' sums are
+// added in wave order. (Without that, relative error against 64 bits of 64 x 4096 x 4096 4.1e-7, of 197 x 771 x 1003
+// 2.5e-7, where the tiled kernel's slices of K had 3.0e-7 and 1.7e-7.) Fp32MatMulM4N12.cpp:9-158, Fp32Im2col.cpp:88-218 are the loops replaced.
 // Measured (us, before: the tiled kernel with its slice sums in a second launch, or conv_f32_small.hip):
-// 64 x 4096 x 4096 35.4 -> 23.5 (4.5 TB/s of its operands and 92 TFLOP/s), 197 x 771 x 1003 nt 19.9 -> 8.2,
+// 64 x 4096 x 4096 35.4 -> 24.0 (2.9 TB/s and 90 TFLOP/s), 197 x 771 x 1003 nt 19.9 -> 7.5,
 // 8 x 284 x 736 16.5 -> 4.0, 1623 x 3660 x 316 73 -> 41; convolution 32 -> 32 on 56 x 56 6.9 -> 5.1, N=8
 // 64 -> 64 on 56 x 56 55 -> 29, N=8 128 -> 128 165 -> 82.
 #include "common.h"
@@ -173,14 +174,25 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
             }
         }
     };
-    ks_v16f acc[MT][NT];
+    ks_v16f acc[MT][NT], sum[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-                acc[i][j][e] = 0.f;
+                acc[i][j][e] = sum[i][j][e] = 0.f;
+    auto close = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    sum[i][j][e] += acc[i][j][e];
+                    acc[i][j][e] = 0.f;
+                }
+    };
     auto multiply = [&](const ks_v4f (&a)[MT], const ks_v4f (&b)[NT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -231,13 +243,16 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         // (whole groups with nothing under a condition: behind a conditional load the compiler has to assume
         //  fewer loads in flight than there are, and waits for more of them)
         int j0 = 0;
-        for (; j0 + 2 * RING <= nj; j0 += RING)
+        for (; j0 + 2 * RING <= nj; j0 += RING) {
             static_for<RING>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
                 multiply(av[r], bv[r]);
                 load_a((j0 + RING) * W + s0 + r * s_ring, av[r]);
                 load_b((j0 + RING) * W + s0 + r * s_ring, bv[r]);
             });
+            if (j0 & RING)
+                close();
+        }
         for (; j0 < nj; j0 += RING)
             static_for<RING>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
@@ -274,7 +289,7 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-                ks_lds[wave * TILE + ((i * NT + j) * 16 + e) * 64 + lane] = acc[i][j][e];
+                ks_lds[wave * TILE + ((i * NT + j) * 16 + e) * 64 + lane] = acc[i][j][e] + sum[i][j][e];
     __syncthreads();
     // register e of a tile: row 8 * (e / 4) + 4 * h + e % 4, column c. Wave w finishes registers w, w + W, ...
     for (int r = wave; r < MT * NT * 16; r += W) {
@@ -374,7 +389,16 @@ double gemm_f32_ks_cycles(const GevmArgs& v) {
     return matmul_plan(v).cost;
 }
 
+// Rows of B that are contiguous along a long K, few of them: a wave's 32 lanes read 32 lines of one channel's stride,
+// and too few CUs share the chain. The tiled kernel's slices of K over the whole chip are faster there (16 x 4096 x
+// 1024 nt 25.2 us here, 20.1 there; 64 x 4096 x 2048 31.1 / 25.7; at K = 2500, 16 x 512, 14.1 / 18.9).
+static bool long_rows_of_few(const GevmArgs& v) {
+    return v.b_cs != 1 && v.K > 3400 && (long)((v.M + 31) / 32) * ((v.N + 31) / 32) <= num_cus() / 2;
+}
+
 bool gemm_f32_ks_supported(const GevmArgs& v) {
+    if (long_rows_of_few(v))
+        return false;
     const long as = 4 * ((long)(v.M - 1) * v.a_rs + (long)(v.K - 1) * v.a_cs + 1);
     const long bs = 4 * ((long)(v.K - 1) * v.b_rs + (long)(v.N - 1) * v.b_cs + 1);
     return v.K >= 1 && as < (1L << 31) - 65536 && bs < (1L << 31) - 65536 && (v.a_cs == 1 || v.a_rs == 1) &&

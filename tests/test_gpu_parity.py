@@ -381,7 +381,7 @@ def test_fully_connected_over_any_k(kernel, m, k, n, act):
 F32_SHARED_K = [
     # few output tiles, K shared by the waves of a workgroup: extents at and around the 32 / 64 tiles, K below
     # one step of 8, with and without a rest, and long enough for whole lines per wave
-    *[MatMulCase(m, k, n, trans_a=ta, trans_b=tb) for m, k, n in ((5, 3, 7), (33, 8, 31), (64, 1031, 32), (300, 4100, 70))
+    *[MatMulCase(m, k, n, trans_a=ta, trans_b=tb) for m, k, n in ((5, 3, 7), (33, 8, 31), (64, 1031, 32), (300, 3100, 70))
       for ta in (False, True) for tb in (False, True)],
     MatMulCase(513, 100, 1100), MatMulCase(513, 100, 1100, trans_b=True), MatMulCase(1000, 1500, 1000, trans_b=True),
     ConvCase(A.FMT_NCHW, A.DENSE, 1, 1, 5, 6, 1, 1, 1, 0, A.IDENTITY, dtype="f32"),
