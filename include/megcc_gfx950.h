@@ -592,9 +592,12 @@ int megcc_gfx950_requant_affine(int nonline_mode, float s_src, float s_flt, floa
 /* Kernel-selection overrides, for regression tests of kernels that un-switched shapes only reach
  * through a fallback: "nopws", "nogevm", "nofcb", "nosmall", "nopm768", "nopm", "nodma512",
  * "nopm256", "nodma", "nofcs", "nopwshare", "nohybrid", "nodot4", "nof32small",
- * "dw_generic", "nodwmfma", "nodwnchw", "nofusesoftmax", "nopoolrows", "nofirstmfma", "norowsplit", "nofusechain", "nofusepwdw", "fusepwdw", "nofcone", "noxcdorder", "noaffine", "nopipeline", "no_graph"; value 1 takes the kernel out
- * of the dispatch, 0 puts it back ("fusepwdw": 1 makes the model runtime take the one-kernel form of a
- * pointwise / channel-wise pair wherever it applies instead of timing both forms). The
+ * "dw_generic", "nodwmfma", "nodwnchw", "nofusesoftmax", "nopoolrows", "nofirstmfma", "norowsplit", "nofusechain", "nofusepwdw", "fusepwdw", "nofcone", "noxcdorder", "noaffine", "nopipeline", "no_graph",
+ * "nofusedwpw", "fusedwpw", "nof32split", "nof32ks"; value 1 takes the kernel out
+ * of the dispatch, 0 puts it back ("fusepwdw", "fusedwpw": 1 makes the model runtime take the one-kernel form of a
+ * pointwise / channel-wise or channel-wise / pointwise pair wherever it applies instead of timing both forms).
+ * "nof32split" keeps f32 MatMul off the bf16 matrix instructions, "nof32ks" f32 MatMul and convolution off the
+ * kernel whose waves share K; "nof32small" takes out that kernel for convolutions and conv_f32_small behind it. The
  * same names in capitals behind MEGCC_ are read from the environment once, at first use.
  * Unknown names return TinyNN_ERROR_NO_FOUND. */
 TinyNNStatus megcc_gfx950_set_option(const char* name, int value);

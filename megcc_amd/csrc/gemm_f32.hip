@@ -584,9 +584,9 @@ extern "C" TinyNNStatus megcc_gfx950_matmul(
     }
 #ifndef MG_HOST_AUDIT
     const GevmArgs ks = {q.A, q.B, q.C, q.M, q.N, q.K, q.a_rs, q.a_cs, q.b_rs, q.b_cs, q.ldc};
-    if (gemm_f32_split_supported(ks))
+    if (!options().no_f32split && gemm_f32_split_supported(ks))
         return gemm_f32_split_launch(ks, ta, tb);
-    if (gemm_f32_ks_supported(ks))
+    if (!options().no_f32ks && gemm_f32_ks_supported(ks))
         return gemm_f32_ks_launch(ks, ta, tb);
 #endif
     gemm_plan_split(q, ws);

@@ -813,6 +813,11 @@ OLDER = [
     ("nofcone", ConvCase(A.FMT_NCHW, A.DENSE, 40, 1024, 1, 1, 200, 1, 1, 0, A.RELU,
                          scales=(0.01, 0.01, unsat(1024) / 2))),
     ("nof32small", ConvCase(A.FMT_NCHW, A.DENSE, 1, 32, 56, 56, 32, 3, 1, 1, A.RELU, dtype="f32")),
+    # f32 products on the f32 instructions where the default splits them into bf16 parts, and on the tiled kernel /
+    # conv_f32_small where the default has the waves of a workgroup share K
+    ("nof32split", MatMulCase(2900, 33, 3001)), ("nof32split", MatMulCase(2900, 33, 3001, trans_a=True, trans_b=True)),
+    ("nof32ks", MatMulCase(64, 1024, 2048)), ("nof32ks", MatMulCase(197, 131, 203, trans_b=True)),
+    ("nof32ks", ConvCase(A.FMT_NCHW, A.DENSE, 1, 32, 56, 56, 32, 3, 1, 1, A.RELU, dtype="f32")),
     ("nopwshare", ConvCase(A.FMT_NCHW44, A.DENSE, 70, 512, 14, 14, 512, 1, 1, 0, A.RELU,
                                  scales=(0.02, 0.01, unsat(512)))),
     ("nopws", ConvCase(A.FMT_NCHW44, A.DENSE, 11, 64, 56, 56, 128, 1, 1, 0, A.IDENTITY,
