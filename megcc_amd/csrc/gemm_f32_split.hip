@@ -179,20 +179,16 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
 #define MG_SP_MUL(SUM, PA, PB)                                                                              \
     _Pragma("unroll") for (int i = 0; i < 2; ++i) _Pragma("unroll") for (int j = 0; j < 2; ++j) SUM[i][j] = \
             __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA][i], b[PB][j], SUM[i][j], 0, 0, 0)
+        // Smallest products first: each running sum of what x = x1 + x2 + x3 times a power of two leaves behind is
+        // then a float (x3, x2 + x3, x), so selecting values (a one-hot column, a permutation) and products of whole
+        // numbers that fit 24 bits are exact, as in f32. x1 + x3 in that order need not be a float.
+        sp_v16f(&small)[2][2] = SHORT ? sum : acc;
+        MG_SP_MUL(small, 0, 2);
+        MG_SP_MUL(small, 2, 0);
+        MG_SP_MUL(small, 1, 1);
+        MG_SP_MUL(small, 0, 1);
+        MG_SP_MUL(small, 1, 0);
         MG_SP_MUL(acc, 0, 0);
-        if (SHORT) {
-            MG_SP_MUL(sum, 0, 2);
-            MG_SP_MUL(sum, 2, 0);
-            MG_SP_MUL(sum, 1, 1);
-            MG_SP_MUL(sum, 0, 1);
-            MG_SP_MUL(sum, 1, 0);
-        } else {
-            MG_SP_MUL(acc, 0, 2);
-            MG_SP_MUL(acc, 2, 0);
-            MG_SP_MUL(acc, 1, 1);
-            MG_SP_MUL(acc, 0, 1);
-            MG_SP_MUL(acc, 1, 0);
-        }
 #undef MG_SP_MUL
     };
     float va[8], vb[8];

@@ -427,6 +427,35 @@ def test_f32_product_on_the_bf16_instructions(case):
     assert np.all(np.abs(got - _product(case, arrays)) <= bound)
 
 
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("k", [300, 531, 1100])
+def test_f32_product_that_f32_holds_exactly(k, tb):
+    """sums whose every partial sum is a float, in whatever order: one non-zero product per output (a one-hot column or
+    row times any value), and whole numbers below 2^24. No rounding is due, so none may show"""
+    r = np.random.default_rng(k)
+    m, n = 1930, 1925
+    case = MatMulCase(m, k, n, trans_b=tb)
+
+    def run(a, b):
+        got = run_gpu(case, {"a": np.ascontiguousarray(a, np.float32), "b": np.ascontiguousarray(b.T if tb else b, np.float32)})
+        assert runtime.last_kernel().startswith("gemm_f32_split"), runtime.last_kernel()
+        return got
+
+    hot, at = np.zeros((k, n), np.float32), r.integers(0, k, n)
+    hot[at, np.arange(n)] = 1
+    for values in (r.standard_normal((m, k)), r.integers(-(2 ** 24), 2 ** 24 + 1, (m, k)), 2 - r.integers(1, 2 ** 12, (m, k)) * 2.0 ** -23):
+        a = values.astype(np.float32)
+        assert np.array_equal(run(a, hot), a[:, at])
+    hot, at = np.zeros((m, k), np.float32), r.integers(0, k, m)
+    hot[np.arange(m), at] = -0.5
+    b = r.standard_normal((k, n)).astype(np.float32)
+    assert np.array_equal(run(hot, b), -0.5 * b[at])
+    # (the magnitudes' sum stays below 2^23, so a partial sum of rounded parts stays below 2^24)
+    a = r.integers(-(2 ** 23 // (7 * k)), 2 ** 23 // (7 * k) + 1, (m, k))
+    b = r.integers(-7, 8, (k, n))
+    assert np.array_equal(run(a, b), a.astype(np.float64) @ b.astype(np.float64))
+
+
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3e38, 2.0 ** 60, 1e-38, 2.0 ** -103, 0.0])
 @pytest.mark.parametrize("k", [112, 600])
 def test_f32_product_of_values_bf16_parts_cannot_hold(k, value):
