@@ -427,6 +427,53 @@ def test_f32_product_on_the_bf16_instructions(case):
     assert np.all(np.abs(got - _product(case, arrays)) <= bound)
 
 
+def _bf16_parts(x):
+    """x (float32) as the sum of three bf16 values, each the rest rounded to nearest"""
+    parts, rest = [], x.astype(np.float64)
+    for _ in range(3):
+        u = rest.astype(np.float32).view(np.uint32)
+        u = (u + np.uint32(0x7fff) + ((u >> np.uint32(16)) & np.uint32(1))) & np.uint32(0xffff0000)
+        parts.append(u.view(np.float32).astype(np.float64))
+        rest = rest - parts[-1]
+    assert not np.any(rest)
+    return parts
+
+
+# (the short sums and, from 531 on, the closed ones; values of one sign, of both, and so small that the smallest of the
+#  six products are subnormal)
+@pytest.mark.parametrize("dist", ["uniform", "positive", "normal", "small"])
+@pytest.mark.parametrize("m,k,n", [(2900, 33, 3001), (2900, 145, 3001), (2040, 512, 1999), (1930, 531, 1925), (2048, 2050, 2048)])
+def test_f32_product_on_the_bf16_instructions_is_as_accurate_as_f32(m, k, n, dist):
+    """relative error against 64 bits no larger than that of the f32 matrix instructions for the same operands. Where
+    the values have both signs, leaving out any one of the five small products would cost several times that limit"""
+    r = np.random.default_rng(k)
+    draw = {"uniform": lambda *s: r.uniform(-1, 1, s), "positive": lambda *s: r.uniform(0, 1, s),
+            "normal": lambda *s: r.standard_normal(s), "small": lambda *s: r.uniform(-1, 1, s) * 2.0 ** -60}[dist]
+    case, arrays = MatMulCase(m, k, n), {"a": draw(m, k).astype(np.float32), "b": draw(k, n).astype(np.float32)}
+    want = _product(case, arrays)
+    norm = np.linalg.norm(want)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().startswith("gemm_f32_split"), runtime.last_kernel()
+    try:
+        for switch in ("nof32split", "nof32ks"):
+            runtime.set_option(switch, 1)
+        in_f32 = run_gpu(case, arrays)
+        assert runtime.last_kernel().startswith("gemm_f32:"), runtime.last_kernel()
+    finally:
+        for switch in ("nof32split", "nof32ks"):
+            runtime.set_option(switch, 0)
+    limit = np.linalg.norm(in_f32 - want) / norm
+    error = np.linalg.norm(got - want) / norm
+    print("relative error %.3g, f32 %.3g" % (error, limit))
+    assert error <= limit
+    if dist == "positive":  # (sums so much larger than their terms that f32 itself loses as much)
+        return
+    a, b = _bf16_parts(arrays["a"][:200]), _bf16_parts(arrays["b"][:, :200])
+    sample = np.linalg.norm(want[:200, :200])
+    for i, j in ((0, 2), (2, 0), (1, 1), (0, 1), (1, 0)):
+        assert np.linalg.norm(a[i] @ b[j]) / sample > 1.5 * limit, (i, j)
+
+
 @pytest.mark.parametrize("tb", [False, True])
 @pytest.mark.parametrize("k", [300, 531, 1100])
 def test_f32_product_that_f32_holds_exactly(k, tb):
