@@ -8,12 +8,15 @@
 //   * Error of the sums. An instruction rounds the running sum once per 16 steps of K where the f32 instruction
 //     does so 8 times, but there are six of them. So K up to 512 keeps the five small products in a sum of their own
 //     (a rounding of it costs 2^-8), and beyond that one running sum is closed every 128 steps into a second set of
-//     registers. Against 64 bits, relative error here / in f32 before: 4096^3 2.2e-7 / 4.1e-7, 2048^3 2.2e-7 /
-//     4.1e-7, K = 1000 2.2e-7 / 2.9e-7, 333 0.9e-7 / 1.7e-7, 64 0.5e-7 / 1.4e-7.
-//   * The decomposition is exact, and no infinity or subnormal appears on the way, for zero and for
-//     2^-102 <= |x| < 2^60. A workgroup looks at every value it splits and, when one lies outside, multiplies its
-//     tile again with v_mfma_f32_32x32x2_f32 (running sums closed every 512 steps of K): Inf, NaN and
-//     extreme values come out as of an f32 product.
+//     registers. Against 64 bits, relative error here / by the f32 instructions (gemm_f32.hip, the same operands):
+//     4096^3 2.0e-7 / 4.1e-7, 2048^3 1.8e-7 / 4.1e-7, K = 768 1.7e-7 / 5.0e-7, 333 0.9e-7 / 3.3e-7, 64 0.5e-7 / 1.4e-7.
+//   * The decomposition is exact, and no infinity appears on the way, for zero and for 2^-102 <= |x| < 2^60. A
+//     workgroup looks at every value it splits, asks after every chain of 8 stages whether one lay outside, and then
+//     multiplies the rest from that chain on (K up to 512, whose sum of small products runs through: from the
+//     start) with v_mfma_f32_32x32x2_f32, running sums closed every 512 steps of K: Inf, NaN and extreme values come
+//     out as of an f32 product. With such values all over (a soft-max of wide logits; us, here / the f32 kernel):
+//     4096^3 1040 / 1080, 2048^3 188 / 181, 1999 x 333 x 2500 52 / 71. One, in the last chain of every tile: 740 / 1080,
+//     120 / 181, and for K up to 512, where it costs both passes, 81 / 71.
 //   * Workgroup: 128 x 128 outputs, 4 waves of 64 x 64, 16 steps of K a stage, two stages in LDS (50 KB),
 //     the next one's values in registers. Two workgroups share a CU, so that one splits while the other multiplies.
 //     A thread fetches 8 steps of K of one row - two 16-byte loads, or 8 dword loads of 256 contiguous bytes a wave
@@ -132,6 +135,7 @@ struct SplitSide {
 template <bool AK, bool BK, bool SHORT>
 __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
     __shared__ __attribute__((aligned(16))) char lds[2][2 * SP_OPERAND];
+    __shared__ int beyond;  // some thread has split a value that the parts cannot hold
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
     int tx, ty;
@@ -197,18 +201,38 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
         sa.store(&lds[buf][0], va, most, least);
         sb.store(&lds[buf][SP_OPERAND], vb, most, least);
     };
-    if (full) {
-        sa.load(0, va);
-        sb.load(0, vb);
-        split(0);
-        const int next = min(1, full - 1) * SP_K;
-        sa.load(next, va);
-        sb.load(next, vb);
-        __syncthreads();
+    // Whether a thread has met such a value: report(), a barrier, reported(). Every thread then reads the same, since
+    // at least one more barrier (a stage's) lies in front of the next report().
+    auto report = [&]() __attribute__((always_inline)) {
+        if (max(most[0], most[1]) >= SP_HIGH || min(least[0], least[1]) < SP_LOW - 1)
+            beyond = 1;
+    };
+    auto reported = [&]() __attribute__((always_inline)) {
+        return __builtin_amdgcn_readfirstlane(*(volatile int*)&beyond) != 0;
+    };
+    // Steps of K whose products are in the sums for good: all of a chain, once no value of it has been reported.
+    // (SHORT adds the small products of every chain to the one sum: nothing is for good before the end.)
+    int kept = 0;
+    bool f32 = false;
+    sa.load(0, va);
+    sb.load(0, vb);
+    if (threadIdx.x == 0)
+        beyond = 0;
+    __syncthreads();
+    split(0);  // (K is at least two stages)
+    sa.load(SP_K, va);
+    sb.load(SP_K, vb);
+    report();
+    __syncthreads();
+    f32 = reported();
+    for (int s0 = 0; s0 < full && !f32; s0 += SP_CHAIN) {
+        if (!SHORT && s0) {
+            close();
+            kept = s0 * SP_K;
+        }
+        const int s1 = min(s0 + SP_CHAIN, full);
         // (the last two rounds fetch and split the last stage again, for no reader, rather than branch)
-        for (int s = 0; s < full; ++s) {
-            if (!SHORT && s && s % SP_CHAIN == 0)
-                close();
+        for (int s = s0; s < s1; ++s) {
             multiply(s & 1);
             split((s + 1) & 1);
             const int k0 = min(s + 2, full - 1) * SP_K;
@@ -216,19 +240,27 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
             sb.load(k0, vb);
             __syncthreads();
         }
+        report();  // (of the stage behind the chain as well)
+        __syncthreads();
+        f32 = reported();
     }
-    if (full * SP_K < q.K) {
+    if (!f32 && full * SP_K < q.K) {
         sa.load_tail(full * SP_K, q.K, va);
         sb.load_tail(full * SP_K, q.K, vb);
         split(0);  // (every reader of either buffer is behind the loop's last barrier)
         __syncthreads();
+        report();
+        __syncthreads();
+        f32 = reported();
         multiply(0);
     }
-    if (__syncthreads_or(max(most[0], most[1]) >= SP_HIGH || min(least[0], least[1]) < SP_LOW - 1)) {
-        // a value the parts cannot hold: the tile once more, in f32; lo holds the closed sums
+    if (f32) {
+        // the rest in f32, from the chain on that met the value
         clear(acc);
-        clear(sum);
-        for (int k0 = 0; k0 < q.K; k0 += SP_K) {
+        if (SHORT)
+            clear(sum);
+        __syncthreads();  // (a wave may still be in the multiply just above, reading what is written next)
+        for (int k0 = kept; k0 < q.K; k0 += SP_K) {
             if (k0 + SP_K <= q.K) {
                 sa.load(k0, va);
                 sb.load(k0, vb);

@@ -530,6 +530,29 @@ def test_f32_product_of_values_bf16_parts_cannot_hold(k, value):
     assert np.array_equal(got[far], plain[far])
 
 
+# (K: whole stages of 16 and a rest; a last chain of 8 stages, of one, of one and a rest; either side of 512)
+@pytest.mark.parametrize("k,at", [(k, at) for k in (112, 140, 528, 640, 1044) for at in (0, 15, 16, 127, 128, 255, 511, 516, k - 1) if at < k])
+def test_f32_product_that_meets_a_value_the_parts_cannot_hold_on_the_way(k, at):
+    """one value at step `at` of K: what its tile had summed before must neither be lost nor counted twice, and an
+    infinity must not have been in the bf16 product"""
+    case = MatMulCase(2560, k, 2560)
+    arrays = case.gen(seed=37)
+    arrays["b"][at] = np.where(arrays["b"][at] == 0, 1, arrays["b"][at])
+    plain = run_gpu(case, arrays)
+    for value in (2.0 ** -120, 2.0 ** 70, np.inf):
+        changed = {"a": arrays["a"].copy(), "b": arrays["b"]}
+        changed["a"][700, at] = value
+        got = run_gpu(case, changed)
+        assert runtime.last_kernel().startswith("gemm_f32_split"), runtime.last_kernel()
+        want, bound = _product(case, changed), _product(case, {n: np.abs(v) for n, v in changed.items()}) * (k * 2.0 ** -24)
+        if np.isinf(value):
+            assert np.array_equal(got[700], want[700])
+            got[700] = want[700] = bound[700] = 0
+        assert np.all(np.abs(got - want) <= bound)
+        rows = np.arange(2560) // 128 != 700 // 128
+        assert np.array_equal(got[rows], plain[rows])
+
+
 def _gather_cases():
     def c(n, ic, ih, iw, oc, k, s, pad, act=A.RELU, **kw):
         return ConvCase(A.FMT_NCHW44, A.DENSE, n, ic, ih, iw, oc, k, s, pad, act, **kw,
