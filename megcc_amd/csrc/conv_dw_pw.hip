@@ -36,6 +36,7 @@
 namespace mg {
 
 static constexpr int DP_THREADS = 512;
+static constexpr int DP_ALL_BUT_MFMA = 0x7f6;  // what may cross a scheduling barrier: vector, scalar and memory instructions
 typedef unsigned dp_v2u __attribute__((ext_vector_type(2)));
 
 struct DwPwParams {
@@ -317,9 +318,12 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
                         "s_nop 1"
                         : "+v"(R[0]), "+v"(R[1]), "+v"(R[2]), "+v"(R[3])
                         : "v"(B[0][0][0]), "v"(B[1][0][0]), "v"(B[2][0][0]), "v"(B[3][0][0]), "v"(cur.rmask));
-            // The short products of all four plane sets first: a long one that follows ITS short one directly has
-            // read sums that were not there yet (channels 0 and 1 of the last pixels), behind three others it never
-            // does.
+            // The short products of all four plane sets first, and every product where it stands (a scheduling
+            // barrier behind each that only products may not cross). Products of ONE shape take their sums from the one
+            // before at any distance; between the two shapes the sum must have been written: a 16x16x64 product
+            // directly behind its 16x16x32 one has read channels 0 and 1 of the last pixels before that. A short
+            // product takes 4 passes of 4 cycles and a few cycles to write; the three products in between alone
+            // take 12 passes. (The build's code is checked for the three: test_mfma_order.py.)
             unsigned w[4];
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
@@ -332,6 +336,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
                 const dp_v2u al = KEEP_D ? A[KEEP_D ? p : 0].e : band_edges(w[p]), bl = {L[p], S == 1 ? R[p] : L[p]};
                 acc[p] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
                         __builtin_bit_cast(long, al), __builtin_bit_cast(long, bl), acc[p], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(DP_ALL_BUT_MFMA);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -343,6 +348,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
                         b[RAG] = (h == 0 ? cur.edge : cur.edgeb) ? 0 : b[RAG];
                     acc[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
                             KEEP_D ? A[KEEP_D ? p : 0].m[h] : band_half(w[p], h), b, acc[p], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(DP_ALL_BUT_MFMA);
                 }
             __builtin_amdgcn_sched_barrier(0);
             // the operands are consumed: the next job's loads fly while this one is requantised
