@@ -328,7 +328,7 @@ TinyNNStatus conv_first_launch(
     // evaluates the literal sequence per output
     const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     static const RequantTable no_table = {};
-    const RequantTable& table = tab ? requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst) : no_table;
+    const RequantTable table = tab ? requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst) : no_table;
     auto kern = tab && g.act == MEGCC_NONLINE_IDENTITY ? conv_first_q8_kernel<MEGCC_NONLINE_IDENTITY>
               : tab && g.act == MEGCC_NONLINE_RELU     ? conv_first_q8_kernel<MEGCC_NONLINE_RELU>
               : tab && g.act == MEGCC_NONLINE_H_SWISH  ? conv_first_q8_kernel<MEGCC_NONLINE_H_SWISH>

@@ -184,9 +184,8 @@ static inline bool requant_table_act(int act) {
     return act == MEGCC_NONLINE_IDENTITY || act == MEGCC_NONLINE_RELU || act == MEGCC_NONLINE_H_SWISH;
 }
 
-// host: the table for (act in {IDENTITY, RELU, H_SWISH}, scales); the reference stays valid for the
-// life of the process (requant_table.hip)
-const RequantTable& requant_table_for(int act, float s_src, float s_flt, float s_dst);
+// host: the table for (act in {IDENTITY, RELU, H_SWISH}, scales); requant_table.hip
+RequantTable requant_table_for(int act, float s_src, float s_flt, float s_dst);
 
 // the lower candidate m (clamped to [lowest output, 126]) of the output for accumulator acc
 template <int ACT>

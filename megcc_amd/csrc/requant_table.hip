@@ -1,12 +1,11 @@
 // Host-side cache of requantisation threshold tables (see epilogue.h): one table per
 // (activation, src scale, filter scale, dst scale), built on first use with the reference's
 // literal float sequence evaluated by the host CPU - the same IEEE single-precision multiply,
-// multiply, divide, roundf the generated C kernels execute - and kept for the life of the process.
+// multiply, divide, roundf the generated C kernels execute - and kept for later calls (at most 4096 of them).
 #include <math.h>
 
 #include <cstring>
 #include <map>
-#include <memory>
 #include <mutex>
 #include <tuple>
 #include <vector>
@@ -16,32 +15,60 @@
 
 namespace mg {
 
-const RequantTable& requant_table_for(int act, float s_src, float s_flt, float s_dst) {
-    static std::mutex lock;
-    static std::map<std::tuple<int, uint32_t, uint32_t, uint32_t>, std::unique_ptr<RequantTable>> cache;
-    auto bits = [](float f) {
-        uint32_t u;
-        memcpy(&u, &f, 4);
-        return u;
-    };
-    const auto key = std::make_tuple(act, bits(s_src), bits(s_flt), bits(s_dst));
-    std::lock_guard<std::mutex> guard(lock);
-    auto it = cache.find(key);
-    if (it != cache.end())
-        return *it->second;
-    std::unique_ptr<RequantTable> t(new RequantTable);
+// what has been worked out for (activation, scales): emptied when it is full, so that a process that meets ever new
+// scales does not grow
+template <typename T>
+class ScaleCache {
+public:
+    static constexpr size_t MOST = 4096;
+    typedef std::tuple<int, uint32_t, uint32_t, uint32_t> Key;
+    static Key key(int act, float s_src, float s_flt, float s_dst) {
+        auto bits = [](float f) {
+            uint32_t u;
+            memcpy(&u, &f, 4);
+            return u;
+        };
+        return std::make_tuple(act, bits(s_src), bits(s_flt), bits(s_dst));
+    }
+    bool find(const Key& k, T* out) {
+        std::lock_guard<std::mutex> guard(lock_);
+        auto it = map_.find(k);
+        if (it == map_.end())
+            return false;
+        *out = it->second;
+        return true;
+    }
+    void put(const Key& k, const T& v) {
+        std::lock_guard<std::mutex> guard(lock_);
+        if (map_.size() >= MOST)
+            map_.clear();
+        map_[k] = v;
+    }
+
+private:
+    std::mutex lock_;
+    std::map<Key, T> map_;
+};
+
+RequantTable requant_table_for(int act, float s_src, float s_flt, float s_dst) {
+    static ScaleCache<RequantTable> cache;
+    const auto key = cache.key(act, s_src, s_flt, s_dst);
+    RequantTable t;
+    if (cache.find(key, &t))
+        return t;
     const float c = make_requant_fast(s_src, s_flt, s_dst).c;
     for (int i = 0; i < REQUANT_TABLE_ENTRIES; ++i) {
         if (i == REQUANT_TABLE_ENTRIES - 1)
-            t->t[i] = 0;
+            t.t[i] = 0;
         else if (act == MEGCC_NONLINE_RELU)
-            t->t[i] = requant_threshold<MEGCC_NONLINE_RELU>(i, s_src, s_flt, s_dst, c);
+            t.t[i] = requant_threshold<MEGCC_NONLINE_RELU>(i, s_src, s_flt, s_dst, c);
         else if (act == MEGCC_NONLINE_H_SWISH)
-            t->t[i] = requant_threshold<MEGCC_NONLINE_H_SWISH>(i, s_src, s_flt, s_dst, c);
+            t.t[i] = requant_threshold<MEGCC_NONLINE_H_SWISH>(i, s_src, s_flt, s_dst, c);
         else
-            t->t[i] = requant_threshold<MEGCC_NONLINE_IDENTITY>(i, s_src, s_flt, s_dst, c);
+            t.t[i] = requant_threshold<MEGCC_NONLINE_IDENTITY>(i, s_src, s_flt, s_dst, c);
     }
-    return *(cache[key] = std::move(t));
+    cache.put(key, t);
+    return t;
 }
 
 // host evaluation of requant_conv_affine (fmaf is the correctly rounded single fused multiply-add,
@@ -53,24 +80,15 @@ static int affine_eval(int a, float c, float d, int lo) {
 }
 
 RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst) {
-    static std::mutex lock;
-    static std::map<std::tuple<int, uint32_t, uint32_t, uint32_t>, RequantAffine> cache;
+    static ScaleCache<RequantAffine> cache;
     const RequantAffine none = {0.f, 0.f};
     if ((act != MEGCC_NONLINE_IDENTITY && act != MEGCC_NONLINE_RELU) || !requant_table_ok(s_src, s_flt, s_dst))
         return none;
-    auto bits = [](float f) {
-        uint32_t u;
-        memcpy(&u, &f, 4);
-        return u;
-    };
-    const auto key = std::make_tuple(act, bits(s_src), bits(s_flt), bits(s_dst));
-    {
-        std::lock_guard<std::mutex> guard(lock);
-        auto it = cache.find(key);
-        if (it != cache.end())
-            return it->second;
-    }
-    const RequantTable& T = requant_table_for(act, s_src, s_flt, s_dst);
+    const auto key = cache.key(act, s_src, s_flt, s_dst);
+    RequantAffine found = none;
+    if (cache.find(key, &found))
+        return found;
+    const RequantTable T = requant_table_for(act, s_src, s_flt, s_dst);
     const int lo = act == MEGCC_NONLINE_RELU ? 0 : -128;
     auto literal = [&](int a) {
         return act == MEGCC_NONLINE_RELU ? requant_conv<MEGCC_NONLINE_RELU>(a, s_src, s_flt, s_dst)
@@ -92,7 +110,6 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
             pts.push_back({t + 1, literal(t + 1)});
     }
     const float c0 = make_requant_fast(s_src, s_flt, s_dst).c;
-    RequantAffine found = none;
     for (int k = 0; k <= 16 && found.d == 0.f; ++k) {
         // c' = c0 moved (k + 1) / 2 ulps up (k odd) or down (k even)
         float c = c0;
@@ -127,10 +144,8 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
             }
         }
     }
-    std::lock_guard<std::mutex> guard(lock);
-    if (cache.size() >= 4096)
-        cache.clear();
-    return cache[key] = found;
+    cache.put(key, found);
+    return found;
 }
 
 // host evaluation of requant_pack4 for one output
@@ -144,25 +159,16 @@ static int pack_eval(int a, int act, const RequantPack& q) {
 }
 
 RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
-    static std::mutex lock;
-    static std::map<std::tuple<int, uint32_t, uint32_t, uint32_t>, RequantPack> cache;
+    static ScaleCache<RequantPack> cache;
     const RequantPack none = {0.f, 0.f, 0.f, 0.f, 0};
     if ((act != MEGCC_NONLINE_IDENTITY && act != MEGCC_NONLINE_RELU) || !requant_table_ok(s_src, s_flt, s_dst) ||
         options().no_affine)
         return none;
-    auto bits = [](float f) {
-        uint32_t u;
-        memcpy(&u, &f, 4);
-        return u;
-    };
-    const auto key = std::make_tuple(act, bits(s_src), bits(s_flt), bits(s_dst));
-    {
-        std::lock_guard<std::mutex> guard(lock);
-        auto it = cache.find(key);
-        if (it != cache.end())
-            return it->second;
-    }
-    const RequantTable& T = requant_table_for(act, s_src, s_flt, s_dst);
+    const auto key = cache.key(act, s_src, s_flt, s_dst);
+    RequantPack found = none;
+    if (cache.find(key, &found))
+        return found;
+    const RequantTable T = requant_table_for(act, s_src, s_flt, s_dst);
     const bool relu = act == MEGCC_NONLINE_RELU;
     auto literal = [&](int a) {
         return relu ? requant_conv<MEGCC_NONLINE_RELU>(a, s_src, s_flt, s_dst)
@@ -192,7 +198,6 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
     const Form forms[] = {{1, 1.f, 1.f, make_requant_fast(s_src, s_flt, s_dst).c * unit},
                           {2, s_src, 1.f, s_flt / s_dst * unit},
                           {2, s_src, s_flt, 1.f / s_dst * unit}};
-    RequantPack found = none;
     std::vector<float> x(pts.size());
     for (const Form& f : forms) {
         for (size_t i = 0; i < pts.size(); ++i)
@@ -230,10 +235,8 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
         if (found.mode)
             break;
     }
-    std::lock_guard<std::mutex> guard(lock);
-    if (cache.size() >= 4096)
-        cache.clear();
-    return cache[key] = found;
+    cache.put(key, found);
+    return found;
 }
 
 RequantAffine requant_affine_pick(bool table, int act, float s_src, float s_flt, float s_dst) {

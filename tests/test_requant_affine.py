@@ -5,6 +5,8 @@ zero input, so that the accumulator is the bias) against the fused multiply-add 
 for every accumulator around the 255 steps and on a dense range. No GPU involved."""
 import json
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -106,3 +108,30 @@ def test_large_and_small_ratios():
                    (0.02, 0.01, 0.0371234), (1.0, 1.0, 1.0), (0.25, 0.5, 0.125)]:
         for act in (abi.RELU, abi.IDENTITY):
             check_pair(act, scales)
+
+
+GROWTH = """
+import os
+from megcc_amd import abi, runtime
+
+def resident():
+    with open("/proc/self/statm") as f:
+        return int(f.read().split()[1]) * os.sysconf("SC_PAGE_SIZE")
+
+def meet(first, count):
+    for i in range(first, first + count):
+        runtime.requant_affine(abi.RELU, 0.02 + i * 1e-7, 0.01, 0.05)
+
+meet(0, 6000)  # (fills what is kept once)
+before = resident()
+meet(6000, 16000)
+print(resident() - before)
+"""
+
+
+def test_scales_that_never_come_back_do_not_pile_up():
+    """what the searches keep for later calls is bounded (4096 tables of 1 KB): a process that meets ever new scales must
+    not grow by one for each. (A process of its own: this one's heap has room from other tests.)"""
+    grown = int(subprocess.run([sys.executable, "-c", GROWTH], cwd=os.path.dirname(HERE), capture_output=True, text=True,
+                               check=True).stdout)
+    assert grown < 8 << 20, grown
