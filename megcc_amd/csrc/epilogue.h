@@ -123,7 +123,7 @@ __device__ __forceinline__ int requant_conv_rt(int act, int acc, float s0, float
 // For a monotone activation (IDENTITY, RELU) the reference's F(acc) = fp32_to_int8(act(acc * s_src
 // * s_flt / s_dst)) is a non-decreasing step function of the integer accumulator, so it is fully
 // described by 255 thresholds T[j] = max{a : F(a) < j}, j = -127..127:  F(a) = lo + #{j : a > T[j]}.
-// The table is built with the reference's literal float sequence (binary search over int32) - on
+// The table is built with the reference's literal float sequence (a search over int32 per level) - on
 // the host, once per (activation, scales) and cached, since x86-64 SSE arithmetic and the device's
 // are the same IEEE operations; it travels to the kernel as an argument and each workgroup copies
 // it to LDS. A kernel then needs only ONE estimate per output:
@@ -132,36 +132,6 @@ __device__ __forceinline__ int requant_conv_rt(int act, int acc, float s0, float
 //     m = clamp(floor(g), lo, 126);   F(a) = m + (a > T[m + 1])
 // No rounding-mode reasoning, no near-tie special case, bit-exact by construction.
 static constexpr int REQUANT_TABLE_ENTRIES = 256;  // entry j + 127, last one unused
-
-// entry `idx` (0..254) of the table: a handful of evaluations of the literal sequence (32 when
-// the estimate from c is useless)
-template <int ACT>
-__host__ __device__ __forceinline__ int requant_threshold(int idx, float s_src, float s_flt, float s_dst, float c) {
-    const int j = idx - 127;
-    auto below = [&](long long a) { return requant_conv<ACT>((int)a, s_src, s_flt, s_dst) < j; };
-    long long lo = INT32_MIN, hi = INT32_MAX;
-    if (!below(lo))
-        return INT32_MIN;  // F never drops below j: entry not used (j <= lowest output)
-    // the threshold is next to (j - 0.5) / c: try a bracket of +-8 around it first
-    if (c > 0.f) {
-        const float est = ((float)j - 0.5f) / c;
-        if (est > -2.0e9f && est < 2.0e9f) {
-            const long long e = (long long)est;
-            if (below(e - 8) && !below(e + 8)) {
-                lo = e - 8;
-                hi = e + 7;
-            }
-        }
-    }
-    while (lo < hi) {  // invariant: F(lo) < j, F(hi + 1) >= j or hi == INT32_MAX
-        const long long mid = lo + (hi - lo + 1) / 2;
-        if (below(mid))
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return (int)lo;
-}
 
 // (int)floorf(x) in one instruction (saturating like the plain conversion)
 __device__ __forceinline__ int cvt_floor_i32(float x) {

@@ -4,11 +4,11 @@
 // multiply, divide, roundf the generated C kernels execute - and kept for later calls (at most 4096 of them).
 #include <math.h>
 
+#include <algorithm>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <tuple>
-#include <vector>
 
 #include "common.h"
 #include "epilogue.h"
@@ -50,6 +50,61 @@ private:
     std::map<Key, T> map_;
 };
 
+// Entry by entry the largest accumulator whose output is still below j: a gallop and a bisection from the estimate,
+// with the literal sequence up to the activation. Its rounding is a comparison here: roundf(x) < j iff x < j - 0.5,
+// or x = j - 0.5 where the half goes away from zero to j - 1 (a NaN is below everything, as the conversion has it).
+// 3 or 4 evaluations an entry. (A first launch with new scales waits for this and for the search below: over 60000
+// scales 13 us -> 3.6 for the table and 8.6 -> 4.6 for the multiply-add's constants on one host core, against
+// a call of the rounding function and a bisection from +-8 for each entry.)
+template <int ACT>
+static void requant_thresholds(float s_src, float s_flt, float s_dst, float c, int* t) {
+    for (int i = 0; i < REQUANT_TABLE_ENTRIES - 1; ++i) {
+        const int j = i - 127;
+        const float edge = (float)j - 0.5f;
+        auto below = [&](long long a) {
+            const float x = act_apply<ACT>((float)(int)a * s_src * s_flt / s_dst);
+            return j > 0 ? !(x >= edge) : !(x > edge);
+        };
+        if (!below(INT32_MIN)) {
+            t[i] = INT32_MIN;  // F never drops below j: entry not used (j <= lowest output)
+            continue;
+        }
+        float v = edge;
+        if (ACT == MEGCC_NONLINE_H_SWISH && v > 0.f && v < 3.f)
+            v = 0.5f * (sqrtf(9.f + 24.f * v) - 3.f);
+        const float est = v / c;
+        long long lo = INT32_MIN, hi = (long long)INT32_MAX + 1;  // F(lo) < j, F(hi) >= j (beyond the last: taken as such)
+        if (est > -2.0e9f && est < 2.0e9f) {
+            const long long e = (long long)est;
+            long long step = 1;
+            if (below(e)) {
+                lo = e;
+                while (lo + step < hi && below(lo + step)) {
+                    lo += step;
+                    step *= 2;
+                }
+                hi = std::min(hi, lo + step);
+            } else {
+                hi = e;
+                while (hi - step > lo && !below(hi - step)) {
+                    hi -= step;
+                    step *= 2;
+                }
+                lo = std::max(lo, hi - step);
+            }
+        }
+        while (hi - lo > 1) {
+            const long long mid = lo + (hi - lo) / 2;
+            if (below(mid))
+                lo = mid;
+            else
+                hi = mid;
+        }
+        t[i] = (int)lo;
+    }
+    t[REQUANT_TABLE_ENTRIES - 1] = 0;
+}
+
 RequantTable requant_table_for(int act, float s_src, float s_flt, float s_dst) {
     static ScaleCache<RequantTable> cache;
     const auto key = cache.key(act, s_src, s_flt, s_dst);
@@ -57,19 +112,75 @@ RequantTable requant_table_for(int act, float s_src, float s_flt, float s_dst) {
     if (cache.find(key, &t))
         return t;
     const float c = make_requant_fast(s_src, s_flt, s_dst).c;
-    for (int i = 0; i < REQUANT_TABLE_ENTRIES; ++i) {
-        if (i == REQUANT_TABLE_ENTRIES - 1)
-            t.t[i] = 0;
-        else if (act == MEGCC_NONLINE_RELU)
-            t.t[i] = requant_threshold<MEGCC_NONLINE_RELU>(i, s_src, s_flt, s_dst, c);
-        else if (act == MEGCC_NONLINE_H_SWISH)
-            t.t[i] = requant_threshold<MEGCC_NONLINE_H_SWISH>(i, s_src, s_flt, s_dst, c);
-        else
-            t.t[i] = requant_threshold<MEGCC_NONLINE_IDENTITY>(i, s_src, s_flt, s_dst, c);
-    }
+    if (act == MEGCC_NONLINE_RELU)
+        requant_thresholds<MEGCC_NONLINE_RELU>(s_src, s_flt, s_dst, c, t.t);
+    else if (act == MEGCC_NONLINE_H_SWISH)
+        requant_thresholds<MEGCC_NONLINE_H_SWISH>(s_src, s_flt, s_dst, c, t.t);
+    else
+        requant_thresholds<MEGCC_NONLINE_IDENTITY>(s_src, s_flt, s_dst, c, t.t);
     cache.put(key, t);
     return t;
 }
+
+// Both sides of every step of F and the ends of the accumulator range, with the outputs there: F(T) is one less than the
+// first level whose threshold is T, F(T + 1) the last such level.
+struct RequantSteps {
+    int n = 0;
+    int a[2 * REQUANT_TABLE_ENTRIES + 2], y[2 * REQUANT_TABLE_ENTRIES + 2];
+    void add(int acc, int out) {
+        a[n] = acc;
+        y[n++] = out;
+    }
+};
+static RequantSteps requant_steps(const RequantTable& T, int lo) {
+    RequantSteps s;
+    int first = lo + 128;  // (levels up to the lowest output have no step)
+    int low = lo, high = lo;  // outputs of the smallest and the largest accumulator
+    while (first < REQUANT_TABLE_ENTRIES - 1 && T.t[first] == INT32_MIN)
+        low = high = first++ - 127;
+    for (int i = first; i < REQUANT_TABLE_ENTRIES - 1; ++i)
+        if (T.t[i] < INT32_MAX)
+            high = i - 127;
+    s.add(INT32_MIN, low);
+    s.add(INT32_MAX, high);
+    for (int i = first; i < REQUANT_TABLE_ENTRIES - 1;) {
+        int k = i;
+        while (k + 1 < REQUANT_TABLE_ENTRIES - 1 && T.t[k + 1] == T.t[i])
+            ++k;
+        s.add(T.t[i], i - 128);
+        if (T.t[i] < INT32_MAX)
+            s.add(T.t[i] + 1, k - 127);
+        i = k + 1;
+    }
+    return s;
+}
+
+// lower and upper bounds for d: at[i] - x[i] c <= d, and <= for the upper ones (the largest of the lower, the smallest of
+// the upper; four chains, since one would wait for each comparison)
+struct RequantBounds {
+    int n = 0;
+    double x[2 * REQUANT_TABLE_ENTRIES + 2], at[2 * REQUANT_TABLE_ENTRIES + 2];
+    void add(double v, double bound) {
+        x[n] = v;
+        at[n++] = bound;
+    }
+    template <bool LOWER>
+    double tightest(double c) const {
+        const double none = LOWER ? -1e30 : 1e30;
+        double m[4] = {none, none, none, none};
+        auto take = [&](int j, int i) {
+            const double v = at[i] - x[i] * c;
+            m[j] = (LOWER ? v > m[j] : v < m[j]) ? v : m[j];
+        };
+        int i = 0;
+        for (; i + 4 <= n; i += 4)
+            for (int j = 0; j < 4; ++j)
+                take(j, i + j);
+        for (; i < n; ++i)
+            take(0, i);
+        return LOWER ? std::max(std::max(m[0], m[1]), std::max(m[2], m[3])) : std::min(std::min(m[0], m[1]), std::min(m[2], m[3]));
+    }
+};
 
 // host evaluation of requant_conv_affine (fmaf is the correctly rounded single fused multiply-add,
 // floorf + saturation what v_cvt_flr_i32_f32 does)
@@ -88,26 +199,14 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
     RequantAffine found = none;
     if (cache.find(key, &found))
         return found;
-    const RequantTable T = requant_table_for(act, s_src, s_flt, s_dst);
     const int lo = act == MEGCC_NONLINE_RELU ? 0 : -128;
-    auto literal = [&](int a) {
-        return act == MEGCC_NONLINE_RELU ? requant_conv<MEGCC_NONLINE_RELU>(a, s_src, s_flt, s_dst)
-                                         : requant_conv<MEGCC_NONLINE_IDENTITY>(a, s_src, s_flt, s_dst);
-    };
-    // both sides of every step of F, and the ends of the accumulator range
-    struct Point {
-        int a, y;
-    };
-    std::vector<Point> pts;
-    pts.push_back({INT32_MIN, literal(INT32_MIN)});
-    pts.push_back({INT32_MAX, literal(INT32_MAX)});
-    for (int i = 0; i < REQUANT_TABLE_ENTRIES - 1; ++i) {
-        const int t = T.t[i];
-        if (t == INT32_MIN)
-            continue;  // F never drops below this level
-        pts.push_back({t, literal(t)});
-        if (t < INT32_MAX)
-            pts.push_back({t + 1, literal(t + 1)});
+    const RequantSteps pts = requant_steps(requant_table_for(act, s_src, s_flt, s_dst), lo);
+    RequantBounds from, to;  // floor(a c + d) == y  <=>  y <= a c + d < y + 1
+    for (int i = 0; i < pts.n; ++i) {
+        if (pts.y[i] > lo)
+            from.add((double)(float)pts.a[i], (double)pts.y[i]);
+        if (pts.y[i] < 127)
+            to.add((double)(float)pts.a[i], (double)pts.y[i] + 1);
     }
     const float c0 = make_requant_fast(s_src, s_flt, s_dst).c;
     for (int k = 0; k <= 16 && found.d == 0.f; ++k) {
@@ -115,14 +214,7 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
         float c = c0;
         for (int s = 0; s < (k + 1) / 2; ++s)
             c = nextafterf(c, (k & 1) ? INFINITY : 0.f);
-        double dlo = -1e30, dhi = 1e30;  // floor(a c + d) == y  <=>  y <= a c + d < y + 1
-        for (const Point& p : pts) {
-            const double prod = (double)(float)p.a * (double)c;
-            if (p.y > lo && (double)p.y - prod > dlo)
-                dlo = (double)p.y - prod;
-            if (p.y < 127 && (double)p.y + 1 - prod < dhi)
-                dhi = (double)p.y + 1 - prod;
-        }
+        const double dlo = from.tightest<true>((double)c), dhi = to.tightest<false>((double)c);
         if (!(dlo < dhi))
             continue;
         // the middle of the interval first (the most room for the rounding of the fused multiply-add),
@@ -133,11 +225,8 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
             if (!(d > 0.f && d < 1.f))
                 continue;
             bool ok = true;
-            for (const Point& p : pts)
-                if (affine_eval(p.a, c, d, lo) != p.y) {
-                    ok = false;
-                    break;
-                }
+            for (int i = 0; i < pts.n && ok; ++i)
+                ok = affine_eval(pts.a[i], c, d, lo) == pts.y[i];
             if (ok) {
                 found = {c, d};
                 break;
@@ -168,27 +257,9 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
     RequantPack found = none;
     if (cache.find(key, &found))
         return found;
-    const RequantTable T = requant_table_for(act, s_src, s_flt, s_dst);
     const bool relu = act == MEGCC_NONLINE_RELU;
-    auto literal = [&](int a) {
-        return relu ? requant_conv<MEGCC_NONLINE_RELU>(a, s_src, s_flt, s_dst)
-                    : requant_conv<MEGCC_NONLINE_IDENTITY>(a, s_src, s_flt, s_dst);
-    };
-    // both sides of every step of F, and the ends of the accumulator range
-    struct Point {
-        int a, y;
-    };
-    std::vector<Point> pts;
-    pts.push_back({INT32_MIN, literal(INT32_MIN)});
-    pts.push_back({INT32_MAX, literal(INT32_MAX)});
-    for (int i = 0; i < REQUANT_TABLE_ENTRIES - 1; ++i) {
-        const int t = T.t[i];
-        if (t == INT32_MIN)
-            continue;  // F never drops below this level
-        pts.push_back({t, literal(t)});
-        if (t < INT32_MAX)
-            pts.push_back({t + 1, literal(t + 1)});
-    }
+    const int lowest = relu ? 0 : -128;
+    const RequantSteps pts = requant_steps(requant_table_for(act, s_src, s_flt, s_dst), lowest);
     // the forms in order of cost: no product in front, one, two
     struct Form {
         int mode;
@@ -198,34 +269,30 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
     const Form forms[] = {{1, 1.f, 1.f, make_requant_fast(s_src, s_flt, s_dst).c * unit},
                           {2, s_src, 1.f, s_flt / s_dst * unit},
                           {2, s_src, s_flt, 1.f / s_dst * unit}};
-    std::vector<float> x(pts.size());
     for (const Form& f : forms) {
-        for (size_t i = 0; i < pts.size(); ++i)
-            x[i] = f.mode == 2 ? (float)pts[i].a * f.s1 * f.s2 : (float)pts[i].a;
+        RequantBounds from, to;  // RELU: 2 y <= rint <= 2 y + 1; IDENTITY: rint == y + 128
+        for (int i = 0; i < pts.n; ++i) {
+            const double x = f.mode == 2 ? (float)pts.a[i] * f.s1 * f.s2 : (float)pts.a[i];
+            const int y = pts.y[i];
+            if (y > lowest)
+                from.add(x, relu ? 2.0 * y - 0.5 : y + 127.5);
+            if (y < 127)
+                to.add(x, relu ? 2.0 * y + 1.5 : y + 128.5);
+        }
         for (int k = 0; k <= 48 && !found.mode; ++k) {
             // c = c0 moved (k + 1) / 2 ulps up (k odd) or down (k even)
             float c = f.c0;
             for (int s = 0; s < (k + 1) / 2; ++s)
                 c = nextafterf(c, (k & 1) ? INFINITY : 0.f);
-            double dlo = -1e30, dhi = 1e30;
-            for (size_t i = 0; i < pts.size(); ++i) {
-                const double prod = (double)x[i] * (double)c;
-                const int y = pts[i].y;
-                // RELU: 2 y <= rint <= 2 y + 1; IDENTITY: rint == y + 128
-                const double lo = relu ? 2.0 * y - 0.5 : y + 127.5, hi = relu ? 2.0 * y + 1.5 : y + 128.5;
-                if (y > (relu ? 0 : -128) && lo - prod > dlo)
-                    dlo = lo - prod;
-                if (y < 127 && hi - prod < dhi)
-                    dhi = hi - prod;
-            }
+            const double dlo = from.tightest<true>((double)c), dhi = to.tightest<false>((double)c);
             if (!(dlo <= dhi))
                 continue;
             static const double kPos[] = {0.5, 0.375, 0.625, 0.25, 0.75, 0.125, 0.875};
             for (double pos : kPos) {
                 const RequantPack q = {f.s1, f.s2, c, (float)(dlo + (dhi - dlo) * pos), f.mode};
                 bool ok = true;
-                for (size_t i = 0; i < pts.size() && ok; ++i)
-                    ok = pack_eval(pts[i].a, act, q) == pts[i].y;
+                for (int i = 0; i < pts.n && ok; ++i)
+                    ok = pack_eval(pts.a[i], act, q) == pts.y[i];
                 if (ok) {
                     found = q;
                     break;
