@@ -32,13 +32,20 @@ __host__ __device__ __forceinline__ float act_apply(float x) {
     return x;
 }
 
+// (int)x by the instruction's name: it saturates and turns NaN into 0, where the conversion in the language is undefined
+// for what an int cannot hold
+__device__ __forceinline__ int cvt_i32(float x) {
+    int r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
 __host__ __device__ __forceinline__ int fp32_to_int8(float v) {
-    // (clamped as a float: the conversion of an out-of-range float is the saturating one on the
-    //  device but not on the host, where the threshold tables are built)
+    // (on the host, where nothing saturates, clamped as a float)
 #if defined(__HIP_DEVICE_COMPILE__)
     // Half away from zero is truncation of the value plus the largest float below a half (the same for every
     // float, checked one by one; a half itself would carry 0.49999997 up): four instructions for nine.
-    const int i = (int)(v + __builtin_copysignf(0x1.fffffep-2f, v));  // (saturating; NaN is 0)
+    const int i = cvt_i32(v + __builtin_copysignf(0x1.fffffep-2f, v));
     return i > 127 ? 127 : (i < -128 ? -128 : i);
 #else
     float r = roundf(v);
@@ -98,7 +105,7 @@ __device__ __forceinline__ int requant_conv_fast(int acc, const RequantFast& q) 
     if (__builtin_expect((!(d <= 0.5f - 0x1p-13f) && __builtin_fabsf(g) < 129.f) || q.c == 0.f, 0)) {
         out = requant_conv<ACT>(acc, q.s_src, q.s_flt, q.s_dst);
     } else {
-        int i = (int)r;  // saturating conversion
+        const int i = cvt_i32(r);
         const int lo = ACT == MEGCC_NONLINE_RELU ? 0 : -128;
         out = i < lo ? lo : (i > 127 ? 127 : i);
     }
