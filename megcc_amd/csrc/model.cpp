@@ -62,6 +62,8 @@ struct Model {
     // one kernel (`fused` owns the replacements); run_opr, nr_opr and the memory plan keep the
     // operator list as it was given
     std::vector<ModelOpr*> schedule, fused;
+    // per operator: whether the pair that begins there measured faster as one kernel (-1: not measured)
+    std::vector<signed char> dw_pw_faster, pw_dw_faster;
     void* arena = nullptr;
     size_t arena_bytes = 0;
     // one scratch buffer shared by all operators (they run one after the other on one stream),
@@ -269,9 +271,19 @@ static TinyNNStatus call_opr(Model* m, ModelOpr* o) {
             &o->desc, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(), (int)o->out_ptrs.size(), &o->ws,
             &m->opt);
 }
+// One wave that looks at the 100 MHz clock until `ticks` have gone by (each look sleeps 64 cycles or more: at most
+// `looks` of them whatever the clock does).
+__global__ void hold_kernel(long long ticks, int looks) {
+    const long long t0 = wall_clock64();
+    while (looks-- > 0 && wall_clock64() - t0 < ticks)
+        __builtin_amdgcn_s_sleep(8);
+}
+
 // Milliseconds `iters` back-to-back rounds of the operators in `ops` take on the library stream
 // (after one untimed round), or a negative value when a launch fails or an operand has no memory.
-static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters) {
+// `device_only`: the device is held until the host has enqueued the rounds, so that the time is the kernels' own also
+// where they are shorter than a launch takes the host.
+static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters, bool device_only = false) {
     for (const ModelOpr* o : ops) {
         for (const Tensor* t : o->in_ptrs)
             if (!t->ptr)
@@ -294,6 +306,11 @@ static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters) {
     }
     float ms = -1.f;
     bool ok = round();
+    if (device_only && ok) {  // (a launch takes the host 3 - 5 us)
+        const int us = 20 + 8 * iters * (int)ops.size();
+        hipLaunchKernelGGL(hold_kernel, dim3(1), dim3(64), 0, stream(), 100LL * us, 8 * us);
+        ok = check_launch("hold") == TinyNN_SUCCESS;
+    }
     ok = ok && hipEventRecord(e0, stream()) == hipSuccess;
     for (int i = 0; ok && i < iters; ++i)
         ok = round();
@@ -304,8 +321,28 @@ static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters) {
     return ok ? ms : -1.f;
 }
 
-static void build_schedule(Model* m, bool allow_pw_dw = true) {
+// `one` in place of `two`: the kernels' own times, measured once per pair (a few rounds on the tensors as they are;
+// their contents do not matter before the first forward). At small sizes plain launches back to back would time the
+// host instead, and the pair always win: it is one launch fewer.
+static bool faster_as_one(Model* m, std::vector<signed char>& known, int at, ModelOpr* one, const std::vector<ModelOpr*>& two) {
+    known.resize(m->oprs.size(), -1);
+    if (known[(size_t)at] < 0) {
+        const float a = time_oprs(m, {one}, 10, true), b = time_oprs(m, two, 10, true);
+        known[(size_t)at] = a > 0.f && b > 0.f && a < 0.97f * b;
+    }
+    return known[(size_t)at] != 0;
+}
+
+// Which pairs a schedule may contain (a pair that may not, or measured slower, stays two kernels).
+struct Pairs {
+    bool dw_pw, pw_dw;
+};
+
+static void build_schedule(Model* m, Pairs allow) {
     m->schedule.clear();
+    for (auto* o : m->fused)
+        delete o;
+    m->fused.clear();
     const int n = (int)m->oprs.size();
     for (int i = 0; i < n; ++i)
         m->oprs[i]->first_index = i;
@@ -377,7 +414,7 @@ static void build_schedule(Model* m, bool allow_pw_dw = true) {
         }
         // A channel-wise 3x3 convolution and the pointwise convolution of its result: one kernel
         // (conv_dw_pw.hip) when nothing else reads the tensor in between and it measures faster.
-        if (!options().no_fuse_dwpw && i + 1 < n && o0->desc.kind == MEGCC_KERN_CONV && !o0->has_processed && o0->out.size() == 1 &&
+        if (allow.dw_pw && !options().no_fuse_dwpw && i + 1 < n && o0->desc.kind == MEGCC_KERN_CONV && !o0->has_processed && o0->out.size() == 1 &&
             o0->desc.attr.conv.sparse == MEGCC_SPARSE_GROUP && o0->in.size() == (o0->desc.attr.conv.with_bias ? 3u : 2u)) {
             ModelOpr* o1 = m->oprs[i + 1];
             if (o1->desc.kind == MEGCC_KERN_CONV && o1->has_processed && o1->out.size() == 1 && o1->in[0] == o0->out[0] &&
@@ -402,10 +439,8 @@ static void build_schedule(Model* m, bool allow_pw_dw = true) {
                 bool take = !shares_bytes(*f->in_ptrs[0], *f->out_ptrs[0]) &&
                             dw_pw_run(&f->desc.attr.pw_dw, f->in_ptrs.data(), (int)f->in_ptrs.size(), f->out_ptrs.data(),
                                       (int)f->out_ptrs.size(), true) == TinyNN_SUCCESS;
-                if (take && !options().fuse_dwpw) {
-                    const float one = time_oprs(m, {f}, 10), two = time_oprs(m, {o0, o1}, 10);
-                    take = one > 0.f && two > 0.f && one < 0.97f * two;
-                }
+                if (take && !options().fuse_dwpw)
+                    take = faster_as_one(m, m->dw_pw_faster, i, f, {o0, o1});
                 if (take) {
                     m->fused.push_back(f);
                     m->schedule.push_back(f);
@@ -418,7 +453,7 @@ static void build_schedule(Model* m, bool allow_pw_dw = true) {
         // A pointwise convolution and the channel-wise 3x3 convolution of its result, on images small
         // enough for a workgroup to hold one: one kernel (megcc_gfx950_pw_dw) when nothing else reads
         // the tensor in between.
-        if (allow_pw_dw && !options().no_fuse_pwdw && i + 1 < n && o0->desc.kind == MEGCC_KERN_CONV && o0->has_processed &&
+        if (allow.pw_dw && !options().no_fuse_pwdw && i + 1 < n && o0->desc.kind == MEGCC_KERN_CONV && o0->has_processed &&
             o0->out.size() == 1 && o0->in.size() == (o0->desc.attr.conv.with_bias ? 3u : 2u)) {
             ModelOpr* o1 = m->oprs[i + 1];
             if (o1->desc.kind == MEGCC_KERN_CONV && !o1->has_processed && o1->out.size() == 1 &&
@@ -449,13 +484,10 @@ static void build_schedule(Model* m, bool allow_pw_dw = true) {
                                     f->out_ptrs.data(), (int)f->out_ptrs.size());
                 // The one kernel saves a launch and the tensor's round trip, but its three phases run
                 // one after the other on a CU, so which form is faster depends on how many images
-                // there are per CU: both forms are run a few times on the tensors as they are (their
-                // contents do not matter before the first forward) and the faster one is kept. The
+                // there are per CU: both forms are timed and the faster one is kept. The
                 // switch "fusepwdw" takes the one kernel without measuring.
-                if (take && !options().fuse_pwdw) {
-                    const float one = time_oprs(m, {f}, 10), two = time_oprs(m, {o0, o1}, 10);
-                    take = one > 0.f && two > 0.f && one < 0.97f * two;
-                }
+                if (take && !options().fuse_pwdw)
+                    take = faster_as_one(m, m->pw_dw_faster, i, f, {o0, o1});
                 if (take) {
                     m->fused.push_back(f);
                     m->schedule.push_back(f);
@@ -692,9 +724,9 @@ static TinyNNStatus forward_eager(Model* m, bool overlap = false, hipEvent_t don
 }
 
 // Milliseconds per forward of eight plain-launch forwards enqueued back to back, the way a finalized
-// model runs them (two streams where the schedule has a tail) - the shorter of two such runs;
+// model runs them (two streams where the schedule has a tail) - the shortest of `reps` such runs;
 // negative when something fails.
-static float time_forwards(Model* m) {
+static float time_forwards(Model* m, int reps = 2) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
         if (e0)
@@ -703,7 +735,7 @@ static float time_forwards(Model* m) {
     }
     float best = -1.f;
     bool ok = forward_eager(m) == TinyNN_SUCCESS;
-    for (int rep = 0; ok && rep < 2; ++rep) {
+    for (int rep = 0; ok && rep < reps; ++rep) {
         float ms = -1.f;
         join_tail(m);
         ok = hipEventRecord(e0, main_stream()) == hipSuccess;
@@ -718,6 +750,107 @@ static float time_forwards(Model* m) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     return ok ? best : -1.f;
+}
+
+// The forward's kernels captured into a graph, on one stream; hipSuccess and *exec, or the forward's own status.
+static TinyNNStatus capture_forward(Model* m, hipGraph_t* graph, hipGraphExec_t* exec) {
+    *graph = nullptr;
+    *exec = nullptr;
+    join_tail(m);  // (before the capture begins: the wait refers to an event outside of it)
+    if (hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal) != hipSuccess) {
+        (void)hipGetLastError();
+        return TinyNN_SUCCESS;
+    }
+    const TinyNNStatus st = forward_eager(m);
+    hipGraph_t g = nullptr;
+    const hipError_t e = hipStreamEndCapture(stream(), &g);
+    if (st == TinyNN_SUCCESS && e == hipSuccess && g && hipGraphInstantiate(exec, g, nullptr, nullptr, 0) == hipSuccess) {
+        *graph = g;
+        return TinyNN_SUCCESS;
+    }
+    *exec = nullptr;
+    if (g)
+        (void)hipGraphDestroy(g);
+    (void)hipGetLastError();  // a failed capture must not poison the plain launches
+    return st;
+}
+
+// forward() never replays a graph of fewer kernels (the depthwise + pooling + addition chain as one kernel takes
+// 7.6 us per forward eagerly, 16.2 us as a graph)
+static bool graph_allowed(const Model* m) {
+    return !options().no_graph && m->schedule.size() >= 5;
+}
+
+// As time_forwards(), of one run of graph replays; negative where the model would not replay.
+static float time_replays(Model* m) {
+    if (!graph_allowed(m))
+        return -1.f;
+    hipGraph_t g = nullptr;
+    hipGraphExec_t exec = nullptr;
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (capture_forward(m, &g, &exec) != TinyNN_SUCCESS || !exec)
+        return -1.f;
+    float ms = -1.f;
+    bool ok = hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess &&
+              hipGraphLaunch(exec, main_stream()) == hipSuccess && hipEventRecord(e0, main_stream()) == hipSuccess;
+    for (int i = 0; ok && i < 8; ++i)
+        ok = hipGraphLaunch(exec, main_stream()) == hipSuccess;
+    ok = ok && hipEventRecord(e1, main_stream()) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
+         hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
+    (void)hipStreamSynchronize(main_stream());
+    (void)hipGraphExecDestroy(exec);
+    (void)hipGraphDestroy(g);
+    if (e0)
+        (void)hipEventDestroy(e0);
+    if (e1)
+        (void)hipEventDestroy(e1);
+    return ok ? ms / 8 : -1.f;
+}
+
+// What a forward of the schedule the pairs give costs, launched the way it would be: plainly (on two streams where
+// that applies, at the boundary that balances the kernels' times; a network large enough for that never gains from a
+// graph) or as a graph. Negative when it cannot be timed.
+static float time_schedule(Model* m, Pairs allow) {
+    reset_tail(m);
+    build_schedule(m, allow);
+    setup_tail(m);
+    const float plain = time_forwards(m, 1);
+    const float replay = plain > 0.f && m->tail_begin < 0 ? time_replays(m) : -1.f;
+    return replay > 0.f && replay < plain ? replay : plain;
+}
+
+// The schedule: with the pairs that measured faster as one kernel, unless whole forwards say otherwise. A pair judged
+// alone, kernel behind kernel, can lose in the forward: on two streams the launch it saves is hidden, and one
+// workgroup per image fills the chip worse (MobileNetV1 batch 64 with its pointwise -> channel-wise pairs as one kernel
+// 248 k img/s, as two 263 k; batch 32 the other way round).
+static void choose_schedule(Model* m) {
+    Pairs best = {true, true};
+    build_schedule(m, best);
+    auto has = [&](bool dw_pw) {
+        for (const ModelOpr* o : m->schedule)
+            if (dw_pw ? o->dw_pw : o->desc.kind == MEGCC_KERN_PW_DW)
+                return true;
+        return false;
+    };
+    if (!options().fuse_dwpw && !options().fuse_pwdw && (has(true) || has(false))) {
+        const bool both = has(true) && has(false);
+        float cost = time_schedule(m, best);
+        auto consider = [&](Pairs p) {
+            const float t = time_schedule(m, p);
+            if (t > 0.f && cost > 0.f && t < 0.98f * cost) {
+                cost = t;
+                best = p;
+            }
+        };
+        // (without channel-wise -> pointwise pairs others become possible)
+        if (both)
+            consider({true, false});
+        consider({false, true});
+        if (has(false))
+            consider({false, false});
+        reset_tail(m);
+        build_schedule(m, best);
+    }
 }
 
 }  // namespace
@@ -1056,17 +1189,15 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
         for (auto* o : m->oprs)
             o->ws.ptr = o->ws.size ? m->workspace : nullptr;
     }
-    build_schedule(m);
+    choose_schedule(m);
     setup_tail(m);
     // The balance of measured kernel times is only a starting point: one kernel more or less on the
     // tail moves MobileNetV1 batch 64 by 3 %. The boundary and its three neighbours on either side are
     // timed as whole forwards and the best one kept.
-    auto tune_tail = [&]() -> float {
-        if (m->tail_begin < 0)
-            return -1.f;
-        int best_tb = m->tail_begin;
+    if (m->tail_begin >= 0) {
+        const int tb0 = m->tail_begin;
+        int best_tb = tb0;
         float best = time_forwards(m);
-        const int tb0 = best_tb;
         for (int cand : {tb0 + 1, tb0 - 1, tb0 + 2, tb0 - 2, tb0 + 3, tb0 - 3}) {
             reset_tail(m);
             setup_tail(m, cand);
@@ -1081,33 +1212,6 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
         if (m->tail_begin != best_tb) {
             reset_tail(m);
             setup_tail(m, best_tb);
-        }
-        return best;
-    };
-    const float with = tune_tail();
-    // Pointwise -> depthwise pairs were judged one by one, kernel behind kernel on one stream. With
-    // two streams the launch floors they save are hidden anyway and their one-workgroup-per-image
-    // form fills the chip worse (MobileNetV1 batch 64: 248 k img/s with the pairs as one kernel, 263 k
-    // as two; batch 32 the other way round): the whole forward is timed both ways and the faster
-    // schedule kept.
-    bool has_pair = false;
-    bool has_dw_pw = false;  // (a pair that saves work, not only a launch: judged well enough one by one)
-    for (const ModelOpr* o : m->schedule) {
-        has_pair = has_pair || o->desc.kind == MEGCC_KERN_PW_DW;
-        has_dw_pw = has_dw_pw || o->dw_pw;
-    }
-    has_pair = has_pair && !has_dw_pw;
-    if (with > 0.f && has_pair && !options().fuse_pwdw) {
-        const std::vector<ModelOpr*> fused_schedule = m->schedule;
-        const int fused_tb = m->tail_begin;
-        reset_tail(m);
-        build_schedule(m, false);
-        setup_tail(m);
-        const float without = tune_tail();
-        if (!(without > 0.f && without < 0.98f * with)) {
-            reset_tail(m);
-            m->schedule = fused_schedule;
-            setup_tail(m, fused_tb);
         }
     }
     m->finalized = true;
@@ -1232,9 +1336,7 @@ TinyNNStatus megcc_gfx950_model_forward(void* model) {
         return forward_eager(m, true);
     // ---- undecided: the first ten forwards (1: plain; 2, 3, 7, 8: timed plain launches; 4: the capture
     //      and its first replay; 5, 6, 9, 10: timed replays)
-    // (schedules of fewer than 5 kernels stay eager without asking: the depthwise + pooling + addition
-    //  chain as one kernel takes 7.6 us per forward eagerly, 16.2 us as a graph)
-    if (options().no_graph || m->schedule.size() < 5) {
+    if (!graph_allowed(m)) {
         m->graph_state = -1;
         return forward_eager(m);
     }
@@ -1276,22 +1378,11 @@ TinyNNStatus megcc_gfx950_model_forward(void* model) {
     if (m->forwards <= 3 || (m->graph_exec && (m->forwards == 7 || m->forwards == 8)))
         return timed(false, m->forwards == 3 || m->forwards == 8, &m->eager_ms);
     if (m->forwards == 4) {
-        join_tail(m);  // (before the capture begins: the wait refers to an event outside of it)
-        if (hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal) == hipSuccess) {
-            TinyNNStatus st = forward_eager(m);
-            hipGraph_t g = nullptr;
-            hipError_t e = hipStreamEndCapture(stream(), &g);
-            if (st == TinyNN_SUCCESS && e == hipSuccess && g &&
-                hipGraphInstantiate(&m->graph_exec, g, nullptr, nullptr, 0) == hipSuccess) {
-                m->graph = g;
-                return replay();
-            }
-            if (g)
-                (void)hipGraphDestroy(g);
-            (void)hipGetLastError();  // a failed capture must not poison the eager path
-            if (st != TinyNN_SUCCESS)
-                return st;
-        }
+        const TinyNNStatus st = capture_forward(m, &m->graph, &m->graph_exec);
+        if (m->graph_exec)
+            return replay();
+        if (st != TinyNN_SUCCESS)
+            return st;
         m->graph_state = -1;
         return forward_eager(m);
     }
