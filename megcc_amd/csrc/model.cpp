@@ -271,19 +271,9 @@ static TinyNNStatus call_opr(Model* m, ModelOpr* o) {
             &o->desc, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(), (int)o->out_ptrs.size(), &o->ws,
             &m->opt);
 }
-// One wave that looks at the 100 MHz clock until `ticks` have gone by (each look sleeps 64 cycles or more: at most
-// `looks` of them whatever the clock does).
-__global__ void hold_kernel(long long ticks, int looks) {
-    const long long t0 = wall_clock64();
-    while (looks-- > 0 && wall_clock64() - t0 < ticks)
-        __builtin_amdgcn_s_sleep(8);
-}
-
 // Milliseconds `iters` back-to-back rounds of the operators in `ops` take on the library stream
 // (after one untimed round), or a negative value when a launch fails or an operand has no memory.
-// `device_only`: the device is held until the host has enqueued the rounds, so that the time is the kernels' own also
-// where they are shorter than a launch takes the host.
-static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters, bool device_only = false) {
+static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters) {
     for (const ModelOpr* o : ops) {
         for (const Tensor* t : o->in_ptrs)
             if (!t->ptr)
@@ -306,11 +296,6 @@ static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters, b
     }
     float ms = -1.f;
     bool ok = round();
-    if (device_only && ok) {  // (a launch takes the host 3 - 5 us)
-        const int us = 20 + 8 * iters * (int)ops.size();
-        hipLaunchKernelGGL(hold_kernel, dim3(1), dim3(64), 0, stream(), 100LL * us, 8 * us);
-        ok = check_launch("hold") == TinyNN_SUCCESS;
-    }
     ok = ok && hipEventRecord(e0, stream()) == hipSuccess;
     for (int i = 0; ok && i < iters; ++i)
         ok = round();
@@ -321,13 +306,14 @@ static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters, b
     return ok ? ms : -1.f;
 }
 
-// `one` in place of `two`: the kernels' own times, measured once per pair (a few rounds on the tensors as they are;
-// their contents do not matter before the first forward). At small sizes plain launches back to back would time the
-// host instead, and the pair always win: it is one launch fewer.
+// `one` in place of `two`: timed once per pair, launched as plain forwards launch them - where the kernels are shorter
+// than a launch takes the host, the launch saved is what counts. (By the kernels' own times, the device held until the
+// host was ahead, MobileNetV1 at batch 10 to 12 kept one more pair apart and took 133 us for 121.) A few rounds on
+// the tensors as they are; their contents do not matter before the first forward.
 static bool faster_as_one(Model* m, std::vector<signed char>& known, int at, ModelOpr* one, const std::vector<ModelOpr*>& two) {
     known.resize(m->oprs.size(), -1);
     if (known[(size_t)at] < 0) {
-        const float a = time_oprs(m, {one}, 10, true), b = time_oprs(m, two, 10, true);
+        const float a = time_oprs(m, {one}, 10), b = time_oprs(m, two, 10);
         known[(size_t)at] = a > 0.f && b > 0.f && a < 0.97f * b;
     }
     return known[(size_t)at] != 0;
@@ -752,105 +738,63 @@ static float time_forwards(Model* m, int reps = 2) {
     return ok ? best : -1.f;
 }
 
-// The forward's kernels captured into a graph, on one stream; hipSuccess and *exec, or the forward's own status.
-static TinyNNStatus capture_forward(Model* m, hipGraph_t* graph, hipGraphExec_t* exec) {
-    *graph = nullptr;
-    *exec = nullptr;
-    join_tail(m);  // (before the capture begins: the wait refers to an event outside of it)
-    if (hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal) != hipSuccess) {
-        (void)hipGetLastError();
-        return TinyNN_SUCCESS;
-    }
-    const TinyNNStatus st = forward_eager(m);
-    hipGraph_t g = nullptr;
-    const hipError_t e = hipStreamEndCapture(stream(), &g);
-    if (st == TinyNN_SUCCESS && e == hipSuccess && g && hipGraphInstantiate(exec, g, nullptr, nullptr, 0) == hipSuccess) {
-        *graph = g;
-        return TinyNN_SUCCESS;
-    }
-    *exec = nullptr;
-    if (g)
-        (void)hipGraphDestroy(g);
-    (void)hipGetLastError();  // a failed capture must not poison the plain launches
-    return st;
-}
-
-// forward() never replays a graph of fewer kernels (the depthwise + pooling + addition chain as one kernel takes
-// 7.6 us per forward eagerly, 16.2 us as a graph)
-static bool graph_allowed(const Model* m) {
-    return !options().no_graph && m->schedule.size() >= 5;
-}
-
-// As time_forwards(), of one run of graph replays; negative where the model would not replay.
-static float time_replays(Model* m) {
-    if (!graph_allowed(m))
-        return -1.f;
-    hipGraph_t g = nullptr;
-    hipGraphExec_t exec = nullptr;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (capture_forward(m, &g, &exec) != TinyNN_SUCCESS || !exec)
-        return -1.f;
-    float ms = -1.f;
-    bool ok = hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess &&
-              hipGraphLaunch(exec, main_stream()) == hipSuccess && hipEventRecord(e0, main_stream()) == hipSuccess;
-    for (int i = 0; ok && i < 8; ++i)
-        ok = hipGraphLaunch(exec, main_stream()) == hipSuccess;
-    ok = ok && hipEventRecord(e1, main_stream()) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
-         hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
-    (void)hipStreamSynchronize(main_stream());
-    (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(g);
-    if (e0)
-        (void)hipEventDestroy(e0);
-    if (e1)
-        (void)hipEventDestroy(e1);
-    return ok ? ms / 8 : -1.f;
-}
-
-// What a forward of the schedule the pairs give costs, launched the way it would be: plainly (on two streams where
-// that applies, at the boundary that balances the kernels' times; a network large enough for that never gains from a
-// graph) or as a graph. Negative when it cannot be timed.
-static float time_schedule(Model* m, Pairs allow) {
-    reset_tail(m);
-    build_schedule(m, allow);
-    setup_tail(m);
-    const float plain = time_forwards(m, 1);
-    const float replay = plain > 0.f && m->tail_begin < 0 ? time_replays(m) : -1.f;
-    return replay > 0.f && replay < plain ? replay : plain;
-}
-
-// The schedule: with the pairs that measured faster as one kernel, unless whole forwards say otherwise. A pair judged
-// alone, kernel behind kernel, can lose in the forward: on two streams the launch it saves is hidden, and one
-// workgroup per image fills the chip worse (MobileNetV1 batch 64 with its pointwise -> channel-wise pairs as one kernel
-// 248 k img/s, as two 263 k; batch 32 the other way round).
-static void choose_schedule(Model* m) {
+// The schedule: with the pairs that measured faster as one kernel, unless whole forwards say otherwise. On two streams a
+// pair judged alone, kernel behind kernel, can lose: the launch it saves is hidden there, and one workgroup per
+// image fills the chip worse (MobileNetV1 batch 64 with its pointwise -> channel-wise pairs as one kernel 248 k img/s,
+// as two 263 k; batch 32 the other way round). A network bound by launches runs on one, as the pairs were
+// timed (MobileNetV1 as chosen / without channel-wise -> pointwise pairs, us: batch 1 113 / 115, 4 125 / 130, 8 129 / 140).
+struct Choice {
+    Pairs pairs;
+    int tail_begin;  // where the second stream takes over, -1: it does not
+};
+static Choice choose_schedule(Model* m) {
     Pairs best = {true, true};
     build_schedule(m, best);
-    auto has = [&](bool dw_pw) {
-        for (const ModelOpr* o : m->schedule)
-            if (dw_pw ? o->dw_pw : o->desc.kind == MEGCC_KERN_PW_DW)
-                return true;
-        return false;
-    };
-    if (!options().fuse_dwpw && !options().fuse_pwdw && (has(true) || has(false))) {
-        const bool both = has(true) && has(false);
-        float cost = time_schedule(m, best);
-        auto consider = [&](Pairs p) {
-            const float t = time_schedule(m, p);
-            if (t > 0.f && cost > 0.f && t < 0.98f * cost) {
-                cost = t;
-                best = p;
-            }
-        };
-        // (without channel-wise -> pointwise pairs others become possible)
-        if (both)
-            consider({true, false});
-        consider({false, true});
-        if (has(false))
-            consider({false, false});
-        reset_tail(m);
-        build_schedule(m, best);
+    setup_tail(m);
+    int tail_begin = m->tail_begin;
+    bool dw_pw = false, pw_dw = false;
+    for (const ModelOpr* o : m->schedule) {
+        dw_pw = dw_pw || o->dw_pw;
+        pw_dw = pw_dw || o->desc.kind == MEGCC_KERN_PW_DW;
     }
+    if (tail_begin < 0 || (!dw_pw && !pw_dw) || options().fuse_dwpw || options().fuse_pwdw)
+        return {best, tail_begin};
+    // a forward with these pairs, at the boundary that balances the kernels' times
+    auto time_pairs = [&](Pairs p) {
+        reset_tail(m);
+        build_schedule(m, p);
+        setup_tail(m);
+        return time_forwards(m, 1);
+    };
+    const float first = time_forwards(m, 1);
+    float cost = first;
+    Pairs winner = best;
+    std::vector<Pairs> others = {{false, true}};  // (others become possible without channel-wise -> pointwise pairs)
+    if (pw_dw)
+        others.push_back({false, false});
+    if (pw_dw && dw_pw)
+        others.push_back({true, false});
+    for (const Pairs& p : others) {
+        const float t = time_pairs(p);
+        if (t > 0.f && t < cost) {
+            cost = t;
+            winner = p;
+        }
+    }
+    // (the first one was timed while the clocks went up: once more, both, before it is given up)
+    if (cost < 0.97f * first) {
+        const float again = time_pairs(best);
+        cost = std::min(cost, time_pairs(winner));
+        if (cost > 0.f && cost < 0.97f * std::min(first, again)) {
+            best = winner;
+            tail_begin = m->tail_begin;
+        }
+    }
+    reset_tail(m);
+    build_schedule(m, best);
+    if (tail_begin >= 0)
+        setup_tail(m, tail_begin);
+    return {best, m->tail_begin};
 }
 
 }  // namespace
@@ -1190,7 +1134,6 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
             o->ws.ptr = o->ws.size ? m->workspace : nullptr;
     }
     choose_schedule(m);
-    setup_tail(m);
     // The balance of measured kernel times is only a starting point: one kernel more or less on the
     // tail moves MobileNetV1 batch 64 by 3 %. The boundary and its three neighbours on either side are
     // timed as whole forwards and the best one kept.
@@ -1336,7 +1279,9 @@ TinyNNStatus megcc_gfx950_model_forward(void* model) {
         return forward_eager(m, true);
     // ---- undecided: the first ten forwards (1: plain; 2, 3, 7, 8: timed plain launches; 4: the capture
     //      and its first replay; 5, 6, 9, 10: timed replays)
-    if (!graph_allowed(m)) {
+    // (schedules of fewer than 5 kernels stay eager without asking: the depthwise + pooling + addition
+    //  chain as one kernel takes 7.6 us per forward eagerly, 16.2 us as a graph)
+    if (options().no_graph || m->schedule.size() < 5) {
         m->graph_state = -1;
         return forward_eager(m);
     }
@@ -1378,11 +1323,22 @@ TinyNNStatus megcc_gfx950_model_forward(void* model) {
     if (m->forwards <= 3 || (m->graph_exec && (m->forwards == 7 || m->forwards == 8)))
         return timed(false, m->forwards == 3 || m->forwards == 8, &m->eager_ms);
     if (m->forwards == 4) {
-        const TinyNNStatus st = capture_forward(m, &m->graph, &m->graph_exec);
-        if (m->graph_exec)
-            return replay();
-        if (st != TinyNN_SUCCESS)
-            return st;
+        join_tail(m);  // (before the capture begins: the wait refers to an event outside of it)
+        if (hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal) == hipSuccess) {
+            TinyNNStatus st = forward_eager(m);
+            hipGraph_t g = nullptr;
+            hipError_t e = hipStreamEndCapture(stream(), &g);
+            if (st == TinyNN_SUCCESS && e == hipSuccess && g &&
+                hipGraphInstantiate(&m->graph_exec, g, nullptr, nullptr, 0) == hipSuccess) {
+                m->graph = g;
+                return replay();
+            }
+            if (g)
+                (void)hipGraphDestroy(g);
+            (void)hipGetLastError();  // a failed capture must not poison the eager path
+            if (st != TinyNN_SUCCESS)
+                return st;
+        }
         m->graph_state = -1;
         return forward_eager(m);
     }
