@@ -62,8 +62,14 @@ struct Model {
     // one kernel (`fused` owns the replacements); run_opr, nr_opr and the memory plan keep the
     // operator list as it was given
     std::vector<ModelOpr*> schedule, fused;
-    // per operator: whether the pair that begins there measured faster as one kernel (-1: not measured)
-    std::vector<signed char> dw_pw_faster, pw_dw_faster;
+    // per operator: whether the pair that begins there measured faster as one kernel, and by how much; what the schedule's
+    // kernels take one by one (both in microseconds, as far as they were timed)
+    struct PairTime {
+        bool known = false, faster = false;
+        double gain_us = 0;
+    };
+    std::vector<PairTime> dw_pw_time, pw_dw_time;
+    double schedule_us = 0;
     void* arena = nullptr;
     size_t arena_bytes = 0;
     // one scratch buffer shared by all operators (they run one after the other on one stream),
@@ -310,13 +316,16 @@ static float time_oprs(Model* m, const std::vector<ModelOpr*>& ops, int iters) {
 // than a launch takes the host, the launch saved is what counts. (By the kernels' own times, the device held until the
 // host was ahead, MobileNetV1 at batch 10 to 12 kept one more pair apart and took 133 us for 121.) A few rounds on
 // the tensors as they are; their contents do not matter before the first forward.
-static bool faster_as_one(Model* m, std::vector<signed char>& known, int at, ModelOpr* one, const std::vector<ModelOpr*>& two) {
-    known.resize(m->oprs.size(), -1);
-    if (known[(size_t)at] < 0) {
+static bool faster_as_one(Model* m, std::vector<Model::PairTime>& times, int at, ModelOpr* one, const std::vector<ModelOpr*>& two) {
+    times.resize(m->oprs.size());
+    Model::PairTime& p = times[(size_t)at];
+    if (!p.known) {
         const float a = time_oprs(m, {one}, 10), b = time_oprs(m, two, 10);
-        known[(size_t)at] = a > 0.f && b > 0.f && a < 0.97f * b;
+        p.known = true;
+        p.faster = a > 0.f && b > 0.f && a < 0.97f * b;
+        p.gain_us = 1e3 / 10 * (b - a);
     }
-    return known[(size_t)at] != 0;
+    return p.faster;
 }
 
 // Which pairs a schedule may contain (a pair that may not, or measured slower, stays two kernels).
@@ -426,7 +435,7 @@ static void build_schedule(Model* m, Pairs allow) {
                             dw_pw_run(&f->desc.attr.pw_dw, f->in_ptrs.data(), (int)f->in_ptrs.size(), f->out_ptrs.data(),
                                       (int)f->out_ptrs.size(), true) == TinyNN_SUCCESS;
                 if (take && !options().fuse_dwpw)
-                    take = faster_as_one(m, m->dw_pw_faster, i, f, {o0, o1});
+                    take = faster_as_one(m, m->dw_pw_time, i, f, {o0, o1});
                 if (take) {
                     m->fused.push_back(f);
                     m->schedule.push_back(f);
@@ -473,7 +482,7 @@ static void build_schedule(Model* m, Pairs allow) {
                 // there are per CU: both forms are timed and the faster one is kept. The
                 // switch "fusepwdw" takes the one kernel without measuring.
                 if (take && !options().fuse_pwdw)
-                    take = faster_as_one(m, m->pw_dw_faster, i, f, {o0, o1});
+                    take = faster_as_one(m, m->pw_dw_time, i, f, {o0, o1});
                 if (take) {
                     m->fused.push_back(f);
                     m->schedule.push_back(f);
@@ -595,6 +604,7 @@ static void setup_tail(Model* m, int forced = -1) {
             }
             total += us[(size_t)s];
         }
+        m->schedule_us = total;
         // A network whose kernels average under 6 us is bound by launches, not by the device: two
         // streams then gain or lose a quarter from run to run (MobileNetV1 batch 1: 7.2 k ... 9.9 k
         // img/s) where one stream or a graph replay is steady. One stream.
@@ -741,7 +751,8 @@ static float time_forwards(Model* m, int reps = 2) {
 // The schedule: with the pairs that measured faster as one kernel, unless whole forwards say otherwise. On two streams a
 // pair judged alone, kernel behind kernel, can lose: the launch it saves is hidden there, and one workgroup per
 // image fills the chip worse (MobileNetV1 batch 64 with its pointwise -> channel-wise pairs as one kernel 248 k img/s,
-// as two 263 k; batch 32 the other way round). A network bound by launches runs on one, as the pairs were
+// as two 263 k; batch 32 the other way round). Channel-wise -> pointwise pairs whose gains make up a tenth of the
+// forward are not asked about again: what overlap took back was 6 %, and each question costs some 17 forwards. A network bound by launches runs on one, as the pairs were
 // timed (MobileNetV1 as chosen / without channel-wise -> pointwise pairs, us: batch 1 113 / 115, 4 125 / 130, 8 129 / 140).
 struct Choice {
     Pairs pairs;
@@ -753,11 +764,18 @@ static Choice choose_schedule(Model* m) {
     setup_tail(m);
     int tail_begin = m->tail_begin;
     bool dw_pw = false, pw_dw = false;
+    double gain = 0;
     for (const ModelOpr* o : m->schedule) {
-        dw_pw = dw_pw || o->dw_pw;
         pw_dw = pw_dw || o->desc.kind == MEGCC_KERN_PW_DW;
+        dw_pw = dw_pw || o->dw_pw;
+        if (o->dw_pw && (size_t)o->first_index < m->dw_pw_time.size())
+            gain += m->dw_pw_time[(size_t)o->first_index].gain_us;
     }
-    if (tail_begin < 0 || (!dw_pw && !pw_dw) || options().fuse_dwpw || options().fuse_pwdw)
+    const bool doubt = dw_pw && gain < 0.1 * (m->schedule_us + gain);
+    // (kernels of under 8 us: two-stream forwards still vary by a quarter from run to run, and one in three comparisons
+    //  at batch 8 and 10 ended with no pairs, 135 us for 129)
+    if (tail_begin < 0 || m->schedule_us < 8.0 * (double)m->schedule.size() || (!doubt && !pw_dw) || options().fuse_dwpw ||
+        options().fuse_pwdw)
         return {best, tail_begin};
     // a forward with these pairs, at the boundary that balances the kernels' times
     auto time_pairs = [&](Pairs p) {
@@ -769,11 +787,13 @@ static Choice choose_schedule(Model* m) {
     const float first = time_forwards(m, 1);
     float cost = first;
     Pairs winner = best;
-    std::vector<Pairs> others = {{false, true}};  // (others become possible without channel-wise -> pointwise pairs)
+    std::vector<Pairs> others;
     if (pw_dw)
-        others.push_back({false, false});
-    if (pw_dw && dw_pw)
         others.push_back({true, false});
+    if (doubt)
+        others.push_back({false, true});  // (other pairs become possible without the channel-wise -> pointwise ones)
+    if (pw_dw && doubt)
+        others.push_back({false, false});
     for (const Pairs& p : others) {
         const float t = time_pairs(p);
         if (t > 0.f && t < cost) {
