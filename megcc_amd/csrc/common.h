@@ -90,6 +90,10 @@ TinyNNStatus noalloc_scratch_setup();
 // (model runtime only); check_only: whether the kernel takes the pair.
 TinyNNStatus dw_pw_run(
         const MegccPwDwAttr* attr, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, bool check_only);
+// whether it could take the pair, before memory is planned and the pointwise filter packed
+bool dw_pw_takes(
+        const MegccConvAttr* dw_attr, const MegccConvAttr* pw_attr, const Tensor* src, const Tensor* dw_flt, const Tensor* mid,
+        const Tensor* pw_flt, const Tensor* dst);
 
 // After a kernel launch: surfaces launch-configuration errors as TinyNN_ERROR_RUNTIME.
 TinyNNStatus check_launch(const char* what);

@@ -859,6 +859,17 @@ extern "C" TinyNNStatus megcc_gfx950_pw_dw(
 // inputs: source, channel-wise filter [, bias], packed pointwise filter [, bias]; attr.mid_scale is the scale
 // of the tensor in between. check_only: TinyNN_SUCCESS when the kernel takes the pair.
 namespace mg {
+bool dw_pw_takes(
+        const MegccConvAttr* dw_attr, const MegccConvAttr* pw_attr, const Tensor* src, const Tensor* dw_flt, const Tensor* mid,
+        const Tensor* pw_flt, const Tensor* dst) {
+    ConvGeom dw, pw;
+    return is_q8(src) && is_q8(dw_flt) && is_q8(mid) && is_q8(pw_flt) && is_q8(dst) && dw_attr->sparse == MEGCC_SPARSE_GROUP &&
+           pw_attr->sparse == MEGCC_SPARSE_DENSE && !is_packed_filter(dw_flt) && !is_packed_filter(pw_flt) &&
+           make_geom(dw_attr, src, dw_flt, mid, false, 0, &dw) == TinyNN_SUCCESS &&
+           make_geom(pw_attr, mid, pw_flt, dst, false, 0, &pw) == TinyNN_SUCCESS &&
+           conv_dw_pw_supported(dw, pw, nullptr, nullptr) && conv_mfma_supported(pw);
+}
+
 TinyNNStatus dw_pw_run(
         const MegccPwDwAttr* a, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, bool check_only) {
     const char* who = "dw_pw";

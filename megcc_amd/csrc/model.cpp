@@ -38,6 +38,8 @@ struct ModelTensor {
     size_t alias_offset = 0;  // MemForward: bytes from the start of that tensor
     int def = -1, last = -1;
     void* owned = nullptr;  // weights: device allocation owned by the model
+    // between the two layers of a pair that runs as one kernel: only run_opr writes and reads it
+    bool between = false;
 };
 
 struct ModelOpr {
@@ -70,6 +72,9 @@ struct Model {
     };
     std::vector<PairTime> dw_pw_time, pw_dw_time;
     double schedule_us = 0;
+    // per operator: the channel-wise -> pointwise pair that begins there may run as one kernel, so the memory plan keeps
+    // the channel-wise layer's source until the pointwise layer is through
+    std::vector<char> dw_pw_may;
     void* arena = nullptr;
     size_t arena_bytes = 0;
     // one scratch buffer shared by all operators (they run one after the other on one stream),
@@ -194,11 +199,8 @@ bool plan_memory(Model* m) {
             o1->in.empty() || o0->out.size() != 1 || o1->in[0] != o0->out[0])
             continue;
         const MegccConvAttr &a = o0->desc.attr.conv, &b = o1->desc.attr.conv;
-        // The same for a channel-wise layer in front of a pointwise one (conv_dw_pw.hip). Not under
-        // "nopipeline", which keeps the plan to the operators as they are.
-        if (!options().no_fuse_dwpw && !options().no_pipeline && a.format == MEGCC_FMT_NCHW44 && a.sparse == MEGCC_SPARSE_GROUP &&
-            a.kernel_h == 3 && a.kernel_w == 3 && b.format == MEGCC_FMT_NCHW44 && b.sparse == MEGCC_SPARSE_DENSE && b.kernel_h == 1 &&
-            b.kernel_w == 1 && b.stride_h == 1 && b.stride_w == 1)
+        // The same for a channel-wise layer in front of a pointwise one (conv_dw_pw.hip).
+        if (i < m->dw_pw_may.size() && m->dw_pw_may[i])
             keep_until[root_of(m, o0->in[0])] = (int)i + 1;
         if (!options().no_fuse_pwdw && a.format == MEGCC_FMT_NCHW44 && a.sparse == MEGCC_SPARSE_DENSE && a.kernel_h == 1 && a.kernel_w == 1 &&
             a.stride_h == 1 && a.stride_w == 1 && a.pad_h == 0 && a.pad_w == 0 && b.format == MEGCC_FMT_NCHW44 &&
@@ -228,7 +230,7 @@ bool plan_memory(Model* m) {
     std::vector<int> ids;
     for (size_t i = 0; i < m->tensors.size(); ++i) {
         ModelTensor* t = m->tensors[i];
-        if (t->is_weight || t->is_input || t->alias_of >= 0 || t->def < 0)
+        if (t->is_weight || t->is_input || t->alias_of >= 0 || t->def < 0 || t->between)
             continue;
         MemInterval iv;
         iv.begin = pinned[i] ? 0 : (size_t)t->def;
@@ -243,8 +245,45 @@ bool plan_memory(Model* m) {
         return false;
     for (size_t k = 0; k < ids.size(); ++k)
         m->tensors[ids[k]]->t.offset = offsets[k];
-    m->arena_bytes = total;
+    // one place for all tensors inside fused pairs: operators run one by one use it one after the other
+    size_t between = 0;
+    for (ModelTensor* t : m->tensors)
+        if (t->between) {
+            t->t.offset = align_up(total, m->dev.alignment);
+            between = std::max(between, tensor_bytes(t->t));
+        }
+    m->arena_bytes = between ? align_up(total, m->dev.alignment) + align_up(between, m->dev.alignment) : total;
     return true;
+}
+
+// how often each tensor's memory is read
+static std::vector<int> count_readers(const Model* m) {
+    std::vector<int> readers(m->tensors.size(), 0);
+    for (const ModelOpr* o : m->oprs)
+        for (int id : o->in)
+            ++readers[root_of(m, id)];
+    return readers;
+}
+// a tensor only one chain of operators touches: its own memory, `nr` readers, neither input, output nor weight
+static bool chain_only(const Model* m, const std::vector<int>& readers, int id, int nr) {
+    const ModelTensor* t = m->tensors[id];
+    return t->alias_of < 0 && !t->is_input && !t->is_output && !t->is_weight && readers[id] == nr;
+}
+
+// Fills dw_pw_may before the memory plan. Not under "nopipeline", which keeps the plan to the operators as they are.
+static void find_dw_pw(Model* m) {
+    m->dw_pw_may.assign(m->oprs.size(), 0);
+    if (m->preplanned || options().no_fuse_dwpw || options().no_pipeline)
+        return;
+    const std::vector<int> readers = count_readers(m);
+    for (size_t i = 0; i + 1 < m->oprs.size(); ++i) {
+        const ModelOpr *o0 = m->oprs[i], *o1 = m->oprs[i + 1];
+        if (o0->desc.kind != MEGCC_KERN_CONV || o1->desc.kind != MEGCC_KERN_CONV || o0->in.size() < 2 || o1->in.size() < 2 ||
+            o0->out.size() != 1 || o1->out.size() != 1 || o1->in[0] != o0->out[0] || !chain_only(m, readers, o0->out[0], 1))
+            continue;
+        m->dw_pw_may[i] = dw_pw_takes(&o0->desc.attr.conv, &o1->desc.attr.conv, &m->tensors[o0->in[0]]->t, &m->tensors[o0->in[1]]->t,
+                                      &m->tensors[o0->out[0]]->t, &m->tensors[o1->in[1]]->t, &m->tensors[o1->out[0]]->t);
+    }
 }
 
 // ---- forward schedule ----------------------------------------------------------------------------
@@ -341,15 +380,8 @@ static void build_schedule(Model* m, Pairs allow) {
     const int n = (int)m->oprs.size();
     for (int i = 0; i < n; ++i)
         m->oprs[i]->first_index = i;
-    std::vector<int> readers(m->tensors.size(), 0);
-    for (auto* o : m->oprs)
-        for (int id : o->in)
-            ++readers[root_of(m, id)];
-    // a tensor only this chain touches: its own memory, `nr` readers, neither input, output nor weight
-    auto temp = [&](int id, int nr) {
-        const ModelTensor* t = m->tensors[id];
-        return t->alias_of < 0 && !t->is_input && !t->is_output && !t->is_weight && readers[id] == nr;
-    };
+    const std::vector<int> readers = count_readers(m);
+    auto temp = [&](int id, int nr) { return chain_only(m, readers, id, nr); };
     auto is_ew = [](const ModelOpr* o, MegccElemwiseMode mode, size_t nin) {
         return o->desc.kind == MEGCC_KERN_ELEMWISE && o->desc.attr.elemwise == mode &&
                o->in.size() == nin && o->out.size() == 1;
@@ -817,6 +849,68 @@ static Choice choose_schedule(Model* m) {
     return {best, m->tail_begin};
 }
 
+// Memory for the arena as planned, and everybody's place in it.
+static TinyNNStatus place_tensors(Model* m) {
+    m->arena = m->dev.malloc(m->arena_bytes ? m->arena_bytes : 1);
+    MG_REQUIRE(m->arena, TinyNN_ERROR_MEMORY_MALLOC, "model_finalize: arena of %zu bytes", m->arena_bytes);
+    for (auto* t : m->tensors)
+        if (!t->is_weight && !t->is_input && t->alias_of < 0)
+            t->t.ptr = (char*)m->arena + t->t.offset;
+    for (size_t i = 0; i < m->tensors.size(); ++i)
+        if (m->tensors[i]->alias_of >= 0) {
+            // a chain of views adds up its offsets (output->ptr = input->ptr + offset,
+            // runtime/src/vm/memforward.c:43-53)
+            size_t shift = 0;
+            int id = (int)i;
+            while (m->tensors[id]->alias_of >= 0) {
+                shift += m->tensors[id]->alias_offset;
+                id = m->tensors[id]->alias_of;
+            }
+            const Tensor& r = m->tensors[id]->t;
+            m->tensors[i]->t.ptr = (char*)r.ptr + shift;
+            m->tensors[i]->t.offset = r.offset + shift;
+        }
+    return TinyNN_SUCCESS;
+}
+
+// The plan the pairs were measured under has room for both forms of each: sources that live one operator longer and
+// the tensors in between (MobileNetV1 batch 256: 756 MB). With the choice made, neither is needed for the pairs that stay
+// two kernels, nor the second for those that run as one - but for one place that run_opr can use. `chosen`: what
+// the schedule was built with.
+static TinyNNStatus plan_again(Model* m, const Choice& chosen) {
+    if (std::find(m->dw_pw_may.begin(), m->dw_pw_may.end(), 1) == m->dw_pw_may.end())
+        return TinyNN_SUCCESS;
+    reset_tail(m);
+    std::vector<char> one(m->oprs.size(), 0);
+    for (const ModelOpr* o : m->schedule)
+        if (o->dw_pw)
+            one[(size_t)o->first_index] = 1;
+    m->dw_pw_may = one;
+    for (size_t i = 0; i < one.size(); ++i)
+        if (one[i])
+            m->tensors[m->oprs[i]->out[0]]->between = true;
+    MG_REQUIRE(plan_memory(m), TinyNN_ERROR_INVALID_LAYOUT, "model_finalize: memory plan");
+    TinyNNStatus st = megcc_gfx950_wait();
+    if (st != TinyNN_SUCCESS)
+        return st;
+    m->dev.free(m->arena);
+    m->arena = nullptr;
+    st = place_tensors(m);
+    if (st != TinyNN_SUCCESS)
+        return st;
+    // (the same pairs: their times are known, and their sources and results share no byte under this plan either)
+    build_schedule(m, chosen.pairs);
+    if (chosen.tail_begin >= 0)
+        setup_tail(m, chosen.tail_begin);
+    for (const ModelOpr* o : m->schedule) {
+        for (const Tensor* t : o->in_ptrs)
+            for (const ModelTensor* b : m->tensors)
+                MG_REQUIRE(!b->between || t != &b->t, TinyNN_ERROR_RUNTIME, "model_finalize: %s reads what was planned away",
+                           o->symbol.c_str());
+    }
+    return TinyNN_SUCCESS;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1056,42 +1150,23 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
     //  may get for themselves - 128 MB or 85 % of that arena, whichever is more: the balanced tail of a
     //  MobileNetV1 needs about that at every batch, and more only cost cache reuse)
     m->tail_opr_begin = -1;
+    find_dw_pw(m);
     MG_REQUIRE(plan_memory(m), TinyNN_ERROR_INVALID_LAYOUT,
                "model_finalize: memory plan");
     choose_tail(m, std::max((size_t)128 << 20, (size_t)(0.85 * (double)m->arena_bytes)));
     MG_REQUIRE(plan_memory(m), TinyNN_ERROR_INVALID_LAYOUT,
                "model_finalize: memory plan (alignment %zu)", (size_t)m->dev.alignment);
-    m->arena = m->dev.malloc(m->arena_bytes ? m->arena_bytes : 1);
-    MG_REQUIRE(m->arena, TinyNN_ERROR_MEMORY_MALLOC, "model_finalize: arena of %zu bytes",
-               m->arena_bytes);
-    for (auto* t : m->tensors) {
-        if (t->is_weight || t->alias_of >= 0)
-            continue;
-        if (t->is_input) {
+    for (auto* t : m->tensors)
+        if (!t->is_weight && t->alias_of < 0 && t->is_input) {
             // user memory in the TinyNN runtime (runtime/src/init.c:456-460); here a device
             // buffer of its own that set_input fills
             t->owned = m->dev.malloc(t->t.size ? t->t.size : 1);
-            MG_REQUIRE(t->owned, TinyNN_ERROR_MEMORY_MALLOC, "model_finalize: input of %zu bytes",
-                       (size_t)t->t.size);
+            MG_REQUIRE(t->owned, TinyNN_ERROR_MEMORY_MALLOC, "model_finalize: input of %zu bytes", (size_t)t->t.size);
             t->t.ptr = t->owned;
-        } else {
-            t->t.ptr = (char*)m->arena + t->t.offset;
         }
-    }
-    for (size_t i = 0; i < m->tensors.size(); ++i)
-        if (m->tensors[i]->alias_of >= 0) {
-            // a chain of views adds up its offsets (output->ptr = input->ptr + offset,
-            // runtime/src/vm/memforward.c:43-53)
-            size_t shift = 0;
-            int id = (int)i;
-            while (m->tensors[id]->alias_of >= 0) {
-                shift += m->tensors[id]->alias_offset;
-                id = m->tensors[id]->alias_of;
-            }
-            const Tensor& r = m->tensors[id]->t;
-            m->tensors[i]->t.ptr = (char*)r.ptr + shift;
-            m->tensors[i]->t.offset = r.offset + shift;
-        }
+    TinyNNStatus placed = place_tensors(m);
+    if (placed != TinyNN_SUCCESS)
+        return placed;
     for (auto* o : m->oprs) {
         for (int id : o->in)
             o->in_ptrs.push_back(&m->tensors[id]->t);
@@ -1153,7 +1228,9 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
         for (auto* o : m->oprs)
             o->ws.ptr = o->ws.size ? m->workspace : nullptr;
     }
-    choose_schedule(m);
+    placed = plan_again(m, choose_schedule(m));
+    if (placed != TinyNN_SUCCESS)
+        return placed;
     // The balance of measured kernel times is only a starting point: one kernel more or less on the
     // tail moves MobileNetV1 batch 64 by 3 %. The boundary and its three neighbours on either side are
     // timed as whole forwards and the best one kept.

@@ -69,3 +69,84 @@ def test_pair_in_one_kernel(cfg):
         bad = int((got != want).sum())
         assert bad == 0, "%s: %d of %d differ" % ("one kernel" if fused else "two kernels", bad, got.size)
         m.close()
+
+
+def _block(c, oc, n=3, h=20, w=18, pairs=2):
+    """`pairs` channel-wise + pointwise pairs behind an operator, all tensors in the arena but the first and the last:
+    (model, ids of its tensors in order, the oracle's results in order, lifetimes (begin, end, bytes) of the arena's)"""
+    from cases import MultiTypeCase
+    bias_scale = lambda k: float(np.float32(k.scales[0]) * np.float32(k.scales[1]))
+    pre = MultiTypeCase(A.Q_RELU, (n, c // 4, h, w, 4), (0.03, 0.01, GENERIC[0]))
+    x0 = np.random.default_rng(61).integers(-128, 128, pre.shape).astype(np.int8)
+    m = runtime.Model()
+    ids, want = [m.tensor("x0", pre.shape, abi.QINT8, 0.03)], [x0]
+    m.mark_input(ids[0])
+    ids.append(m.tensor("x", pre.shape, abi.QINT8, GENERIC[0]))
+    want.append(pre.run_port({"a": x0, "b": None}))
+    m.opr(pre.symbol(), [ids[0]], [ids[1]])
+    scale = GENERIC[0]
+    for p in range(pairs):
+        dw = ConvCase(A.FMT_NCHW44, A.GROUP, n, c, h, w, c, 3, 1, 1, A.RELU, scales=(scale,) + GENERIC[1:], flt_range=(-30, 30))
+        pw = ConvCase(A.FMT_NCHW44, A.DENSE, n, c, h, w, oc, 1, 1, 0, A.RELU, scales=(GENERIC[2], GENERIC[1], GENERIC[2] * 5))
+        for case in (dw, pw):
+            arrays = case.gen(70 + len(ids))
+            arrays["src"] = want[-1]
+            want.append(case.run_port(arrays))
+            name = "t%d" % len(ids)
+            ids.append(m.tensor(name, case.dst_shape(), abi.QINT8, case.scales[2]))
+            m.opr(case.symbol(), [ids[-2], m.weight(name + ".w", arrays["flt"], abi.QINT8, case.scales[1]),
+                                  m.weight(name + ".b", arrays["bias"], abi.QINT32, bias_scale(case))], [ids[-1]])
+        scale, c = pw.scales[2], oc
+    m.mark_output(ids[-1])
+    bytes_of = [int(np.prod(t.shape)) for t in want]
+    last = len(ids) - 2
+    life = [(k - 1, k + 1, bytes_of[k]) for k in range(1, len(ids) - 1)] + [(last, last + 2, bytes_of[-1])]
+    return m, ids, want, life
+
+
+def _planned(life):
+    _, arena, _ = runtime.plan_memory(*[[r[k] for r in life] for k in (0, 1, 2)], 256)
+    return int(arena)
+
+
+def test_a_pair_the_kernel_does_not_take_costs_no_memory():
+    """24 channels: no kernel of its own. The arena is that of the operators as they are"""
+    m, ids, want, life = _block(24, 24)
+    m.finalize()
+    assert m.nr_kernel == 5
+    assert m.arena_bytes == _planned(life)
+    m.set_input(ids[0], want[0])
+    m.forward()
+    assert np.array_equal(m.get(ids[-1]), want[-1])
+    m.close()
+
+
+@pytest.mark.parametrize("switch", ["fusedwpw", "nofusedwpw", None])
+def test_the_tensor_inside_a_pair_is_planned_for_operators_run_one_by_one(switch):
+    """as one kernel the pair needs no memory for the tensor in between; operators run one by one get one place for all
+    of them, and forwards before and behind are as they were"""
+    m, ids, want, life = _block(64, 64)
+    if switch:
+        runtime.set_option(switch, 1)
+    try:
+        m.finalize()
+    finally:
+        if switch:
+            runtime.set_option(switch, 0)
+    kernels = m.nr_kernel
+    if switch:
+        assert kernels == (3 if switch == "fusedwpw" else 5)
+    up = lambda v: (v + 255) // 256 * 256
+    if kernels == 3:  # sources and results of the pairs (one operator longer), one tensor in between
+        ends = [(b, e + 1, s) for b, e, s in life[0:-1:2]] + [life[-1]]
+        assert m.arena_bytes == up(_planned(ends)) + up(max(s for _, _, s in life[1:-1:2]))
+    elif kernels == 5:
+        assert m.arena_bytes == _planned(life)
+    for _ in range(2):
+        m.set_input(ids[0], want[0])
+        m.forward()
+        assert np.array_equal(m.get(ids[-1]), want[-1])
+        for k in range(len(ids) - 1):
+            m.run_opr(k)
+            assert np.array_equal(m.get(ids[k + 1]), want[k + 1]), k
+    m.close()
