@@ -63,9 +63,11 @@ struct DwPwParams {
 template <int ACT, int N>
 __device__ __forceinline__ void dp_requant(int (&a)[N], uint32_t (&out)[N / 4], const RequantPack& q, float c, const int* table) {
     auto here = [&]() __attribute__((always_inline)) {
+#ifndef MG_HOST_AUDIT
 #pragma unroll
         for (int i = 0; i < N; ++i)
             asm volatile("" : "+v"(a[i]));
+#endif
     };
     if (q.mode == 1) {  // (uniform)
         here();
@@ -298,6 +300,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
                 L[p] = E[p];
                 R[p] = E[p];
             }
+#ifndef MG_HOST_AUDIT
             // (one block: a DPP read needs two cycles behind a vector write of its source)
             asm volatile(
                     "s_nop 1\n\t"
@@ -318,6 +321,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
                         "s_nop 1"
                         : "+v"(R[0]), "+v"(R[1]), "+v"(R[2]), "+v"(R[3])
                         : "v"(B[0][0][0]), "v"(B[1][0][0]), "v"(B[2][0][0]), "v"(B[3][0][0]), "v"(cur.rmask));
+#endif
             // The short products of all four plane sets first, and every product where it stands (a scheduling
             // barrier behind each that only products may not cross). Products of ONE shape take their sums from the one
             // before at any distance; between the two shapes the sum must have been written: a 16x16x64 product
@@ -501,12 +505,12 @@ bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* sr
 }
 
 template <int S, int KC, int SUB, int MT, int NT>
-static const void* dp_kernel(int rag, int dact, int pact) {
+static void (*dp_kernel(int rag, int dact, int pact))(DwPwParams) {
     // (MobileNets use RELU behind both layers; a RELU-less pointwise layer is the linear bottleneck)
 #define MG_DP_ACT(R_)                                                                                                   \
     (dact == MEGCC_NONLINE_RELU                                                                                          \
-             ? (pact == MEGCC_NONLINE_RELU ? (const void*)conv_dw_pw_kernel<S, KC, SUB, MT, NT, R_, MEGCC_NONLINE_RELU, MEGCC_NONLINE_RELU>        \
-                                           : (const void*)conv_dw_pw_kernel<S, KC, SUB, MT, NT, R_, MEGCC_NONLINE_RELU, MEGCC_NONLINE_IDENTITY>)   \
+             ? (pact == MEGCC_NONLINE_RELU ? conv_dw_pw_kernel<S, KC, SUB, MT, NT, R_, MEGCC_NONLINE_RELU, MEGCC_NONLINE_RELU>        \
+                                           : conv_dw_pw_kernel<S, KC, SUB, MT, NT, R_, MEGCC_NONLINE_RELU, MEGCC_NONLINE_IDENTITY>)   \
              : nullptr)
     return rag == 0 ? MG_DP_ACT(0) : rag == 1 ? MG_DP_ACT(1) : rag == 2 ? MG_DP_ACT(2) : MG_DP_ACT(3);
 #undef MG_DP_ACT
@@ -563,7 +567,7 @@ TinyNNStatus conv_dw_pw_launch(
     if (q.pq.mode == 0)
         q.ptable = requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
     const int rag = dw.iw & 3;
-    const void* kern = nullptr;
+    void (*kern)(DwPwParams) = nullptr;
     size_t lds = 0;
 #define MG_DP(KC_, SUB_, MT_, NT_)                                                                                   \
     if (s.kc == KC_ && s.mt == MT_ && s.nt == NT_) {                                                                   \
@@ -580,7 +584,7 @@ TinyNNStatus conv_dw_pw_launch(
     MG_DP(32, 1, 2, 2)
 #undef MG_DP
     MG_REQUIRE(kern, TinyNN_ERROR_NO_IMPLEMENT, "conv_dw_pw: no instance");
-    const int resident = dp_resident(kern, lds);
+    const int resident = dp_resident((const void*)kern, lds);
     MG_REQUIRE(resident > 0, TinyNN_ERROR_RUNTIME, "conv_dw_pw: %d bytes of LDS", (int)lds);
     // as many workgroups as are resident, each with a run of tiles
     long runs = (long)num_cus() * resident / q.slices;
@@ -590,9 +594,7 @@ TinyNNStatus conv_dw_pw_launch(
         runs = q.tiles;
     note_kernel("conv_dw_pw", dw.ic / 32, dw.sh, q.slices);
     note_requant_affine(q.dq.mode != 0 && q.pq.mode != 0);
-    void* args[] = {&q};
-    hipError_t e = hipLaunchKernel(kern, dim3((unsigned)(runs * q.slices)), dim3(DP_THREADS), args, lds, stream());
-    MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_dw_pw: %s", hipGetErrorString(e));
+    hipLaunchKernelGGL(kern, dim3((unsigned)(runs * q.slices)), dim3(DP_THREADS), lds, stream(), q);
     return check_launch("conv_dw_pw");
 }
 

@@ -35,8 +35,10 @@ __host__ __device__ __forceinline__ float act_apply(float x) {
 // (int)x by the instruction's name: it saturates and turns NaN into 0, where the conversion in the language is undefined
 // for what an int cannot hold
 __device__ __forceinline__ int cvt_i32(float x) {
-    int r;
+    int r = 0;
+#ifndef MG_HOST_AUDIT  // (a host build that looks at addresses only)
     asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+#endif
     return r;
 }
 
@@ -142,8 +144,10 @@ static constexpr int REQUANT_TABLE_ENTRIES = 256;  // entry j + 127, last one un
 
 // (int)floorf(x) in one instruction (saturating like the plain conversion)
 __device__ __forceinline__ int cvt_floor_i32(float x) {
-    int r;
+    int r = 0;
+#ifndef MG_HOST_AUDIT
     asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+#endif
     return r;
 }
 
@@ -236,7 +240,6 @@ struct RequantPack {
 };
 RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst);
 
-#ifndef MG_HOST_AUDIT  // (the conversion has no host form)
 // MODE, ACT compile-time; channels (or pixels) 0..3 of one dword
 template <int MODE, int ACT>
 __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3, const RequantPack& q) {
@@ -251,7 +254,6 @@ __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3
     }
     return ACT == MEGCC_NONLINE_RELU ? (r >> 1) & 0x7f7f7f7fu : r ^ 0x80808080u;
 }
-#endif
 
 // host side: the estimate above is valid (else kernels use the literal sequence per element)
 static inline bool requant_table_ok(float s_src, float s_flt, float s_dst) {

@@ -1,7 +1,6 @@
 // Host-side bounds audit of kernels that load unconditionally from clamped indices.
 //
-// Linked with the library's OWN kernel sources (gemm_f32.hip, gevm_f32.hip, conv_f32_small.hip,
-// fc_stream.hip, fc_gevm_q8.hip) compiled as host C++ against tests/host_audit/hip/hip_runtime.h,
+// Linked with the library's OWN kernel sources (test_bounds_audit.py lists them) compiled as host C++ against tests/host_audit/hip/hip_runtime.h,
 // where a launch runs every thread of every workgroup one after the other on the CPU. The operand
 // buffers are fenced: each sits at the very end (then, in a second pass, at the very start) of a
 // mapping whose neighbouring page is inaccessible, so a load or store one element outside a tensor
@@ -16,6 +15,11 @@
 //   first  n ic ih iw oc k s p bias           f32 first layer, NCHW source -> NCHW44 result
 //   fcone  M K OC packed_bytes bias           qsi8 FullyConnected, M <= 64, one launch
 //   fcgevm M K OC packed_bytes bias           qsi8 FullyConnected, M <= 4
+//   fctile M K OC packed_bytes bias           qsi8 FullyConnected, any M and K
+//   ks     M K N ta tb lda_pad ldb_pad        f32 MatMul whose waves share K (whatever the dispatch would choose)
+//   split  M K N ta tb lda_pad ldb_pad        f32 MatMul on the bf16 instructions, K >= 32 (likewise)
+//   gather n ic ih iw oc k s p d bias packed_bytes       qsi8 dense NCHW44 convolution without staging
+//   dwpw   n c oc h w stride bias packed_bytes           qsi8 channel-wise 3x3 + pointwise 1x1 in one kernel
 #include <hip/hip_runtime.h>
 #include <signal.h>
 #include <stdarg.h>
@@ -30,6 +34,9 @@
 
 #include "common.h"
 #include "conv_geom.h"
+#include "epilogue.h"
+#include "gemm_f32_ks.h"
+#include "gemm_f32_split.h"
 #include "gevm_f32.h"
 
 namespace mg {
@@ -49,6 +56,10 @@ Options& options() {
     return o;
 }
 void note_kernel(const char*, int, int, int, int, int) {}
+void note_requant_affine(bool) {}
+// (of the case at hand: the library's own figure, which the test passes in)
+static size_t g_packed_bytes = 0;
+size_t conv_mfma_packed_bytes(const ConvGeom&) { return g_packed_bytes; }
 TinyNNStatus check_launch(const char*) { return TinyNN_SUCCESS; }
 TinyNNStatus check_io(Tensor** in, int nin, int lo, int hi, Tensor** out, int nout, const char* who) {
     if (!in || !out || nin < lo || nin > hi || nout != 1)
@@ -58,6 +69,10 @@ TinyNNStatus check_io(Tensor** in, int nin, int lo, int hi, Tensor** out, int no
 // dynamic LDS of fc_stream.hip / fc_gevm_q8.hip (`extern __shared__ ... name[]`)
 __attribute__((aligned(16))) int8_t lds[160 * 1024];
 __attribute__((aligned(16))) int fg_lds[40 * 1024];
+// ... of gemm_f32_ks.hip, conv_gather_i8.hip and conv_dw_pw.hip
+__attribute__((aligned(16))) float ks_lds[40 * 1024];
+__attribute__((aligned(16))) int gather_lds[40 * 1024];
+__attribute__((aligned(16))) int8_t dp_lds_mem[160 * 1024];
 
 size_t gemm_f32_workspace_bytes(long M, long N, long K, bool conv);
 size_t conv_f32_gemm_workspace_bytes(const ConvGeom& g);
@@ -72,7 +87,16 @@ bool fc_one_supported(const ConvGeom& g, const void* src);
 TinyNNStatus fc_one_launch(const ConvGeom&, const void*, const void*, const void*, void*);
 bool fc_gevm_q8_supported(const ConvGeom& g);
 TinyNNStatus fc_gevm_q8_launch(const ConvGeom&, const void*, const void*, const void*, void*);
+bool fc_tile_supported(const ConvGeom& g);
+TinyNNStatus fc_tile_launch(const ConvGeom&, const void*, const void*, const void*, void*);
+bool conv_gather_i8_supported(const ConvGeom& g);
+TinyNNStatus conv_gather_i8_launch(const ConvGeom&, const void*, const void*, const void*, void*);
+bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dst);
+TinyNNStatus conv_dw_pw_launch(const ConvGeom&, const ConvGeom&, const void*, const void*, const void*, const void*, const void*, void*);
 }  // namespace mg
+
+// the bf16 conversion of the compiler's vector types (its value does not matter here)
+extern "C" __bf16 __truncsfbf2(float) { return __builtin_bit_cast(__bf16, (unsigned short)0); }
 
 extern "C" TinyNNStatus megcc_gfx950_matmul(
         const MegccMatMulAttr*, Tensor**, int, Tensor**, int, const Workspace*, const RuntimeOpt*);
@@ -152,6 +176,56 @@ static bool run_case(const std::string& line, bool at_end) {
         Workspace w = {wsb ? W.ptr : nullptr, wsb, 0};
         return megcc_gfx950_matmul(&attr, in, 2, out, 1, &w, nullptr) == TinyNN_SUCCESS;
     }
+    if (kind == "ks" || kind == "split") {
+        int M, K, N, ta, tb, pa, pb;
+        ss >> M >> K >> N >> ta >> tb >> pa >> pb;
+        const int ar = ta ? K : M, ac = ta ? M : K, br = tb ? N : K, bc = tb ? K : N;
+        const long lda = ac + pa, ldb = bc + pb;
+        Fenced A(((size_t)(ar - 1) * lda + ac) * 4, at_end, 16), B(((size_t)(br - 1) * ldb + bc) * 4, at_end, 16),
+                Cm((size_t)M * N * 4, at_end, 16);
+        const GevmArgs v = {(const float*)A.ptr, (const float*)B.ptr, (float*)Cm.ptr, M, N, K, ta ? 1 : lda, ta ? lda : 1,
+                            tb ? 1 : ldb, tb ? ldb : 1, N};
+        return (kind == "ks" ? gemm_f32_ks_launch(v, ta, tb) : gemm_f32_split_launch(v, ta, tb)) == TinyNN_SUCCESS;
+    }
+    if (kind == "gather") {
+        ConvGeom g;
+        memset(&g, 0, sizeof(g));
+        int k, s, p, d, bias;
+        ss >> g.n >> g.ic >> g.ih >> g.iw >> g.oc >> k >> s >> p >> d >> bias >> g_packed_bytes;
+        g.fh = g.fw = k, g.sh = g.sw = s, g.ph = g.pw = p, g.dh = g.dw = d;
+        g.oh = (g.ih + 2 * p - (d * (k - 1) + 1)) / s + 1;
+        g.ow = (g.iw + 2 * p - (d * (k - 1) + 1)) / s + 1;
+        // (an activation without a threshold table: there is no kernel-argument segment to read one from)
+        g.groups = 1, g.fmt = MEGCC_FMT_NCHW44, g.act = MEGCC_NONLINE_SIGMOID, g.has_bias = bias;
+        g.s_src = g.s_flt = 0.01f, g.s_dst = 0.1f;
+        Fenced src((size_t)g.n * g.ic * g.ih * g.iw, at_end, 4), wp(g_packed_bytes, at_end, 16), b((size_t)g.oc * 4, at_end, 4),
+                dst((size_t)g.n * g.oc * g.oh * g.ow, at_end, 4);
+        if (!conv_gather_i8_supported(g)) {
+            fprintf(stderr, "not a conv_gather_i8 layer: %s\n", line.c_str());
+            return false;
+        }
+        return conv_gather_i8_launch(g, src.ptr, wp.ptr, bias ? b.ptr : nullptr, dst.ptr) == TinyNN_SUCCESS;
+    }
+    if (kind == "dwpw") {
+        ConvGeom dw, pw;
+        memset(&dw, 0, sizeof(dw));
+        int oc, stride, bias;
+        ss >> dw.n >> dw.ic >> oc >> dw.ih >> dw.iw >> stride >> bias >> g_packed_bytes;
+        dw.oc = dw.groups = dw.ic, dw.fh = dw.fw = 3, dw.sh = dw.sw = stride, dw.ph = dw.pw = dw.dh = dw.dw = 1;
+        dw.oh = (dw.ih - 1) / stride + 1, dw.ow = (dw.iw - 1) / stride + 1;
+        dw.fmt = MEGCC_FMT_NCHW44, dw.act = MEGCC_NONLINE_RELU, dw.has_bias = bias;
+        dw.s_src = dw.s_flt = 0.01f, dw.s_dst = 0.1f;
+        pw = dw;
+        pw.oc = oc, pw.groups = 1, pw.ih = dw.oh, pw.iw = dw.ow, pw.fh = pw.fw = pw.sh = pw.sw = 1, pw.ph = pw.pw = 0;
+        Fenced src((size_t)dw.n * dw.ic * dw.ih * dw.iw, at_end, 16), df((size_t)dw.ic * 9, at_end, 4), db((size_t)dw.ic * 4, at_end, 4),
+                wp(g_packed_bytes, at_end, 16), pb((size_t)oc * 4, at_end, 4), dst((size_t)dw.n * oc * dw.oh * dw.ow, at_end, 4);
+        if (!conv_dw_pw_supported(dw, pw, src.ptr, dst.ptr)) {
+            fprintf(stderr, "not a conv_dw_pw pair: %s\n", line.c_str());
+            return false;
+        }
+        return conv_dw_pw_launch(dw, pw, src.ptr, df.ptr, bias ? db.ptr : nullptr, wp.ptr, bias ? pb.ptr : nullptr, dst.ptr) ==
+               TinyNN_SUCCESS;
+    }
     if (kind == "conv" || kind == "small") {
         ConvGeom g;
         memset(&g, 0, sizeof(g));
@@ -209,7 +283,7 @@ static bool run_case(const std::string& line, bool at_end) {
         }
         return dwconv44_f32_launch(g, src.ptr, flt.ptr, bias ? b.ptr : nullptr, dst.ptr) == TinyNN_SUCCESS;
     }
-    if (kind == "fcone" || kind == "fcgevm") {
+    if (kind == "fcone" || kind == "fcgevm" || kind == "fctile") {
         ConvGeom g;
         memset(&g, 0, sizeof(g));
         long packed;
@@ -220,6 +294,13 @@ static bool run_case(const std::string& line, bool at_end) {
         g.s_src = g.s_flt = 0.01f, g.s_dst = 0.1f;
         Fenced src((size_t)g.n * g.ic, at_end, 16), wp((size_t)packed, at_end, 16), b((size_t)g.oc * 4, at_end, 4),
                 dst((size_t)g.n * g.oc, at_end, g.oc % 4 ? 1 : 4);
+        if (kind == "fctile") {
+            if (!fc_tile_supported(g)) {
+                fprintf(stderr, "not an fc_tile layer: %s\n", line.c_str());
+                return false;
+            }
+            return fc_tile_launch(g, src.ptr, wp.ptr, bias ? b.ptr : nullptr, dst.ptr) == TinyNN_SUCCESS;
+        }
         if (kind == "fcone") {
             if (!fc_one_supported(g, src.ptr)) {
                 fprintf(stderr, "not an fc_one layer: %s\n", line.c_str());

@@ -65,6 +65,40 @@ inline const char* hipGetErrorString(hipError_t) { return "host audit"; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipFuncSetAttribute(const void*, int, int) { return hipSuccess; }
 
+inline hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) { return *n = 1, hipSuccess; }
+
+// Buffer loads and stores: dwords whose whole offset, the lane's and the scalar one, lies beyond the buffer read zero
+// or are dropped (each dword for itself, as the hardware does it), everything else is dereferenced.
+struct audit_rsrc {
+    char* p;
+    unsigned bytes;
+};
+typedef unsigned audit_v4u __attribute__((ext_vector_type(4)));
+inline unsigned audit_load(audit_rsrc r, unsigned off, unsigned soff) {
+    unsigned v = 0;
+    if ((unsigned long long)off + soff < r.bytes)
+        v = *(volatile unsigned*)(r.p + off + soff);
+    return v;
+}
+inline audit_v4u audit_load4(audit_rsrc r, unsigned off, unsigned soff) {
+    return audit_v4u{audit_load(r, off, soff), audit_load(r, off + 4, soff), audit_load(r, off + 8, soff), audit_load(r, off + 12, soff)};
+}
+inline void audit_store(unsigned v, audit_rsrc r, unsigned off, unsigned soff) {
+    if ((unsigned long long)off + soff < r.bytes)
+        *(volatile unsigned*)(r.p + off + soff) = v;
+}
+#define __amdgpu_buffer_rsrc_t audit_rsrc
+#define __builtin_amdgcn_make_buffer_rsrc(ptr, stride, bytes, flags) (audit_rsrc{(char*)(ptr), (unsigned)(bytes)})
+#define __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, aux) audit_load(r, (unsigned)(off), (unsigned)(soff))
+#define __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, aux) audit_load4(r, (unsigned)(off), (unsigned)(soff))
+#define __builtin_amdgcn_raw_buffer_store_b32(v, r, off, soff, aux) audit_store(v, r, (unsigned)(off), (unsigned)(soff))
+
+inline float __uint_as_float(unsigned u) {
+    float f;
+    memcpy(&f, &u, 4);
+    return f;
+}
+
 inline void __syncthreads() {}
 template <typename T>
 inline T __shfl_down(T v, int, int = 64) { return v; }
@@ -77,8 +111,12 @@ inline unsigned __umulhi(unsigned a, unsigned b) { return (unsigned)(((unsigned 
 #define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) (c)
+#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) (c)
 #define __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, x, y, z) (c)
+#define __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, x, y, z) (c)
+#define __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, c, x, y, z) (c)
 #define __builtin_amdgcn_sdot4(a, b, c, clamp) (c)
+#define __builtin_amdgcn_cvt_pk_u8_f32(x, i, r) (r)
 #define __builtin_amdgcn_perm(a, b, sel) ((a) ^ (b) ^ (sel))
 #define __builtin_amdgcn_s_barrier() ((void)0)
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)

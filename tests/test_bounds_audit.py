@@ -1,6 +1,8 @@
 """Host-side bounds audit of the kernels that issue their loads unconditionally from clamped
-indices (gemm_f32: all four transpositions and the implicit-GEMM gather; gevm_f32; conv_f32_small; the
-f32 NCHW44 channel-wise and first-layer kernels; fc_one32 / fc_one; fc_gevm_q8). tests/host_audit/audit.cpp links the library's own kernel sources,
+indices or through range-checked buffers (gemm_f32: all four transpositions and the implicit-GEMM gather; gemm_f32_ks and
+gemm_f32_split: all four transpositions; gevm_f32; conv_f32_small; the f32 NCHW44 channel-wise and first-layer kernels;
+fc_one32 / fc_one; fc_tile; fc_gevm_q8; conv_gather_i8; conv_dw_pw). Not gemm_f32_ks's convolution, whose addresses come
+through LDS from other threads. tests/host_audit/audit.cpp links the library's own kernel sources,
 compiled as host C++ against a stand-in HIP header that runs every thread of every workgroup on
 the CPU, and fences each operand buffer with inaccessible pages: one element outside a tensor ends
 the run. No GPU involved; the shapes are every case of the GPU sweeps plus a seeded sweep of ragged
@@ -20,13 +22,14 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 AUDIT_DIR = os.path.join(HERE, "host_audit")
 CSRC = os.path.join(os.path.dirname(HERE), "megcc_amd", "csrc")
 CLANG = "/opt/rocm/llvm/bin/clang++"
-SOURCES = ["gemm_f32", "gevm_f32", "conv_f32_small", "conv_f32_nchw44", "fc_stream", "fc_gevm_q8"]
+SOURCES = ["gemm_f32", "gevm_f32", "conv_f32_small", "conv_f32_nchw44", "fc_stream", "fc_gevm_q8", "fc_tile", "gemm_f32_ks",
+           "gemm_f32_split", "conv_gather_i8", "conv_dw_pw", "requant_table"]
 
 pytestmark = pytest.mark.skipif(not os.path.exists(CLANG), reason="needs ROCm's clang++ for the kernels' vector types")
 
 
-def compile_audit(out_dir, replace=None):
-    """replace: {source name: path of another file to compile in its place}"""
+def compile_audit(out_dir, replace=None, have=None):
+    """replace: {source name: path of another file to compile in its place}; have: folder with the objects of the others"""
     os.makedirs(out_dir, exist_ok=True)
     flags = ["-x", "c++", "-std=c++17", "-O1", "-g", "-I" + AUDIT_DIR, "-I" + CSRC,
              "-I" + os.path.join(os.path.dirname(HERE), "include"), "-ffp-contract=off", "-Wno-unknown-attributes"]
@@ -37,8 +40,12 @@ def compile_audit(out_dir, replace=None):
         if replace and name in replace:
             src = replace[name]
         obj = os.path.join(out_dir, name + ".o")
+        if have and not (replace and name in replace):
+            objs.append(os.path.join(have, name + ".o"))
+            continue
         objs.append(obj)
-        jobs.append(subprocess.Popen([CLANG] + flags + ["-c", src, "-o", obj], stderr=subprocess.PIPE, text=True))
+        last = ["-O0", "-g0"] if name == "conv_dw_pw" else []  # (128 instances: half a minute with the optimiser)
+        jobs.append(subprocess.Popen([CLANG] + flags + last + ["-c", src, "-o", obj], stderr=subprocess.PIPE, text=True))
     for j in jobs:
         err = j.communicate()[1]
         assert j.returncode == 0, err[-4000:]
@@ -144,6 +151,30 @@ def audit_lines():
             continue
         lines.append("first %d %d %d %d %d %d %d %d %d" % (r.integers(1, 4), r.integers(1, 5), ih, iw,
                                                          4 * r.choice([1, 2, 8, 9, 16]), k, s, p, r.integers(0, 2)))
+    # f32 products whose waves share K and those on the bf16 instructions: edges of the 32 / 64 / 128 tiles, K with and
+    # without a rest, every transposition, padded rows
+    for i in range(32):
+        m, n = (int(r.choice([1, 5, 31, 32, 33, 64, 65, 127, 128, 129, 200])) for _ in range(2))
+        k = int(r.choice([1, 3, 7, 8, 9, 31, 64, 100, 300]))
+        tail = "%d %d %d %d" % (r.integers(0, 2), r.integers(0, 2), r.choice([0, 1, 4, 7]), r.choice([0, 1, 4, 7]))
+        lines.append("ks %d %d %d %s" % (m, k, n, tail))
+        lines.append("split %d %d %d %s" % (m, 32 + int(r.choice([0, 1, 15, 16, 17, 100, 143, 500])), n, tail))
+    # FullyConnected of any K on tiles: rows at any byte, the tensor's last 16 bytes anywhere in a piece
+    for m, k, oc in ((65, 5, 9), (64, 1, 3), (16, 1, 1), (65, 129, 67), (70, 295, 70), (225, 515, 361), (66, 128, 64), (130, 260, 257),
+                     (100, 1123, 65), (65, 127, 129), (300, 33, 31)):
+        case = ConvCase(abi.FMT_NCHW, abi.DENSE, m, k, 1, 1, oc, 1, 1, 0, abi.RELU, scales=(0.01, 0.01, 0.1))
+        lines.append("fctile %d %d %d %d %d" % (m, k, oc, packed_bytes(case), i & 1))
+    # qsi8 layers without staging, and channel-wise + pointwise pairs: the shapes of their GPU tests
+    for case in gp.GATHER:
+        if case.n * case.oh * case.ow <= 6000:
+            lines.append("gather %d %d %d %d %d %d %d %d %d %d %d" % (case.n, case.ic, case.ih, case.iw, case.oc, case.fh, case.sh,
+                                                                     case.ph, case.dh, int(case.bias), packed_bytes(case)))
+    import test_dw_pw
+    for n, c, oc, h, w, s, act, _ in test_dw_pw.PAIRS:
+        n = min(n, 3)
+        if n * c * h * w <= 1 << 19:
+            pw = ConvCase(abi.FMT_NCHW44, abi.DENSE, n, c, (h - 1) // s + 1, (w - 1) // s + 1, oc, 1, 1, 0, act, scales=(0.01, 0.01, 0.1))
+            lines.append("dwpw %d %d %d %d %d %d %d %d" % (n, c, oc, h, w, s, (h + w) & 1, packed_bytes(pw)))
     # qsi8 FullyConnected: 1..64 rows, K = 1..32 blocks of 128 (and beyond 4096), channel counts off every tile size
     for i in range(24):
         m = int(r.choice([1, 2, 3, 4, 5, 31, 32, 33, 63, 64]))
@@ -171,6 +202,18 @@ def test_the_audit_sees_the_out_of_bounds_read_a_missing_clamp_causes(audit_exe,
     assert src.count(clamp) == 1
     mutated = tmp_path / "gemm_f32.hip"
     mutated.write_text(src.replace(clamp, "const int cn = n0 + tid % BN;"))
-    exe = compile_audit(str(tmp_path / "build"), replace={"gemm_f32": str(mutated)})
+    exe = compile_audit(str(tmp_path / "build"), replace={"gemm_f32": str(mutated)}, have=os.path.dirname(audit_exe))
     r = subprocess.run([exe], input="conv 3 86 45 42 117 5 2 3 1 1 1\n", capture_output=True, text=True, timeout=300)
+    assert r.returncode == 3 and "OUT OF BOUNDS" in r.stderr, (r.returncode, r.stderr[-500:])
+
+
+def test_the_audit_sees_a_row_read_past_the_end_of_its_tensor(audit_exe, tmp_path):
+    """likewise for loads at any byte: without the step back to the tensor's last 16 bytes"""
+    src = open(os.path.join(CSRC, "fc_tile.hip")).read()
+    clamp = "min(roff[i] + b, q.last16)"
+    assert src.count(clamp) == 1
+    mutated = tmp_path / "fc_tile.hip"
+    mutated.write_text(src.replace(clamp, "(roff[i] + b)"))
+    exe = compile_audit(str(tmp_path / "build"), replace={"fc_tile": str(mutated)}, have=os.path.dirname(audit_exe))
+    r = subprocess.run([exe], input="fctile 65 129 67 65536 0\n", capture_output=True, text=True, timeout=300)
     assert r.returncode == 3 and "OUT OF BOUNDS" in r.stderr, (r.returncode, r.stderr[-500:])
