@@ -692,6 +692,9 @@ TinyNNStatus megcc_gfx950_model_forward(void* model);
 TinyNNStatus megcc_gfx950_model_join(void* model);
 /* how many of megcc_gfx950_model_nr_kernel's kernels those last operators are (0: none) */
 int megcc_gfx950_model_nr_tail_kernel(void* model);
+/* Bytes of one forward when each of its nr_kernel kernels reads its operands and writes its results
+ * once; what a bandwidth roofline of the forward is priced against. */
+size_t megcc_gfx950_model_forward_bytes(void* model);
 /* megcc_gfx950_model_get_output without the host waiting: the copy is enqueued behind the forward
  * that produced the tensor (on the second stream when that forward's last operators are there) and
  * the bytes are in `host` - pinned memory, for the copy to be asynchronous - after

@@ -1447,6 +1447,19 @@ TinyNNStatus megcc_gfx950_model_forward(void* model) {
     return st;
 }
 
+// Bytes of one forward when each kernel of its schedule reads its operands and writes its results once (a chain that
+// runs as one kernel neither writes nor reads the tensors in between).
+size_t megcc_gfx950_model_forward_bytes(void* model) {
+    Model* m = (Model*)model;
+    size_t bytes = 0;
+    if (m && m->finalized)
+        for (const ModelOpr* o : m->schedule)
+            for (const std::vector<int>* ids : {&o->in, &o->out})
+                for (int id : *ids)
+                    bytes += tensor_bytes(m->tensors[id]->t);
+    return bytes;
+}
+
 // Kernels of one forward that go to the second stream under plain launches (0: none).
 int megcc_gfx950_model_nr_tail_kernel(void* model) {
     Model* m = (Model*)model;

@@ -139,3 +139,30 @@ def test_softmax_chain_runs_as_one_kernel_and_gives_the_same_result():
     np.testing.assert_array_equal(results[0], results[2])
     for m in (fused, plain, kept):
         m.close()
+
+
+@pytest.mark.gpu
+def test_forward_bytes_are_those_of_the_kernels_that_run():
+    """every operator on its own: the operators' bytes; operator chains as one kernel: without the tensors in between,
+    each of which is written once and read once"""
+    apart = ("nofusesoftmax", "nofusepwdw", "nofusedwpw")
+    for o in apart:
+        runtime.set_option(o, 1)
+    try:
+        model, _ = mobilenet.Net(2).build_gpu()
+    finally:
+        for o in apart:
+            runtime.set_option(o, 0)
+    assert model.nr_kernel == model.nr_opr and model.forward_bytes == mobilenet.algorithmic_bytes(2)
+    model.close()
+    runtime.set_option("fusedwpw", 1)
+    try:
+        model, _ = mobilenet.Net(2).build_gpu()
+    finally:
+        runtime.set_option("fusedwpw", 0)
+    between = sum(2 * c.n * c.oc * c.oh * c.ow for name, c in mobilenet.conv_layers(2) if name.startswith("dw"))
+    logits, row = 2 * 1000 * 4, 2 * 4  # dequantised, max, sub, exp, sum: written once and read 2, 1, 1, 2, 1 times
+    between += 3 * logits + 2 * row + 2 * logits + 3 * logits + 2 * row
+    assert model.nr_kernel == model.nr_opr - 13 - 5
+    assert model.forward_bytes == mobilenet.algorithmic_bytes(2) - between
+    model.close()
