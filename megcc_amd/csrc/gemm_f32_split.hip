@@ -24,8 +24,8 @@
 //     a lane of the instruction reads: no bank conflicts either way.
 //   * Loads are unconditional from clamped rows (their results are not stored); the last K % 16 steps are fetched
 //     element by element and masked.
-// Measured (us, before: the f32 kernels): 4096^3 1087 -> 719 (191 TFLOP/s of the product, 1.15 PFLOP/s of bf16), 2048^3 139 ->
-// 110, 1536^3 100 -> 69, 1999 x 333 x 2500 58 -> 32, 4096 x 77 x 4096 40 -> 29.
+// Measured (us, before: the f32 kernels): 4096^3 1087 -> 709 (194 TFLOP/s of the product, 1.16 PFLOP/s of bf16), 2048^3 139 ->
+// 107, 1536^3 100 -> 69, 1999 x 333 x 2500 58 -> 33, 4096 x 77 x 4096 40 -> 28.
 // The matrix units are busy 60 % of 4096^3, at the 1.85 GHz the card holds under this load (2.4 without); the
 // rest is the split's vector instructions, which both cost issue slots and power.
 // Fp32MatMulM4N12.cpp:9-158 is the loop replaced.
