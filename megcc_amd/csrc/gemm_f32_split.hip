@@ -11,12 +11,12 @@
 //     registers. Against 64 bits, relative error here / by the f32 instructions (gemm_f32.hip, the same operands):
 //     4096^3 2.0e-7 / 4.1e-7, 2048^3 1.8e-7 / 4.1e-7, K = 768 1.7e-7 / 5.0e-7, 333 0.9e-7 / 3.3e-7, 64 0.5e-7 / 1.4e-7.
 //   * The decomposition is exact, and no infinity appears on the way, for zero and for 2^-102 <= |x| < 2^60. A
-//     workgroup looks at every value it splits, asks after every chain of 8 stages whether one lay outside, and then
-//     multiplies the rest from that chain on (K up to 512, whose sum of small products runs through: from the
-//     start) with v_mfma_f32_32x32x2_f32, running sums closed every 512 steps of K: Inf, NaN and extreme values come
+//     workgroup looks at every value it splits, asks after the first stage and every chain of 8 (K up to 512, whose sum of
+//     small products runs through, is one chain) whether one lay outside, and then multiplies the rest from that chain
+//     on with v_mfma_f32_32x32x2_f32, running sums closed every 512 steps of K: Inf, NaN and extreme values come
 //     out as of an f32 product. With such values all over (a soft-max of wide logits; us, here / the f32 kernel):
-//     4096^3 1040 / 1080, 2048^3 188 / 181, 1999 x 333 x 2500 52 / 71. One, in the last chain of every tile: 740 / 1080,
-//     120 / 181, and for K up to 512, where it costs both passes, 81 / 71.
+//     4096^3 1040 / 1080, 2048^3 160 / 155 (gemm_f32_ks), 1999 x 333 x 2500 52 / 54. One, late in every tile: 740 / 1080,
+//     121 / 155, and for K up to 512, where it costs both passes, 81 / 54.
 //   * Workgroup: 128 x 128 outputs, 4 waves of 64 x 64, 16 steps of K a stage, two stages in LDS (50 KB),
 //     the next one's values in registers. Two workgroups share a CU, so that one splits while the other multiplies.
 //     A thread fetches 8 steps of K of one row - two 16-byte loads, or 8 dword loads of 256 contiguous bytes a wave
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
         return __builtin_amdgcn_readfirstlane(*(volatile int*)&beyond) != 0;
     };
     // Steps of K whose products are in the sums for good: all of a chain, once no value of it has been reported.
-    // (SHORT adds the small products of every chain to the one sum: nothing is for good before the end.)
+    // (SHORT's sum of small products runs through: one chain, nothing is for good before its end.)
     int kept = 0;
     bool f32 = false;
     sa.load(0, va);
@@ -225,12 +225,12 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
     report();
     __syncthreads();
     f32 = reported();
-    for (int s0 = 0; s0 < full && !f32; s0 += SP_CHAIN) {
+    for (int s0 = 0; s0 < full && !f32; s0 += SHORT ? full : SP_CHAIN) {
         if (!SHORT && s0) {
             close();
             kept = s0 * SP_K;
         }
-        const int s1 = min(s0 + SP_CHAIN, full);
+        const int s1 = SHORT ? full : min(s0 + SP_CHAIN, full);
         // (the last two rounds fetch and split the last stage again, for no reader, rather than branch)
         for (int s = s0; s < s1; ++s) {
             multiply(s & 1);
@@ -260,17 +260,28 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
         if (SHORT)
             clear(sum);
         __syncthreads();  // (a wave may still be in the multiply just above, reading what is written next)
+        if (!SHORT) {
+            sa.load(kept, va);  // (a chain begins with a whole stage)
+            sb.load(kept, vb);
+        }
         for (int k0 = kept; k0 < q.K; k0 += SP_K) {
-            if (k0 + SP_K <= q.K) {
-                sa.load(k0, va);
-                sb.load(k0, vb);
-            } else {
-                sa.load_tail(k0, q.K, va);
-                sb.load_tail(k0, q.K, vb);
+            // (the next stage in flight while this one is multiplied, but for SHORT, whose bf16 loop would spill registers)
+            const int buf = (k0 / SP_K) & 1, kf = SHORT ? k0 : k0 + SP_K;
+            if (!SHORT) {
+                sa.store_f32(&lds[buf][0], va);
+                sb.store_f32(&lds[buf][SP_OPERAND], vb);
             }
-            const int buf = (k0 / SP_K) & 1;
-            sa.store_f32(&lds[buf][0], va);
-            sb.store_f32(&lds[buf][SP_OPERAND], vb);
+            if (kf + SP_K <= q.K) {
+                sa.load(kf, va);
+                sb.load(kf, vb);
+            } else if (SHORT || kf < q.K) {
+                sa.load_tail(kf, q.K, va);
+                sb.load_tail(kf, q.K, vb);
+            }
+            if (SHORT) {
+                sa.store_f32(&lds[buf][0], va);
+                sb.store_f32(&lds[buf][SP_OPERAND], vb);
+            }
             __syncthreads();
 #pragma unroll
             for (int c = 0; c < 2; ++c) {

@@ -61,8 +61,8 @@ struct Model {
     std::vector<ModelTensor*> tensors;
     std::vector<ModelOpr*> oprs;
     // what forward() launches: the operators in order, with recognised operator chains replaced by
-    // one kernel (`fused` owns the replacements); run_opr, nr_opr and the memory plan keep the
-    // operator list as it was given
+    // one kernel (`fused` owns the replacements); run_opr and nr_opr keep the operator list as it was
+    // given, and so does the memory plan but for the tensors inside channel-wise -> pointwise pairs (plan_again)
     std::vector<ModelOpr*> schedule, fused;
     // per operator: whether the pair that begins there measured faster as one kernel, and by how much; what the schedule's
     // kernels take one by one (both in microseconds, as far as they were timed)
