@@ -57,11 +57,16 @@ __host__ __device__ __forceinline__ int fp32_to_int8(float v) {
 #endif
 }
 
-// acc already includes the int32 bias.
+// acc already includes the int32 bias. (Rounded like fp32_to_int8, but clamped while it is a float, which the compiler can
+// see through: FullyConnected tiles lost 2 % to the instruction by name.)
 template <int ACT>
 __host__ __device__ __forceinline__ int requant_conv(int acc, float s_src, float s_flt, float s_dst) {
-    float v = (float)acc * s_src * s_flt / s_dst;
-    return fp32_to_int8(act_apply<ACT>(v));
+    const float v = act_apply<ACT>((float)acc * s_src * s_flt / s_dst);
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (int)__builtin_amdgcn_fmed3f(v + __builtin_copysignf(0x1.fffffep-2f, v), -128.f, 127.f);
+#else
+    return fp32_to_int8(v);
+#endif
 }
 
 // ---- exact requantisation at a third of the instructions ---------------------------------------
@@ -107,9 +112,8 @@ __device__ __forceinline__ int requant_conv_fast(int acc, const RequantFast& q) 
     if (__builtin_expect((!(d <= 0.5f - 0x1p-13f) && __builtin_fabsf(g) < 129.f) || q.c == 0.f, 0)) {
         out = requant_conv<ACT>(acc, q.s_src, q.s_flt, q.s_dst);
     } else {
-        const int i = cvt_i32(r);
-        const int lo = ACT == MEGCC_NONLINE_RELU ? 0 : -128;
-        out = i < lo ? lo : (i > 127 ? 127 : i);
+        const float lo = ACT == MEGCC_NONLINE_RELU ? 0.f : -128.f;
+        out = (int)__builtin_amdgcn_fmed3f(r, lo, 127.f);  // (clamped as a float: an int holds it)
     }
     return out;
 }

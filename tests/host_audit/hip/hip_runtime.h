@@ -116,6 +116,7 @@ inline unsigned __umulhi(unsigned a, unsigned b) { return (unsigned)(((unsigned 
 #define __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, x, y, z) (c)
 #define __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, c, x, y, z) (c)
 #define __builtin_amdgcn_sdot4(a, b, c, clamp) (c)
+#define __builtin_amdgcn_fmed3f(x, lo, hi) (lo)
 #define __builtin_amdgcn_cvt_pk_u8_f32(x, i, r) (r)
 #define __builtin_amdgcn_perm(a, b, sel) ((a) ^ (b) ^ (sel))
 #define __builtin_amdgcn_s_barrier() ((void)0)
