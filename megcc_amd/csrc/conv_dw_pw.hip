@@ -563,9 +563,9 @@ TinyNNStatus conv_dw_pw_launch(
     q.dc = make_requant_fast(dw.s_src, dw.s_flt, dw.s_dst).c;
     q.pc = make_requant_fast(pw.s_src, pw.s_flt, pw.s_dst).c;
     if (q.dq.mode == 0)
-        q.dtable = requant_table_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
+        q.dtable = *requant_table_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
     if (q.pq.mode == 0)
-        q.ptable = requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
+        q.ptable = *requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
     const int rag = dw.iw & 3;
     void (*kern)(DwPwParams) = nullptr;
     size_t lds = 0;

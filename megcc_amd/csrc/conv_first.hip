@@ -280,7 +280,7 @@ static TinyNNStatus conv_first_mfma_launch(
     q.dOHW = make_fastdiv(q.OHW);
     const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     if (tab)
-        q.table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
     const int act = tab ? g.act : -1;
     const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
     q.aff_c = aff.c;
@@ -328,7 +328,8 @@ TinyNNStatus conv_first_launch(
     // evaluates the literal sequence per output
     const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     static const RequantTable no_table = {};
-    const RequantTable table = tab ? requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst) : no_table;
+    std::shared_ptr<const RequantTable> kept;
+    const RequantTable& table = tab ? *(kept = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst)) : no_table;
     auto kern = tab && g.act == MEGCC_NONLINE_IDENTITY ? conv_first_q8_kernel<MEGCC_NONLINE_IDENTITY>
               : tab && g.act == MEGCC_NONLINE_RELU     ? conv_first_q8_kernel<MEGCC_NONLINE_RELU>
               : tab && g.act == MEGCC_NONLINE_H_SWISH  ? conv_first_q8_kernel<MEGCC_NONLINE_H_SWISH>

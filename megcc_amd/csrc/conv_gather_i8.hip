@@ -256,7 +256,7 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     q.c = make_requant_fast(g.s_src, g.s_flt, g.s_dst).c;
     const bool table = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     if (table)
-        q.table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
     // 64 x 64 outputs a wave where that gives every SIMD one, else less. 32 x 32: four groups share a long K however many
     // tiles there are (7 x 124 -> 240 29 x 23 11.4 us with one, 10.4 with four; 256 -> 256 28 x 28 5.6 with four, 6.0
     // with eight), a shorter one while SIMDs are idle (24 x 56 -> 16 66 x 66 stride 2 6.9 with two, 7.3 with four; 3 x 20 ->

@@ -696,7 +696,7 @@ TinyNNStatus conv_mfma_launch(
     q.rq = make_requant_fast(g.s_src, g.s_flt, g.s_dst);
     if (pipe && requant_table_act(g.act) && !(fc && g.act == MEGCC_NONLINE_H_SWISH) &&
         requant_table_ok(g.s_src, g.s_flt, g.s_dst))
-        q.rq_table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+        q.rq_table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
     q.dOW = make_fastdiv(q.OW);
     q.dOH = make_fastdiv(q.OH);
     q.dVW = make_fastdiv(q.VW);

@@ -399,8 +399,8 @@ TinyNNStatus conv_pw_dw_launch(
     q.dw_lo = dw.act == MEGCC_NONLINE_RELU ? 0 : -128;
     q.pw_c = make_requant_fast(pw.s_src, pw.s_flt, pw.s_dst).c;
     q.dw_c = make_requant_fast(dw.s_src, dw.s_flt, dw.s_dst).c;
-    q.pw_table = requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
-    q.dw_table = requant_table_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
+    q.pw_table = *requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
+    q.dw_table = *requant_table_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
     const RequantAffine a0 = requant_affine_pick(true, pw.act, pw.s_src, pw.s_flt, pw.s_dst);
     const RequantAffine a1 = requant_affine_pick(true, dw.act, dw.s_src, dw.s_flt, dw.s_dst);
     q.pw_ac = a0.c;

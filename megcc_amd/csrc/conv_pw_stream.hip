@@ -379,7 +379,7 @@ TinyNNStatus conv_pw_stream_launch(
     q.dOHW = make_fastdiv(q.OHW);
     const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     if (tab)
-        q.table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
     const int act = tab ? g.act : -1;
 
     const void* kern = nullptr;

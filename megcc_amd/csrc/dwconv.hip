@@ -346,7 +346,8 @@ TinyNNStatus dwconv44_chain_launch(
     const bool tab = (g.act == MEGCC_NONLINE_IDENTITY || g.act == MEGCC_NONLINE_RELU) &&
                      requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     static const RequantTable no_table = {};
-    const RequantTable table = tab ? requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst) : no_table;
+    std::shared_ptr<const RequantTable> kept;
+    const RequantTable& table = tab ? *(kept = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst)) : no_table;
     const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
     rq3.aff_c = aff.c;
     rq3.aff_d = aff.d;
@@ -429,7 +430,8 @@ TinyNNStatus dwconv44_launch(
         // evaluates the literal sequence per output
         const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
         static const RequantTable no_table = {};
-        const RequantTable table = tab ? requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst) : no_table;
+        std::shared_ptr<const RequantTable> kept;
+    const RequantTable& table = tab ? *(kept = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst)) : no_table;
         const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
         rq3.aff_c = aff.c;
         rq3.aff_d = aff.d;

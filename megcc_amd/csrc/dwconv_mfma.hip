@@ -432,7 +432,7 @@ static TinyNNStatus dwconv44_mfma_run(
         return TinyNN_SUCCESS;
     const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     if (tab)
-        q.table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
     const int act = tab ? g.act : -1;
     // (the chain kernel has no table instantiation for H_SWISH: the pair is only asked for where one runs)
     const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);

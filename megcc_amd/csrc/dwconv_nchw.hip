@@ -197,7 +197,7 @@ TinyNNStatus dwconv_nchw_launch(
     const bool tab = (g.act == MEGCC_NONLINE_IDENTITY || g.act == MEGCC_NONLINE_RELU) &&
                      requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     if (tab)
-        q.table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
     const int act = tab ? g.act : -1;
     const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
     q.aff_c = aff.c;

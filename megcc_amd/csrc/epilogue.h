@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <memory>
+
 #include "megcc_gfx950.h"
 
 namespace mg {
@@ -170,7 +172,7 @@ static inline bool requant_table_act(int act) {
 }
 
 // host: the table for (act in {IDENTITY, RELU, H_SWISH}, scales); requant_table.hip
-RequantTable requant_table_for(int act, float s_src, float s_flt, float s_dst);
+std::shared_ptr<const RequantTable> requant_table_for(int act, float s_src, float s_flt, float s_dst);
 
 // the lower candidate m (clamped to [lowest output, 126]) of the output for accumulator acc
 template <int ACT>

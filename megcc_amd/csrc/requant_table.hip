@@ -105,19 +105,20 @@ static void requant_thresholds(float s_src, float s_flt, float s_dst, float c, i
     t[REQUANT_TABLE_ENTRIES - 1] = 0;
 }
 
-RequantTable requant_table_for(int act, float s_src, float s_flt, float s_dst) {
-    static ScaleCache<RequantTable> cache;
+std::shared_ptr<const RequantTable> requant_table_for(int act, float s_src, float s_flt, float s_dst) {
+    static ScaleCache<std::shared_ptr<const RequantTable>> cache;
     const auto key = cache.key(act, s_src, s_flt, s_dst);
-    RequantTable t;
-    if (cache.find(key, &t))
-        return t;
+    std::shared_ptr<const RequantTable> found;
+    if (cache.find(key, &found))
+        return found;
+    const std::shared_ptr<RequantTable> t = std::make_shared<RequantTable>();
     const float c = make_requant_fast(s_src, s_flt, s_dst).c;
     if (act == MEGCC_NONLINE_RELU)
-        requant_thresholds<MEGCC_NONLINE_RELU>(s_src, s_flt, s_dst, c, t.t);
+        requant_thresholds<MEGCC_NONLINE_RELU>(s_src, s_flt, s_dst, c, t->t);
     else if (act == MEGCC_NONLINE_H_SWISH)
-        requant_thresholds<MEGCC_NONLINE_H_SWISH>(s_src, s_flt, s_dst, c, t.t);
+        requant_thresholds<MEGCC_NONLINE_H_SWISH>(s_src, s_flt, s_dst, c, t->t);
     else
-        requant_thresholds<MEGCC_NONLINE_IDENTITY>(s_src, s_flt, s_dst, c, t.t);
+        requant_thresholds<MEGCC_NONLINE_IDENTITY>(s_src, s_flt, s_dst, c, t->t);
     cache.put(key, t);
     return t;
 }
@@ -200,7 +201,7 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
     if (cache.find(key, &found))
         return found;
     const int lo = act == MEGCC_NONLINE_RELU ? 0 : -128;
-    const RequantSteps pts = requant_steps(requant_table_for(act, s_src, s_flt, s_dst), lo);
+    const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), lo);
     RequantBounds from, to;  // floor(a c + d) == y  <=>  y <= a c + d < y + 1
     for (int i = 0; i < pts.n; ++i) {
         if (pts.y[i] > lo)
@@ -259,7 +260,7 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
         return found;
     const bool relu = act == MEGCC_NONLINE_RELU;
     const int lowest = relu ? 0 : -128;
-    const RequantSteps pts = requant_steps(requant_table_for(act, s_src, s_flt, s_dst), lowest);
+    const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), lowest);
     // the forms in order of cost: no product in front, one, two
     struct Form {
         int mode;
