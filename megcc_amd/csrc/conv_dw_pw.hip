@@ -23,8 +23,11 @@
 //   product runs; two tile buffers, one barrier per tile.
 // Both requantisations are the exact ones of epilogue.h, so the result is bit for bit the two kernels'.
 // Bound: HBM on the large maps, the vector ALU's requantisation and the filter's way from L2 on the small
-// ones. Measured (N=64, us, one kernel / two): 32x112x112->64 22.5 / 33.8, 64 s2 -> 128 18.4 / 26.6,
-// 128x56x56->128 19.6 / 29.5, 256x28x28->256 15.7 / 23.0, 512x14x14->512 11.4 / 22.3; N=256: 87 / 119 and 34 / 49.
+// ones; with one tile a workgroup the way from the launch to the first load (dp_begin).
+// Measured (N=64, us, one kernel / two): 32x112x112->64 20.2 / 32.4, 64 s2 -> 128 17.2 / 25.5, 128x56x56->128 17.3 / 28.8,
+// 256x28x28->256 13.3 / 22.1, 512x14x14->512 10.5 / 21.7, 1024x7x7->1024 14.3 / 20.2; N=1: 4.3 / 6.8, 4.8 / 6.3, 4.2 / 6.9,
+// 5.6 / 7.3, 9.0 / 8.0, 13.4 / 9.9; N=256: 88 / 117 and, 512 channels, 32.7 / 49.5. (With the arguments read where they are
+// used, a filter ring of 8 chunks and every store's address of its own, N=1: 5.1, 5.6, 5.2, 6.4, 9.7, 17.0.)
 #include <map>
 #include <mutex>
 
@@ -40,6 +43,7 @@ static constexpr int DP_ALL_BUT_MFMA = 0x7f6;  // what may cross a scheduling ba
 typedef unsigned dp_v2u __attribute__((ext_vector_type(2)));
 
 struct DwPwParams {
+    // read together at the start of the kernel (dp_begin)
     const uint32_t* src;
     const uint32_t* dflt;    // [C/4][3][3] dwords of 4 channel bytes
     const int32_t* dbias;    // or NULL
@@ -49,13 +53,25 @@ struct DwPwParams {
     int src_bytes, dst_bytes;
     int ih, iw, oh, ow, OC, OCP;
     int plane;               // bytes of an input plane set
-    int xg, groups, tiles;   // groups of 4 pixels per row, in all; tiles of 16 SUB groups
+    int xg, groups;          // groups of 4 pixels per row, in all (a tile: 16 SUB groups)
     int slices;              // workgroups that share a tile's output channels
-    FastDiv d_xg, d_oh;
+    int nb, run_q, run_r;    // workgroups; tiles of a run, and how many runs have one more
+    FastDiv d_xg, d_oh, d_slices;
     RequantPack dq, pq;
     float dc, pc;            // estimates for the tables (mode 0)
     RequantTable dtable, ptable;
 };
+
+// The arguments as the first thing, all of them in one round trip: the compiler otherwise asks for each where it is used, and
+// nine round trips one after the other stood in front of the first load (3300 of a workgroup's 22000 cycles at 512 channels;
+// 0.9 us of every launch).
+__device__ __forceinline__ void dp_begin(const DwPwParams& q) {
+#ifndef MG_HOST_AUDIT
+    asm volatile("" ::"s"(q.src), "s"(q.dflt), "s"(q.dbias), "s"(q.wp), "s"(q.pbias), "s"(q.dst), "s"(q.src_bytes), "s"(q.dst_bytes), "s"(q.ih),
+                 "s"(q.iw), "s"(q.oh), "s"(q.ow), "s"(q.OC), "s"(q.OCP), "s"(q.plane), "s"(q.xg), "s"(q.groups), "s"(q.slices), "s"(q.nb),
+                 "s"(q.run_q), "s"(q.run_r), "s"(q.d_xg.mul), "s"(q.d_oh.mul), "s"(q.d_slices.mul), "s"(q.dq.mode), "s"(q.pq.mode));
+#endif
+}
 
 // 16 accumulators of one column -> 4 dwords (each 4 consecutive registers)
 // The empty volatile statements keep each form inside its branch: the compiler otherwise computes one of
@@ -108,9 +124,11 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
     constexpr int JW = NQ * SUB / 8;                 // channel-wise jobs per wave and tile
     constexpr int WP = T / (32 * NT), WO = 8 / WP;   // waves along the pixels, along the channels
     constexpr bool KEEP_D = JW == 1 && S == 1, KEEP_P = KC * MT <= 8;
-    // chunks of the pointwise filter in flight (not KEEP_P): as many as the registers hold without spilling
-    constexpr int RING = KC >= 32 ? 2 : KC == 16 && S == 2 ? 4 : 8;
+    // chunks of the pointwise filter in flight (not KEEP_P). More of them only stand in front of the channel-wise
+    // operands: 8 for 4 chunks, 512 channels at N=256 33.1 for 32.2 us, stride 2 21.2 for 20.4
+    constexpr int RING = KC >= 16 ? 4 : 8;
     static_assert(JW >= 1 && WP >= 1 && WO >= 1 && WP * WO == 8, "8 waves");
+    dp_begin(q);
     extern __shared__ __attribute__((aligned(16))) int8_t dp_lds_mem[];
     int8_t* const mid = dp_lds_mem;                             // [2][NQ][T] 16-byte pieces
     int* const wl = (int*)(mid + 2 * T * C);                    // [C][4]: per channel the filter's 3 rows
@@ -123,11 +141,9 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
     int* const ptbl = dtbl + REQUANT_TABLE_ENTRIES;
 
     // workgroup -> (slice, run of tiles); each XCD gets a contiguous stretch of the runs
-    const int nb = gridDim.x;
-    const int lb = (nb & 7) == 0 ? (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
-    const int slice = lb % q.slices, wi = lb / q.slices, nw = nb / q.slices;
-    const int run_q = q.tiles / nw, run_r = q.tiles - run_q * nw;
-    const int t_begin = wi * run_q + min(wi, run_r), t_end = t_begin + run_q + (wi < run_r ? 1 : 0);
+    const int lb = (q.nb & 7) == 0 ? (blockIdx.x & 7) * (q.nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    const int wi = (int)fdiv(lb, q.d_slices), slice = lb - wi * q.slices;
+    const int t_begin = wi * q.run_q + min(wi, q.run_r), t_end = t_begin + q.run_q + (wi < q.run_r ? 1 : 0);
 
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)q.src, 0, q.src_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)q.dst, 0, q.dst_bytes, 0x00020000);
@@ -230,22 +246,26 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
     // pointwise filter rows of this wave
     const int wo = wave % WO, wpx = wave / WO;
     const int oc_wave = slice * ocs + wo * (32 * MT);
-    const int8_t* prow[MT];
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)q.wp, 0, KC * KROW * q.OCP, 0x00020000);
+    const int cstep = q.OCP * KROW;
+    int prow[MT];
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi) {
         const int oc = min(oc_wave + mi * 32, q.OCP - 32) + col;
-        prow[mi] = q.wp + (size_t)oc * KROW + (((kg ^ (oc >> 3)) & 1) << 4);
+        prow[mi] = oc * KROW + (((kg ^ (oc >> 3)) & 1) << 4);
     }
-    const size_t cstep = (size_t)q.OCP * KROW;
     v4i P[KEEP_P ? KC : RING][MT];
+    auto filter = [&](v4i (&P)[MT], int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi)
+            P[mi] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, prow[mi], c * cstep, 0));
+    };
     if (KEEP_P) {
 #pragma unroll
         for (int c = 0; c < KC; ++c)
-#pragma unroll
-            for (int mi = 0; mi < MT; ++mi)
-                P[KEEP_P ? c : 0][mi] = *(const v4i*)(prow[mi] + c * cstep);
+            filter(P[KEEP_P ? c : 0], c);
     }
-    __syncthreads();
+    lds_barrier();
     struct Band {
         v4i m[S];
         dp_v2u e;  // left, right
@@ -273,162 +293,158 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
         }
     }
 
-    // (nothing in flight from here: the loop's own waits are then exact)
-    wait_vmcnt<0>();
-    for (int t = t_begin, buf = 0; t < t_end; ++t, buf ^= 1) {
-        // the pointwise filter's first chunks fly while the channel-wise stage runs
-        if (!KEEP_P) {
+    // one channel-wise job: 16 channels (plane sets 4 quad ..), 64 pixels; `next` asks for what comes after it as soon as
+    // its operands are consumed, so that those loads fly while this one is requantised
+    auto channelwise = [&](int quad, int u, int8_t* m, auto next) __attribute__((always_inline)) {
+        v4i acc[4];
+        // the pixels left and right of each column's group
+        unsigned L[4], R[4];
 #pragma unroll
-            for (int c = 0; c < RING; ++c)
-#pragma unroll
-                for (int mi = 0; mi < MT; ++mi)
-                    P[c][mi] = *(const v4i*)(prow[mi] + c * cstep);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int p = 0; p < 4; ++p) {
+            L[p] = E[p];
+            R[p] = E[p];
         }
-        int8_t* const m = mid + buf * (T * C);
-        // ---- channel-wise ----------------------------------------------------------------------------
-#pragma unroll
-        for (int i = 0; i < JW; ++i) {
-            const int quad = quad_of(i), u = sub_of(i);
-            v4i acc[4];
-            if (i == 0)
-                cur = rows;
-            // the pixels left and right of each column's group
-            unsigned L[4], R[4];
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                L[p] = E[p];
-                R[p] = E[p];
-            }
 #ifndef MG_HOST_AUDIT
-            // (one block: a DPP read needs two cycles behind a vector write of its source)
+        // (one block: a DPP read needs two cycles behind a vector write of its source)
+        asm volatile(
+                "s_nop 1\n\t"
+                "v_and_b32_dpp %0, %4, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                "v_and_b32_dpp %1, %5, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                "v_and_b32_dpp %2, %6, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                "v_and_b32_dpp %3, %7, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                "s_nop 1"
+                : "+v"(L[0]), "+v"(L[1]), "+v"(L[2]), "+v"(L[3])
+                : "v"(B[0][S - 1][3]), "v"(B[1][S - 1][3]), "v"(B[2][S - 1][3]), "v"(B[3][S - 1][3]), "v"(cur.lmask));
+        if (S == 1)
             asm volatile(
                     "s_nop 1\n\t"
-                    "v_and_b32_dpp %0, %4, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
-                    "v_and_b32_dpp %1, %5, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
-                    "v_and_b32_dpp %2, %6, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
-                    "v_and_b32_dpp %3, %7, %8 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                    "v_and_b32_dpp %0, %4, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                    "v_and_b32_dpp %1, %5, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                    "v_and_b32_dpp %2, %6, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                    "v_and_b32_dpp %3, %7, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
                     "s_nop 1"
-                    : "+v"(L[0]), "+v"(L[1]), "+v"(L[2]), "+v"(L[3])
-                    : "v"(B[0][S - 1][3]), "v"(B[1][S - 1][3]), "v"(B[2][S - 1][3]), "v"(B[3][S - 1][3]), "v"(cur.lmask));
-            if (S == 1)
-                asm volatile(
-                        "s_nop 1\n\t"
-                        "v_and_b32_dpp %0, %4, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
-                        "v_and_b32_dpp %1, %5, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
-                        "v_and_b32_dpp %2, %6, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
-                        "v_and_b32_dpp %3, %7, %8 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
-                        "s_nop 1"
-                        : "+v"(R[0]), "+v"(R[1]), "+v"(R[2]), "+v"(R[3])
-                        : "v"(B[0][0][0]), "v"(B[1][0][0]), "v"(B[2][0][0]), "v"(B[3][0][0]), "v"(cur.rmask));
+                    : "+v"(R[0]), "+v"(R[1]), "+v"(R[2]), "+v"(R[3])
+                    : "v"(B[0][0][0]), "v"(B[1][0][0]), "v"(B[2][0][0]), "v"(B[3][0][0]), "v"(cur.rmask));
 #endif
-            // The short products of all four plane sets first, and every product where it stands (a scheduling
-            // barrier behind each that only products may not cross). Products of ONE shape take their sums from the one
-            // before at any distance; between the two shapes the sum must have been written: a 16x16x64 product
-            // directly behind its 16x16x32 one has read channels 0 and 1 of the last pixels before that. A short
-            // product takes 4 passes of 4 cycles and a few cycles to write; the three products in between alone
-            // take 12 passes. (The build's code is checked for the three: test_mfma_order.py.)
-            unsigned w[4];
+        // The short products of all four plane sets first, and every product where it stands (a scheduling
+        // barrier behind each that only products may not cross). Products of ONE shape take their sums from the one
+        // before at any distance; between the two shapes the sum must have been written: a 16x16x64 product
+        // directly behind its 16x16x32 one has read channels 0 and 1 of the last pixels before that. A short
+        // product takes 4 passes of 4 cycles and a few cycles to write; the three products in between alone
+        // take 12 passes. (The build's code is checked for the three: test_mfma_order.py.)
+        unsigned w[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            acc[p] = *(const v4i*)(db + quad * 16 + p * 4);
+            if (!KEEP_D)
+                w[p] = band_filter(quad, p);
+        }
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const dp_v2u al = KEEP_D ? A[KEEP_D ? p : 0].e : band_edges(w[p]), bl = {L[p], S == 1 ? R[p] : L[p]};
+            acc[p] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                    __builtin_bit_cast(long, al), __builtin_bit_cast(long, bl), acc[p], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(DP_ALL_BUT_MFMA);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < S; ++h)
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
-                acc[p] = *(const v4i*)(db + quad * 16 + p * 4);
-                if (!KEEP_D)
-                    w[p] = band_filter(quad, p);
-            }
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const dp_v2u al = KEEP_D ? A[KEEP_D ? p : 0].e : band_edges(w[p]), bl = {L[p], S == 1 ? R[p] : L[p]};
-                acc[p] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
-                        __builtin_bit_cast(long, al), __builtin_bit_cast(long, bl), acc[p], 0, 0, 0);
+                v4i b = B[p][h];
+                if (RAG)
+                    b[RAG] = (h == 0 ? cur.edge : cur.edgeb) ? 0 : b[RAG];
+                acc[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                        KEEP_D ? A[KEEP_D ? p : 0].m[h] : band_half(w[p], h), b, acc[p], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(DP_ALL_BUT_MFMA);
             }
-            __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_sched_barrier(0);
+        next();
+        int a[16];
 #pragma unroll
-            for (int h = 0; h < S; ++h)
+        for (int p = 0; p < 4; ++p)
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    v4i b = B[p][h];
-                    if (RAG)
-                        b[RAG] = (h == 0 ? cur.edge : cur.edgeb) ? 0 : b[RAG];
-                    acc[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                            KEEP_D ? A[KEEP_D ? p : 0].m[h] : band_half(w[p], h), b, acc[p], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(DP_ALL_BUT_MFMA);
-                }
-            __builtin_amdgcn_sched_barrier(0);
-            // the operands are consumed: the next job's loads fly while this one is requantised
+            for (int e = 0; e < 4; ++e)
+                a[p * 4 + e] = acc[p][e];
+        uint32_t d[4];
+        dp_requant<DACT>(a, d, q.dq, q.dc, dtbl);
+        *(v4i*)(m + (quad * T + u * 64 + colq * 4 + kg4) * 16) = v4i{(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
+    };
+    // ---- pointwise: where a column's results go. (Stores are issued whether or not the place exists: what is under no
+    // condition the compiler can count, and the next tile then waits for its loads, not for these stores.)
+    const int ostep = q.oh * q.ow * 4;  // bytes of a plane set of the result
+    auto where = [&](int t, int ni) __attribute__((always_inline)) {
+        const int s = (wpx * NT + ni) * 32 + col;
+        const int g = t * (16 * SUB) + (s >> 2);
+        const int rg = (int)fdiv(g, q.d_xg), x = (g - rg * q.xg) * 4 + (s & 3);
+        const int n = (int)fdiv(rg, q.d_oh), y = rg - n * q.oh;
+        const unsigned o = (unsigned)((n * (q.OC >> 2) * q.oh + y) * q.ow + x) * 4u + (unsigned)(kg * ostep);
+        return g < q.groups && x < q.ow ? o : OOB;
+    };
+    auto bias_of = [&](int mi, v16i& acc) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+            const v4i bv = *(const v4i*)(pb + wo * (32 * MT) + mi * 32 + e4 * 8 + kg * 4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                acc[e4 * 4 + k] = bv[k];
+        }
+    };
+    auto finish = [&](int mi, unsigned w, const v16i& acc) __attribute__((always_inline)) {
+        int a[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            a[e] = acc[e];
+        uint32_t d[4];
+        dp_requant<PACT>(a, d, q.pq, q.pc, ptbl);
+        // (OC is a multiple of 32: all of the tile's channels exist or none)
+        const bool there = oc_wave + mi * 32 < q.OC;
+        const unsigned o = there ? w : OOB;
+        const int plane = there ? (oc_wave + mi * 32) >> 2 : 0;
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4)
+            __builtin_amdgcn_raw_buffer_store_b32(d[e4], rd, (int)o, (plane + e4 * 2) * ostep, 0);
+    };
+    auto operand = [&](const int8_t* m, int c, int ni) __attribute__((always_inline)) {
+        return *(const v4i*)(m + ((2 * c + kg) * T + (wpx * NT + ni) * 32 + col) * 16);
+    };
+    // (nothing in flight from here: the loop's own waits are then exact)
+    if (KEEP_P)
+        wait_vmcnt<0>();
+    for (int t = t_begin, buf = 0; t < t_end; ++t, buf ^= 1) {
+        int8_t* const m = mid + buf * (T * C);
+        cur = rows;
+        static_for<JW>([&](auto ii) {
+            constexpr int i = decltype(ii)::value;
             // (several jobs a tile: tiles of 64 pixels, the same rows for all of them)
             static_assert(JW == 1 || SUB == 1, "");
-            if (KEEP_P || i + 1 < JW) {
-                if (i + 1 == JW)
+            channelwise(quad_of(i), sub_of(i), m, [&]() __attribute__((always_inline)) {
+                if (i + 1 < JW) {
+                    request(rows, quad_of(i + 1));
+                } else if (KEEP_P) {
                     rows = rows_of(t + 1, sub_of(0));
-                request(rows, quad_of(i + 1 < JW ? i + 1 : 0));
-            }
-            int a[16];
+                    request(rows, quad_of(0));
+                } else {
+                    // the pointwise filter's first chunks
 #pragma unroll
-            for (int p = 0; p < 4; ++p)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    a[p * 4 + e] = acc[p][e];
-            uint32_t d[4];
-            dp_requant<DACT>(a, d, q.dq, q.dc, dtbl);
-            *(v4i*)(m + (quad * T + u * 64 + colq * 4 + kg4) * 16) = v4i{(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
-        }
+                    for (int c = 0; c < RING; ++c)
+                        filter(P[c], c);
+                }
+            });
+        });
         lds_barrier();
-        // ---- pointwise -------------------------------------------------------------------------------
-        // where a column's results go. (Stores are issued whether or not the place exists: what is under no
-        // condition the compiler can count, and the next tile then waits for its loads, not for these stores.)
-        struct Where {
-            unsigned base;
-            bool ok;
-        };
-        auto where = [&](int ni) __attribute__((always_inline)) -> Where {
-            const int s = (wpx * NT + ni) * 32 + col;
-            const int g = t * (16 * SUB) + (s >> 2);
-            const int rg = (int)fdiv(g, q.d_xg), x = (g - rg * q.xg) * 4 + (s & 3);
-            const int n = (int)fdiv(rg, q.d_oh), y = rg - n * q.oh;
-            Where w;
-            w.ok = g < q.groups && x < q.ow;
-            w.base = (unsigned)((n * (q.OC >> 2) * q.oh + y) * q.ow + x) * 4u;
-            return w;
-        };
-        const unsigned ostep = (unsigned)(q.oh * q.ow) * 4u;
-        auto bias_of = [&](int mi, v16i& acc) __attribute__((always_inline)) {
-#pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                const v4i bv = *(const v4i*)(pb + wo * (32 * MT) + mi * 32 + e4 * 8 + kg * 4);
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    acc[e4 * 4 + k] = bv[k];
-            }
-        };
-        auto finish = [&](int mi, const Where& w, const v16i& acc) __attribute__((always_inline)) {
-            int a[16];
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                a[e] = acc[e];
-            uint32_t d[4];
-            dp_requant<PACT>(a, d, q.pq, q.pc, ptbl);
-#pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                const int oc4 = ((oc_wave + mi * 32) >> 2) + e4 * 2 + kg;
-                __builtin_amdgcn_raw_buffer_store_b32(d[e4], rd, (int)(oc4 * 4 < q.OC && w.ok ? w.base + (unsigned)oc4 * ostep : OOB), 0, 0);
-            }
-        };
-        auto operand = [&](int c, int ni) __attribute__((always_inline)) {
-            return *(const v4i*)(m + ((2 * c + kg) * T + (wpx * NT + ni) * 32 + col) * 16);
-        };
         if constexpr (KEEP_P) {
             // one 32 x 32 tile after the other: 16 accumulators live, four waves to a SIMD
 #pragma unroll
             for (int ni = 0; ni < NT; ++ni) {
-                const Where w = where(ni);
+                const unsigned w = where(t, ni);
 #pragma unroll
                 for (int mi = 0; mi < MT; ++mi) {
                     v16i acc;
                     bias_of(mi, acc);
 #pragma unroll
                     for (int c = 0; c < KC; ++c)
-                        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(P[c][mi], operand(c, ni), acc, 0, 0, 0);
+                        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(P[c][mi], operand(m, c, ni), acc, 0, 0, 0);
                     finish(mi, w, acc);
                 }
             }
@@ -445,16 +461,13 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
                 constexpr int c = decltype(cc)::value, slot = c % RING;
 #pragma unroll
                 for (int ni = 0; ni < NT; ++ni) {
-                    const v4i b = operand(c, ni);
+                    const v4i b = operand(m, c, ni);
 #pragma unroll
                     for (int mi = 0; mi < MT; ++mi)
                         acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(P[slot][mi], b, acc[mi][ni], 0, 0, 0);
                 }
-                if (c + RING < KC) {
-#pragma unroll
-                    for (int mi = 0; mi < MT; ++mi)
-                        P[slot][mi] = *(const v4i*)(prow[mi] + (c + RING) * cstep);
-                }
+                if (c + RING < KC)
+                    filter(P[slot], c + RING);
                 // the next tile's first job, behind the last chunk of the filter: loads come back in the order they
                 // were issued, and one asked for after these would wait for them
                 if (c + (RING < KC ? RING : KC) == KC) {
@@ -465,7 +478,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
             });
 #pragma unroll
             for (int ni = 0; ni < NT; ++ni) {
-                const Where w = where(ni);
+                const unsigned w = where(t, ni);
 #pragma unroll
                 for (int mi = 0; mi < MT; ++mi)
                     finish(mi, w, acc[mi][ni]);
@@ -553,11 +566,12 @@ TinyNNStatus conv_dw_pw_launch(
     q.plane = dw.ih * dw.iw * 4;
     q.xg = (dw.ow + 3) / 4;
     q.groups = dw.n * dw.oh * q.xg;
-    q.tiles = (q.groups + 16 * s.sub - 1) / (16 * s.sub);
+    const int tiles = (q.groups + 16 * s.sub - 1) / (16 * s.sub);
     const int wo = 8 / (64 * s.sub / (32 * s.nt)), ocs = wo * 32 * s.mt;
     q.slices = (pw.oc + ocs - 1) / ocs;
     q.d_xg = make_fastdiv(q.xg);
     q.d_oh = make_fastdiv(q.oh);
+    q.d_slices = make_fastdiv(q.slices);
     q.dq = requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
     q.pq = requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
     q.dc = make_requant_fast(dw.s_src, dw.s_flt, dw.s_dst).c;
@@ -569,7 +583,7 @@ TinyNNStatus conv_dw_pw_launch(
     const int rag = dw.iw & 3;
     void (*kern)(DwPwParams) = nullptr;
     size_t lds = 0;
-#define MG_DP(KC_, SUB_, MT_, NT_)                                                                                   \
+#define MG_DP(KC_, SUB_, MT_, NT_)                                                                               \
     if (s.kc == KC_ && s.mt == MT_ && s.nt == NT_) {                                                                   \
         kern = dw.sh == 1 ? dp_kernel<1, KC_, SUB_, MT_, NT_>(rag, dw.act, pw.act) : dp_kernel<2, KC_, SUB_, MT_, NT_>(rag, dw.act, pw.act); \
         lds = (size_t)dp_lds<KC_, SUB_>(ocs);                                                                          \
@@ -590,11 +604,13 @@ TinyNNStatus conv_dw_pw_launch(
     long runs = (long)num_cus() * resident / q.slices;
     if (runs < 1)
         runs = 1;
-    if (runs > q.tiles)
-        runs = q.tiles;
+    if (runs > tiles)
+        runs = tiles;
+    q.nb = (int)runs * q.slices;
+    q.run_q = tiles / (int)runs, q.run_r = tiles - q.run_q * (int)runs;
     note_kernel("conv_dw_pw", dw.ic / 32, dw.sh, q.slices);
     note_requant_affine(q.dq.mode != 0 && q.pq.mode != 0);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(runs * q.slices)), dim3(DP_THREADS), lds, stream(), q);
+    hipLaunchKernelGGL(kern, dim3((unsigned)q.nb), dim3(DP_THREADS), lds, stream(), q);
     return check_launch("conv_dw_pw");
 }
 
