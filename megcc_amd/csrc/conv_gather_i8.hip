@@ -9,29 +9,31 @@
 //     contiguous KB of the packed filter; the activation operand of 32 pixels is four dwords per lane, pixel = lane,
 //     32 lanes on consecutive pixels of one channel group's plane;
 //   * a tap outside the image turns the lane's offset into one beyond the tensor, which a buffer load answers with
-//     zero; channel groups beyond the last meet zero filter rows, and offsets beyond the tensor read zero too. Steps
-//     beyond a wave's share read zero the same way, so no load is under a condition. The whole offset is in the
-//     lane's register: the range check sees all of it;
+//     zero; channel groups beyond the last meet zero filter rows, and offsets beyond the tensor read zero too. The
+//     whole offset is in the lane's register: the range check sees all of it;
 //   * RING steps are in flight per wave;
 //   * the waves of a workgroup share K (KW groups) and the pixels (the rest): small layers split K so that every CU
 //     has work; the groups' int32 sums meet in LDS, each group finishing its share of the tile.
 // Bound by the loads' way through the CU's address and data path (64 x 64 outputs a wave: 64 cycles of it a step for
-// 32 of its matrix units) on large layers and by the chain of steps of one wave on small ones. Measured (us, before:
-// the one-stage kernel of conv_mfma_i8.hip, beyond 9 taps conv_dot4.hip): 6 x 88 -> 148 57 x 43 stride 2 14.6 -> 7.1, 4 x
-// 24 -> 68 98 x 98 stride 2 14.8 -> 5.7, 1 x 356 -> 52 68 x 81 21.2 -> 8.5, 1 x 256 -> 256 28 x 28 8.0 -> 5.7, 47 x 104 -> 48 89 x 89 95.8 -> 51.2, 58 x
-// 264 -> 320 70 x 70 stride 2 216 -> 183; 5x5: 1 x 120 -> 280 19 x 19 134 -> 6.7, 60 x 28 -> 20 63 x 63 137 -> 21.7.
+// 32 of its matrix units; on small layers too, 4 waves' steps of 5 loads each). Measured (us, before: the one-stage
+// kernel of conv_mfma_i8.hip, beyond 9 taps conv_dot4.hip; then with steps beyond a wave's share fetched as zeros, the
+// table read before the first operand and the arguments where they are used; now): 6 x 88 -> 148 57 x 43 stride 2
+// 14.6, 7.1, 5.9; 4 x 24 -> 68 98 x 98 stride 2 14.8, 5.7, 4.2; 1 x 356 -> 52 68 x 81 21.2, 8.4, 7.6; 1 x 256 -> 256 28 x 28
+// 8.0, 5.6, 5.0; 47 x 104 -> 48 89 x 89 95.8, 50.5, 41.9; 58 x 264 -> 320 70 x 70 stride 2 216, 176, 171; 5x5: 1 x 120 -> 280
+// 19 x 19 134, 6.6, 5.8; 60 x 28 -> 20 63 x 63 137, 21.4, 17.4.
 // Reference loop: BareMetal/ConvKernel.cpp:305-344.
 #include "conv_mfma_i8.h"
 
 namespace mg {
 
 struct GatherParams {
+    // (what is read together at the start of the kernel: gather_begin)
     const int8_t* src;
     const int8_t* wp;     // packed filter [chunk][tap][OCP][32], 16-byte halves swapped when (oc >> 3) & 1
     const int32_t* bias;  // [OC] or NULL
     int8_t* dst;
     unsigned src_bytes, wp_bytes;
-    int P, OC, steps, taps, kw;  // steps = chunks * taps
+    int P, OC, steps, taps, lkw;  // steps = chunks * taps; log2 of the groups that share K
     unsigned step_bytes;         // of the packed filter
     unsigned plane, image, row;  // bytes of the source
     int IH, IW, OHW, OW, FW, SH, SW, PH, PW, DH, DW;
@@ -42,6 +44,16 @@ struct GatherParams {
     RequantTable table;
 };
 
+// The arguments as the first thing, in one round trip: asked for where they are used, up to four round trips one
+// after the other stood in front of the first load.
+__device__ __forceinline__ void gather_begin(const GatherParams& q) {
+#ifndef MG_HOST_AUDIT
+    asm volatile("" ::"s"(q.src), "s"(q.wp), "s"(q.bias), "s"(q.dst), "s"(q.src_bytes), "s"(q.wp_bytes), "s"(q.P), "s"(q.OC), "s"(q.steps), "s"(q.taps),
+                 "s"(q.lkw), "s"(q.step_bytes), "s"(q.plane), "s"(q.image), "s"(q.row), "s"(q.IH), "s"(q.IW), "s"(q.OHW), "s"(q.OW), "s"(q.SH), "s"(q.SW),
+                 "s"(q.PH), "s"(q.PW), "s"(q.DH), "s"(q.DW), "s"(q.dOHW.mul), "s"(q.dOW.mul), "s"(q.dTaps.mul), "s"(q.dFW.mul), "s"(q.aff_d));
+#endif
+}
+
 // Entry i of the table, straight from the kernel-argument segment (conv_mfma_i8.h: kernarg_rq_table)
 __device__ __forceinline__ int gather_table(int i) {
     typedef const __attribute__((address_space(4))) char* kptr;
@@ -50,22 +62,21 @@ __device__ __forceinline__ int gather_table(int i) {
 }
 
 // ACT: an activation whose outputs the threshold table describes, or -1 (the literal sequence of q.act)
-static constexpr int GATHER_WAVES = 4;  // of a workgroup
+static constexpr int GATHER_LOG2_WAVES = 2, GATHER_WAVES = 1 << GATHER_LOG2_WAVES;  // of a workgroup
 
 template <int MT, int NT, int ACT>
 __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(GatherParams q) {
-    constexpr int RING = 4;
+    constexpr int RING = 4;  // steps in flight (8: no step faster, 256 -> 256 28 x 28 5.1 us for 5.0, 4 x 24 -> 68 4.9 for 4.2)
+    static_assert(64 * GATHER_WAVES == REQUANT_TABLE_ENTRIES, "an entry a thread");
     extern __shared__ __attribute__((aligned(16))) int gather_lds[];
-    if (ACT >= 0) {
-        if (threadIdx.x < REQUANT_TABLE_ENTRIES)
-            gather_lds[threadIdx.x] = gather_table(threadIdx.x);
-        __syncthreads();
-    }
-    int* const parts = gather_lds + REQUANT_TABLE_ENTRIES;
+    gather_begin(q);
+    int* const bias = gather_lds + REQUANT_TABLE_ENTRIES;  // [32 MT]
+    int* const parts = bias + 32 * MT;
     const int lane = threadIdx.x & 63, col = lane & 31, kg = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
-    const int kw = q.kw, pw = waves / kw;           // groups that share K, waves side by side in pixels
-    const int grp = wave / pw, sub = wave - grp * pw;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // groups that share K, waves side by side in pixels
+    const int kw = 1 << q.lkw, lpw = GATHER_LOG2_WAVES - q.lkw, pw = 1 << lpw;
+    const int grp = wave >> lpw, sub = wave & (pw - 1);
     const int oc0 = blockIdx.y * (32 * MT), p0 = (blockIdx.x * pw + sub) * (32 * NT);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)q.src, 0, (int)q.src_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)q.wp, 0, (int)q.wp_bytes, 0x00020000);
@@ -122,19 +133,45 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
 #pragma unroll
     for (int r = 0; r < RING; ++r)
         load(grp + r * kw, A[r], B[r]);
-    for (int t = 0; t < mine; t += RING) {
+    // What the outputs need is asked for behind the operands and waits in registers till the products are done.
+    const bool table = ACT >= 0 && q.aff_d == 0.f;
+    int entry = 0, bv = 0;
+    if (table)
+        entry = gather_table(threadIdx.x);
+    if (q.bias && threadIdx.x < 32 * MT)
+        bv = q.bias[min(oc0 + (int)threadIdx.x, q.OC - 1)];
+    auto multiply = [&](const v4i (&a)[MT], const v4i (&b)[NT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i], b[j], acc[i][j], 0, 0, 0);
+    };
+    int t = 0;
+    for (; t + 2 * RING <= mine; t += RING) {
 #pragma unroll
         for (int r = 0; r < RING; ++r) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[r][i], B[r][j], acc[i][j], 0, 0, 0);
+            multiply(A[r], B[r]);
             load(grp + (t + r + RING) * kw, A[r], B[r]);
         }
     }
+    // The last steps one by one: steps beyond the wave's share are neither asked for nor multiplied. (They read nothing,
+    // but 18 steps of the 28 x 28 layer of 256 channels went through the CU's address path as 24.)
+    for (; t < mine; t += RING) {
+#pragma unroll
+        for (int r = 0; r < RING; ++r)
+            if (t + r < mine) {
+                multiply(A[r], B[r]);
+                if (t + r + RING < mine)
+                    load(grp + (t + r + RING) * kw, A[r], B[r]);
+            }
+    }
     // [group][wave of it][quad][lane]: a quad is 4 neighbouring channels of the lane's pixel
     constexpr int QUADS = MT * NT * 4;
+    if (table)
+        gather_lds[threadIdx.x] = entry;
+    if (threadIdx.x < 32 * MT)
+        bias[threadIdx.x] = bv;
     if (kw > 1) {
 #pragma unroll
         for (int x = 0; x < QUADS; ++x)
@@ -143,8 +180,8 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
                 *(v4i*)(parts + ((wave * QUADS + x) * 64 + lane) * 4) =
                         v4i{t[x % 4 * 4], t[x % 4 * 4 + 1], t[x % 4 * 4 + 2], t[x % 4 * 4 + 3]};
             }
-        __syncthreads();
     }
+    __syncthreads();
 #pragma unroll
     for (int x = 0; x < QUADS; ++x) {
         if ((x & (kw - 1)) != grp)
@@ -163,19 +200,15 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
                 s[e] += o[e];
         }
         const int oc = oc0 + 32 * i + 8 * e4 + 4 * kg;
-        // (the bias of a lane without an output: some other channel's)
-        int bv[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            bv[e] = q.bias ? q.bias[min(oc, q.OC - 4) + e] : 0;
+        const v4i bq = *(const v4i*)(bias + 32 * i + 8 * e4 + 4 * kg);
         if (oc >= q.OC || p0 + 32 * j + col >= q.P)
             continue;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            s[e] += bv[e];
+            s[e] += bq[e];
         int r[4];
         if constexpr (ACT == MEGCC_NONLINE_IDENTITY || ACT == MEGCC_NONLINE_RELU) {
-            if (q.aff_d != 0.f) {
+            if (!table) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     r[e] = requant_conv_affine<ACT>(s[e], q.aff_c, q.aff_d);
@@ -275,7 +308,6 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     } else if (mt * nt == 4 && q.steps >= 72 && tiles() < 4 * full) {
         kw = 2;
     }
-    constexpr int waves = GATHER_WAVES;
 #define MG_GATHER_A(MT_, NT_)                                                                          \
     (!table                              ? conv_gather_i8_kernel<MT_, NT_, -1>                         \
      : g.act == MEGCC_NONLINE_IDENTITY   ? conv_gather_i8_kernel<MT_, NT_, MEGCC_NONLINE_IDENTITY>     \
@@ -284,19 +316,19 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     void (*kern)(GatherParams) = mt == 2 ? (nt == 2 ? MG_GATHER_A(2, 2) : MG_GATHER_A(2, 1))
                                          : (nt == 2 ? MG_GATHER_A(1, 2) : MG_GATHER_A(1, 1));
 #undef MG_GATHER_A
-    const int pw = waves / kw;
+    const int pw = GATHER_WAVES / kw;
     const dim3 grid((unsigned)((q.P + 32 * nt * pw - 1) / (32 * nt * pw)), (unsigned)((g.oc + 32 * mt - 1) / (32 * mt)));
-    q.kw = kw;
+    q.lkw = kw == 4 ? 2 : kw == 2 ? 1 : 0;
     note_kernel("conv_mfma_i8_gather", 32 * mt, 32 * nt, kw);
     const RequantAffine aff = requant_affine_pick(table, g.act, g.s_src, g.s_flt, g.s_dst);
     q.aff_c = aff.c;
     q.aff_d = aff.d;
-    const size_t lds = REQUANT_TABLE_ENTRIES * 4 + (kw > 1 ? (size_t)waves * mt * nt * 4096 : 0);
+    const size_t lds = (REQUANT_TABLE_ENTRIES + 32 * mt) * 4 + (kw > 1 ? (size_t)GATHER_WAVES * mt * nt * 4096 : 0);
     if (lds > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_gather_i8: LDS attribute: %s", hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(kern, grid, dim3(64 * waves), lds, stream(), q);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * GATHER_WAVES), lds, stream(), q);
     return check_launch("conv_gather_i8");
 }
 
