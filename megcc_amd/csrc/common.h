@@ -41,16 +41,20 @@ TinyNNStatus fail(TinyNNStatus st, const char* fmt, ...) __attribute__((format(p
 struct XcdOrder {
     int w;
 };
-inline XcdOrder make_xcd_order(int gx, int gy) {
-    const long nb = (long)gx * gy;
-    if (nb < 64 || (nb & 7) != 0)
-        return {0};
+// the strip for `tiles` tiles in rows of gx; 0: too few
+inline int xcd_strip(int gx, long tiles) {
+    if (tiles < 64)
+        return 0;
     // w ~ sqrt(tiles per XCD / 2): the half of its share an XCD has resident at a time is about square
     // (a round of workgroups streams its panels through the 4 MB L2 once; the next round starts over)
     int w = 1;
-    while ((long)w * w * 8 <= nb / 8)
+    while ((long)w * w * 8 <= tiles / 8)
         w *= 2;
-    return {w < gx ? w : gx};
+    return w < gx ? w : gx;
+}
+inline XcdOrder make_xcd_order(int gx, int gy) {
+    const long nb = (long)gx * gy;
+    return {(nb & 7) != 0 ? 0 : xcd_strip(gx, nb)};
 }
 __device__ __forceinline__ void xcd_tile(XcdOrder o, int bx, int by, int gx, int gy, int& tx, int& ty) {
     tx = bx;

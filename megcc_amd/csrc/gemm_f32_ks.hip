@@ -21,10 +21,11 @@
 // Sums: a wave closes its running sums every 64 values of K into a second set of registers; the waves' sums are
 // added in wave order. (Without that, relative error against 64 bits of 64 x 4096 x 4096 4.1e-7, of 197 x 771 x 1003
 // 2.5e-7, where the tiled kernel's slices of K had 3.0e-7 and 1.7e-7.) Fp32MatMulM4N12.cpp:9-158, Fp32Im2col.cpp:88-218 are the loops replaced.
-// Measured (us, before: the tiled kernel with its slice sums in a second launch, or conv_f32_small.hip):
-// 64 x 4096 x 4096 35.4 -> 24.0 (2.9 TB/s and 90 TFLOP/s), 197 x 771 x 1003 nt 19.9 -> 7.5,
-// 8 x 284 x 736 16.5 -> 4.0, 1623 x 3660 x 316 73 -> 41; convolution 32 -> 32 on 56 x 56 6.9 -> 5.1, N=8
-// 64 -> 64 on 56 x 56 55 -> 29, N=8 128 -> 128 165 -> 82.
+// Where there are too few 32 x 32 tiles for every CU, 16 x 16 ones (v_mfma_f32_16x16x4_f32, steps of 16, one tile a workgroup).
+// Measured (us, before: the tiled kernel with its slice sums in a second launch, or conv_f32_small.hip; with 32 x 32 tiles; now):
+// 64 x 4096 x 4096 35.4, 24.0, 23.6 (2.9 TB/s and 90 TFLOP/s), 197 x 771 x 1003 nt 19.9, 7.5, 7.5, 8 x 284 x 736 16.5, 4.0, 3.7,
+// 1623 x 3660 x 316 73, 38, 35, 64 x 1024 x 1000 7.5, 4.8 with 16 x 16, 50 x 4000 x 500 21.1, 10.9, 128 x 2048 x 512 nt 17.0, 9.1;
+// convolution 32 -> 32 on 56 x 56 6.9, 5.0, 4.2, 64 -> 64 28 x 28 6.7, 4.4, N=8 64 -> 64 on 56 x 56 55, 28, 27.6.
 #include "common.h"
 #include "conv_geom.h"
 #include "conv_mfma_i8.h"
@@ -35,6 +36,17 @@ namespace mg {
 
 typedef float ks_v16f __attribute__((ext_vector_type(16)));
 typedef float ks_v4f __attribute__((ext_vector_type(4)));
+// the sums of an R x R tile and its product with K = 64 / R
+template <int R>
+struct KsTile {
+    typedef ks_v16f Sums;
+    static __device__ __forceinline__ Sums multiply(float a, float b, Sums c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+};
+template <>
+struct KsTile<16> {
+    typedef ks_v4f Sums;
+    static __device__ __forceinline__ Sums multiply(float a, float b, Sums c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+};
 
 enum { KS_CONTIG = 0, KS_STRIDED = 1, KS_CONV = 2, KS_CONV1 = 3 };  // along K: contiguous, strided, gathered, 1x1 filter
 
@@ -45,13 +57,30 @@ struct KsParams {
     const float* bias;
     unsigned a_bytes, b_bytes;
     unsigned a_row, a_k, b_row, b_k;  // byte strides: of A's rows / B's columns, and along K
+    // tiles in strips of strip_w columns, row by row inside a strip; per_xcd: of them on each XCD (0: as the workgroups come)
+    int tiles, per_xcd, strip_w, strips;
+    FastDiv d_strip, d_w, d_last;
     int M, N, K, ldc;
+    int lw;  // log2 of the waves
     int act;
     // convolution
     int ic, ih, iw, ow, ohw, fh, fw, sh, sw, ph, pw, dh, dw;
     FastDiv d_ohw, d_ow, d_taps, d_fw;
-    XcdOrder xo;
 };
+
+// The arguments as the first thing, in one round trip: asked for where they are used, two to five round trips one after
+// the other stood in front of the first load.
+template <bool CONV>
+__device__ __forceinline__ void ks_begin(const KsParams& q) {
+#ifndef MG_HOST_AUDIT
+    asm volatile("" ::"s"(q.A), "s"(q.B), "s"(q.C), "s"(q.a_bytes), "s"(q.b_bytes), "s"(q.a_row), "s"(q.a_k), "s"(q.b_row), "s"(q.b_k), "s"(q.M),
+                 "s"(q.N), "s"(q.K), "s"(q.ldc), "s"(q.lw), "s"(q.tiles), "s"(q.per_xcd), "s"(q.strip_w), "s"(q.strips),
+                 "s"(q.d_strip.mul), "s"(q.d_w.mul), "s"(q.d_last.mul));
+    if (CONV)
+        asm volatile("" ::"s"(q.bias), "s"(q.act), "s"(q.ic), "s"(q.ih), "s"(q.iw), "s"(q.ow), "s"(q.ohw), "s"(q.fh), "s"(q.fw), "s"(q.sh), "s"(q.sw),
+                     "s"(q.ph), "s"(q.pw), "s"(q.dh), "s"(q.dw), "s"(q.d_ohw.mul), "s"(q.d_ow.mul), "s"(q.d_taps.mul), "s"(q.d_fw.mul));
+#endif
+}
 
 __device__ __forceinline__ float ks_act(int act, float x) {
     switch (act) {
@@ -65,44 +94,53 @@ __device__ __forceinline__ float ks_act(int act, float x) {
 static constexpr int KS_MAX_WAVES = 8;
 static constexpr int KS_MAX_CONV_K = 4096;  // table entries (8 bytes each)
 
-template <int AM, int BMODE, int MT, int NT, bool TAIL>
+template <int AM, int BMODE, int R, int MT, int NT, bool TAIL>
 __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams q) {
-    constexpr int RING = 4;
+    constexpr int RING = 4;  // (full >> (2 + lw) below)
     constexpr bool GATHER = BMODE == KS_CONV, CONV = GATHER || BMODE == KS_CONV1;
+    // lanes along an operand's rows, groups of lanes along K, values of K a step, sums of a tile per lane
+    constexpr int H = 64 / R, KS = 4 * H, LKS = R == 32 ? 3 : 4, SUMS = R * R / 64;
+    typedef typename KsTile<R>::Sums Sums;
     static_assert(!CONV || NT == 1, "one pixel per lane");
     extern __shared__ __attribute__((aligned(16))) float ks_lds[];
+    ks_begin<CONV>(q);
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), W = blockDim.x >> 6;
-    const int h = lane >> 5, c = lane & 31;
-    int tx, ty;
-    xcd_tile(q.xo, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, tx, ty);
-    const int m0 = ty * (32 * MT), n0 = tx * (32 * NT);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lw = q.lw, W = 1 << lw;
+    const int h = lane / R, c = lane & (R - 1);
+    const int place = q.per_xcd ? (int)(blockIdx.x & 7) * q.per_xcd + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+    if (place >= q.tiles)  // (the whole workgroup)
+        return;
+    const int strip = (int)fdiv(place, q.d_strip), in = place - strip * (int)q.d_strip.d;
+    const bool last = strip == q.strips - 1;
+    const int ty = last ? (int)fdiv(in, q.d_last) : (int)fdiv(in, q.d_w);
+    const int tx = strip * q.strip_w + in - ty * (int)(last ? q.d_last.d : q.d_w.d);
+    const int m0 = ty * (R * MT), n0 = tx * (R * NT);
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)q.A, 0, (int)q.a_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)q.B, 0, (int)q.b_bytes, 0x00020000);
 
     // Whole steps, dealt to the waves RING at a time where K is long - 4 steps are one 128-byte line of an
     // operand that is contiguous along K, fetched by one wave back to back instead of by four waves that
     // drift apart - and one at a time where that would leave waves without work.
-    const int full = q.K >> 3;
+    const int full = q.K >> LKS;
     const bool lines = full >= 4 * RING * W;
     const int s_wave = lines ? RING : 1, s_ring = lines ? 1 : W;  // step = j0 * W + wave * s_wave + r * s_ring
-    const int rounds = full / (RING * W), over = full - rounds * (RING * W);
+    const int rounds = full >> (2 + lw), over = full - (rounds << (2 + lw));
     const int nj = lines ? rounds * RING + min(max(over - RING * wave, 0), RING)
-                         : full > wave ? (full - wave + W - 1) / W : 0;
+                         : full > wave ? (full - wave + W - 1) >> lw : 0;
 
     // byte offset of (row, k = 4 h) of each operand tile
     unsigned aoff[MT], boff[NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
-        aoff[i] = (unsigned)min(m0 + i * 32 + c, q.M - 1) * q.a_row + (unsigned)(4 * h) * q.a_k;
+        aoff[i] = (unsigned)min(m0 + i * R + c, q.M - 1) * q.a_row + (unsigned)(4 * h) * q.a_k;
     int* const tab = (int*)ks_lds;
-    int* const pix = tab + (GATHER ? (q.K + 7) / 8 * 16 : 0);  // [offset, outside, image, place in it][32]
+    int* const pix = tab + (GATHER ? (q.K + KS - 1) / KS * (2 * KS) : 0);  // [offset, outside, image, place in it][32]
     if (CONV) {
         // The lane's pixel and, for a gather, the table: per k the byte offset and 31 - tap (0 - the bit
         // that is always set - beyond K), in groups of four: 4 offsets, 4 shifts. One wave works out the 32
         // pixels and the others the table: done by every wave, the index arithmetic was half of a small
         // layer's time.
-        if (wave == 0 && lane < 32) {
+        if (wave == 0 && lane < R) {
             const int p = min(n0 + lane, q.N - 1);
             const int img = (int)fdiv(p, q.d_ohw), rem = p - img * q.ohw;
             const int oh = (int)fdiv(rem, q.d_ow), ow = rem - oh * q.ow;
@@ -121,7 +159,7 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
             pix[96 + lane] = rem;
         } else if (GATHER && wave > 0) {
             const int taps = q.fh * q.fw;
-            for (int k = tid - 64; k < (q.K + 7) / 8 * 8; k += blockDim.x - 64) {
+            for (int k = tid - 64; k < (q.K + KS - 1) / KS * KS; k += 64 * W - 64) {
                 const int ic = (int)fdiv(k, q.d_taps), t = k - ic * taps;
                 const int y = (int)fdiv(t, q.d_fw), x = t - y * q.fw;
                 const int e = (k >> 2) * 8 + (k & 3);
@@ -132,7 +170,7 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
     } else {
 #pragma unroll
         for (int j = 0; j < NT; ++j)
-            boff[j] = (unsigned)min(n0 + j * 32 + c, q.N - 1) * q.b_row + (unsigned)(4 * h) * q.b_k;
+            boff[j] = (unsigned)min(n0 + j * R + c, q.N - 1) * q.b_row + (unsigned)(4 * h) * q.b_k;
     }
     unsigned outside = 0;
     int img = 0, rem = 0;
@@ -141,9 +179,9 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             if (AM == KS_CONTIG) {
-                v[i] = __builtin_bit_cast(ks_v4f, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(aoff[i] + (unsigned)s * 32u), 0, 0));
+                v[i] = __builtin_bit_cast(ks_v4f, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(aoff[i] + (unsigned)s * (4u * KS)), 0, 0));
             } else {
-                const unsigned o = aoff[i] + (unsigned)s * (8u * q.a_k);
+                const unsigned o = aoff[i] + (unsigned)s * ((unsigned)KS * q.a_k);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     v[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, (int)(o + (unsigned)e * q.a_k), 0, 0));
@@ -152,7 +190,7 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
     };
     auto load_b = [&](int s, ks_v4f (&v)[NT]) __attribute__((always_inline)) {
         if (GATHER) {
-            const v4i o = *(const v4i*)(tab + (2 * s + h) * 8), sh = *(const v4i*)(tab + (2 * s + h) * 8 + 4);
+            const v4i o = *(const v4i*)(tab + (H * s + h) * 8), sh = *(const v4i*)(tab + (H * s + h) * 8 + 4);
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -165,32 +203,42 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             if (BMODE == KS_CONTIG) {
-                v[j] = __builtin_bit_cast(ks_v4f, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(boff[j] + (unsigned)s * 32u), 0, 0));
+                v[j] = __builtin_bit_cast(ks_v4f, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(boff[j] + (unsigned)s * (4u * KS)), 0, 0));
             } else {
-                const unsigned o = boff[j] + (unsigned)s * (8u * q.b_k);
+                const unsigned o = boff[j] + (unsigned)s * ((unsigned)KS * q.b_k);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     v[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, (int)(o + (unsigned)e * q.b_k), 0, 0));
             }
         }
     };
-    ks_v16f acc[MT][NT], sum[MT][NT];
+    // (the one tile of 16 x 16 has a chain for each product of a step: four in flight, and shorter sums - relative error of
+    // 100 x 500 x 600 1.65e-7 with one, 0.97e-7 with four, 1.54e-7 with 32 x 32 tiles)
+    constexpr int CHAINS = R == 16 ? 4 : 1;
+    Sums acc[CHAINS][MT][NT], sum[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                acc[i][j][e] = sum[i][j][e] = 0.f;
+            for (int e = 0; e < SUMS; ++e) {
+                sum[i][j][e] = 0.f;
+#pragma unroll
+                for (int x = 0; x < CHAINS; ++x)
+                    acc[x][i][j][e] = 0.f;
+            }
     auto close = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    sum[i][j][e] += acc[i][j][e];
-                    acc[i][j][e] = 0.f;
+                for (int e = 0; e < SUMS; ++e) {
+                    sum[i][j][e] += CHAINS == 4 ? (acc[0][i][j][e] + acc[1 % CHAINS][i][j][e]) + (acc[2 % CHAINS][i][j][e] + acc[3 % CHAINS][i][j][e])
+                                                : acc[0][i][j][e];
+#pragma unroll
+                    for (int x = 0; x < CHAINS; ++x)
+                        acc[x][i][j][e] = 0.f;
                 }
     };
     auto multiply = [&](const ks_v4f (&a)[MT], const ks_v4f (&b)[NT]) __attribute__((always_inline)) {
@@ -200,12 +248,12 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
             for (int i = 0; i < MT; ++i)
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+                    acc[e % CHAINS][i][j] = KsTile<R>::multiply(a[i][e], b[j][e], acc[e % CHAINS][i][j]);
     };
 
     // the step behind the last whole one, element by element
     ks_v4f at[MT], bt[NT];
-    auto tail_k = [&](int e) { return min(full * 8 + 4 * h + e, q.K - 1) - 4 * h; };
+    auto tail_k = [&](int e) { return min(full * KS + 4 * h + e, q.K - 1) - 4 * h; };
     if (TAIL)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -220,6 +268,15 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
             constexpr int r = decltype(rc)::value;
             load_a(step(0, r), av[r]);
         });
+    // (the biases of the rows this wave finishes: asked for here, not behind the sums)
+    float bias[4] = {0.f, 0.f, 0.f, 0.f};
+    if (CONV && q.bias) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = min(wave + i * W, SUMS - 1);
+            bias[i] = q.bias[min(m0 + (R == 32 ? 8 * (r >> 2) : 0) + 4 * h + (r & 3), q.M - 1)];
+        }
+    }
     if (CONV) {
         __syncthreads();
         boff[0] = (unsigned)pix[c] + (BMODE == KS_CONV1 ? (unsigned)(4 * h) * q.b_k : 0u);
@@ -250,10 +307,10 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
                 load_a((j0 + RING) * W + s0 + r * s_ring, av[r]);
                 load_b((j0 + RING) * W + s0 + r * s_ring, bv[r]);
             });
-            if (j0 & RING)
+            if (KS == 16 || (j0 & RING))  // (every 64 values of K)
                 close();
         }
-        for (; j0 < nj; j0 += RING)
+        for (; j0 < nj; j0 += RING) {
             static_for<RING>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
                 if (j0 + r < nj) {
@@ -264,11 +321,14 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
                     }
                 }
             });
+            if (KS == 16)
+                close();
+        }
     }
-    if (TAIL && wave == (lines ? W - 1 : full % W)) {  // (the wave whose turn it is)
+    if (TAIL && wave == (lines ? W - 1 : full & (W - 1))) {  // (the wave whose turn it is)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const bool in = full * 8 + 4 * h + e < q.K;
+            const bool in = full * KS + 4 * h + e < q.K;
 #pragma unroll
             for (int i = 0; i < MT; ++i)
                 at[i][e] = in ? at[i][e] : 0.f;
@@ -279,30 +339,37 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         multiply(at, bt);
     }
 
+    close();
+
     // the waves' sums meet in LDS: [wave][tile][register][lane]
     if (CONV)
         __syncthreads();  // (the table's room is used again)
-    constexpr int TILE = MT * NT * 1024;
+    constexpr int TILE = MT * NT * R * R;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                ks_lds[wave * TILE + ((i * NT + j) * 16 + e) * 64 + lane] = acc[i][j][e] + sum[i][j][e];
+            for (int e = 0; e < SUMS; ++e)
+                ks_lds[wave * TILE + ((i * NT + j) * SUMS + e) * 64 + lane] = sum[i][j][e];
     __syncthreads();
-    // register e of a tile: row 8 * (e / 4) + 4 * h + e % 4, column c. Wave w finishes registers w, w + W, ...
-    for (int r = wave; r < MT * NT * 16; r += W) {
-        const int t = r >> 4, e = r & 15, i = t / NT, j = t - i * NT;
+    // register e of a tile: row 8 * (e / 4) + 4 * h + e % 4 (16 x 16: 4 * h + e), column c. Wave w finishes registers w, w + W, ...
+    constexpr int TURNS = (MT * NT * SUMS + 3) / 4;  // (of four waves; eight are done after half of them)
+#pragma unroll
+    for (int i_r = 0; i_r < TURNS; ++i_r) {
+        const int r = wave + i_r * W;
+        if (r >= MT * NT * SUMS)
+            break;
+        const int t = r / SUMS, e = r & (SUMS - 1), i = t / NT, j = t - i * NT;
         float v = 0.f;
 #pragma unroll 4
         for (int w = 0; w < W; ++w)
             v += ks_lds[w * TILE + r * 64 + lane];
-        const int m = m0 + i * 32 + 8 * (e >> 2) + 4 * h + (e & 3), n = n0 + j * 32 + c;
+        const int m = m0 + i * R + (R == 32 ? 8 * (e >> 2) : 0) + 4 * h + (e & 3), n = n0 + j * R + c;
         if (m >= q.M || n >= q.N)
             continue;
         if (CONV) {
-            q.C[((size_t)img * q.M + m) * q.ohw + rem] = ks_act(q.act, v + (q.bias ? q.bias[m] : 0.f));
+            q.C[((size_t)img * q.M + m) * q.ohw + rem] = ks_act(q.act, v + bias[i_r & 3]);
         } else {
             q.C[(size_t)m * q.ldc + n] = v;
         }
@@ -311,8 +378,8 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
 
 // ---- choice of tile and waves -------------------------------------------------------------------------
 struct KsPlan {
-    int mt, nt, waves;
-    double cost;  // estimated cycles of the busiest CU
+    int r, mt, nt, waves;  // tiles of r mt x r nt
+    double cost;           // estimated cycles of the busiest CU
 };
 
 // Cycles of the busiest CU: its tiles' MFMAs (K / 2 of 64 cycles per 32 x 32 outputs, over four SIMDs) plus
@@ -321,7 +388,7 @@ struct KsPlan {
 // it at once. (Fitted: 2048^3 nt measured 248 / 203 / 159 us with tiles of 32x32 / 32x64 / 64x64, this says 238 /
 // 208 / 178.)
 static KsPlan ks_plan(long M, long N, long K, bool a_contig, bool b_contig, bool conv) {
-    KsPlan best = {0, 0, 0, 1e30};
+    KsPlan best = {0, 0, 0, 0, 1e30};
     static const int kResident[] = {0, 5, 3, 0, 2};
     for (int mt = 1; mt <= (conv ? 1 : 2); ++mt)
         for (int nt = 1; nt <= (conv ? 1 : 2); ++nt) {
@@ -332,11 +399,21 @@ static KsPlan ks_plan(long M, long N, long K, bool a_contig, bool b_contig, bool
                                 (mt * nt == 4 ? 5000.0 : 3000.0) * (double)((per_cu + kResident[mt * nt] - 1) / kResident[mt * nt]);
             if (cost < best.cost * 0.98) {
                 // eight waves where a CU has one tile of a long K, or where there are few tiles (64 x 4096 x 4096:
-                // 29.5 us with 4, 23.5 with 8, 25.2 with 16; 197 x 771 x 1003: 8.2, 9.8, 9.7)
-                const int w = per_cu <= 1 && (K >= 1024 || tiles <= num_cus() / 2) ? 8 : 4;
-                best = {mt, nt, w, cost};
+                // 29.5 us with 4, 23.5 with 8, 25.2 with 16; 197 x 771 x 1003: 7.5, 8.6, 9.7; 64 -> 64 28 x 28 N=4 8.0, 7.0;
+                // 400 x 640 x 333 6.0, 6.2)
+                const int w = per_cu <= 1 && (K >= 1024 || tiles <= num_cus() / 2 || (conv ? K >= 512 : K >= 700 && tiles <= num_cus() * 5L / 8)) ? 8 : 4;
+                best = {32, mt, nt, w, cost};
             }
         }
+    // 16 x 16 tiles (the same rate on the matrix cores, four times the workgroups) where 32 x 32 ones leave CUs without any: a
+    // tile's own chain is a quarter (64 x 1024 x 1000 7.5 us with 32 x 32, 4.8 with 16 x 16; 128 x 2048 x 512 nt 17.0 / 9.1; 33 x 500 x
+    // 200 5.6 / 3.6; convolution 64 -> 64 28 x 28 6.7 / 4.3). Two a CU are still one round (32 -> 32 56 x 56 4.9 / 4.2, 300 x 2000 x
+    // 400 13.4 / 9.6), unless one row of 32 x 32 tiles is all there is and the other operand, beyond the L2s, would be read
+    // twice (20 x 3000 x 4000 16.0 / 17.0); with more, the operands' way in costs more than the idle CUs (500^3 6.0 / 8.1, 8 -> 16 112 x 112 4.7 / 5.4).
+    const long small = ((M + 15) / 16) * ((N + 15) / 16);
+    const bool one_row = ((M > 16 && M <= 32) || (N > 16 && N <= 32)) && K * (M > N ? M : N) > (1L << 22);
+    if (small <= num_cus() || (small <= 2L * num_cus() && !one_row))
+        best = {16, 1, 1, small <= num_cus() && K >= 256 ? 8 : 4, (double)K * 4.75 * (small <= num_cus() ? 1.0 : 2.0) + 3000.0};
     return best;
 }
 
@@ -354,20 +431,34 @@ static bool ks_wins(long M, long N, long K, bool conv, const KsPlan& p) {
 
 template <int AM, int BMODE>
 static TinyNNStatus ks_launch(KsParams& q, const KsPlan& p, const char* what) {
-    const bool tail = (q.K & 7) != 0;
+    const bool tail = (q.K & (p.r == 32 ? 7 : 15)) != 0;
     constexpr bool CONV = BMODE == KS_CONV || BMODE == KS_CONV1;
-#define MG_KS_T(MT_, NT_) (tail ? gemm_f32_ks_kernel<AM, BMODE, MT_, NT_, true> : gemm_f32_ks_kernel<AM, BMODE, MT_, NT_, false>)
+#define MG_KS_T(R_, MT_, NT_) (tail ? gemm_f32_ks_kernel<AM, BMODE, R_, MT_, NT_, true> : gemm_f32_ks_kernel<AM, BMODE, R_, MT_, NT_, false>)
     void (*kern)(KsParams);
-    if constexpr (CONV)  // (wider tiles never measured better for a convolution)
-        kern = MG_KS_T(1, 1);
+    if (p.r == 16)
+        kern = MG_KS_T(16, 1, 1);
+    else if constexpr (CONV)  // (wider tiles never measured better for a convolution)
+        kern = MG_KS_T(32, 1, 1);
     else
-        kern = p.mt == 1 ? (p.nt == 1 ? MG_KS_T(1, 1) : MG_KS_T(1, 2)) : (p.nt == 1 ? MG_KS_T(2, 1) : MG_KS_T(2, 2));
+        kern = p.mt == 1 ? (p.nt == 1 ? MG_KS_T(32, 1, 1) : MG_KS_T(32, 1, 2)) : (p.nt == 1 ? MG_KS_T(32, 2, 1) : MG_KS_T(32, 2, 2));
 #undef MG_KS_T
-    const dim3 grid((unsigned)((q.N + 32 * p.nt - 1) / (32 * p.nt)), (unsigned)((q.M + 32 * p.mt - 1) / (32 * p.mt)));
-    q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y);
-    note_kernel(what, p.mt * 32, p.nt * 32, p.waves, q.xo.w);
-    size_t lds = (size_t)p.waves * p.mt * p.nt * 4096;
-    const size_t table = (BMODE == KS_CONV ? (size_t)(q.K + 7) / 8 * 64 : 0) + (CONV ? 512 : 0);
+    const int tm = p.r * p.mt, tn = p.r * p.nt;
+    const int gx = (q.N + tn - 1) / tn, gy = (q.M + tm - 1) / tm;
+    q.tiles = gx * gy;
+    // The order of common.h's XcdOrder. For 16 x 16 tiles also where their number is no multiple of the eight XCDs, with up to
+    // seven workgroups without a tile: a tile's rows are half lines, and two XCDs would fetch each (64 x 4096 x 1000 17.2 us
+    // without, 11.8 with; of whole lines the plain order is the faster one then, 200 x 1000 x 700 7.5 / 7.9).
+    const int w = options().no_xcdorder || ((p.r == 32 || CONV) && (q.tiles & 7) != 0) ? 0 : xcd_strip(gx, q.tiles);
+    q.per_xcd = w ? (q.tiles + 7) / 8 : 0;
+    q.strip_w = w ? w : gx, q.strips = (gx + q.strip_w - 1) / q.strip_w;
+    q.d_strip = make_fastdiv((uint32_t)(q.strip_w * gy));
+    q.d_w = make_fastdiv((uint32_t)q.strip_w);
+    q.d_last = make_fastdiv((uint32_t)(gx - (q.strips - 1) * q.strip_w));
+    const dim3 grid((unsigned)(w ? 8 * q.per_xcd : q.tiles));
+    q.lw = p.waves == 8 ? 3 : 2;
+    note_kernel(what, tm, tn, p.waves, w);
+    size_t lds = (size_t)p.waves * tm * tn * 4;
+    const size_t table = (BMODE == KS_CONV ? (size_t)(q.K + 15) / 16 * 128 : 0) + (CONV ? 512 : 0);
     if (lds < table)
         lds = table;
     if (lds > 48 * 1024) {
@@ -393,7 +484,8 @@ double gemm_f32_ks_cycles(const GevmArgs& v) {
 // and too few CUs share the chain. The tiled kernel's slices of K over the whole chip are faster there (16 x 4096 x
 // 1024 nt 25.2 us here, 20.1 there; 64 x 4096 x 2048 31.1 / 25.7; at K = 2500, 16 x 512, 14.1 / 18.9).
 static bool long_rows_of_few(const GevmArgs& v) {
-    return v.b_cs != 1 && v.K > 3400 && (long)((v.M + 31) / 32) * ((v.N + 31) / 32) <= num_cus() / 2;
+    return v.b_cs != 1 && v.K > 3400 && (long)((v.M + 31) / 32) * ((v.N + 31) / 32) <= num_cus() / 2 &&
+           (long)((v.M + 15) / 16) * ((v.N + 15) / 16) > num_cus();
 }
 
 bool gemm_f32_ks_supported(const GevmArgs& v) {

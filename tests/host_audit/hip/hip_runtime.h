@@ -111,6 +111,7 @@ inline unsigned __umulhi(unsigned a, unsigned b) { return (unsigned)(((unsigned 
 #define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) (c)
+#define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) (c)
 #define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) (c)
 #define __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, x, y, z) (c)
 #define __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, x, y, z) (c)

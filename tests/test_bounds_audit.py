@@ -159,6 +159,10 @@ def audit_lines():
         tail = "%d %d %d %d" % (r.integers(0, 2), r.integers(0, 2), r.choice([0, 1, 4, 7]), r.choice([0, 1, 4, 7]))
         lines.append("ks %d %d %d %s" % (m, k, n, tail))
         lines.append("split %d %d %d %s" % (m, 32 + int(r.choice([0, 1, 15, 16, 17, 100, 143, 500])), n, tail))
+    # ... 16 x 16 tiles up to two a CU, in strips with workgroups left over; then 32 x 32
+    for m, k, n in ((15, 17, 16), (17, 15, 33), (100, 33, 300), (357, 16, 301), (40, 300, 1700), (513, 9, 530), (600, 31, 700)):
+        for t in range(4):
+            lines.append("ks %d %d %d %d %d 0 0" % (m, k, n, t & 1, t >> 1))
     # FullyConnected of any K on tiles: rows at any byte, the tensor's last 16 bytes anywhere in a piece
     for m, k, oc in ((65, 5, 9), (64, 1, 3), (16, 1, 1), (65, 129, 67), (70, 295, 70), (225, 515, 361), (66, 128, 64), (130, 260, 257),
                      (100, 1123, 65), (65, 127, 129), (300, 33, 31)):

@@ -1,13 +1,14 @@
 """Kernels whose waves walk K in steps with a ring of operands in flight: shares below, at and beyond the ring and its
 multiples, where the last steps are taken one by one."""
+import numpy as np
 import pytest
 
-from cases import ConvCase
+from cases import ConvCase, MatMulCase
 from golden_cases import unsat
 from megcc_amd import abi as A
 from megcc_amd import runtime
 from oracle import port
-from test_gpu_parity import compare, run_gpu
+from test_gpu_parity import _product, compare, run_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -23,4 +24,34 @@ def test_shares_of_k_in_dense_layers_without_staging(ic, k, stride, ties, bias):
     arrays = case.gen(seed=41)
     got = run_gpu(case, arrays)
     assert runtime.last_kernel().startswith("conv_mfma_i8_gather"), runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
+# rows, columns and K at the edges of the 16 x 16 tiles and their steps of 16, four and eight waves; tiles that are no multiple
+# of eight, in strips; one and two tiles a CU, and the first size beyond
+@pytest.mark.parametrize("m,k,n", [(5, 1, 5), (16, 15, 16), (17, 16, 15), (15, 17, 33), (33, 63, 31), (31, 64, 49), (16, 65, 32), (48, 255, 16),
+                                   (33, 256, 17), (64, 257, 100), (100, 1031, 130), (357, 40, 301), (200, 300, 700), (40, 1300, 1700),
+                                   (512, 70, 256), (512, 270, 257), (23, 2000, 3100)])
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_f32_products_of_few_tiles(m, k, n, ta, tb):
+    case = MatMulCase(m, k, n, trans_a=ta, trans_b=tb)
+    arrays = case.gen(seed=43)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().startswith("gemm_f32_ks"), runtime.last_kernel()
+    # each of the k products and sums is rounded once, in whatever order
+    bound = _product(case, {x: np.abs(v) for x, v in arrays.items()}) * (k * 2.0 ** -24)
+    assert np.all(np.abs(got - _product(case, arrays)) <= bound)
+    assert np.array_equal(run_gpu(case, {x: np.round(8 * v) for x, v in arrays.items()}), _product(case, {x: np.round(8 * v) for x, v in arrays.items()}))
+
+
+@pytest.mark.parametrize("n,ic,ih,iw,oc,k,stride", [(1, 1, 4, 4, 16, 3, 1), (1, 5, 9, 9, 17, 3, 1), (2, 28, 13, 11, 33, 3, 2), (1, 29, 14, 15, 15, 3, 1),
+                                                    (1, 64, 28, 28, 64, 3, 1), (1, 32, 56, 56, 32, 3, 1), (3, 100, 14, 13, 30, 1, 1), (1, 21, 17, 16, 40, 5, 2)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_f32_convolutions_of_few_tiles(n, ic, ih, iw, oc, k, stride, bias):
+    port.set_threads(8)
+    case = ConvCase(A.FMT_NCHW, A.DENSE, n, ic, ih, iw, oc, k, stride, k // 2, A.RELU, dtype="f32", bias=bias)
+    arrays = case.gen(seed=44)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().startswith("conv_f32_gemm_ks:16,16"), runtime.last_kernel()
     compare(got, case.run_port(arrays), repr(case))
