@@ -25,9 +25,9 @@
 // Bound: HBM on the large maps, the vector ALU's requantisation and the filter's way from L2 on the small
 // ones; with one tile a workgroup the way from the launch to the first load (dp_begin).
 // Measured (N=64, us, one kernel / two): 32x112x112->64 20.2 / 32.4, 64 s2 -> 128 17.2 / 25.5, 128x56x56->128 17.3 / 28.8,
-// 256x28x28->256 13.3 / 22.1, 512x14x14->512 10.5 / 21.7, 1024x7x7->1024 14.3 / 20.2; N=1: 4.3 / 6.8, 4.8 / 6.3, 4.2 / 6.9,
-// 5.6 / 7.3, 9.0 / 8.0, 13.4 / 9.9; N=256: 88 / 117 and, 512 channels, 32.7 / 49.5. (With the arguments read where they are
-// used, a filter ring of 8 chunks and every store's address of its own, N=1: 5.1, 5.6, 5.2, 6.4, 9.7, 17.0.)
+// 256x28x28->256 13.3 / 22.1, 512x14x14->512 10.5 / 21.7, 1024x7x7->1024 12.4 / 20.2; N=1: 4.3 / 6.8, 4.8 / 6.3, 4.2 / 6.9,
+// 5.0 / 7.3, 7.0 / 8.0, 10.5 / 9.9; N=256: 88 / 117 and, 512 channels, 32.7 / 49.5. (With the arguments read where they are
+// used, slices as wide as they come, a filter ring of 8 chunks and every store's address of its own, N=1: 5.1, 5.6, 5.2, 6.4, 9.7, 17.0.)
 #include <map>
 #include <mutex>
 
@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
     constexpr bool KEEP_D = JW == 1 && S == 1, KEEP_P = KC * MT <= 8;
     // chunks of the pointwise filter in flight (not KEEP_P). More of them only stand in front of the channel-wise
     // operands: 8 for 4 chunks, 512 channels at N=256 33.1 for 32.2 us, stride 2 21.2 for 20.4
-    constexpr int RING = KC >= 16 ? 4 : 8;
+    constexpr int RING = MT == 1 || KC < 16 ? 8 : 4;
     static_assert(JW >= 1 && WP >= 1 && WO >= 1 && WP * WO == 8, "8 waves");
     dp_begin(q);
     extern __shared__ __attribute__((aligned(16))) int8_t dp_lds_mem[];
@@ -491,7 +491,19 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
 struct DpShape {
     int kc, sub, mt, nt;
 };
-static bool dp_shape(int c, int oc, DpShape* s) {
+static bool dp_shape(int c, int oc, long groups, DpShape* s) {
+    // Slices of 128 or 256 channels while every slice of a tile has a CU to itself: the channel-wise layer is worked out
+    // once a slice, but a workgroup's filter, products and requantisation are a quarter or half of 512 channels'. With two
+    // slices to a CU that is no gain (us, with slices of 512 / 256 / 128 channels: 512 14 x 14 N=1 9.1 / - / 7.0, N=32
+    // 9.6 / 8.3 / 11.7, N=64 10.5 / - / 19.9; 1024 7 x 7 N=1 13.3 / - / 10.5, N=64 14.3 / 12.4 / 18.5; 256 -> 512 stride 2 N=1
+    // 7.1 / - / 5.4, N=64 8.4 / - / 12.5).
+    const long tiles = (groups + 15) / 16;
+    if (c == 256 || c == 512 || c == 1024)
+        for (int nt = 1; nt <= 2; ++nt)
+            if (tiles * ((oc + 128 * nt - 1) / (128 * nt)) <= num_cus()) {
+                *s = {c / 32, 1, 1, nt};
+                return true;
+            }
     switch (c) {
         case 32: *s = {1, 4, 2, 1}; break;                        // 64 channels a slice
         case 64: *s = {2, 2, 2, 1}; break;                        // 128
@@ -509,7 +521,7 @@ bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* sr
     return dw.fmt == MEGCC_FMT_NCHW44 && dw.groups == dw.ic && dw.ic == dw.oc && dw.fh == 3 && dw.fw == 3 && dw.ph == 1 &&
            dw.pw == 1 && dw.dh == 1 && dw.dw == 1 && dw.sh == dw.sw && (dw.sh == 1 || dw.sh == 2) &&
            pw.fmt == MEGCC_FMT_NCHW44 && pw.groups == 1 && pw.fh == 1 && pw.fw == 1 && pw.sh == 1 && pw.sw == 1 && pw.ph == 0 &&
-           pw.pw == 0 && pw.ic == dw.oc && (pw.oc & 31) == 0 && dp_shape(dw.ic, pw.oc, &s) &&
+           pw.pw == 0 && pw.ic == dw.oc && (pw.oc & 31) == 0 && dp_shape(dw.ic, pw.oc, 0, &s) &&
            dw.act == MEGCC_NONLINE_RELU &&
            (pw.act == MEGCC_NONLINE_IDENTITY || pw.act == MEGCC_NONLINE_RELU) &&
            requant_table_ok(dw.s_src, dw.s_flt, dw.s_dst) && requant_table_ok(pw.s_src, pw.s_flt, pw.s_dst) &&
@@ -551,7 +563,9 @@ TinyNNStatus conv_dw_pw_launch(
         const void* pbias, void* dst) {
     DwPwParams q = {};
     DpShape s;
-    MG_REQUIRE(dp_shape(dw.ic, pw.oc, &s), TinyNN_ERROR_NO_IMPLEMENT, "conv_dw_pw: %d channels", dw.ic);
+    q.xg = (dw.ow + 3) / 4;
+    q.groups = dw.n * dw.oh * q.xg;
+    MG_REQUIRE(dp_shape(dw.ic, pw.oc, q.groups, &s), TinyNN_ERROR_NO_IMPLEMENT, "conv_dw_pw: %d channels", dw.ic);
     q.src = (const uint32_t*)src;
     q.dflt = (const uint32_t*)dflt;
     q.dbias = (const int32_t*)dbias;
@@ -564,8 +578,6 @@ TinyNNStatus conv_dw_pw_launch(
     q.OC = pw.oc;
     q.OCP = (pw.oc + OC_PAD - 1) / OC_PAD * OC_PAD;
     q.plane = dw.ih * dw.iw * 4;
-    q.xg = (dw.ow + 3) / 4;
-    q.groups = dw.n * dw.oh * q.xg;
     const int tiles = (q.groups + 16 * s.sub - 1) / (16 * s.sub);
     const int wo = 8 / (64 * s.sub / (32 * s.nt)), ocs = wo * 32 * s.mt;
     q.slices = (pw.oc + ocs - 1) / ocs;
@@ -592,9 +604,14 @@ TinyNNStatus conv_dw_pw_launch(
     MG_DP(2, 2, 2, 1)
     MG_DP(4, 1, 1, 1)
     MG_DP(4, 1, 1, 2)
+    MG_DP(8, 1, 1, 1)
     MG_DP(8, 1, 1, 2)
     MG_DP(8, 1, 2, 2)
+    MG_DP(16, 1, 1, 1)
+    MG_DP(16, 1, 1, 2)
     MG_DP(16, 1, 2, 2)
+    MG_DP(32, 1, 1, 1)
+    MG_DP(32, 1, 1, 2)
     MG_DP(32, 1, 2, 2)
 #undef MG_DP
     MG_REQUIRE(kern, TinyNN_ERROR_NO_IMPLEMENT, "conv_dw_pw: no instance");

@@ -8,6 +8,8 @@ from golden_cases import unsat
 from megcc_amd import abi as A
 from megcc_amd import runtime
 from oracle import port
+
+import test_dw_pw
 from test_gpu_parity import _product, compare, run_gpu
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +57,16 @@ def test_f32_convolutions_of_few_tiles(n, ic, ih, iw, oc, k, stride, bias):
     got = run_gpu(case, arrays)
     assert runtime.last_kernel().startswith("conv_f32_gemm_ks:16,16"), runtime.last_kernel()
     compare(got, case.run_port(arrays), repr(case))
+
+
+GENERIC, TIES = test_dw_pw.GENERIC, test_dw_pw.TIES
+
+
+# (n, c, oc, h, w, stride, activation, scales) with slices of 128, 256 and 512 channels of the result, the last one in part
+@pytest.mark.parametrize("cfg", [
+    (1, 256, 160, 9, 10, 1, A.RELU, TIES), (2, 512, 288, 5, 6, 2, A.RELU, GENERIC), (1, 1024, 96, 6, 7, 1, A.IDENTITY, GENERIC), (1, 1024, 416, 7, 8, 2, A.RELU, TIES),
+    (20, 512, 512, 14, 13, 1, A.RELU, GENERIC), (66, 512, 544, 14, 15, 2, A.RELU, TIES), (40, 1024, 1056, 7, 7, 1, A.RELU, GENERIC), (17, 256, 288, 28, 27, 1, A.RELU, GENERIC),
+    (70, 1024, 32, 20, 12, 1, A.RELU, TIES), (280, 1024, 32, 19, 13, 2, A.RELU, GENERIC), (70, 512, 32, 20, 10, 1, A.RELU, GENERIC), (280, 512, 64, 20, 11, 2, A.IDENTITY, TIES),
+    (280, 256, 288, 20, 11, 2, A.RELU, GENERIC), (40, 256, 288, 28, 28, 1, A.RELU, TIES)], ids=lambda c: "n%d_c%d_oc%d_%dx%d_s%d_a%d" % c[:7])
+def test_slices_of_channel_wise_pointwise_pairs(cfg):
+    test_dw_pw.test_pair_in_one_kernel(cfg)
