@@ -24,10 +24,12 @@
 // Both requantisations are the exact ones of epilogue.h, so the result is bit for bit the two kernels'.
 // Bound: HBM on the large maps, the vector ALU's requantisation and the filter's way from L2 on the small
 // ones; with one tile a workgroup the way from the launch to the first load (dp_begin).
-// Measured (N=64, us, one kernel / two): 32x112x112->64 20.2 / 32.4, 64 s2 -> 128 17.2 / 25.5, 128x56x56->128 17.3 / 28.8,
-// 256x28x28->256 13.3 / 22.1, 512x14x14->512 10.5 / 21.7, 1024x7x7->1024 12.4 / 20.2; N=1: 4.3 / 6.8, 4.8 / 6.3, 4.2 / 6.9,
-// 5.0 / 7.3, 7.0 / 8.0, 10.5 / 9.9; N=256: 88 / 117 and, 512 channels, 32.7 / 49.5. (With the arguments read where they are
-// used, slices as wide as they come, a filter ring of 8 chunks and every store's address of its own, N=1: 5.1, 5.6, 5.2, 6.4, 9.7, 17.0.)
+// Measured (N=64, us, one kernel / two): 32x112x112->64 20.2 / 32.4, 64 s2 -> 128 17.0 / 25.5, 128x56x56->128 17.4 / 28.5,
+// 256x28x28->256 13.3 / 22.1, 512x14x14->512 9.9 / 21.7, 1024x7x7->1024 11.3 / 20.2; N=1: 4.4 / 6.9, 4.8 / 6.6, 4.3 / 7.0,
+// 5.0 / 7.2, 6.7 / 7.9, 9.8 / 9.9; N=256: 88 / 117 and, 512 channels, 31.9 / 49.5. Before the arguments came in one round trip,
+// slices followed the number of tiles and addresses were constants from one place, N=1: 5.1, 5.6, 5.2, 6.4, 9.7, 17.0; N=64, 512 and
+// 1024 channels: 10.9, 18.3. (Two jobs' operands in flight, 16 waves of 128 registers, the whole filter in registers, jobs
+// and products of two wave halves in opposite order: each slower, 512 channels N=1 by 0.4 - 1.6 us.)
 #include <map>
 #include <mutex>
 
@@ -69,8 +71,19 @@ __device__ __forceinline__ void dp_begin(const DwPwParams& q) {
 #ifndef MG_HOST_AUDIT
     asm volatile("" ::"s"(q.src), "s"(q.dflt), "s"(q.dbias), "s"(q.wp), "s"(q.pbias), "s"(q.dst), "s"(q.src_bytes), "s"(q.dst_bytes), "s"(q.ih),
                  "s"(q.iw), "s"(q.oh), "s"(q.ow), "s"(q.OC), "s"(q.OCP), "s"(q.plane), "s"(q.xg), "s"(q.groups), "s"(q.slices), "s"(q.nb),
-                 "s"(q.run_q), "s"(q.run_r), "s"(q.d_xg.mul), "s"(q.d_oh.mul), "s"(q.d_slices.mul), "s"(q.dq.mode), "s"(q.pq.mode));
+                 "s"(q.run_q), "s"(q.run_r), "s"(q.d_xg.mul), "s"(q.d_oh.mul), "s"(q.d_slices.mul));
+    asm volatile("" ::"s"(q.d_xg.shift), "s"(q.d_xg.d), "s"(q.d_oh.shift), "s"(q.d_oh.d), "s"(q.d_slices.shift), "s"(q.d_slices.d), "s"(q.dq.mode),
+                 "s"(q.dq.c), "s"(q.dq.d), "s"(q.pq.mode), "s"(q.pq.c), "s"(q.pq.d));
 #endif
+}
+
+// a scalar whose origin the compiler does not know: sums made from it stay where they are written, instead of one register (and,
+// beyond what there are, one spill) for every chunk and plane ahead of the loop
+__device__ __forceinline__ int dp_opaque(int v) {
+#ifndef MG_HOST_AUDIT
+    asm volatile("" : "+s"(v));
+#endif
+    return v;
 }
 
 // 16 accumulators of one column -> 4 dwords (each 4 consecutive registers)
@@ -178,21 +191,24 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
     };
     v4i B[4][S];
     unsigned E[4];
-    auto request = [&](const Rows& r, int quad) __attribute__((always_inline)) {
+    // job i of this wave: channels 16 quad .. + 15, pixels 64 u .. + 63 of the tile
+    // (several jobs a tile: tiles of 64 pixels)
+    static_assert(JW == 1 || SUB == 1, "");
+    const int quad0 = SUB == 1 ? wave : wave % NQ, sub0 = SUB == 1 ? 0 : wave / NQ;
+    const int plane0 = quad0 * 4 * q.plane;
+    auto request = [&](const Rows& r, int i) __attribute__((always_inline)) {
+        int pl = dp_opaque(plane0 + i * (32 * q.plane));
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            const int pl = (quad * 4 + p) * q.plane;
             B[p][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)r.off, pl, 0));
             if (S == 2)
                 B[p][S - 1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)r.offb, pl, 0));
             E[p] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)r.eoff, pl, 0);
+            pl += q.plane;
         }
     };
-    // job i of this wave: channels 16 quad .. + 15, pixels 64 u .. + 63 of the tile
-    auto quad_of = [&](int i) { return (wave + 8 * i) % NQ; };
-    auto sub_of = [&](int i) { return (wave + 8 * i) / NQ; };
-    Rows rows = rows_of(t_begin, sub_of(0)), cur;
-    request(rows, quad_of(0));
+    Rows rows = rows_of(t_begin, sub0), cur;
+    request(rows, 0);
 
     // ---- set-up: filters, biases, tables -----------------------------------------------------------
     // (all loads of a thread before its first store: a round trip for the whole set-up, not one per turn)
@@ -208,33 +224,14 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
         for (int j = 0; j < 3; ++j)
             wv[k][j] = w[j];
     }
+    // (no bias: some other bytes, not used)
+    const int32_t *dbp = q.dbias ? q.dbias : (const int32_t*)q.dflt, *pbp = q.pbias ? q.pbias : (const int32_t*)q.wp;
 #pragma unroll
     for (int k = 0; k < BI; ++k)
-        dbv[k] = q.dbias ? q.dbias[min(tid + k * DP_THREADS, C - 1)] : 0;
+        dbv[k] = dbp[min(tid + k * DP_THREADS, C - 1)];
 #pragma unroll
     for (int k = 0; k < PI; ++k)
-        pbv[k] = q.pbias ? q.pbias[min(slice * ocs + tid + k * DP_THREADS, q.OC - 1)] : 0;
-#pragma unroll
-    for (int k = 0; k < WI; ++k) {
-        const int i = tid + k * DP_THREADS, dy = i & 3, sh = 8 * ((i >> 2) & 3);
-        const uint32_t v = ((wv[k][0] >> sh) & 0xff) | (((wv[k][1] >> sh) & 0xff) << 8) | (((wv[k][2] >> sh) & 0xff) << 16);
-        if (i < C * 4)
-            wl[i] = dy < 3 ? (int)v : 0;  // (a fourth row of zeros)
-    }
-#pragma unroll
-    for (int k = 0; k < BI; ++k)
-        if (tid + k * DP_THREADS < C)
-            db[tid + k * DP_THREADS] = dbv[k];
-#pragma unroll
-    for (int k = 0; k < PI; ++k)
-        if (tid + k * DP_THREADS < ocs)
-            pb[tid + k * DP_THREADS] = pbv[k];
-    if (tid < REQUANT_TABLE_ENTRIES) {
-        if (q.dq.mode == 0)
-            dtbl[tid] = q.dtable.t[tid];
-    } else if (q.pq.mode == 0) {
-        ptbl[tid - REQUANT_TABLE_ENTRIES] = q.ptable.t[tid - REQUANT_TABLE_ENTRIES];
-    }
+        pbv[k] = pbp[min(slice * ocs + tid + k * DP_THREADS, q.OC - 1)];
     // byte selectors of the banded matrices: row = (pixel colq >> 2, channel colq & 3) of the group, input row kg4;
     // the group's input pixel k meets it through filter column k + 1 - S px
     const int px = colq >> 2, sh = 8 * (colq & 3);
@@ -255,22 +252,52 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
         prow[mi] = oc * KROW + (((kg ^ (oc >> 3)) & 1) << 4);
     }
     v4i P[KEEP_P ? KC : RING][MT];
-    auto filter = [&](v4i (&P)[MT], int c) __attribute__((always_inline)) {
+    int next_chunk = 0;  // byte offset of the chunk to ask for next
+    auto filter = [&](v4i (&P)[MT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int mi = 0; mi < MT; ++mi)
-            P[mi] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, prow[mi], c * cstep, 0));
+            P[mi] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, prow[mi], next_chunk, 0));
+        next_chunk = dp_opaque(next_chunk + cstep);
     };
+    // (what follows waits for the loads; nothing of the above may move behind it)
+#ifndef MG_HOST_AUDIT
+#pragma unroll
+    for (int k = 0; k < 4 * S; ++k)
+        asm volatile("" : "+v"(sel[k]));
+    asm volatile("" : "+v"(sell), "+v"(selr), "+v"(prow[0]));
+#endif
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < WI; ++k) {
+        const int i = tid + k * DP_THREADS, dy = i & 3, sh = 8 * ((i >> 2) & 3);
+        const uint32_t v = ((wv[k][0] >> sh) & 0xff) | (((wv[k][1] >> sh) & 0xff) << 8) | (((wv[k][2] >> sh) & 0xff) << 16);
+        if (i < C * 4)
+            wl[i] = dy < 3 ? (int)v : 0;  // (a fourth row of zeros)
+    }
+#pragma unroll
+    for (int k = 0; k < BI; ++k)
+        if (tid + k * DP_THREADS < C)
+            db[tid + k * DP_THREADS] = q.dbias ? dbv[k] : 0;
+#pragma unroll
+    for (int k = 0; k < PI; ++k)
+        if (tid + k * DP_THREADS < ocs)
+            pb[tid + k * DP_THREADS] = q.pbias ? pbv[k] : 0;
+    if (tid < REQUANT_TABLE_ENTRIES) {
+        if (q.dq.mode == 0)
+            dtbl[tid] = q.dtable.t[tid];
+    } else if (q.pq.mode == 0) {
+        ptbl[tid - REQUANT_TABLE_ENTRIES] = q.ptable.t[tid - REQUANT_TABLE_ENTRIES];
+    }
     if (KEEP_P) {
 #pragma unroll
         for (int c = 0; c < KC; ++c)
-            filter(P[KEEP_P ? c : 0], c);
+            filter(P[KEEP_P ? c : 0]);
     }
     lds_barrier();
     struct Band {
         v4i m[S];
         dp_v2u e;  // left, right
     };
-    auto band_filter = [&](int quad, int p) { return (unsigned)wl[((quad * 4 + p) * 4 + (colq & 3)) * 4 + kg4]; };
     auto band_half = [&](unsigned w, int h) __attribute__((always_inline)) {
         v4i m;
 #pragma unroll
@@ -285,7 +312,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
     if (KEEP_D) {
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            const unsigned w = band_filter(quad_of(0), p);
+            const unsigned w = (unsigned)wl[((quad0 * 4 + p) * 4 + (colq & 3)) * 4 + kg4];
 #pragma unroll
             for (int h = 0; h < S; ++h)
                 A[KEEP_D ? p : 0].m[h] = band_half(w, h);
@@ -293,9 +320,14 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
         }
     }
 
+    // LDS places of a lane in job 0 and in the first pixel part of a product; everything else is a constant away
+    const int* const wl0 = wl + ((quad0 * 4) * 4 + (colq & 3)) * 4 + kg4;
+    const int* const db0 = db + quad0 * 16;
+    const int mid0 = (quad0 * T + sub0 * 64 + colq * 4 + kg4) * 16;
+    const int op0 = (kg * T + wpx * NT * 32 + col) * 16;
     // one channel-wise job: 16 channels (plane sets 4 quad ..), 64 pixels; `next` asks for what comes after it as soon as
     // its operands are consumed, so that those loads fly while this one is requantised
-    auto channelwise = [&](int quad, int u, int8_t* m, auto next) __attribute__((always_inline)) {
+    auto channelwise = [&](int i, int8_t* m, auto next) __attribute__((always_inline)) {
         v4i acc[4];
         // the pixels left and right of each column's group
         unsigned L[4], R[4];
@@ -335,9 +367,9 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
         unsigned w[4];
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            acc[p] = *(const v4i*)(db + quad * 16 + p * 4);
+            acc[p] = *(const v4i*)(db0 + i * 128 + p * 4);
             if (!KEEP_D)
-                w[p] = band_filter(quad, p);
+                w[p] = (unsigned)wl0[(i * 32 + p) * 16];
         }
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -368,7 +400,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
                 a[p * 4 + e] = acc[p][e];
         uint32_t d[4];
         dp_requant<DACT>(a, d, q.dq, q.dc, dtbl);
-        *(v4i*)(m + (quad * T + u * 64 + colq * 4 + kg4) * 16) = v4i{(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
+        *(v4i*)(m + mid0 + i * (8 * T * 16)) = v4i{(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
     };
     // ---- pointwise: where a column's results go. (Stores are issued whether or not the place exists: what is under no
     // condition the compiler can count, and the next tile then waits for its loads, not for these stores.)
@@ -406,9 +438,9 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
             __builtin_amdgcn_raw_buffer_store_b32(d[e4], rd, (int)o, (plane + e4 * 2) * ostep, 0);
     };
     auto operand = [&](const int8_t* m, int c, int ni) __attribute__((always_inline)) {
-        return *(const v4i*)(m + ((2 * c + kg) * T + (wpx * NT + ni) * 32 + col) * 16);
+        return *(const v4i*)(m + op0 + c * (2 * T * 16) + ni * 512);
     };
-    // (nothing in flight from here: the loop's own waits are then exact)
+    // (KEEP_P: nothing in flight from here, the loop's own waits are then exact)
     if (KEEP_P)
         wait_vmcnt<0>();
     for (int t = t_begin, buf = 0; t < t_end; ++t, buf ^= 1) {
@@ -416,19 +448,18 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
         cur = rows;
         static_for<JW>([&](auto ii) {
             constexpr int i = decltype(ii)::value;
-            // (several jobs a tile: tiles of 64 pixels, the same rows for all of them)
-            static_assert(JW == 1 || SUB == 1, "");
-            channelwise(quad_of(i), sub_of(i), m, [&]() __attribute__((always_inline)) {
+            channelwise(i, m, [&]() __attribute__((always_inline)) {
                 if (i + 1 < JW) {
-                    request(rows, quad_of(i + 1));
+                    request(rows, i + 1);
                 } else if (KEEP_P) {
-                    rows = rows_of(t + 1, sub_of(0));
-                    request(rows, quad_of(0));
+                    rows = rows_of(t + 1, sub0);
+                    request(rows, 0);
                 } else {
                     // the pointwise filter's first chunks
+                    next_chunk = 0;
 #pragma unroll
                     for (int c = 0; c < RING; ++c)
-                        filter(P[c], c);
+                        filter(P[c]);
                 }
             });
         });
@@ -467,12 +498,12 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
                         acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(P[slot][mi], b, acc[mi][ni], 0, 0, 0);
                 }
                 if (c + RING < KC)
-                    filter(P[slot], c + RING);
+                    filter(P[slot]);
                 // the next tile's first job, behind the last chunk of the filter: loads come back in the order they
                 // were issued, and one asked for after these would wait for them
                 if (c + (RING < KC ? RING : KC) == KC) {
-                    rows = rows_of(t + 1, sub_of(0));
-                    request(rows, quad_of(0));
+                    rows = rows_of(t + 1, sub0);
+                    request(rows, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
