@@ -57,7 +57,10 @@ struct DwPwParams {
     int plane;               // bytes of an input plane set
     int xg, groups;          // groups of 4 pixels per row, in all (a tile: 16 SUB groups)
     int slices;              // workgroups that share a tile's output channels
-    int nb, run_q, run_r;    // workgroups; tiles of a run, and how many runs have one more
+    // tiles of an XCD and how many XCDs have one more, runs of an XCD; tiles of a run and how many runs of an XCD with
+    // the fewer tiles have one more (a single "XCD" where the runs are no multiple of eight); workgroups of an XCD where
+    // those are one, else 0
+    int xcds, xcd_q, xcd_r, xcd_runs, run_q, run_r, per_xcd;
     FastDiv d_xg, d_oh, d_slices;
     RequantPack dq, pq;
     float dc, pc;            // estimates for the tables (mode 0)
@@ -70,8 +73,8 @@ struct DwPwParams {
 __device__ __forceinline__ void dp_begin(const DwPwParams& q) {
 #ifndef MG_HOST_AUDIT
     asm volatile("" ::"s"(q.src), "s"(q.dflt), "s"(q.dbias), "s"(q.wp), "s"(q.pbias), "s"(q.dst), "s"(q.src_bytes), "s"(q.dst_bytes), "s"(q.ih),
-                 "s"(q.iw), "s"(q.oh), "s"(q.ow), "s"(q.OC), "s"(q.OCP), "s"(q.plane), "s"(q.xg), "s"(q.groups), "s"(q.slices), "s"(q.nb),
-                 "s"(q.run_q), "s"(q.run_r), "s"(q.d_xg.mul), "s"(q.d_oh.mul), "s"(q.d_slices.mul));
+                 "s"(q.iw), "s"(q.oh), "s"(q.ow), "s"(q.OC), "s"(q.OCP), "s"(q.plane), "s"(q.xg), "s"(q.groups), "s"(q.slices), "s"(q.xcds),
+                 "s"(q.xcd_q), "s"(q.xcd_r), "s"(q.xcd_runs), "s"(q.per_xcd), "s"(q.run_q), "s"(q.run_r), "s"(q.d_xg.mul), "s"(q.d_oh.mul), "s"(q.d_slices.mul));
     asm volatile("" ::"s"(q.d_xg.shift), "s"(q.d_xg.d), "s"(q.d_oh.shift), "s"(q.d_oh.d), "s"(q.d_slices.shift), "s"(q.d_slices.d), "s"(q.dq.mode),
                  "s"(q.dq.c), "s"(q.dq.d), "s"(q.pq.mode), "s"(q.pq.c), "s"(q.pq.d));
 #endif
@@ -153,10 +156,15 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
     int* const dtbl = pb + ocs;
     int* const ptbl = dtbl + REQUANT_TABLE_ENTRIES;
 
-    // workgroup -> (slice, run of tiles); each XCD gets a contiguous stretch of the runs
-    const int lb = (q.nb & 7) == 0 ? (blockIdx.x & 7) * (q.nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
-    const int wi = (int)fdiv(lb, q.d_slices), slice = lb - wi * q.slices;
-    const int t_begin = wi * q.run_q + min(wi, q.run_r), t_end = t_begin + q.run_q + (wi < q.run_r ? 1 : 0);
+    // Workgroup -> (slice, run of tiles). Each XCD gets a contiguous eighth of the tiles, and the runs with a tile more are the
+    // first ones of every XCD: one to a CU, not two (the first runs of all were, and sat on the same XCDs: 784 tiles for two
+    // workgroups a CU were four tiles for the CUs of three XCDs and two for the others).
+    const int bx = blockIdx.x & 7, bi = blockIdx.x >> 3;
+    const int xcd = q.xcds == 8 ? bx : 0, xi = q.xcds == 8 ? bi : q.per_xcd ? bx * q.per_xcd + bi : blockIdx.x;
+    const int wi = (int)fdiv(xi, q.d_slices), slice = xi - wi * q.slices;
+    const bool more = xcd < q.xcd_r, full = more && q.run_r + 1 == q.xcd_runs;  // (a tile more makes every run longer)
+    const int run_q = q.run_q + (full ? 1 : 0), run_r = full ? 0 : q.run_r + (more ? 1 : 0);
+    const int t_begin = xcd * q.xcd_q + min(xcd, q.xcd_r) + wi * run_q + min(wi, run_r), t_end = t_begin + run_q + (wi < run_r ? 1 : 0);
 
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)q.src, 0, q.src_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)q.dst, 0, q.dst_bytes, 0x00020000);
@@ -654,11 +662,14 @@ TinyNNStatus conv_dw_pw_launch(
         runs = 1;
     if (runs > tiles)
         runs = tiles;
-    q.nb = (int)runs * q.slices;
-    q.run_q = tiles / (int)runs, q.run_r = tiles - q.run_q * (int)runs;
+    q.xcds = runs % 8 == 0 ? 8 : 1;
+    q.xcd_q = tiles / q.xcds, q.xcd_r = tiles - q.xcd_q * q.xcds;
+    q.xcd_runs = (int)runs / q.xcds;
+    q.per_xcd = runs * q.slices % 8 == 0 ? (int)runs * q.slices / 8 : 0;
+    q.run_q = q.xcd_q / q.xcd_runs, q.run_r = q.xcd_q - q.run_q * q.xcd_runs;
     note_kernel("conv_dw_pw", dw.ic / 32, dw.sh, q.slices);
     note_requant_affine(q.dq.mode != 0 && q.pq.mode != 0);
-    hipLaunchKernelGGL(kern, dim3((unsigned)q.nb), dim3(DP_THREADS), lds, stream(), q);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(runs * q.slices)), dim3(DP_THREADS), lds, stream(), q);
     return check_launch("conv_dw_pw");
 }
 
