@@ -91,9 +91,14 @@ void note_requant_affine(bool on);
 TinyNNStatus noalloc_scratch_setup();
 
 // conv_api.hip: a channel-wise 3x3 convolution and the pointwise convolution of its result as one kernel
-// (model runtime only); check_only: whether the kernel takes the pair.
+// (model runtime only). CHECK: whether the kernel takes the pair; PREPARE: everything a launch needs is in the pair's block,
+// which belongs to the caller and keeps the kernel's arguments on the device from one launch to the next.
+struct DwPwBlock;
+DwPwBlock* dw_pw_block_create();
+void dw_pw_block_destroy(DwPwBlock* block);
+enum class DwPw { CHECK, PREPARE, RUN };
 TinyNNStatus dw_pw_run(
-        const MegccPwDwAttr* attr, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, bool check_only);
+        const MegccPwDwAttr* attr, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, DwPwBlock* block, DwPw what);
 // whether it could take the pair, before memory is planned and the pointwise filter packed
 bool dw_pw_takes(
         const MegccConvAttr* dw_attr, const MegccConvAttr* pw_attr, const Tensor* src, const Tensor* dw_flt, const Tensor* mid,

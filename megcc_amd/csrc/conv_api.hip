@@ -55,7 +55,7 @@ TinyNNStatus conv_pw_dw_launch(
 bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dst);
 TinyNNStatus conv_dw_pw_launch(
         const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dflt, const void* dbias, const void* packed,
-        const void* pbias, void* dst);
+        const void* pbias, void* dst, DwPwBlock* block, bool prepare_only);
 
 // A filter that went through megcc_gfx950_conv2d_init is a 1-d byte tensor.
 static bool is_packed_filter(const Tensor* flt) {
@@ -857,7 +857,7 @@ extern "C" TinyNNStatus megcc_gfx950_pw_dw(
 
 // ---- channel-wise 3x3 -> pointwise 1x1 as one operator (model runtime only) ------------------------
 // inputs: source, channel-wise filter [, bias], packed pointwise filter [, bias]; attr.mid_scale is the scale
-// of the tensor in between. check_only: TinyNN_SUCCESS when the kernel takes the pair.
+// of the tensor in between.
 namespace mg {
 bool dw_pw_takes(
         const MegccConvAttr* dw_attr, const MegccConvAttr* pw_attr, const Tensor* src, const Tensor* dw_flt, const Tensor* mid,
@@ -871,7 +871,7 @@ bool dw_pw_takes(
 }
 
 TinyNNStatus dw_pw_run(
-        const MegccPwDwAttr* a, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, bool check_only) {
+        const MegccPwDwAttr* a, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, DwPwBlock* block, DwPw what) {
     const char* who = "dw_pw";
     MG_REQUIRE(a && inputs && outputs && nr_output == 1 && outputs[0] &&
                        nr_input == 3 + (a->pw.with_bias ? 1 : 0) + (a->dw.with_bias ? 1 : 0),
@@ -919,9 +919,11 @@ TinyNNStatus dw_pw_run(
     MG_REQUIRE(conv_dw_pw_supported(dw, pw, src->ptr, dst->ptr) && conv_mfma_supported(pw) &&
                        nr_elem(packed->layout) == conv_mfma_packed_bytes(pw) && aligned16(packed->ptr) && aligned4(dflt->ptr),
                TinyNN_ERROR_NO_IMPLEMENT, "%s: shape, activation or alignment the kernel does not take", who);
-    if (check_only)
+    if (what == DwPw::CHECK)
         return TinyNN_SUCCESS;
+    MG_REQUIRE(block, TinyNN_ERROR_NULL_PTR, "%s: block", who);
     return conv_dw_pw_launch(
-            dw, pw, src->ptr, dflt->ptr, dbias ? dbias->ptr : nullptr, packed->ptr, pbias ? pbias->ptr : nullptr, dst->ptr);
+            dw, pw, src->ptr, dflt->ptr, dbias ? dbias->ptr : nullptr, packed->ptr, pbias ? pbias->ptr : nullptr, dst->ptr, block,
+            what == DwPw::PREPARE);
 }
 }  // namespace mg

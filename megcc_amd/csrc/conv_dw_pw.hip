@@ -30,6 +30,7 @@
 // slices followed the number of tiles and addresses were constants from one place, N=1: 5.1, 5.6, 5.2, 6.4, 9.7, 17.0; N=64, 512 and
 // 1024 channels: 10.9, 18.3. (Two jobs' operands in flight, 16 waves of 128 registers, the whole filter in registers, jobs
 // and products of two wave halves in opposite order: each slower, 512 channels N=1 by 0.4 - 1.6 us.)
+#include <cstring>
 #include <map>
 #include <mutex>
 
@@ -44,8 +45,7 @@ static constexpr int DP_THREADS = 512;
 static constexpr int DP_ALL_BUT_MFMA = 0x7f6;  // what may cross a scheduling barrier: vector, scalar and memory instructions
 typedef unsigned dp_v2u __attribute__((ext_vector_type(2)));
 
-struct DwPwParams {
-    // read together at the start of the kernel (dp_begin)
+struct DwPwArgs {
     const uint32_t* src;
     const uint32_t* dflt;    // [C/4][3][3] dwords of 4 channel bytes
     const int32_t* dbias;    // or NULL
@@ -64,21 +64,73 @@ struct DwPwParams {
     FastDiv d_xg, d_oh, d_slices;
     RequantPack dq, pq;
     float dc, pc;            // estimates for the tables (mode 0)
+};
+// What a workgroup reads at its start, in whole 64-byte lines, and the tables. The kernel gets its address: 8 bytes of
+// arguments, which the launch costs the host 2.5 us, where the 2 KB themselves cost 3.9 (up to 104 bytes 2.6, up to 300 3.3),
+// and an argument that short is in registers when a wave starts (the build asks for it), so that the first round trip goes
+// to these lines instead of the argument segment. Launched again and again, 32 channels N=1 4.5 -> 4.0 us, 512 6.8 -> 6.3.
+struct DwPwParams {
+    union {
+        DwPwArgs a;
+        unsigned words[64];
+    };
     RequantTable dtable, ptable;
 };
+static_assert(sizeof(DwPwArgs) <= 256, "four lines");
 
-// The arguments as the first thing, all of them in one round trip: the compiler otherwise asks for each where it is used, and
-// nine round trips one after the other stood in front of the first load (3300 of a workgroup's 22000 cycles at 512 channels;
-// 0.9 us of every launch).
-__device__ __forceinline__ void dp_begin(const DwPwParams& q) {
-#ifndef MG_HOST_AUDIT
-    asm volatile("" ::"s"(q.src), "s"(q.dflt), "s"(q.dbias), "s"(q.wp), "s"(q.pbias), "s"(q.dst), "s"(q.src_bytes), "s"(q.dst_bytes), "s"(q.ih),
-                 "s"(q.iw), "s"(q.oh), "s"(q.ow), "s"(q.OC), "s"(q.OCP), "s"(q.plane), "s"(q.xg), "s"(q.groups), "s"(q.slices), "s"(q.xcds),
-                 "s"(q.xcd_q), "s"(q.xcd_r), "s"(q.xcd_runs), "s"(q.per_xcd), "s"(q.run_q), "s"(q.run_r), "s"(q.d_xg.mul), "s"(q.d_oh.mul), "s"(q.d_slices.mul));
-    asm volatile("" ::"s"(q.d_xg.shift), "s"(q.d_xg.d), "s"(q.d_oh.shift), "s"(q.d_oh.d), "s"(q.d_slices.shift), "s"(q.d_slices.d), "s"(q.dq.mode),
-                 "s"(q.dq.c), "s"(q.dq.d), "s"(q.pq.mode), "s"(q.pq.c), "s"(q.pq.d));
+// All of the arguments in one round trip: the compiler otherwise asks for each where it is used, and nine round trips one
+// after the other stood in front of the first load (3300 of a workgroup's 22000 cycles at 512 channels; 0.9 us of a launch).
+__device__ __forceinline__ DwPwArgs dp_args(const DwPwParams* p) {
+#ifdef MG_HOST_AUDIT
+    return p->a;
+#else
+    typedef unsigned v16u __attribute__((ext_vector_type(16)));
+    typedef const __attribute__((address_space(4))) v16u* lines;
+    union {
+        v16u v[4];
+        DwPwArgs a;
+    } u;
+    const lines w = (lines)(uintptr_t)p;
+    u.v[0] = w[0], u.v[1] = w[1], u.v[2] = w[2], u.v[3] = w[3];
+    return u.a;
 #endif
 }
+
+// what is kept of a pair between launches: the arguments on the device, and what they were written from
+struct DwPwBlock {
+    void* dev = nullptr;
+    bool valid = false;
+    DwPwParams host;
+};
+#ifndef MG_HOST_AUDIT
+DwPwBlock* dw_pw_block_create() {
+    return new DwPwBlock();
+}
+void dw_pw_block_destroy(DwPwBlock* b) {
+    if (b && b->dev)
+        megcc_gfx950_free(b->dev);
+    delete b;
+}
+static TinyNNStatus dp_upload(DwPwBlock* b, const DwPwParams& all) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    MG_REQUIRE(hipStreamIsCapturing(stream(), &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone, TinyNN_ERROR_RUNTIME,
+               "conv_dw_pw: other arguments under a capture");
+    b->valid = false;
+    if (!b->dev)
+        b->dev = megcc_gfx950_malloc(sizeof(all));
+    MG_REQUIRE(b->dev, TinyNN_ERROR_MEMORY_MALLOC, "conv_dw_pw: arguments");
+    // (launches that read what was there are over, and this copy is, before anything else reads it on whichever stream)
+    TinyNNStatus st = megcc_gfx950_wait();
+    if (st == TinyNN_SUCCESS)
+        st = megcc_gfx950_memcpy_h2d(b->dev, &all, sizeof(all));
+    if (st != TinyNN_SUCCESS)
+        return st;
+    MG_REQUIRE(hipStreamSynchronize(stream()) == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_dw_pw: arguments");
+    b->host = all;
+    b->valid = true;
+    return TinyNN_SUCCESS;
+}
+#endif
 
 // a scalar whose origin the compiler does not know: sums made from it stay where they are written, instead of one register (and,
 // beyond what there are, one spill) for every chunk and plane ahead of the loop
@@ -135,7 +187,7 @@ constexpr int dp_lds(int oc) {
 // wave of the pointwise product; RAG: IW % 4 (the input pixel right of a row's end is in its last piece)
 // DACT, PACT: activations of the two layers (IDENTITY / RELU)
 template <int S, int KC, int SUB, int MT, int NT, int RAG, int DACT, int PACT>
-__global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q) {
+__global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwParams* __restrict__ params) {
     constexpr int C = 32 * KC, NQ = 2 * KC, T = 64 * SUB;
     constexpr int JW = NQ * SUB / 8;                 // channel-wise jobs per wave and tile
     constexpr int WP = T / (32 * NT), WO = 8 / WP;   // waves along the pixels, along the channels
@@ -144,7 +196,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
     // operands: 8 for 4 chunks, 512 channels at N=256 33.1 for 32.2 us, stride 2 21.2 for 20.4
     constexpr int RING = MT == 1 || KC < 16 ? 8 : 4;
     static_assert(JW >= 1 && WP >= 1 && WO >= 1 && WP * WO == 8, "8 waves");
-    dp_begin(q);
+    const DwPwArgs q = dp_args(params);
     extern __shared__ __attribute__((aligned(16))) int8_t dp_lds_mem[];
     int8_t* const mid = dp_lds_mem;                             // [2][NQ][T] 16-byte pieces
     int* const wl = (int*)(mid + 2 * T * C);                    // [C][4]: per channel the filter's 3 rows
@@ -292,9 +344,9 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(DwPwParams q)
             pb[tid + k * DP_THREADS] = q.pbias ? pbv[k] : 0;
     if (tid < REQUANT_TABLE_ENTRIES) {
         if (q.dq.mode == 0)
-            dtbl[tid] = q.dtable.t[tid];
+            dtbl[tid] = params->dtable.t[tid];
     } else if (q.pq.mode == 0) {
-        ptbl[tid - REQUANT_TABLE_ENTRIES] = q.ptable.t[tid - REQUANT_TABLE_ENTRIES];
+        ptbl[tid - REQUANT_TABLE_ENTRIES] = params->ptable.t[tid - REQUANT_TABLE_ENTRIES];
     }
     if (KEEP_P) {
 #pragma unroll
@@ -569,7 +621,7 @@ bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* sr
 }
 
 template <int S, int KC, int SUB, int MT, int NT>
-static void (*dp_kernel(int rag, int dact, int pact))(DwPwParams) {
+static void (*dp_kernel(int rag, int dact, int pact))(const DwPwParams*) {
     // (MobileNets use RELU behind both layers; a RELU-less pointwise layer is the linear bottleneck)
 #define MG_DP_ACT(R_)                                                                                                   \
     (dact == MEGCC_NONLINE_RELU                                                                                          \
@@ -599,8 +651,10 @@ static int dp_resident(const void* kern, size_t lds) {
 
 TinyNNStatus conv_dw_pw_launch(
         const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dflt, const void* dbias, const void* packed,
-        const void* pbias, void* dst) {
-    DwPwParams q = {};
+        const void* pbias, void* dst, DwPwBlock* block, bool prepare_only) {
+    DwPwParams all;
+    memset(all.words, 0, sizeof(all.words));
+    DwPwArgs& q = all.a;
     DpShape s;
     q.xg = (dw.ow + 3) / 4;
     q.groups = dw.n * dw.oh * q.xg;
@@ -628,11 +682,11 @@ TinyNNStatus conv_dw_pw_launch(
     q.dc = make_requant_fast(dw.s_src, dw.s_flt, dw.s_dst).c;
     q.pc = make_requant_fast(pw.s_src, pw.s_flt, pw.s_dst).c;
     if (q.dq.mode == 0)
-        q.dtable = *requant_table_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
+        all.dtable = *requant_table_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
     if (q.pq.mode == 0)
-        q.ptable = *requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
+        all.ptable = *requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
     const int rag = dw.iw & 3;
-    void (*kern)(DwPwParams) = nullptr;
+    void (*kern)(const DwPwParams*) = nullptr;
     size_t lds = 0;
 #define MG_DP(KC_, SUB_, MT_, NT_)                                                                               \
     if (s.kc == KC_ && s.mt == MT_ && s.nt == NT_) {                                                                   \
@@ -667,9 +721,24 @@ TinyNNStatus conv_dw_pw_launch(
     q.xcd_runs = (int)runs / q.xcds;
     q.per_xcd = runs * q.slices % 8 == 0 ? (int)runs * q.slices / 8 : 0;
     q.run_q = q.xcd_q / q.xcd_runs, q.run_r = q.xcd_q - q.run_q * q.xcd_runs;
+#ifdef MG_HOST_AUDIT
+    const DwPwParams* const args = &all;
+#else
+    // the copy on the device is written when the arguments are others than the last time
+    const auto table_differs = [](int mode, const RequantTable& x, const RequantTable& y) { return mode == 0 && memcmp(&x, &y, sizeof(x)) != 0; };
+    if (!block->valid || memcmp(block->host.words, all.words, sizeof(all.words)) != 0 || table_differs(q.dq.mode, block->host.dtable, all.dtable) ||
+        table_differs(q.pq.mode, block->host.ptable, all.ptable)) {
+        TinyNNStatus st = dp_upload(block, all);
+        if (st != TinyNN_SUCCESS)
+            return st;
+    }
+    if (prepare_only)
+        return TinyNN_SUCCESS;
+    const DwPwParams* const args = (const DwPwParams*)block->dev;
+#endif
     note_kernel("conv_dw_pw", dw.ic / 32, dw.sh, q.slices);
     note_requant_affine(q.dq.mode != 0 && q.pq.mode != 0);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(runs * q.slices)), dim3(DP_THREADS), lds, stream(), q);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(runs * q.slices)), dim3(DP_THREADS), lds, stream(), args);
     return check_launch("conv_dw_pw");
 }
 

@@ -53,6 +53,10 @@ struct ModelOpr {
     Workspace ws;
     int first_index = -1;  // index in Model::oprs of the (first) operator this schedule entry stands for
     bool dw_pw = false;    // a channel-wise + pointwise pair as one kernel (desc.attr.pw_dw, no kind of its own)
+    DwPwBlock* block = nullptr;  // ... and its arguments
+    ModelOpr() = default;
+    ModelOpr(const ModelOpr&) = delete;
+    ~ModelOpr() { dw_pw_block_destroy(block); }
 };
 
 struct Model {
@@ -311,7 +315,7 @@ static bool shares_bytes(const Tensor& a, const Tensor& b) {
 static TinyNNStatus call_opr(Model* m, ModelOpr* o) {
     if (o->dw_pw)
         return dw_pw_run(&o->desc.attr.pw_dw, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(),
-                         (int)o->out_ptrs.size(), false);
+                         (int)o->out_ptrs.size(), o->block, DwPw::RUN);
     return megcc_gfx950_call(
             &o->desc, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(), (int)o->out_ptrs.size(), &o->ws,
             &m->opt);
@@ -465,7 +469,9 @@ static void build_schedule(Model* m, Pairs allow) {
                 f->out_ptrs = o1->out_ptrs;
                 bool take = !shares_bytes(*f->in_ptrs[0], *f->out_ptrs[0]) &&
                             dw_pw_run(&f->desc.attr.pw_dw, f->in_ptrs.data(), (int)f->in_ptrs.size(), f->out_ptrs.data(),
-                                      (int)f->out_ptrs.size(), true) == TinyNN_SUCCESS;
+                                      (int)f->out_ptrs.size(), nullptr, DwPw::CHECK) == TinyNN_SUCCESS;
+                if (take)
+                    f->block = dw_pw_block_create();
                 if (take && !options().fuse_dwpw)
                     take = faster_as_one(m, m->dw_pw_time, i, f, {o0, o1});
                 if (take) {
@@ -1254,6 +1260,14 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
             setup_tail(m, best_tb);
         }
     }
+    // (what the first forward would otherwise wait for)
+    for (ModelOpr* o : m->schedule)
+        if (o->dw_pw) {
+            placed = dw_pw_run(&o->desc.attr.pw_dw, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(), (int)o->out_ptrs.size(),
+                               o->block, DwPw::PREPARE);
+            if (placed != TinyNN_SUCCESS)
+                return placed;
+        }
     m->finalized = true;
     return megcc_gfx950_wait();
 }

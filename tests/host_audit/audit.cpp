@@ -92,7 +92,8 @@ TinyNNStatus fc_tile_launch(const ConvGeom&, const void*, const void*, const voi
 bool conv_gather_i8_supported(const ConvGeom& g);
 TinyNNStatus conv_gather_i8_launch(const ConvGeom&, const void*, const void*, const void*, void*);
 bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dst);
-TinyNNStatus conv_dw_pw_launch(const ConvGeom&, const ConvGeom&, const void*, const void*, const void*, const void*, const void*, void*);
+TinyNNStatus conv_dw_pw_launch(
+        const ConvGeom&, const ConvGeom&, const void*, const void*, const void*, const void*, const void*, void*, DwPwBlock*, bool);
 }  // namespace mg
 
 // the bf16 conversion of the compiler's vector types (its value does not matter here)
@@ -223,8 +224,8 @@ static bool run_case(const std::string& line, bool at_end) {
             fprintf(stderr, "not a conv_dw_pw pair: %s\n", line.c_str());
             return false;
         }
-        return conv_dw_pw_launch(dw, pw, src.ptr, df.ptr, bias ? db.ptr : nullptr, wp.ptr, bias ? pb.ptr : nullptr, dst.ptr) ==
-               TinyNN_SUCCESS;
+        return conv_dw_pw_launch(dw, pw, src.ptr, df.ptr, bias ? db.ptr : nullptr, wp.ptr, bias ? pb.ptr : nullptr, dst.ptr, nullptr,
+                                 false) == TinyNN_SUCCESS;
     }
     if (kind == "conv" || kind == "small") {
         ConvGeom g;
