@@ -643,10 +643,13 @@ static void setup_tail(Model* m, int forced = -1) {
             total += us[(size_t)s];
         }
         m->schedule_us = total;
-        // A network whose kernels average under 6 us is bound by launches, not by the device: two
-        // streams then gain or lose a quarter from run to run (MobileNetV1 batch 1: 7.2 k ... 9.9 k
-        // img/s) where one stream or a graph replay is steady. One stream.
-        if (total < 6.0 * n)
+        // A network whose kernels average under 4 us is nothing but launches: what a second stream
+        // could overlap, the host does not enqueue in time. One stream. (Between 4 and 6 us the device
+        // is as busy as the host. MobileNetV1, one stream / two, us for each of many forwards: batch 1
+        // 100 / 96, 2 106 / 98, 4 116 / 101, 8 120 / 102; one blocking forward at a time is the same
+        // on both, 163 and 245 us at batch 1 and 4, copies included. Finding the boundary takes 14 ms,
+        // once for each shape.)
+        if (total < 4.0 * n)
             return;
         double tail = 0;
         for (int s = tb; s < n; ++s)
