@@ -114,11 +114,21 @@ __global__ void __launch_bounds__(CF_THREADS) conv_first_q8_kernel(
 // v_dot4 kernel above spends per output - 9 dot products next to the 10 instructions of the exact
 // requantisation - is what an MFMA saves: here the reduction index is k = 4 * (ic * 3 + fh) + fw with a
 // zero weight at fw = 3, so a lane's 16 K-bytes of the B operand are the 4 bytes at input columns
-// 2 * ox - 1 .. 2 * ox + 2 of four (channel, filter row) pairs = four dword loads from byte addresses,
-// no byte is moved by hand; 9 pairs x 4 bytes = 36 > 32, so a second MFMA takes the ninth pair.
-// A lane's loads stay inside their image row: the first column loads one byte to the right and shifts
-// (its byte 0 is the left padding), the last column one byte to the left.
+// 2 * ox - 1 .. 2 * ox + 2 of four (channel, filter row) pairs; 9 pairs x 4 bytes = 36 > 32, so a second
+// MFMA takes the ninth pair.
+// A wave takes 64 pixels a step, a lane the horizontally adjacent ones 2m and 2m + 1 - columns of two
+// products with the same weights. Both are cut out of the same two aligned dwords (input columns
+// 4m - 4 .. 4m + 3), so a pair of filter rows costs one 8-byte load for two pixels, the results leave as
+// one 8-byte store a plane, and nothing but the very first pixel's dword is special. A wave's steps
+// are consecutive (input rows that two output rows read are in its CU's L1), their number the same for
+// every wave but the last ones. The requantisation by one fused multiply-add needs no table: without
+// one the arguments are an eighth.
+// What bounds it: memory (N = 256: 141 MB in 27.5 us is what a large copy reaches), below 64 images the set-up and
+// the first round trip. 3 x 224 x 224 -> 32 in us, with one pixel a lane, its filter bytes and biases loaded
+// one by one and steps 8192 waves apart (the last round of four nearly empty at N = 64) / as it is:
+// N = 1 3.5 / 3.3, 8 5.2 / 4.5, 32 9.0 / 7.7, 64 13.1 / 11.5, 128 20.0 / 15.8, 256 33.9 / 27.5.
 typedef int cfm_v4i __attribute__((ext_vector_type(4)));
+typedef int cfm_v2i __attribute__((ext_vector_type(2)));
 typedef int cfm_v16i __attribute__((ext_vector_type(16)));
 
 struct ConvFirstMfmaParams {
@@ -126,50 +136,26 @@ struct ConvFirstMfmaParams {
     const int8_t* flt;
     const int32_t* bias;
     uint32_t* dst;
-    int src_bytes;
-    int N, IH, IW, OH, OW, OHW, P, tiles, OC;
+    int src_bytes, dst_bytes;
+    int IH, IW, OW2, OHW, pairs, steps, run, oc4n;
     int act;
     float s_src, s_flt, s_dst, c;
-    float aff_c, aff_d;  // requantisation by one fused multiply-add (epilogue.h); aff_d == 0: table
-    FastDiv dOW, dOHW;
-    RequantTable table;
+    float aff_c, aff_d;  // requantisation by one fused multiply-add (epilogue.h)
+    FastDiv dOW2, dOHW2;
 };
+struct ConvFirstNoTable {};
+static constexpr int CFM_WAVES = 5;  // waves a SIMD holds (N = 256 in us: 2 29.2, 3 28.5, 4 28.3, 5 27.5)
 
-template <int MT, int ACT>
-__global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParams q) {
-    __shared__ int tbl[REQUANT_TABLE_ENTRIES];
+// TABLE: RequantTable, or ConvFirstNoTable where ACT < 0 (the literal sequence) or the fused multiply-add is used
+template <int MT, int ACT, class TABLE>
+__global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParams q, TABLE table) {
+    constexpr bool TAB = sizeof(TABLE) > 64;
+    constexpr int OC = MT * 32;
+    __shared__ int tbl[TAB ? REQUANT_TABLE_ENTRIES : 1];
+    __shared__ __attribute__((aligned(16))) int wlds[9 * OC], blds[OC];
     const int tid = threadIdx.x, lane = tid & 63;
     const int col = lane & 31, kg = lane >> 5;
-    if (ACT >= 0) {
-        tbl[tid] = q.table.t[tid];
-        __syncthreads();
-    }
-    // ---- filter rows of this lane's output channels: A1 = pairs 4 * kg .. 4 * kg + 3, A2 = pair 8
-    auto weight_dword = [&](int oc, int pair) {
-        const int ic = pair / 3, fh = pair - ic * 3;
-        uint32_t w = 0;
-#pragma unroll
-        for (int fw = 0; fw < 3; ++fw)
-            w |= (uint32_t)(uint8_t)q.flt[((((size_t)(oc >> 2) * 3 + fh) * 3 + fw) * 3 + ic) * 4 + (oc & 3)] << (8 * fw);
-        return (int)w;
-    };
-    cfm_v4i A1[MT], A2[MT];
-    int biasv[MT][4][4];
-#pragma unroll
-    for (int mi = 0; mi < MT; ++mi) {
-        const int oc = mi * 32 + col;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            A1[mi][j] = weight_dword(oc, 4 * kg + j);
-        A2[mi] = cfm_v4i{kg == 0 ? weight_dword(oc, 8) : 0, 0, 0, 0};
-        // accumulator register e is channel 8 * (e / 4) + 4 * kg + e % 4 of the row tile
-#pragma unroll
-        for (int e4 = 0; e4 < 4; ++e4)
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                biasv[mi][e4][k] = q.bias ? q.bias[mi * 32 + e4 * 8 + kg * 4 + k] : 0;
-    }
-    // byte offset of this lane's pairs inside an image, relative to (row 2 * oy - 1, column 2 * ox - 1)
+    // byte offset of this lane's (channel, filter row) pairs inside an image, relative to row 2 * oy - 1
     int pair_off[4];
     bool pair_top[4];  // the pair's filter row is 0: above the image when oy == 0
 #pragma unroll
@@ -181,82 +167,110 @@ __global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParam
     const int pair8_off = (2 * q.IH + 2) * q.IW;  // channel 2, filter row 2
     const __amdgpu_buffer_rsrc_t rs =
             __builtin_amdgcn_make_buffer_rsrc((void*)q.src, 0, q.src_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rd =
+            __builtin_amdgcn_make_buffer_rsrc((void*)q.dst, 0, q.dst_bytes, 0x00020000);
     const int OOB = (int)0x80000000u;
-    const int oc4n = q.OC >> 2;
-
-    const int gw = blockIdx.x * 4 + (tid >> 6), nw = gridDim.x * 4;
-    // operands of a tile (requested one tile ahead: the loads fly during the epilogue before them)
-    struct Tile {
-        cfm_v4i B1, B2;
-        int obase;
-        bool ok, first, last;
+    // operands of a step (requested one step ahead: the loads fly during the epilogue before them)
+    struct Step {
+        cfm_v2i d[5];
+        int out;  // byte offset of the two pixels in plane kg
+        bool first;
     };
-    auto request = [&](int t) __attribute__((always_inline)) {
-        Tile r;
+    auto request = [&](int t, int end) __attribute__((always_inline)) {
+        Step r;
         const int p = t * 32 + col;
-        r.ok = t < q.tiles && p < q.P;
-        const int n = fdiv(p, q.dOHW), rem = p - n * q.OHW;
-        const int oy = fdiv(rem, q.dOW), ox = rem - oy * q.OW;
-        // first column: load from column 0 and shift one byte up (byte 0 = padding);
-        // last column: load from column 2 * ox - 2 and shift one byte down (its byte 3 has weight 0)
-        r.first = ox == 0;
-        r.last = 2 * ox + 2 >= q.IW;
-        const int base = n * 3 * q.IH * q.IW + (2 * oy - 1) * q.IW + 2 * ox - 1 + (r.first ? 1 : r.last ? -1 : 0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const bool row_ok = r.ok && !(pair_top[j] && oy == 0);
-            r.B1[j] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, row_ok ? base + pair_off[j] : OOB, 0, 0);
-        }
-        r.B2 = cfm_v4i{(int)__builtin_amdgcn_raw_buffer_load_b32(rs, r.ok && kg == 0 ? base + pair8_off : OOB, 0, 0), 0, 0, 0};
-        r.obase = n * oc4n * q.OHW + rem;
-        return r;
-    };
-    Tile next = request(gw);
-    for (int t = gw; t < q.tiles; t += nw) {
-        const Tile cur = next;
-        auto fix = [&](int v) { return (int)(cur.first ? (unsigned)v << 8 : cur.last ? (unsigned)v >> 8 : (unsigned)v); };
-        cfm_v4i B1, B2 = {fix(cur.B2[0]), 0, 0, 0};
+        const bool ok = t < end && p < q.pairs;
+        const int n = fdiv(p, q.dOHW2), rem = p - n * (q.OHW >> 1);
+        const int oy = fdiv(rem, q.dOW2), m = rem - oy * q.OW2;
+        // the first pixels' left dword is padding: they load one dword further right and use the first one
+        r.first = m == 0;
+        const int base = n * 3 * q.IH * q.IW + (2 * oy - 1) * q.IW + 4 * m - (r.first ? 0 : 4);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            B1[j] = fix(cur.B1[j]);
-        cfm_v16i acc[MT];
+            r.d[j] = __builtin_amdgcn_raw_buffer_load_b64(rs, ok && !(pair_top[j] && oy == 0) ? base + pair_off[j] : OOB, 0, 0);
+        r.d[4] = __builtin_amdgcn_raw_buffer_load_b64(rs, ok && kg == 0 ? base + pair8_off : OOB, 0, 0);
+        r.out = ok ? 4 * ((n * q.oc4n + kg) * q.OHW + 2 * rem) : OOB;
+        return r;
+    };
+    const int t0 = (blockIdx.x * 4 + (tid >> 6)) * q.run, t1 = min(t0 + q.run, q.steps);
+    Step next = request(t0, t1);
+    // ---- filter and bias once per workgroup: 15 single bytes and 16 biases a lane kept the address path busy for 3 us
+    if (tid < OC / 4 * 9) {  // (channel group, pair): four channels' dwords (w0, w1, w2, 0)
+        const int g4 = tid / 9, pair = tid - g4 * 9, ic = pair / 3, fh = pair - ic * 3;
+        const uint32_t* f = (const uint32_t*)q.flt + (g4 * 3 + fh) * 9 + ic;
+        const uint32_t f0 = f[0], f1 = f[3], f2 = f[6];
+        const uint32_t lo = __builtin_amdgcn_perm(f1, f0, 0x05010400u), hi = __builtin_amdgcn_perm(f1, f0, 0x07030602u);
+        *(cfm_v4i*)(wlds + pair * OC + g4 * 4) = cfm_v4i{
+                (int)__builtin_amdgcn_perm(f2, lo, 0x0c040100u), (int)__builtin_amdgcn_perm(f2, lo, 0x0c050302u),
+                (int)__builtin_amdgcn_perm(f2, hi, 0x0c060100u), (int)__builtin_amdgcn_perm(f2, hi, 0x0c070302u)};
+    }
+    if (tid >= 256 - OC)
+        blds[tid - (256 - OC)] = q.bias ? q.bias[tid - (256 - OC)] : 0;
+    if constexpr (TAB)
+        tbl[tid] = table.t[tid];
+    __syncthreads();
+    // filter rows of this lane's output channels: A1 = pairs 4 * kg .. 4 * kg + 3, A2 = pair 8
+    cfm_v4i A1[MT], A2[MT], biasv[MT][4];
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            A1[mi][j] = wlds[(4 * kg + j) * OC + mi * 32 + col];
+        A2[mi] = cfm_v4i{kg == 0 ? wlds[8 * OC + mi * 32 + col] : 0, 0, 0, 0};
+        // accumulator register e is channel 8 * (e / 4) + 4 * kg + e % 4 of the row tile
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4)
+            biasv[mi][e4] = *(const cfm_v4i*)(blds + mi * 32 + e4 * 8 + kg * 4);
+    }
+    auto requant = [&](int a) __attribute__((always_inline)) {
+        if constexpr (ACT < 0)
+            return requant_conv_rt(q.act, a, q.s_src, q.s_flt, q.s_dst);
+        else if constexpr (TAB)
+            return requant_conv_table<ACT>(a, q.c, tbl);
+        else
+            return requant_conv_affine<ACT>(a, q.aff_c, q.aff_d);
+    };
+    for (int t = t0; t < t1; ++t) {
+        cfm_v4i be, bo;  // B operands of the even and the odd pixels
+        int be8, bo8;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) {
+            const uint32_t lo = next.first ? 0u : (uint32_t)next.d[j][0], hi = (uint32_t)(next.first ? next.d[j][0] : next.d[j][1]);
+            const int e = (int)__builtin_amdgcn_alignbyte(hi, lo, 3), o = (int)(hi >> 8);
+            if (j < 4) {
+                be[j] = e;
+                bo[j] = o;
+            } else {
+                be8 = e;
+                bo8 = o;
+            }
+        }
+        const int out = next.out;
+        next = request(t + 1, t1);
 #pragma unroll
         for (int mi = 0; mi < MT; ++mi) {
+            cfm_v16i ae, ao;
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-                acc[mi][e] = biasv[mi][e >> 2][e & 3];
-            acc[mi] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1[mi], B1, acc[mi], 0, 0, 0);
-            acc[mi] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A2[mi], B2, acc[mi], 0, 0, 0);
-        }
-        next = request(t + nw);
+                ae[e] = ao[e] = biasv[mi][e >> 2][e & 3];
+            ae = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1[mi], be, ae, 0, 0, 0);
+            ao = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1[mi], bo, ao, 0, 0, 0);
+            ae = __builtin_amdgcn_mfma_i32_32x32x32_i8(A2[mi], cfm_v4i{be8, 0, 0, 0}, ae, 0, 0, 0);
+            ao = __builtin_amdgcn_mfma_i32_32x32x32_i8(A2[mi], cfm_v4i{bo8, 0, 0, 0}, ao, 0, 0, 0);
 #pragma unroll
-        for (int mi = 0; mi < MT; ++mi) {
-            int r[16];
-            if (ACT >= 0 && q.aff_d != 0.f) {  // (uniform)
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    r[e] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(acc[mi][e], q.aff_c, q.aff_d);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    if (ACT < 0)
-                        r[e] = requant_conv_rt(q.act, acc[mi][e], q.s_src, q.s_flt, q.s_dst);
-                    else
-                        r[e] = requant_conv_table<(ACT < 0 ? 0 : ACT)>(acc[mi][e], q.c, tbl);
-                }
-            }
-            if (cur.ok) {
-#pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4)
-                    q.dst[cur.obase + (mi * 8 + e4 * 2 + kg) * q.OHW] =
-                            pack4_perm(r[e4 * 4], r[e4 * 4 + 1], r[e4 * 4 + 2], r[e4 * 4 + 3]);
+            for (int e4 = 0; e4 < 4; ++e4) {
+                cfm_v2i v;
+                v[0] = (int)pack4_perm(requant(ae[e4 * 4]), requant(ae[e4 * 4 + 1]), requant(ae[e4 * 4 + 2]), requant(ae[e4 * 4 + 3]));
+                v[1] = (int)pack4_perm(requant(ao[e4 * 4]), requant(ao[e4 * 4 + 1]), requant(ao[e4 * 4 + 2]), requant(ao[e4 * 4 + 3]));
+                __builtin_amdgcn_raw_buffer_store_b64(v, rd, out, (mi * 8 + e4 * 2) * q.OHW * 4, 0);
             }
         }
     }
 }
 
-static bool conv_first_mfma_ok(const ConvGeom& g) {
-    return (g.oc == 32 || g.oc == 64) && g.iw >= 4 && (long)g.n * 3 * g.ih * g.iw < (1L << 31) &&
+// (iw >= 8: the first pixels' 8 bytes are in their row)
+static bool conv_first_mfma_ok(const ConvGeom& g, const void* flt) {
+    return ((uintptr_t)flt & 3) == 0 && (g.oc == 32 || g.oc == 64) && g.iw >= 8 && (long)g.n * 3 * g.ih * g.iw < (1L << 31) &&
            (long)g.n * g.oc * g.oh * g.ow < (1L << 31) && !options().no_firstmfma;
 }
 
@@ -268,37 +282,45 @@ static TinyNNStatus conv_first_mfma_launch(
     q.bias = (const int32_t*)bias;
     q.dst = (uint32_t*)dst;
     q.src_bytes = (int)((long)g.n * 3 * g.ih * g.iw);
-    q.N = g.n; q.IH = g.ih; q.IW = g.iw; q.OH = g.oh; q.OW = g.ow;
+    q.dst_bytes = (int)((long)g.n * g.oc * g.oh * g.ow);
+    q.IH = g.ih; q.IW = g.iw; q.OW2 = g.ow / 2;
     q.OHW = g.oh * g.ow;
-    q.P = g.n * q.OHW;
-    q.tiles = (q.P + 31) / 32;
-    q.OC = g.oc;
+    q.pairs = g.n * (q.OHW / 2);
+    q.steps = (q.pairs + 31) / 32;
+    q.oc4n = g.oc / 4;
     q.act = g.act;
     q.s_src = g.s_src; q.s_flt = g.s_flt; q.s_dst = g.s_dst;
     q.c = make_requant_fast(g.s_src, g.s_flt, g.s_dst).c;
-    q.dOW = make_fastdiv(q.OW);
-    q.dOHW = make_fastdiv(q.OHW);
+    q.dOW2 = make_fastdiv(q.OW2);
+    q.dOHW2 = make_fastdiv(q.OHW / 2);
     const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
-    if (tab)
-        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
-    const int act = tab ? g.act : -1;
     const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
     q.aff_c = aff.c;
     q.aff_d = aff.d;
-    const void* kern;
-#define MG_CFM(MT_)                                                                                     \
-    (act == MEGCC_NONLINE_IDENTITY ? (const void*)conv_first_mfma_kernel<MT_, MEGCC_NONLINE_IDENTITY>     \
-     : act == MEGCC_NONLINE_RELU   ? (const void*)conv_first_mfma_kernel<MT_, MEGCC_NONLINE_RELU>         \
-     : act == MEGCC_NONLINE_H_SWISH ? (const void*)conv_first_mfma_kernel<MT_, MEGCC_NONLINE_H_SWISH>     \
-                                   : (const void*)conv_first_mfma_kernel<MT_, -1>)
-    kern = g.oc == 32 ? MG_CFM(1) : MG_CFM(2);
+    // as many waves as are resident at once, and of those only as many as the longest run of steps needs
+    const int most = num_cus() * 4 * CFM_WAVES;
+    q.run = (q.steps + most - 1) / most;
+    const unsigned blocks = (unsigned)(((q.steps + q.run - 1) / q.run + 3) / 4);
+    hipError_t e;
+    const int act = tab ? g.act : -1;
+#define MG_CFM(ACT_, TABLE_) \
+    (g.oc == 32 ? (const void*)conv_first_mfma_kernel<1, ACT_, TABLE_> : (const void*)conv_first_mfma_kernel<2, ACT_, TABLE_>)
+    if (!tab || aff.d != 0.f) {
+        const void* kern = act == MEGCC_NONLINE_IDENTITY ? MG_CFM(MEGCC_NONLINE_IDENTITY, ConvFirstNoTable)
+                         : act == MEGCC_NONLINE_RELU     ? MG_CFM(MEGCC_NONLINE_RELU, ConvFirstNoTable)
+                                                         : MG_CFM(-1, ConvFirstNoTable);
+        ConvFirstNoTable none;
+        void* args[] = {&q, &none};
+        e = hipLaunchKernel(kern, dim3(blocks), dim3(256), args, 0, stream());
+    } else {
+        const void* kern = act == MEGCC_NONLINE_IDENTITY ? MG_CFM(MEGCC_NONLINE_IDENTITY, RequantTable)
+                         : act == MEGCC_NONLINE_RELU     ? MG_CFM(MEGCC_NONLINE_RELU, RequantTable)
+                                                         : MG_CFM(MEGCC_NONLINE_H_SWISH, RequantTable);
+        const std::shared_ptr<const RequantTable> table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+        void* args[] = {&q, (void*)table.get()};
+        e = hipLaunchKernel(kern, dim3(blocks), dim3(256), args, 0, stream());
+    }
 #undef MG_CFM
-    long blocks = (q.tiles + 3) / 4;
-    const long cap = (long)num_cus() * 8;
-    if (blocks > cap)
-        blocks = cap;
-    void* args[] = {&q};
-    hipError_t e = hipLaunchKernel(kern, dim3((unsigned)blocks), dim3(256), args, 0, stream());
     MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_first_mfma: %s", hipGetErrorString(e));
     return check_launch("conv_first_mfma");
 }
@@ -316,7 +338,7 @@ TinyNNStatus conv_first_launch(
     const long pairs = (long)g.n * g.oh * (g.ow / 2);
     if (pairs == 0)
         return TinyNN_SUCCESS;
-    if (conv_first_mfma_ok(g)) {
+    if (conv_first_mfma_ok(g, flt)) {
         note_kernel("conv_first_mfma", g.oc / 32);
         return conv_first_mfma_launch(g, src, flt, bias, dst);
     }

@@ -70,3 +70,23 @@ GENERIC, TIES = test_dw_pw.GENERIC, test_dw_pw.TIES
     (280, 256, 288, 20, 11, 2, A.RELU, GENERIC), (40, 256, 288, 28, 28, 1, A.RELU, TIES)], ids=lambda c: "n%d_c%d_oc%d_%dx%d_s%d_a%d" % c[:7])
 def test_slices_of_channel_wise_pointwise_pairs(cfg):
     test_dw_pw.test_pair_in_one_kernel(cfg)
+
+
+# image widths from the smallest the kernel takes, one output row, steps of 64 pixels that end inside a row, inside an image and
+# behind the last one, one and two steps a wave; every form of the requantisation
+@pytest.mark.parametrize("n,ih,iw", [(1, 2, 8), (3, 2, 8), (1, 6, 12), (5, 10, 36), (2, 4, 132), (1, 34, 260), (30, 224, 224)])
+@pytest.mark.parametrize("oc", [32, 64])
+@pytest.mark.parametrize("act,noaffine", [(A.RELU, 0), (A.IDENTITY, 0), (A.RELU, 1), (A.IDENTITY, 1), (A.H_SWISH, 0), (A.SIGMOID, 0)])
+def test_first_layer_steps(n, ih, iw, oc, act, noaffine):
+    port.set_threads(8)
+    if n == 30 and (noaffine or act in (A.H_SWISH, A.SIGMOID)):
+        pytest.skip("the same steps as with the other activations")
+    case = ConvCase(A.FMT_NCHW_NCHW44, A.DENSE, n, 3, ih, iw, oc, 3, 2, 1, act, bias=n != 3, scales=(0.02, 0.01, unsat(27)))
+    arrays = case.gen(seed=45)
+    runtime.set_option("noaffine", noaffine)
+    try:
+        got = run_gpu(case, arrays)
+        assert runtime.last_kernel().startswith("conv_first_mfma"), runtime.last_kernel()
+    finally:
+        runtime.set_option("noaffine", 0)
+    compare(got, case.run_port(arrays), repr(case))
