@@ -445,10 +445,10 @@ static TinyNNStatus ks_launch(KsParams& q, const KsPlan& p, const char* what) {
     const int tm = p.r * p.mt, tn = p.r * p.nt;
     const int gx = (q.N + tn - 1) / tn, gy = (q.M + tm - 1) / tm;
     q.tiles = gx * gy;
-    // The order of common.h's XcdOrder. For 16 x 16 tiles also where their number is no multiple of the eight XCDs, with up to
-    // seven workgroups without a tile: a tile's rows are half lines, and two XCDs would fetch each (64 x 4096 x 1000 17.2 us
-    // without, 11.8 with; of whole lines the plain order is the faster one then, 200 x 1000 x 700 7.5 / 7.9).
-    const int w = options().no_xcdorder || ((p.r == 32 || CONV) && (q.tiles & 7) != 0) ? 0 : xcd_strip(gx, q.tiles);
+    // The order of common.h's XcdOrder (without / with: 64 x 4096 x 1000 17.2 / 11.8 us, 64 x 3000 x 3900 28.3 / 20.4, 200 x 2000 x 1100
+    // 16.3 / 12.3, 200 x 1000 x 700 7.4 / 7.4), but with the same number of tiles for every XCD and up to seven workgroups
+    // without one where that is no multiple of eight: strips begin with an XCD more often (64 x 4096 x 1000 12.5 / 12.0).
+    const int w = options().no_xcdorder ? 0 : xcd_strip(gx, q.tiles);
     q.per_xcd = w ? (q.tiles + 7) / 8 : 0;
     q.strip_w = w ? w : gx, q.strips = (gx + q.strip_w - 1) / q.strip_w;
     q.d_strip = make_fastdiv((uint32_t)(q.strip_w * gy));

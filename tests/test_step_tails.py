@@ -33,7 +33,7 @@ def test_shares_of_k_in_dense_layers_without_staging(ic, k, stride, ties, bias):
 # of eight, in strips; one and two tiles a CU, and the first size beyond
 @pytest.mark.parametrize("m,k,n", [(5, 1, 5), (16, 15, 16), (17, 16, 15), (15, 17, 33), (33, 63, 31), (31, 64, 49), (16, 65, 32), (48, 255, 16),
                                    (33, 256, 17), (64, 257, 100), (100, 1031, 130), (357, 40, 301), (200, 300, 700), (40, 1300, 1700),
-                                   (512, 70, 256), (512, 270, 257), (23, 2000, 3100)])
+                                   (512, 70, 256), (512, 270, 257), (23, 2000, 3100), (64, 300, 3900), (200, 90, 1111)])
 @pytest.mark.parametrize("ta", [False, True])
 @pytest.mark.parametrize("tb", [False, True])
 def test_f32_products_of_few_tiles(m, k, n, ta, tb):
