@@ -29,6 +29,24 @@ def test_shares_of_k_in_dense_layers_without_staging(ic, k, stride, ties, bias):
     compare(got, case.run_port(arrays), repr(case))
 
 
+# images beyond an XCD's L2, whose tiles are dealt to the XCDs in runs: one, two and several channel tiles, a number of tiles that is and
+# is not a multiple of eight
+@pytest.mark.parametrize("n,ic,ih,iw,oc,k,stride", [(21, 116, 47, 59, 20, 3, 1), (17, 64, 66, 66, 72, 3, 2), (67, 132, 23, 21, 36, 3, 2), (35, 52, 58, 58, 352, 3, 2)])
+@pytest.mark.parametrize("plain", [0, 1])
+def test_tiles_in_runs_on_the_xcds(n, ic, ih, iw, oc, k, stride, plain):
+    port.set_threads(8)
+    assert n * ic * ih * iw > 1 << 22
+    case = ConvCase(A.FMT_NCHW44, A.DENSE, n, ic, ih, iw, oc, k, stride, k // 2, A.RELU, scales=(0.02, 0.01, unsat(ic * k * k)))
+    arrays = case.gen(seed=42)
+    runtime.set_option("noxcdorder", plain)
+    try:
+        got = run_gpu(case, arrays)
+        assert runtime.last_kernel().startswith("conv_mfma_i8_gather"), runtime.last_kernel()
+    finally:
+        runtime.set_option("noxcdorder", 0)
+    compare(got, case.run_port(arrays), repr(case))
+
+
 # rows, columns and K at the edges of the 16 x 16 tiles and their steps of 16, four and eight waves; tiles that are no multiple
 # of eight, in strips; one and two tiles a CU, and the first size beyond
 @pytest.mark.parametrize("m,k,n", [(5, 1, 5), (16, 15, 16), (17, 16, 15), (15, 17, 33), (33, 63, 31), (31, 64, 49), (16, 65, 32), (48, 255, 16),
