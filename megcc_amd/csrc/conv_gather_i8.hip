@@ -19,7 +19,7 @@
 // kernel of conv_mfma_i8.hip, beyond 9 taps conv_dot4.hip; then with steps beyond a wave's share fetched as zeros, the
 // table read before the first operand and the arguments where they are used; now): 6 x 88 -> 148 57 x 43 stride 2
 // 14.6, 7.1, 5.9; 4 x 24 -> 68 98 x 98 stride 2 14.8, 5.7, 4.2; 1 x 356 -> 52 68 x 81 21.2, 8.4, 7.6; 1 x 256 -> 256 28 x 28
-// 8.0, 5.6, 5.0; 47 x 104 -> 48 89 x 89 95.8, 50.5, 40.8; 58 x 264 -> 320 70 x 70 stride 2 216, 176, 156; 5x5: 1 x 120 -> 280
+// 8.0, 5.6, 4.9; 47 x 104 -> 48 89 x 89 95.8, 50.5, 40.8; 58 x 264 -> 320 70 x 70 stride 2 216, 176, 156; 5x5: 1 x 120 -> 280
 // 19 x 19 134, 6.6, 5.8; 60 x 28 -> 20 63 x 63 137, 21.4, 17.4.
 // Reference loop: BareMetal/ConvKernel.cpp:305-344.
 #include "conv_mfma_i8.h"
@@ -34,8 +34,6 @@ struct GatherParams {
     int8_t* dst;
     unsigned src_bytes, wp_bytes;
     int P, OC, steps, taps, lkw;  // steps = chunks * taps; log2 of the groups that share K
-    int tiles;  // in a row: an eighth of them on each XCD, channel tiles (dOct: their number) first; 0: a grid of pixel x channel tiles
-    FastDiv dOct;
     unsigned step_bytes;         // of the packed filter
     unsigned plane, image, row;  // bytes of the source
     int IH, IW, OHW, OW, FW, SH, SW, PH, PW, DH, DW;
@@ -43,6 +41,10 @@ struct GatherParams {
     int act;
     float s_src, s_flt, s_dst;
     float c, aff_c, aff_d;  // scale of the table's estimate; the fused multiply-add (aff_d 0: none, the table)
+    // (tiles in runs on the XCDs) pixel tiles; whether a channel tile hangs over, which is then behind all the others of
+    // its XCD; the number of the others
+    int ptiles, ragged;
+    FastDiv dOct;
     RequantTable table;
 };
 
@@ -51,7 +53,7 @@ struct GatherParams {
 __device__ __forceinline__ void gather_begin(const GatherParams& q) {
 #ifndef MG_HOST_AUDIT
     asm volatile("" ::"s"(q.src), "s"(q.wp), "s"(q.bias), "s"(q.dst), "s"(q.src_bytes), "s"(q.wp_bytes), "s"(q.P), "s"(q.OC), "s"(q.steps), "s"(q.taps),
-                 "s"(q.lkw), "s"(q.tiles), "s"(q.step_bytes), "s"(q.plane), "s"(q.image), "s"(q.row), "s"(q.IH), "s"(q.IW), "s"(q.OHW), "s"(q.OW), "s"(q.SH), "s"(q.SW),
+                 "s"(q.lkw), "s"(q.step_bytes), "s"(q.plane), "s"(q.image), "s"(q.row), "s"(q.IH), "s"(q.IW), "s"(q.OHW), "s"(q.OW), "s"(q.SH), "s"(q.SW),
                  "s"(q.PH), "s"(q.PW), "s"(q.DH), "s"(q.DW), "s"(q.dOHW.mul), "s"(q.dOW.mul), "s"(q.dTaps.mul), "s"(q.dFW.mul), "s"(q.aff_d));
 #endif
 }
@@ -66,12 +68,18 @@ __device__ __forceinline__ int gather_table(int i) {
 // ACT: an activation whose outputs the threshold table describes, or -1 (the literal sequence of q.act)
 static constexpr int GATHER_LOG2_WAVES = 2, GATHER_WAVES = 1 << GATHER_LOG2_WAVES;  // of a workgroup
 
-template <int MT, int NT, int ACT>
+// RUNS: every XCD has an eighth of the pixel tiles, each with all its channel tiles, in a row (conv_gather_i8_launch); else a
+// grid of pixel x channel tiles
+template <int MT, int NT, int ACT, bool RUNS>
 __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(GatherParams q) {
     constexpr int RING = 4;  // steps in flight (8: no step faster, 256 -> 256 28 x 28 5.1 us for 5.0, 4 x 24 -> 68 4.9 for 4.2)
     static_assert(64 * GATHER_WAVES == REQUANT_TABLE_ENTRIES, "an entry a thread");
     extern __shared__ __attribute__((aligned(16))) int gather_lds[];
     gather_begin(q);
+    // (Never taken. The block's end keeps the whole set-up behind the one wait for the arguments, where the compiler had it
+    // wait for single ones again: 256 -> 256 28 x 28 5.05 -> 4.91 us, 1 x 512 -> 512 7 x 7 7.0 -> 6.8.)
+    if (!RUNS && q.P <= 0)
+        return;
     int* const bias = gather_lds + REQUANT_TABLE_ENTRIES;  // [32 MT]
     int* const parts = bias + 32 * MT;
     const int lane = threadIdx.x & 63, col = lane & 31, kg = lane >> 5;
@@ -80,10 +88,18 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
     const int kw = 1 << q.lkw, lpw = GATHER_LOG2_WAVES - q.lkw, pw = 1 << lpw;
     const int grp = wave >> lpw, sub = wave & (pw - 1);
     int tx = blockIdx.x, ty = blockIdx.y;
-    if (q.tiles) {
-        const int xcd = tx & 7, place = xcd * (q.tiles >> 3) + min(xcd, q.tiles & 7) + (tx >> 3);
-        tx = (int)fdiv(place, q.dOct);
-        ty = place - tx * (int)q.dOct.d;
+    if constexpr (RUNS) {
+        const int xcd = tx & 7, i = tx >> 3, extra = q.ptiles & 7, mine = (q.ptiles >> 3) + (xcd < extra);
+        const int first = xcd * (q.ptiles >> 3) + min(xcd, extra), whole = mine * (int)q.dOct.d;
+        tx = (int)fdiv(i, q.dOct);
+        ty = i - tx * (int)q.dOct.d;
+        if (i >= whole) {
+            tx = i - whole;
+            ty = (int)q.dOct.d;
+            if (!q.ragged || tx >= mine)  // (the whole workgroup: an XCD with a pixel tile less)
+                return;
+        }
+        tx += first;
     }
     const int oc0 = ty * (32 * MT), p0 = (tx * pw + sub) * (32 * NT);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)q.src, 0, (int)q.src_bytes, 0x00020000);
@@ -316,24 +332,29 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     } else if (mt * nt == 4 && q.steps >= 72 && tiles() < 4 * full) {
         kw = 2;
     }
-#define MG_GATHER_A(MT_, NT_)                                                                          \
-    (!table                              ? conv_gather_i8_kernel<MT_, NT_, -1>                         \
-     : g.act == MEGCC_NONLINE_IDENTITY   ? conv_gather_i8_kernel<MT_, NT_, MEGCC_NONLINE_IDENTITY>     \
-     : g.act == MEGCC_NONLINE_RELU       ? conv_gather_i8_kernel<MT_, NT_, MEGCC_NONLINE_RELU>         \
-                                         : conv_gather_i8_kernel<MT_, NT_, MEGCC_NONLINE_H_SWISH>)
-    void (*kern)(GatherParams) = mt == 2 ? (nt == 2 ? MG_GATHER_A(2, 2) : MG_GATHER_A(2, 1))
-                                         : (nt == 2 ? MG_GATHER_A(1, 2) : MG_GATHER_A(1, 1));
-#undef MG_GATHER_A
-    const int pw = GATHER_WAVES / kw;
-    const int gx = (q.P + 32 * nt * pw - 1) / (32 * nt * pw), gy = (g.oc + 32 * mt - 1) / (32 * mt);
     // Where the image is more than an XCD's L2 holds, neighbouring pixels - rows of the image that both read - and a pixel
     // tile's channel tiles on one XCD (us without / with: 58 x 264 -> 320 70 x 70 stride 2 171 / 156, 21 x 116 -> 20 47 x 59
     // 10.4 / 8.9, 50 x 192 -> 20 58 x 42 stride 2 12.3 / 10.9, 47 x 104 -> 48 89 x 89 41.9 / 40.8, 10 x 136 -> 20 84 x 84 14.8 /
-    // 14.8; below, 256 -> 256 28 x 28 5.01 / 5.08, from the order's arithmetic).
-    const bool spread = q.src_bytes > (1u << 22) && !options().no_xcdorder;
-    q.tiles = spread ? gx * gy : 0;
-    q.dOct = make_fastdiv(gy);
-    const dim3 grid((unsigned)(spread ? gx * gy : gx), (unsigned)(spread ? 1 : gy));
+    // 14.9; in one kernel with the grid's order the arithmetic cost smaller layers 0.1 - 0.2 us). A channel tile that hangs over is the
+    // quicker one and fills the last round best, behind the others: 23 x 36 -> 144 87 x 74 31.9 us without, 34.6 with the three side
+    // by side, 31.7; 23 x 100 -> 144 48.6, 48.7, 46.0.
+    const bool runs = q.src_bytes > (1u << 22) && !options().no_xcdorder;
+    const int pw = GATHER_WAVES / kw;
+    const int gx = (q.P + 32 * nt * pw - 1) / (32 * nt * pw), gy = (g.oc + 32 * mt - 1) / (32 * mt);
+    q.ptiles = gx;
+    q.ragged = g.oc % (32 * mt) != 0 && gy > 1;
+    q.dOct = make_fastdiv(gy - q.ragged);
+    const dim3 grid((unsigned)(runs ? (gx + 7) / 8 * 8 * gy : gx), (unsigned)(runs ? 1 : gy));
+#define MG_GATHER_R(MT_, NT_, ACT_) (runs ? conv_gather_i8_kernel<MT_, NT_, ACT_, true> : conv_gather_i8_kernel<MT_, NT_, ACT_, false>)
+#define MG_GATHER_A(MT_, NT_)                                                                \
+    (!table                              ? MG_GATHER_R(MT_, NT_, -1)                         \
+     : g.act == MEGCC_NONLINE_IDENTITY   ? MG_GATHER_R(MT_, NT_, MEGCC_NONLINE_IDENTITY)     \
+     : g.act == MEGCC_NONLINE_RELU       ? MG_GATHER_R(MT_, NT_, MEGCC_NONLINE_RELU)         \
+                                         : MG_GATHER_R(MT_, NT_, MEGCC_NONLINE_H_SWISH))
+    void (*kern)(GatherParams) = mt == 2 ? (nt == 2 ? MG_GATHER_A(2, 2) : MG_GATHER_A(2, 1))
+                                         : (nt == 2 ? MG_GATHER_A(1, 2) : MG_GATHER_A(1, 1));
+#undef MG_GATHER_A
+#undef MG_GATHER_R
     q.lkw = kw == 4 ? 2 : kw == 2 ? 1 : 0;
     note_kernel("conv_mfma_i8_gather", 32 * mt, 32 * nt, kw);
     const RequantAffine aff = requant_affine_pick(table, g.act, g.s_src, g.s_flt, g.s_dst);

@@ -29,9 +29,10 @@ def test_shares_of_k_in_dense_layers_without_staging(ic, k, stride, ties, bias):
     compare(got, case.run_port(arrays), repr(case))
 
 
-# images beyond an XCD's L2, whose tiles are dealt to the XCDs in runs: one, two and several channel tiles, a number of tiles that is and
-# is not a multiple of eight
-@pytest.mark.parametrize("n,ic,ih,iw,oc,k,stride", [(21, 116, 47, 59, 20, 3, 1), (17, 64, 66, 66, 72, 3, 2), (67, 132, 23, 21, 36, 3, 2), (35, 52, 58, 58, 352, 3, 2)])
+# images beyond an XCD's L2, whose tiles are dealt to the XCDs in runs: one, two and several channel tiles, the last one whole or hanging over,
+# a number of pixel tiles that is and is not a multiple of eight
+@pytest.mark.parametrize("n,ic,ih,iw,oc,k,stride", [(21, 116, 47, 59, 20, 3, 1), (17, 64, 66, 66, 72, 3, 2), (67, 132, 23, 21, 36, 3, 2), (35, 52, 58, 58, 352, 3, 2), (23, 36, 87, 74, 144, 3, 1),
+                                                    (23, 36, 87, 74, 64, 3, 1)])
 @pytest.mark.parametrize("plain", [0, 1])
 def test_tiles_in_runs_on_the_xcds(n, ic, ih, iw, oc, k, stride, plain):
     port.set_threads(8)
