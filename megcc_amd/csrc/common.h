@@ -37,8 +37,9 @@ TinyNNStatus fail(TinyNNStatus st, const char* fmt, ...) __attribute__((format(p
 // ones of a tile more where the number is no multiple of 8) of an order that walks the grid in strips of `w`
 // columns, row by row inside a strip: the tiles one XCD owns are then a compact rectangle and each
 // operand panel is fetched by the one or two XCDs that need it. w = 0 keeps the plain order. Any w >= 1
-// gives a bijection. (Without / with where the number is no multiple of 8, us: FullyConnected 246 x 3742 x 2207
-// 16.2 / 14.8, 591 x 1822 x 2221 15.3 / 13.9, 873 x 4053 x 3853 48.0 / 44.4, 1596 x 3557 x 3128 50.2 / 49.3.)
+// gives a bijection. Where the number is no multiple of 8, only for operands (`bytes`) of more than half an L2
+// (without / with, us: FullyConnected 246 x 3742 x 2207 16.2 / 14.8, 591 x 1822 x 2221 15.3 / 13.9, 873 x 4053 x 3853
+// 48.0 / 44.4, 2355 x 717 x 2650 18.9 / 18.3; below, 898 x 1104 x 690 7.5 / 7.7, 3844 x 171 x 2463 19.3 / 20.4).
 struct XcdOrder {
     int w;
 };
@@ -53,8 +54,8 @@ inline int xcd_strip(int gx, long tiles) {
         w *= 2;
     return w < gx ? w : gx;
 }
-inline XcdOrder make_xcd_order(int gx, int gy) {
-    return {xcd_strip(gx, (long)gx * gy)};
+inline XcdOrder make_xcd_order(int gx, int gy, long bytes) {
+    return {((long)gx * gy & 7) != 0 && bytes <= (2L << 20) ? 0 : xcd_strip(gx, (long)gx * gy)};
 }
 __device__ __forceinline__ void xcd_tile(XcdOrder o, int bx, int by, int gx, int gy, int& tx, int& ty) {
     tx = bx;

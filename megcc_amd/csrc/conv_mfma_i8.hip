@@ -710,7 +710,7 @@ TinyNNStatus conv_mfma_launch(
     if (pipe) {
         // (FullyConnected tiles: each XCD a compact rectangle of the tile grid, common.h)
         q.xo = pc.fcb && !options().no_xcdorder
-                       ? make_xcd_order((q.P + q.range_len - 1) / q.range_len, (q.OC + pc.bm - 1) / pc.bm)
+                       ? make_xcd_order((q.P + q.range_len - 1) / q.range_len, (q.OC + pc.bm - 1) / pc.bm, (long)(q.P + q.OC) * g.ic)
                        : XcdOrder{0};
         if (pc.fcb && pc.bm == 256 && q.dst_fc == 2)
             q.dst_fc = 3;  // rows leave through the kernel's staging area in LDS

@@ -255,7 +255,7 @@ TinyNNStatus fc_tile_launch(const ConvGeom& g, const void* src, const void* pack
 #undef MG_FCT
     const int b = wide ? 128 : 64;
     const dim3 grid((g.oc + b - 1) / b, (g.n + b - 1) / b);
-    q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y);
+    q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y, (long)(q.M + q.OC) * q.K);
     note_kernel(q.xo.w ? "fc_tile_xo" : "fc_tile", b, kw);
     hipLaunchKernelGGL(kern, grid, dim3(256 * kw), 0, stream(), q);
     return check_launch("fc_tile");

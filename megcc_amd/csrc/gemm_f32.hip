@@ -509,14 +509,14 @@ TinyNNStatus conv_f32_gemm_launch(
     const bool longk = q.kchunk > 1024;
     if (q.M <= 64 && (long)((q.N + 255) / 256) * q.split >= 128) {
         dim3 grid((q.N + 255) / 256, 1, q.split);
-        q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y);
+        q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y, 4L * (q.M + q.N) * q.K);
         if (longk)
             hipLaunchKernelGGL((gemm_f32_kernel<true, true, true, 64, true>), grid, dim3(256), 0, stream(), q);
         else
             hipLaunchKernelGGL((gemm_f32_kernel<true, true, true, 64>), grid, dim3(256), 0, stream(), q);
     } else {
         dim3 grid((q.N + GBN - 1) / GBN, (q.M + GBM - 1) / GBM, q.split);
-        q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y);
+        q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y, 4L * (q.M + q.N) * q.K);
         if (longk)
             hipLaunchKernelGGL((gemm_f32_kernel<true, true, true, 128, true>), grid, dim3(256), 0, stream(), q);
         else
@@ -594,7 +594,7 @@ extern "C" TinyNNStatus megcc_gfx950_matmul(
     const bool skinny = q.M <= 64 && (long)((q.N + 255) / 256) * q.split >= 128;
     dim3 grid(skinny ? (q.N + 255) / 256 : (q.N + GBN - 1) / GBN, skinny ? 1 : (q.M + GBM - 1) / GBM,
               q.split);
-    q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y);
+    q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y, 4L * (q.M + q.N) * q.K);
     note_kernel("gemm_f32", skinny ? 64 : 128, q.split, q.kchunk > 1024, q.xo.w);
     const bool longk = q.kchunk > 1024;
 #define MG_GEMM_LAUNCH(AK, BN_)                                                                  \

@@ -57,7 +57,7 @@ struct KsParams {
     const float* bias;
     unsigned a_bytes, b_bytes;
     unsigned a_row, a_k, b_row, b_k;  // byte strides: of A's rows / B's columns, and along K
-    // tiles in strips of strip_w columns, row by row inside a strip; per_xcd: of them on each XCD (0: as the workgroups come)
+    // tiles in strips of strip_w columns, row by row inside a strip; per_xcd: of them on each XCD (0: a grid of tiles)
     int tiles, per_xcd, strip_w, strips;
     FastDiv d_strip, d_w, d_last;
     int M, N, K, ldc;
@@ -107,13 +107,16 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lw = q.lw, W = 1 << lw;
     const int h = lane / R, c = lane & (R - 1);
-    const int place = q.per_xcd ? (int)(blockIdx.x & 7) * q.per_xcd + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
-    if (place >= q.tiles)  // (the whole workgroup)
-        return;
-    const int strip = (int)fdiv(place, q.d_strip), in = place - strip * (int)q.d_strip.d;
-    const bool last = strip == q.strips - 1;
-    const int ty = last ? (int)fdiv(in, q.d_last) : (int)fdiv(in, q.d_w);
-    const int tx = strip * q.strip_w + in - ty * (int)(last ? q.d_last.d : q.d_w.d);
+    int tx = blockIdx.x, ty = blockIdx.y;
+    if (q.per_xcd) {
+        const int place = (tx & 7) * q.per_xcd + (tx >> 3);
+        if (place >= q.tiles)  // (the whole workgroup)
+            return;
+        const int strip = (int)fdiv(place, q.d_strip), in = place - strip * (int)q.d_strip.d;
+        const bool last = strip == q.strips - 1;
+        ty = last ? (int)fdiv(in, q.d_last) : (int)fdiv(in, q.d_w);
+        tx = strip * q.strip_w + in - ty * (int)(last ? q.d_last.d : q.d_w.d);
+    }
     const int m0 = ty * (R * MT), n0 = tx * (R * NT);
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)q.A, 0, (int)q.a_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)q.B, 0, (int)q.b_bytes, 0x00020000);
@@ -268,15 +271,11 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
             constexpr int r = decltype(rc)::value;
             load_a(step(0, r), av[r]);
         });
-    // (the biases of the rows this wave finishes: asked for here, not behind the sums)
-    float bias[4] = {0.f, 0.f, 0.f, 0.f};
-    if (CONV && q.bias) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = min(wave + i * W, SUMS - 1);
-            bias[i] = q.bias[min(m0 + (R == 32 ? 8 * (r >> 2) : 0) + 4 * h + (r & 3), q.M - 1)];
-        }
-    }
+    // (16 x 16: the bias of the row this lane finishes, asked for here, not behind the sums. 32 x 32 tiles, several a CU, fetch
+    // theirs where they are used: with four prefetched and an epilogue unrolled for them, 21 -> 69 26 x 30 N=13 10.1 us for 9.6.)
+    float bias = 0.f;
+    if (CONV && R == 16 && q.bias)
+        bias = q.bias[min(m0 + 4 * h + (wave & 3), q.M - 1)];
     if (CONV) {
         __syncthreads();
         boff[0] = (unsigned)pix[c] + (BMODE == KS_CONV1 ? (unsigned)(4 * h) * q.b_k : 0u);
@@ -339,7 +338,8 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         multiply(at, bt);
     }
 
-    close();
+    if (R == 16)
+        close();
 
     // the waves' sums meet in LDS: [wave][tile][register][lane]
     if (CONV)
@@ -351,15 +351,10 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int e = 0; e < SUMS; ++e)
-                ks_lds[wave * TILE + ((i * NT + j) * SUMS + e) * 64 + lane] = sum[i][j][e];
+                ks_lds[wave * TILE + ((i * NT + j) * SUMS + e) * 64 + lane] = R == 16 ? sum[i][j][e] : acc[0][i][j][e] + sum[i][j][e];
     __syncthreads();
     // register e of a tile: row 8 * (e / 4) + 4 * h + e % 4 (16 x 16: 4 * h + e), column c. Wave w finishes registers w, w + W, ...
-    constexpr int TURNS = (MT * NT * SUMS + 3) / 4;  // (of four waves; eight are done after half of them)
-#pragma unroll
-    for (int i_r = 0; i_r < TURNS; ++i_r) {
-        const int r = wave + i_r * W;
-        if (r >= MT * NT * SUMS)
-            break;
+    for (int r = wave; r < MT * NT * SUMS; r += W) {
         const int t = r / SUMS, e = r & (SUMS - 1), i = t / NT, j = t - i * NT;
         float v = 0.f;
 #pragma unroll 4
@@ -369,7 +364,7 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         if (m >= q.M || n >= q.N)
             continue;
         if (CONV) {
-            q.C[((size_t)img * q.M + m) * q.ohw + rem] = ks_act(q.act, v + bias[i_r & 3]);
+            q.C[((size_t)img * q.M + m) * q.ohw + rem] = ks_act(q.act, v + (R == 16 ? bias : q.bias ? q.bias[m] : 0.f));
         } else {
             q.C[(size_t)m * q.ldc + n] = v;
         }
@@ -445,16 +440,19 @@ static TinyNNStatus ks_launch(KsParams& q, const KsPlan& p, const char* what) {
     const int tm = p.r * p.mt, tn = p.r * p.nt;
     const int gx = (q.N + tn - 1) / tn, gy = (q.M + tm - 1) / tm;
     q.tiles = gx * gy;
-    // The order of common.h's XcdOrder (without / with: 64 x 4096 x 1000 17.2 / 11.8 us, 64 x 3000 x 3900 28.3 / 20.4, 200 x 2000 x 1100
-    // 16.3 / 12.3, 200 x 1000 x 700 7.4 / 7.4), but with the same number of tiles for every XCD and up to seven workgroups
-    // without one where that is no multiple of eight: strips begin with an XCD more often (64 x 4096 x 1000 12.5 / 12.0).
-    const int w = options().no_xcdorder ? 0 : xcd_strip(gx, q.tiles);
+    // The order of common.h's XcdOrder, but where the number of tiles is no multiple of eight with the same number for every
+    // XCD and up to seven workgroups without one: strips begin with an XCD more often (64 x 4096 x 1000 12.5 / 12.0 us). Then for
+    // 16 x 16 tiles - a row of theirs is half a line, and two XCDs would fetch each (64 x 4096 x 1000 17.2 without, 12.0 with) -
+    // and for operands beyond an L2 (64 x 3000 x 3900 28.3 / 20.0, 200 x 2000 x 1100 16.3 / 12.6, 64 x 250 x 3900 4.65 / 4.64; below,
+    // 1109 x 309 x 402 nt 7.6 / 7.9), not for convolutions (18 -> 48 27 x 46 N=13 9.0 / 9.9, 11 -> 98 29 x 29 N=8 7.9 / 8.3).
+    const bool odd = (q.tiles & 7) != 0, order = !odd || (!CONV && (p.r == 16 || 4L * (q.M + q.N) * q.K > (4L << 20)));
+    const int w = options().no_xcdorder || !order ? 0 : xcd_strip(gx, q.tiles);
     q.per_xcd = w ? (q.tiles + 7) / 8 : 0;
     q.strip_w = w ? w : gx, q.strips = (gx + q.strip_w - 1) / q.strip_w;
     q.d_strip = make_fastdiv((uint32_t)(q.strip_w * gy));
     q.d_w = make_fastdiv((uint32_t)q.strip_w);
     q.d_last = make_fastdiv((uint32_t)(gx - (q.strips - 1) * q.strip_w));
-    const dim3 grid((unsigned)(w ? 8 * q.per_xcd : q.tiles));
+    const dim3 grid((unsigned)(w ? 8 * q.per_xcd : gx), (unsigned)(w ? 1 : gy));
     q.lw = p.waves == 8 ? 3 : 2;
     note_kernel(what, tm, tn, p.waves, w);
     size_t lds = (size_t)p.waves * tm * tn * 4;

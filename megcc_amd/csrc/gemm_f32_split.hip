@@ -359,7 +359,7 @@ TinyNNStatus gemm_f32_split_launch(const GevmArgs& v, int ta, int tb) {
     q.a_bytes = side_bytes(v.M, v.a_rs, v.a_cs, v.K);
     q.b_bytes = side_bytes(v.N, v.b_cs, v.b_rs, v.K);
     const dim3 grid((unsigned)((q.N + SP_T - 1) / SP_T), (unsigned)((q.M + SP_T - 1) / SP_T));
-    q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y);
+    q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y, 4L * (q.M + q.N) * q.K);
     note_kernel("gemm_f32_split", SP_T, SP_T, q.xo.w);
 #define MG_SP_K(AK_, BK_) (v.K <= SP_SHORT_K ? gemm_f32_split_kernel<AK_, BK_, true> : gemm_f32_split_kernel<AK_, BK_, false>)
     void (*kern)(SplitParams) = !ta ? (tb ? MG_SP_K(true, true) : MG_SP_K(true, false))
