@@ -116,6 +116,10 @@ struct Model {
     hipStream_t tail_stream = nullptr;
     hipEvent_t ev_head = nullptr, ev_tail = nullptr;
     bool tail_pending = false, tail_reads_input = false;
+    // The caller has waited for a result since the last forward: nothing is left that the next one's head could overlap, and
+    // on one stream it is over sooner, with no event between head and tail (batch 1, image in, forward, result out, us: 184 -
+    // 187 and unsteady on two, 171 - 173 on one).
+    bool drained = false;
     std::vector<char> waits_tail;
     std::vector<const Tensor*> tail_writes;  // tensors the tail's operators write
     void* tail_workspace = nullptr;
@@ -646,9 +650,9 @@ static void setup_tail(Model* m, int forced = -1) {
         // A network whose kernels average under 4 us is nothing but launches: what a second stream
         // could overlap, the host does not enqueue in time. One stream. (Between 4 and 6 us the device
         // is as busy as the host. MobileNetV1, one stream / two, us for each of many forwards: batch 1
-        // 100 / 96, 2 106 / 98, 4 116 / 101, 8 120 / 102; one blocking forward at a time is the same
-        // on both, 163 and 245 us at batch 1 and 4, copies included. Finding the boundary takes 14 ms,
-        // once for each shape.)
+        // 100 / 96, 2 106 / 98, 4 116 / 101, 8 120 / 102; a forward whose result is waited for before
+        // the next one runs on one stream: Model::drained. Finding the boundary takes 14 ms, once for
+        // each shape.)
         if (total < 4.0 * n)
             return;
         double tail = 0;
@@ -1351,7 +1355,9 @@ TinyNNStatus megcc_gfx950_model_get_output(void* model, int tensor, void* host, 
     MG_REQUIRE(bytes == tensor_bytes(t), TinyNN_ERROR_INVALID_LAYOUT,
                "model_get_output: %zu bytes asked, tensor has %zu", bytes, tensor_bytes(t));
     join_tail(m);
-    return megcc_gfx950_memcpy_d2h(host, t.ptr, bytes);
+    const TinyNNStatus st = megcc_gfx950_memcpy_d2h(host, t.ptr, bytes);
+    m->drained = st == TinyNN_SUCCESS;
+    return st;
 }
 
 // The copy is enqueued behind the forward that produced the tensor - on the tail stream when the last
@@ -1389,8 +1395,11 @@ TinyNNStatus megcc_gfx950_model_forward(void* model) {
     };
     if (m->graph_state == 1)
         return replay();
-    if (m->graph_state == -1)
-        return forward_eager(m, true);
+    if (m->graph_state == -1) {
+        const bool alone = m->drained;
+        m->drained = false;
+        return forward_eager(m, !alone);
+    }
     // ---- undecided: the first ten forwards (1: plain; 2, 3, 7, 8: timed plain launches; 4: the capture
     //      and its first replay; 5, 6, 9, 10: timed replays)
     // (schedules of fewer than 5 kernels stay eager without asking: the depthwise + pooling + addition
