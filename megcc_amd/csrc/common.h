@@ -92,8 +92,8 @@ void note_requant_affine(bool on);
 TinyNNStatus noalloc_scratch_setup();
 
 // conv_api.hip: a channel-wise 3x3 convolution and the pointwise convolution of its result as one kernel
-// (model runtime only). CHECK: whether the kernel takes the pair; PREPARE: everything a launch needs is in the pair's block,
-// which belongs to the caller and keeps the kernel's arguments on the device from one launch to the next.
+// (model runtime only). CHECK: whether the kernel takes the pair; PREPARE, once: everything a launch on these operands needs is
+// in the pair's block, which belongs to the caller and keeps the kernel's arguments on the device; RUN: the launch, nothing else.
 struct DwPwBlock;
 DwPwBlock* dw_pw_block_create();
 void dw_pw_block_destroy(DwPwBlock* block);

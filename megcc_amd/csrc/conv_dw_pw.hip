@@ -76,7 +76,7 @@ struct DwPwParams {
     };
     RequantTable dtable, ptable;
 };
-static_assert(sizeof(DwPwArgs) <= 256, "four lines");
+static_assert(sizeof(DwPwArgs) <= 256 && sizeof(DwPwParams) % 64 == 0, "four lines");
 
 // All of the arguments in one round trip: the compiler otherwise asks for each where it is used, and nine round trips one
 // after the other stood in front of the first load (3300 of a workgroup's 22000 cycles at 512 channels; 0.9 us of a launch).
@@ -96,11 +96,19 @@ __device__ __forceinline__ DwPwArgs dp_args(const DwPwParams* p) {
 #endif
 }
 
-// what is kept of a pair between launches: the arguments on the device, and what they were written from
+// What is kept of a pair from one launch to the next: how it is launched, and its arguments on the device - both forms that the
+// requantisation's switch chooses between, written once and never again: whatever is launched, captured or replayed
+// later, on whichever stream, finds them as they were.
+typedef void (*DwPwKernel)(const DwPwParams*);
+struct DpLaunch {
+    DwPwKernel kern;
+    size_t lds;
+    unsigned workgroups;
+};
 struct DwPwBlock {
-    void* dev = nullptr;
-    bool valid = false;
-    DwPwParams host;
+    DwPwParams* dev = nullptr;  // [2]: by the proven multiply-adds where there are any, by the tables
+    DwPwParams host[2];
+    DpLaunch launch;
 };
 #ifndef MG_HOST_AUDIT
 DwPwBlock* dw_pw_block_create() {
@@ -111,24 +119,18 @@ void dw_pw_block_destroy(DwPwBlock* b) {
         megcc_gfx950_free(b->dev);
     delete b;
 }
-static TinyNNStatus dp_upload(DwPwBlock* b, const DwPwParams& all) {
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    MG_REQUIRE(hipStreamIsCapturing(stream(), &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone, TinyNN_ERROR_RUNTIME,
-               "conv_dw_pw: other arguments under a capture");
-    b->valid = false;
-    if (!b->dev)
-        b->dev = megcc_gfx950_malloc(sizeof(all));
-    MG_REQUIRE(b->dev, TinyNN_ERROR_MEMORY_MALLOC, "conv_dw_pw: arguments");
-    // (launches that read what was there are over, and this copy is, before anything else reads it on whichever stream)
-    TinyNNStatus st = megcc_gfx950_wait();
-    if (st == TinyNN_SUCCESS)
-        st = megcc_gfx950_memcpy_h2d(b->dev, &all, sizeof(all));
+static TinyNNStatus dp_upload(DwPwBlock* b) {
+    DwPwParams* const dev = (DwPwParams*)megcc_gfx950_malloc(sizeof(b->host));
+    MG_REQUIRE(dev, TinyNN_ERROR_MEMORY_MALLOC, "conv_dw_pw: arguments");
+    // (the copy is over before anything reads it, on whichever stream)
+    TinyNNStatus st = megcc_gfx950_memcpy_h2d(dev, b->host, sizeof(b->host));
+    if (st == TinyNN_SUCCESS && hipStreamSynchronize(stream()) != hipSuccess)
+        st = fail(TinyNN_ERROR_RUNTIME, "conv_dw_pw: arguments");
     if (st != TinyNN_SUCCESS)
-        return st;
-    MG_REQUIRE(hipStreamSynchronize(stream()) == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_dw_pw: arguments");
-    b->host = all;
-    b->valid = true;
-    return TinyNN_SUCCESS;
+        megcc_gfx950_free(dev);
+    else
+        b->dev = dev;
+    return st;
 }
 #endif
 
@@ -649,10 +651,10 @@ static int dp_resident(const void* kern, size_t lds) {
     return cache[kern] = n;
 }
 
-TinyNNStatus conv_dw_pw_launch(
+// `affine`: with the proven multiply-adds, where there are any
+static TinyNNStatus dp_plan(
         const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dflt, const void* dbias, const void* packed,
-        const void* pbias, void* dst, DwPwBlock* block, bool prepare_only) {
-    DwPwParams all;
+        const void* pbias, void* dst, bool affine, DwPwParams& all, DpLaunch& l) {
     memset(all.words, 0, sizeof(all.words));
     DwPwArgs& q = all.a;
     DpShape s;
@@ -677,8 +679,10 @@ TinyNNStatus conv_dw_pw_launch(
     q.d_xg = make_fastdiv(q.xg);
     q.d_oh = make_fastdiv(q.oh);
     q.d_slices = make_fastdiv(q.slices);
-    q.dq = requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
-    q.pq = requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
+    if (affine) {
+        q.dq = requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
+        q.pq = requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
+    }
     q.dc = make_requant_fast(dw.s_src, dw.s_flt, dw.s_dst).c;
     q.pc = make_requant_fast(pw.s_src, pw.s_flt, pw.s_dst).c;
     if (q.dq.mode == 0)
@@ -686,7 +690,7 @@ TinyNNStatus conv_dw_pw_launch(
     if (q.pq.mode == 0)
         all.ptable = *requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
     const int rag = dw.iw & 3;
-    void (*kern)(const DwPwParams*) = nullptr;
+    DwPwKernel kern = nullptr;
     size_t lds = 0;
 #define MG_DP(KC_, SUB_, MT_, NT_)                                                                               \
     if (s.kc == KC_ && s.mt == MT_ && s.nt == NT_) {                                                                   \
@@ -721,24 +725,40 @@ TinyNNStatus conv_dw_pw_launch(
     q.xcd_runs = (int)runs / q.xcds;
     q.per_xcd = runs * q.slices % 8 == 0 ? (int)runs * q.slices / 8 : 0;
     q.run_q = q.xcd_q / q.xcd_runs, q.run_r = q.xcd_q - q.run_q * q.xcd_runs;
+    l = {kern, lds, (unsigned)(runs * q.slices)};
+    return TinyNN_SUCCESS;
+}
+
+TinyNNStatus conv_dw_pw_launch(
+        const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dflt, const void* dbias, const void* packed,
+        const void* pbias, void* dst, DwPwBlock* block, bool prepare) {
+    const bool affine = !options().no_affine;
 #ifdef MG_HOST_AUDIT
-    const DwPwParams* const args = &all;
+    DwPwBlock here;
+    block = &here;
+    TinyNNStatus st = dp_plan(dw, pw, src, dflt, dbias, packed, pbias, dst, affine, here.host[!affine], here.launch);
+    if (st != TinyNN_SUCCESS)
+        return st;
+    const DwPwParams* const args = &here.host[!affine];
 #else
-    // the copy on the device is written when the arguments are others than the last time
-    const auto table_differs = [](int mode, const RequantTable& x, const RequantTable& y) { return mode == 0 && memcmp(&x, &y, sizeof(x)) != 0; };
-    if (!block->valid || memcmp(block->host.words, all.words, sizeof(all.words)) != 0 || table_differs(q.dq.mode, block->host.dtable, all.dtable) ||
-        table_differs(q.pq.mode, block->host.ptable, all.ptable)) {
-        TinyNNStatus st = dp_upload(block, all);
-        if (st != TinyNN_SUCCESS)
-            return st;
+    if (prepare) {
+        MG_REQUIRE(!block->dev, TinyNN_ERROR_RUNTIME, "conv_dw_pw: prepared before");
+        for (int i = 0; i < 2; ++i) {
+            TinyNNStatus st = dp_plan(dw, pw, src, dflt, dbias, packed, pbias, dst, i == 0, block->host[i], block->launch);
+            if (st != TinyNN_SUCCESS)
+                return st;
+        }
+        return dp_upload(block);
     }
-    if (prepare_only)
-        return TinyNN_SUCCESS;
-    const DwPwParams* const args = (const DwPwParams*)block->dev;
+    MG_REQUIRE(block->dev, TinyNN_ERROR_RUNTIME, "conv_dw_pw: not prepared");
+    const DwPwParams* const args = block->dev + !affine;
 #endif
+    const DwPwArgs& q = block->host[!affine].a;
+    MG_REQUIRE(q.src == src && q.dflt == dflt && q.dbias == dbias && q.wp == packed && q.pbias == pbias && q.dst == dst,
+               TinyNN_ERROR_RUNTIME, "conv_dw_pw: not the operands it was prepared for");
     note_kernel("conv_dw_pw", dw.ic / 32, dw.sh, q.slices);
     note_requant_affine(q.dq.mode != 0 && q.pq.mode != 0);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(runs * q.slices)), dim3(DP_THREADS), lds, stream(), args);
+    hipLaunchKernelGGL(block->launch.kern, dim3(block->launch.workgroups), dim3(DP_THREADS), block->launch.lds, stream(), args);
     return check_launch("conv_dw_pw");
 }
 

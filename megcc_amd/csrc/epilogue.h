@@ -244,6 +244,7 @@ struct RequantPack {
     float s1, s2, c, d;
     int mode;
 };
+// (whatever the switch "noaffine" says: the caller asks it)
 RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst);
 
 // MODE, ACT compile-time; channels (or pixels) 0..3 of one dword

@@ -474,8 +474,11 @@ static void build_schedule(Model* m, Pairs allow) {
                 bool take = !shares_bytes(*f->in_ptrs[0], *f->out_ptrs[0]) &&
                             dw_pw_run(&f->desc.attr.pw_dw, f->in_ptrs.data(), (int)f->in_ptrs.size(), f->out_ptrs.data(),
                                       (int)f->out_ptrs.size(), nullptr, DwPw::CHECK) == TinyNN_SUCCESS;
-                if (take)
+                if (take) {
                     f->block = dw_pw_block_create();
+                    take = dw_pw_run(&f->desc.attr.pw_dw, f->in_ptrs.data(), (int)f->in_ptrs.size(), f->out_ptrs.data(),
+                                     (int)f->out_ptrs.size(), f->block, DwPw::PREPARE) == TinyNN_SUCCESS;
+                }
                 if (take && !options().fuse_dwpw)
                     take = faster_as_one(m, m->dw_pw_time, i, f, {o0, o1});
                 if (take) {
@@ -1267,14 +1270,6 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
             setup_tail(m, best_tb);
         }
     }
-    // (what the first forward would otherwise wait for)
-    for (ModelOpr* o : m->schedule)
-        if (o->dw_pw) {
-            placed = dw_pw_run(&o->desc.attr.pw_dw, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(), (int)o->out_ptrs.size(),
-                               o->block, DwPw::PREPARE);
-            if (placed != TinyNN_SUCCESS)
-                return placed;
-        }
     m->finalized = true;
     return megcc_gfx950_wait();
 }

@@ -251,8 +251,7 @@ static int pack_eval(int a, int act, const RequantPack& q) {
 RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
     static ScaleCache<RequantPack> cache;
     const RequantPack none = {0.f, 0.f, 0.f, 0.f, 0};
-    if ((act != MEGCC_NONLINE_IDENTITY && act != MEGCC_NONLINE_RELU) || !requant_table_ok(s_src, s_flt, s_dst) ||
-        options().no_affine)
+    if ((act != MEGCC_NONLINE_IDENTITY && act != MEGCC_NONLINE_RELU) || !requant_table_ok(s_src, s_flt, s_dst))
         return none;
     const auto key = cache.key(act, s_src, s_flt, s_dst);
     RequantPack found = none;

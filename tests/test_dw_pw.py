@@ -150,3 +150,32 @@ def test_the_tensor_inside_a_pair_is_planned_for_operators_run_one_by_one(switch
             m.run_opr(k)
             assert np.array_equal(m.get(ids[k + 1]), want[k + 1]), k
     m.close()
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_the_requantisation_is_switched_between_forwards(graph):
+    """the switch "noaffine" changes what a pair is launched with: at the forward that is captured, between replays and
+    between plain launches, every forward runs and gives the oracle's result"""
+    m, ids, want, _ = _block(64, 64, pairs=4)
+    runtime.set_option("fusedwpw", 1)
+    try:
+        m.finalize()
+    finally:
+        runtime.set_option("fusedwpw", 0)
+    assert m.nr_kernel == 5  # (the fewest a forward is captured with)
+    m.set_input(ids[0], want[0])
+    runtime.set_option("no_graph", int(not graph))
+    try:
+        for k in range(1, 15):
+            runtime.set_option("noaffine", int(k in (1, 4, 6, 7, 11, 13)))
+            m.forward()
+            # (a replayed graph launches nothing of its own; the pair's layers have multiply-adds for these scales)
+            if not graph:
+                assert runtime.last_kernel().endswith("+affine") == (k not in (1, 4, 6, 7, 11, 13)), k
+            if k != 2:  # (forwards 2 and 3 are timed as a pair, one behind the other)
+                assert np.array_equal(m.get(ids[-1]), want[-1]), k
+        assert m.launch_mode()[0] == -1 or (graph and m.launch_mode()[0] == 1)
+    finally:
+        runtime.set_option("noaffine", 0)
+        runtime.set_option("no_graph", 0)
+    m.close()
