@@ -651,11 +651,8 @@ static void setup_tail(Model* m, int forced = -1) {
         }
         m->schedule_us = total;
         // A network whose kernels average under 4 us is nothing but launches: what a second stream
-        // could overlap, the host does not enqueue in time. One stream. (Between 4 and 6 us the device
-        // is as busy as the host. MobileNetV1, one stream / two, us for each of many forwards: batch 1
-        // 100 / 96, 2 106 / 98, 4 116 / 101, 8 120 / 102; a forward whose result is waited for before
-        // the next one runs on one stream: Model::drained. Finding the boundary takes 14 ms, once for
-        // each shape.)
+        // could overlap, the host does not enqueue in time (12 FullyConnected layers of 3.6 us: 47 us on one stream, 57
+        // on two). One stream; from there settle_tail() decides.
         if (total < 4.0 * n)
             return;
         double tail = 0;
@@ -768,9 +765,9 @@ static TinyNNStatus forward_eager(Model* m, bool overlap = false, hipEvent_t don
 }
 
 // Milliseconds per forward of eight plain-launch forwards enqueued back to back, the way a finalized
-// model runs them (two streams where the schedule has a tail) - the shortest of `reps` such runs;
+// model runs them (two streams where the schedule has a tail; `overlap` false: one) - the shortest of `reps` such runs;
 // negative when something fails.
-static float time_forwards(Model* m, int reps = 2) {
+static float time_forwards(Model* m, int reps = 2, bool overlap = true) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
         if (e0)
@@ -784,7 +781,7 @@ static float time_forwards(Model* m, int reps = 2) {
         join_tail(m);
         ok = hipEventRecord(e0, main_stream()) == hipSuccess;
         for (int i = 0; ok && i < 8; ++i)
-            ok = forward_eager(m, true) == TinyNN_SUCCESS;
+            ok = forward_eager(m, overlap) == TinyNN_SUCCESS;
         join_tail(m);
         ok = ok && hipEventRecord(e1, main_stream()) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
              hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
@@ -863,6 +860,45 @@ static Choice choose_schedule(Model* m) {
     if (tail_begin >= 0)
         setup_tail(m, tail_begin);
     return {best, m->tail_begin};
+}
+
+// Where the second stream takes over, by whole forwards, and whether it does.
+// The balance of measured kernel times is only a starting point: one kernel more or less on the tail moves MobileNetV1 batch 64 by
+// 3 %. The boundary and its three neighbours on either side are timed and the best one kept.
+// A launch on alternating streams costs the host about twice as much, so two streams win where the device takes longer than
+// that: always from kernels of 6 us on average, by no rule on the average below, where the best boundary is compared with one
+// stream. us a forward, one / two: MobileNetV1 (5.3 - 5.7 us a kernel) batch 1 97 / 79, 4 111 / 90, 8 116 / 92; 27 operators of a
+// residual network, 64 channels at 56 x 56 to 512 at 7 x 7, batch 1 (4.6) 128 / 140, 4 (5.1) 142 / 145, 8 (5.8) 161 / 147; 16 layers
+// 64 -> 64 28 x 28 batch 4 (5.1) 80 / 90, 16 (6.0) 98 / 92; 12 f32 layers 32 -> 32 56 x 56 batch 1 (4.8) 57 / 63, 2 (6.1) 77 / 73;
+// channel-wise and pointwise layers, 16 - 256 channels from 80 x 80, batch 16 (5.0) 68 / 74. Eight forwards of each, as
+// time_forwards takes, said so for all of them (the residual network at batch 1: 123 / 147).
+static void settle_tail(Model* m) {
+    const bool ask = m->schedule_us < 6.0 * (double)m->schedule.size();
+    const float one = ask ? time_forwards(m, 2, false) : -1.f;
+    const int tb0 = m->tail_begin;
+    int best_tb = tb0;
+    float best = time_forwards(m);
+    if (ask && one > 0.f && (best <= 0.f || best > 1.1f * one)) {  // (no boundary made up for that)
+        reset_tail(m);
+        return;
+    }
+    for (int cand : {tb0 + 1, tb0 - 1, tb0 + 2, tb0 - 2, tb0 + 3, tb0 - 3}) {
+        reset_tail(m);
+        setup_tail(m, cand);
+        if (m->tail_begin != cand)
+            continue;
+        const float t = time_forwards(m);
+        if (t > 0.f && (best <= 0.f || t < best)) {
+            best = t;
+            best_tb = cand;
+        }
+    }
+    if (m->tail_begin != best_tb) {
+        reset_tail(m);
+        setup_tail(m, best_tb);
+    }
+    if (ask && one > 0.f && one <= best)
+        reset_tail(m);
 }
 
 // Memory for the arena as planned, and everybody's place in it.
@@ -1247,29 +1283,8 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
     placed = plan_again(m, choose_schedule(m));
     if (placed != TinyNN_SUCCESS)
         return placed;
-    // The balance of measured kernel times is only a starting point: one kernel more or less on the
-    // tail moves MobileNetV1 batch 64 by 3 %. The boundary and its three neighbours on either side are
-    // timed as whole forwards and the best one kept.
-    if (m->tail_begin >= 0) {
-        const int tb0 = m->tail_begin;
-        int best_tb = tb0;
-        float best = time_forwards(m);
-        for (int cand : {tb0 + 1, tb0 - 1, tb0 + 2, tb0 - 2, tb0 + 3, tb0 - 3}) {
-            reset_tail(m);
-            setup_tail(m, cand);
-            if (m->tail_begin != cand)
-                continue;
-            const float t = time_forwards(m);
-            if (t > 0.f && (best <= 0.f || t < best)) {
-                best = t;
-                best_tb = cand;
-            }
-        }
-        if (m->tail_begin != best_tb) {
-            reset_tail(m);
-            setup_tail(m, best_tb);
-        }
-    }
+    if (m->tail_begin >= 0)
+        settle_tail(m);
     m->finalized = true;
     return megcc_gfx950_wait();
 }
