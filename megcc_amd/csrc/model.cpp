@@ -866,38 +866,44 @@ static Choice choose_schedule(Model* m) {
 // The balance of measured kernel times is only a starting point: one kernel more or less on the tail moves MobileNetV1 batch 64 by
 // 3 %. The boundary and its three neighbours on either side are timed and the best one kept.
 // A launch on alternating streams costs the host about twice as much, so two streams win where the device takes longer than
-// that: always from kernels of 6 us on average, by no rule on the average below, where the best boundary is compared with one
-// stream. us a forward, one / two: MobileNetV1 (5.3 - 5.7 us a kernel) batch 1 97 / 79, 4 111 / 90, 8 116 / 92; 27 operators of a
-// residual network, 64 channels at 56 x 56 to 512 at 7 x 7, batch 1 (4.6) 128 / 140, 4 (5.1) 142 / 145, 8 (5.8) 161 / 147; 16 layers
-// 64 -> 64 28 x 28 batch 4 (5.1) 80 / 90, 16 (6.0) 98 / 92; 12 f32 layers 32 -> 32 56 x 56 batch 1 (4.8) 57 / 63, 2 (6.1) 77 / 73;
-// channel-wise and pointwise layers, 16 - 256 channels from 80 x 80, batch 16 (5.0) 68 / 74. Eight forwards of each, as
-// time_forwards takes, said so for all of them (the residual network at batch 1: 123 / 147).
+// that: always from kernels of 6 us on average, by no rule on the average below, where eight forwards on two streams, as
+// time_forwards takes them, are compared with eight on one (not with the sum of the kernels' times: each behind itself finds its
+// operands in the caches, 98 us for the 111 of MobileNetV1 batch 4). us a forward, one stream / two:
+// MobileNetV1 (5.3 - 5.7 us a kernel) batch 1 97 / 79, 4 111 / 90, 8 116 / 92; 27 operators of a residual network, 64 channels at
+// 56 x 56 to 512 at 7 x 7, batch 1 (4.6) 128 / 140, 4 (5.1) 142 / 145, 8 (5.8) 161 / 147; 16 layers 64 -> 64 28 x 28 batch 4 (5.1)
+// 80 / 90, 16 (6.0) 98 / 92; 12 f32 layers 32 -> 32 56 x 56 batch 1 (4.8) 57 / 63, 2 (6.1) 77 / 73; channel-wise and pointwise
+// layers, 16 - 256 channels from 80 x 80, batch 16 (5.0) 68 / 74. The comparison said so for all of them (residual, batch 1:
+// 123 / 147), and the best boundary had the balanced one's tail or a shorter one: launches there are the dear ones. So only
+// those are tried below 6 us, as long as they gain (a network whose results are read one by one runs on one stream anyway:
+// loading MobileNetV1 batch 1 took 14 ms for the seven boundaries).
 static void settle_tail(Model* m) {
     const bool ask = m->schedule_us < 6.0 * (double)m->schedule.size();
-    const float one = ask ? time_forwards(m, 2, false) : -1.f;
+    const float one = ask ? time_forwards(m, 1, false) : 1e30f;
     const int tb0 = m->tail_begin;
     int best_tb = tb0;
     float best = time_forwards(m);
-    if (ask && one > 0.f && (best <= 0.f || best > 1.1f * one)) {  // (no boundary made up for that)
+    if (one > 0.f && best > 1.1f * one) {  // (no boundary makes up for that)
         reset_tail(m);
         return;
     }
     for (int cand : {tb0 + 1, tb0 - 1, tb0 + 2, tb0 - 2, tb0 + 3, tb0 - 3}) {
+        if (ask && cand < tb0)
+            continue;
         reset_tail(m);
         setup_tail(m, cand);
-        if (m->tail_begin != cand)
-            continue;
-        const float t = time_forwards(m);
+        const float t = m->tail_begin == cand ? time_forwards(m) : -1.f;
         if (t > 0.f && (best <= 0.f || t < best)) {
             best = t;
             best_tb = cand;
+        } else if (ask) {
+            break;
         }
     }
     if (m->tail_begin != best_tb) {
         reset_tail(m);
         setup_tail(m, best_tb);
     }
-    if (ask && one > 0.f && one <= best)
+    if (one > 0.f && best >= one)
         reset_tail(m);
 }
 

@@ -265,3 +265,36 @@ def test_two_streams_only_where_forwards_gain():
     assert best[model] <= 1.07 * best[serial]
     model.close()
     serial.close()
+
+
+def test_loading_a_small_network_costs_few_forwards():
+    """what finalize tries on a network of 5 us kernels takes less time than 130 of its forwards (seven boundaries between
+    the streams: 160)"""
+    import time
+    net = mobilenet.Net(1)
+    lengths = []
+
+    class Timed(runtime.Model):
+        def finalize(self):
+            t = time.perf_counter()
+            super().finalize()
+            lengths.append(time.perf_counter() - t)
+
+    for _ in range(5):  # (the first one loads the kernels)
+        model, ids = net.build_gpu(model=Timed())
+        model.set_input(ids["image"], mobilenet.draw_input(1, seed=1))
+        for _ in range(20):
+            model.forward()
+        if len(lengths) < 5:
+            model.close()
+    forward = 1e9
+    for _ in range(5):
+        runtime.wait()
+        t = time.perf_counter()
+        for _ in range(20):
+            model.forward()
+            runtime.wait()
+        forward = min(forward, (time.perf_counter() - t) / 20)
+    print("finalize ms", [round(1e3 * v, 1) for v in lengths], "forward us", 1e6 * forward)
+    assert min(lengths[1:]) <= 130 * forward
+    model.close()
