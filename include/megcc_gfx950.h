@@ -692,6 +692,9 @@ TinyNNStatus megcc_gfx950_model_forward(void* model);
 TinyNNStatus megcc_gfx950_model_join(void* model);
 /* how many of megcc_gfx950_model_nr_kernel's kernels those last operators are (0: none) */
 int megcc_gfx950_model_nr_tail_kernel(void* model);
+/* and how many of the last forward's went there: none behind a wait (a blocking read, or
+ * megcc_gfx950_wait() since the forward before it), where there is nothing to overlap */
+int megcc_gfx950_model_launched_tail_kernel(void* model);
 /* Bytes of one forward when each of its nr_kernel kernels reads its operands and writes its results
  * once; what a bandwidth roofline of the forward is priced against. */
 size_t megcc_gfx950_model_forward_bytes(void* model);

@@ -19,6 +19,12 @@ void set_stream_override(hipStream_t s, bool on);
 void register_aux_stream(hipStream_t s);
 void unregister_aux_stream(hipStream_t s);
 
+// How often the host has waited for the library stream, and for that and all of the streams above.
+struct HostWaits {
+    unsigned long library, all;
+};
+HostWaits host_waits();
+
 // Compute units of the current device (256 when the query fails).
 int num_cus();
 

@@ -6,6 +6,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -78,6 +79,12 @@ void note_requant_affine(bool on) {
 static thread_local hipStream_t g_stream_override = nullptr;
 static thread_local bool g_stream_override_on = false;
 static std::mutex g_aux_lock;
+static std::atomic<unsigned long> g_library_waits, g_all_waits;
+
+HostWaits host_waits() {
+    return {g_library_waits.load(), g_all_waits.load()};
+}
+
 static std::vector<hipStream_t> g_aux_streams;
 
 hipStream_t main_stream() {
@@ -205,6 +212,7 @@ TinyNNStatus megcc_gfx950_memcpy_d2h(void* dst, const void* src, size_t length) 
     if (e == hipSuccess)
         e = hipStreamSynchronize(stream());
     MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "memcpy_d2h: %s", hipGetErrorString(e));
+    ++g_library_waits;
     return TinyNN_SUCCESS;
 }
 
@@ -228,6 +236,8 @@ TinyNNStatus megcc_gfx950_wait(void) {
         e = hipStreamSynchronize(s);
         MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "wait: %s", hipGetErrorString(e));
     }
+    ++g_library_waits;
+    ++g_all_waits;
     return TinyNN_SUCCESS;
 }
 

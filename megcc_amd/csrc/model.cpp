@@ -116,10 +116,13 @@ struct Model {
     hipStream_t tail_stream = nullptr;
     hipEvent_t ev_head = nullptr, ev_tail = nullptr;
     bool tail_pending = false, tail_reads_input = false;
-    // The caller has waited for a result since the last forward: nothing is left that the next one's head could overlap, and
-    // on one stream it is over sooner, with no event between head and tail (batch 1, image in, forward, result out, us: 184 -
-    // 187 and unsteady on two, 171 - 173 on one).
-    bool drained = false;
+    // The host's waits when the last forward had been launched (the library stream's: when it had been ordered behind that forward).
+    // Where the host has waited since, by whichever call - a blocking read, megcc_gfx950_wait() after a forward or an asynchronous
+    // read -, nothing is left that the next forward's head could overlap, and on one stream it is over sooner, with no event
+    // between head and tail (MobileNetV1, each forward waited for, us on two streams / one: batch 1 123 / 108, 4 139 / 122, 8 145 /
+    // 128; with image in and result out, batch 1: 184 - 187 and unsteady / 171 - 173).
+    HostWaits waits = {0, 0};
+    int launched_tail = 0;  // entries of the last forward that went to the tail stream
     std::vector<char> waits_tail;
     std::vector<const Tensor*> tail_writes;  // tensors the tail's operators write
     void* tail_workspace = nullptr;
@@ -706,7 +709,16 @@ static void join_tail(Model* m) {
     if (m->tail_pending) {
         (void)hipStreamWaitEvent(main_stream(), m->ev_tail, 0);
         m->tail_pending = false;
+        const HostWaits now = host_waits();
+        if (now.all == m->waits.all)  // (else the host has waited for the tail already)
+            m->waits.library = now.library;
     }
+}
+
+// Whether the host has waited for all of the last forward (see Model::waits).
+static bool drained(const Model* m) {
+    const HostWaits now = host_waits();
+    return m->tail_pending ? now.all != m->waits.all : now.library != m->waits.library;
 }
 
 // Undoes setup_tail (the schedule is about to be rebuilt).
@@ -761,6 +773,8 @@ static TinyNNStatus forward_eager(Model* m, bool overlap = false, hipEvent_t don
     }
     if (done)
         (void)hipEventRecord(done, tb >= 0 ? m->tail_stream : main_stream());
+    m->launched_tail = tb >= 0 ? (int)m->schedule.size() - tb : 0;
+    m->waits = host_waits();
     return st;
 }
 
@@ -1371,9 +1385,7 @@ TinyNNStatus megcc_gfx950_model_get_output(void* model, int tensor, void* host, 
     MG_REQUIRE(bytes == tensor_bytes(t), TinyNN_ERROR_INVALID_LAYOUT,
                "model_get_output: %zu bytes asked, tensor has %zu", bytes, tensor_bytes(t));
     join_tail(m);
-    const TinyNNStatus st = megcc_gfx950_memcpy_d2h(host, t.ptr, bytes);
-    m->drained = st == TinyNN_SUCCESS;
-    return st;
+    return megcc_gfx950_memcpy_d2h(host, t.ptr, bytes);
 }
 
 // The copy is enqueued behind the forward that produced the tensor - on the tail stream when the last
@@ -1405,17 +1417,15 @@ TinyNNStatus megcc_gfx950_model_forward(void* model) {
     ++m->forwards;
     auto replay = [&]() -> TinyNNStatus {
         join_tail(m);  // (a plain-launch forward before this one may have left its tail on the second stream)
+        m->launched_tail = 0;
         hipError_t e = hipGraphLaunch(m->graph_exec, stream());
         MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "model_forward: graph launch: %s", hipGetErrorString(e));
         return TinyNN_SUCCESS;
     };
     if (m->graph_state == 1)
         return replay();
-    if (m->graph_state == -1) {
-        const bool alone = m->drained;
-        m->drained = false;
-        return forward_eager(m, !alone);
-    }
+    if (m->graph_state == -1)
+        return forward_eager(m, !drained(m));
     // ---- undecided: the first ten forwards (1: plain; 2, 3, 7, 8: timed plain launches; 4: the capture
     //      and its first replay; 5, 6, 9, 10: timed replays)
     // (schedules of fewer than 5 kernels stay eager without asking: the depthwise + pooling + addition
@@ -1506,6 +1516,12 @@ size_t megcc_gfx950_model_forward_bytes(void* model) {
 int megcc_gfx950_model_nr_tail_kernel(void* model) {
     Model* m = (Model*)model;
     return m && m->finalized && m->tail_begin >= 0 ? (int)m->schedule.size() - m->tail_begin : 0;
+}
+
+// ... and of the last forward, those that did.
+int megcc_gfx950_model_launched_tail_kernel(void* model) {
+    Model* m = (Model*)model;
+    return m && m->finalized ? m->launched_tail : 0;
 }
 
 // Orders the library stream behind everything the model's forwards have launched (the last

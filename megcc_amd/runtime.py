@@ -117,7 +117,7 @@ EXPORTS = [
     "megcc_gfx950_model_mark_io", "megcc_gfx950_model_finalize", "megcc_gfx950_model_arena_bytes",
     "megcc_gfx950_model_set_plan", "megcc_gfx950_model_nr_kernel", "megcc_gfx950_model_launch_mode",
     "megcc_gfx950_model_tensor_ptr", "megcc_gfx950_model_set_input",
-    "megcc_gfx950_model_get_output", "megcc_gfx950_model_forward", "megcc_gfx950_model_join", "megcc_gfx950_model_nr_tail_kernel", "megcc_gfx950_model_forward_bytes", "megcc_gfx950_model_get_output_async", "megcc_gfx950_model_nr_opr",
+    "megcc_gfx950_model_get_output", "megcc_gfx950_model_forward", "megcc_gfx950_model_join", "megcc_gfx950_model_nr_tail_kernel", "megcc_gfx950_model_launched_tail_kernel", "megcc_gfx950_model_forward_bytes", "megcc_gfx950_model_get_output_async", "megcc_gfx950_model_nr_opr",
     "megcc_gfx950_model_run_opr", "megcc_gfx950_plan_memory", "megcc_gfx950_model_load",
     "megcc_gfx950_tiny_describe",
 ]
@@ -412,6 +412,13 @@ class Model:
         L = lib()
         L.megcc_gfx950_model_nr_tail_kernel.argtypes = [C.c_void_p]
         return L.megcc_gfx950_model_nr_tail_kernel(self.h)
+
+    @property
+    def launched_tail_kernel(self):
+        """how many of the last forward's kernels went to the second stream (none behind a wait)"""
+        L = lib()
+        L.megcc_gfx950_model_launched_tail_kernel.argtypes = [C.c_void_p]
+        return L.megcc_gfx950_model_launched_tail_kernel(self.h)
 
     @property
     def forward_bytes(self):

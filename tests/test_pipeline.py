@@ -197,6 +197,69 @@ def test_two_hundred_overlapped_forwards(planned):
     serial.close()
 
 
+def test_a_forward_behind_a_wait_runs_on_one_stream():
+    """whichever way the host has waited for the last forward - a blocking read, wait() after it, an asynchronous read and
+    wait(), wait() and join() in either order with the next input in between -, the next one finds nothing to overlap; without a
+    wait it uses the second stream. Every result is the one of its input"""
+    net = mobilenet.Net(BATCH)
+    images = [mobilenet.draw_input(BATCH, seed=s) for s in (31, 32, 33)]
+    pipe, ids = build(net, False, no_graph=1)
+    serial, _ = build(net, False, no_graph=1, nopipeline=1)
+    tail = pipe.nr_tail_kernel
+    assert tail >= 2
+    want = []
+    for img in images:
+        serial.set_input(ids["image"], img)
+        serial.forward()
+        want.append(serial.get(ids["softmax"]).copy())
+    out = np.zeros((BATCH, 1000), np.float32)
+    runtime.set_option("no_graph", 1)  # (asked at the first forward: plain launches from then on)
+    try:
+        pipe.forward()
+        pipe.get(ids["softmax"])
+    finally:
+        runtime.set_option("no_graph", 0)
+    assert pipe.launch_mode()[0] == -1
+
+    def get():
+        np.testing.assert_array_equal(pipe.get(ids["softmax"]), want[at])
+
+    def get_async():
+        pipe.get_async(ids["softmax"], out)
+
+    def check():
+        np.testing.assert_array_equal(out, want[at])
+
+    ways = {  # what the caller does between two forwards: whether the second one's tail may overlap
+        "nothing": ([], False), "get": ([get], True), "wait": ([runtime.wait], True), "async, wait": ([get_async, runtime.wait, check], True),
+        "async": ([get_async], False), "join": ([pipe.join], False), "join, wait": ([pipe.join, runtime.wait], True),
+        "wait, join": ([runtime.wait, pipe.join], True), "get, async": ([get, get_async], True), "wait, get": ([runtime.wait, get], True),
+        # a read of another model waits for the library stream, on which this one's head is
+        "other's get": ([lambda: serial.get(ids["softmax"])], False), "join, other's get": ([pipe.join, lambda: serial.get(ids["softmax"])], True),
+    }
+    at, before = 0, None
+    for order in (list(ways), list(ways)[::-1], list(ways)[::2] * 2):
+        for name in order:
+            calls, waited = ways[name]
+            # two forwards in front, the second one on two streams unless the first one's caller has waited
+            at = (at + 1) % 3
+            pipe.set_input(ids["image"], images[at])
+            pipe.forward()
+            pipe.forward()
+            assert pipe.launched_tail_kernel == tail, (name, before)
+            for call in calls:
+                call()
+            pipe.forward()
+            assert pipe.launched_tail_kernel == (0 if waited else tail), (name, before)
+            at = (at + 1) % 3
+            pipe.set_input(ids["image"], images[at])
+            pipe.forward()
+            get()
+            before = name
+    pipe.close()
+    serial.close()
+
+
 def residual_net(n):
     """27 operators: four stages of two blocks (3x3, 3x3, addition), 64 channels at 56 x 56 to 512 at 7 x 7"""
     from cases import ConvCase, MultiTypeCase
