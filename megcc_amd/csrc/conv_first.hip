@@ -130,6 +130,7 @@ __global__ void __launch_bounds__(CF_THREADS) conv_first_q8_kernel(
 typedef int cfm_v4i __attribute__((ext_vector_type(4)));
 typedef int cfm_v2i __attribute__((ext_vector_type(2)));
 typedef int cfm_v16i __attribute__((ext_vector_type(16)));
+typedef uint32_t cfm_word __attribute__((aligned(1)));  // of a filter, which may begin at any byte
 
 struct ConvFirstMfmaParams {
     const int8_t* src;
@@ -182,7 +183,8 @@ __global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParam
         const bool ok = t < end && p < q.pairs;
         const int n = fdiv(p, q.dOHW2), rem = p - n * (q.OHW >> 1);
         const int oy = fdiv(rem, q.dOW2), m = rem - oy * q.OW2;
-        // the first pixels' left dword is padding: they load one dword further right and use the first one
+        // the first pixels' left dword is padding: they load one dword further right and use the first one (the other may be
+        // another row's, or beyond the images, where a buffer load reads nothing)
         r.first = m == 0;
         const int base = n * 3 * q.IH * q.IW + (2 * oy - 1) * q.IW + 4 * m - (r.first ? 0 : 4);
 #pragma unroll
@@ -197,7 +199,7 @@ __global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParam
     // ---- filter and bias once per workgroup: 15 single bytes and 16 biases a lane kept the address path busy for 3 us
     if (tid < OC / 4 * 9) {  // (channel group, pair): four channels' dwords (w0, w1, w2, 0)
         const int g4 = tid / 9, pair = tid - g4 * 9, ic = pair / 3, fh = pair - ic * 3;
-        const uint32_t* f = (const uint32_t*)q.flt + (g4 * 3 + fh) * 9 + ic;
+        const cfm_word* f = (const cfm_word*)q.flt + (g4 * 3 + fh) * 9 + ic;
         const uint32_t f0 = f[0], f1 = f[3], f2 = f[6];
         const uint32_t lo = __builtin_amdgcn_perm(f1, f0, 0x05010400u), hi = __builtin_amdgcn_perm(f1, f0, 0x07030602u);
         *(cfm_v4i*)(wlds + pair * OC + g4 * 4) = cfm_v4i{
@@ -268,9 +270,8 @@ __global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParam
     }
 }
 
-// (iw >= 8: the first pixels' 8 bytes are in their row)
-static bool conv_first_mfma_ok(const ConvGeom& g, const void* flt) {
-    return ((uintptr_t)flt & 3) == 0 && (g.oc == 32 || g.oc == 64) && g.iw >= 8 && (long)g.n * 3 * g.ih * g.iw < (1L << 31) &&
+static bool conv_first_mfma_ok(const ConvGeom& g) {
+    return (g.oc == 32 || g.oc == 64) && (long)g.n * 3 * g.ih * g.iw < (1L << 31) &&
            (long)g.n * g.oc * g.oh * g.ow < (1L << 31) && !options().no_firstmfma;
 }
 
@@ -338,7 +339,7 @@ TinyNNStatus conv_first_launch(
     const long pairs = (long)g.n * g.oh * (g.ow / 2);
     if (pairs == 0)
         return TinyNN_SUCCESS;
-    if (conv_first_mfma_ok(g, flt)) {
+    if (conv_first_mfma_ok(g)) {
         note_kernel("conv_first_mfma", g.oc / 32);
         return conv_first_mfma_launch(g, src, flt, bias, dst);
     }

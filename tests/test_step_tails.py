@@ -93,7 +93,7 @@ def test_slices_of_channel_wise_pointwise_pairs(cfg):
 
 # image widths from the smallest the kernel takes, one output row, steps of 64 pixels that end inside a row, inside an image and
 # behind the last one, one and two steps a wave; every form of the requantisation
-@pytest.mark.parametrize("n,ih,iw", [(1, 2, 8), (3, 2, 8), (1, 6, 12), (5, 10, 36), (2, 4, 132), (1, 34, 260), (30, 224, 224)])
+@pytest.mark.parametrize("n,ih,iw", [(1, 2, 4), (3, 2, 4), (50, 6, 4), (1, 2, 8), (3, 2, 8), (1, 6, 12), (5, 10, 36), (2, 4, 132), (1, 34, 260), (30, 224, 224)])
 @pytest.mark.parametrize("oc", [32, 64])
 @pytest.mark.parametrize("act,noaffine", [(A.RELU, 0), (A.IDENTITY, 0), (A.RELU, 1), (A.IDENTITY, 1), (A.H_SWISH, 0), (A.SIGMOID, 0)])
 def test_first_layer_steps(n, ih, iw, oc, act, noaffine):
@@ -108,4 +108,19 @@ def test_first_layer_steps(n, ih, iw, oc, act, noaffine):
         assert runtime.last_kernel().startswith("conv_first_mfma"), runtime.last_kernel()
     finally:
         runtime.set_option("noaffine", 0)
+    compare(got, case.run_port(arrays), repr(case))
+
+
+# a filter that begins at any byte, and the narrowest images with it
+@pytest.mark.parametrize("n,ih,iw", [(1, 2, 4), (5, 10, 36)])
+@pytest.mark.parametrize("oc", [32, 64])
+@pytest.mark.parametrize("at", [1, 2, 3])
+def test_first_layer_filters_off_a_dword(n, ih, iw, oc, at):
+    case = ConvCase(A.FMT_NCHW_NCHW44, A.DENSE, n, 3, ih, iw, oc, 3, 2, 1, A.RELU, scales=(0.02, 0.01, unsat(27)))
+    arrays = case.gen(seed=46)
+    ins, outs = case.specs(arrays)
+    ins[1].array = np.concatenate([np.full(at, 77, np.int8), arrays["flt"].ravel()])
+    ins[1].offset = at
+    got = runtime.run_symbol(case.symbol(), ins, outs)
+    assert runtime.last_kernel().startswith("conv_first_mfma"), runtime.last_kernel()
     compare(got, case.run_port(arrays), repr(case))
