@@ -70,12 +70,13 @@ struct KsParams {
 
 // The arguments as the first thing, in one round trip: asked for where they are used, two to five round trips one after
 // the other stood in front of the first load.
-template <bool CONV>
+template <bool CONV, bool STRIPS>
 __device__ __forceinline__ void ks_begin(const KsParams& q) {
 #ifndef MG_HOST_AUDIT
     asm volatile("" ::"s"(q.A), "s"(q.B), "s"(q.C), "s"(q.a_bytes), "s"(q.b_bytes), "s"(q.a_row), "s"(q.a_k), "s"(q.b_row), "s"(q.b_k), "s"(q.M),
-                 "s"(q.N), "s"(q.K), "s"(q.ldc), "s"(q.lw), "s"(q.tiles), "s"(q.per_xcd), "s"(q.strip_w), "s"(q.strips),
-                 "s"(q.d_strip.mul), "s"(q.d_w.mul), "s"(q.d_last.mul));
+                 "s"(q.N), "s"(q.K), "s"(q.ldc), "s"(q.lw));
+    if (STRIPS)
+        asm volatile("" ::"s"(q.tiles), "s"(q.per_xcd), "s"(q.strip_w), "s"(q.strips), "s"(q.d_strip.mul), "s"(q.d_w.mul), "s"(q.d_last.mul));
     if (CONV)
         asm volatile("" ::"s"(q.bias), "s"(q.act), "s"(q.ic), "s"(q.ih), "s"(q.iw), "s"(q.ow), "s"(q.ohw), "s"(q.fh), "s"(q.fw), "s"(q.sh), "s"(q.sw),
                      "s"(q.ph), "s"(q.pw), "s"(q.dh), "s"(q.dw), "s"(q.d_ohw.mul), "s"(q.d_ow.mul), "s"(q.d_taps.mul), "s"(q.d_fw.mul));
@@ -93,8 +94,16 @@ __device__ __forceinline__ float ks_act(int act, float x) {
 
 static constexpr int KS_MAX_WAVES = 8;
 static constexpr int KS_MAX_CONV_K = 4096;  // table entries (8 bytes each)
+static constexpr int KS_SHORT = 28;         // steps of a short K: up to seven for each of four waves
 
-template <int AM, int BMODE, int R, int MT, int NT, bool TAIL>
+// STRIPS: tiles in strips on the XCDs (ks_launch); else a grid of tiles.
+// SHORT: four waves of up to seven steps each, which never come to the loop that keeps the ring full and have no sums to close
+// (32 x 32: 155 registers for 236 with 64 x 64 outputs). In one instantiation with a number of waves from the arguments and the
+// strips' arithmetic, products of K under 230 had lost 2 - 6 % to the kernel before there were strips. us, that kernel, all in one, apart:
+// 2882 x 226 x 641 nt 17.3, 18.3, 17.1, 2000 x 200 x 900 tn 13.0, 13.4, 11.7, 637 x 117 x 1589 tn 6.9, 7.0, 6.0, 3118 x 140 x 293
+// 7.7, 7.8, 6.95, 2500 x 200 x 700 13.2, 13.4, 11.8; convolution 9 -> 101 77 x 77 N=2 10.8, 11.0, 9.8, 21 -> 69 26 x 30 N=13 9.5,
+// 9.6, 9.2. (The number of waves fixed for a long K too: the addresses of all its steps spilled, 1024^3 tn 56.4 us for 21.6.)
+template <int AM, int BMODE, int R, int MT, int NT, bool TAIL, bool STRIPS, bool SHORT>
 __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams q) {
     constexpr int RING = 4;  // (full >> (2 + lw) below)
     constexpr bool GATHER = BMODE == KS_CONV, CONV = GATHER || BMODE == KS_CONV1;
@@ -103,12 +112,12 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
     typedef typename KsTile<R>::Sums Sums;
     static_assert(!CONV || NT == 1, "one pixel per lane");
     extern __shared__ __attribute__((aligned(16))) float ks_lds[];
-    ks_begin<CONV>(q);
+    ks_begin<CONV, STRIPS>(q);
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lw = q.lw, W = 1 << lw;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lw = SHORT ? 2 : q.lw, W = 1 << lw;
     const int h = lane / R, c = lane & (R - 1);
     int tx = blockIdx.x, ty = blockIdx.y;
-    if (q.per_xcd) {
+    if constexpr (STRIPS) {
         const int place = (tx & 7) * q.per_xcd + (tx >> 3);
         if (place >= q.tiles)  // (the whole workgroup)
             return;
@@ -124,8 +133,12 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
     // Whole steps, dealt to the waves RING at a time where K is long - 4 steps are one 128-byte line of an
     // operand that is contiguous along K, fetched by one wave back to back instead of by four waves that
     // drift apart - and one at a time where that would leave waves without work.
+    // SHORT: a wave's steps follow one another too, as many for each wave; where both operands are contiguous along K that is
+    // twice the lines a wave comes back to, more than the L1 holds, and the waves take the steps of a line in turn (us in
+    // turn / one run: 2500 x 180 x 700 15.2 / 13.3, 1500 x 170 x 1500 16.3 / 15.1; nt 2882 x 226 x 641 17.1 / 18.9, 2500 x 224 x 700
+    // 14.7 / 14.3, 274 x 186 x 2814 8.9 / 9.1).
     const int full = q.K >> LKS;
-    const bool lines = full >= 4 * RING * W;
+    const bool lines = !SHORT && full >= 4 * RING * W;
     const int s_wave = lines ? RING : 1, s_ring = lines ? 1 : W;  // step = j0 * W + wave * s_wave + r * s_ring
     const int rounds = full >> (2 + lw), over = full - (rounds << (2 + lw));
     const int nj = lines ? rounds * RING + min(max(over - RING * wave, 0), RING)
@@ -264,8 +277,9 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
             for (int e = 0; e < 4; ++e)
                 at[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, (int)(aoff[i] + (unsigned)tail_k(e) * q.a_k), 0, 0));
     ks_v4f av[RING][MT], bv[RING][NT];
-    const int s0 = wave * s_wave;
-    auto step = [&](int j0, int r) { return min(j0 * W + s0 + r * s_ring, full - 1); };
+    constexpr bool RUN = SHORT && !(AM == KS_CONTIG && BMODE == KS_CONTIG);
+    const int s0 = RUN ? wave * (full >> 2) + min(wave, full & 3) : wave * s_wave;
+    auto step = [&](int j0, int r) { return min(RUN ? s0 + j0 + r : j0 * W + s0 + r * s_ring, full - 1); };
     if (nj > 0)
         static_for<RING>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
@@ -299,7 +313,7 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         // (whole groups with nothing under a condition: behind a conditional load the compiler has to assume
         //  fewer loads in flight than there are, and waits for more of them)
         int j0 = 0;
-        for (; j0 + 2 * RING <= nj; j0 += RING) {
+        for (; !SHORT && j0 + 2 * RING <= nj; j0 += RING) {
             static_for<RING>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
                 multiply(av[r], bv[r]);
@@ -351,7 +365,7 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int e = 0; e < SUMS; ++e)
-                ks_lds[wave * TILE + ((i * NT + j) * SUMS + e) * 64 + lane] = R == 16 ? sum[i][j][e] : acc[0][i][j][e] + sum[i][j][e];
+                ks_lds[wave * TILE + ((i * NT + j) * SUMS + e) * 64 + lane] = R == 16 ? sum[i][j][e] : SHORT ? acc[0][i][j][e] : acc[0][i][j][e] + sum[i][j][e];
     __syncthreads();
     // register e of a tile: row 8 * (e / 4) + 4 * h + e % 4 (16 x 16: 4 * h + e), column c. Wave w finishes registers w, w + W, ...
     for (int r = wave; r < MT * NT * SUMS; r += W) {
@@ -405,10 +419,12 @@ static KsPlan ks_plan(long M, long N, long K, bool a_contig, bool b_contig, bool
     // 200 5.6 / 3.6; convolution 64 -> 64 28 x 28 6.7 / 4.3). Two a CU are still one round (32 -> 32 56 x 56 4.9 / 4.2, 300 x 2000 x
     // 400 13.4 / 9.6), unless one row of 32 x 32 tiles is all there is and the other operand, beyond the L2s, would be read
     // twice (20 x 3000 x 4000 16.0 / 17.0); with more, the operands' way in costs more than the idle CUs (500^3 6.0 / 8.1, 8 -> 16 112 x 112 4.7 / 5.4).
+    // Eight waves where four would have more than seven steps each (16 x 312 x 1000 nt 3.7 us with four, 4.4 with eight, 4.0 with
+    // 32 x 32 tiles; 16 x 512 x 1000 nt 4.0, 4.0; convolution 64 -> 64 28 x 28 4.6, 4.4).
     const long small = ((M + 15) / 16) * ((N + 15) / 16);
     const bool one_row = ((M > 16 && M <= 32) || (N > 16 && N <= 32)) && K * (M > N ? M : N) > (1L << 22);
     if (small <= num_cus() || (small <= 2L * num_cus() && !one_row))
-        best = {16, 1, 1, small <= num_cus() && K >= 256 ? 8 : 4, (double)K * 4.75 * (small <= num_cus() ? 1.0 : 2.0) + 3000.0};
+        best = {16, 1, 1, small <= num_cus() && K >= 16 * (KS_SHORT + 1) ? 8 : 4, (double)K * 4.75 * (small <= num_cus() ? 1.0 : 2.0) + 3000.0};
     return best;
 }
 
@@ -428,15 +444,6 @@ template <int AM, int BMODE>
 static TinyNNStatus ks_launch(KsParams& q, const KsPlan& p, const char* what) {
     const bool tail = (q.K & (p.r == 32 ? 7 : 15)) != 0;
     constexpr bool CONV = BMODE == KS_CONV || BMODE == KS_CONV1;
-#define MG_KS_T(R_, MT_, NT_) (tail ? gemm_f32_ks_kernel<AM, BMODE, R_, MT_, NT_, true> : gemm_f32_ks_kernel<AM, BMODE, R_, MT_, NT_, false>)
-    void (*kern)(KsParams);
-    if (p.r == 16)
-        kern = MG_KS_T(16, 1, 1);
-    else if constexpr (CONV)  // (wider tiles never measured better for a convolution)
-        kern = MG_KS_T(32, 1, 1);
-    else
-        kern = p.mt == 1 ? (p.nt == 1 ? MG_KS_T(32, 1, 1) : MG_KS_T(32, 1, 2)) : (p.nt == 1 ? MG_KS_T(32, 2, 1) : MG_KS_T(32, 2, 2));
-#undef MG_KS_T
     const int tm = p.r * p.mt, tn = p.r * p.nt;
     const int gx = (q.N + tn - 1) / tn, gy = (q.M + tm - 1) / tm;
     q.tiles = gx * gy;
@@ -453,6 +460,20 @@ static TinyNNStatus ks_launch(KsParams& q, const KsPlan& p, const char* what) {
     q.d_w = make_fastdiv((uint32_t)q.strip_w);
     q.d_last = make_fastdiv((uint32_t)(gx - (q.strips - 1) * q.strip_w));
     const dim3 grid((unsigned)(w ? 8 * q.per_xcd : gx), (unsigned)(w ? 1 : gy));
+    const bool brief = p.waves == 4 && (q.K >> (p.r == 32 ? 3 : 4)) <= KS_SHORT;
+#define MG_KS_B(R_, MT_, NT_, T_, S_) (brief ? gemm_f32_ks_kernel<AM, BMODE, R_, MT_, NT_, T_, S_, true> : gemm_f32_ks_kernel<AM, BMODE, R_, MT_, NT_, T_, S_, false>)
+#define MG_KS_S(R_, MT_, NT_, T_) (w ? MG_KS_B(R_, MT_, NT_, T_, true) : MG_KS_B(R_, MT_, NT_, T_, false))
+#define MG_KS_T(R_, MT_, NT_) (tail ? MG_KS_S(R_, MT_, NT_, true) : MG_KS_S(R_, MT_, NT_, false))
+    void (*kern)(KsParams);
+    if (p.r == 16)
+        kern = MG_KS_T(16, 1, 1);
+    else if constexpr (CONV)  // (wider tiles never measured better for a convolution)
+        kern = MG_KS_T(32, 1, 1);
+    else
+        kern = p.mt == 1 ? (p.nt == 1 ? MG_KS_T(32, 1, 1) : MG_KS_T(32, 1, 2)) : (p.nt == 1 ? MG_KS_T(32, 2, 1) : MG_KS_T(32, 2, 2));
+#undef MG_KS_T
+#undef MG_KS_S
+#undef MG_KS_B
     q.lw = p.waves == 8 ? 3 : 2;
     note_kernel(what, tm, tn, p.waves, w);
     size_t lds = (size_t)p.waves * tm * tn * 4;

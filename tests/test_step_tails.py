@@ -66,6 +66,29 @@ def test_f32_products_of_few_tiles(m, k, n, ta, tb):
     assert np.array_equal(run_gpu(case, {x: np.round(8 * v) for x, v in arrays.items()}), _product(case, {x: np.round(8 * v) for x, v in arrays.items()}))
 
 
+# 32 x 32, 32 x 64 and 64 x 64 tiles, with and without strips, at the edges of the steps, of the four waves' shares and of the
+# short loop (28 steps of 8); 16 x 16 ones at theirs (28 of 16)
+@pytest.mark.parametrize("m,n,ks", [(700, 800, (1, 7, 8, 9, 33, 224, 231, 232)), (637, 1589, (17, 32, 224, 232)), (2500, 700, (1, 31, 72, 226, 231, 233)),
+                                    (2562, 675, (8, 100, 224)), (60, 500, (447, 448, 463, 464))])
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_f32_products_of_short_k(m, n, ks, ta, tb):
+    for k in ks:
+        test_f32_products_of_few_tiles(m, k, n, ta, tb)
+
+
+# the same edges in K = (channel, row, column) and pixels
+@pytest.mark.parametrize("n,ic,ih,iw,oc,k", [(2, 1, 77, 77, 101, 3), (2, 9, 77, 77, 101, 3), (13, 21, 26, 30, 69, 3), (9, 24, 28, 30, 69, 3), (9, 25, 28, 29, 69, 3),
+                                             (9, 26, 29, 29, 69, 3), (5, 224, 33, 31, 70, 1), (5, 232, 33, 31, 70, 1), (5, 3, 35, 51, 70, 1)])
+def test_f32_convolutions_of_short_k(n, ic, ih, iw, oc, k):
+    port.set_threads(8)
+    case = ConvCase(A.FMT_NCHW, A.DENSE, n, ic, ih, iw, oc, k, 1, k // 2, A.RELU, dtype="f32")
+    arrays = case.gen(seed=47)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().startswith("conv_f32_gemm_ks:32,32"), runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
 @pytest.mark.parametrize("n,ic,ih,iw,oc,k,stride", [(1, 1, 4, 4, 16, 3, 1), (1, 5, 9, 9, 17, 3, 1), (2, 28, 13, 11, 33, 3, 2), (1, 29, 14, 15, 15, 3, 1),
                                                     (1, 64, 28, 28, 64, 3, 1), (1, 32, 56, 56, 32, 3, 1), (3, 100, 14, 13, 30, 1, 1), (1, 21, 17, 16, 40, 5, 2)])
 @pytest.mark.parametrize("bias", [True, False])
