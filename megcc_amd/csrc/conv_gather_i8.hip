@@ -18,9 +18,9 @@
 // 32 of its matrix units; on small layers too, 4 waves' steps of 5 loads each). Measured (us, before: the one-stage
 // kernel of conv_mfma_i8.hip, beyond 9 taps conv_dot4.hip; then with steps beyond a wave's share fetched as zeros, the
 // table read before the first operand and the arguments where they are used; now): 6 x 88 -> 148 57 x 43 stride 2
-// 14.6, 7.1, 5.9; 4 x 24 -> 68 98 x 98 stride 2 14.8, 5.7, 4.2; 1 x 356 -> 52 68 x 81 21.2, 8.4, 7.6; 1 x 256 -> 256 28 x 28
-// 8.0, 5.6, 4.9; 47 x 104 -> 48 89 x 89 95.8, 50.5, 40.8; 58 x 264 -> 320 70 x 70 stride 2 216, 176, 156; 5x5: 1 x 120 -> 280
-// 19 x 19 134, 6.6, 5.8; 60 x 28 -> 20 63 x 63 137, 21.4, 17.4.
+// 14.6, 7.1, 5.9; 4 x 24 -> 68 98 x 98 stride 2 14.8, 5.7, 4.15; 1 x 356 -> 52 68 x 81 21.2, 8.4, 7.5; 1 x 256 -> 256 28 x 28
+// 8.0, 5.6, 4.8; 47 x 104 -> 48 89 x 89 95.8, 50.5, 40.3; 58 x 264 -> 320 70 x 70 stride 2 216, 176, 155; 5x5: 1 x 120 -> 280
+// 19 x 19 134, 6.6, 5.6; 60 x 28 -> 20 63 x 63 137, 21.4, 17.0.
 // Reference loop: BareMetal/ConvKernel.cpp:305-344.
 #include "conv_mfma_i8.h"
 
@@ -76,10 +76,6 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
     static_assert(64 * GATHER_WAVES == REQUANT_TABLE_ENTRIES, "an entry a thread");
     extern __shared__ __attribute__((aligned(16))) int gather_lds[];
     gather_begin(q);
-    // (Never taken. The block's end keeps the whole set-up behind the one wait for the arguments, where the compiler had it
-    // wait for single ones again: 256 -> 256 28 x 28 5.05 -> 4.91 us, 1 x 512 -> 512 7 x 7 7.0 -> 6.8.)
-    if (!RUNS && q.P <= 0)
-        return;
     int* const bias = gather_lds + REQUANT_TABLE_ENTRIES;  // [32 MT]
     int* const parts = bias + 32 * MT;
     const int lane = threadIdx.x & 63, col = lane & 31, kg = lane >> 5;
@@ -215,10 +211,13 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             s[e] = acc[i][j][e4 * 4 + e];
-        for (int g = 0; g < kw; ++g) {
-            if (g == grp)
-                continue;
-            const v4i o = *(const v4i*)(parts + (((g * pw + sub) * QUADS + x) * 64 + lane) * 4);
+        // (the other groups from the one behind this wave's, no question which of them is its own: 256 -> 256 28 x 28 5.05 -> 4.75 us,
+        // 512 -> 512 7 x 7 7.0 -> 6.65)
+#pragma unroll
+        for (int g = 1; g < GATHER_WAVES; ++g) {
+            if (g >= kw)
+                break;
+            const v4i o = *(const v4i*)(parts + (((((grp + g) & (kw - 1)) * pw + sub) * QUADS + x) * 64 + lane) * 4);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 s[e] += o[e];
