@@ -265,20 +265,30 @@ bool conv_gather_i8_supported(const ConvGeom& g) {
            (g.oc + 31) / 32 < 65536;
 }
 
-// The layers this kernel takes from the LDS-direct one (its variant `picked`). Measured over 3x3 and 5x5 layers of
-// 32 .. 512 channels, 7 x 7 .. 56 x 56, batch 1 .. 32 (us there / here):
-//   * the small-layer variants 6 and 7, one 32-channel tile a workgroup: when there is less than a 32 x 32 tile for
-//     every CU, and K is long enough to share (256 -> 256 28 x 28 8.0 / 5.6, 128 -> 128
-//     28 x 28 5.5 / 4.8; with 64 channels 4.7 / 4.7, with two tiles a CU 8.2 / 11.0);
-//   * the variants 8 and 9, a filter row a stage: when the tiles leave SIMDs without one (128 -> 128 28 x 28 N=8 20.2 /
-//     14.6, 64 -> 64 28 x 28 N=16 10.1 / 9.6; with more, 20.3 / 24.2), 9 when there are half as many (164 -> 60 18 x 17
-//     stride 2 N=56 29.2 / 21.9, 64 -> 64 56 x 56 stride 2 N=16 12.5 / 13.3). Layers of 48 channels and fewer would gain
-//     too (32 -> 32 28 x 28 N=16 6.9 / 5.1) but are what the row-split kernel is tested with.
+// The layers this kernel takes from the LDS-direct one (its variant `picked`), by how many 32 x 32 tiles there are for a CU.
+// Measured over 340 3x3 and 5x5 layers of 16 .. 512 channels, 7 x 7 .. 100 x 100, batch 1 .. 40 (us there / here):
+//   * the small-layer variants 6 and 7, one 32-channel tile a workgroup: under two tiles a CU (256 -> 256 28 x 28 7.9 / 4.8,
+//     128 -> 128 28 x 28 N=4 5.25 / 4.6, 512 -> 512 28 x 28 10.4 / 9.7, 64 -> 64 14 x 14 N=16 5.2 / 3.9; beyond, 256 -> 256 28 x 28 N=3
+//     7.7 / 7.9, 512 -> 128 14 x 14 N=24 12.9 / 14.9); with 32 channels both are at a launch's time, 6 slightly below (4.3 / 4.45);
+//   * 1 and 4, 128 channels by 256 pixels on part of the CUs: under three (140 -> 96 24 x 22 N=8 7.6 / 5.2, 388 -> 80 39 x 39 N=4 13.8 /
+//     10.4, 176 -> 96 57 x 68 N=2 8.2 / 6.55, 32 -> 64 56 x 56 N=3 4.8 / 4.6; beyond, 380 -> 112 17 x 16 N=24 13.7 / 14.6, 396 -> 220
+//     69 x 73 stride 2 N=4 19.6 / 29.1, 256 -> 64 28 x 28 N=22 10.4 / 10.9);
+//   * 8 and 9, a filter row a stage: under six (128 -> 64 56 x 56 N=5 16.7 / 10.9, 64 -> 60 54 x 48 N=8 10.7 / 9.0, 72 -> 140 23 x 26
+//     N=13 16.9 / 14.2; beyond, 172 -> 372 13 x 12 N=27 30.1 / 33.8) and under four (128 -> 32 56 x 56 stride 2 N=23 22.7 / 16.4, 292 ->
+//     112 90 x 63 stride 2 N=4 45.1 / 28.3; beyond, 256 -> 128 56 x 56 stride 2 N=11 44.4 / 48.0). Layers of 48 channels and fewer
+//     would gain too (32 -> 32 28 x 28 N=16 7.2 / 4.1) but are what the row-split kernel is tested with.
 bool conv_gather_i8_wins(const ConvGeom& g, int picked) {
     const long tiles = (((long)g.n * g.oh * g.ow + 31) / 32) * ((g.oc + 31) / 32);
-    if (picked == 6 || picked == 7)
-        return tiles < num_cus() && (long)((g.ic + 31) / 32) * g.fh * g.fw >= 36;
-    return (picked == 8 || picked == 9) && g.ic > 48 && tiles < (picked == 8 ? 4L : 2L) * num_cus();
+    const int taps = g.fh * g.fw;
+    switch (picked) {
+        case 6: return tiles < 2L * num_cus() && (long)((g.ic + 31) / 32) * taps > 9;
+        case 7: return tiles < 2L * num_cus();
+        case 1:
+        case 4: return tiles < 3L * num_cus() && taps > 1;
+        case 8: return tiles < 6L * num_cus() && g.ic > 48;
+        case 9: return tiles < 4L * num_cus() && g.ic > 48;
+        default: return false;
+    }
 }
 
 TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const void* packed, const void* bias, void* dst) {
@@ -313,11 +323,16 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     const bool table = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     if (table)
         q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
-    // 64 x 64 outputs a wave where that gives every SIMD one, else less. 32 x 32: four groups share a long K however many
-    // tiles there are (7 x 124 -> 240 29 x 23 11.4 us with one, 10.4 with four; 256 -> 256 28 x 28 5.6 with four, 6.0
-    // with eight), a shorter one while SIMDs are idle (24 x 56 -> 16 66 x 66 stride 2 6.9 with two, 7.3 with four; 3 x 20 ->
-    // 404 42 x 32 6.5 with one, 7.9 with four). 64 x 64: two share a long K where a SIMD has under four waves, to
-    // even out the last round (10 x 452 -> 108 75 x 91 77.5 with one, 68.1 with two).
+    // 64 x 64 outputs a wave where that gives every SIMD one, else less. Groups share K (1310 layers, kw 1, 2 and 4):
+    //   * 32 x 32: a long K however many tiles there are (7 x 124 -> 240 29 x 23 11.4 us with one group, 10.4 with four; 256 -> 256
+    //     28 x 28 5.6 with four, 6.0 with eight); a shorter one until there are 1.6 waves a SIMD - the second round is then as short
+    //     as the first (64 -> 64 28 x 28 N=24 6.5 with one, 5.5 with two, 32 -> 128 14 x 14 5x5 N=24 6.0 with two, 5.3 with four, 3 x 64 ->
+    //     64 90 x 90 6.2 with one, 5.3 with two; beyond, 32 -> 128 90 x 90 stride 2 N=8 6.3, 6.1 and, with four, 6.95);
+    //   * 64 x 32: the tiles are between one and two for a SIMD, two groups even out the last round (256 -> 256 56 x 56 N=3 19.7 with
+    //     one, 15.2 with two, 13.4 with four; 20 -> 404 28 x 28 N=8 6.05, 5.4, 6.7), four where it is nearly empty (96 -> 32 56 x 56 5x5
+    //     N=24 24.1, 18.6, 15.7; 1778 tiles, 20 -> 404 90 x 90 5x5 9.6, 8.7, 9.45);
+    //   * 64 x 64: two where a SIMD has under four waves (10 x 452 -> 108 75 x 91 77.5 with one, 68.1 with two; 124 -> 240 28 x 28
+    //     N=24 18.9, 17.7; 25 steps, 20 -> 404 56 x 56 N=3 11.8, 12.8).
     int mt = g.oc > 32 ? 2 : 1, nt = 2, kw = 1;
     const long full = 4L * num_cus();
     auto tiles = [&] { return (long)((q.P + 32 * nt - 1) / (32 * nt)) * ((g.oc + 32 * mt - 1) / (32 * mt)); };
@@ -326,9 +341,11 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     if (tiles() < full)
         mt = 1;
     if (mt * nt == 1) {
-        while (kw < 4 && q.steps >= 8 * kw && (tiles() * kw < full || q.steps >= 27))
+        while (kw < 4 && q.steps >= 8 * kw && (5 * tiles() * kw < 8 * full || q.steps >= 27))
             kw *= 2;
-    } else if (mt * nt == 4 && q.steps >= 72 && tiles() < 4 * full) {
+    } else if (mt * nt == 2) {
+        kw = q.steps >= 25 && 4 * tiles() < 5 * full ? 4 : q.steps >= 8 ? 2 : 1;
+    } else if (q.steps >= 36 && tiles() < 4 * full) {
         kw = 2;
     }
     // Where the image is more than an XCD's L2 holds, neighbouring pixels - rows of the image that both read - and a pixel

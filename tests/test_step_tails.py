@@ -29,6 +29,39 @@ def test_shares_of_k_in_dense_layers_without_staging(ic, k, stride, ties, bias):
     compare(got, case.run_port(arrays), repr(case))
 
 
+# both sides of the border between the LDS-direct kernel (by its variants) and the one without staging, channels and pixels that
+# fill no whole tile among them
+@pytest.mark.parametrize("n,ic,ih,iw,oc,k,stride,kernel", [
+    (5, 128, 28, 28, 100, 3, 1, "gather"), (6, 128, 28, 28, 100, 3, 1, "dma:6"), (2, 32, 28, 28, 64, 3, 1, "dma:6"), (2, 64, 28, 28, 64, 3, 1, "gather"),
+    (10, 96, 14, 14, 232, 3, 1, "gather"), (11, 96, 14, 14, 232, 3, 1, "dma:7"), (7, 32, 14, 14, 64, 3, 1, "gather"),
+    (8, 76, 24, 22, 96, 3, 1, "gather"), (5, 88, 48, 38, 80, 3, 1, "dma:1"), (6, 40, 56, 55, 100, 3, 2, "gather"),
+    (2, 76, 57, 68, 96, 3, 1, "gather"), (24, 44, 17, 16, 112, 3, 1, "dma:4"),
+    (8, 56, 30, 29, 84, 5, 1, "gather"), (14, 52, 24, 24, 196, 5, 1, "dma:8"),
+    (5, 52, 46, 44, 100, 5, 2, "gather"), (7, 64, 26, 21, 268, 5, 1, "dma:9")])
+def test_layers_on_both_sides_of_the_staging_border(n, ic, ih, iw, oc, k, stride, kernel):
+    port.set_threads(8)
+    case = ConvCase(A.FMT_NCHW44, A.DENSE, n, ic, ih, iw, oc, k, stride, k // 2, A.RELU, scales=(0.02, 0.01, unsat(ic * k * k)))
+    arrays = case.gen(seed=48)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().startswith("conv_mfma_i8_" + kernel), runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
+# the groups that share K: one, two and four with 32 x 32, 64 x 32, 32 x 64 and 64 x 64 outputs a wave, on both sides of each line
+@pytest.mark.parametrize("n,ic,ih,iw,oc,k,stride,kernel", [
+    (36, 60, 28, 30, 36, 3, 2, "32,32,4"), (70, 60, 29, 30, 64, 3, 2, "32,32,2"), (130, 60, 29, 30, 64, 3, 2, "32,32,1"),
+    (80, 20, 29, 30, 100, 3, 2, "64,32,2"), (80, 80, 29, 30, 100, 3, 2, "64,32,4"), (100, 68, 29, 30, 100, 3, 2, "64,32,2"),
+    (28, 56, 41, 59, 16, 3, 1, "32,64,2"), (24, 40, 56, 55, 16, 5, 1, "32,64,4"),
+    (150, 20, 29, 30, 100, 3, 2, "64,64,1"), (150, 100, 29, 30, 100, 3, 2, "64,64,2")])
+def test_groups_that_share_k(n, ic, ih, iw, oc, k, stride, kernel):
+    port.set_threads(8)
+    case = ConvCase(A.FMT_NCHW44, A.DENSE, n, ic, ih, iw, oc, k, stride, k // 2, A.RELU, scales=(0.02, 0.01, unsat(ic * k * k)))
+    arrays = case.gen(seed=49)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().split("+")[0] == "conv_mfma_i8_gather:" + kernel, runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
 # images beyond an XCD's L2, whose tiles are dealt to the XCDs in runs: one, two and several channel tiles, the last one whole or hanging over,
 # a number of pixel tiles that is and is not a multiple of eight
 @pytest.mark.parametrize("n,ic,ih,iw,oc,k,stride", [(21, 116, 47, 59, 20, 3, 1), (17, 64, 66, 66, 72, 3, 2), (67, 132, 23, 21, 36, 3, 2), (35, 52, 58, 58, 352, 3, 2), (23, 36, 87, 74, 144, 3, 1),
