@@ -323,7 +323,7 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     const bool table = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
     if (table)
         q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
-    // 64 x 64 outputs a wave where that gives every SIMD one, else less. Groups share K (1310 layers, kw 1, 2 and 4):
+    // 64 x 64 outputs a wave where that gives every SIMD one, else less. Groups share K (1300 layers, kw 1, 2 and 4):
     //   * 32 x 32: a long K however many tiles there are (7 x 124 -> 240 29 x 23 11.4 us with one group, 10.4 with four; 256 -> 256
     //     28 x 28 5.6 with four, 6.0 with eight); a shorter one until there are 1.6 waves a SIMD - the second round is then as short
     //     as the first (64 -> 64 28 x 28 N=24 6.5 with one, 5.5 with two, 32 -> 128 14 x 14 5x5 N=24 6.0 with two, 5.3 with four, 3 x 64 ->

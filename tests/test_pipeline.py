@@ -40,7 +40,12 @@ def build(net, planned, keep_all=False, **options):
     for k, v in options.items():
         runtime.set_option(k, v)
     try:
-        return net.build_gpu(keep_all=keep_all, model=PlannedModel(net) if planned else None)
+        model, ids = net.build_gpu(keep_all=keep_all, model=PlannedModel(net) if planned else None)
+        if options.get("no_graph"):  # (asked at the first forward: plain launches from then on)
+            model.set_input(ids["image"], np.zeros((net.batch, 3, 224, 224), np.float32))
+            model.forward()
+            assert model.launch_mode()[0] == -1
+        return model, ids
     finally:
         for k in options:
             runtime.set_option(k, 0)
@@ -50,7 +55,7 @@ def build(net, planned, keep_all=False, **options):
 def test_overlapped_forwards_equal_forwards_run_one_after_the_other(planned):
     net = mobilenet.Net(BATCH)
     images = [mobilenet.draw_input(BATCH, seed=s) for s in (1, 2, 3, 4, 5)]
-    # (no_graph: plain launches from the first forward on, no measuring phase)
+    # (no_graph: plain launches, no measuring phase)
     pipe, ids = build(net, planned, no_graph=1)
     serial, _ = build(net, planned, no_graph=1, nopipeline=1)
     assert pipe.nr_tail_kernel >= 2 and serial.nr_tail_kernel == 0
@@ -102,7 +107,7 @@ def test_asynchronous_read_of_a_tensor_the_first_stream_writes():
     mid = np.zeros(pipe.shapes[ids["pw3"]][0], np.int8)
     last = np.zeros((BATCH, 1000), np.float32)
     pipe.set_input(ids["image"], images[0])
-    pipe.forward()  # (the first forward of a model runs on one stream)
+    pipe.forward()
     for img in images:
         pipe.set_input(ids["image"], img)
         pipe.forward()
@@ -138,7 +143,9 @@ def test_a_network_of_a_few_operators_keeps_one_stream():
         m.finalize()
     finally:
         runtime.set_option("no_graph", 0)
-    assert m.nr_kernel == 5 and m.nr_tail_kernel == 0
+    m.set_input(x, np.zeros((4, 64, 56, 56), np.int8))
+    m.forward()
+    assert m.nr_kernel == 5 and m.nr_tail_kernel == 0 and m.launched_tail_kernel == 0
     m.close()
 
 
@@ -213,13 +220,6 @@ def test_a_forward_behind_a_wait_runs_on_one_stream():
         serial.forward()
         want.append(serial.get(ids["softmax"]).copy())
     out = np.zeros((BATCH, 1000), np.float32)
-    runtime.set_option("no_graph", 1)  # (asked at the first forward: plain launches from then on)
-    try:
-        pipe.forward()
-        pipe.get(ids["softmax"])
-    finally:
-        runtime.set_option("no_graph", 0)
-    assert pipe.launch_mode()[0] == -1
 
     def get():
         np.testing.assert_array_equal(pipe.get(ids["softmax"]), want[at])
