@@ -24,9 +24,9 @@
 // Both requantisations are the exact ones of epilogue.h, so the result is bit for bit the two kernels'.
 // Bound: HBM on the large maps, the vector ALU's requantisation and the filter's way from L2 on the small
 // ones; with one tile a workgroup the way from the launch to the first load (dp_begin).
-// Measured (N=64, us, one kernel / two): 32x112x112->64 20.2 / 32.4, 64 s2 -> 128 17.0 / 25.5, 128x56x56->128 17.4 / 28.5,
-// 256x28x28->256 13.3 / 22.1, 512x14x14->512 9.9 / 21.7, 1024x7x7->1024 11.3 / 20.2; N=1: 4.4 / 6.9, 4.8 / 6.6, 4.3 / 7.0,
-// 5.0 / 7.2, 6.7 / 7.9, 9.8 / 9.9; N=256: 88 / 117 and, 512 channels, 31.9 / 49.5. Before the arguments came in one round trip,
+// Measured (N=64, us, one kernel / two): 32x112x112->64 19.8 / 32.0, 64 s2 -> 128 17.0 / 25.5, 128x56x56->128 17.4 / 27.9,
+// 256x28x28->256 12.8 / 22.1, 512x14x14->512 9.5 / 21.5, 1024x7x7->1024 11.0 / 20.2; N=1: 4.0 / 7.0, 4.4 / 6.5, 3.9 / 7.1,
+// 4.6 / 7.2, 6.2 / 7.9, 9.5 / 9.9; N=256: 86 / 117 and, 512 channels, 31.0 / 49.2. Before the arguments came in one round trip,
 // slices followed the number of tiles and addresses were constants from one place, N=1: 5.1, 5.6, 5.2, 6.4, 9.7, 17.0; N=64, 512 and
 // 1024 channels: 10.9, 18.3. (Two jobs' operands in flight, 16 waves of 128 registers, the whole filter in registers, jobs
 // and products of two wave halves in opposite order: each slower, 512 channels N=1 by 0.4 - 1.6 us.)
@@ -68,7 +68,7 @@ struct DwPwArgs {
 // What a workgroup reads at its start, in whole 64-byte lines, and the tables. The kernel gets its address: 8 bytes of
 // arguments, which the launch costs the host 2.5 us, where the 2 KB themselves cost 3.9 (up to 104 bytes 2.6, up to 300 3.3),
 // and an argument that short is in registers when a wave starts (the build asks for it), so that the first round trip goes
-// to these lines instead of the argument segment. Launched again and again, 32 channels N=1 4.5 -> 4.0 us, 512 6.8 -> 6.3.
+// to these lines instead of the argument segment. Launched again and again, 32 channels N=1 4.5 -> 4.0 us, 512 6.8 -> 6.2.
 struct DwPwParams {
     union {
         DwPwArgs a;
