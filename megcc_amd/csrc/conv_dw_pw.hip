@@ -63,10 +63,9 @@ struct DwPwArgs {
     int xcds, xcd_q, xcd_r, xcd_runs, run_q, run_r, per_xcd;
     FastDiv d_xg, d_oh, d_slices;
     RequantPack dq, pq;
-    float dc, pc;            // estimates for the tables (mode 0)
 };
-// What a workgroup reads at its start, in whole 64-byte lines, and the tables. The kernel gets its address: 8 bytes of
-// arguments, which the launch costs the host 2.5 us, where the 2 KB themselves cost 3.9 (up to 104 bytes 2.6, up to 300 3.3),
+// What a workgroup reads at its start, in whole 64-byte lines. The kernel gets its address: 8 bytes of
+// arguments, which the launch costs the host 2.5 us, where the 256 themselves cost 3.3 (up to 104 bytes 2.6, 2 KB 3.9),
 // and an argument that short is in registers when a wave starts (the build asks for it), so that the first round trip goes
 // to these lines instead of the argument segment. Launched again and again, 32 channels N=1 4.5 -> 4.0 us, 512 6.8 -> 6.2.
 struct DwPwParams {
@@ -74,7 +73,6 @@ struct DwPwParams {
         DwPwArgs a;
         unsigned words[64];
     };
-    RequantTable dtable, ptable;
 };
 static_assert(sizeof(DwPwArgs) <= 256 && sizeof(DwPwParams) % 64 == 0, "four lines");
 
@@ -106,7 +104,7 @@ struct DpLaunch {
     unsigned workgroups;
 };
 struct DwPwBlock {
-    DwPwParams* dev = nullptr;  // [2]: by the proven multiply-adds where there are any, by the tables
+    DwPwParams* dev = nullptr;  // [2]: by the proven multiply-adds where there are any, by the literal sequence
     DwPwParams host[2];
     DpLaunch launch;
 };
@@ -143,46 +141,11 @@ __device__ __forceinline__ int dp_opaque(int v) {
     return v;
 }
 
-// 16 accumulators of one column -> 4 dwords (each 4 consecutive registers)
-// The empty volatile statements keep each form inside its branch: the compiler otherwise computes one of
-// them ahead of the branch and throws it away, 80 instructions of 120.
-template <int ACT, int N>
-__device__ __forceinline__ void dp_requant(int (&a)[N], uint32_t (&out)[N / 4], const RequantPack& q, float c, const int* table) {
-    auto here = [&]() __attribute__((always_inline)) {
-#ifndef MG_HOST_AUDIT
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-            asm volatile("" : "+v"(a[i]));
-#endif
-    };
-    if (q.mode == 1) {  // (uniform)
-        here();
-#pragma unroll
-        for (int i = 0; i < N / 4; ++i)
-            out[i] = requant_pack4<1, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
-    } else if (q.mode == 2) {
-        here();
-#pragma unroll
-        for (int i = 0; i < N / 4; ++i)
-            out[i] = requant_pack4<2, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
-    } else {
-        here();
-#pragma unroll
-        for (int i = 0; i < N / 4; ++i) {
-            int r[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                r[e] = requant_conv_table<ACT>(a[4 * i + e], c, table);
-            out[i] = pack4_perm(r[0], r[1], r[2], r[3]);
-        }
-    }
-}
-
 // LDS bytes of an instantiation
 template <int KC, int SUB>
 constexpr int dp_lds(int oc) {
     const int C = 32 * KC;
-    return 2 * (64 * SUB) * C + C * 16 + C * 4 + oc * 4 + 2 * 4 * REQUANT_TABLE_ENTRIES;
+    return 2 * (64 * SUB) * C + C * 16 + C * 4 + oc * 4;
 }
 
 // S: stride; KC: 32-channel chunks; SUB: 64-pixel parts of a tile; MT, NT: 32-channel and 32-pixel tiles per
@@ -207,8 +170,6 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwPar
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ocs = WO * 32 * MT;                               // channels of a slice
-    int* const dtbl = pb + ocs;
-    int* const ptbl = dtbl + REQUANT_TABLE_ENTRIES;
 
     // Workgroup -> (slice, run of tiles). Each XCD gets a contiguous eighth of the tiles, and the runs with a tile more are the
     // first ones of every XCD: one to a CU, not two (the first runs of all were, and sat on the same XCDs: 784 tiles for two
@@ -272,7 +233,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwPar
     Rows rows = rows_of(t_begin, sub0), cur;
     request(rows, 0);
 
-    // ---- set-up: filters, biases, tables -----------------------------------------------------------
+    // ---- set-up: filters, biases -----------------------------------------------------------
     // (all loads of a thread before its first store: a round trip for the whole set-up, not one per turn)
     constexpr int WI = (C * 4 + DP_THREADS - 1) / DP_THREADS, BI = (C + DP_THREADS - 1) / DP_THREADS;
     constexpr int PI = (WO * 32 * MT + DP_THREADS - 1) / DP_THREADS;
@@ -344,12 +305,6 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwPar
     for (int k = 0; k < PI; ++k)
         if (tid + k * DP_THREADS < ocs)
             pb[tid + k * DP_THREADS] = q.pbias ? pbv[k] : 0;
-    if (tid < REQUANT_TABLE_ENTRIES) {
-        if (q.dq.mode == 0)
-            dtbl[tid] = params->dtable.t[tid];
-    } else if (q.pq.mode == 0) {
-        ptbl[tid - REQUANT_TABLE_ENTRIES] = params->ptable.t[tid - REQUANT_TABLE_ENTRIES];
-    }
     if (KEEP_P) {
 #pragma unroll
         for (int c = 0; c < KC; ++c)
@@ -461,7 +416,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwPar
             for (int e = 0; e < 4; ++e)
                 a[p * 4 + e] = acc[p][e];
         uint32_t d[4];
-        dp_requant<DACT>(a, d, q.dq, q.dc, dtbl);
+        requant_dwords<DACT>(a, d, q.dq);
         *(v4i*)(m + mid0 + i * (8 * T * 16)) = v4i{(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
     };
     // ---- pointwise: where a column's results go. (Stores are issued whether or not the place exists: what is under no
@@ -490,7 +445,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwPar
         for (int e = 0; e < 16; ++e)
             a[e] = acc[e];
         uint32_t d[4];
-        dp_requant<PACT>(a, d, q.pq, q.pc, ptbl);
+        requant_dwords<PACT>(a, d, q.pq);
         // (OC is a multiple of 32: all of the tile's channels exist or none)
         const bool there = oc_wave + mi * 32 < q.OC;
         const unsigned o = there ? w : OOB;
@@ -617,7 +572,8 @@ bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* sr
            pw.pw == 0 && pw.ic == dw.oc && (pw.oc & 31) == 0 && dp_shape(dw.ic, pw.oc, 0, &s) &&
            dw.act == MEGCC_NONLINE_RELU &&
            (pw.act == MEGCC_NONLINE_IDENTITY || pw.act == MEGCC_NONLINE_RELU) &&
-           requant_table_ok(dw.s_src, dw.s_flt, dw.s_dst) && requant_table_ok(pw.s_src, pw.s_flt, pw.s_dst) &&
+           requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst, false).mode != 0 &&
+           requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst, false).mode != 0 &&
            ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 3) == 0 && (long)dw.n * dw.ic * dw.ih * dw.iw < (1L << 31) &&
            (long)pw.n * pw.oc * pw.oh * pw.ow < (1L << 31) && (long)dw.ih * dw.iw < (1L << 24) && dw.oh > 0 && dw.ow > 0;
 }
@@ -679,16 +635,8 @@ static TinyNNStatus dp_plan(
     q.d_xg = make_fastdiv(q.xg);
     q.d_oh = make_fastdiv(q.oh);
     q.d_slices = make_fastdiv(q.slices);
-    if (affine) {
-        q.dq = requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
-        q.pq = requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
-    }
-    q.dc = make_requant_fast(dw.s_src, dw.s_flt, dw.s_dst).c;
-    q.pc = make_requant_fast(pw.s_src, pw.s_flt, pw.s_dst).c;
-    if (q.dq.mode == 0)
-        all.dtable = *requant_table_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst);
-    if (q.pq.mode == 0)
-        all.ptable = *requant_table_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst);
+    q.dq = requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst, affine);
+    q.pq = requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst, affine);
     const int rag = dw.iw & 3;
     DwPwKernel kern = nullptr;
     size_t lds = 0;
@@ -757,7 +705,7 @@ TinyNNStatus conv_dw_pw_launch(
     MG_REQUIRE(q.src == src && q.dflt == dflt && q.dbias == dbias && q.wp == packed && q.pbias == pbias && q.dst == dst,
                TinyNN_ERROR_RUNTIME, "conv_dw_pw: not the operands it was prepared for");
     note_kernel("conv_dw_pw", dw.ic / 32, dw.sh, q.slices);
-    note_requant_affine(q.dq.mode != 0 && q.pq.mode != 0);
+    note_requant_affine(q.dq.affine() && q.pq.affine());
     hipLaunchKernelGGL(block->launch.kern, dim3(block->launch.workgroups), dim3(DP_THREADS), block->launch.lds, stream(), args);
     return check_launch("conv_dw_pw");
 }

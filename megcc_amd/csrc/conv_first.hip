@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(CF_THREADS) conv_first_q8_kernel(
 // 4m - 4 .. 4m + 3), so a pair of filter rows costs one 8-byte load for two pixels, the results leave as
 // one 8-byte store a plane, and nothing but the very first pixel's dword is special. A wave's steps
 // are consecutive (input rows that two output rows read are in its CU's L1), their number the same for
-// every wave but the last ones. The requantisation by one fused multiply-add needs no table: without
+// every wave but the last ones. The requantisation needs no table: without
 // one the arguments are an eighth.
 // What bounds it: memory (N = 256: 141 MB in 27.5 us is what a large copy reaches), below 64 images the set-up and
 // the first round trip. 3 x 224 x 224 -> 32 in us, with one pixel a lane, its filter bytes and biases loaded
@@ -140,19 +140,14 @@ struct ConvFirstMfmaParams {
     int src_bytes, dst_bytes;
     int IH, IW, OW2, OHW, pairs, steps, run, oc4n;
     int act;
-    float s_src, s_flt, s_dst, c;
-    float aff_c, aff_d;  // requantisation by one fused multiply-add (epilogue.h)
+    RequantPack rq;
     FastDiv dOW2, dOHW2;
 };
-struct ConvFirstNoTable {};
 static constexpr int CFM_WAVES = 5;  // waves a SIMD holds (N = 256 in us: 2 29.2, 3 28.5, 4 28.3, 5 27.5)
 
-// TABLE: RequantTable, or ConvFirstNoTable where ACT < 0 (the literal sequence) or the fused multiply-add is used
-template <int MT, int ACT, class TABLE>
-__global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParams q, TABLE table) {
-    constexpr bool TAB = sizeof(TABLE) > 64;
+template <int MT, int ACT>
+__global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParams q) {
     constexpr int OC = MT * 32;
-    __shared__ int tbl[TAB ? REQUANT_TABLE_ENTRIES : 1];
     __shared__ __attribute__((aligned(16))) int wlds[9 * OC], blds[OC];
     const int tid = threadIdx.x, lane = tid & 63;
     const int col = lane & 31, kg = lane >> 5;
@@ -208,8 +203,6 @@ __global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParam
     }
     if (tid >= 256 - OC)
         blds[tid - (256 - OC)] = q.bias ? q.bias[tid - (256 - OC)] : 0;
-    if constexpr (TAB)
-        tbl[tid] = table.t[tid];
     __syncthreads();
     // filter rows of this lane's output channels: A1 = pairs 4 * kg .. 4 * kg + 3, A2 = pair 8
     cfm_v4i A1[MT], A2[MT], biasv[MT][4];
@@ -224,14 +217,6 @@ __global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParam
         for (int e4 = 0; e4 < 4; ++e4)
             biasv[mi][e4] = *(const cfm_v4i*)(blds + mi * 32 + e4 * 8 + kg * 4);
     }
-    auto requant = [&](int a) __attribute__((always_inline)) {
-        if constexpr (ACT < 0)
-            return requant_conv_rt(q.act, a, q.s_src, q.s_flt, q.s_dst);
-        else if constexpr (TAB)
-            return requant_conv_table<ACT>(a, q.c, tbl);
-        else
-            return requant_conv_affine<ACT>(a, q.aff_c, q.aff_d);
-    };
     for (int t = t0; t < t1; ++t) {
         cfm_v4i be, bo;  // B operands of the even and the odd pixels
         int be8, bo8;
@@ -259,13 +244,17 @@ __global__ void __launch_bounds__(256) conv_first_mfma_kernel(ConvFirstMfmaParam
             ao = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1[mi], bo, ao, 0, 0, 0);
             ae = __builtin_amdgcn_mfma_i32_32x32x32_i8(A2[mi], cfm_v4i{be8, 0, 0, 0}, ae, 0, 0, 0);
             ao = __builtin_amdgcn_mfma_i32_32x32x32_i8(A2[mi], cfm_v4i{bo8, 0, 0, 0}, ao, 0, 0, 0);
+            int a[32];  // by plane: four channels of the even pixel, of the odd one
 #pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                cfm_v2i v;
-                v[0] = (int)pack4_perm(requant(ae[e4 * 4]), requant(ae[e4 * 4 + 1]), requant(ae[e4 * 4 + 2]), requant(ae[e4 * 4 + 3]));
-                v[1] = (int)pack4_perm(requant(ao[e4 * 4]), requant(ao[e4 * 4 + 1]), requant(ao[e4 * 4 + 2]), requant(ao[e4 * 4 + 3]));
-                __builtin_amdgcn_raw_buffer_store_b64(v, rd, out, (mi * 8 + e4 * 2) * q.OHW * 4, 0);
+            for (int e = 0; e < 16; ++e) {
+                a[e / 4 * 8 + e % 4] = ae[e];
+                a[e / 4 * 8 + 4 + e % 4] = ao[e];
             }
+            uint32_t d[8];
+            requant_dwords<ACT>(a, d, q.rq, q.act);
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4)
+                __builtin_amdgcn_raw_buffer_store_b64(cfm_v2i{(int)d[e4 * 2], (int)d[e4 * 2 + 1]}, rd, out, (mi * 8 + e4 * 2) * q.OHW * 4, 0);
         }
     }
 }
@@ -290,38 +279,23 @@ static TinyNNStatus conv_first_mfma_launch(
     q.steps = (q.pairs + 31) / 32;
     q.oc4n = g.oc / 4;
     q.act = g.act;
-    q.s_src = g.s_src; q.s_flt = g.s_flt; q.s_dst = g.s_dst;
-    q.c = make_requant_fast(g.s_src, g.s_flt, g.s_dst).c;
+    q.rq = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
+    note_requant_affine(q.rq.affine());
     q.dOW2 = make_fastdiv(q.OW2);
     q.dOHW2 = make_fastdiv(q.OHW / 2);
-    const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
-    const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
-    q.aff_c = aff.c;
-    q.aff_d = aff.d;
     // as many waves as are resident at once, and of those only as many as the longest run of steps needs
     const int most = num_cus() * 4 * CFM_WAVES;
     q.run = (q.steps + most - 1) / most;
     const unsigned blocks = (unsigned)(((q.steps + q.run - 1) / q.run + 3) / 4);
-    hipError_t e;
-    const int act = tab ? g.act : -1;
-#define MG_CFM(ACT_, TABLE_) \
-    (g.oc == 32 ? (const void*)conv_first_mfma_kernel<1, ACT_, TABLE_> : (const void*)conv_first_mfma_kernel<2, ACT_, TABLE_>)
-    if (!tab || aff.d != 0.f) {
-        const void* kern = act == MEGCC_NONLINE_IDENTITY ? MG_CFM(MEGCC_NONLINE_IDENTITY, ConvFirstNoTable)
-                         : act == MEGCC_NONLINE_RELU     ? MG_CFM(MEGCC_NONLINE_RELU, ConvFirstNoTable)
-                                                         : MG_CFM(-1, ConvFirstNoTable);
-        ConvFirstNoTable none;
-        void* args[] = {&q, &none};
-        e = hipLaunchKernel(kern, dim3(blocks), dim3(256), args, 0, stream());
-    } else {
-        const void* kern = act == MEGCC_NONLINE_IDENTITY ? MG_CFM(MEGCC_NONLINE_IDENTITY, RequantTable)
-                         : act == MEGCC_NONLINE_RELU     ? MG_CFM(MEGCC_NONLINE_RELU, RequantTable)
-                                                         : MG_CFM(MEGCC_NONLINE_H_SWISH, RequantTable);
-        const std::shared_ptr<const RequantTable> table = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
-        void* args[] = {&q, (void*)table.get()};
-        e = hipLaunchKernel(kern, dim3(blocks), dim3(256), args, 0, stream());
-    }
+    const int act = q.rq.mode ? g.act : -1;
+#define MG_CFM(ACT_) (g.oc == 32 ? (const void*)conv_first_mfma_kernel<1, ACT_> : (const void*)conv_first_mfma_kernel<2, ACT_>)
+    const void* kern = act == MEGCC_NONLINE_IDENTITY  ? MG_CFM(MEGCC_NONLINE_IDENTITY)
+                       : act == MEGCC_NONLINE_RELU    ? MG_CFM(MEGCC_NONLINE_RELU)
+                       : act == MEGCC_NONLINE_H_SWISH ? MG_CFM(MEGCC_NONLINE_H_SWISH)
+                                                      : MG_CFM(-1);
 #undef MG_CFM
+    void* args[] = {&q};
+    const hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(256), args, 0, stream());
     MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_first_mfma: %s", hipGetErrorString(e));
     return check_launch("conv_first_mfma");
 }

@@ -39,13 +39,11 @@ struct GatherParams {
     int IH, IW, OHW, OW, FW, SH, SW, PH, PW, DH, DW;
     FastDiv dOHW, dOW, dTaps, dFW;
     int act;
-    float s_src, s_flt, s_dst;
-    float c, aff_c, aff_d;  // scale of the table's estimate; the fused multiply-add (aff_d 0: none, the table)
+    RequantPack rq;
     // (tiles in runs on the XCDs) pixel tiles; whether a channel tile hangs over, which is then behind all the others of
     // its XCD; the number of the others
     int ptiles, ragged;
     FastDiv dOct;
-    RequantTable table;
 };
 
 // The arguments as the first thing, in one round trip: asked for where they are used, up to four round trips one
@@ -54,18 +52,11 @@ __device__ __forceinline__ void gather_begin(const GatherParams& q) {
 #ifndef MG_HOST_AUDIT
     asm volatile("" ::"s"(q.src), "s"(q.wp), "s"(q.bias), "s"(q.dst), "s"(q.src_bytes), "s"(q.wp_bytes), "s"(q.P), "s"(q.OC), "s"(q.steps), "s"(q.taps),
                  "s"(q.lkw), "s"(q.step_bytes), "s"(q.plane), "s"(q.image), "s"(q.row), "s"(q.IH), "s"(q.IW), "s"(q.OHW), "s"(q.OW), "s"(q.SH), "s"(q.SW),
-                 "s"(q.PH), "s"(q.PW), "s"(q.DH), "s"(q.DW), "s"(q.dOHW.mul), "s"(q.dOW.mul), "s"(q.dTaps.mul), "s"(q.dFW.mul), "s"(q.aff_d));
+                 "s"(q.PH), "s"(q.PW), "s"(q.DH), "s"(q.DW), "s"(q.dOHW.mul), "s"(q.dOW.mul), "s"(q.dTaps.mul), "s"(q.dFW.mul), "s"(q.rq.mode));
 #endif
 }
 
-// Entry i of the table, straight from the kernel-argument segment (conv_mfma_i8.h: kernarg_rq_table)
-__device__ __forceinline__ int gather_table(int i) {
-    typedef const __attribute__((address_space(4))) char* kptr;
-    const kptr base = (kptr)__builtin_amdgcn_kernarg_segment_ptr();
-    return *(const __attribute__((address_space(4))) int*)(base + offsetof(GatherParams, table) + 4 * i);
-}
-
-// ACT: an activation whose outputs the threshold table describes, or -1 (the literal sequence of q.act)
+// ACT: an activation with a requantisation of its own (q.rq), or -1 (the literal sequence of q.act)
 static constexpr int GATHER_LOG2_WAVES = 2, GATHER_WAVES = 1 << GATHER_LOG2_WAVES;  // of a workgroup
 
 // RUNS: every XCD has an eighth of the pixel tiles, each with all its channel tiles, in a row (conv_gather_i8_launch); else a
@@ -73,10 +64,9 @@ static constexpr int GATHER_LOG2_WAVES = 2, GATHER_WAVES = 1 << GATHER_LOG2_WAVE
 template <int MT, int NT, int ACT, bool RUNS>
 __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(GatherParams q) {
     constexpr int RING = 4;  // steps in flight (8: no step faster, 256 -> 256 28 x 28 5.1 us for 5.0, 4 x 24 -> 68 4.9 for 4.2)
-    static_assert(64 * GATHER_WAVES == REQUANT_TABLE_ENTRIES, "an entry a thread");
     extern __shared__ __attribute__((aligned(16))) int gather_lds[];
     gather_begin(q);
-    int* const bias = gather_lds + REQUANT_TABLE_ENTRIES;  // [32 MT]
+    int* const bias = gather_lds;  // [32 MT]
     int* const parts = bias + 32 * MT;
     const int lane = threadIdx.x & 63, col = lane & 31, kg = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -154,10 +144,7 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
     for (int r = 0; r < RING; ++r)
         load(grp + r * kw, A[r], B[r]);
     // What the outputs need is asked for behind the operands and waits in registers till the products are done.
-    const bool table = ACT >= 0 && q.aff_d == 0.f;
-    int entry = 0, bv = 0;
-    if (table)
-        entry = gather_table(threadIdx.x);
+    int bv = 0;
     if (q.bias && threadIdx.x < 32 * MT)
         bv = q.bias[min(oc0 + (int)threadIdx.x, q.OC - 1)];
     auto multiply = [&](const v4i (&a)[MT], const v4i (&b)[NT]) __attribute__((always_inline)) {
@@ -188,8 +175,6 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
     }
     // [group][wave of it][quad][lane]: a quad is 4 neighbouring channels of the lane's pixel
     constexpr int QUADS = MT * NT * 4;
-    if (table)
-        gather_lds[threadIdx.x] = entry;
     if (threadIdx.x < 32 * MT)
         bias[threadIdx.x] = bv;
     if (kw > 1) {
@@ -229,27 +214,9 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             s[e] += bq[e];
-        int r[4];
-        if constexpr (ACT == MEGCC_NONLINE_IDENTITY || ACT == MEGCC_NONLINE_RELU) {
-            if (!table) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    r[e] = requant_conv_affine<ACT>(s[e], q.aff_c, q.aff_d);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    r[e] = requant_conv_table<ACT>(s[e], q.c, gather_lds);
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if constexpr (ACT < 0)
-                    r[e] = requant_conv_rt(q.act, s[e], q.s_src, q.s_flt, q.s_dst);
-                else
-                    r[e] = requant_conv_table<ACT>(s[e], q.c, gather_lds);
-            }
-        }
-        ((uint32_t*)q.dst)[((size_t)img[j] * (q.OC >> 2) + (oc >> 2)) * q.OHW + rem[j]] = pack4_perm(r[0], r[1], r[2], r[3]);
+        uint32_t d[1];
+        requant_dwords<ACT>(s, d, q.rq, q.act);
+        ((uint32_t*)q.dst)[((size_t)img[j] * (q.OC >> 2) + (oc >> 2)) * q.OHW + rem[j]] = d[0];
     }
 }
 
@@ -316,13 +283,6 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     q.dTaps = make_fastdiv(q.taps);
     q.dFW = make_fastdiv(g.fw);
     q.act = g.act;
-    q.s_src = g.s_src;
-    q.s_flt = g.s_flt;
-    q.s_dst = g.s_dst;
-    q.c = make_requant_fast(g.s_src, g.s_flt, g.s_dst).c;
-    const bool table = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
-    if (table)
-        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
     // 64 x 64 outputs a wave where that gives every SIMD one, else less. Groups share K (1300 layers, kw 1, 2 and 4):
     //   * 32 x 32: a long K however many tiles there are (7 x 124 -> 240 29 x 23 11.4 us with one group, 10.4 with four; 256 -> 256
     //     28 x 28 5.6 with four, 6.0 with eight); a shorter one until there are 1.6 waves a SIMD - the second round is then as short
@@ -363,20 +323,19 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     const dim3 grid((unsigned)(runs ? (gx + 7) / 8 * 8 * gy : gx), (unsigned)(runs ? 1 : gy));
 #define MG_GATHER_R(MT_, NT_, ACT_) (runs ? conv_gather_i8_kernel<MT_, NT_, ACT_, true> : conv_gather_i8_kernel<MT_, NT_, ACT_, false>)
 #define MG_GATHER_A(MT_, NT_)                                                                \
-    (!table                              ? MG_GATHER_R(MT_, NT_, -1)                         \
+    (q.rq.mode == 0                      ? MG_GATHER_R(MT_, NT_, -1)                         \
      : g.act == MEGCC_NONLINE_IDENTITY   ? MG_GATHER_R(MT_, NT_, MEGCC_NONLINE_IDENTITY)     \
      : g.act == MEGCC_NONLINE_RELU       ? MG_GATHER_R(MT_, NT_, MEGCC_NONLINE_RELU)         \
                                          : MG_GATHER_R(MT_, NT_, MEGCC_NONLINE_H_SWISH))
+    q.lkw = kw == 4 ? 2 : kw == 2 ? 1 : 0;
+    note_kernel("conv_mfma_i8_gather", 32 * mt, 32 * nt, kw);
+    q.rq = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
+    note_requant_affine(q.rq.affine());
     void (*kern)(GatherParams) = mt == 2 ? (nt == 2 ? MG_GATHER_A(2, 2) : MG_GATHER_A(2, 1))
                                          : (nt == 2 ? MG_GATHER_A(1, 2) : MG_GATHER_A(1, 1));
 #undef MG_GATHER_A
 #undef MG_GATHER_R
-    q.lkw = kw == 4 ? 2 : kw == 2 ? 1 : 0;
-    note_kernel("conv_mfma_i8_gather", 32 * mt, 32 * nt, kw);
-    const RequantAffine aff = requant_affine_pick(table, g.act, g.s_src, g.s_flt, g.s_dst);
-    q.aff_c = aff.c;
-    q.aff_d = aff.d;
-    const size_t lds = (REQUANT_TABLE_ENTRIES + 32 * mt) * 4 + (kw > 1 ? (size_t)GATHER_WAVES * mt * nt * 4096 : 0);
+    const size_t lds = 32 * mt * 4 + (kw > 1 ? (size_t)GATHER_WAVES * mt * nt * 4096 : 0);
     if (lds > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_gather_i8: LDS attribute: %s", hipGetErrorString(e));

@@ -40,26 +40,14 @@ struct MfmaParams {
     int range_len;  // pixels per workgroup of the pipelined kernel (multiple of 32)
     int act;
     float s_src, s_flt, s_dst;
-    RequantFast rq;
+    RequantPack rq;
     // split-K of the one-stage kernel: blockIdx.z handles stages [z*sps, (z+1)*sps) and writes raw
     // int32 sums to partial[z][P][round_up(OC,4)]; conv_mfma_reduce_kernel finishes
     int split, sps;
     int32_t* partial;
     XcdOrder xo;  // FullyConnected tiles of the LDS-direct kernel: tile order (set at launch)
     FastDiv dOW, dOH, dVW, dVH, dL, dOHW;
-    // exact requantisation thresholds for IDENTITY / RELU (built on the host, epilogue.h); only
-    // the kernels that look outputs up in LDS read it
-    RequantTable rq_table;
 };
-
-// Entry i of the threshold table of a kernel whose ONLY argument is an MfmaParams, read straight
-// from the kernel-argument segment (indexing the by-value struct with a run-time index can make
-// the compiler copy all of it to scratch).
-__device__ __forceinline__ int kernarg_rq_table(int i) {
-    typedef const __attribute__((address_space(4))) char* kptr;
-    const kptr base = (kptr)__builtin_amdgcn_kernarg_segment_ptr();
-    return *(const __attribute__((address_space(4))) int*)(base + offsetof(MfmaParams, rq_table) + 4 * i);
-}
 
 // virtual pixel index of output pixel p at tap (0,0): rows of the zero-padded images stacked
 __device__ __forceinline__ int vp_of(const MfmaParams& q, int p) {

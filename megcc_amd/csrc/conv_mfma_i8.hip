@@ -230,28 +230,32 @@ __global__ void __launch_bounds__(THREADS) conv_mfma_i8_kernel(MfmaParams q) {
 #pragma unroll
                 for (int ni = 0; ni < NT; ++ni) {
                     if (pix_n[ni] >= 0) {
-                        int r[4];
+                        int a[4];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const int a = acc[mi][ni][e4 * 4 + e] + bv[e];
-                            if constexpr (ACT == ACT_RUNTIME)
-                                r[e] = requant_conv_rt(q.act, a, q.s_src, q.s_flt, q.s_dst);
-                            else
-                                r[e] = requant_conv_fast<ACT>(a, q.rq);
+                        for (int e = 0; e < 4; ++e)
+                            a[e] = acc[mi][ni][e4 * 4 + e] + bv[e];
+                        uint32_t d[1];
+                        if constexpr (ACT == ACT_RUNTIME) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                a[e] = requant_conv_rt(q.act, a[e], q.s_src, q.s_flt, q.s_dst);
+                            d[0] = pack4_perm(a[0], a[1], a[2], a[3]);
+                        } else {
+                            requant_dwords<ACT>(a, d, q.rq);
                         }
                         if (!q.dst_fc) {
                             size_t o = ((size_t)pix_n[ni] * (q.OC >> 2) + (oc >> 2)) * q.OHW + pix_rem[ni];
-                            ((uint32_t*)q.dst)[o] = pack4(r[0], r[1], r[2], r[3]);
+                            ((uint32_t*)q.dst)[o] = d[0];
                         } else {
                             const int p = p0 + wn * 64 + ni * 32 + (lane & 31);
                             int8_t* o = q.dst + (size_t)p * q.OC + oc;
                             if (((q.OC & 3) == 0)) {
-                                *(uint32_t*)o = pack4(r[0], r[1], r[2], r[3]);
+                                *(uint32_t*)o = d[0];
                             } else {
 #pragma unroll
                                 for (int e = 0; e < 4; ++e)
                                     if (oc + e < q.OC)
-                                        o[e] = (int8_t)r[e];
+                                        o[e] = (int8_t)(d[0] >> (8 * e));
                             }
                         }
                     }
@@ -693,10 +697,7 @@ TinyNNStatus conv_mfma_launch(
     q.s_src = g.s_src;
     q.s_flt = g.s_flt;
     q.s_dst = g.s_dst;
-    q.rq = make_requant_fast(g.s_src, g.s_flt, g.s_dst);
-    if (pipe && requant_table_act(g.act) && !(fc && g.act == MEGCC_NONLINE_H_SWISH) &&
-        requant_table_ok(g.s_src, g.s_flt, g.s_dst))
-        q.rq_table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
+    q.rq = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
     q.dOW = make_fastdiv(q.OW);
     q.dOH = make_fastdiv(q.OH);
     q.dVW = make_fastdiv(q.VW);
@@ -716,11 +717,7 @@ TinyNNStatus conv_mfma_launch(
             q.dst_fc = 3;  // rows leave through the kernel's staging area in LDS
         note_kernel(q.xo.w ? "conv_mfma_i8_dma_xo" : "conv_mfma_i8_dma", picked,
                     pc.bm, pc.bn, q.Lmax, pc.ks);
-        const RequantAffine aff = requant_affine_pick(
-                requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst), g.act, g.s_src, g.s_flt,
-                g.s_dst);
-        q.rq.aff_c = aff.c;
-        q.rq.aff_d = aff.d;
+        note_requant_affine(q.rq.affine());
         return conv_mfma_pipe_launch(pc, q);
     }
     const int split = conv_mfma_split(g);
@@ -758,10 +755,10 @@ TinyNNStatus conv_mfma_launch(
     MG_REQUIRE(lds <= 160 * 1024, TinyNN_ERROR_OUT_OF_RANGE, "conv_mfma: %zu bytes of LDS", lds);
     dim3 grid((q.P + BN - 1) / BN, (g.oc + bm - 1) / bm, q.split);
     void (*kern)(MfmaParams);
-    if (g.act == MEGCC_NONLINE_IDENTITY)
+    if (q.rq.mode && g.act == MEGCC_NONLINE_IDENTITY)
         kern = bm == 64 ? conv_mfma_i8_kernel<64, MEGCC_NONLINE_IDENTITY>
                         : conv_mfma_i8_kernel<128, MEGCC_NONLINE_IDENTITY>;
-    else if (g.act == MEGCC_NONLINE_RELU)
+    else if (q.rq.mode && g.act == MEGCC_NONLINE_RELU)
         kern = bm == 64 ? conv_mfma_i8_kernel<64, MEGCC_NONLINE_RELU>
                         : conv_mfma_i8_kernel<128, MEGCC_NONLINE_RELU>;
     else

@@ -16,7 +16,7 @@
 // One workgroup = 8 waves (2 x 4) on a 128 oc x 256 pixel tile, 64 accumulators per lane. The
 // loads of the next sub-tile's first stages are already in flight while a sub-tile's epilogue runs.
 //
-// Requantisation uses the exact threshold table (epilogue.h) built once per workgroup.
+// Requantisation: epilogue.h.
 #include <stdlib.h>
 
 #include "conv_mfma_i8.h"
@@ -86,8 +86,7 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
     static_assert(N_FLIGHT < 64 && DM_NBUF >= 2, "vmcnt range");
 
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
-    int* const rq_table = (int*)(lds + DM_NBUF * BUF_BYTES);
-    int* const bias_lds = rq_table + REQUANT_TABLE_ENTRIES;
+    int* const bias_lds = (int*)(lds + DM_NBUF * BUF_BYTES);
 
     // (the wave index through readfirstlane: everything derived from it - which chunks a wave loads,
     //  ring positions, the column count of a ragged sub-tile, the stage counters updated under it -
@@ -109,11 +108,7 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
     const int n_tiles = (range1 - range0 + DM_BNP - 1) / DM_BNP;
     const int G = n_tiles * stages;
 
-    // ---- once per workgroup: requantisation thresholds and the bias slice of this oc tile
-    if constexpr (ACT != ACT_RT) {
-        if (tid < REQUANT_TABLE_ENTRIES)
-            rq_table[tid] = kernarg_rq_table(tid);
-    }
+    // ---- once per workgroup: the bias slice of this oc tile
     for (int i = tid; i < DM_BM; i += DM_THREADS)
         bias_lds[i] = (q.bias && oc0 + i < q.OC) ? q.bias[oc0 + i] : 0;
 
@@ -264,49 +259,39 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
     v16i acc[MT][NT];
 
     // Epilogue of one 32 oc x 32 pixel MFMA tile (16 outputs per lane = 4 NCHW44 dwords), written
-    // as one straight-line block so that its 4 bias reads and 16 table look-ups are in flight
-    // together. ob: dword index in dst of this lane's pixel in oc-group 0 (-1: lane beyond the
+    // as one straight-line block. ob: dword index in dst of this lane's pixel in oc-group 0 (-1: lane beyond the
     // sub-tile, -2: whole 32-pixel column beyond it, wave-uniform).
-    // the 16 requantised outputs of this lane in tile (mi, ni)
-    auto requant_tile = [&](auto mic, auto nic, int (&r)[16], const int* tbl) __attribute__((always_inline)) {
+    // the 16 requantised outputs of this lane in tile (mi, ni): 4 channels a dword
+    auto requant_tile = [&](auto mic, auto nic, uint32_t (&w)[4]) __attribute__((always_inline)) {
         constexpr int mi = decltype(mic)::value, ni = decltype(nic)::value;
+        int a[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            a[e] = acc[mi][ni][e];
         if constexpr (ACT == ACT_RT) {
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-                r[e] = requant_conv_rt(q.act, acc[mi][ni][e], q.s_src, q.s_flt, q.s_dst);
-        } else if (ACT != MEGCC_NONLINE_H_SWISH && q.rq.aff_d != 0.f) {  // (uniform)
+                a[e] = requant_conv_rt(q.act, a[e], q.s_src, q.s_flt, q.s_dst);
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                r[e] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(acc[mi][ni][e], q.rq.aff_c, q.rq.aff_d);
+            for (int e4 = 0; e4 < 4; ++e4)
+                w[e4] = pack4_perm(a[e4 * 4], a[e4 * 4 + 1], a[e4 * 4 + 2], a[e4 * 4 + 3]);
         } else {
-            int m[16], t[16];
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                m[e] = requant_table_candidate<ACT>(acc[mi][ni][e], q.rq.c);
-                t[e] = tbl[m[e] + 128];
-            }
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                r[e] = m[e] + (acc[mi][ni][e] > t[e] ? 1 : 0);
+            requant_dwords<ACT>(a, w, q.rq);
         }
     };
     // (FC, dst_fc >= 2) the lane's 16 bytes of tile (mi, ni): channels 16 kg .. + 15 of the tile, row =
     // the lane's column. A lane's four dwords are channels 8 e4 + 4 kg .. + 3, so lanes l and l + 32
     // (same row, the two K-halves) together own 32 consecutive bytes; two v_permlane32_swap give the
     // lower lane the first 16 of them and the upper lane the rest.
-    auto fc_piece = [&](auto mic, auto nic, const int* tbl) __attribute__((always_inline)) -> v4u {
+    auto fc_piece = [&](auto mic, auto nic) __attribute__((always_inline)) -> v4u {
         typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
-        int r[16];
-        requant_tile(mic, nic, r, tbl);
         uint32_t w[4];
-#pragma unroll
-        for (int e4 = 0; e4 < 4; ++e4)
-            w[e4] = pack4_perm(r[e4 * 4], r[e4 * 4 + 1], r[e4 * 4 + 2], r[e4 * 4 + 3]);
+        requant_tile(mic, nic, w);
         const v2u_t s02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
         const v2u_t s13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
         return v4u{s02[0], s02[1], s13[0], s13[1]};
     };
-    auto emit_tile = [&](auto mic, auto nic, const int ob, const int* tbl) __attribute__((always_inline)) {
+    auto emit_tile = [&](auto mic, auto nic, const int ob) __attribute__((always_inline)) {
         constexpr int mi = decltype(mic)::value;
         if (ob < -1)
             return;
@@ -316,21 +301,21 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
             // store per lane instead of four dword stores 4096 bytes apart from their neighbours' (the
             // dword stores were half of the 4096 x 4096 x 4096 layer's time).
             if (q.dst_fc >= 2) {  // (uniform)
-                const v4u px = fc_piece(mic, nic, tbl);
+                const v4u px = fc_piece(mic, nic);
                 if (ob >= 0 && oc0 + (wm * MT + mi) * 32 < q.OC)  // (whole tiles: OC is a multiple of 32)
                     *(v4u*)(q.dst + (size_t)ob * q.OC + oc0 + (wm * MT + mi) * 32 + kg * 16) = px;
                 return;
             }
         }
-        int r[16];
-        requant_tile(mic, nic, r, tbl);
+        uint32_t d[4];
+        requant_tile(mic, nic, d);
         if (ob >= 0) {
 #pragma unroll
             for (int e4 = 0; e4 < 4; ++e4) {
                 const int oc = oc0 + ocl + e4 * 8;
                 if (oc >= q.OC)
                     continue;
-                const uint32_t w = pack4_perm(r[e4 * 4], r[e4 * 4 + 1], r[e4 * 4 + 2], r[e4 * 4 + 3]);
+                const uint32_t w = d[e4];
                 if constexpr (!FC) {
                     // scalar base (channel group) + 32-bit lane offset (pixel and K-half's plane)
                     int8_t* const base =
@@ -481,8 +466,8 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
                     const int row0 = p0 + (ni * WGN + wn) * 32;  // first row of this 32-row column
                     static_for<MT / 2>([&](auto hc) {
                         constexpr int h = decltype(hc)::value;
-                        const v4u pa = fc_piece(std::integral_constant<int, 2 * h>{}, nic, rq_table);
-                        const v4u pb = fc_piece(std::integral_constant<int, 2 * h + 1>{}, nic, rq_table);
+                        const v4u pa = fc_piece(std::integral_constant<int, 2 * h>{}, nic);
+                        const v4u pb = fc_piece(std::integral_constant<int, 2 * h + 1>{}, nic);
                         *(v4u*)(stage + (lane & 31) * FC_STAGE_ROW + kg * 16) = pa;
                         *(v4u*)(stage + (lane & 31) * FC_STAGE_ROW + 32 + kg * 16) = pb;
                         const int ocb = oc0 + (wm * MT + 2 * h) * 32;  // (64 channels from here on)
@@ -499,18 +484,18 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
             }
         }
         static_for<MT>([&](auto mic) {
-            static_for<NT>([&](auto nic) { emit_tile(mic, nic, cur_o[decltype(nic)::value], rq_table); });
+            static_for<NT>([&](auto nic) { emit_tile(mic, nic, cur_o[decltype(nic)::value]); });
         });
     }
 }
 
 // ---- configurations --------------------------------------------------------------------------
 template <int FH, int FW, int KS, int LMAX, bool FC, int MT = 2, int DM_NBUF = 3, int WGM = 2, int BPC = 1, int NT = 2, bool FCB = false, bool PM = false>
-static PipeConfig make_dma_config(int act, bool table_ok);
+static PipeConfig make_dma_config(int act, bool proven);
 
 // row-split configurations (filters of more than 9 taps): 64 * MT oc x 128 * NT px, FW taps per stage
 template <int FW, int LMAX, int MT, int DM_NBUF, int NT>
-static PipeConfig make_rs_config(int act, bool table_ok) {
+static PipeConfig make_rs_config(int act, bool proven) {
     PipeConfig c;
     c.bm = 64 * MT;
     c.bn = 128 * NT;
@@ -521,19 +506,19 @@ static PipeConfig make_rs_config(int act, bool table_ok) {
     c.a_bytes = FW * c.bm * KROW;
     c.fixed_lmax = LMAX;
     c.rs = 1;
-    c.extra_lds = REQUANT_TABLE_ENTRIES * 4 + 128 * 4;
+    c.extra_lds = 128 * 4;
     c.kernel = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, ACT_RT, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
-    if (act == MEGCC_NONLINE_IDENTITY && table_ok)
+    if (act == MEGCC_NONLINE_IDENTITY && proven)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, MEGCC_NONLINE_IDENTITY, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
-    else if (act == MEGCC_NONLINE_RELU && table_ok)
+    else if (act == MEGCC_NONLINE_RELU && proven)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, MEGCC_NONLINE_RELU, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
-    else if (act == MEGCC_NONLINE_H_SWISH && table_ok)
+    else if (act == MEGCC_NONLINE_H_SWISH && proven)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, MEGCC_NONLINE_H_SWISH, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
     return c;
 }
 
 template <int FH, int FW, int KS, int LMAX, bool FC, int MT, int DM_NBUF, int WGM, int BPC, int NT, bool FCB, bool PM>
-static PipeConfig make_dma_config(int act, bool table_ok) {
+static PipeConfig make_dma_config(int act, bool proven) {
     constexpr int DM_BM = 32 * MT * WGM;
     PipeConfig c;
     c.bm = DM_BM;
@@ -545,16 +530,16 @@ static PipeConfig make_dma_config(int act, bool table_ok) {
     c.a_bytes = FH * FW * KS * c.bm * KROW;
     c.fixed_lmax = LMAX;
     c.pm = PM ? 1 : 0;
-    c.extra_lds = REQUANT_TABLE_ENTRIES * 4 + (DM_BM > 128 ? DM_BM : 128) * 4 +
+    c.extra_lds = (DM_BM > 128 ? DM_BM : 128) * 4 +
                   (FCB && MT == 4 ? 4 * WGM * 32 * 80 : 0);  // (32 rows x 80 bytes of staging per wave)
     c.fcb = FCB ? 1 : 0;
     c.kernel = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, ACT_RT, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
-    if (act == MEGCC_NONLINE_IDENTITY && table_ok)
+    if (act == MEGCC_NONLINE_IDENTITY && proven)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, MEGCC_NONLINE_IDENTITY, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
-    else if (act == MEGCC_NONLINE_RELU && table_ok)
+    else if (act == MEGCC_NONLINE_RELU && proven)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, MEGCC_NONLINE_RELU, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
     if constexpr (!FC) {  // (FullyConnected with H_SWISH keeps the literal sequence)
-        if (act == MEGCC_NONLINE_H_SWISH && table_ok)
+        if (act == MEGCC_NONLINE_H_SWISH && proven)
             c.kernel = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, MEGCC_NONLINE_H_SWISH, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
     }
     return c;
@@ -575,7 +560,7 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
         if (fc || g.fmt != MEGCC_FMT_NCHW44 || !(g.fw == 5 || g.fw == 7) || g.fh != g.fw || g.oc < 32 ||
             P < 2048 || (long)g.n * g.oc * g.oh * g.ow >= (1L << 31))
             return false;
-        const bool okt = requant_table_ok(g.s_src, g.s_flt, g.s_dst);
+        const bool okt = requant_pack_for(g.act, g.s_src, g.s_flt, g.s_dst, false).mode != 0;
         const bool wide = g.oc >= 128;
         if (variant == 8)
             *c = g.fw == 5 ? (wide ? make_rs_config<5, 512, 2, 3, 2>(g.act, okt) : make_rs_config<5, 512, 1, 3, 2>(g.act, okt))
@@ -599,7 +584,7 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
             P * ((g.oc + 127) / 128) >= (P >= 4096 ? 32L : 64L) * num_cus() || g.oc < 32 || (g.ic & 31) ||
             (long)g.n * g.oc * g.oh * g.ow >= (1L << 31))
             return false;
-        const bool okt = requant_table_ok(g.s_src, g.s_flt, g.s_dst);
+        const bool okt = requant_pack_for(g.act, g.s_src, g.s_flt, g.s_dst, false).mode != 0;
         if (variant == 6) {
             if (g.sw != 1 || (g.iw & 3) || !b128_ok ||
                 ((long)g.n * (g.ih + 2 * g.ph) + 2L * g.fh * g.dh) * (g.iw + g.pw + 3) >= (1L << 31))
@@ -616,7 +601,7 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
         return false;  // 64-channel tiles: 3x3 layers and the 1x1 with 32 input channels
     if ((long)g.n * g.oc * g.oh * g.ow >= (1L << 31))
         return false;  // 32-bit output offsets
-    const bool ok = requant_table_ok(g.s_src, g.s_flt, g.s_dst);
+    const bool ok = requant_pack_for(g.act, g.s_src, g.s_flt, g.s_dst, false).mode != 0;
     // measured slower on the 256-channel 56x56 layer (91 us): two 256-thread workgroups per CU
     // with 64-channel tiles and two buffers (100 us), four waves of 128 oc x 64 pixels (107 us)
     if (variant == 2 || variant == 3) {

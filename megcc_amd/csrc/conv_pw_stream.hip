@@ -18,7 +18,7 @@
 // them can be resident and the memory latency is hidden by occupancy.
 //
 // Same arithmetic as the other qsi8 kernels: int32 accumulators starting from the bias, exact
-// requantisation by threshold table (epilogue.h). Reference loop: BareMetal/ConvKernel.cpp:305-344.
+// requantisation (epilogue.h). Reference loop: BareMetal/ConvKernel.cpp:305-344.
 #include <stdlib.h>
 
 #include <map>
@@ -44,19 +44,11 @@ struct PwParams {
     int image_stride;  // bytes
     int plane_stride;  // bytes
     int act;
-    float s_src, s_flt, s_dst, c;
-    float aff_c, aff_d;  // requantisation by one fused multiply-add (epilogue.h); aff_d == 0: table
+    RequantPack rq;
     FastDiv dOHW;
-    RequantTable table;
 };
 
-__device__ __forceinline__ int pw_kernarg_table(int i) {
-    typedef const __attribute__((address_space(4))) char* kptr;
-    const kptr base = (kptr)__builtin_amdgcn_kernarg_segment_ptr();
-    return *(const __attribute__((address_space(4))) int*)(base + offsetof(PwParams, table) + 4 * i);
-}
-
-// KC: 32-channel K chunks (IC = 32 * KC). ACT: IDENTITY / RELU use the table, -1 evaluates the
+// KC: 32-channel K chunks (IC = 32 * KC). ACT: as in requant_dwords, -1 evaluates the
 // literal sequence with the run-time activation.
 // MT: 32-channel MFMA row tiles per wave (a wave owns 32 * MT output channels).
 // RG: ragged channel counts - IC below 32 * KC (the planes beyond IC are not fetched: out-of-range
@@ -64,7 +56,6 @@ __device__ __forceinline__ int pw_kernarg_table(int i) {
 // wave's surplus channels are computed from zero filter rows and not stored).
 template <int KC, int MT, int ACT, bool RG = false>
 __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) {
-    __shared__ int tbl[REQUANT_TABLE_ENTRIES];
     __shared__ __attribute__((aligned(16))) int bias_lds[PW_MAX_OC];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, kg = lane >> 5;
@@ -125,9 +116,7 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
         load_chunk(tile_base(t + s / KC), s % KC, ring[s]);
     });
 
-    // threshold table and bias to LDS while those loads are in flight
-    if (ACT >= 0)
-        tbl[tid] = pw_kernarg_table(tid);
+    // bias to LDS while those loads are in flight
     for (int i = tid; i < (RG ? q.groups * (32 * MT) : q.OC); i += PW_THREADS)
         bias_lds[i] = q.bias && i < q.OC ? q.bias[i] : 0;
     __syncthreads();
@@ -172,27 +161,18 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
                 for (int mi = 0; mi < MT; ++mi) {
                     if (RG && (og * MT + mi) * 32 >= q.OC)  // (wave-uniform: a tile of surplus channels)
                         continue;
-                    int r[16];
-                    if (ACT < 0) {
+                    int a[16];
 #pragma unroll
-                        for (int e = 0; e < 16; ++e)
-                            r[e] = requant_conv_rt(q.act, acc[mi][e], q.s_src, q.s_flt, q.s_dst);
-                    } else if (q.aff_d != 0.f) {  // (uniform)
-#pragma unroll
-                        for (int e = 0; e < 16; ++e)
-                            r[e] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(acc[mi][e], q.aff_c, q.aff_d);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 16; ++e)
-                            r[e] = requant_conv_table<(ACT < 0 ? 0 : ACT)>(acc[mi][e], q.c, tbl);
-                    }
+                    for (int e = 0; e < 16; ++e)
+                        a[e] = acc[mi][e];
+                    uint32_t d[4];
+                    requant_dwords<ACT>(a, d, q.rq, q.act);
                     if (ok) {
 #pragma unroll
                         for (int e4 = 0; e4 < 4; ++e4) {
                             const int oc4 = og * (8 * MT) + mi * 8 + e4 * 2 + kg;
                             if (!RG || oc4 * 4 < q.OC)
-                                q.dst[obase + oc4 * q.OHW] =
-                                        pack4_perm(r[e4 * 4], r[e4 * 4 + 1], r[e4 * 4 + 2], r[e4 * 4 + 3]);
+                                q.dst[obase + oc4 * q.OHW] = d[e4];
                         }
                     }
                 }
@@ -214,7 +194,6 @@ template <int KC, int ACT>
 __global__ void __launch_bounds__(PW_THREADS) conv_pw_share_kernel(PwParams q) {
     static_assert(KC % 4 == 0, "a quarter of the chunks per wave");
     constexpr int CW = KC / 4;  // chunks a wave fetches per tile
-    __shared__ int tbl[REQUANT_TABLE_ENTRIES];
     __shared__ __attribute__((aligned(16))) int bias_lds[PW_MAX_OC];
     __shared__ __attribute__((aligned(16))) int8_t btile[2][KC * 1024];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -262,8 +241,6 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_share_kernel(PwParams q) {
 
     v4i nxt[CW];
     request(t0, nxt);
-    if (ACT >= 0)
-        tbl[tid] = pw_kernarg_table(tid);
     for (int i = tid; i < q.OC; i += PW_THREADS)
         bias_lds[i] = q.bias ? q.bias[i] : 0;
     park(0, nxt);
@@ -295,26 +272,16 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_share_kernel(PwParams q) {
         const bool ok = p < q.P;
         const int n = fdiv(p, q.dOHW);
         const int obase = n * (q.OC >> 2) * q.OHW + (p - n * q.OHW);
-        int r[16];
-        if (ACT < 0) {
+        int a[16];
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                r[e] = requant_conv_rt(q.act, acc[e], q.s_src, q.s_flt, q.s_dst);
-        } else if (q.aff_d != 0.f) {  // (uniform)
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                r[e] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(acc[e], q.aff_c, q.aff_d);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                r[e] = requant_conv_table<(ACT < 0 ? 0 : ACT)>(acc[e], q.c, tbl);
-        }
+        for (int e = 0; e < 16; ++e)
+            a[e] = acc[e];
+        uint32_t d[4];
+        requant_dwords<ACT>(a, d, q.rq, q.act);
         if (ok) {
 #pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                const int oc4 = og * 8 + e4 * 2 + kg;
-                q.dst[obase + oc4 * q.OHW] = pack4_perm(r[e4 * 4], r[e4 * 4 + 1], r[e4 * 4 + 2], r[e4 * 4 + 3]);
-            }
+            for (int e4 = 0; e4 < 4; ++e4)
+                q.dst[obase + (og * 8 + e4 * 2 + kg) * q.OHW] = d[e4];
         }
         if (t + 1 < tend)
             park(buf ^ 1, nxt);
@@ -372,15 +339,9 @@ TinyNNStatus conv_pw_stream_launch(
     q.image_stride = g.ic * q.OHW;
     q.plane_stride = q.OHW * 4;
     q.act = g.act;
-    q.s_src = g.s_src;
-    q.s_flt = g.s_flt;
-    q.s_dst = g.s_dst;
-    q.c = make_requant_fast(g.s_src, g.s_flt, g.s_dst).c;
     q.dOHW = make_fastdiv(q.OHW);
-    const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
-    if (tab)
-        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
-    const int act = tab ? g.act : -1;
+    q.rq = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
+    const int act = q.rq.mode ? g.act : -1;
 
     const void* kern = nullptr;
 #define MG_PW_PICK_RG(KC_, MT_, RG_)                                                                      \
@@ -419,9 +380,7 @@ TinyNNStatus conv_pw_stream_launch(
                 runs = 1;
             void* sargs[] = {&q};
             note_kernel("conv_pw_share", g.ic / 32);
-            const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
-            q.aff_c = aff.c;
-            q.aff_d = aff.d;
+            note_requant_affine(q.rq.affine());
             hipError_t e = hipLaunchKernel(sk, dim3((unsigned)(runs * gblocks)), dim3(PW_THREADS), sargs, 0, stream());
             MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_pw_share: %s", hipGetErrorString(e));
             return check_launch("conv_pw_share");
@@ -444,9 +403,7 @@ TinyNNStatus conv_pw_stream_launch(
     const unsigned blocks = (unsigned)(waves / 4);
 
     note_kernel("conv_pw_stream", kc, ragged);
-    const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
-    q.aff_c = aff.c;
-    q.aff_d = aff.d;
+    note_requant_affine(q.rq.affine());
     void* args[] = {&q};
     hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(PW_THREADS), args, 0, stream());
     MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_pw_stream: %s", hipGetErrorString(e));

@@ -98,15 +98,10 @@ struct DwChain {
 
 template <int S, int ACT, int R, bool RAGGED, int FUSE = 0>
 __global__ void __launch_bounds__(256) dwconv44_3x3_kernel(
-        ConvGeom g, RequantFast rq, const uint32_t* __restrict__ src, const uint32_t* __restrict__ flt,
+        ConvGeom g, RequantPack rq, const uint32_t* __restrict__ src, const uint32_t* __restrict__ flt,
         const int32_t* __restrict__ bias, uint32_t* __restrict__ dst, int total, int src_bytes,
-        FastDiv d_ogn, FastDiv d_ohn, FastDiv d_c4n, RequantTable table, DwChain fz) {
+        FastDiv d_ogn, FastDiv d_ohn, FastDiv d_c4n, DwChain fz) {
     static_assert(FUSE == 0 || R == 2, "a pooling window is two output rows");
-    __shared__ int tbl[REQUANT_TABLE_ENTRIES];
-    if (ACT >= 0) {
-        tbl[threadIdx.x] = table.t[threadIdx.x];
-        __syncthreads();
-    }
     constexpr int ROWS = (R - 1) * S + 3;   // input rows they need
     const int c4n = g.oc >> 2;
     const int ogn = (g.ow + 3) >> 2;  // groups of 4 output pixels per row
@@ -221,81 +216,58 @@ __global__ void __launch_bounds__(256) dwconv44_3x3_kernel(
                                 acc[orow * 16 + j * 4 + c], false);
             }
         }
-        if (FUSE && ACT >= 0) {
-            // with the threshold table the requantisation is a non-decreasing function of the
-            // accumulator, so max F(a_i) = F(max a_i): pool the int32 accumulators first and requantise
-            // 8 instead of 32 values (the pooled ones land where the code below looks for window k:
-            // row 0, pixel 2 * k; the other three places get the same value)
-            int m[8], f[8];
+        if constexpr (FUSE != 0) {
+            float pooled[8];  // [window][channel], requantised
+            if constexpr (ACT >= 0) {
+                // the requantisation is a non-decreasing function of the
+                // accumulator, so max F(a_i) = F(max a_i): pool the int32 accumulators first and requantise
+                // 8 instead of 32 values
+                int m[8];
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
+                for (int k = 0; k < 2; ++k)
 #pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    m[k * 4 + c] = max(max(acc[(2 * k) * 4 + c], acc[(2 * k + 1) * 4 + c]),
-                                       max(acc[16 + (2 * k) * 4 + c], acc[16 + (2 * k + 1) * 4 + c]));
-            if (rq.aff_d != 0.f) {  // (uniform; one branch around all eight)
+                    for (int c = 0; c < 4; ++c)
+                        m[k * 4 + c] = max(max(acc[(2 * k) * 4 + c], acc[(2 * k + 1) * 4 + c]),
+                                           max(acc[16 + (2 * k) * 4 + c], acc[16 + (2 * k + 1) * 4 + c]));
+                uint32_t d[2];
+                requant_dwords<ACT>(m, d, rq);
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-                    f[i] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(m[i], rq.aff_c, rq.aff_d);
+                    pooled[i] = ACT == MEGCC_NONLINE_RELU ? (float)((d[i >> 2] >> (8 * (i & 3))) & 0xff) : (float)sbyte(d[i >> 2], i & 3);
             } else {
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    f[i] = requant_conv_table<(ACT < 0 ? 0 : ACT)>(m[i], rq.c, tbl);
+                for (int e = 0; e < R * 16; ++e)
+                    acc[e] = requant_conv_rt(g.act, acc[e], g.s_src, g.s_flt, g.s_dst);
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        pooled[k * 4 + c] = (float)max(max(acc[(2 * k) * 4 + c], acc[(2 * k + 1) * 4 + c]),
+                                                       max(acc[16 + (2 * k) * 4 + c], acc[16 + (2 * k + 1) * 4 + c]));
             }
-#pragma unroll
-            for (int k = 0; k < 2; ++k)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    acc[(2 * k) * 4 + c] = acc[(2 * k + 1) * 4 + c] = f[k * 4 + c];
-                    acc[16 + (2 * k) * 4 + c] = acc[16 + (2 * k + 1) * 4 + c] = f[k * 4 + c];
-                }
-        } else if (ACT < 0) {
-#pragma unroll
-            for (int e = 0; e < R * 16; ++e)
-                acc[e] = requant_conv_rt(g.act, acc[e], g.s_src, g.s_flt, g.s_dst);
-        } else if (rq.aff_d != 0.f) {  // (uniform)
-#pragma unroll
-            for (int e = 0; e < R * 16; ++e)
-                acc[e] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(acc[e], rq.aff_c, rq.aff_d);
-        } else {
-#pragma unroll
-            for (int e = 0; e < R * 16; ++e)
-                acc[e] = requant_conv_table<(ACT < 0 ? 0 : ACT)>(acc[e], rq.c, tbl);
-        }
-        if (FUSE) {
             const int py = oh >> 1;  // (oh is even: R = 2)
             if (py < fz.poh) {
                 const size_t row = ((size_t)(n * c4n + c4) * fz.poh + py) * fz.pow;
+                float sum[8];
 #pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const int px = og * 2 + k;
-                    if (px >= fz.pow)
-                        break;
-                    const uint32_t b4 = other4[k];
-                    int r[4];
+                for (int i = 0; i < 8; ++i)
+                    sum[i] = fz.s_a * pooled[i] + fz.s_b * (float)sbyte(other4[i >> 2], i & 3);
+                uint32_t res[2];
+                requant_sums<FUSE == 2>(sum, res, fz.sdiv);
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const int m0 = max(acc[(2 * k) * 4 + c], acc[(2 * k + 1) * 4 + c]);
-                        const int m1 = max(acc[16 + (2 * k) * 4 + c], acc[16 + (2 * k + 1) * 4 + c]);
-                        const float v0 = fz.s_a * (float)max(m0, m1);
-                        const float v1 = fz.s_b * (float)sbyte(b4, c);
-                        const float sum = v0 + v1;
-                        r[c] = fp32_to_int8((FUSE == 2 ? (sum > 0 ? sum : 0) : sum) * fz.sdiv);
-                    }
-                    dst[row + px] = pack4_perm(r[0], r[1], r[2], r[3]);
-                }
+                for (int k = 0; k < 2; ++k)
+                    if (og * 2 + k < fz.pow)
+                        dst[row + og * 2 + k] = res[k];
             }
             continue;
         }
+        uint32_t out4[R * 4];
+        requant_dwords<ACT>(acc, out4, rq, g.act);
 #pragma unroll
         for (int orow = 0; orow < R; ++orow) {
             if (oh + orow >= g.oh)
                 break;
-            uint32_t o[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                o[j] = pack4_perm(acc[orow * 16 + j * 4], acc[orow * 16 + j * 4 + 1],
-                                  acc[orow * 16 + j * 4 + 2], acc[orow * 16 + j * 4 + 3]);
+            const uint32_t* const o = out4 + 4 * orow;
             uint32_t* out = dst + ((size_t)(n * c4n + c4) * g.oh + oh + orow) * g.ow + og * 4;
             if (og * 4 + 4 <= g.ow && (g.ow & 3) == 0) {
                 *(uint4*)out = make_uint4(o[0], o[1], o[2], o[3]);
@@ -342,15 +314,10 @@ TinyNNStatus dwconv44_chain_launch(
     if (groups4 == 0)
         return TinyNN_SUCCESS;
     const unsigned nb = (unsigned)((groups4 + 255) / 256);
-    RequantFast rq3 = make_requant_fast(g.s_src, g.s_flt, g.s_dst);
-    const bool tab = (g.act == MEGCC_NONLINE_IDENTITY || g.act == MEGCC_NONLINE_RELU) &&
-                     requant_table_ok(g.s_src, g.s_flt, g.s_dst);
-    static const RequantTable no_table = {};
-    std::shared_ptr<const RequantTable> kept;
-    const RequantTable& table = tab ? *(kept = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst)) : no_table;
-    const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
-    rq3.aff_c = aff.c;
-    rq3.aff_d = aff.d;
+    // (anything but IDENTITY / RELU by the literal sequence)
+    const RequantPack rq3 = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
+    const bool tab = rq3.mode != 0 && (g.act == MEGCC_NONLINE_IDENTITY || g.act == MEGCC_NONLINE_RELU);
+    note_requant_affine(rq3.affine());
     DwChain fz;
     fz.other = (const uint32_t*)other;
     fz.poh = g.oh / 2;
@@ -358,8 +325,8 @@ TinyNNStatus dwconv44_chain_launch(
     fz.s_a = g.s_dst;
     fz.s_b = s_other;
     fz.sdiv = 1.f / s_out;
-    void (*k)(ConvGeom, RequantFast, const uint32_t*, const uint32_t*, const int32_t*, uint32_t*, int, int, FastDiv,
-              FastDiv, FastDiv, RequantTable, DwChain);
+    void (*k)(ConvGeom, RequantPack, const uint32_t*, const uint32_t*, const int32_t*, uint32_t*, int, int, FastDiv,
+              FastDiv, FastDiv, DwChain);
 #define MG_DWC_ACT(S_, G_, F_)                                                                             \
     (tab && g.act == MEGCC_NONLINE_IDENTITY ? dwconv44_3x3_kernel<S_, MEGCC_NONLINE_IDENTITY, 2, G_, F_>     \
      : tab && g.act == MEGCC_NONLINE_RELU   ? dwconv44_3x3_kernel<S_, MEGCC_NONLINE_RELU, 2, G_, F_>         \
@@ -374,8 +341,7 @@ TinyNNStatus dwconv44_chain_launch(
 #undef MG_DWC_ACT
     hipLaunchKernelGGL(k, dim3(nb), dim3(256), 0, stream(), g, rq3, (const uint32_t*)src, (const uint32_t*)flt,
                        (const int32_t*)bias, (uint32_t*)dst, groups4, (int)((long)g.n * g.ic * g.ih * g.iw),
-                       make_fastdiv((g.ow + 3) / 4), make_fastdiv((g.oh + R - 1) / R), make_fastdiv(g.oc >> 2), table,
-                       fz);
+                       make_fastdiv((g.ow + 3) / 4), make_fastdiv((g.oh + R - 1) / R), make_fastdiv(g.oc >> 2), fz);
     return check_launch("dwconv44_chain");
 }
 
@@ -423,18 +389,11 @@ TinyNNStatus dwconv44_launch(
         const int R = shape & 15;
         const int groups4 = (int)((long)g.n * (g.oc >> 2) * ((g.oh + R - 1) / R) * ((g.ow + 3) / 4));
         unsigned nb = (unsigned)((groups4 + 255) / 256);
-        RequantFast rq3 = make_requant_fast(g.s_src, g.s_flt, g.s_dst);
-        void (*k3)(ConvGeom, RequantFast, const uint32_t*, const uint32_t*, const int32_t*, uint32_t*, int, int,
-                   FastDiv, FastDiv, FastDiv, RequantTable, DwChain);
-        // exact thresholds for the monotone activations; anything else (and extreme scales)
-        // evaluates the literal sequence per output
-        const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
-        static const RequantTable no_table = {};
-        std::shared_ptr<const RequantTable> kept;
-    const RequantTable& table = tab ? *(kept = requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst)) : no_table;
-        const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
-        rq3.aff_c = aff.c;
-        rq3.aff_d = aff.d;
+        void (*k3)(ConvGeom, RequantPack, const uint32_t*, const uint32_t*, const int32_t*, uint32_t*, int, int,
+                   FastDiv, FastDiv, FastDiv, DwChain);
+        const RequantPack rq3 = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
+        const bool tab = rq3.mode != 0;
+        note_requant_affine(rq3.affine());
 #define MG_DW_PICK(S_, R_, G_)                                                                      \
     (tab && g.act == MEGCC_NONLINE_IDENTITY ? dwconv44_3x3_kernel<S_, MEGCC_NONLINE_IDENTITY, R_, G_> \
      : tab && g.act == MEGCC_NONLINE_RELU   ? dwconv44_3x3_kernel<S_, MEGCC_NONLINE_RELU, R_, G_>     \
@@ -451,7 +410,7 @@ TinyNNStatus dwconv44_launch(
         hipLaunchKernelGGL(k3, dim3(nb), dim3(256), 0, stream(), g, rq3, (const uint32_t*)src,
                            (const uint32_t*)flt, (const int32_t*)bias, (uint32_t*)dst, groups4,
                            (int)((long)g.n * g.ic * g.ih * g.iw), make_fastdiv((g.ow + 3) / 4),
-                           make_fastdiv((g.oh + R - 1) / R), make_fastdiv(g.oc >> 2), table, DwChain{});
+                           make_fastdiv((g.oh + R - 1) / R), make_fastdiv(g.oc >> 2), DwChain{});
         return check_launch("dwconv44_3x3");
     }
     unsigned blocks = (unsigned)((total + 255) / 256);

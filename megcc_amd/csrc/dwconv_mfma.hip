@@ -62,15 +62,14 @@ struct DwMfmaParams {
     int xblocks;           // ceil(OW / 8)
     int tiles;             // per plane set: ceil(cols / 32)
     int act;
-    float s_src, s_flt, s_dst, c;
-    float aff_c, aff_d;   // requantisation by one fused multiply-add (epilogue.h); aff_d == 0: table
+    float s_src, s_flt, s_dst;
+    RequantPack rq;
     FastDiv d_ohp, d_xb;  // division by ohp, by xblocks
     // FUSE: the second operand of the addition that follows the pooling ([N][C/4][poh][pow] dwords), the
     // extent of the pooled tensor, the scales of the pooled operand and of `other`, 1 / the result's
     const uint32_t* other;
     int poh, pow;
     float s_a, s_b, sdiv;
-    RequantTable table;
 };
 
 struct DwMfmaChain {
@@ -95,7 +94,7 @@ typedef unsigned dw_v4u __attribute__((ext_vector_type(4)));
 // S: stride (only 1 is instantiated: with stride 2 the layer reads four bytes per byte written and
 // the v_dot4 kernel of dwconv.hip already runs at the rate of a copy - measured 7.8 us against
 // 9.8 us for this one on N=64 C=32 112x112). RAGGED: IW is not a multiple of 4, so the last 16-byte load of a row runs into the
-// next row and is masked. ACT: IDENTITY / RELU / H_SWISH use the threshold table, -1 evaluates the literal
+// next row and is masked. ACT: as in requant_dwords, -1 evaluates the literal
 // sequence with the run-time activation. F: filter rows = filter columns (3, 5 or 7; pad F / 2).
 template <int S, bool RAGGED, int ACT, int F = 3, int R = 1, int FUSE = 0>
 __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
@@ -104,7 +103,6 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
     constexpr int PAD = F / 2;
     constexpr int NS = S + 1;            // K steps a group of 8 output pixels reads
     constexpr int IR = (R - 1) * S + F;  // input rows they read
-    __shared__ int tbl[REQUANT_TABLE_ENTRIES];
     const int tid = threadIdx.x, lane = tid & 63;
     const int col_l = lane & 31, kg = lane >> 5;
     // Workgroups are handed to the 8 XCDs in turn and every XCD has an L2 of its own: workgroup b
@@ -200,16 +198,9 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
         return w;
     };
 
-    // Order of the set-up: threshold table to LDS (one barrier), then the first tile's rows are
-    // requested, then the banded matrices are built while those loads fly. (Requesting the rows
-    // before the table copy made the barrier wait for them: 5 - 8 % slower on 14 x 14 and 112 x 112
-    // maps alike.)
+    // Order of the set-up: the first tile's rows are requested, then the banded matrices are built while those loads fly.
     v4i B[IR][NS];
     int tile = t_begin;
-    if (ACT >= 0) {
-        tbl[tid] = q.table.t[tid];
-        __syncthreads();
-    }
     Where next = request(tile < t_end ? tile : q.tiles, B);
     // ---- the banded weight matrices of this plane set -------------------------------------------
     // row m = lane & 31 = (output pixel m / 4, channel m % 4); the lane's 16 K bytes are input
@@ -269,40 +260,33 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
         next = request(tile + 1 < t_end ? tile + 1 : q.tiles, B);
         if constexpr (FUSE != 0) {
             // ---- pool, requantise, add, store ----------------------------------------------------
-            // With the threshold table the requantisation F is a non-decreasing function of the
+            // The requantisation F is a non-decreasing function of the
             // accumulator (epilogue.h), so max F(a_i) = F(max a_i): the maximum is taken over the
             // int32 accumulators and 8 instead of 32 values per lane are requantised. The literal
             // sequence (SIGMOID, extreme scales) requantises first.
-            int pooled[2][4];  // [window of this lane][channel], requantised
+            float pooled[2][4];  // [window of this lane][channel], requantised
             if (ACT >= 0) {
                 int v[16];  // vertical maximum: pixel 2 * (e / 4) + kg, channel e % 4
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
                     v[e] = max(acc[0][e], acc[1][e]);
                 // lower half wave: both halves of windows 0 and 1; upper: of windows 2 and 3
-                int w0[4], w1[4];  // the windows' maxima over the accumulators
+                int w[8];  // the windows' maxima over the accumulators
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     const dwm_v2u s02 = __builtin_amdgcn_permlane32_swap((unsigned)v[c], (unsigned)v[8 + c], false, false);
                     const dwm_v2u s13 = __builtin_amdgcn_permlane32_swap((unsigned)v[4 + c], (unsigned)v[12 + c], false, false);
-                    w0[c] = max((int)s02[0], (int)s02[1]);
-                    w1[c] = max((int)s13[0], (int)s13[1]);
+                    w[c] = max((int)s02[0], (int)s02[1]);
+                    w[4 + c] = max((int)s13[0], (int)s13[1]);
                 }
-                // (one uniform branch around all eight, so that the look-ups of the table form stay in
-                //  flight together)
-                if (q.aff_d != 0.f) {
+                uint32_t d[2];
+                requant_dwords<ACT>(w, d, q.rq);
+                // (never negative with RELU: the conversion takes any unsigned byte of a register)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        pooled[0][c] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(w0[c], q.aff_c, q.aff_d);
-                        pooled[1][c] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(w1[c], q.aff_c, q.aff_d);
-                    }
-                } else {
+                for (int k = 0; k < 2; ++k)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        pooled[0][c] = requant_conv_table<(ACT < 0 ? 0 : ACT)>(w0[c], q.c, tbl);
-                        pooled[1][c] = requant_conv_table<(ACT < 0 ? 0 : ACT)>(w1[c], q.c, tbl);
-                    }
-                }
+                    for (int c = 0; c < 4; ++c)
+                        pooled[k][c] = ACT == MEGCC_NONLINE_RELU ? (float)((d[k] >> (8 * c)) & 0xff) : (float)sbyte(d[k], c);
             } else {
                 unsigned d[4];  // vertical maximum of pixel 2 * j + kg, 4 requantised channel bytes
 #pragma unroll
@@ -318,24 +302,19 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
                 const dwm_v2u s13 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    pooled[0][c] = max(sbyte(s02[0], c), sbyte(s02[1], c));
-                    pooled[1][c] = max(sbyte(s13[0], c), sbyte(s13[1], c));
+                    pooled[0][c] = (float)max(sbyte(s02[0], c), sbyte(s02[1], c));
+                    pooled[1][c] = (float)max(sbyte(s13[0], c), sbyte(s13[1], c));
                 }
             }
-            dwm_v2u out;
+            float sum[8];
 #pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const uint32_t b4 = cur.b4[k];
-                int r4[4];
+            for (int k = 0; k < 2; ++k)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const float v0 = q.s_a * (float)pooled[k][c];
-                    const float v1 = q.s_b * (float)sbyte(b4, c);
-                    const float sum = v0 + v1;
-                    r4[c] = fp32_to_int8((FUSE == 2 ? (sum > 0 ? sum : 0) : sum) * q.sdiv);
-                }
-                out[k] = pack4_perm(r4[0], r4[1], r4[2], r4[3]);
-            }
+                for (int c = 0; c < 4; ++c)
+                    sum[4 * k + c] = q.s_a * pooled[k][c] + q.s_b * (float)sbyte(cur.b4[k], c);
+            uint32_t res[2];
+            requant_sums<FUSE == 2>(sum, res, q.sdiv);
+            const dwm_v2u out = {res[0], res[1]};
             if ((q.pow & 1) == 0) {
                 __builtin_amdgcn_raw_buffer_store_b64(out, rd, cur.pleft > 0 ? cur.pidx * 4 : OOB, 0, 0);
             } else {
@@ -348,24 +327,12 @@ __global__ void __launch_bounds__(256) dwconv44_mfma_kernel(DwMfmaParams q) {
         // ---- requantise, pack, exchange, store ---------------------------------------------------
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            int o[16];
-            if (ACT < 0) {
+            int a[16];
 #pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    o[e] = requant_conv_rt(q.act, acc[r][e], q.s_src, q.s_flt, q.s_dst);
-            } else if (q.aff_d != 0.f) {  // (uniform)
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    o[e] = requant_conv_affine<(ACT == MEGCC_NONLINE_RELU ? ACT : 0)>(acc[r][e], q.aff_c, q.aff_d);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    o[e] = requant_conv_table<(ACT < 0 ? 0 : ACT)>(acc[r][e], q.c, tbl);
-            }
-            unsigned d[4];  // pixel 2 * j + kg
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                d[j] = pack4_perm(o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]);
+            for (int e = 0; e < 16; ++e)
+                a[e] = acc[r][e];
+            uint32_t d[4];  // pixel 2 * j + kg
+            requant_dwords<ACT>(a, d, q.rq, q.act);
             // lower half wave: pixels 0 2 4 6, upper: 1 3 5 7  ->  lower 0 1 2 3, upper 4 5 6 7
             const dwm_v2u s02 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
             const dwm_v2u s13 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
@@ -425,19 +392,13 @@ static TinyNNStatus dwconv44_mfma_run(
     q.s_src = g.s_src;
     q.s_flt = g.s_flt;
     q.s_dst = g.s_dst;
-    q.c = make_requant_fast(g.s_src, g.s_flt, g.s_dst).c;
+    q.rq = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
     q.d_ohp = make_fastdiv(q.ohp);
     q.d_xb = make_fastdiv(q.xblocks);
     if ((long)q.tiles * q.c4n == 0)
         return TinyNN_SUCCESS;
-    const bool tab = requant_table_act(g.act) && requant_table_ok(g.s_src, g.s_flt, g.s_dst);
-    if (tab)
-        q.table = *requant_table_for(g.act, g.s_src, g.s_flt, g.s_dst);
-    const int act = tab ? g.act : -1;
-    // (the chain kernel has no table instantiation for H_SWISH: the pair is only asked for where one runs)
-    const RequantAffine aff = requant_affine_pick(tab, g.act, g.s_src, g.s_flt, g.s_dst);
-    q.aff_c = aff.c;
-    q.aff_d = aff.d;
+    const int act = q.rq.mode ? g.act : -1;
+    note_requant_affine(q.rq.affine());
     const bool ragged = (g.iw & 3) != 0;
     const void* kern = nullptr;
 #define MG_DWM_ACT(S_, R_, F_)                                                                        \
@@ -447,7 +408,7 @@ static TinyNNStatus dwconv44_mfma_run(
                                    : (const void*)dwconv44_mfma_kernel<S_, R_, -1, F_>)
 #define MG_DWM_F(S_, F_) (ragged ? MG_DWM_ACT(S_, true, F_) : MG_DWM_ACT(S_, false, F_))
     if (chain) {
-        // (IDENTITY / RELU through the table, anything else the literal sequence)
+        // (anything but IDENTITY / RELU by the literal sequence)
         const int a2 = act == MEGCC_NONLINE_H_SWISH ? -1 : act;
 #define MG_DWM_CHAIN(R_, FZ_)                                                                                  \
     (a2 == MEGCC_NONLINE_IDENTITY ? (const void*)dwconv44_mfma_kernel<1, R_, MEGCC_NONLINE_IDENTITY, 3, 2, FZ_> \

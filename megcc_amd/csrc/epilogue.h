@@ -228,51 +228,166 @@ __device__ __forceinline__ int requant_conv_affine(int acc, float c, float d) {
     return m < LO ? LO : (m > 127 ? 127 : m);
 }
 
-// ---- four outputs at a time: scale, round, saturate and pack in one conversion ---------------------
+// bytes 0 of a, b, c, d -> one dword
+__device__ __forceinline__ uint32_t pack4_perm(int a, int b, int c, int d) {
+    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)b, (uint32_t)a, 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)c, 0x0c0c0400u);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
+// ---- four outputs at a time, without a table ------------------------------------------------------
 // v_cvt_pk_u8_f32 rounds to nearest (ties to even), saturates to 0..255 and puts the byte where it
-// belongs, which makes the floor, the clamp and the byte shuffling of the forms above unnecessary: 3
-// instructions per output and 1 / 2 per four of them. In RELU's case the byte is 2 out (+ 1): 0..255 covers
-// 0..127.5, and the one bit that is dropped afterwards turns the rounding into a floor; in IDENTITY's it
-// is out + 128. The value converted is
+// belongs, which makes the floor, the clamp and the byte shuffling of the forms above unnecessary. In RELU's
+// (and H_SWISH's) case the byte is 2 out (+ 1): 0..255 covers 0..127.5, and the one bit that is dropped
+// afterwards turns the rounding into a floor; in IDENTITY's it is out + 128. The value converted is
 //     mode 1: fma((float)a, c, d)              mode 2: fma(((float)a * s1) * s2, c, d)
 // - mode 2 repeats the reference's own first two roundings (or one of them: s2 = 1) and finds constants
 // where mode 1 has none (many input channels: c is small, and so is the room between the steps). All of
 // it is non-decreasing in a, so it equals the reference on all of int32 iff it does on both sides of each
-// of its steps: the host search (requant_table.hip) checks exactly that. Scales with exact ties whose
-// roundings land on either side have no such constants (mode 0) and keep the table.
+// of its steps: the host search (requant_table.hip) checks exactly that. (IDENTITY has no mode 2.)
+//     mode 4 (IDENTITY): requant_conv_affine's pair, which more scales have - the 128 cost the sum one bit.
+//     mode 3: the reference's own sequence, for scales with exact ties whose roundings land on either side and for
+// H_SWISH. Its division costs two instructions: with c + d the 48-bit reciprocal of s_dst, v = fma(x, c, x d) is
+// the quotient to 2^-47 before its one rounding, so it is the correctly rounded one but for quotients that close
+// to halfway between two floats, where it is the float on the other side; the host checks every accumulator
+// whose output that could change. Half away from zero is then exact for every float: truncation of v plus the
+// largest float below a half, and for outputs that are never negative the conversion of 2 v plus that float
+// (ties to even: 2 v + 0.5 of v = k + 0.5 is 2 k + 1.5, which goes to the even 2 k + 2).
+// Vector instructions for four outputs: 14, 18 - 22, 19, and mode 3 30 (RELU), 39 (IDENTITY), 46 (H_SWISH); the
+// threshold table's look-ups took 35 (H_SWISH 51) and four gathers from LDS, and its 1 KB among a launch's
+// arguments 0.7 us of the host's time.
+// (mode 0: none of these was proven; s1, s2, c are then the reference's three scales, for requant_conv)
 struct RequantPack {
     float s1, s2, c, d;
     int mode;
+    bool affine() const { return mode != 0 && mode != 3; }
 };
-// (whatever the switch "noaffine" says: the caller asks it)
-RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst);
+// `affine`: any mode, else 3 or 0
+RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst, bool affine);
+// what a launch uses: modes 1, 2 and 4 unless the switch "noaffine" is on (a launch with them is noted as "+affine")
+RequantPack requant_pack_pick(int act, float s_src, float s_flt, float s_dst);
 
 // MODE, ACT compile-time; channels (or pixels) 0..3 of one dword
 template <int MODE, int ACT>
 __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3, const RequantPack& q) {
     const int a[4] = {a0, a1, a2, a3};
     uint32_t r = 0;
+    if constexpr (MODE == 3) {
+        constexpr float HALF = 0x1.fffffep-2f;
+        int o[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        float x = (float)a[i];
-        if (MODE == 2)
-            x = x * q.s1 * q.s2;
-        r = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(x, q.c, q.d), i, r);
+        for (int i = 0; i < 4; ++i) {
+            const float x = (float)a[i] * q.s1 * q.s2;
+            float v = __builtin_fmaf(x, q.c, x * q.d);  // (RELU: twice the quotient)
+            if (ACT == MEGCC_NONLINE_IDENTITY) {
+                const int t = cvt_i32(v + __builtin_copysignf(HALF, v));
+                o[i] = t > 127 ? 127 : (t < -128 ? -128 : t);
+                continue;
+            }
+            if (ACT == MEGCC_NONLINE_H_SWISH)
+                v = v * __builtin_amdgcn_fmed3f(v + 3, 0.f, 6.f) * (2.f * (1.f / 6.f));
+            r = __builtin_amdgcn_cvt_pk_u8_f32(v + HALF, i, r);
+        }
+        if (ACT == MEGCC_NONLINE_IDENTITY)
+            return pack4_perm(o[0], o[1], o[2], o[3]);
+        return (r >> 1) & 0x7f7f7f7fu;
+    } else if constexpr (MODE == 4) {
+        int o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o[i] = requant_conv_affine<ACT>(a[i], q.c, q.d);
+        return pack4_perm(o[0], o[1], o[2], o[3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float x = (float)a[i];
+            if (MODE == 2)
+                x = x * q.s1 * q.s2;
+            r = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(x, q.c, q.d), i, r);
+        }
+        return ACT == MEGCC_NONLINE_RELU ? (r >> 1) & 0x7f7f7f7fu : r ^ 0x80808080u;
     }
-    return ACT == MEGCC_NONLINE_RELU ? (r >> 1) & 0x7f7f7f7fu : r ^ 0x80808080u;
+}
+
+// N accumulators -> N / 4 dwords (each 4 consecutive ones), the form by a uniform branch. ACT < 0: the literal sequence of
+// `act` (mode 0, SIGMOID), whose scales stand where mode 0 has them.
+// The empty volatile statements keep each form inside its branch: the compiler otherwise computes one of
+// them ahead of the branch and throws it away, 80 instructions of 120.
+template <int ACT, int N>
+__device__ __forceinline__ void requant_dwords(int (&a)[N], uint32_t (&out)[N / 4], const RequantPack& q, int act = ACT) {
+    auto here = [&]() __attribute__((always_inline)) {
+#ifndef MG_HOST_AUDIT
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            asm volatile("" : "+v"(a[i]));
+#endif
+    };
+    if constexpr (ACT < 0) {
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i) {
+            int r[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                r[e] = requant_conv_rt(act, a[4 * i + e], q.s1, q.s2, q.c);
+            out[i] = pack4_perm(r[0], r[1], r[2], r[3]);
+        }
+    } else if constexpr (ACT == MEGCC_NONLINE_H_SWISH) {
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i)
+            out[i] = requant_pack4<3, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+    } else if (q.mode == 1) {  // (uniform)
+        here();
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i)
+            out[i] = requant_pack4<1, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+    } else if (ACT == MEGCC_NONLINE_RELU ? q.mode == 2 : q.mode == 4) {
+        here();
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i)
+            out[i] = requant_pack4<ACT == MEGCC_NONLINE_RELU ? 2 : 4, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+    } else {
+        here();
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i)
+            out[i] = requant_pack4<3, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+    }
+}
+
+// fp32_to_int8(sum * sdiv) (RELU: of max(sum, 0) * sdiv) of 4 N sums, QADD's and QFUSE_ADD_RELU's last step (elemwise.hip). RELU's
+// is never negative where sdiv is not, and the conversion above serves: 3 vector instructions a value for 6.
+template <bool RELU, int N>
+__device__ __forceinline__ void requant_sums(float (&sum)[4 * N], uint32_t (&out)[N], float sdiv) {
+    if (RELU && (int)__builtin_bit_cast(unsigned, sdiv) > 0) {  // (uniform; the sign and what is no number, without a vector compare)
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            uint32_t r = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#ifndef MG_HOST_AUDIT
+                asm volatile("" : "+v"(sum[4 * i + e]));  // (as in requant_dwords)
+#endif
+                r = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(sum[4 * i + e] * sdiv, 2.f, 0x1.fffffep-2f), e, r);
+            }
+            out[i] = (r >> 1) & 0x7f7f7f7fu;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            int r[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float s = sum[4 * i + e];
+                r[e] = fp32_to_int8((RELU ? (s > 0 ? s : 0) : s) * sdiv);
+            }
+            out[i] = pack4_perm(r[0], r[1], r[2], r[3]);
+        }
+    }
 }
 
 // host side: the estimate above is valid (else kernels use the literal sequence per element)
 static inline bool requant_table_ok(float s_src, float s_flt, float s_dst) {
     const RequantFast q = make_requant_fast(s_src, s_flt, s_dst);
     return q.c != 0.f && q.c * 2147483648.f > 1000.f;
-}
-
-// bytes 0 of a, b, c, d -> one dword
-__device__ __forceinline__ uint32_t pack4_perm(int a, int b, int c, int d) {
-    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)b, (uint32_t)a, 0x0c0c0400u);
-    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)c, 0x0c0c0400u);
-    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 }
 
 __device__ __forceinline__ uint32_t pack4(int a, int b, int c, int d) {

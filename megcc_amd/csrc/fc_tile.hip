@@ -34,8 +34,7 @@ struct FcTileParams {
     unsigned last16;     // offset of the last 16 bytes of src
     int M, K, OC, OCP, nblk;  // nblk: blocks of 128 bytes of K
     int act;
-    float s_src, s_flt, s_dst;
-    RequantFast rq;
+    RequantPack rq;
     XcdOrder xo;  // tile order (set at launch from the grid)
 };
 
@@ -186,16 +185,13 @@ __global__ void __launch_bounds__(256 * KW) fc_tile_kernel(FcTileParams q) {
                     bv[e] = q.bias ? q.bias[min(oc + e, q.OC - 1)] : 0;
 #pragma unroll
                 for (int ni = 0; ni < NT; ++ni) {
-                    int r[4];
+                    int a[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int a = acc[mi][ni][e4 * 4 + e] + bv[e];
-                        if constexpr (ACT < 0)
-                            r[e] = requant_conv_rt(q.act, a, q.s_src, q.s_flt, q.s_dst);
-                        else
-                            r[e] = requant_conv_fast<ACT>(a, q.rq);
-                    }
-                    *(uint32_t*)(lds + (wn * (32 * NT) + ni * 32 + col) * OPITCH + ocl) = pack4_perm(r[0], r[1], r[2], r[3]);
+                    for (int e = 0; e < 4; ++e)
+                        a[e] = acc[mi][ni][e4 * 4 + e] + bv[e];
+                    uint32_t d[1];
+                    requant_dwords<ACT>(a, d, q.rq, q.act);
+                    *(uint32_t*)(lds + (wn * (32 * NT) + ni * 32 + col) * OPITCH + ocl) = d[0];
                 }
             }
     }
@@ -236,20 +232,18 @@ TinyNNStatus fc_tile_launch(const ConvGeom& g, const void* src, const void* pack
     q.OCP = (g.oc + OC_PAD - 1) / OC_PAD * OC_PAD;
     q.nblk = (g.ic + 127) / 128;
     q.act = g.act;
-    q.s_src = g.s_src;
-    q.s_flt = g.s_flt;
-    q.s_dst = g.s_dst;
-    q.rq = make_requant_fast(g.s_src, g.s_flt, g.s_dst);
+    q.rq = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
     // 128 x 128 tiles where they give every CU one; else 64 x 64, with up to four groups of waves sharing
     // K while the groups still have a block each and the chip is not full
     const long big = (long)((g.n + 127) / 128) * ((g.oc + 127) / 128);
     const long small = (long)((g.n + 63) / 64) * ((g.oc + 63) / 64);
     const bool wide = big >= num_cus();
     const int kw = wide || small >= 2L * num_cus() || q.nblk < 2 ? 1 : small >= num_cus() || q.nblk < 4 ? 2 : 4;
-    const int act = g.act == MEGCC_NONLINE_IDENTITY || g.act == MEGCC_NONLINE_RELU ? g.act : -1;
+    const int act = q.rq.mode ? g.act : -1;
 #define MG_FCT(MT_, NT_, KW_)                                                                        \
     (act == MEGCC_NONLINE_IDENTITY ? fc_tile_kernel<MT_, NT_, KW_, MEGCC_NONLINE_IDENTITY>           \
      : act == MEGCC_NONLINE_RELU   ? fc_tile_kernel<MT_, NT_, KW_, MEGCC_NONLINE_RELU>               \
+     : act == MEGCC_NONLINE_H_SWISH ? fc_tile_kernel<MT_, NT_, KW_, MEGCC_NONLINE_H_SWISH>           \
                                    : fc_tile_kernel<MT_, NT_, KW_, -1>)
     void (*kern)(FcTileParams) = wide ? MG_FCT(2, 2, 1) : kw == 1 ? MG_FCT(1, 1, 1) : kw == 2 ? MG_FCT(1, 1, 2) : MG_FCT(1, 1, 4);
 #undef MG_FCT
@@ -257,6 +251,7 @@ TinyNNStatus fc_tile_launch(const ConvGeom& g, const void* src, const void* pack
     const dim3 grid((g.oc + b - 1) / b, (g.n + b - 1) / b);
     q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y, (long)(q.M + q.OC) * q.K);
     note_kernel(q.xo.w ? "fc_tile_xo" : "fc_tile", b, kw);
+    note_requant_affine(q.rq.affine());
     hipLaunchKernelGGL(kern, grid, dim3(256 * kw), 0, stream(), q);
     return check_launch("fc_tile");
 }

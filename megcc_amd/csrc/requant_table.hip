@@ -156,32 +156,60 @@ static RequantSteps requant_steps(const RequantTable& T, int lo) {
     return s;
 }
 
-// lower and upper bounds for d: at[i] - x[i] c <= d, and <= for the upper ones (the largest of the lower, the smallest of
-// the upper; four chains, since one would wait for each comparison)
+// Lower (or upper) bounds for d: at[i] - x[i] c <= d (>=), of which the largest (smallest) counts for a given c. Bounds come in
+// the order of x, and those that are the tightest for no c at all are dropped as they come: what stays is one side of the
+// points' convex hull, a dozen of 255, and a slope costs as many products. (All 255 kept, the searches below took 40 us.)
+template <bool LOWER>
 struct RequantBounds {
     int n = 0;
-    double x[2 * REQUANT_TABLE_ENTRIES + 2], at[2 * REQUANT_TABLE_ENTRIES + 2];
-    void add(double v, double bound) {
+    double x[REQUANT_TABLE_ENTRIES], at[REQUANT_TABLE_ENTRIES];
+    int point[REQUANT_TABLE_ENTRIES];  // which step's
+    static bool tighter(double a, double b) { return LOWER ? a > b : a < b; }
+    void add(double v, double bound, int p) {
+        if (n && x[n - 1] == v) {
+            if (!tighter(bound, at[n - 1]))
+                return;
+            --n;
+        }
+        // (the last one is not beyond the line from the one before it to this one)
+        while (n >= 2 && !tighter((at[n - 1] - at[n - 2]) * (v - x[n - 2]), (bound - at[n - 2]) * (x[n - 1] - x[n - 2])))
+            --n;
         x[n] = v;
-        at[n++] = bound;
+        at[n] = bound;
+        point[n++] = p;
     }
-    template <bool LOWER>
     double tightest(double c) const {
-        const double none = LOWER ? -1e30 : 1e30;
-        double m[4] = {none, none, none, none};
-        auto take = [&](int j, int i) {
-            const double v = at[i] - x[i] * c;
-            m[j] = (LOWER ? v > m[j] : v < m[j]) ? v : m[j];
-        };
-        int i = 0;
-        for (; i + 4 <= n; i += 4)
-            for (int j = 0; j < 4; ++j)
-                take(j, i + j);
-        for (; i < n; ++i)
-            take(0, i);
-        return LOWER ? std::max(std::max(m[0], m[1]), std::max(m[2], m[3])) : std::min(std::min(m[0], m[1]), std::min(m[2], m[3]));
+        double m = LOWER ? -1e30 : 1e30;
+        for (int i = 0; i < n; ++i)
+            if (tighter(at[i] - x[i] * c, m))
+                m = at[i] - x[i] * c;
+        return m;
     }
 };
+
+// the float `n` floats above (a positive, normal) v
+static float by_ulps(float v, int n) {
+    uint32_t u;
+    memcpy(&u, &v, 4);
+    u += (uint32_t)n;
+    memcpy(&v, &u, 4);
+    return v;
+}
+
+// whether `eval` gives the outputs of every step: first where the bounds are tightest, where a wrong candidate shows
+template <typename F>
+static bool requant_verified(const RequantSteps& pts, const RequantBounds<true>& from, const RequantBounds<false>& to, F eval) {
+    for (int i = 0; i < from.n; ++i)
+        if (eval(pts.a[from.point[i]]) != pts.y[from.point[i]])
+            return false;
+    for (int i = 0; i < to.n; ++i)
+        if (eval(pts.a[to.point[i]]) != pts.y[to.point[i]])
+            return false;
+    for (int i = 0; i < pts.n; ++i)
+        if (eval(pts.a[i]) != pts.y[i])
+            return false;
+    return true;
+}
 
 // host evaluation of requant_conv_affine (fmaf is the correctly rounded single fused multiply-add,
 // floorf + saturation what v_cvt_flr_i32_f32 does)
@@ -202,20 +230,19 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
         return found;
     const int lo = act == MEGCC_NONLINE_RELU ? 0 : -128;
     const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), lo);
-    RequantBounds from, to;  // floor(a c + d) == y  <=>  y <= a c + d < y + 1
-    for (int i = 0; i < pts.n; ++i) {
+    RequantBounds<true> from;  // floor(a c + d) == y  <=>  y <= a c + d < y + 1
+    RequantBounds<false> to;
+    for (int i = 2; i < pts.n; ++i) {  // (the ends of the range bound nothing)
         if (pts.y[i] > lo)
-            from.add((double)(float)pts.a[i], (double)pts.y[i]);
+            from.add((double)(float)pts.a[i], (double)pts.y[i], i);
         if (pts.y[i] < 127)
-            to.add((double)(float)pts.a[i], (double)pts.y[i] + 1);
+            to.add((double)(float)pts.a[i], (double)pts.y[i] + 1, i);
     }
     const float c0 = make_requant_fast(s_src, s_flt, s_dst).c;
     for (int k = 0; k <= 16 && found.d == 0.f; ++k) {
         // c' = c0 moved (k + 1) / 2 ulps up (k odd) or down (k even)
-        float c = c0;
-        for (int s = 0; s < (k + 1) / 2; ++s)
-            c = nextafterf(c, (k & 1) ? INFINITY : 0.f);
-        const double dlo = from.tightest<true>((double)c), dhi = to.tightest<false>((double)c);
+        const float c = by_ulps(c0, (k & 1) ? (k + 1) / 2 : -(k / 2));
+        const double dlo = from.tightest((double)c), dhi = to.tightest((double)c);
         if (!(dlo < dhi))
             continue;
         // the middle of the interval first (the most room for the rounding of the fused multiply-add),
@@ -225,10 +252,7 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
             const float d = (float)(dlo + (dhi - dlo) * pos);
             if (!(d > 0.f && d < 1.f))
                 continue;
-            bool ok = true;
-            for (int i = 0; i < pts.n && ok; ++i)
-                ok = affine_eval(pts.a[i], c, d, lo) == pts.y[i];
-            if (ok) {
+            if (requant_verified(pts, from, to, [&](int a) { return affine_eval(a, c, d, lo); })) {
                 found = {c, d};
                 break;
             }
@@ -241,26 +265,34 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
 // host evaluation of requant_pack4 for one output
 static int pack_eval(int a, int act, const RequantPack& q) {
     float x = (float)a;
-    if (q.mode == 2)
+    if (q.mode == 2 || q.mode == 3)
         x = x * q.s1 * q.s2;
-    const float r = rintf(fmaf(x, q.c, q.d));  // (round to nearest even: the host's default mode)
+    float y;
+    if (q.mode == 3) {
+        float v = fmaf(x, q.c, x * q.d);
+        if (act == MEGCC_NONLINE_IDENTITY)
+            return fp32_to_int8(v);  // (half away from zero: what the device's form is for every float)
+        if (act == MEGCC_NONLINE_H_SWISH) {
+            const float t = v + 3;
+            v = v * std::min(std::max(t, 0.f), 6.f) * (2.f * (1.f / 6.f));
+        }
+        y = v + 0x1.fffffep-2f;
+    } else {
+        y = fmaf(x, q.c, q.d);
+    }
+    const float r = rintf(y);  // (round to nearest even: the host's default mode)
     const int u = r < 0.f ? 0 : r > 255.f ? 255 : (int)r;
-    return act == MEGCC_NONLINE_RELU ? u >> 1 : u - 128;
+    return act == MEGCC_NONLINE_IDENTITY ? u - 128 : u >> 1;
 }
 
-RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
-    static ScaleCache<RequantPack> cache;
-    const RequantPack none = {0.f, 0.f, 0.f, 0.f, 0};
-    if ((act != MEGCC_NONLINE_IDENTITY && act != MEGCC_NONLINE_RELU) || !requant_table_ok(s_src, s_flt, s_dst))
-        return none;
-    const auto key = cache.key(act, s_src, s_flt, s_dst);
-    RequantPack found = none;
-    if (cache.find(key, &found))
-        return found;
+// Mode 1, 2 or 4, or mode 0 where none has constants.
+static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst) {
+    RequantPack found = {s_src, s_flt, s_dst, 0.f, 0};
     const bool relu = act == MEGCC_NONLINE_RELU;
     const int lowest = relu ? 0 : -128;
     const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), lowest);
-    // the forms in order of cost: no product in front, one, two
+    // the forms in order of cost: no product in front, one, two (IDENTITY, whose outputs are rounded 128 away from zero, hardly
+    // ever has constants for those where it has none without)
     struct Form {
         int mode;
         float s1, s2, c0;
@@ -270,30 +302,28 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
                           {2, s_src, 1.f, s_flt / s_dst * unit},
                           {2, s_src, s_flt, 1.f / s_dst * unit}};
     for (const Form& f : forms) {
-        RequantBounds from, to;  // RELU: 2 y <= rint <= 2 y + 1; IDENTITY: rint == y + 128
-        for (int i = 0; i < pts.n; ++i) {
+        if (f.mode == 2 && !relu)
+            break;
+        RequantBounds<true> from;  // RELU: 2 y <= rint <= 2 y + 1; IDENTITY: rint == y + 128
+        RequantBounds<false> to;
+        for (int i = 2; i < pts.n; ++i) {
             const double x = f.mode == 2 ? (float)pts.a[i] * f.s1 * f.s2 : (float)pts.a[i];
             const int y = pts.y[i];
             if (y > lowest)
-                from.add(x, relu ? 2.0 * y - 0.5 : y + 127.5);
+                from.add(x, relu ? 2.0 * y - 0.5 : y + 127.5, i);
             if (y < 127)
-                to.add(x, relu ? 2.0 * y + 1.5 : y + 128.5);
+                to.add(x, relu ? 2.0 * y + 1.5 : y + 128.5, i);
         }
         for (int k = 0; k <= 48 && !found.mode; ++k) {
             // c = c0 moved (k + 1) / 2 ulps up (k odd) or down (k even)
-            float c = f.c0;
-            for (int s = 0; s < (k + 1) / 2; ++s)
-                c = nextafterf(c, (k & 1) ? INFINITY : 0.f);
-            const double dlo = from.tightest<true>((double)c), dhi = to.tightest<false>((double)c);
+            const float c = by_ulps(f.c0, (k & 1) ? (k + 1) / 2 : -(k / 2));
+            const double dlo = from.tightest((double)c), dhi = to.tightest((double)c);
             if (!(dlo <= dhi))
                 continue;
             static const double kPos[] = {0.5, 0.375, 0.625, 0.25, 0.75, 0.125, 0.875};
             for (double pos : kPos) {
                 const RequantPack q = {f.s1, f.s2, c, (float)(dlo + (dhi - dlo) * pos), f.mode};
-                bool ok = true;
-                for (int i = 0; i < pts.n && ok; ++i)
-                    ok = pack_eval(pts.a[i], act, q) == pts.y[i];
-                if (ok) {
+                if (requant_verified(pts, from, to, [&](int a) { return pack_eval(a, act, q); })) {
                     found = q;
                     break;
                 }
@@ -302,8 +332,64 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst) {
         if (found.mode)
             break;
     }
-    cache.put(key, found);
+    if (!found.mode && !relu) {
+        const RequantAffine a = requant_affine_for(act, s_src, s_flt, s_dst);
+        if (a.d != 0.f)
+            found = {0.f, 0.f, a.c, a.d, 4};
+    }
     return found;
+}
+
+// Mode 3, or mode 0 where it is not proven. The quotient it works with is at most one float from the reference's, so
+// outputs can only differ where the reference's own value is within two of its floats of a step, 2 * 2^-17 for outputs up
+// to 128: accumulators on both sides of each step are compared, and as many beyond them as lie within 1e-4 of it (with
+// H_SWISH the output changes by half to one and a half of what the quotient does).
+static RequantPack pack_exact(int act, float s_src, float s_flt, float s_dst) {
+    const RequantPack none = {s_src, s_flt, s_dst, 0.f, 0};
+    auto mid = [](float s) { return s >= 1e-12f && s <= 1e12f; };  // (nothing overflows or loses bits on the way)
+    const float c = make_requant_fast(s_src, s_flt, s_dst).c;
+    if (!mid(s_src) || !mid(s_flt) || !mid(s_dst) || !(c >= 1.6e-6f && c <= 1e12f))
+        return none;
+    const double inv = (act == MEGCC_NONLINE_RELU ? 2.0 : 1.0) / (double)s_dst;
+    RequantPack q = {s_src, s_flt, (float)inv, 0.f, 3};
+    q.d = (float)(inv - (double)q.c);
+    const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), act == MEGCC_NONLINE_IDENTITY ? -128 : 0);
+    const long long near = (long long)(1e-4f / c);
+    // (pts: the ends of the range, then each step's last accumulator below and first one above)
+    for (int i = 0; i < pts.n; ++i) {
+        const bool above = i >= 2 && pts.y[i] > pts.y[i - 1] && pts.a[i] == pts.a[i - 1] + 1;
+        const long long from = i < 2 || above ? pts.a[i] : std::max<long long>(pts.a[i] - near, i > 2 ? pts.a[i - 1] : INT32_MIN);
+        const long long to = i < 2 || !above ? pts.a[i] : std::min<long long>(pts.a[i] + near, i + 1 < pts.n ? pts.a[i + 1] : INT32_MAX);
+        for (long long a = from; a <= to; ++a)
+            if (pack_eval((int)a, act, q) != pts.y[i])
+                return none;
+    }
+    return q;
+}
+
+RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst, bool affine) {
+    static ScaleCache<RequantPack> multiply_adds, exact;
+    if (!requant_table_act(act) || !requant_table_ok(s_src, s_flt, s_dst))
+        return {s_src, s_flt, s_dst, 0.f, 0};
+    const auto key = multiply_adds.key(act, s_src, s_flt, s_dst);
+    RequantPack found;
+    if (affine && act != MEGCC_NONLINE_H_SWISH) {
+        if (!multiply_adds.find(key, &found)) {
+            found = pack_affine(act, s_src, s_flt, s_dst);
+            multiply_adds.put(key, found);
+        }
+        if (found.mode)
+            return found;
+    }
+    if (!exact.find(key, &found)) {
+        found = pack_exact(act, s_src, s_flt, s_dst);
+        exact.put(key, found);
+    }
+    return found;
+}
+
+RequantPack requant_pack_pick(int act, float s_src, float s_flt, float s_dst) {
+    return requant_pack_for(act, s_src, s_flt, s_dst, !options().no_affine);
 }
 
 RequantAffine requant_affine_pick(bool table, int act, float s_src, float s_flt, float s_dst) {
