@@ -593,9 +593,10 @@ int megcc_gfx950_requant_affine(int nonline_mode, float s_src, float s_flt, floa
  * through a fallback: "nopws", "nogevm", "nofcb", "nosmall", "nopm768", "nopm", "nodma512",
  * "nopm256", "nodma", "nofcs", "nopwshare", "nohybrid", "nodot4", "nof32small",
  * "dw_generic", "nodwmfma", "nodwnchw", "nofusesoftmax", "nopoolrows", "nofirstmfma", "norowsplit", "nofusechain", "nofusepwdw", "fusepwdw", "nofcone", "noxcdorder", "noaffine", "nopipeline", "no_graph",
- * "nofusedwpw", "fusedwpw", "nof32split", "nof32ks"; value 1 takes the kernel out
+ * "nofusedwpw", "fusedwpw", "nofusestem", "fusestem", "nof32split", "nof32ks"; value 1 takes the kernel out
  * of the dispatch, 0 puts it back ("fusepwdw", "fusedwpw": 1 makes the model runtime take the one-kernel form of a
- * pointwise / channel-wise or channel-wise / pointwise pair wherever it applies instead of timing both forms).
+ * pointwise / channel-wise or channel-wise / pointwise pair wherever it applies instead of timing both forms; "fusestem" the same for those pairs and for a network's head - the f32
+ * image's conversion, the first convolution and the pair behind it -, which "fusedwpw" leaves apart).
  * "nof32split" keeps f32 MatMul off the bf16 matrix instructions, "nof32ks" f32 MatMul and convolution off the
  * kernel whose waves share K; "nof32small" takes out that kernel for convolutions and conv_f32_small behind it. The
  * same names in capitals behind MEGCC_ are read from the environment once, at first use.

@@ -81,7 +81,7 @@ __device__ __forceinline__ void xcd_tile(XcdOrder o, int bx, int by, int gx, int
 // environment (MEGCC_NOPWS=1, ...) ONCE, when the library first consults them; later changes go
 // through megcc_gfx950_set_option(). Nothing on a launch path scans the environment.
 struct Options {
-    bool no_pws, no_gevm, no_fcb, no_small, no_pm768, no_pm, no_dma512, no_pm256, no_dma, no_fcs, no_pwshare, no_hybrid, no_dot4, no_f32small, dw_generic, no_dwmfma, no_dwnchw, no_fuse_softmax, no_graph, no_poolrows, no_firstmfma, no_rowsplit, no_fuse_chain, no_fuse_pwdw, fuse_pwdw, no_fcone, no_xcdorder, no_affine, no_pipeline, no_fuse_dwpw, fuse_dwpw, no_f32split, no_f32ks;
+    bool no_pws, no_gevm, no_fcb, no_small, no_pm768, no_pm, no_dma512, no_pm256, no_dma, no_fcs, no_pwshare, no_hybrid, no_dot4, no_f32small, dw_generic, no_dwmfma, no_dwnchw, no_fuse_softmax, no_graph, no_poolrows, no_firstmfma, no_rowsplit, no_fuse_chain, no_fuse_pwdw, fuse_pwdw, no_fcone, no_xcdorder, no_affine, no_pipeline, no_fuse_dwpw, fuse_dwpw, no_fuse_stem, fuse_stem, no_f32split, no_f32ks;
 };
 Options& options();
 
@@ -110,6 +110,15 @@ TinyNNStatus dw_pw_run(
 bool dw_pw_takes(
         const MegccConvAttr* dw_attr, const MegccConvAttr* pw_attr, const Tensor* src, const Tensor* dw_flt, const Tensor* mid,
         const Tensor* pw_flt, const Tensor* dst);
+
+// conv_api.hip: the image's conversion to qsi8, the first convolution of the quantised image, the channel-wise 3x3 and the pointwise
+// convolution behind it as one kernel (model runtime only). inputs: f32 image, then each layer's filter [, bias], the
+// pointwise one packed; the scales of the three tensors in between. `launch` false: only whether the kernel takes them.
+struct StemAttr {
+    MegccConvAttr first, dw, pw;
+    float s_image, s_first, s_mid;
+};
+TinyNNStatus stem_run(const StemAttr& attr, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, bool launch);
 
 // After a kernel launch: surfaces launch-configuration errors as TinyNN_ERROR_RUNTIME.
 TinyNNStatus check_launch(const char* what);

@@ -8,6 +8,7 @@
 //   qsi8 NCHW44 dense, anything else (5x5, 7x7, filter not packed)   -> conv_dot4.hip
 //   f32 NCHW DENSE                                                  -> gemm_f32.hip
 //   everything else ConvGeneral accepts                             -> conv_direct.hip
+#include <initializer_list>
 #include <mutex>
 
 #include "common.h"
@@ -56,6 +57,11 @@ bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* sr
 TinyNNStatus conv_dw_pw_launch(
         const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dflt, const void* dbias, const void* packed,
         const void* pbias, void* dst, DwPwBlock* block, bool prepare_only);
+
+bool conv_stem_supported(const ConvGeom& c0, const ConvGeom& dw, const ConvGeom& pw, const void* image, const void* dst);
+TinyNNStatus conv_stem_launch(
+        const ConvGeom& c0, const ConvGeom& dw, const ConvGeom& pw, const void* image, const void* flt0, const void* bias0, const void* dflt,
+        const void* dbias, const void* packed, const void* pbias, void* dst);
 
 // A filter that went through megcc_gfx950_conv2d_init is a 1-d byte tensor.
 static bool is_packed_filter(const Tensor* flt) {
@@ -870,6 +876,29 @@ bool dw_pw_takes(
            conv_dw_pw_supported(dw, pw, nullptr, nullptr) && conv_mfma_supported(pw);
 }
 
+// a tensor inside a chain, which has no memory
+static Tensor dense_q8(std::initializer_list<int> dims, float scale) {
+    Tensor t = {};
+    t.dtype.type_enum = TinyNN_QINT8;
+    t.dtype.param.scale = scale;
+    t.layout.nr_dim = (int)dims.size();
+    int i = 0, stride = 1;
+    for (int d : dims)
+        t.layout.dims[i++] = (uint32_t)d;
+    while (i-- > 0) {
+        t.layout.stride[i] = stride;
+        stride *= (int)t.layout.dims[i];
+    }
+    return t;
+}
+// a layer's bias, where it has one, as megcc_gfx950_conv2d takes it
+static bool chain_bias_ok(const Tensor* b, const ConvGeom& g) {
+    if (!b)
+        return true;
+    const float d = g.s_src * g.s_flt - b->dtype.param.scale;
+    return is_q32(b) && nr_elem(b->layout) == (size_t)g.oc && is_contiguous(b->layout) && aligned4(b->ptr) && (d < 0 ? -d : d) < 1e-5f;
+}
+
 TinyNNStatus dw_pw_run(
         const MegccPwDwAttr* a, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, DwPwBlock* block, DwPw what) {
     const char* who = "dw_pw";
@@ -894,28 +923,11 @@ TinyNNStatus dw_pw_run(
     if (st != TinyNN_SUCCESS)
         return st;
     dw.s_dst = a->mid_scale;
-    Tensor mid = {};
-    mid.dtype.type_enum = TinyNN_QINT8;
-    mid.dtype.param.scale = a->mid_scale;
-    mid.layout.nr_dim = 5;
-    const uint32_t md[5] = {(uint32_t)dw.n, (uint32_t)(dw.oc / 4), (uint32_t)dw.oh, (uint32_t)dw.ow, 4u};
-    int stride = 1;
-    for (int i = 4; i >= 0; --i) {
-        mid.layout.dims[i] = md[i];
-        mid.layout.stride[i] = stride;
-        stride *= (int)md[i];
-    }
+    const Tensor mid = dense_q8({dw.n, dw.oc / 4, dw.oh, dw.ow, 4}, a->mid_scale);
     st = make_geom(&a->pw, &mid, packed, dst, true, 0, &pw);
     if (st != TinyNN_SUCCESS)
         return st;
-    for (const Tensor* b : {dbias, pbias}) {
-        if (!b)
-            continue;
-        const ConvGeom& g = b == dbias ? dw : pw;
-        const float d = g.s_src * g.s_flt - b->dtype.param.scale;
-        MG_REQUIRE(nr_elem(b->layout) == (size_t)g.oc && is_contiguous(b->layout) && aligned4(b->ptr) && (d < 0 ? -d : d) < 1e-5f,
-                   TinyNN_ERROR_INVALID_LAYOUT, "%s: bias", who);
-    }
+    MG_REQUIRE(chain_bias_ok(dbias, dw) && chain_bias_ok(pbias, pw), TinyNN_ERROR_INVALID_LAYOUT, "%s: bias", who);
     MG_REQUIRE(conv_dw_pw_supported(dw, pw, src->ptr, dst->ptr) && conv_mfma_supported(pw) &&
                        nr_elem(packed->layout) == conv_mfma_packed_bytes(pw) && aligned16(packed->ptr) && aligned4(dflt->ptr),
                TinyNN_ERROR_NO_IMPLEMENT, "%s: shape, activation or alignment the kernel does not take", who);
@@ -925,5 +937,53 @@ TinyNNStatus dw_pw_run(
     return conv_dw_pw_launch(
             dw, pw, src->ptr, dflt->ptr, dbias ? dbias->ptr : nullptr, packed->ptr, pbias ? pbias->ptr : nullptr, dst->ptr, block,
             what == DwPw::PREPARE);
+}
+
+TinyNNStatus stem_run(const StemAttr& a, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, bool launch) {
+    const char* who = "stem";
+    const MegccConvAttr* const attr[3] = {&a.first, &a.dw, &a.pw};
+    const Tensor *flt[3], *bias[3];
+    int k = 1;
+    MG_REQUIRE(inputs && outputs && nr_output == 1 && outputs[0] &&
+                       nr_input == 4 + (a.first.with_bias ? 1 : 0) + (a.dw.with_bias ? 1 : 0) + (a.pw.with_bias ? 1 : 0),
+               TinyNN_ERROR_NULL_PTR, "%s: operands", who);
+    for (int i = 0; i < nr_input; ++i)
+        MG_REQUIRE(inputs[i], TinyNN_ERROR_NULL_PTR, "%s: input %d", who, i);
+    for (int l = 0; l < 3; ++l) {
+        flt[l] = inputs[k++];
+        bias[l] = attr[l]->with_bias ? inputs[k++] : nullptr;
+        MG_REQUIRE(is_q8(flt[l]) && is_packed_filter(flt[l]) == (l == 2), TinyNN_ERROR_INVALID_LAYOUT, "%s: filters", who);
+    }
+    const Tensor *image = inputs[0], *dst = outputs[0];
+    MG_REQUIRE(is_f32(image) && image->layout.nr_dim == 4 && is_contiguous(image->layout) && dst->dtype.type_enum == TinyNN_QINT8 &&
+                       a.first.format == MEGCC_FMT_NCHW_NCHW44 && a.first.sparse == MEGCC_SPARSE_DENSE && a.dw.format == MEGCC_FMT_NCHW44 &&
+                       a.dw.sparse == MEGCC_SPARSE_GROUP && a.pw.format == MEGCC_FMT_NCHW44 && a.pw.sparse == MEGCC_SPARSE_DENSE &&
+                       a.s_image > 0.f && a.s_first > 0.f && a.s_mid > 0.f && dst->dtype.param.scale > 0.f,
+               TinyNN_ERROR_INVALID_LAYOUT, "%s: operand types", who);
+    ConvGeom c0, dw, pw;
+    const uint32_t* id = image->layout.dims;
+    const Tensor quantised = dense_q8({(int)id[0], (int)id[1], (int)id[2], (int)id[3]}, a.s_image);
+    TinyNNStatus st = make_geom(&a.first, &quantised, flt[0], nullptr, false, 0, &c0);
+    if (st != TinyNN_SUCCESS)
+        return st;
+    c0.s_dst = a.s_first;
+    const Tensor first = dense_q8({c0.n, c0.oc / 4, c0.oh, c0.ow, 4}, a.s_first);
+    st = make_geom(&a.dw, &first, flt[1], nullptr, false, 0, &dw);
+    if (st != TinyNN_SUCCESS)
+        return st;
+    dw.s_dst = a.s_mid;
+    const Tensor mid = dense_q8({dw.n, dw.oc / 4, dw.oh, dw.ow, 4}, a.s_mid);
+    st = make_geom(&a.pw, &mid, flt[2], dst, true, 0, &pw);
+    if (st != TinyNN_SUCCESS)
+        return st;
+    MG_REQUIRE(chain_bias_ok(bias[0], c0) && chain_bias_ok(bias[1], dw) && chain_bias_ok(bias[2], pw), TinyNN_ERROR_INVALID_LAYOUT,
+               "%s: bias", who);
+    MG_REQUIRE(conv_stem_supported(c0, dw, pw, image->ptr, dst->ptr) && conv_mfma_supported(pw) &&
+                       nr_elem(flt[2]->layout) == conv_mfma_packed_bytes(pw) && aligned16(flt[2]->ptr) && aligned4(flt[1]->ptr),
+               TinyNN_ERROR_NO_IMPLEMENT, "%s: shape, activation or alignment the kernel does not take", who);
+    if (!launch)
+        return TinyNN_SUCCESS;
+    auto ptr = [](const Tensor* t) { return t ? t->ptr : nullptr; };
+    return conv_stem_launch(c0, dw, pw, image->ptr, flt[0]->ptr, ptr(bias[0]), flt[1]->ptr, ptr(bias[1]), flt[2]->ptr, ptr(bias[2]), dst->ptr);
 }
 }  // namespace mg

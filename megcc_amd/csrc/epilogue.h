@@ -253,7 +253,11 @@ __device__ __forceinline__ uint32_t pack4_perm(int a, int b, int c, int d) {
 // whose output that could change. Half away from zero is then exact for every float: truncation of v plus the
 // largest float below a half, and for outputs that are never negative the conversion of 2 v plus that float
 // (ties to even: 2 v + 0.5 of v = k + 0.5 is 2 k + 1.5, which goes to the even 2 k + 2).
-// Vector instructions for four outputs: 14, 18 - 22, 19, and mode 3 30 (RELU), 39 (IDENTITY), 46 (H_SWISH); the
+//     mode 5: mode 1 without its conversion, for kernels whose sums start from requant_bias(): the bits of the sum are then
+// those of the float 1.5 * 2^23 + a + m as long as |a + m| < 2^22, where all steps lie (it is asked for), and beyond
+// that floats that still grow with a. d is about 10^4 / c of its last bit there, too coarse to put it between the
+// steps; the whole number m, a few hundred at most, shifts them until a float falls there.
+// Vector instructions for four outputs: 10 (mode 5), 14, 18 - 22, 19, and mode 3 30 (RELU), 39 (IDENTITY), 46 (H_SWISH); the
 // threshold table's look-ups took 35 (H_SWISH 51) and four gathers from LDS, and its 1 KB among a launch's
 // arguments 0.7 us of the host's time.
 // (mode 0: none of these was proven; s1, s2, c are then the reference's three scales, for requant_conv)
@@ -264,6 +268,12 @@ struct RequantPack {
 };
 // `affine`: any mode, else 3 or 0
 RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst, bool affine);
+// mode 5, or mode 0 where it has no constants
+RequantPack requant_shifted_for(int act, float s_src, float s_flt, float s_dst);
+// A bias for mode 5. Clamped: sums of a few thousand products on top of +-2^29 have the outputs of the largest and the smallest sums.
+__device__ __forceinline__ int requant_bias(int bias, const RequantPack& q) {
+    return (bias > (1 << 29) ? 1 << 29 : bias < -(1 << 29) ? -(1 << 29) : bias) + __builtin_bit_cast(int, q.s1);
+}
 // what a launch uses: modes 1, 2 and 4 unless the switch "noaffine" is on (a launch with them is noted as "+affine")
 RequantPack requant_pack_pick(int act, float s_src, float s_flt, float s_dst);
 
@@ -300,7 +310,7 @@ __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3
     } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            float x = (float)a[i];
+            float x = MODE == 5 ? __builtin_bit_cast(float, a[i]) : (float)a[i];
             if (MODE == 2)
                 x = x * q.s1 * q.s2;
             r = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(x, q.c, q.d), i, r);

@@ -54,6 +54,9 @@ struct ModelOpr {
     int first_index = -1;  // index in Model::oprs of the (first) operator this schedule entry stands for
     bool dw_pw = false;    // a channel-wise + pointwise pair as one kernel (desc.attr.pw_dw, no kind of its own)
     DwPwBlock* block = nullptr;  // ... and its arguments
+    // the image's conversion, the first convolution and the pair behind it as one kernel; operator of that pair, -1: another kernel
+    StemAttr stem;
+    int stem_pair = -1;
     ModelOpr() = default;
     ModelOpr(const ModelOpr&) = delete;
     ~ModelOpr() { dw_pw_block_destroy(block); }
@@ -74,7 +77,7 @@ struct Model {
         bool known = false, faster = false;
         double gain_us = 0;
     };
-    std::vector<PairTime> dw_pw_time, pw_dw_time;
+    std::vector<PairTime> dw_pw_time, pw_dw_time, stem_time;
     double schedule_us = 0;
     // per operator: the channel-wise -> pointwise pair that begins there may run as one kernel, so the memory plan keeps
     // the channel-wise layer's source until the pointwise layer is through
@@ -320,6 +323,8 @@ static bool shares_bytes(const Tensor& a, const Tensor& b) {
 }
 // one entry of the schedule
 static TinyNNStatus call_opr(Model* m, ModelOpr* o) {
+    if (o->stem_pair >= 0)
+        return stem_run(o->stem, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(), (int)o->out_ptrs.size(), true);
     if (o->dw_pw)
         return dw_pw_run(&o->desc.attr.pw_dw, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(),
                          (int)o->out_ptrs.size(), o->block, DwPw::RUN);
@@ -382,6 +387,58 @@ static bool faster_as_one(Model* m, std::vector<Model::PairTime>& times, int at,
 struct Pairs {
     bool dw_pw, pw_dw;
 };
+
+// The f32 image's conversion to qsi8 and the first convolution, the last two entries of the schedule, with the pair `pair` behind
+// them as one kernel (conv_stem.hip), where nothing else reads the tensors in between and it measures faster. The image is the
+// caller's memory, not the arena's: it shares no byte with the result.
+static bool stem_taken(Model* m, const std::vector<int>& readers, ModelOpr* pair) {
+    const size_t n = m->schedule.size();
+    if (n < 2 || options().no_fuse_stem || options().fuse_dwpw)
+        return false;
+    ModelOpr *cv = m->schedule[n - 2], *c0 = m->schedule[n - 1];
+    if (cv->desc.kind != MEGCC_KERN_TYPECVT || c0->desc.kind != MEGCC_KERN_CONV || cv->dw_pw || c0->dw_pw || c0->has_processed ||
+        cv->in.size() != 1 || cv->out.size() != 1 || c0->out.size() != 1 || c0->in.size() != (c0->desc.attr.conv.with_bias ? 3u : 2u) ||
+        c0->in[0] != cv->out[0] || pair->in[0] != c0->out[0] || !chain_only(m, readers, cv->out[0], 1) ||
+        !chain_only(m, readers, c0->out[0], 1) || !m->tensors[cv->in[0]]->is_input || m->tensors[cv->in[0]]->alias_of >= 0)
+        return false;
+    const Tensor &image = m->tensors[cv->in[0]]->t, &quantised = m->tensors[cv->out[0]]->t, &first = m->tensors[c0->out[0]]->t;
+    if (image.layout.nr_dim != quantised.layout.nr_dim ||
+        !std::equal(image.layout.dims, image.layout.dims + image.layout.nr_dim, quantised.layout.dims) ||
+        quantised.dtype.type_enum != TinyNN_QINT8 || !is_contiguous(quantised.layout))
+        return false;
+    ModelOpr* f = new ModelOpr();
+    f->first_index = cv->first_index;
+    f->stem_pair = pair->first_index;
+    memset(&f->desc, 0, sizeof(f->desc));
+    memset(&f->ws, 0, sizeof(f->ws));
+    f->symbol = "quantise + first convolution + depthwise 3x3 + pointwise 1x1 (fused)";
+    f->stem.first = c0->desc.attr.conv;
+    f->stem.dw = pair->desc.attr.pw_dw.dw;
+    f->stem.pw = pair->desc.attr.pw_dw.pw;
+    f->stem.s_image = quantised.dtype.param.scale;
+    f->stem.s_first = first.dtype.param.scale;
+    f->stem.s_mid = pair->desc.attr.pw_dw.mid_scale;
+    f->in = cv->in;
+    f->in_ptrs = cv->in_ptrs;
+    for (const ModelOpr* o : {c0, pair})
+        for (size_t k = 1; k < o->in.size(); ++k) {
+            f->in.push_back(o->in[k]);
+            f->in_ptrs.push_back(o->in_ptrs[k]);
+        }
+    f->out = pair->out;
+    f->out_ptrs = pair->out_ptrs;
+    bool take = stem_run(f->stem, f->in_ptrs.data(), (int)f->in_ptrs.size(), f->out_ptrs.data(), (int)f->out_ptrs.size(), false) ==
+                TinyNN_SUCCESS;
+    take = take && (options().fuse_stem || faster_as_one(m, m->stem_time, f->first_index, f, {cv, c0, pair}));
+    if (!take) {
+        delete f;
+        return false;
+    }
+    m->schedule.resize(n - 2);
+    m->schedule.push_back(f);
+    m->fused.push_back(f);
+    return true;
+}
 
 static void build_schedule(Model* m, Pairs allow) {
     m->schedule.clear();
@@ -482,11 +539,12 @@ static void build_schedule(Model* m, Pairs allow) {
                     take = dw_pw_run(&f->desc.attr.pw_dw, f->in_ptrs.data(), (int)f->in_ptrs.size(), f->out_ptrs.data(),
                                      (int)f->out_ptrs.size(), f->block, DwPw::PREPARE) == TinyNN_SUCCESS;
                 }
-                if (take && !options().fuse_dwpw)
+                if (take && !options().fuse_dwpw && !options().fuse_stem)
                     take = faster_as_one(m, m->dw_pw_time, i, f, {o0, o1});
                 if (take) {
                     m->fused.push_back(f);
-                    m->schedule.push_back(f);
+                    if (!stem_taken(m, readers, f))
+                        m->schedule.push_back(f);
                     i += 1;
                     continue;
                 }
@@ -826,15 +884,16 @@ static Choice choose_schedule(Model* m) {
     double gain = 0;
     for (const ModelOpr* o : m->schedule) {
         pw_dw = pw_dw || o->desc.kind == MEGCC_KERN_PW_DW;
-        dw_pw = dw_pw || o->dw_pw;
-        if (o->dw_pw && (size_t)o->first_index < m->dw_pw_time.size())
-            gain += m->dw_pw_time[(size_t)o->first_index].gain_us;
+        const int pair = o->dw_pw ? o->first_index : o->stem_pair;
+        dw_pw = dw_pw || pair >= 0;
+        if (pair >= 0 && (size_t)pair < m->dw_pw_time.size())
+            gain += m->dw_pw_time[(size_t)pair].gain_us;
     }
     const bool doubt = dw_pw && gain < 0.1 * (m->schedule_us + gain);
     // (kernels of under 8 us: two-stream forwards still vary by a quarter from run to run, and one in three comparisons
     //  at batch 8 and 10 ended with no pairs, 135 us for 129)
     if (tail_begin < 0 || m->schedule_us < 8.0 * (double)m->schedule.size() || (!doubt && !pw_dw) || options().fuse_dwpw ||
-        options().fuse_pwdw)
+        options().fuse_pwdw || options().fuse_stem)
         return {best, tail_begin};
     // a forward with these pairs, at the boundary that balances the kernels' times
     auto time_pairs = [&](Pairs p) {
@@ -955,8 +1014,8 @@ static TinyNNStatus plan_again(Model* m, const Choice& chosen) {
     reset_tail(m);
     std::vector<char> one(m->oprs.size(), 0);
     for (const ModelOpr* o : m->schedule)
-        if (o->dw_pw)
-            one[(size_t)o->first_index] = 1;
+        if (o->dw_pw || o->stem_pair >= 0)
+            one[(size_t)(o->dw_pw ? o->first_index : o->stem_pair)] = 1;
     m->dw_pw_may = one;
     for (size_t i = 0; i < one.size(); ++i)
         if (one[i])

@@ -265,6 +265,12 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
 // host evaluation of requant_pack4 for one output
 static int pack_eval(int a, int act, const RequantPack& q) {
     float x = (float)a;
+    if (q.mode == 5) {
+        uint32_t u;
+        memcpy(&u, &q.s1, 4);
+        u += (uint32_t)a;
+        memcpy(&x, &u, 4);
+    }
     if (q.mode == 2 || q.mode == 3)
         x = x * q.s1 * q.s2;
     float y;
@@ -365,6 +371,76 @@ static RequantPack pack_exact(int act, float s_src, float s_flt, float s_dst) {
                 return none;
     }
     return q;
+}
+
+// Mode 5: for each slope near the quotient the interval that mode 1's d may lie in, moved to where the sums' floats are; of the
+// shifts m up to 1023 those whose d comes closest to its middle are verified.
+static RequantPack pack_shifted(int act, float s_src, float s_flt, float s_dst) {
+    const RequantPack none = {s_src, s_flt, s_dst, 0.f, 0};
+    const bool relu = act == MEGCC_NONLINE_RELU;
+    const int lowest = relu ? 0 : -128;
+    const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), lowest);
+    RequantBounds<true> from;
+    RequantBounds<false> to;
+    for (int i = 2; i < pts.n; ++i) {
+        if (std::abs((long long)pts.a[i]) >= (1 << 22) - 1024)
+            return none;
+        const double x = pts.a[i];
+        if (pts.y[i] > lowest)
+            from.add(x, relu ? 2.0 * pts.y[i] - 0.5 : pts.y[i] + 127.5, i);
+        if (pts.y[i] < 127)
+            to.add(x, relu ? 2.0 * pts.y[i] + 1.5 : pts.y[i] + 128.5, i);
+    }
+    // (the outputs at the ends of the range are then those beyond the first and the last step; the ends themselves have no float)
+    RequantSteps inner;
+    for (int i = 2; i < pts.n; ++i)
+        inner.add(pts.a[i], pts.y[i]);
+    for (int i = 0; i < from.n; ++i)
+        from.point[i] -= 2;
+    for (int i = 0; i < to.n; ++i)
+        to.point[i] -= 2;
+    const float c0 = make_requant_fast(s_src, s_flt, s_dst).c * (relu ? 2.f : 1.f);
+    for (int k = 0; k <= 48; ++k) {
+        const float c = by_ulps(c0, (k & 1) ? (k + 1) / 2 : -(k / 2));
+        const double dlo = from.tightest((double)c), dhi = to.tightest((double)c);
+        if (!(dlo <= dhi))
+            continue;
+        const double middle = (dlo + dhi) / 2 - 12582912.0 * (double)c;
+        struct {
+            double off;
+            int m;
+        } best[2] = {{1e30, 0}, {1e30, 0}};
+        for (int m = 0; m < 1024; ++m) {
+            const double d = middle - (double)c * m;
+            const double off = std::fabs((double)(float)d - d);
+            if (off < best[1].off) {
+                best[1] = {off, m};
+                if (off < best[0].off)
+                    std::swap(best[0], best[1]);
+            }
+        }
+        for (const auto& b : best) {
+            const int bits = 0x4b400000 + b.m;
+            RequantPack q = {0.f, 0.f, c, (float)(middle - (double)c * b.m), 5};
+            memcpy(&q.s1, &bits, 4);
+            if (b.off <= (dhi - dlo) / 2 && requant_verified(inner, from, to, [&](int a) { return pack_eval(a, act, q); }))
+                return q;
+        }
+    }
+    return none;
+}
+
+RequantPack requant_shifted_for(int act, float s_src, float s_flt, float s_dst) {
+    static ScaleCache<RequantPack> cache;
+    RequantPack found = {s_src, s_flt, s_dst, 0.f, 0};
+    if ((act != MEGCC_NONLINE_IDENTITY && act != MEGCC_NONLINE_RELU) || !requant_table_ok(s_src, s_flt, s_dst))
+        return found;
+    const auto key = cache.key(act, s_src, s_flt, s_dst);
+    if (!cache.find(key, &found)) {
+        found = pack_shifted(act, s_src, s_flt, s_dst);
+        cache.put(key, found);
+    }
+    return found;
 }
 
 RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst, bool affine) {
