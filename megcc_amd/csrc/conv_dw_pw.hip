@@ -300,11 +300,11 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwPar
 #pragma unroll
     for (int k = 0; k < BI; ++k)
         if (tid + k * DP_THREADS < C)
-            db[tid + k * DP_THREADS] = q.dbias ? dbv[k] : 0;
+            db[tid + k * DP_THREADS] = requant_start(q.dbias ? dbv[k] : 0, q.dq);
 #pragma unroll
     for (int k = 0; k < PI; ++k)
         if (tid + k * DP_THREADS < ocs)
-            pb[tid + k * DP_THREADS] = q.pbias ? pbv[k] : 0;
+            pb[tid + k * DP_THREADS] = requant_start(q.pbias ? pbv[k] : 0, q.pq);
     if (KEEP_P) {
 #pragma unroll
         for (int c = 0; c < KC; ++c)
@@ -416,7 +416,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwPar
             for (int e = 0; e < 4; ++e)
                 a[p * 4 + e] = acc[p][e];
         uint32_t d[4];
-        requant_dwords<DACT>(a, d, q.dq);
+        requant_dwords<DACT, true>(a, d, q.dq);
         *(v4i*)(m + mid0 + i * (8 * T * 16)) = v4i{(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
     };
     // ---- pointwise: where a column's results go. (Stores are issued whether or not the place exists: what is under no
@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(DP_THREADS, 2) conv_dw_pw_kernel(const DwPwPar
         for (int e = 0; e < 16; ++e)
             a[e] = acc[e];
         uint32_t d[4];
-        requant_dwords<PACT>(a, d, q.pq);
+        requant_dwords<PACT, true>(a, d, q.pq);
         // (OC is a multiple of 32: all of the tile's channels exist or none)
         const bool there = oc_wave + mi * 32 < q.OC;
         const unsigned o = there ? w : OOB;
@@ -635,8 +635,8 @@ static TinyNNStatus dp_plan(
     q.d_xg = make_fastdiv(q.xg);
     q.d_oh = make_fastdiv(q.oh);
     q.d_slices = make_fastdiv(q.slices);
-    q.dq = requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst, affine);
-    q.pq = requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst, affine);
+    q.dq = requant_started_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst, affine);
+    q.pq = requant_started_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst, affine);
     const int rag = dw.iw & 3;
     DwPwKernel kern = nullptr;
     size_t lds = 0;

@@ -270,9 +270,15 @@ struct RequantPack {
 RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst, bool affine);
 // mode 5, or mode 0 where it has no constants
 RequantPack requant_shifted_for(int act, float s_src, float s_flt, float s_dst);
+// for kernels whose sums start from requant_start(): mode 5 where there is one, else 2, 4, 3 or 0 (mode 1 as mode 2 with products by
+// one); `affine` as above
+RequantPack requant_started_for(int act, float s_src, float s_flt, float s_dst, bool affine);
 // A bias for mode 5. Clamped: sums of a few thousand products on top of +-2^29 have the outputs of the largest and the smallest sums.
 __device__ __forceinline__ int requant_bias(int bias, const RequantPack& q) {
     return (bias > (1 << 29) ? 1 << 29 : bias < -(1 << 29) ? -(1 << 29) : bias) + __builtin_bit_cast(int, q.s1);
+}
+__device__ __forceinline__ int requant_start(int bias, const RequantPack& q) {
+    return q.mode == 5 ? requant_bias(bias, q) : bias;  // (uniform)
 }
 // what a launch uses: modes 1, 2 and 4 unless the switch "noaffine" is on (a launch with them is noted as "+affine")
 RequantPack requant_pack_pick(int act, float s_src, float s_flt, float s_dst);
@@ -320,10 +326,10 @@ __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3
 }
 
 // N accumulators -> N / 4 dwords (each 4 consecutive ones), the form by a uniform branch. ACT < 0: the literal sequence of
-// `act` (mode 0, SIGMOID), whose scales stand where mode 0 has them.
+// `act` (mode 0, SIGMOID), whose scales stand where mode 0 has them. STARTED: the sums started from requant_start().
 // The empty volatile statements keep each form inside its branch: the compiler otherwise computes one of
 // them ahead of the branch and throws it away, 80 instructions of 120.
-template <int ACT, int N>
+template <int ACT, bool STARTED = false, int N>
 __device__ __forceinline__ void requant_dwords(int (&a)[N], uint32_t (&out)[N / 4], const RequantPack& q, int act = ACT) {
     auto here = [&]() __attribute__((always_inline)) {
 #ifndef MG_HOST_AUDIT
@@ -345,11 +351,11 @@ __device__ __forceinline__ void requant_dwords(int (&a)[N], uint32_t (&out)[N / 
 #pragma unroll
         for (int i = 0; i < N / 4; ++i)
             out[i] = requant_pack4<3, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
-    } else if (q.mode == 1) {  // (uniform)
+    } else if (q.mode == (STARTED ? 5 : 1)) {  // (uniform)
         here();
 #pragma unroll
         for (int i = 0; i < N / 4; ++i)
-            out[i] = requant_pack4<1, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+            out[i] = requant_pack4<STARTED ? 5 : 1, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
     } else if (ACT == MEGCC_NONLINE_RELU ? q.mode == 2 : q.mode == 4) {
         here();
 #pragma unroll

@@ -464,6 +464,23 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst, boo
     return found;
 }
 
+RequantPack requant_started_for(int act, float s_src, float s_flt, float s_dst, bool affine) {
+    if (affine) {
+        RequantPack q = requant_shifted_for(act, s_src, s_flt, s_dst);
+        if (q.mode)
+            return q;
+        q = requant_pack_for(act, s_src, s_flt, s_dst, true);
+        if (q.mode != 1)
+            return q;
+        if (act == MEGCC_NONLINE_RELU)
+            return {1.f, 1.f, q.c, q.d, 2};
+        const RequantAffine a = requant_affine_for(act, s_src, s_flt, s_dst);
+        if (a.d != 0.f)
+            return {0.f, 0.f, a.c, a.d, 4};
+    }
+    return requant_pack_for(act, s_src, s_flt, s_dst, false);
+}
+
 RequantPack requant_pack_pick(int act, float s_src, float s_flt, float s_dst) {
     return requant_pack_for(act, s_src, s_flt, s_dst, !options().no_affine);
 }
