@@ -6,21 +6,22 @@
 // A workgroup of 8 waves owns a strip of rows of one image and walks down it two output rows a step. Four stages work at the
 // same time, each a step behind the one that feeds it, one barrier a step:
 //   A  four rows of the image, asked for a step earlier, are quantised into a ring of rows in LDS (every pixel once);
-//   B  the first convolution, as in conv_first.hip (k = 4 (ic 3 + fh) + fw, a zero weight at fw = 3, two products): 32 pixels a wave,
-//      whose four bytes of a row are cut out of two dwords of the ring. Its result goes to a second ring, channel group
-//      by channel group as NCHW44 has it; rows outside of the image are written as the zeros the next layer pads with;
+//   B  the first convolution, as in conv_first.hip (k = 4 (ic 3 + fh) + fw; the fourth bytes, where a filter row has no weight, take the
+//      ninth pair (ic, fh), so that one product does): 32 pixels a wave, whose four bytes of a row are cut out of two dwords of the
+//      ring. Its result goes to a second ring, channel group by channel group as NCHW44 has it; rows outside of the image
+//      are written as the zeros the next layer pads with;
 //   C  the channel-wise layer as in conv_dw_pw.hip: a product with a banded matrix, 16 channels x 64 pixels a wave, whose operands
 //      are 16-byte pieces of the second ring and the pixels left and right of them;
 //   D  the pointwise layer: 32 pixels a wave, the filter in registers, four channels of a pixel a store.
 // So a strip pays three steps before its first result (and computes three rows that its neighbours compute too); how many
 // strips an image has follows from how many images there are for a CU (stem_strips).
-// A workgroup has a CU to itself: 216 registers, so that all biases stay in them (read from LDS for every product they were two
-// thirds of the 16-byte reads) and a step's operands, products and results of the stages overlap in each wave.
 // The requantisations are those of epilogue.h, so the result is bit for bit the four operators'.
-// What bounds it: a step's 1.29 us are 0.65 of the vector ALU and the waves' operands out of LDS in front of it, at the same time in
-// all of them since the barrier; from 256 images on memory (359 MB in 86 us). Measured (us, 3 x 224 x 224 -> 64, as three kernels
-// / this one): N=1 10.2 / 5.6, 8 13.5 / 7.7, 32 27.5 / 16.0, 64 37.6 / 25.5, 128 60 / 44, 256 142 / 86. With two workgroups a CU of 128
-// registers a step of both took 2.7 us; with the conversion of every sum to a float (mode 1 for 5) 1.50 for 1.29.
+// What bounds it: a step's 1.4 us are the waves' operands out of LDS, products and conversions one after the other, about 0.65 us of
+// them the vector ALU's; from 256 images on memory (359 MB). Measured (us, 3 x 224 x 224 -> 64, as three kernels / this one):
+// N=1 9.5 / 5.7, 8 13.0 / 7.9, 32 26.6 / 16.7, 64 36.6 / 26.8, 128 59 / 47, 256 141 / 90. 112 registers are two waves a SIMD beside two of the
+// 144 that conv_dw_pw has at 512 channels: in a network the tail of the forward before runs on the same CUs. (216 registers, all
+// biases in them and the stages' operands asked for together took 1.29 us a step and made no network faster; with the conversion of
+// every sum to a float, mode 1 for 5, 1.50.)
 #include "common.h"
 #include "conv_geom.h"
 #include "conv_mfma_i8.h"
@@ -55,10 +56,9 @@ struct StemParams {
 };
 
 // MT: 32-channel tiles of the pointwise layer; PACT: its activation (the other two have RELU). FMA: all three requantise by
-// mode 5, so that a step is one block of code in which the stages' operands, products and
-// conversions overlap; else by whichever form, with branches in between and the stages one after the other.
+// mode 5, else by whichever form.
 template <int MT, int PACT, bool FMA>
-__global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) {
+__global__ void __launch_bounds__(ST_THREADS, 4) conv_stem_kernel(StemParams q) {
     __shared__ __attribute__((aligned(16))) uint32_t img[ST_IRING * 3 * ST_IROW + 1];  // (the widest rows' last padding is the next row's first dword)
     __shared__ __attribute__((aligned(16))) uint32_t first[ST_CRING * (ST_C / 4) * ST_CROW];
     __shared__ __attribute__((aligned(16))) v4i mid[2][2 * ST_T];  // [16 channels][pixel] pieces
@@ -149,11 +149,11 @@ __global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) 
     wait_vmcnt<0>();  // (the filters are there: no wait for them is left in the loop)
     ask(4 * s0 + 2, 4);
     __syncthreads();
-    v4i A1, A2;
+    // rows of the first filter: pairs 4 kg .. + 3 of this half of K; the three weights of pair 8 where pairs 0 to 2 have their zeros
+    v4i A1;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-        A1[j] = w0[(4 * kg + j) * ST_C + col];
-    A2 = v4i{kg == 0 ? w0[8 * ST_C + col] : 0, 0, 0, 0};
+        A1[j] = w0[(4 * kg + j) * ST_C + col] | (kg == 0 && j < 3 ? w0[8 * ST_C + col] >> (8 * j) << 24 : 0);
     // ---- B: this lane's pixel of a step's two rows and where its bytes begin in a ring row
     const int slot = wave * 32 + col;
     const bool there = slot < 2 * q.ow;
@@ -191,15 +191,6 @@ __global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) 
                 acc[e4 * 4 + e] = bv[e];
         }
     };
-    v16i bias0, biasp[MT];
-    v4i biasd[4];
-    bias_of(b0, bias0);
-#pragma unroll
-    for (int mi = 0; mi < MT; ++mi)
-        bias_of(pb + mi * 32, biasp[mi]);
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-        biasd[p] = *(const v4i*)(db + quad * 16 + p * 4);
     auto requant = [&](auto act, int (&a)[16], uint32_t (&d)[4], const RequantPack& r) __attribute__((always_inline)) {
         constexpr int ACT = decltype(act)::value;
         if constexpr (FMA) {
@@ -236,16 +227,20 @@ __global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) 
 #pragma unroll
         for (int j = 0; j < 5; ++j)
             b[j] = (int)__builtin_amdgcn_alignbyte(w[j][1], w[j][0], cut);
-        const v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1, v4i{b[0], b[1], b[2], b[3]}, bias0, 0, 0, 0);
-        return __builtin_amdgcn_mfma_i32_32x32x32_i8(A2, v4i{b[4], 0, 0, 0}, acc, 0, 0, 0);
+        v16i acc;
+        bias_of(b0, acc);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)  // byte j of pair 8 in the place of pair j's fourth (the other half of K has no weight there)
+            b[j] = (int)__builtin_amdgcn_perm((unsigned)b[4], (unsigned)b[j], 0x00020100u + ((4u + j) << 24));
+        return __builtin_amdgcn_mfma_i32_32x32x32_i8(A1, v4i{b[0], b[1], b[2], b[3]}, acc, 0, 0, 0);
     };
-    auto first_results = [&](int i, const v16i& acc, auto inside) __attribute__((always_inline)) {
+    auto first_results = [&](int i, const v16i& acc) __attribute__((always_inline)) {
         const int y = 2 * i - 1 + row;
         int a[16];
         uint32_t d[4];
         sums(acc, a);
         requant(std::integral_constant<int, MEGCC_NONLINE_RELU>{}, a, d, q.r0);
-        const bool in = decltype(inside)::value || (unsigned)y < (unsigned)q.oh;
+        const bool in = (unsigned)y < (unsigned)q.oh;
         if (there) {
             uint32_t* const o = first + ((y & (ST_CRING - 1)) * (ST_C / 4) + kg) * ST_CROW + 4 + x;
 #pragma unroll
@@ -264,7 +259,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) 
         for (int p = 0; p < 4; ++p) {
             o.b[p] = *(const v4i*)(src + p * ST_CROW);
             o.e[p] = st_v2u{src[p * ST_CROW - 1], src[p * ST_CROW + 4]};
-            o.acc[p] = biasd[p];
+            o.acc[p] = *(const v4i*)(db + quad * 16 + p * 4);
         }
     };
     // (the short products first and every product where it stands, as conv_dw_pw.hip has it: a long product must not
@@ -297,18 +292,16 @@ __global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) 
         mid[t & 1][quad * ST_T + (sub * 16 + colq) * 4 + kg4] = v4i{(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
     };
     // D, rows 2 t and 2 t + 1 of the pointwise layer
-    auto pw_products = [&](const v4i& b, v16i (&acc)[MT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int mi = 0; mi < MT; ++mi)
-            acc[mi] = __builtin_amdgcn_mfma_i32_32x32x32_i8(P[mi], b, biasp[mi], 0, 0, 0);
-    };
-    auto pw_results = [&](int t, const v16i (&acc)[MT]) __attribute__((always_inline)) {
+    auto pointwise = [&](int t, const v4i& b) __attribute__((always_inline)) {
         const unsigned o = there && 2 * t + row < q.oh ? (unsigned)(obase + 2 * t * q.ow * 4) : OOB;
 #pragma unroll
         for (int mi = 0; mi < MT; ++mi) {
+            v16i acc;
+            bias_of(pb + mi * 32, acc);
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(P[mi], b, acc, 0, 0, 0);
             int a[16];
             uint32_t d[4];
-            sums(acc[mi], a);
+            sums(acc, a);
             requant(std::integral_constant<int, PACT>{}, a, d, q.pq);
 #pragma unroll
             for (int e4 = 0; e4 < 4; ++e4)
@@ -317,8 +310,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) 
     };
     const bool mine = wave * 32 < 2 * q.ow;       // pixels for this wave (B, D)
     const bool pieces = sub * 16 < 2 * xg;        // ... groups (C)
-    // Some stages at work, each for itself
-    auto some = [&](int i) __attribute__((always_inline)) {
+    for (int i = s0; i < s1 + 3; ++i) {
         if (i < s1) {
             quantise(4 * i + 2, 4);
             ask(i + 1 < s1 ? 4 * i + 6 : q.ih, 4);
@@ -326,7 +318,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) 
         if (i <= s1 && mine) {
             uint32_t w[5][2];
             first_words(i, w);
-            first_results(i, first_products(w), std::false_type{});
+            first_results(i, first_products(w));
         }
         if (i - 2 >= s0 && i - 2 < s1 && pieces) {
             Pieces o;
@@ -334,50 +326,9 @@ __global__ void __launch_bounds__(ST_THREADS, 2) conv_stem_kernel(StemParams q) 
             dw_products(o);
             dw_results(i - 2, o);
         }
-        if (i - 3 >= s0 && mine) {
-            v16i acc[MT];
-            pw_products(mid[(i - 3) & 1][kg * ST_T + slot], acc);
-            pw_results(i - 3, acc);
-        }
+        if (i - 3 >= s0 && mine)
+            pointwise(i - 3, mid[(i - 3) & 1][kg * ST_T + slot]);
         lds_barrier();
-    };
-    // All stages at work, no row outside of the image: operands, products, results, so that a wave waits for none of them
-    // (waves without pixels too: what they work out has no place)
-    auto all = [&](int i) __attribute__((always_inline)) {
-        Pieces o;
-        uint32_t w[5][2];
-        dw_operands(i - 2, o);
-        first_words(i, w);
-        const v4i m = mid[(i - 3) & 1][kg * ST_T + slot];
-        __builtin_amdgcn_sched_barrier(0);
-        quantise(4 * i + 2, 4);
-        ask(i + 1 < s1 ? 4 * i + 6 : q.ih, 4);
-        __builtin_amdgcn_sched_barrier(0);
-        dw_products(o);
-        const v16i accb = first_products(w);
-        v16i accd[MT];
-        pw_products(m, accd);
-        __builtin_amdgcn_sched_barrier(0);
-        if (pieces)
-            dw_results(i - 2, o);
-        first_results(i, accb, std::true_type{});
-        pw_results(i - 3, accd);
-        lds_barrier();
-    };
-    const int s3 = FMA ? min(s0 + 3, s1 + 3) : s1 + 3;  // the first step with all stages
-    int i = s0;
-    for (int part = 0; part < 2; ++part) {
-        for (const int end = part == 0 ? s3 : s1 + 3; i < end; ++i)
-            some(i);
-        if (FMA && i < s1) {
-            // As many stores as a step has, to no place: the loop's wait for the pieces of the image then is one for what is older than
-            // the step's stores, also at its start, where the compiler would otherwise wait for every store before it.
-#pragma unroll
-            for (int k = 0; k < 4 * MT; ++k)
-                __builtin_amdgcn_raw_buffer_store_b32(0u, rd, (int)OOB, k * ostep, 0);
-            for (; i < s1; ++i)
-                all(i);
-        }
     }
 }
 
@@ -397,8 +348,9 @@ bool conv_stem_supported(const ConvGeom& c0, const ConvGeom& dw, const ConvGeom&
            (long)pw.n * pw.oc * pw.oh * pw.ow < (1L << 31);
 }
 
-// Workgroups of an image: a CU holds one, and a strip has three steps on top of its own (us, 3 x 224 x 224 -> 64: N=64 4 strips 25.4,
-// 7 31, 8 29; N=32 7 17.3, 8 16.0, 14 20.0; N=256 1 86, 2 90).
+// Workgroups of an image: one for a CU, and a strip has three steps on top of its own. (A CU holds two, and on its own the kernel is
+// the quicker for it: N=64 4 strips 26.8 us, 8 23.7; 256 1 90, 2 79. In a network their room is the other stream's: MobileNetV1
+// batch 64 147 and 155, 256 488 and 487, 16 14 strips 94.3, 28 94.7.)
 static int stem_strips(long n, int steps) {
     int best = 1;
     long least = 1L << 60;
