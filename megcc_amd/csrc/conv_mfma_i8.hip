@@ -635,11 +635,13 @@ TinyNNStatus conv_mfma_launch(
     if ((!pipe || conv_gather_i8_wins(g, picked)) && conv_gather_i8_supported(g) &&
         (!options().no_small || g.fh * g.fw > MAX_TAPS_STAGE))
         return conv_gather_i8_launch(g, src, packed, bias, dst);  // (notes its own variant)
-    // FullyConnected: the LDS-direct kernel's 256 x 256 tiles win from half a chip of them on (2048 x 4096
-    // x 4096, 128 tiles: 43.7 us against 46.6; 4096 x 2048 x 1024, 64 tiles: 21.5 against 21.2; 2048 x 1024
-    // x 1000, 32 tiles: 14.8 against 8.6; 200 x 1024 x 1000: 13.0 on the one-stage kernel against 6.6)
-    if (is_fc(g) && g.n > 64 && fc_tile_supported(g) && !options().no_fcs &&
-        !(pipe && (long)((g.n + 255) / 256) * ((g.oc + 255) / 256) >= num_cus() / 2))
+    // FullyConnected: the LDS-direct kernel's 256 x 256 tiles win from half a chip of them on if K is long, and over a shorter one where
+    // they fill it (us for it / fc_tile: 2048 x 4096 x 4096, 128 tiles, 42.0 / 43.4; 3156 x 2048 x 3456, 182 tiles, 32.2 / 33.1;
+    // 4096 x 512 x 4096, 256 tiles, 17.2 / 18.8; 8192 x 256 x 4096, 512 tiles, 23.1 / 24.3; but 3156 x 512 x 3456 15.1 / 13.3, 2304 x 512 x
+    // 4096, 144 tiles, 13.3 / 11.6, 8192 x 128 x 4096 19.4 / 18.7, 3156 x 128 x 3456 10.9 / 8.1; 64 tiles, 4096 x 2048 x 1024, 21.5 / 21.2)
+    const long tiles256 = (long)((g.n + 255) / 256) * ((g.oc + 255) / 256);
+    const bool tiles_win = tiles256 >= num_cus() / 2 && (g.ic >= 1024 || (g.ic >= 256 && tiles256 >= num_cus()));
+    if (is_fc(g) && g.n > 64 && fc_tile_supported(g) && !options().no_fcs && !(pipe && tiles_win))
         return fc_tile_launch(g, src, packed, bias, dst);
     if (!pipe) {
         range_len = 0;

@@ -378,6 +378,27 @@ def test_fully_connected_over_any_k(kernel, m, k, n, act):
     compare(got, case.run_port(arrays), repr(case))
 
 
+FC_PARTS = [
+    # each part of a tiled FullyConnected (128, 64 alone and with four groups sharing K, 32), K of one block, a few and many, rows at
+    # odd bytes and on words; K of whole blocks either side of the LDS-direct kernel
+    (2049, 2050, 2050, ",128,1"), (2050, 2052, 2049, ",128,1"),
+    (1025, 65, 1100, ",64,1"), (1500, 260, 1537, ",64,1"), (1100, 511, 1100, ",64,1"),
+    (830, 2049, 961, ",64,4"), (833, 2052, 960, ",64,4"),
+    (97, 2049, 97, ",32,4"), (97, 1028, 100, ",32,4"), (450, 16, 30, ",32,4"), (65, 1, 33, ",32,4"),
+    (2305, 384, 2561, "fc_tile"), (2305, 1024, 2561, "fc_tile"), (2049, 1024, 3841, "dma"),
+]
+
+
+@pytest.mark.parametrize("m,k,n,kernel", FC_PARTS)
+def test_fully_connected_parts(m, k, n, kernel):
+    port.set_threads(8)
+    case = ConvCase(A.FMT_NCHW, A.DENSE, m, k, 1, 1, n, 1, 1, 0, A.RELU, scales=(0.01, 0.01, 0.01 * unsat(k) / 0.02))
+    arrays = case.gen(seed=23)
+    got = run_gpu(case, arrays)
+    assert kernel in runtime.last_kernel(), runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
 F32_SHARED_K = [
     # few output tiles, K shared by the waves of a workgroup: extents at and around the 32 / 64 tiles, K below
     # one step of 8, with and without a rest, and long enough for whole lines per wave
