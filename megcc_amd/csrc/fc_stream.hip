@@ -163,7 +163,7 @@ struct FcOneParams {
     const int32_t* bias;
     int8_t* dst;  // [M][OC]
     int M, K, OC, OCP, act;
-    unsigned last16;  // offset of the last 16 bytes of src
+    unsigned src_off, src_bytes;  // fc_one32_kernel: src points to a word, its first byte in it, whole words to the last byte
     float s_src, s_flt, s_dst;
 };
 
@@ -284,42 +284,63 @@ __global__ void __launch_bounds__(64 * FO_WAVES) fc_one_kernel(FcOneParams q) {
 // condition. A load that is issued under a condition (a prefetch inside `if (block + 2 < blocks)`,
 // a row test around the load) leaves the compiler unable to count how many loads are outstanding
 // behind an earlier one, and it then waits for ALL of them before the first use: each prefetch
-// became a round trip of its own. Here a wave with fewer blocks than NB, or none, fetches a block it
-// has a right to read again and multiplies it with zeros; rows beyond M read row M - 1 and are
-// zeroed on their way into LDS. ANYK: K is no multiple of 128 or the rows start at any byte - the last
-// block's surplus bytes meet the packed filter's zeros, and a piece that would run past the end of the
-// tensor is read 16 bytes before it and shifted into place (fc_tile.hip says more).
-template <int NB, bool ANYK>
+// became a round trip of its own. Here a wave with fewer blocks than NB, or none, asks a buffer of no bytes for them, which
+// answers with zeros and sends nothing to memory (blocks fetched a second time cost what the first did: NB = 3 by four
+// blocks each, 22 x 3000 x 3000 5.6 -> 4.2 us); rows beyond M and what lies beyond the tensor's last word are zeros likewise.
+// K need be no multiple of 128 - the last block's surplus bytes meet the packed filter's zeros. ODD: rows may start at any byte; words
+// and the one behind them are read and moved into place (16-byte loads at odd bytes, the bias read where it is added and the
+// above: 43 x 2541 x 2400 7.5 -> 5.4 us, 64 x 3000 x 500 5.5 -> 4.2; the bias alone 64 x 4096 x 4096 5.8 -> 5.3). Bound by what a CU
+// fetches: 64 rows of K of filter and activations, half of it shared in its L2.
+template <int NB, bool ODD>
 __global__ void __launch_bounds__(64 * FO_WAVES) fc_one32_kernel(FcOneParams q) {
-    __shared__ int32_t red[FO_WAVES][16][64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ __attribute__((aligned(16))) int8_t lds[FO_WAVES * 4096];  // a block or the sums of each wave
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, kg = lane >> 5;
-    const int oct = blockIdx.x, oc = oct * 32 + col;
-    const int row0 = blockIdx.y * 32;
-    const int blocks = ANYK ? (q.K + 127) >> 7 : q.K >> 7;
-    const int myb = wave < blocks ? (blocks - wave + FO_WAVES - 1) / FO_WAVES : 0;  // <= NB
-    const int wv = myb ? wave : 0;
-    const size_t astep = (size_t)q.OCP * KROW;
-    const int8_t* arow = q.wp + ((size_t)(wv * 4) * q.OCP + oc) * KROW + (((kg ^ (oc >> 3)) & 1) << 4);
-    int8_t* stage = (int8_t*)&red[wave][0][0];  // 4 KB: 32 rows of 128 bytes, pieces at piece ^ (row & 7)
+    const int oct = blockIdx.x, row0 = blockIdx.y * 32;
+    const int blocks = (q.K + 127) >> 7;
+    int8_t* stage = lds + wave * 4096;  // 32 rows of 128 bytes, pieces at piece ^ (row & 7)
     const int srow = lane >> 3, apc = lane & 7;
+    // the four channels that this thread will finish
+    const int e4 = wave & 3, ocb = oct * 32 + e4 * 8 + kg * 4;
+    int bias[4] = {0, 0, 0, 0};
+    if (q.bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            bias[e] = q.bias[min(ocb + e, q.OC - 1)];
+    }
+    // words of the activations (ODD: src is the word of the first byte, which is byte src_off of it); a block that is not
+    // there has a buffer of no bytes, in which every load is answered with zeros and none reaches memory
     v4i areg[NB][4], ring[NB * 4];
+    int next[NB][4];
+    unsigned aoff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        aoff[i] = (unsigned)(row0 + i * 8 + srow) * (unsigned)q.K + q.src_off + (unsigned)(wave * 128 + apc * 16);
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const int bc = b < myb ? b : 0;
+        const int blk = wave + FO_WAVES * b;
+        const __amdgpu_buffer_rsrc_t rs =
+                __builtin_amdgcn_make_buffer_rsrc((void*)q.src, 0, blk < blocks ? q.src_bytes : 0, 0x00020000);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int row = min(row0 + i * 8 + srow, q.M - 1);
-            const unsigned off = (unsigned)row * (unsigned)q.K + (unsigned)((wv + FO_WAVES * bc) * 128 + apc * 16);
-            areg[b][i] = ANYK ? (v4i)*(const v4i_any*)(q.src + min(off, q.last16)) : *(const v4i*)(q.src + off);
+            const unsigned o = (aoff[i] + (unsigned)(b * FO_WAVES * 128)) & ~3u;
+            areg[b][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)o, 0, 0));
+            if (ODD)
+                next[b][i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)(o + 16), 0, 0);
         }
     }
+    const int aw = col * KROW + (((kg ^ (col >> 3)) & 1) << 4);
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const int bc = b < myb ? b : 0;
+        const int blk = wave + FO_WAVES * b;
 #pragma unroll
-        for (int cc = 0; cc < 4; ++cc)
-            ring[b * 4 + cc] = *(const v4i*)(arow + (size_t)(bc * (4 * FO_WAVES) + cc) * astep);
+        for (int cc = 0; cc < 4; ++cc) {
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+                    (void*)(q.wp + ((size_t)(min(blk, blocks - 1) * 4 + cc) * q.OCP + oct * 32) * KROW), 0,
+                    blk < blocks ? 32 * KROW : 0, 0x00020000);
+            ring[b * 4 + cc] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, aw, 0, 0));
+        }
     }
     // (the scheduler otherwise moves each load down to a few instructions before its use)
     __builtin_amdgcn_sched_barrier(0);
@@ -331,19 +352,17 @@ __global__ void __launch_bounds__(64 * FO_WAVES) fc_one32_kernel(FcOneParams q) 
     for (int b = 0; b < NB; ++b) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const bool ok = row0 + i * 8 + srow < q.M && b < myb;
             v4i v = areg[b][i];
-            if (ANYK) {
-                const unsigned off = (unsigned)min(row0 + i * 8 + srow, q.M - 1) * (unsigned)q.K +
-                                     (unsigned)((wv + FO_WAVES * (b < myb ? b : 0)) * 128 + apc * 16);
-                if (off > q.last16)
-                    v = fc_tail_piece(v, off - q.last16);
+            if (ODD) {
+                const unsigned sh = (aoff[i] & 3u) * 8u;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    v[j] = (int)(uint32_t)((((uint64_t)(uint32_t)(j < 3 ? v[j < 3 ? j + 1 : 0] : next[b][i]) << 32) | (uint32_t)v[j]) >> sh);
             }
-            v.x = ok ? v.x : 0, v.y = ok ? v.y : 0, v.z = ok ? v.z : 0, v.w = ok ? v.w : 0;
             *(v4i*)(stage + (i * 8 + srow) * 128 + ((apc ^ srow) << 4)) = v;  // (a wave's LDS operations execute in order)
         }
-        // (no `if (b < myb)` here: the compiler would sink the block's filter loads into it, next to
-        //  their use, one round trip each; a block the wave does not own multiplies zeros)
+        // (no `if (blk < blocks)` here: the compiler would sink the block's filter loads into it, next to
+        //  their use, one round trip each; a block that is not there multiplies zeros)
 #pragma unroll
         for (int cc = 0; cc < 4; ++cc) {
             const v4i bo = *(const v4i*)(stage + col * 128 + (((cc * 2 + kg) ^ (col & 7)) << 4));
@@ -351,28 +370,22 @@ __global__ void __launch_bounds__(64 * FO_WAVES) fc_one32_kernel(FcOneParams q) 
         }
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-        red[wave][e][lane] = acc[e];
+    for (int e = 0; e < 4; ++e)
+        *(v4i*)(stage + e * 1024 + lane * 16) = v4i{acc[4 * e], acc[4 * e + 1], acc[4 * e + 2], acc[4 * e + 3]};
     __syncthreads();
-    const int e4 = tid >> 6;
-    if (e4 >= 4)
+    if (wave >= 4)
         return;
-    const int row = row0 + col, ocb = oct * 32 + e4 * 8 + kg * 4;
+    const int row = row0 + col;
     if (row >= q.M || ocb >= q.OC)
         return;
-    int bias[4];
+    v4i sum = {bias[0], bias[1], bias[2], bias[3]};
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-        bias[e] = q.bias ? q.bias[min(ocb + e, q.OC - 1)] : 0;
+    for (int w = 0; w < FO_WAVES; ++w)
+        sum += *(const v4i*)(lds + w * 4096 + e4 * 1024 + lane * 16);
     int r[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        int sum = 0;
-#pragma unroll
-        for (int w = 0; w < FO_WAVES; ++w)
-            sum += red[w][e4 * 4 + e][lane];
-        r[e] = requant_conv_rt(q.act, sum + bias[e], q.s_src, q.s_flt, q.s_dst);
-    }
+    for (int e = 0; e < 4; ++e)
+        r[e] = requant_conv_rt(q.act, sum[e], q.s_src, q.s_flt, q.s_dst);
     int8_t* o = q.dst + (size_t)row * q.OC + ocb;
     if ((q.OC & 3) == 0) {
         *(u32_any*)o = pack4(r[0], r[1], r[2], r[3]);
@@ -411,7 +424,6 @@ TinyNNStatus fc_one_launch(
     q.OC = g.oc;
     q.OCP = (g.oc + OC_PAD - 1) / OC_PAD * OC_PAD;
     q.act = g.act;
-    q.last16 = (unsigned)((long)g.n * g.ic - 16);
     q.s_src = g.s_src;
     q.s_flt = g.s_flt;
     q.s_dst = g.s_dst;
@@ -424,13 +436,18 @@ TinyNNStatus fc_one_launch(
     const int nb = rows32 && g.ic <= 4096 ? ((g.ic + 127) / 128 + FO_WAVES - 1) / FO_WAVES : 0;  // blocks per wave
     note_kernel("fc_one", rows32 ? 32 : 64, nb, any ? 1 : -1);
     const dim3 grid32(oc_tiles, (g.n + 31) / 32), block(64 * FO_WAVES);
-    if (nb == 1)
-        hipLaunchKernelGGL((any ? fc_one32_kernel<1, true> : fc_one32_kernel<1, false>), grid32, block, 0, stream(), q);
-    else if (nb == 2)
-        hipLaunchKernelGGL((any ? fc_one32_kernel<2, true> : fc_one32_kernel<2, false>), grid32, block, 0, stream(), q);
-    else if (nb >= 3)
-        hipLaunchKernelGGL((any ? fc_one32_kernel<4, true> : fc_one32_kernel<4, false>), grid32, block, 0, stream(), q);
-    else if (rows32)
+    if (nb > 0) {
+        const bool odd = (g.ic & 3) || ((uintptr_t)src & 3);
+        q.src_off = (unsigned)((uintptr_t)src & 3);
+        q.src -= q.src_off;
+        q.src_bytes = (q.src_off + (unsigned)((long)g.n * g.ic) + 3) & ~3u;
+        void (*kern)(FcOneParams) = nb == 1   ? odd ? fc_one32_kernel<1, true> : fc_one32_kernel<1, false>
+                                    : nb == 2 ? odd ? fc_one32_kernel<2, true> : fc_one32_kernel<2, false>
+                                    : nb == 3 ? odd ? fc_one32_kernel<3, true> : fc_one32_kernel<3, false>
+                                    : odd     ? fc_one32_kernel<4, true>
+                                              : fc_one32_kernel<4, false>;
+        hipLaunchKernelGGL(kern, grid32, block, 0, stream(), q);
+    } else if (rows32)
         hipLaunchKernelGGL(fc_one_kernel<1>, dim3(oc_tiles, (g.n + 31) / 32), dim3(64 * FO_WAVES), 0, stream(), q);
     else
         hipLaunchKernelGGL(fc_one_kernel<2>, dim3(oc_tiles), dim3(64 * FO_WAVES), 0, stream(), q);

@@ -385,6 +385,8 @@ FC_PARTS = [
     (1025, 65, 1100, ",64,1"), (1500, 260, 1537, ",64,1"), (1100, 511, 1100, ",64,1"),
     (830, 2049, 961, ",64,4"), (833, 2052, 960, ",64,4"),
     (97, 2049, 97, ",32,4"), (97, 1028, 100, ",32,4"), (450, 16, 30, ",32,4"), (65, 1, 33, ",32,4"),
+    # up to 64 rows: one to four blocks a wave, some waves with one less, rows at odd bytes and on words
+    (40, 1025, 65, "fc_one:32,2"), (7, 1500, 33, "fc_one:32,2"), (31, 2501, 36, "fc_one:32,3"), (64, 3196, 31, "fc_one:32,4"),
     (2305, 384, 2561, "fc_tile"), (2305, 1024, 2561, "fc_tile"), (2049, 1024, 3841, "dma"),
 ]
 
