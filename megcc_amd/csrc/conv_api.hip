@@ -22,6 +22,8 @@ TinyNNStatus conv_mfma_pack(const ConvGeom& g, const void* flt, void* packed);
 TinyNNStatus conv_mfma_launch(const ConvGeom&, const void*, const void*, const void*, void*,
                               const Workspace*);
 size_t conv_mfma_workspace_bytes(const ConvGeom& g);
+bool conv_pw_stream_takes_stride(const ConvGeom& g);
+TinyNNStatus conv_pw_stream_launch(const ConvGeom&, const void*, const void*, const void*, void*);
 bool conv_hybrid_mfma_supported(const ConvGeom& g);
 TinyNNStatus conv_hybrid_mfma_launch(const ConvGeom&, const void*, const void*, const void*, void*);
 bool conv_dot4_supported(const ConvGeom& g);
@@ -169,8 +171,9 @@ static bool aligned16(const void* p) {
 
 // A 1x1 convolution with a stride (the projection shortcut of ResNet-like networks) reads one
 // input pixel per output pixel: it is the stride-1 pointwise convolution of the sub-sampled
-// input. The pixels it keeps are gathered into the workspace by one strided copy (4-byte
-// elements = a pixel's 4 channels), then the pointwise kernels run on dense data.
+// input. The streaming kernel reads them where they are (conv_pw_stream_takes_stride); for the others they
+// are gathered into the workspace by one strided copy (4-byte elements = a pixel's 4 channels), then the
+// pointwise kernels run on dense data. The workspace is asked for either way.
 static bool strided_pointwise(const ConvGeom& g) {
     return g.fmt == MEGCC_FMT_NCHW44 && g.groups == 1 && g.fh == 1 && g.fw == 1 && g.ph == 0 &&
            g.pw == 0 && (g.sh > 1 || g.sw > 1) && (g.ic & 3) == 0;
@@ -424,6 +427,11 @@ static TinyNNStatus conv2d_run(
                    TinyNN_ERROR_OUT_OF_RANGE,
                    "conv2d: a strided 1x1 convolution needs %zu bytes of workspace",
                    inner + gather_bytes(g));
+        // (pixels gathered first are out of the way of a result that lies over them)
+        const char *from_p = (const char*)src->ptr, *to_p = (const char*)dst->ptr;
+        const bool apart = from_p + (size_t)g.n * g.ic * g.ih * g.iw <= to_p || to_p + (size_t)g.n * g.oc * g.oh * g.ow <= from_p;
+        if (apart && conv_pw_stream_takes_stride(g) && !options().no_pws)
+            return conv_pw_stream_launch(g, src->ptr, flt->ptr, b, dst->ptr);  // (notes its own variant)
         void* gathered = (char*)workspace->ptr + inner;
         Layout from = {}, to = {};
         from.nr_dim = to.nr_dim = 3;  // [N * C/4, OH, OW] of 4-byte pixels

@@ -1,4 +1,4 @@
-// qsi8 pointwise (1x1, stride 1) NCHW44 convolution with few input channels: a streaming kernel.
+// qsi8 pointwise (1x1) NCHW44 convolution with few input channels, with or without a stride: a streaming kernel.
 //
 // With K = IC <= 512 a pointwise layer does one to sixteen MFMAs per 32 x 32 output tile and then
 // requantises 16 outputs per lane: the layer is bound by HBM and by the epilogue's vector
@@ -14,7 +14,7 @@
 //     tile's MFMAs;
 //   * results leave like in the tiled kernels: 4 consecutive accumulator registers are the 4
 //     channels of one NCHW44 dword, 32 lanes store 128 contiguous bytes.
-// Waves never synchronise after the set-up (threshold table and bias to LDS), so any number of
+// Waves never synchronise after the set-up (bias to LDS), so any number of
 // them can be resident and the memory latency is hidden by occupancy.
 //
 // Same arithmetic as the other qsi8 kernels: int32 accumulators starting from the bias, exact
@@ -46,7 +46,19 @@ struct PwParams {
     int act;
     RequantPack rq;
     FastDiv dOHW;
+    // STRIDED: bytes from an output row's / pixel's input to the next one's
+    int row_step, pix_step, OW;
+    FastDiv dOW;
 };
+
+// byte offset of an output pixel's input in its plane
+template <bool STRIDED>
+__device__ __forceinline__ int pw_pixel(const PwParams& q, int r) {
+    if (!STRIDED)
+        return r * 4;
+    const int y = (int)fdiv(r, q.dOW);
+    return y * q.row_step + (r - y * q.OW) * q.pix_step;
+}
 
 // KC: 32-channel K chunks (IC = 32 * KC). ACT: as in requant_dwords, -1 evaluates the
 // literal sequence with the run-time activation.
@@ -54,7 +66,7 @@ struct PwParams {
 // RG: ragged channel counts - IC below 32 * KC (the planes beyond IC are not fetched: out-of-range
 // offset, zeros; the packed filter holds zeros there too) and / or OC no multiple of 32 * MT (the last
 // wave's surplus channels are computed from zero filter rows and not stored).
-template <int KC, int MT, int ACT, bool RG = false>
+template <int KC, int MT, int ACT, bool RG, bool STRIDED>
 __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) {
     __shared__ __attribute__((aligned(16))) int bias_lds[PW_MAX_OC];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -96,7 +108,7 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
         const int p = tile * 32 + col;
         const int n = fdiv(p, q.dOHW);
         return tile < tend && p < q.P
-                       ? (unsigned)(n * q.image_stride + (p - n * q.OHW) * 4 + kg * 4 * q.plane_stride)
+                       ? (unsigned)(n * q.image_stride + pw_pixel<STRIDED>(q, p - n * q.OHW) + kg * 4 * q.plane_stride)
                        : 0x80000000u;
     };
     const int planes_left = q.IC4 - 4 * kg;  // RG: this lane reads plane c * 8 + j while that is below
@@ -190,7 +202,7 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
 // words, no bank conflicts). Two LDS tiles: the chunks of tile t + 1 are requested before tile t
 // is computed and written after it, one barrier per tile. A quarter of the L2 traffic and of the
 // load instructions of the streaming form.
-template <int KC, int ACT>
+template <int KC, int ACT, bool STRIDED>
 __global__ void __launch_bounds__(PW_THREADS) conv_pw_share_kernel(PwParams q) {
     static_assert(KC % 4 == 0, "a quarter of the chunks per wave");
     constexpr int CW = KC / 4;  // chunks a wave fetches per tile
@@ -220,7 +232,7 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_share_kernel(PwParams q) {
         const int p = tile * 32 + col;
         const int n = fdiv(p, q.dOHW);
         return tile < tend && p < q.P
-                       ? (unsigned)(n * q.image_stride + (p - n * q.OHW) * 4 + kg * 4 * q.plane_stride)
+                       ? (unsigned)(n * q.image_stride + pw_pixel<STRIDED>(q, p - n * q.OHW) + kg * 4 * q.plane_stride)
                        : 0x80000000u;
     };
     // this wave's chunks wave * CW .. + CW - 1 of `tile`
@@ -303,16 +315,30 @@ static int pw_resident_blocks(const void* kern) {
     return cache[kern] = n;
 }
 
-bool conv_pw_stream_supported(const ConvGeom& g) {
+static bool pw_stream_layer(const ConvGeom& g) {
     const long P = (long)g.n * g.oh * g.ow;
-    return g.fmt == MEGCC_FMT_NCHW44 && g.groups == 1 && g.fh == 1 && g.fw == 1 && g.sh == 1 &&
-           g.sw == 1 && g.ph == 0 && g.pw == 0 && (g.ic & 3) == 0 && (g.oc & 3) == 0 && (g.ic <= 512 ||
+    return g.fmt == MEGCC_FMT_NCHW44 && g.groups == 1 && g.fh == 1 && g.fw == 1 && g.ph == 0 && g.pw == 0 && (g.ic & 3) == 0 && (g.oc & 3) == 0 && (g.ic <= 512 ||
             // (1024: layers too small for the LDS-staged kernel, where one round trip wins, and the
             //  workgroup-shared form up to a few thousand pixels)
             (g.ic == 1024 && (P < 2048 || (P <= 4096 && (g.oc & 127) == 0 && !options().no_pwshare &&
                                          (P + 31) / 32 * (g.oc / 128) >= 256)))) &&
            ((g.oc & 63) == 0 || g.ic <= 512) && g.oc <= PW_MAX_OC && P >= 32 &&
            (long)g.n * g.ic * g.ih * g.iw < (1L << 31) && P * g.oc < (1L << 31);
+}
+
+bool conv_pw_stream_supported(const ConvGeom& g) {
+    return g.sh == 1 && g.sw == 1 && pw_stream_layer(g);
+}
+
+// A layer with a stride whose pixels are read where they are instead of gathered by a kernel of its own first (us gathered /
+// here: 6 x 20 -> 56 56 x 58 6.9 / 3.5, 64 x 32 -> 32 112 x 112 12.7 / 6.0, 64 x 256 -> 64 56 x 56 16.3 / 8.6, 32 x 256 -> 512 56 x 56 19.2 /
+// 18.8, 16 x 512 -> 512 28 x 28 9.5 / 6.0). A pixel of every line read is one of two, for each group of channels again: many groups of a
+// long K on a large map are better off with dense pixels (8 x 500 -> 500 40 x 40 10.6 / 11.5, 32 x 512 -> 400 28 x 28 15.7 / 16.4, 64 x
+// 512 -> 512 28 x 28 19.4 / 22.8; 2 x 1024 -> 1024 28 x 28 8.3 / 8.8).
+bool conv_pw_stream_takes_stride(const ConvGeom& g) {
+    const bool share = g.ic == 512 && g.oc % 128 == 0;  // (four groups side by side read them once)
+    const long reads = (long)g.n * g.oh * g.ow * g.ic * (share ? g.oc / 128 : (g.oc + 31) / 32);
+    return (g.sh > 1 || g.sw > 1) && g.ic <= 512 && (g.ic <= 256 || g.oc <= 256 || reads <= 20L << 20) && pw_stream_layer(g);
 }
 
 TinyNNStatus conv_pw_stream_launch(
@@ -336,19 +362,23 @@ TinyNNStatus conv_pw_stream_launch(
     const int per_wave = kc > 8 ? 32 : 64;
     const bool ragged = g.ic != kc * 32 || g.oc % per_wave != 0;
     q.groups = (g.oc + per_wave - 1) / per_wave;
-    q.image_stride = g.ic * q.OHW;
-    q.plane_stride = q.OHW * 4;
+    q.image_stride = g.ic * g.ih * g.iw;
+    q.plane_stride = g.ih * g.iw * 4;
+    const bool strided = g.sh > 1 || g.sw > 1;
+    q.row_step = g.sh * g.iw * 4, q.pix_step = g.sw * 4, q.OW = g.ow;
+    q.dOW = make_fastdiv(g.ow);
     q.act = g.act;
     q.dOHW = make_fastdiv(q.OHW);
     q.rq = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
     const int act = q.rq.mode ? g.act : -1;
 
     const void* kern = nullptr;
-#define MG_PW_PICK_RG(KC_, MT_, RG_)                                                                      \
-    (act == MEGCC_NONLINE_IDENTITY ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_IDENTITY, RG_> \
-     : act == MEGCC_NONLINE_RELU   ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_RELU, RG_>     \
-     : act == MEGCC_NONLINE_H_SWISH ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_H_SWISH, RG_> \
-                                   : (const void*)conv_pw_stream_kernel<KC_, MT_, -1, RG_>)
+#define MG_PW_PICK_ST(KC_, MT_, RG_, ST_)                                                                      \
+    (act == MEGCC_NONLINE_IDENTITY ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_IDENTITY, RG_, ST_> \
+     : act == MEGCC_NONLINE_RELU   ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_RELU, RG_, ST_>     \
+     : act == MEGCC_NONLINE_H_SWISH ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_H_SWISH, RG_, ST_> \
+                                   : (const void*)conv_pw_stream_kernel<KC_, MT_, -1, RG_, ST_>)
+#define MG_PW_PICK_RG(KC_, MT_, RG_) (strided ? MG_PW_PICK_ST(KC_, MT_, RG_, true) : MG_PW_PICK_ST(KC_, MT_, RG_, false))
 #define MG_PW_PICK(KC_, MT_) (ragged ? MG_PW_PICK_RG(KC_, MT_, true) : MG_PW_PICK_RG(KC_, MT_, false))
     switch (kc) {
         case 1: kern = MG_PW_PICK(1, 2); break;
@@ -360,16 +390,19 @@ TinyNNStatus conv_pw_stream_launch(
     }
 #undef MG_PW_PICK
 #undef MG_PW_PICK_RG
+#undef MG_PW_PICK_ST
 
     // 512 input channels and more tiles than resident waves: the workgroup-shared form
     if ((g.ic == 512 || g.ic == 1024) && !ragged && (q.groups & 3) == 0 && !options().no_pwshare) {
-#define MG_PWS_PICK(KC_)                                                                                  \
-    (act == MEGCC_NONLINE_IDENTITY ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_IDENTITY>         \
-     : act == MEGCC_NONLINE_RELU   ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_RELU>             \
-     : act == MEGCC_NONLINE_H_SWISH ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_H_SWISH>         \
-                                   : (const void*)conv_pw_share_kernel<KC_, -1>)
+#define MG_PWS_PICK_ST(KC_, ST_)                                                                          \
+    (act == MEGCC_NONLINE_IDENTITY ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_IDENTITY, ST_>    \
+     : act == MEGCC_NONLINE_RELU   ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_RELU, ST_>        \
+     : act == MEGCC_NONLINE_H_SWISH ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_H_SWISH, ST_>    \
+                                   : (const void*)conv_pw_share_kernel<KC_, -1, ST_>)
+#define MG_PWS_PICK(KC_) (strided ? MG_PWS_PICK_ST(KC_, true) : MG_PWS_PICK_ST(KC_, false))
         const void* sk = g.ic == 512 ? MG_PWS_PICK(16) : MG_PWS_PICK(32);
 #undef MG_PWS_PICK
+#undef MG_PWS_PICK_ST
         const long gblocks = q.groups / 4;
         const long capb = (long)num_cus() * pw_resident_blocks(sk);
         if ((long)q.tiles * gblocks >= capb / 2) {

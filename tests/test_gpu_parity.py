@@ -776,6 +776,26 @@ def test_strided_pointwise(case):
     compare(run_gpu(case, arrays), case.run_port(arrays), repr(case))
 
 
+STRIDED_1X1_IN_PLACE = [
+    # strided pixels read where they are: every number of K chunks, whole and ragged channels, maps of odd sides, several images in
+    # a tile, the workgroup-shared form, and a layer either side of where they are gathered first
+    *[ConvCase(A.FMT_NCHW44, A.DENSE, n, ic, ih, iw, oc, 1, s, 0, act, scales=(0.02, 0.01, unsat(ic)))
+      for n, ic, ih, iw, oc, s, act in (
+          (1, 32, 16, 9, 64, 2, A.RELU), (3, 20, 13, 11, 36, 2, A.IDENTITY), (2, 64, 21, 8, 64, 3, A.RELU),
+          (5, 40, 7, 7, 20, 2, A.H_SWISH), (2, 128, 12, 17, 128, 2, A.RELU), (1, 100, 23, 29, 68, 2, A.IDENTITY),
+          (1, 256, 15, 15, 64, 2, A.RELU), (2, 136, 19, 10, 12, 4, A.RELU), (1, 512, 13, 13, 32, 2, A.IDENTITY),
+          (2, 300, 11, 14, 100, 2, A.H_SWISH), (64, 512, 12, 12, 256, 2, A.RELU), (8, 500, 40, 40, 500, 2, A.RELU),
+          (1, 4, 63, 2, 4, 2, A.IDENTITY))],
+]
+
+
+@pytest.mark.parametrize("case", STRIDED_1X1_IN_PLACE, ids=[repr(c) for c in STRIDED_1X1_IN_PLACE])
+def test_strided_pointwise_in_place(case):
+    port.set_threads(8)
+    arrays = case.gen(seed=59)
+    compare(run_gpu(case, arrays), case.run_port(arrays), repr(case))
+
+
 DOT4 = [
     # dense NCHW44 layers the matrix-core kernels do not take (more than 9 taps): the dot-product
     # kernel; both channel-group widths, an odd number of channel groups, stride, dilation,
