@@ -187,37 +187,37 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) conv_gather_i8_kernel(Gathe
             }
     }
     __syncthreads();
+    requant_by_form<ACT>(q.rq, q.act, [&](const auto& form) __attribute__((always_inline)) {
 #pragma unroll
-    for (int x = 0; x < QUADS; ++x) {
-        if ((x & (kw - 1)) != grp)
-            continue;
-        const int i = x / (NT * 4), j = x / 4 % NT, e4 = x % 4;
-        int s[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            s[e] = acc[i][j][e4 * 4 + e];
-        // (the other groups from the one behind this wave's, no question which of them is its own: 256 -> 256 28 x 28 5.05 -> 4.75 us,
-        // 512 -> 512 7 x 7 7.0 -> 6.65)
-#pragma unroll
-        for (int g = 1; g < GATHER_WAVES; ++g) {
-            if (g >= kw)
-                break;
-            const v4i o = *(const v4i*)(parts + (((((grp + g) & (kw - 1)) * pw + sub) * QUADS + x) * 64 + lane) * 4);
+        for (int x = 0; x < QUADS; ++x) {
+            if ((x & (kw - 1)) != grp)
+                continue;
+            const int i = x / (NT * 4), j = x / 4 % NT, e4 = x % 4;
+            int s[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                s[e] += o[e];
-        }
-        const int oc = oc0 + 32 * i + 8 * e4 + 4 * kg;
-        const v4i bq = *(const v4i*)(bias + 32 * i + 8 * e4 + 4 * kg);
-        if (oc >= q.OC || p0 + 32 * j + col >= q.P)
-            continue;
+                s[e] = acc[i][j][e4 * 4 + e];
+            // (the other groups from the one behind this wave's, no question which of them is its own: 256 -> 256 28 x 28 5.05 -> 4.75 us,
+            // 512 -> 512 7 x 7 7.0 -> 6.65)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            s[e] += bq[e];
-        uint32_t d[1];
-        requant_dwords<ACT>(s, d, q.rq, q.act);
-        ((uint32_t*)q.dst)[((size_t)img[j] * (q.OC >> 2) + (oc >> 2)) * q.OHW + rem[j]] = d[0];
-    }
+            for (int g = 1; g < GATHER_WAVES; ++g) {
+                if (g >= kw)
+                    break;
+                const v4i o = *(const v4i*)(parts + (((((grp + g) & (kw - 1)) * pw + sub) * QUADS + x) * 64 + lane) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    s[e] += o[e];
+            }
+            const int oc = oc0 + 32 * i + 8 * e4 + 4 * kg;
+            const v4i bq = *(const v4i*)(bias + 32 * i + 8 * e4 + 4 * kg);
+            if (oc >= q.OC || p0 + 32 * j + col >= q.P)
+                continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s[e] += bq[e];
+            ((uint32_t*)q.dst)[((size_t)img[j] * (q.OC >> 2) + (oc >> 2)) * q.OHW + rem[j]] = form(s[0], s[1], s[2], s[3]);
+        }
+    });
 }
 
 size_t conv_mfma_packed_bytes(const ConvGeom& g);

@@ -246,6 +246,9 @@ __device__ __forceinline__ uint32_t pack4_perm(int a, int b, int c, int d) {
 // it is non-decreasing in a, so it equals the reference on all of int32 iff it does on both sides of each
 // of its steps: the host search (requant_table.hip) checks exactly that. (IDENTITY has no mode 2.)
 //     mode 4 (IDENTITY): requant_conv_affine's pair, which more scales have - the 128 cost the sum one bit.
+//     mode 6 (IDENTITY): trunc(fma(x, c, copysign(d, x))) with mode 2's x: half away from zero is one function of the magnitude, so an
+// exact tie is a step like any other, and only the steps of one sign bound c and d. Most of IDENTITY's scales that have neither of
+// the above up to a K of a thousand (300 input channels, calibrated scales: 116 of 157).
 //     mode 3: the reference's own sequence, for scales with exact ties whose roundings land on either side and for
 // H_SWISH. Its division costs two instructions: with c + d the 48-bit reciprocal of s_dst, v = fma(x, c, x d) is
 // the quotient to 2^-47 before its one rounding, so it is the correctly rounded one but for quotients that close
@@ -257,7 +260,7 @@ __device__ __forceinline__ uint32_t pack4_perm(int a, int b, int c, int d) {
 // those of the float 1.5 * 2^23 + a + m as long as |a + m| < 2^22, where all steps lie (it is asked for), and beyond
 // that floats that still grow with a. d is about 10^4 / c of its last bit there, too coarse to put it between the
 // steps; the whole number m, a few hundred at most, shifts them until a float falls there.
-// Vector instructions for four outputs: 10 (mode 5), 14, 18 - 22, 19, and mode 3 30 (RELU), 39 (IDENTITY), 46 (H_SWISH); the
+// Vector instructions for four outputs: 10 (mode 5), 14, 18 - 22, 19, 31 (mode 6), and mode 3 30 (RELU), 39 (IDENTITY), 46 (H_SWISH); the
 // threshold table's look-ups took 35 (H_SWISH 51) and four gathers from LDS, and its 1 KB among a launch's
 // arguments 0.7 us of the host's time.
 // (mode 0: none of these was proven; s1, s2, c are then the reference's three scales, for requant_conv)
@@ -270,7 +273,7 @@ struct RequantPack {
 RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst, bool affine);
 // mode 5, or mode 0 where it has no constants
 RequantPack requant_shifted_for(int act, float s_src, float s_flt, float s_dst);
-// for kernels whose sums start from requant_start(): mode 5 where there is one, else 2, 4, 3 or 0 (mode 1 as mode 2 with products by
+// for kernels whose sums start from requant_start(): mode 5 where there is one, else 2, 4, 6, 3 or 0 (mode 1 as mode 2 with products by
 // one); `affine` as above
 RequantPack requant_started_for(int act, float s_src, float s_flt, float s_dst, bool affine);
 // A bias for mode 5. Clamped: sums of a few thousand products on top of +-2^29 have the outputs of the largest and the smallest sums.
@@ -280,7 +283,7 @@ __device__ __forceinline__ int requant_bias(int bias, const RequantPack& q) {
 __device__ __forceinline__ int requant_start(int bias, const RequantPack& q) {
     return q.mode == 5 ? requant_bias(bias, q) : bias;  // (uniform)
 }
-// what a launch uses: modes 1, 2 and 4 unless the switch "noaffine" is on (a launch with them is noted as "+affine")
+// what a launch uses: modes 1, 2, 4 and 6 unless the switch "noaffine" is on (a launch with them is noted as "+affine")
 RequantPack requant_pack_pick(int act, float s_src, float s_flt, float s_dst);
 
 // MODE, ACT compile-time; channels (or pixels) 0..3 of one dword
@@ -307,6 +310,15 @@ __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3
         if (ACT == MEGCC_NONLINE_IDENTITY)
             return pack4_perm(o[0], o[1], o[2], o[3]);
         return (r >> 1) & 0x7f7f7f7fu;
+    } else if constexpr (MODE == 6) {
+        int o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float x = (float)a[i] * q.s1 * q.s2;
+            const int t = cvt_i32(__builtin_fmaf(x, q.c, __builtin_copysignf(q.d, x)));
+            o[i] = t > 127 ? 127 : (t < -128 ? -128 : t);
+        }
+        return pack4_perm(o[0], o[1], o[2], o[3]);
     } else if constexpr (MODE == 4) {
         int o[4];
 #pragma unroll
@@ -327,15 +339,15 @@ __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3
 
 // N accumulators -> N / 4 dwords (each 4 consecutive ones), the form by a uniform branch. ACT < 0: the literal sequence of
 // `act` (mode 0, SIGMOID), whose scales stand where mode 0 has them. STARTED: the sums started from requant_start().
-// The empty volatile statements keep each form inside its branch: the compiler otherwise computes one of
-// them ahead of the branch and throws it away, 80 instructions of 120.
+// The empty volatile statement keeps each form inside its branch: the compiler otherwise computes one of them ahead of the
+// branch and throws it away, 80 instructions of 120. (On the four constants: on the sums themselves it copied every
+// one of them: 16 x 300 -> 300 56 x 56 pointwise 21.6 / 19.9 us, of IDENTITY 23.9 / 22.2, 11 x 296 -> 208 86 x 101 31.6 / 29.7.)
 template <int ACT, bool STARTED = false, int N>
 __device__ __forceinline__ void requant_dwords(int (&a)[N], uint32_t (&out)[N / 4], const RequantPack& q, int act = ACT) {
+    RequantPack p = q;
     auto here = [&]() __attribute__((always_inline)) {
 #ifndef MG_HOST_AUDIT
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-            asm volatile("" : "+v"(a[i]));
+        asm volatile("" : "+s"(p.s1), "+s"(p.s2), "+s"(p.c), "+s"(p.d));
 #endif
     };
     if constexpr (ACT < 0) {
@@ -355,17 +367,63 @@ __device__ __forceinline__ void requant_dwords(int (&a)[N], uint32_t (&out)[N / 
         here();
 #pragma unroll
         for (int i = 0; i < N / 4; ++i)
-            out[i] = requant_pack4<STARTED ? 5 : 1, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+            out[i] = requant_pack4<STARTED ? 5 : 1, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], p);
     } else if (ACT == MEGCC_NONLINE_RELU ? q.mode == 2 : q.mode == 4) {
         here();
 #pragma unroll
         for (int i = 0; i < N / 4; ++i)
-            out[i] = requant_pack4<ACT == MEGCC_NONLINE_RELU ? 2 : 4, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+            out[i] = requant_pack4<ACT == MEGCC_NONLINE_RELU ? 2 : 4, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], p);
+    } else if (ACT == MEGCC_NONLINE_IDENTITY && q.mode == 6) {
+        here();
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i)
+            out[i] = requant_pack4<6, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], p);
     } else {
         here();
 #pragma unroll
         for (int i = 0; i < N / 4; ++i)
-            out[i] = requant_pack4<3, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], q);
+            out[i] = requant_pack4<3, ACT>(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3], p);
+    }
+}
+
+// One form for a whole epilogue: f(form) in the branch of q's mode, form(a0, a1, a2, a3) -> dword. For epilogues of many separate
+// dwords, whose every one had the branches in front of it (64 x 64 outputs a wave: sixteen times; 34 x 44 -> 60 67 x 67 3x3 17.4 / 16.1 us).
+template <int MODE, int ACT>
+struct RequantForm {
+    RequantPack q;
+    int act;
+    __device__ __forceinline__ uint32_t operator()(int a0, int a1, int a2, int a3) const {
+        if constexpr (MODE < 0)
+            return pack4_perm(requant_conv_rt(act, a0, q.s1, q.s2, q.c), requant_conv_rt(act, a1, q.s1, q.s2, q.c),
+                              requant_conv_rt(act, a2, q.s1, q.s2, q.c), requant_conv_rt(act, a3, q.s1, q.s2, q.c));
+        else
+            return requant_pack4<MODE, ACT>(a0, a1, a2, a3, q);
+    }
+};
+template <int ACT, typename F>
+__device__ __forceinline__ void requant_by_form(const RequantPack& q, int act, F f) {
+    RequantPack p = q;
+    auto here = [&]() __attribute__((always_inline)) {
+#ifndef MG_HOST_AUDIT
+        asm volatile("" : "+s"(p.s1), "+s"(p.s2), "+s"(p.c), "+s"(p.d));  // (as in requant_dwords)
+#endif
+    };
+    if constexpr (ACT < 0) {
+        f(RequantForm<-1, ACT>{p, act});
+    } else if constexpr (ACT == MEGCC_NONLINE_H_SWISH) {
+        f(RequantForm<3, ACT>{p, act});
+    } else if (q.mode == 1) {  // (uniform)
+        here();
+        f(RequantForm<1, ACT>{p, act});
+    } else if (ACT == MEGCC_NONLINE_RELU ? q.mode == 2 : q.mode == 4) {
+        here();
+        f(RequantForm<ACT == MEGCC_NONLINE_RELU ? 2 : 4, ACT>{p, act});
+    } else if (ACT == MEGCC_NONLINE_IDENTITY && q.mode == 6) {
+        here();
+        f(RequantForm<6, ACT>{p, act});
+    } else {
+        here();
+        f(RequantForm<3, ACT>{p, act});
     }
 }
 

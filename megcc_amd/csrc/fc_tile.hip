@@ -232,19 +232,20 @@ __global__ void __launch_bounds__(256 * KW) fc_tile_kernel(FcTileParams q) {
 #pragma unroll
         for (int mi = 0; mi < MT; ++mi)
 #pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                const int ocl = wm * (32 * MT) + mi * 32 + e4 * 8 + kg * 4;
-                const v4i bv = *(const v4i*)(bias_lds + ocl);
+            for (int ni = 0; ni < NT; ++ni) {
+                int a[16];
 #pragma unroll
-                for (int ni = 0; ni < NT; ++ni) {
-                    int a[4];
+                for (int e4 = 0; e4 < 4; ++e4) {
+                    const v4i bv = *(const v4i*)(bias_lds + wm * (32 * MT) + mi * 32 + e4 * 8 + kg * 4);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        a[e] = acc[mi][ni][e4 * 4 + e] + bv[e];
-                    uint32_t d[1];
-                    requant_dwords<ACT>(a, d, q.rq, q.act);
-                    *(uint32_t*)(lds + (wn * (32 * NT) + ni * 32 + col) * OPITCH + ocl) = d[0];
+                        a[e4 * 4 + e] = acc[mi][ni][e4 * 4 + e] + bv[e];
                 }
+                uint32_t d[4];
+                requant_dwords<ACT>(a, d, q.rq, q.act);
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4)
+                    *(uint32_t*)(lds + (wn * (32 * NT) + ni * 32 + col) * OPITCH + wm * (32 * MT) + mi * 32 + e4 * 8 + kg * 4) = d[e4];
             }
     }
     __syncthreads();

@@ -271,9 +271,13 @@ static int pack_eval(int a, int act, const RequantPack& q) {
         u += (uint32_t)a;
         memcpy(&x, &u, 4);
     }
-    if (q.mode == 2 || q.mode == 3)
+    if (q.mode == 2 || q.mode == 3 || q.mode == 6)
         x = x * q.s1 * q.s2;
     float y;
+    if (q.mode == 6) {
+        const float t = truncf(fmaf(x, q.c, copysignf(q.d, x)));  // (v_cvt_i32_f32 truncates and saturates)
+        return (int)std::min(std::max(t, -128.f), 127.f);
+    }
     if (q.mode == 3) {
         float v = fmaf(x, q.c, x * q.d);
         if (act == MEGCC_NONLINE_IDENTITY)
@@ -291,7 +295,42 @@ static int pack_eval(int a, int act, const RequantPack& q) {
     return act == MEGCC_NONLINE_IDENTITY ? u - 128 : u >> 1;
 }
 
-// Mode 1, 2 or 4, or mode 0 where none has constants.
+// Mode 6, or mode 0 where it has no constants. Of IDENTITY's steps those above zero and the one to -128: the others are their
+// mirror images, here as in the reference (which is checked like the rest).
+static RequantPack pack_symmetric(const RequantSteps& pts, float s_src, float s_flt, float s_dst) {
+    RequantBounds<true> from;  // trunc(x c + d) == y  <=>  y <= x c + d < y + 1
+    RequantBounds<false> to;
+    auto value = [&](int a) { return std::fabs((double)((float)a * s_src * s_flt)); };
+    for (int i = 2; i < pts.n; ++i) {
+        if (pts.y[i] > 0)
+            from.add(value(pts.a[i]), (double)pts.y[i], i);
+        if (pts.y[i] >= 0 && pts.a[i] >= 0 && pts.y[i] < 127)
+            to.add(value(pts.a[i]), (double)pts.y[i] + 1, i);
+    }
+    for (int i = 2; i < pts.n; ++i) {
+        if (pts.y[i] == -128)
+            from.add(value(pts.a[i]), 128., i);
+        if (pts.y[i] == -127 && pts.a[i - 1] == pts.a[i] - 1)
+            to.add(value(pts.a[i]), 128., i);
+    }
+    const float c0 = 1.f / s_dst;
+    for (int k = 0; k <= 8; ++k) {  // (up to 48: one scale in a hundred more)
+        const float c = by_ulps(c0, (k & 1) ? (k + 1) / 2 : -(k / 2));
+        const double dlo = from.tightest((double)c), dhi = to.tightest((double)c);
+        if (!(dlo <= dhi))
+            continue;
+        static const double kPos[] = {0.5, 0.375, 0.625, 0.25, 0.75, 0.125, 0.875};
+        for (double pos : kPos) {
+            const RequantPack q = {s_src, s_flt, c, (float)(dlo + (dhi - dlo) * pos), 6};
+            if (q.d >= 0.f && q.d < 1.f &&
+                requant_verified(pts, from, to, [&](int a) { return pack_eval(a, MEGCC_NONLINE_IDENTITY, q); }))
+                return q;
+        }
+    }
+    return {s_src, s_flt, s_dst, 0.f, 0};
+}
+
+// Mode 1, 2, 4 or 6, or mode 0 where none has constants.
 static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst) {
     RequantPack found = {s_src, s_flt, s_dst, 0.f, 0};
     const bool relu = act == MEGCC_NONLINE_RELU;
@@ -342,6 +381,8 @@ static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst) {
         const RequantAffine a = requant_affine_for(act, s_src, s_flt, s_dst);
         if (a.d != 0.f)
             found = {0.f, 0.f, a.c, a.d, 4};
+        else
+            found = pack_symmetric(pts, s_src, s_flt, s_dst);
     }
     return found;
 }

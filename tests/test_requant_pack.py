@@ -18,7 +18,7 @@ def _calibrated(taps, seed):
 
 
 SCALES = [(0.02, 0.01, 0.05), (0.01, 0.01, 0.1), (0.25, 0.5, 0.125), (0.5, 0.5, 0.1), (0.0013, 0.00127, 0.9), (0.001, 0.001, 0.9),
-          *[_calibrated(t, 7 * t + k) for t in (9, 64, 256, 800, 4096) for k in range(3)]]
+          *[_calibrated(t, 7 * t + k) for t in (9, 64, 256, 300, 800, 4096) for k in range(3)]]
 
 
 @pytest.mark.gpu
