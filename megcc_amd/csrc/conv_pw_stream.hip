@@ -423,7 +423,11 @@ TinyNNStatus conv_pw_stream_launch(
     // once - a small layer is then one memory round trip - and never more than are resident (every
     // wave pays the set-up once and then streams over its tiles)
     const long items = (long)q.tiles * q.groups;
-    const long cap = (long)num_cus() * 4 * pw_resident_blocks(kern);
+    // (256 input channels: two workgroups a CU of the three that fit - each wave fetches 16 KB of filter rows before its first tile. us with
+    // three / two: 16 x 200 -> 300 56 x 56 12.0 / 11.4, 32 x 256 -> 256 28 x 28 7.1 / 6.7, 32 x 256 -> 512 56 x 56 stride 2 18.7 / 17.1; one 15.8 on
+    // that, 13.7 on the first. 128: 9.2 / 8.9 and 18.5 / 19.6)
+    const long resident = pw_resident_blocks(kern);
+    const long cap = (long)num_cus() * 4 * (kc == 8 && resident > 2 ? 2 : resident);
     long waves = items < cap ? items : cap;
     long gcd = q.groups, rest = 4;  // unit = lcm(groups, waves per workgroup)
     while (rest) {
