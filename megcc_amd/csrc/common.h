@@ -123,6 +123,18 @@ TinyNNStatus stem_run(const StemAttr& attr, Tensor** inputs, int nr_input, Tenso
 // After a kernel launch: surfaces launch-configuration errors as TinyNN_ERROR_RUNTIME.
 TinyNNStatus check_launch(const char* what);
 
+// device.cpp: small reads of device memory by a blocking caller, through pinned memory of their own. A copy to pageable memory and the
+// wait for it took 28 us behind a forward of 100; here a kernel writes the bytes and then a number to pinned memory, and the host
+// looks for the number: less than the wait for the stream alone (us behind 280 of work: 4 KB 316 / 285, 64 KB 348 / 290,
+// the wait with no copy 288). Reads of more than HOST_STAGE_BYTES, and one while another thread's is under way, go by the copy.
+static constexpr size_t HOST_STAGE_BYTES = 64 << 10;
+struct HostStage;
+HostStage* host_stage_create();  // NULL: no pinned memory
+void host_stage_destroy(HostStage* stage);
+TinyNNStatus host_stage_read(HostStage* stage, void* host, const void* src, size_t bytes);
+// relayout.hip: `bytes` bytes to pinned memory, then `number` behind them all
+TinyNNStatus copy_to_host_launch(const void* src, void* pinned, size_t bytes, unsigned* where, unsigned number);
+
 // relayout.hip: copies `src` (layout sl) to `dst` (layout dl), elements of `es` bytes; one launch.
 TinyNNStatus strided_copy(
         const void* src, const Layout& sl, void* dst, const Layout& dl, size_t es, const char* who);

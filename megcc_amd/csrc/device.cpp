@@ -7,6 +7,7 @@
 #include <string.h>
 
 #include <atomic>
+#include <chrono>
 #include <mutex>
 #include <vector>
 
@@ -83,6 +84,60 @@ static std::atomic<unsigned long> g_library_waits, g_all_waits;
 
 HostWaits host_waits() {
     return {g_library_waits.load(), g_all_waits.load()};
+}
+
+struct HostStage {
+    std::mutex lock;
+    char* mem;  // HOST_STAGE_BYTES, and behind them the number
+    unsigned number;
+};
+
+HostStage* host_stage_create() {
+    HostStage* s = new HostStage;
+    if (hipHostMalloc((void**)&s->mem, HOST_STAGE_BYTES + 64, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        delete s;
+        return nullptr;
+    }
+    s->number = 0;
+    *(unsigned*)(s->mem + HOST_STAGE_BYTES) = 0;
+    return s;
+}
+
+void host_stage_destroy(HostStage* s) {
+    if (!s)
+        return;
+    (void)hipHostFree(s->mem);
+    delete s;
+}
+
+TinyNNStatus host_stage_read(HostStage* s, void* host, const void* src, size_t bytes) {
+    std::unique_lock<std::mutex> mine;
+    if (s && host && src && bytes && bytes <= HOST_STAGE_BYTES)
+        mine = std::unique_lock<std::mutex>(s->lock, std::try_to_lock);
+    if (!mine.owns_lock())
+        return megcc_gfx950_memcpy_d2h(host, src, bytes);
+    unsigned* const where = (unsigned*)(s->mem + HOST_STAGE_BYTES);
+    const unsigned number = ++s->number;
+    const TinyNNStatus st = copy_to_host_launch(src, s->mem, bytes, where, number);
+    if (st != TinyNN_SUCCESS)
+        return st;
+    // (a millisecond, then the runtime's own wait, which also reports what kept the number away)
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+    bool seen = false;
+    for (int i = 1; !(seen = __atomic_load_n(where, __ATOMIC_ACQUIRE) == number); ++i) {
+        __builtin_ia32_pause();
+        if ((i & 63) == 0 && std::chrono::steady_clock::now() > until)
+            break;
+    }
+    if (!seen) {
+        const hipError_t e = hipStreamSynchronize(stream());
+        MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "read of a tensor: %s", hipGetErrorString(e));
+        MG_REQUIRE(__atomic_load_n(where, __ATOMIC_ACQUIRE) == number, TinyNN_ERROR_RUNTIME, "read of a tensor: its copy did not run");
+    }
+    memcpy(host, s->mem, bytes);
+    ++g_library_waits;
+    return TinyNN_SUCCESS;
 }
 
 static std::vector<hipStream_t> g_aux_streams;

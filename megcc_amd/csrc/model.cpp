@@ -124,6 +124,7 @@ struct Model {
     // an asynchronous read -, nothing is left that the next forward's head could overlap, and on one stream it is over sooner, with
     // no event between head and tail (MobileNetV1, each forward waited for, us on two streams / one: batch 1 123 / 109, 4 139 /
     // 125, 8 145 / 129; with image in and result out, batch 1: 184 - 187 and unsteady / 171 - 173).
+    HostStage* stage = nullptr;  // get_output's, where an output is small enough for it
     HostWaits waits = {0, 0};
     int launched_tail = 0;  // entries of the last forward that went to the tail stream
     std::vector<char> waits_tail;
@@ -1072,6 +1073,7 @@ void megcc_gfx950_model_destroy(void* model) {
         (void)hipEventDestroy(m->ev_tail);
     if (m->tail_workspace)
         m->dev.free(m->tail_workspace);
+    host_stage_destroy(m->stage);
     for (auto* o : m->oprs) {
         if (o->processed_mem)
             m->dev.free(o->processed_mem);
@@ -1364,6 +1366,9 @@ TinyNNStatus megcc_gfx950_model_finalize(void* model) {
         return placed;
     if (m->tail_begin >= 0)
         settle_tail(m);
+    for (const ModelTensor* t : m->tensors)
+        if (t->is_output && !m->stage && tensor_bytes(t->t) <= HOST_STAGE_BYTES)
+            m->stage = host_stage_create();
     m->finalized = true;
     return megcc_gfx950_wait();
 }
@@ -1444,7 +1449,7 @@ TinyNNStatus megcc_gfx950_model_get_output(void* model, int tensor, void* host, 
     MG_REQUIRE(bytes == tensor_bytes(t), TinyNN_ERROR_INVALID_LAYOUT,
                "model_get_output: %zu bytes asked, tensor has %zu", bytes, tensor_bytes(t));
     join_tail(m);
-    return megcc_gfx950_memcpy_d2h(host, t.ptr, bytes);
+    return host_stage_read(m->stage, host, t.ptr, bytes);
 }
 
 // The copy is enqueued behind the forward that produced the tensor - on the tail stream when the last

@@ -578,6 +578,25 @@ TinyNNStatus strided_copy(
     return check_launch(who);
 }
 
+// One workgroup: the number may only be seen after every byte.
+__global__ void __launch_bounds__(1024) copy_to_host_kernel(const char* src, char* pinned, int n16, int bytes, unsigned* where, unsigned number) {
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    for (int i = threadIdx.x; i < n16; i += 1024)
+        ((v4i*)pinned)[i] = ((const v4i*)src)[i];
+    for (int i = n16 * 16 + threadIdx.x; i < bytes; i += 1024)
+        pinned[i] = src[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(where, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+TinyNNStatus copy_to_host_launch(const void* src, void* pinned, size_t bytes, unsigned* where, unsigned number) {
+    const int n16 = ((uintptr_t)src & 15) ? 0 : (int)(bytes / 16);
+    hipLaunchKernelGGL(copy_to_host_kernel, dim3(1), dim3(1024), 0, stream(), (const char*)src, (char*)pinned, n16, (int)bytes, where, number);
+    return check_launch("copy_to_host");
+}
+
 }  // namespace mg
 
 using namespace mg;
