@@ -18,9 +18,9 @@
 // 32 of its matrix units; on small layers too, 4 waves' steps of 5 loads each). Measured (us, before: the one-stage
 // kernel of conv_mfma_i8.hip, beyond 9 taps conv_dot4.hip; then with steps beyond a wave's share fetched as zeros, the
 // table read before the first operand and the arguments where they are used; now): 6 x 88 -> 148 57 x 43 stride 2
-// 14.6, 7.1, 5.9; 4 x 24 -> 68 98 x 98 stride 2 14.8, 5.7, 4.15; 1 x 356 -> 52 68 x 81 21.2, 8.4, 7.5; 1 x 256 -> 256 28 x 28
-// 8.0, 5.6, 4.8; 47 x 104 -> 48 89 x 89 95.8, 50.5, 40.3; 58 x 264 -> 320 70 x 70 stride 2 216, 176, 155; 5x5: 1 x 120 -> 280
-// 19 x 19 134, 6.6, 5.6; 60 x 28 -> 20 63 x 63 137, 21.4, 17.0.
+// 14.6, 7.1, 5.9 (5.3 with tiles by the rule at conv_gather_i8_launch); 4 x 24 -> 68 98 x 98 stride 2 14.8, 5.7, 4.15; 1 x 356 -> 52 68 x 81
+// 21.2, 8.4, 7.5; 1 x 256 -> 256 28 x 28 8.0, 5.6, 4.8; 47 x 104 -> 48 89 x 89 95.8, 50.5, 40.3; 58 x 264 -> 320 70 x 70 stride 2 216, 176,
+// 155; 5x5: 1 x 120 -> 280 19 x 19 134, 6.6, 5.6; 60 x 28 -> 20 63 x 63 137, 21.4, 17.0.
 // Reference loop: BareMetal/ConvKernel.cpp:305-344.
 #include "conv_mfma_i8.h"
 
@@ -233,27 +233,41 @@ bool conv_gather_i8_supported(const ConvGeom& g) {
 }
 
 // The layers this kernel takes from the LDS-direct one (its variant `picked`), by how many 32 x 32 tiles there are for a CU.
-// Measured over 340 3x3 and 5x5 layers of 16 .. 512 channels, 7 x 7 .. 100 x 100, batch 1 .. 40 (us there / here):
+// Measured over 640 3x3 and 5x5 layers of 16 .. 512 channels, 7 x 7 .. 112 x 112, batch 1 .. 64 (us there / here):
 //   * the small-layer variants 6 and 7, one 32-channel tile a workgroup: under two tiles a CU (256 -> 256 28 x 28 7.9 / 4.8,
 //     128 -> 128 28 x 28 N=4 5.25 / 4.6, 512 -> 512 28 x 28 10.4 / 9.7, 64 -> 64 14 x 14 N=16 5.2 / 3.9; beyond, 256 -> 256 28 x 28 N=3
 //     7.7 / 7.9, 512 -> 128 14 x 14 N=24 12.9 / 14.9); with 32 channels both are at a launch's time, 6 slightly below (4.3 / 4.45);
-//   * 1 and 4, 128 channels by 256 pixels on part of the CUs: under three (140 -> 96 24 x 22 N=8 7.6 / 5.2, 388 -> 80 39 x 39 N=4 13.8 /
-//     10.4, 176 -> 96 57 x 68 N=2 8.2 / 6.55, 32 -> 64 56 x 56 N=3 4.8 / 4.6; beyond, 380 -> 112 17 x 16 N=24 13.7 / 14.6, 396 -> 220
-//     69 x 73 stride 2 N=4 19.6 / 29.1, 256 -> 64 28 x 28 N=22 10.4 / 10.9);
+//   * 1 and 4, 128 (or 64) channels by 256 pixels on part of the CUs: under three (140 -> 96 24 x 22 N=8 7.6 / 5.2, 388 -> 80 39 x 39 N=4
+//     13.8 / 10.4, 176 -> 96 57 x 68 N=2 8.2 / 6.55, 32 -> 64 56 x 56 N=3 4.8 / 4.6; beyond, 380 -> 112 17 x 16 N=24 13.7 / 14.6, 228 -> 68 37 x
+//     43 N=12 11.8 / 13.4, 256 -> 64 28 x 28 N=22 10.4 / 10.9). From 128 channels on, where it is the taller tile that leaves CUs idle, under
+//     seven, for up to 36 steps eight (424 -> 344 31 x 31 N=5 19.6 / 16.5, 248 -> 316 50 x 50 N=2 13.7 / 11.4, 64 -> 164 56 x 56 N=3 7.4 / 5.6; 232 -> 204 23 x 23 N=16
+//     13.6 / 14.6), with a stride for up to 36 steps only (20 -> 316 28 x 19 N=35 6.4 / 5.4, 124 -> 340 54 x 66 N=6 10.2 / 10.0; 356 -> 184 25 x 25
+//     N=53 19.2 / 27.6), and, of 1, under sixteen with 32 input channels (20 -> 208 21 x 21 N=23 6.3 / 5.2, 32 -> 276 23 x 23 N=21 7.5 / 6.2; 20 -> 464
+//     19 x 19 N=25 7.7 / 8.1);
+//   * 0, 128 by 512, with 32 input channels: under 32 (20 -> 268 31 x 31 N=24 10.4 / 9.0, 28 -> 188 47 x 47 N=19 12.2 / 9.6, 20 -> 76 27 x 35
+//     N=55 8.7 / 7.6; beyond, 24 -> 240 55 x 55 N=17 13.2 / 14.4);
 //   * 8 and 9, a filter row a stage: under six (128 -> 64 56 x 56 N=5 16.7 / 10.9, 64 -> 60 54 x 48 N=8 10.7 / 9.0, 72 -> 140 23 x 26
-//     N=13 16.9 / 14.2; beyond, 172 -> 372 13 x 12 N=27 30.1 / 33.8) and under four (128 -> 32 56 x 56 stride 2 N=23 22.7 / 16.4, 292 ->
-//     112 90 x 63 stride 2 N=4 45.1 / 28.3; beyond, 256 -> 128 56 x 56 stride 2 N=11 44.4 / 48.0). Layers of 48 channels and fewer
-//     would gain too (32 -> 32 28 x 28 N=16 7.2 / 4.1) but are what the row-split kernel is tested with.
+//     N=13 16.9 / 14.2; beyond, 172 -> 372 13 x 12 N=27 30.1 / 33.8) and under four (128 -> 32 56 x 56 stride 2 N=23 22.7 / 16.4), with
+//     a stride under eight (80 -> 36 65 x 65 stride 2 N=30 20.1 / 17.2, 44 -> 224 42 x 42 15.1 / 12.0; beyond, 156 -> 496 64 x 72 N=4 30.5 /
+//     36.3). Rows of 40 pixels and more without a stride, whose patches leave 9 a 128-pixel tile, however many there are (84 -> 116
+//     102 x 112 N=9 95.7 / 50.1, 184 -> 192 60 x 60 N=10 92.4 / 54.1, 144 -> 512 97 x 97 N=3 107 / 79, 20 -> 152 110 x 110 N=35 177 / 88).
+//     Layers of 48 channels and fewer with fewer tiles than that would gain too (32 -> 32 28 x 28 N=16 7.2 / 4.1) but are what the
+//     row-split kernel is tested with.
 bool conv_gather_i8_wins(const ConvGeom& g, int picked) {
-    const long tiles = (((long)g.n * g.oh * g.ow + 31) / 32) * ((g.oc + 31) / 32);
+    const long tiles = (((long)g.n * g.oh * g.ow + 31) / 32) * ((g.oc + 31) / 32), cus = num_cus();
     const int taps = g.fh * g.fw;
+    const long steps = (long)((g.ic + 31) / 32) * taps;
+    const bool stride = g.sh > 1 || g.sw > 1, wide = !stride && g.iw >= 40;
     switch (picked) {
-        case 6: return tiles < 2L * num_cus() && (long)((g.ic + 31) / 32) * taps > 9;
-        case 7: return tiles < 2L * num_cus();
+        case 0: return taps > 1 && steps <= 9 && tiles < 32 * cus;
+        case 6: return tiles < 2 * cus && steps > 9;
+        case 7: return tiles < 2 * cus;
         case 1:
-        case 4: return tiles < 3L * num_cus() && taps > 1;
-        case 8: return tiles < 6L * num_cus() && g.ic > 48;
-        case 9: return tiles < 4L * num_cus() && g.ic > 48;
+        case 4:
+            return taps > 1 && (tiles < 3 * cus || (g.oc >= 128 && ((steps <= 36 ? tiles < 8 * cus : !stride && tiles < 7 * cus) ||
+                                                                   (picked == 1 && tiles < 16 * cus && steps <= 9))));
+        case 8: return tiles < 6 * cus && g.ic > 48;
+        case 9: return g.ic > 48 ? tiles < (stride ? 8 : 4) * cus || wide : tiles >= 24 * cus && wide;
         default: return false;
     }
 }
@@ -301,6 +315,29 @@ TinyNNStatus conv_gather_i8_launch(const ConvGeom& g, const void* src, const voi
     if (tiles() < full)
         mt = 1;
     if (mt * nt == 1) {
+        // With four groups a workgroup is one tile, and what bounds it is its CU's data path: 16 accesses of the L1 a step for 32 channels'
+        // filter, some 68 for 32 pixels (a dword a lane) - a larger tile is fewer accesses an output, unless its rounds over the
+        // CUs cost more. From 80 steps on with pixels too; a shorter K does not hide what the larger tile's sums cost (us 32 x 32 / 64
+        // channels x 32 pixels / 64 x 64: 56 x 164 -> 60 18 x 17 5x5 stride 2 20.7 / 13.1 / 22.2, 10 x 428 -> 476 17 x 16 stride 2 17.6 / 11.4 /
+        // 18.6, 13 x 196 -> 380 27 x 25 stride 2 16.6 / 10.9 / 10.9, 31 x 484 -> 172 30 x 22 5x5 stride 2 61.0 / 37.9 / 33.6, 9 x 176 -> 460
+        // 13 x 13 5x5 16.3 / 14.4 / 13.5, 1 x 176 -> 364 95 x 101 stride 2 10.8 / 8.2 / 8.6; one round either way: 1 x 256 -> 256 28 x 28 4.8 /
+        // 5.4 / 7.6; 420 layers of 5 us and more: 6 % in the mean, nothing by more than two runs differ).
+        auto port = [&](int m, int n) {
+            const long t = (long)((q.P + 32 * n - 1) / (32 * n)) * ((g.oc + 32 * m - 1) / (32 * m));
+            return (t + num_cus() - 1) / num_cus() * (16 * m + 68 * n);
+        };
+        long least = port(1, 1);
+        auto consider = [&](int m, int n, int steps) {
+            if (q.steps >= steps && (m == 1 || g.oc > 32) && port(m, n) < least)
+                least = port(m, n), mt = m, nt = n, kw = 4;
+        };
+        consider(2, 1, 25);
+        consider(2, 2, 80);
+        consider(1, 2, 80);
+    }
+    if (kw > 1) {
+        // (as just chosen)
+    } else if (mt * nt == 1) {
         while (kw < 4 && q.steps >= 8 * kw && (5 * tiles() * kw < 8 * full || q.steps >= 27))
             kw *= 2;
     } else if (mt * nt == 2) {
