@@ -5,7 +5,7 @@
 // them inside S*x0 - 4 .. S*x0 + 8*S + 3 while F/2 <= 3).
 //
 // A depthwise layer moves two bytes per output and has to requantise every output exactly, which
-// costs 7 vector instructions and a table look-up (epilogue.h). Done with v_dot4 the multiply-adds
+// costs 3 to 8 vector instructions and its share of a store (epilogue.h). Done with v_dot4 the multiply-adds
 // and the byte shuffling in front of them cost another 10 vector instructions per output, and the
 // layer is bound by the vector ALU at a third of the memory rate. Here the multiply-adds go to the
 // MFMA unit, which is otherwise idle, as a product with a banded matrix:
@@ -88,8 +88,8 @@ typedef unsigned dw_v4u __attribute__((ext_vector_type(4)));
 // are the halves of four pooling windows whose other halves the lane 32 further on holds: after the
 // vertical maximum the same two v_permlane32_swap that prepare the 16-byte stores of the plain
 // kernel hand each lane both halves of two windows; it stores 2 pixels of the final tensor.
-// Bound by the vector ALU beside memory: 267 vector instructions a tile (312 with a rounding of nine
-// instructions, a branch around each pixel's load and store): N=64 C=512 112x112 167 -> 150 us = 4.1 TB/s.
+// Bound by memory with the vector ALU beside it: N=64 C=512 112x112 167 us with a rounding of nine instructions and a branch around
+// each pixel's load and store, 150 with 267 vector instructions a tile, 144 = 4.3 TB/s since four outputs share a conversion.
 
 // S: stride (only 1 is instantiated: with stride 2 the layer reads four bytes per byte written and
 // the v_dot4 kernel of dwconv.hip already runs at the rate of a copy - measured 7.8 us against

@@ -85,7 +85,6 @@ __host__ __device__ __forceinline__ int requant_conv(int acc, float s_src, float
 struct RequantFast {
     float c;       // fl(fl(s_src*s_flt)/s_dst); 0 disables the fast path (extreme scales)
     float s_src, s_flt, s_dst;
-    float aff_c, aff_d;  // requant_conv_affine's pair when the launch picked one (below); aff_d == 0: none
 };
 
 // host side: c, or 0 when a scale is so extreme that the error bound above does not hold
@@ -99,7 +98,6 @@ static inline RequantFast make_requant_fast(float s_src, float s_flt, float s_ds
     auto mid = [](float x) { return x > 1e-30f && x < 1e30f; };
     const bool sane = mid(s_src) && mid(s_flt) && mid(p) && mid(s_dst) && mid(c);
     q.c = sane ? c : 0.f;
-    q.aff_c = q.aff_d = 0.f;
     return q;
 }
 
