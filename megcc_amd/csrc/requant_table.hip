@@ -133,7 +133,10 @@ struct RequantSteps {
         y[n++] = out;
     }
 };
-static RequantSteps requant_steps(const RequantTable& T, int lo) {
+static RequantSteps requant_steps(int act, float s_src, float s_flt, float s_dst) {
+    const std::shared_ptr<const RequantTable> table = requant_table_for(act, s_src, s_flt, s_dst);
+    const RequantTable& T = *table;
+    const int lo = act == MEGCC_NONLINE_IDENTITY ? -128 : 0;
     RequantSteps s;
     int first = lo + 128;  // (levels up to the lowest output have no step)
     int low = lo, high = lo;  // outputs of the smallest and the largest accumulator
@@ -156,6 +159,30 @@ static RequantSteps requant_steps(const RequantTable& T, int lo) {
     return s;
 }
 
+// A search for constants, F, for processors with a fused multiply-add, where fmaf, rintf and floorf are an instruction each, and for
+// the others, where they are calls of the library. All are exact: the results are the same.
+// (us on one core, scales of calibrated layers with 64 / 1152 / 4096 products to a sum, with this, one pass over the steps for all searches and
+// IDENTITY's two floors sharing their hulls: IDENTITY 26 / 25 / 26 -> 13 / 15 / 16, RELU 6.0 / 14.0 / 16.4 -> 4.9 / 11.9 / 14.4.)
+#define MG_INLINE __attribute__((always_inline))
+#if defined(__HIP_DEVICE_COMPILE__)
+#define MG_FMA
+#else
+#define MG_FMA __attribute__((target("fma")))
+#endif
+template <auto F>
+MG_FMA static auto search_fma(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
+    return F(act, s_src, s_flt, s_dst, pts);
+}
+template <auto F>
+static auto search(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
+#if !defined(__HIP_DEVICE_COMPILE__)
+    static const bool fma = __builtin_cpu_supports("fma");
+    if (fma)
+        return search_fma<F>(act, s_src, s_flt, s_dst, pts);
+#endif
+    return F(act, s_src, s_flt, s_dst, pts);
+}
+
 // Lower (or upper) bounds for d: at[i] - x[i] c <= d (>=), of which the largest (smallest) counts for a given c. Bounds come in
 // the order of x, and those that are the tightest for no c at all are dropped as they come: what stays is one side of the
 // points' convex hull, a dozen of 255, and a slope costs as many products. (All 255 kept, the searches below took 40 us.)
@@ -165,7 +192,7 @@ struct RequantBounds {
     double x[REQUANT_TABLE_ENTRIES], at[REQUANT_TABLE_ENTRIES];
     int point[REQUANT_TABLE_ENTRIES];  // which step's
     static bool tighter(double a, double b) { return LOWER ? a > b : a < b; }
-    void add(double v, double bound, int p) {
+    MG_INLINE void add(double v, double bound, int p) {
         if (n && x[n - 1] == v) {
             if (!tighter(bound, at[n - 1]))
                 return;
@@ -178,13 +205,18 @@ struct RequantBounds {
         at[n] = bound;
         point[n++] = p;
     }
-    double tightest(double c) const {
-        double m = LOWER ? -1e30 : 1e30;
-        for (int i = 0; i < n; ++i)
-            if (tighter(at[i] - x[i] * c, m))
-                m = at[i] - x[i] * c;
+    // (a hull: from the bound that was the tightest for another slope, downhill)
+    MG_INLINE double tightest(double c) {
+        if (!n)
+            return LOWER ? -1e30 : 1e30;
+        double m = at[best] - x[best] * c, v;
+        for (; best + 1 < n && tighter(v = at[best + 1] - x[best + 1] * c, m); ++best)
+            m = v;
+        for (; best > 0 && tighter(v = at[best - 1] - x[best - 1] * c, m); --best)
+            m = v;
         return m;
     }
+    int best = 0;
 };
 
 // the float `n` floats above (a positive, normal) v
@@ -198,7 +230,7 @@ static float by_ulps(float v, int n) {
 
 // whether `eval` gives the outputs of every step: first where the bounds are tightest, where a wrong candidate shows
 template <typename F>
-static bool requant_verified(const RequantSteps& pts, const RequantBounds<true>& from, const RequantBounds<false>& to, F eval) {
+MG_INLINE static bool requant_verified(const RequantSteps& pts, const RequantBounds<true>& from, const RequantBounds<false>& to, F eval) {
     for (int i = 0; i < from.n; ++i)
         if (eval(pts.a[from.point[i]]) != pts.y[from.point[i]])
             return false;
@@ -213,10 +245,48 @@ static bool requant_verified(const RequantSteps& pts, const RequantBounds<true>&
 
 // host evaluation of requant_conv_affine (fmaf is the correctly rounded single fused multiply-add,
 // floorf + saturation what v_cvt_flr_i32_f32 does)
-static int affine_eval(int a, float c, float d, int lo) {
+MG_INLINE static int affine_eval(int a, float c, float d, int lo) {
     const float g = floorf(fmaf((float)a, c, d));
     const float r = g < (float)lo ? (float)lo : (g > 127.f ? 127.f : g);
     return (int)r;
+}
+
+// from, to: y + up <= a c + d < y + 1 + up for an output y (another `up` moves the hulls as they are)
+MG_INLINE static RequantAffine affine_within(
+        const RequantSteps& pts, RequantBounds<true>& from, RequantBounds<false>& to, double up, int lo, float c0) {
+    RequantAffine found = {0.f, 0.f};
+    for (int k = 0; k <= 16 && found.d == 0.f; ++k) {
+        // c' = c0 moved (k + 1) / 2 ulps up (k odd) or down (k even)
+        const float c = by_ulps(c0, (k & 1) ? (k + 1) / 2 : -(k / 2));
+        const double dlo = from.tightest((double)c) - up, dhi = to.tightest((double)c) - up;
+        if (!(dlo < dhi))
+            continue;
+        // the middle of the interval first (the most room for the rounding of the fused multiply-add),
+        // then points nearer its ends
+        static const double kPos[] = {0.5, 0.375, 0.625, 0.25, 0.75};
+        for (double pos : kPos) {
+            const float d = (float)(dlo + (dhi - dlo) * pos);
+            if (!(d > 0.f && d < 1.f))
+                continue;
+            if (requant_verified(pts, from, to, [&](int a) MG_INLINE { return affine_eval(a, c, d, lo); })) {
+                found = {c, d};
+                break;
+            }
+        }
+    }
+    return found;
+}
+MG_INLINE static RequantAffine affine_constants(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
+    const int lo = act == MEGCC_NONLINE_RELU ? 0 : -128;
+    RequantBounds<true> from;  // floor(a c + d) == y  <=>  y <= a c + d < y + 1
+    RequantBounds<false> to;
+    for (int i = 2; i < pts.n; ++i) {  // (the ends of the range bound nothing)
+        if (pts.y[i] > lo)
+            from.add((double)(float)pts.a[i], (double)pts.y[i], i);
+        if (pts.y[i] < 127)
+            to.add((double)(float)pts.a[i], (double)pts.y[i] + 1, i);
+    }
+    return affine_within(pts, from, to, 0., lo, make_requant_fast(s_src, s_flt, s_dst).c);
 }
 
 RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst) {
@@ -228,42 +298,13 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
     RequantAffine found = none;
     if (cache.find(key, &found))
         return found;
-    const int lo = act == MEGCC_NONLINE_RELU ? 0 : -128;
-    const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), lo);
-    RequantBounds<true> from;  // floor(a c + d) == y  <=>  y <= a c + d < y + 1
-    RequantBounds<false> to;
-    for (int i = 2; i < pts.n; ++i) {  // (the ends of the range bound nothing)
-        if (pts.y[i] > lo)
-            from.add((double)(float)pts.a[i], (double)pts.y[i], i);
-        if (pts.y[i] < 127)
-            to.add((double)(float)pts.a[i], (double)pts.y[i] + 1, i);
-    }
-    const float c0 = make_requant_fast(s_src, s_flt, s_dst).c;
-    for (int k = 0; k <= 16 && found.d == 0.f; ++k) {
-        // c' = c0 moved (k + 1) / 2 ulps up (k odd) or down (k even)
-        const float c = by_ulps(c0, (k & 1) ? (k + 1) / 2 : -(k / 2));
-        const double dlo = from.tightest((double)c), dhi = to.tightest((double)c);
-        if (!(dlo < dhi))
-            continue;
-        // the middle of the interval first (the most room for the rounding of the fused multiply-add),
-        // then points nearer its ends
-        static const double kPos[] = {0.5, 0.375, 0.625, 0.25, 0.75};
-        for (double pos : kPos) {
-            const float d = (float)(dlo + (dhi - dlo) * pos);
-            if (!(d > 0.f && d < 1.f))
-                continue;
-            if (requant_verified(pts, from, to, [&](int a) { return affine_eval(a, c, d, lo); })) {
-                found = {c, d};
-                break;
-            }
-        }
-    }
+    found = search<affine_constants>(act, s_src, s_flt, s_dst, requant_steps(act, s_src, s_flt, s_dst));
     cache.put(key, found);
     return found;
 }
 
 // host evaluation of requant_pack4 for one output
-static int pack_eval(int a, int act, const RequantPack& q) {
+MG_INLINE static int pack_eval(int a, int act, const RequantPack& q) {
     float x = (float)a;
     if (q.mode == 5) {
         uint32_t u;
@@ -297,10 +338,10 @@ static int pack_eval(int a, int act, const RequantPack& q) {
 
 // Mode 6, or mode 0 where it has no constants. Of IDENTITY's steps those above zero and the one to -128: the others are their
 // mirror images, here as in the reference (which is checked like the rest).
-static RequantPack pack_symmetric(const RequantSteps& pts, float s_src, float s_flt, float s_dst) {
+MG_INLINE static RequantPack pack_symmetric(const RequantSteps& pts, float s_src, float s_flt, float s_dst) {
     RequantBounds<true> from;  // trunc(x c + d) == y  <=>  y <= x c + d < y + 1
     RequantBounds<false> to;
-    auto value = [&](int a) { return std::fabs((double)((float)a * s_src * s_flt)); };
+    auto value = [&](int a) MG_INLINE { return std::fabs((double)((float)a * s_src * s_flt)); };
     for (int i = 2; i < pts.n; ++i) {
         if (pts.y[i] > 0)
             from.add(value(pts.a[i]), (double)pts.y[i], i);
@@ -323,7 +364,7 @@ static RequantPack pack_symmetric(const RequantSteps& pts, float s_src, float s_
         for (double pos : kPos) {
             const RequantPack q = {s_src, s_flt, c, (float)(dlo + (dhi - dlo) * pos), 6};
             if (q.d >= 0.f && q.d < 1.f &&
-                requant_verified(pts, from, to, [&](int a) { return pack_eval(a, MEGCC_NONLINE_IDENTITY, q); }))
+                requant_verified(pts, from, to, [&](int a) MG_INLINE { return pack_eval(a, MEGCC_NONLINE_IDENTITY, q); }))
                 return q;
         }
     }
@@ -331,11 +372,10 @@ static RequantPack pack_symmetric(const RequantSteps& pts, float s_src, float s_
 }
 
 // Mode 1, 2, 4 or 6, or mode 0 where none has constants.
-static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst) {
+MG_INLINE static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
     RequantPack found = {s_src, s_flt, s_dst, 0.f, 0};
     const bool relu = act == MEGCC_NONLINE_RELU;
     const int lowest = relu ? 0 : -128;
-    const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), lowest);
     // the forms in order of cost: no product in front, one, two (IDENTITY, whose outputs are rounded 128 away from zero, hardly
     // ever has constants for those where it has none without)
     struct Form {
@@ -347,8 +387,6 @@ static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst) {
                           {2, s_src, 1.f, s_flt / s_dst * unit},
                           {2, s_src, s_flt, 1.f / s_dst * unit}};
     for (const Form& f : forms) {
-        if (f.mode == 2 && !relu)
-            break;
         RequantBounds<true> from;  // RELU: 2 y <= rint <= 2 y + 1; IDENTITY: rint == y + 128
         RequantBounds<false> to;
         for (int i = 2; i < pts.n; ++i) {
@@ -368,7 +406,7 @@ static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst) {
             static const double kPos[] = {0.5, 0.375, 0.625, 0.25, 0.75, 0.125, 0.875};
             for (double pos : kPos) {
                 const RequantPack q = {f.s1, f.s2, c, (float)(dlo + (dhi - dlo) * pos), f.mode};
-                if (requant_verified(pts, from, to, [&](int a) { return pack_eval(a, act, q); })) {
+                if (requant_verified(pts, from, to, [&](int a) MG_INLINE { return pack_eval(a, act, q); })) {
                     found = q;
                     break;
                 }
@@ -376,13 +414,14 @@ static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst) {
         }
         if (found.mode)
             break;
-    }
-    if (!found.mode && !relu) {
-        const RequantAffine a = requant_affine_for(act, s_src, s_flt, s_dst);
-        if (a.d != 0.f)
-            found = {0.f, 0.f, a.c, a.d, 4};
-        else
-            found = pack_symmetric(pts, s_src, s_flt, s_dst);
+        if (!relu) {
+            const RequantAffine a = affine_within(pts, from, to, 127.5, lowest, f.c0);
+            if (a.d != 0.f)
+                found = {0.f, 0.f, a.c, a.d, 4};
+            else
+                found = pack_symmetric(pts, s_src, s_flt, s_dst);
+            break;
+        }
     }
     return found;
 }
@@ -391,7 +430,7 @@ static RequantPack pack_affine(int act, float s_src, float s_flt, float s_dst) {
 // outputs can only differ where the reference's own value is within two of its floats of a step, 2 * 2^-17 for outputs up
 // to 128: accumulators on both sides of each step are compared, and as many beyond them as lie within 1e-4 of it (with
 // H_SWISH the output changes by half to one and a half of what the quotient does).
-static RequantPack pack_exact(int act, float s_src, float s_flt, float s_dst) {
+MG_INLINE static RequantPack pack_exact(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
     const RequantPack none = {s_src, s_flt, s_dst, 0.f, 0};
     auto mid = [](float s) { return s >= 1e-12f && s <= 1e12f; };  // (nothing overflows or loses bits on the way)
     const float c = make_requant_fast(s_src, s_flt, s_dst).c;
@@ -400,7 +439,6 @@ static RequantPack pack_exact(int act, float s_src, float s_flt, float s_dst) {
     const double inv = (act == MEGCC_NONLINE_RELU ? 2.0 : 1.0) / (double)s_dst;
     RequantPack q = {s_src, s_flt, (float)inv, 0.f, 3};
     q.d = (float)(inv - (double)q.c);
-    const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), act == MEGCC_NONLINE_IDENTITY ? -128 : 0);
     const long long near = (long long)(1e-4f / c);
     // (pts: the ends of the range, then each step's last accumulator below and first one above)
     for (int i = 0; i < pts.n; ++i) {
@@ -416,11 +454,10 @@ static RequantPack pack_exact(int act, float s_src, float s_flt, float s_dst) {
 
 // Mode 5: for each slope near the quotient the interval that mode 1's d may lie in, moved to where the sums' floats are; of the
 // shifts m up to 1023 those whose d comes closest to its middle are verified.
-static RequantPack pack_shifted(int act, float s_src, float s_flt, float s_dst) {
+MG_INLINE static RequantPack pack_shifted(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
     const RequantPack none = {s_src, s_flt, s_dst, 0.f, 0};
     const bool relu = act == MEGCC_NONLINE_RELU;
     const int lowest = relu ? 0 : -128;
-    const RequantSteps pts = requant_steps(*requant_table_for(act, s_src, s_flt, s_dst), lowest);
     RequantBounds<true> from;
     RequantBounds<false> to;
     for (int i = 2; i < pts.n; ++i) {
@@ -464,7 +501,7 @@ static RequantPack pack_shifted(int act, float s_src, float s_flt, float s_dst) 
             const int bits = 0x4b400000 + b.m;
             RequantPack q = {0.f, 0.f, c, (float)(middle - (double)c * b.m), 5};
             memcpy(&q.s1, &bits, 4);
-            if (b.off <= (dhi - dlo) / 2 && requant_verified(inner, from, to, [&](int a) { return pack_eval(a, act, q); }))
+            if (b.off <= (dhi - dlo) / 2 && requant_verified(inner, from, to, [&](int a) MG_INLINE { return pack_eval(a, act, q); }))
                 return q;
         }
     }
@@ -478,7 +515,7 @@ RequantPack requant_shifted_for(int act, float s_src, float s_flt, float s_dst) 
         return found;
     const auto key = cache.key(act, s_src, s_flt, s_dst);
     if (!cache.find(key, &found)) {
-        found = pack_shifted(act, s_src, s_flt, s_dst);
+        found = search<pack_shifted>(act, s_src, s_flt, s_dst, requant_steps(act, s_src, s_flt, s_dst));
         cache.put(key, found);
     }
     return found;
@@ -490,16 +527,20 @@ RequantPack requant_pack_for(int act, float s_src, float s_flt, float s_dst, boo
         return {s_src, s_flt, s_dst, 0.f, 0};
     const auto key = multiply_adds.key(act, s_src, s_flt, s_dst);
     RequantPack found;
+    RequantSteps pts;
     if (affine && act != MEGCC_NONLINE_H_SWISH) {
         if (!multiply_adds.find(key, &found)) {
-            found = pack_affine(act, s_src, s_flt, s_dst);
+            pts = requant_steps(act, s_src, s_flt, s_dst);
+            found = search<pack_affine>(act, s_src, s_flt, s_dst, pts);
             multiply_adds.put(key, found);
         }
         if (found.mode)
             return found;
     }
     if (!exact.find(key, &found)) {
-        found = pack_exact(act, s_src, s_flt, s_dst);
+        if (!pts.n)
+            pts = requant_steps(act, s_src, s_flt, s_dst);
+        found = search<pack_exact>(act, s_src, s_flt, s_dst, pts);
         exact.put(key, found);
     }
     return found;
