@@ -63,7 +63,7 @@ TinyNNStatus conv_dw_pw_launch(
 bool conv_stem_supported(const ConvGeom& c0, const ConvGeom& dw, const ConvGeom& pw, const void* image, const void* dst);
 TinyNNStatus conv_stem_launch(
         const ConvGeom& c0, const ConvGeom& dw, const ConvGeom& pw, const void* image, const void* flt0, const void* bias0, const void* dflt,
-        const void* dbias, const void* packed, const void* pbias, void* dst);
+        const void* dbias, const void* packed, const void* pbias, void* dst, bool launch);
 
 // A filter that went through megcc_gfx950_conv2d_init is a 1-d byte tensor.
 static bool is_packed_filter(const Tensor* flt) {
@@ -989,9 +989,7 @@ TinyNNStatus stem_run(const StemAttr& a, Tensor** inputs, int nr_input, Tensor**
     MG_REQUIRE(conv_stem_supported(c0, dw, pw, image->ptr, dst->ptr) && conv_mfma_supported(pw) &&
                        nr_elem(flt[2]->layout) == conv_mfma_packed_bytes(pw) && aligned16(flt[2]->ptr) && aligned4(flt[1]->ptr),
                TinyNN_ERROR_NO_IMPLEMENT, "%s: shape, activation or alignment the kernel does not take", who);
-    if (!launch)
-        return TinyNN_SUCCESS;
     auto ptr = [](const Tensor* t) { return t ? t->ptr : nullptr; };
-    return conv_stem_launch(c0, dw, pw, image->ptr, flt[0]->ptr, ptr(bias[0]), flt[1]->ptr, ptr(bias[1]), flt[2]->ptr, ptr(bias[2]), dst->ptr);
+    return conv_stem_launch(c0, dw, pw, image->ptr, flt[0]->ptr, ptr(bias[0]), flt[1]->ptr, ptr(bias[1]), flt[2]->ptr, ptr(bias[2]), dst->ptr, launch);
 }
 }  // namespace mg

@@ -104,7 +104,7 @@ struct DpLaunch {
     unsigned workgroups;
 };
 struct DwPwBlock {
-    DwPwParams* dev = nullptr;  // [2]: by the proven multiply-adds where there are any, by the literal sequence
+    DwPwParams* dev = nullptr;  // [2]: by the proven multiply-adds where there are any, by the reference's sequence (mode 3)
     DwPwParams host[2];
     DpLaunch launch;
 };
@@ -564,6 +564,7 @@ static bool dp_shape(int c, int oc, long groups, DpShape* s) {
     return true;
 }
 
+// (but for the scales: whether there are constants for them is asked when the arguments are written, not on every forward)
 bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dst) {
     DpShape s;
     return dw.fmt == MEGCC_FMT_NCHW44 && dw.groups == dw.ic && dw.ic == dw.oc && dw.fh == 3 && dw.fw == 3 && dw.ph == 1 &&
@@ -572,8 +573,6 @@ bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* sr
            pw.pw == 0 && pw.ic == dw.oc && (pw.oc & 31) == 0 && dp_shape(dw.ic, pw.oc, 0, &s) &&
            dw.act == MEGCC_NONLINE_RELU &&
            (pw.act == MEGCC_NONLINE_IDENTITY || pw.act == MEGCC_NONLINE_RELU) &&
-           requant_pack_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst, false).mode != 0 &&
-           requant_pack_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst, false).mode != 0 &&
            ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 3) == 0 && (long)dw.n * dw.ic * dw.ih * dw.iw < (1L << 31) &&
            (long)pw.n * pw.oc * pw.oh * pw.ow < (1L << 31) && (long)dw.ih * dw.iw < (1L << 24) && dw.oh > 0 && dw.ow > 0;
 }
@@ -637,6 +636,7 @@ static TinyNNStatus dp_plan(
     q.d_slices = make_fastdiv(q.slices);
     q.dq = requant_started_for(dw.act, dw.s_src, dw.s_flt, dw.s_dst, affine);
     q.pq = requant_started_for(pw.act, pw.s_src, pw.s_flt, pw.s_dst, affine);
+    MG_REQUIRE(q.dq.mode && q.pq.mode, TinyNN_ERROR_NO_IMPLEMENT, "conv_dw_pw: scales without proven constants");
     const int rag = dw.iw & 3;
     DwPwKernel kern = nullptr;
     size_t lds = 0;

@@ -164,7 +164,8 @@ struct PipeConfig {
     int pm = 0;          // plane-major activation patch (virtual rows padded to a multiple of 4)
     int rs = 0;          // a stage is ONE filter row of a 32-channel chunk (filters of more than 9 taps)
     int fcb = 0;         // FullyConnected with 16-byte activation loads (K a multiple of 128)
-    const void* kernel;
+    const void* kernel;   // the activation's requantisation by constants, ...
+    const void* literal;  // ... for scales that have none (which of the two is the launch's question)
 };
 
 }  // namespace mg

@@ -720,6 +720,8 @@ TinyNNStatus conv_mfma_launch(
         note_kernel(q.xo.w ? "conv_mfma_i8_dma_xo" : "conv_mfma_i8_dma", picked,
                     pc.bm, pc.bn, q.Lmax, pc.ks);
         note_requant_affine(q.rq.affine());
+        if (!q.rq.mode)
+            pc.kernel = pc.literal;
         return conv_mfma_pipe_launch(pc, q);
     }
     const int split = conv_mfma_split(g);

@@ -491,11 +491,11 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
 
 // ---- configurations --------------------------------------------------------------------------
 template <int FH, int FW, int KS, int LMAX, bool FC, int MT = 2, int DM_NBUF = 3, int WGM = 2, int BPC = 1, int NT = 2, bool FCB = false, bool PM = false>
-static PipeConfig make_dma_config(int act, bool proven);
+static PipeConfig make_dma_config(int act);
 
 // row-split configurations (filters of more than 9 taps): 64 * MT oc x 128 * NT px, FW taps per stage
 template <int FW, int LMAX, int MT, int DM_NBUF, int NT>
-static PipeConfig make_rs_config(int act, bool proven) {
+static PipeConfig make_rs_config(int act) {
     PipeConfig c;
     c.bm = 64 * MT;
     c.bn = 128 * NT;
@@ -507,18 +507,18 @@ static PipeConfig make_rs_config(int act, bool proven) {
     c.fixed_lmax = LMAX;
     c.rs = 1;
     c.extra_lds = 128 * 4;
-    c.kernel = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, ACT_RT, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
-    if (act == MEGCC_NONLINE_IDENTITY && proven)
+    c.kernel = c.literal = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, ACT_RT, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
+    if (act == MEGCC_NONLINE_IDENTITY)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, MEGCC_NONLINE_IDENTITY, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
-    else if (act == MEGCC_NONLINE_RELU && proven)
+    else if (act == MEGCC_NONLINE_RELU)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, MEGCC_NONLINE_RELU, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
-    else if (act == MEGCC_NONLINE_H_SWISH && proven)
+    else if (act == MEGCC_NONLINE_H_SWISH)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<1, FW, 1, LMAX, MEGCC_NONLINE_H_SWISH, false, MT, DM_NBUF, 2, 1, NT, false, false, true>;
     return c;
 }
 
 template <int FH, int FW, int KS, int LMAX, bool FC, int MT, int DM_NBUF, int WGM, int BPC, int NT, bool FCB, bool PM>
-static PipeConfig make_dma_config(int act, bool proven) {
+static PipeConfig make_dma_config(int act) {
     constexpr int DM_BM = 32 * MT * WGM;
     PipeConfig c;
     c.bm = DM_BM;
@@ -533,13 +533,13 @@ static PipeConfig make_dma_config(int act, bool proven) {
     c.extra_lds = (DM_BM > 128 ? DM_BM : 128) * 4 +
                   (FCB && MT == 4 ? 4 * WGM * 32 * 80 : 0);  // (32 rows x 80 bytes of staging per wave)
     c.fcb = FCB ? 1 : 0;
-    c.kernel = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, ACT_RT, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
-    if (act == MEGCC_NONLINE_IDENTITY && proven)
+    c.kernel = c.literal = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, ACT_RT, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
+    if (act == MEGCC_NONLINE_IDENTITY)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, MEGCC_NONLINE_IDENTITY, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
-    else if (act == MEGCC_NONLINE_RELU && proven)
+    else if (act == MEGCC_NONLINE_RELU)
         c.kernel = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, MEGCC_NONLINE_RELU, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
     if constexpr (!FC) {  // (FullyConnected with H_SWISH keeps the literal sequence)
-        if (act == MEGCC_NONLINE_H_SWISH && proven)
+        if (act == MEGCC_NONLINE_H_SWISH)
             c.kernel = (const void*)conv_mfma_i8_dma_kernel<FH, FW, KS, LMAX, MEGCC_NONLINE_H_SWISH, FC, MT, DM_NBUF, WGM, BPC, NT, FCB, PM>;
     }
     return c;
@@ -560,14 +560,13 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
         if (fc || g.fmt != MEGCC_FMT_NCHW44 || !(g.fw == 5 || g.fw == 7) || g.fh != g.fw || g.oc < 32 ||
             P < 2048 || (long)g.n * g.oc * g.oh * g.ow >= (1L << 31))
             return false;
-        const bool okt = requant_pack_for(g.act, g.s_src, g.s_flt, g.s_dst, false).mode != 0;
         const bool wide = g.oc >= 128;
         if (variant == 8)
-            *c = g.fw == 5 ? (wide ? make_rs_config<5, 512, 2, 3, 2>(g.act, okt) : make_rs_config<5, 512, 1, 3, 2>(g.act, okt))
-                           : (wide ? make_rs_config<7, 512, 2, 3, 2>(g.act, okt) : make_rs_config<7, 512, 1, 3, 2>(g.act, okt));
+            *c = g.fw == 5 ? (wide ? make_rs_config<5, 512, 2, 3, 2>(g.act) : make_rs_config<5, 512, 1, 3, 2>(g.act))
+                           : (wide ? make_rs_config<7, 512, 2, 3, 2>(g.act) : make_rs_config<7, 512, 1, 3, 2>(g.act));
         else
-            *c = g.fw == 5 ? (wide ? make_rs_config<5, 1024, 2, 2, 1>(g.act, okt) : make_rs_config<5, 1024, 1, 2, 1>(g.act, okt))
-                           : (wide ? make_rs_config<7, 1024, 2, 2, 1>(g.act, okt) : make_rs_config<7, 1024, 1, 2, 1>(g.act, okt));
+            *c = g.fw == 5 ? (wide ? make_rs_config<5, 1024, 2, 2, 1>(g.act) : make_rs_config<5, 1024, 1, 2, 1>(g.act))
+                           : (wide ? make_rs_config<7, 1024, 2, 2, 1>(g.act) : make_rs_config<7, 1024, 1, 2, 1>(g.act));
         return true;
     }
     if (g.fh * g.fw > MAX_TAPS_STAGE)
@@ -584,14 +583,13 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
             P * ((g.oc + 127) / 128) >= (P >= 4096 ? 32L : 64L) * num_cus() || g.oc < 32 || (g.ic & 31) ||
             (long)g.n * g.oc * g.oh * g.ow >= (1L << 31))
             return false;
-        const bool okt = requant_pack_for(g.act, g.s_src, g.s_flt, g.s_dst, false).mode != 0;
         if (variant == 6) {
             if (g.sw != 1 || (g.iw & 3) || !b128_ok ||
                 ((long)g.n * (g.ih + 2 * g.ph) + 2L * g.fh * g.dh) * (g.iw + g.pw + 3) >= (1L << 31))
                 return false;
-            *c = make_dma_config<3, 3, 1, 512, false, 1, 3, 1, 1, 1, false, true>(g.act, okt);
+            *c = make_dma_config<3, 3, 1, 512, false, 1, 3, 1, 1, 1, false, true>(g.act);
         } else {
-            *c = make_dma_config<3, 3, 1, 384, false, 1, 3, 1, 1, 1>(g.act, okt);
+            *c = make_dma_config<3, 3, 1, 384, false, 1, 3, 1, 1, 1>(g.act);
         }
         return true;
     }
@@ -601,7 +599,6 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
         return false;  // 64-channel tiles: 3x3 layers and the 1x1 with 32 input channels
     if ((long)g.n * g.oc * g.oh * g.ow >= (1L << 31))
         return false;  // 32-bit output offsets
-    const bool ok = requant_pack_for(g.act, g.s_src, g.s_flt, g.s_dst, false).mode != 0;
     // measured slower on the 256-channel 56x56 layer (91 us): two 256-thread workgroups per CU
     // with 64-channel tiles and two buffers (100 us), four waves of 128 oc x 64 pixels (107 us)
     if (variant == 2 || variant == 3) {
@@ -612,13 +609,13 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
         // 768 slots hold a 512-pixel sub-tile of rows up to ~60 slots inside one image; a sub-tile
         // that crosses into the next image also spans the padding rows between them
         if (g.oc < 128 && variant == 2)
-            *c = make_dma_config<3, 3, 1, 768, false, 1, 2, 2, 1, 4, false, true>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 768, false, 1, 2, 2, 1, 4, false, true>(g.act);
         else if (g.oc < 128)
-            *c = make_dma_config<3, 3, 1, 1024, false, 1, 2, 2, 1, 4, false, true>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 1024, false, 1, 2, 2, 1, 4, false, true>(g.act);
         else if (variant == 2)
-            *c = make_dma_config<3, 3, 1, 768, false, 2, 2, 2, 1, 4, false, true>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 768, false, 2, 2, 2, 1, 4, false, true>(g.act);
         else
-            *c = make_dma_config<3, 3, 1, 1024, false, 2, 2, 2, 1, 4, false, true>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 1024, false, 2, 2, 2, 1, 4, false, true>(g.act);
         return true;
     }
     if (variant == 4) {  // variant 1 (256-pixel sub-tiles, three buffers) with the plane-major patch
@@ -626,9 +623,9 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
             ((long)g.n * (g.ih + 2 * g.ph) + 2L * g.fh * g.dh) * (g.iw + g.pw + 3) >= (1L << 31))
             return false;
         if (g.oc < 128)
-            *c = make_dma_config<3, 3, 1, 512, false, 1, 3, 2, 1, 2, false, true>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 512, false, 1, 3, 2, 1, 2, false, true>(g.act);
         else
-            *c = make_dma_config<3, 3, 1, 512, false, 2, 3, 2, 1, 2, false, true>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 512, false, 2, 3, 2, 1, 2, false, true>(g.act);
         return true;
     }
     // 3x3 with stride 2 (down-sampling layers): the patch of a sub-tile holds four input pixels per
@@ -641,39 +638,39 @@ bool conv_mfma_dma_config(const ConvGeom& g, bool fc, int variant, bool b128_ok,
         if (g.oc < 128 || (variant == 0 && P < 32768))
             return false;
         if (variant == 0)
-            *c = make_dma_config<3, 3, 1, 1280, false, 2, 2>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 1280, false, 2, 2>(g.act);
         else
-            *c = make_dma_config<3, 3, 1, 768, false, 2, 2, 2, 1, 1>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 768, false, 2, 2, 2, 1, 1>(g.act);
         return true;
     }
     if (variant == 0) {
         if (!k3)
             return false;
         if (g.oc < 128)  // 64 oc x 512 px: each wave 32 oc x 128 px
-            *c = make_dma_config<3, 3, 1, 768, false, 1, 2, 2, 1, 4>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 768, false, 1, 2, 2, 1, 4>(g.act);
         else
-            *c = make_dma_config<3, 3, 1, 768, false, 2, 2, 2, 1, 4>(g.act, ok);
+            *c = make_dma_config<3, 3, 1, 768, false, 2, 2, 2, 1, 4>(g.act);
         return true;
     }
     if (k3 && g.oc < 128)
-        *c = make_dma_config<3, 3, 1, 512, false, 1>(g.act, ok);
+        *c = make_dma_config<3, 3, 1, 512, false, 1>(g.act);
     else if (k3)
-        *c = make_dma_config<3, 3, 1, 512, false>(g.act, ok);
+        *c = make_dma_config<3, 3, 1, 512, false>(g.act);
     else if (fc && (g.ic & 127) == 0 && b128_ok && g.oc >= 256)
         // 256 x 256 tile, each wave 128 oc x 64 rows (4 x 2 MFMA tiles: 0.75 KB of LDS per MFMA;
         // measured 86 us on 4096^3 against 105 us with the 128 x 256 tile)
-        *c = make_dma_config<1, 1, 4, 256, true, 4, 2, 2, 1, 2, true>(g.act, ok);
+        *c = make_dma_config<1, 1, 4, 256, true, 4, 2, 2, 1, 2, true>(g.act);
     else if (fc && (g.ic & 127) == 0 && b128_ok)
-        *c = make_dma_config<1, 1, 4, 256, true, 2, 3, 2, 1, 2, true>(g.act, ok);
+        *c = make_dma_config<1, 1, 4, 256, true, 2, 3, 2, 1, 2, true>(g.act);
     else if (fc)
-        *c = make_dma_config<1, 1, 4, 256, true>(g.act, ok);
+        *c = make_dma_config<1, 1, 4, 256, true>(g.act);
     else if (g.oc < 128)
-        *c = make_dma_config<1, 1, 1, 256, false, 1, 8>(g.act, ok);
+        *c = make_dma_config<1, 1, 1, 256, false, 1, 8>(g.act);
     else if (g.ic <= 128)
-        *c = make_dma_config<1, 1, 2, 256, false, 2, 6>(g.act, ok);
+        *c = make_dma_config<1, 1, 2, 256, false, 2, 6>(g.act);
 
     else
-        *c = make_dma_config<1, 1, 4, 256, false>(g.act, ok);
+        *c = make_dma_config<1, 1, 4, 256, false>(g.act);
     return true;
 }
 

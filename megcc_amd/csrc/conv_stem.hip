@@ -332,9 +332,8 @@ __global__ void __launch_bounds__(ST_THREADS, 4) conv_stem_kernel(StemParams q) 
     }
 }
 
-// c0: the first convolution (its s_src the quantised image's scale), dw, pw
+// c0: the first convolution (its s_src the quantised image's scale), dw, pw. (The scales are conv_stem_launch's question.)
 bool conv_stem_supported(const ConvGeom& c0, const ConvGeom& dw, const ConvGeom& pw, const void* image, const void* dst) {
-    auto proven = [](const ConvGeom& g) { return requant_pack_for(g.act, g.s_src, g.s_flt, g.s_dst, false).mode != 0; };
     return c0.fmt == MEGCC_FMT_NCHW_NCHW44 && c0.groups == 1 && c0.ic == 3 && c0.oc == ST_C && c0.fh == 3 && c0.fw == 3 && c0.sh == 2 &&
            c0.sw == 2 && c0.ph == 1 && c0.pw == 1 && c0.dh == 1 && c0.dw == 1 && c0.act == MEGCC_NONLINE_RELU && c0.ih == 2 * c0.oh &&
            c0.iw == 2 * c0.ow && (c0.ow & 3) == 0 && c0.ow >= 4 && c0.ow <= ST_MAXW && c0.oh >= 1 &&
@@ -343,7 +342,7 @@ bool conv_stem_supported(const ConvGeom& c0, const ConvGeom& dw, const ConvGeom&
            dw.ih == c0.oh && dw.iw == c0.ow &&
            pw.fmt == MEGCC_FMT_NCHW44 && pw.groups == 1 && pw.ic == ST_C && (pw.oc == 32 || pw.oc == 64) && pw.fh == 1 && pw.fw == 1 &&
            pw.sh == 1 && pw.sw == 1 && pw.ph == 0 && pw.pw == 0 && (pw.act == MEGCC_NONLINE_IDENTITY || pw.act == MEGCC_NONLINE_RELU) &&
-           pw.n == c0.n && pw.ih == c0.oh && pw.iw == c0.ow && proven(c0) && proven(dw) && proven(pw) &&
+           pw.n == c0.n && pw.ih == c0.oh && pw.iw == c0.ow &&
            ((uintptr_t)image & 3) == 0 && ((uintptr_t)dst & 3) == 0 && (long)c0.n * 3 * c0.ih * c0.iw * 4 < (1L << 31) - (1 << 20) &&
            (long)pw.n * pw.oc * pw.oh * pw.ow < (1L << 31);
 }
@@ -364,9 +363,17 @@ static int stem_strips(long n, int steps) {
     return best;
 }
 
+// `launch` false: only whether the scales have constants
 TinyNNStatus conv_stem_launch(
         const ConvGeom& c0, const ConvGeom& dw, const ConvGeom& pw, const void* image, const void* flt0, const void* bias0, const void* dflt,
-        const void* dbias, const void* packed, const void* pbias, void* dst) {
+        const void* dbias, const void* packed, const void* pbias, void* dst, bool launch) {
+    const ConvGeom* const layers[] = {&c0, &dw, &pw};
+    if (!launch) {  // (there are constants whatever the switch says)
+        for (const ConvGeom* g : layers)
+            MG_REQUIRE(requant_pack_for(g->act, g->s_src, g->s_flt, g->s_dst, false).mode, TinyNN_ERROR_NO_IMPLEMENT,
+                       "conv_stem: scales without proven constants");
+        return TinyNN_SUCCESS;
+    }
     if (c0.n == 0)
         return TinyNN_SUCCESS;
     StemParams q = {};
@@ -387,7 +394,6 @@ TinyNNStatus conv_stem_launch(
     q.scale = 1.f / c0.s_src;  // (as the conversion on its own has it)
     q.d_strips = make_fastdiv(q.strips);
     q.d_quads = make_fastdiv(c0.iw / 4);
-    const ConvGeom* const layers[] = {&c0, &dw, &pw};
     RequantPack* const packs[] = {&q.r0, &q.dq, &q.pq};
     bool fma = !options().no_affine, affine = true;
     for (int l = 0; l < 3; ++l) {
@@ -402,6 +408,7 @@ TinyNNStatus conv_stem_launch(
             *packs[l] = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
         affine = affine && packs[l]->affine();
     }
+    MG_REQUIRE(q.r0.mode && q.dq.mode && q.pq.mode, TinyNN_ERROR_NO_IMPLEMENT, "conv_stem: scales without proven constants");
 #define MG_STEM(MT_, ACT_) (fma ? conv_stem_kernel<MT_, ACT_, true> : conv_stem_kernel<MT_, ACT_, false>)
     void (*const kern)(StemParams) = pw.oc == 64 ? (pw.act == MEGCC_NONLINE_RELU ? MG_STEM(2, MEGCC_NONLINE_RELU) : MG_STEM(2, MEGCC_NONLINE_IDENTITY))
                                                  : (pw.act == MEGCC_NONLINE_RELU ? MG_STEM(1, MEGCC_NONLINE_RELU) : MG_STEM(1, MEGCC_NONLINE_IDENTITY));
