@@ -133,6 +133,11 @@ struct RequantSteps {
         y[n++] = out;
     }
 };
+// (from the third point on) the first accumulator with its output, which bounds d from below - the last one with an output
+// bounds it from above, and for no slope that is positive does the other bound of either count
+static inline bool above_step(int i) {
+    return i & 1;
+}
 static RequantSteps requant_steps(int act, float s_src, float s_flt, float s_dst) {
     const std::shared_ptr<const RequantTable> table = requant_table_for(act, s_src, s_flt, s_dst);
     const RequantTable& T = *table;
@@ -161,13 +166,14 @@ static RequantSteps requant_steps(int act, float s_src, float s_flt, float s_dst
 
 // A search for constants, F, for processors with a fused multiply-add, where fmaf, rintf and floorf are an instruction each, and for
 // the others, where they are calls of the library. All are exact: the results are the same.
-// (us on one core, scales of calibrated layers with 64 / 1152 / 4096 products to a sum, with this, one pass over the steps for all searches and
-// IDENTITY's two floors sharing their hulls: IDENTITY 26 / 25 / 26 -> 13 / 15 / 16, RELU 6.0 / 14.0 / 16.4 -> 4.9 / 11.9 / 14.4.)
+// (us on one core for a launch's constants, table and all, scales of calibrated layers with 64 / 1152 / 4096 products to a sum: IDENTITY 9.5 /
+// 12.8 / 13.8, RELU 4.9 / 12.2 / 13.8, H_SWISH 3.1 / 3.5 / 3.7; with both sides of a step in both hulls and the points one by one 11.2 / 16.1 /
+// 16.7, 5.8 / 14.6 / 15.9 and 4.0 / 4.1 / 4.5.)
 #define MG_INLINE __attribute__((always_inline))
 #if defined(__HIP_DEVICE_COMPILE__)
 #define MG_FMA
 #else
-#define MG_FMA __attribute__((target("fma")))
+#define MG_FMA __attribute__((target("avx2,fma")))
 #endif
 template <auto F>
 MG_FMA static auto search_fma(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
@@ -176,7 +182,7 @@ MG_FMA static auto search_fma(int act, float s_src, float s_flt, float s_dst, co
 template <auto F>
 static auto search(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
 #if !defined(__HIP_DEVICE_COMPILE__)
-    static const bool fma = __builtin_cpu_supports("fma");
+    static const bool fma = __builtin_cpu_supports("fma") && __builtin_cpu_supports("avx2");
     if (fma)
         return search_fma<F>(act, s_src, s_flt, s_dst, pts);
 #endif
@@ -237,10 +243,10 @@ MG_INLINE static bool requant_verified(const RequantSteps& pts, const RequantBou
     for (int i = 0; i < to.n; ++i)
         if (eval(pts.a[to.point[i]]) != pts.y[to.point[i]])
             return false;
+    int wrong = 0;  // (no way out of this loop: eight points at a time)
     for (int i = 0; i < pts.n; ++i)
-        if (eval(pts.a[i]) != pts.y[i])
-            return false;
-    return true;
+        wrong |= eval(pts.a[i]) ^ pts.y[i];
+    return !wrong;
 }
 
 // host evaluation of requant_conv_affine (fmaf is the correctly rounded single fused multiply-add,
@@ -281,9 +287,9 @@ MG_INLINE static RequantAffine affine_constants(int act, float s_src, float s_fl
     RequantBounds<true> from;  // floor(a c + d) == y  <=>  y <= a c + d < y + 1
     RequantBounds<false> to;
     for (int i = 2; i < pts.n; ++i) {  // (the ends of the range bound nothing)
-        if (pts.y[i] > lo)
+        if (above_step(i))
             from.add((double)(float)pts.a[i], (double)pts.y[i], i);
-        if (pts.y[i] < 127)
+        else
             to.add((double)(float)pts.a[i], (double)pts.y[i] + 1, i);
     }
     return affine_within(pts, from, to, 0., lo, make_requant_fast(s_src, s_flt, s_dst).c);
@@ -321,8 +327,10 @@ MG_INLINE static int pack_eval(int a, int act, const RequantPack& q) {
     }
     if (q.mode == 3) {
         float v = fmaf(x, q.c, x * q.d);
-        if (act == MEGCC_NONLINE_IDENTITY)
-            return fp32_to_int8(v);  // (half away from zero: what the device's form is for every float)
+        if (act == MEGCC_NONLINE_IDENTITY) {
+            const float t = truncf(v + copysignf(0x1.fffffep-2f, v));
+            return (int)(t < -128.f ? -128.f : t > 127.f ? 127.f : t);
+        }
         if (act == MEGCC_NONLINE_H_SWISH) {
             const float t = v + 3;
             v = v * std::min(std::max(t, 0.f), 6.f) * (2.f * (1.f / 6.f));
@@ -343,9 +351,9 @@ MG_INLINE static RequantPack pack_symmetric(const RequantSteps& pts, float s_src
     RequantBounds<false> to;
     auto value = [&](int a) MG_INLINE { return std::fabs((double)((float)a * s_src * s_flt)); };
     for (int i = 2; i < pts.n; ++i) {
-        if (pts.y[i] > 0)
+        if (above_step(i) && pts.y[i] > 0)
             from.add(value(pts.a[i]), (double)pts.y[i], i);
-        if (pts.y[i] >= 0 && pts.a[i] >= 0 && pts.y[i] < 127)
+        if (!above_step(i) && pts.y[i] >= 0 && pts.a[i] >= 0)
             to.add(value(pts.a[i]), (double)pts.y[i] + 1, i);
     }
     for (int i = 2; i < pts.n; ++i) {
@@ -392,9 +400,9 @@ MG_INLINE static RequantPack pack_affine(int act, float s_src, float s_flt, floa
         for (int i = 2; i < pts.n; ++i) {
             const double x = f.mode == 2 ? (float)pts.a[i] * f.s1 * f.s2 : (float)pts.a[i];
             const int y = pts.y[i];
-            if (y > lowest)
+            if (above_step(i))
                 from.add(x, relu ? 2.0 * y - 0.5 : y + 127.5, i);
-            if (y < 127)
+            else
                 to.add(x, relu ? 2.0 * y + 1.5 : y + 128.5, i);
         }
         for (int k = 0; k <= 48 && !found.mode; ++k) {
@@ -440,6 +448,12 @@ MG_INLINE static RequantPack pack_exact(int act, float s_src, float s_flt, float
     RequantPack q = {s_src, s_flt, (float)inv, 0.f, 3};
     q.d = (float)(inv - (double)q.c);
     const long long near = (long long)(1e-4f / c);
+    if (near == 0) {  // (no other accumulator is that near to a step: the points alone, eight at a time)
+        int wrong = 0;
+        for (int i = 0; i < pts.n; ++i)
+            wrong |= pack_eval(pts.a[i], act, q) ^ pts.y[i];
+        return wrong ? none : q;
+    }
     // (pts: the ends of the range, then each step's last accumulator below and first one above)
     for (int i = 0; i < pts.n; ++i) {
         const bool above = i >= 2 && pts.y[i] > pts.y[i - 1] && pts.a[i] == pts.a[i - 1] + 1;
@@ -464,9 +478,9 @@ MG_INLINE static RequantPack pack_shifted(int act, float s_src, float s_flt, flo
         if (std::abs((long long)pts.a[i]) >= (1 << 22) - 1024)
             return none;
         const double x = pts.a[i];
-        if (pts.y[i] > lowest)
+        if (above_step(i))
             from.add(x, relu ? 2.0 * pts.y[i] - 0.5 : pts.y[i] + 127.5, i);
-        if (pts.y[i] < 127)
+        else
             to.add(x, relu ? 2.0 * pts.y[i] + 1.5 : pts.y[i] + 128.5, i);
     }
     // (the outputs at the ends of the range are then those beyond the first and the last step; the ends themselves have no float)
