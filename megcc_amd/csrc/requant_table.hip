@@ -437,12 +437,12 @@ MG_INLINE static RequantPack pack_affine(int act, float s_src, float s_flt, floa
 // Mode 3, or mode 0 where it is not proven. The quotient it works with is at most one float from the reference's, so
 // outputs can only differ where the reference's own value is within two of its floats of a step, 2 * 2^-17 for outputs up
 // to 128: accumulators on both sides of each step are compared, and as many beyond them as lie within 1e-4 of it (with
-// H_SWISH the output changes by half to one and a half of what the quotient does).
+// H_SWISH the output changes by half to one and a half of what the quotient does): 215 a step at the smallest ratios.
 MG_INLINE static RequantPack pack_exact(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
     const RequantPack none = {s_src, s_flt, s_dst, 0.f, 0};
     auto mid = [](float s) { return s >= 1e-12f && s <= 1e12f; };  // (nothing overflows or loses bits on the way)
     const float c = make_requant_fast(s_src, s_flt, s_dst).c;
-    if (!mid(s_src) || !mid(s_flt) || !mid(s_dst) || !(c >= 1.6e-6f && c <= 1e12f))
+    if (!mid(s_src) || !mid(s_flt) || !mid(s_dst) || !(c <= 1e12f))
         return none;
     const double inv = (act == MEGCC_NONLINE_RELU ? 2.0 : 1.0) / (double)s_dst;
     RequantPack q = {s_src, s_flt, (float)inv, 0.f, 3};

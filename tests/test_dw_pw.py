@@ -10,7 +10,7 @@ from oracle import port
 
 pytestmark = pytest.mark.gpu
 
-TIES = (0.02, 0.01, 0.05)            # exact ties: both layers requantise by table
+TIES = (0.02, 0.01, 0.05)            # exact ties: both layers requantise by the reference's own sequence
 GENERIC = (0.0213, 0.0097, 0.0371)
 
 PAIRS = [
@@ -178,4 +178,37 @@ def test_the_requantisation_is_switched_between_forwards(graph):
     finally:
         runtime.set_option("noaffine", 0)
         runtime.set_option("no_graph", 0)
+    m.close()
+
+
+def test_a_pair_with_ratios_near_a_millionth():
+    """scales for which there are no multiply-adds but the reference's sequence is proven: the pair is one kernel like any other"""
+    n, c, scales = 2, 64, (0.001, 0.001, 0.9)
+    dw = ConvCase(A.FMT_NCHW44, A.GROUP, n, c, 9, 12, c, 3, 1, 1, A.RELU, scales=scales)
+    pw = ConvCase(A.FMT_NCHW44, A.DENSE, n, c, 9, 12, c, 1, 1, 0, A.IDENTITY, scales=(0.9, 0.001, 0.9 * 0.001 / 9.0e-7))
+    a0, a1 = dw.gen(5), pw.gen(6)
+    for case, arrays, lowest in ((dw, a0, 0), (pw, a1, -128)):
+        ratio = case.scales[0] * case.scales[1] / case.scales[2]
+        arrays["bias"].reshape(-1)[...] = np.linspace((lowest - 2) / ratio, 129 / ratio, c).astype(np.int32)
+    a1["src"] = dw.run_port(a0)
+    want = pw.run_port(a1)
+    bias_scale = lambda k: float(np.float32(k.scales[0]) * np.float32(k.scales[1]))
+    m = runtime.Model()
+    t = x = m.tensor("x", dw.src_shape(), abi.QINT8, dw.scales[0])
+    m.mark_input(x)
+    for k, case, arrays in (("dw", dw, a0), ("pw", pw, a1)):
+        y = m.tensor(k, case.dst_shape(), abi.QINT8, case.scales[2])
+        m.opr(case.symbol(), [t, m.weight(k + ".w", arrays["flt"], abi.QINT8, case.scales[1]),
+                              m.weight(k + ".b", arrays["bias"], abi.QINT32, bias_scale(case))], [y])
+        t = y
+    m.mark_output(t)
+    runtime.set_option("fusedwpw", 1)
+    try:
+        m.finalize()
+    finally:
+        runtime.set_option("fusedwpw", 0)
+    assert m.nr_kernel == 1
+    m.set_input(x, a0["src"])
+    m.forward()
+    assert np.array_equal(m.get(t), want)
     m.close()

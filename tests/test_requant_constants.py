@@ -2,7 +2,7 @@
 the library's own search, its results evaluated with the device's instructions written out in plain C++ (a fused multiply-add is fmaf, the
 conversion to an unsigned byte rounds to even and saturates), on both sides of every step of the output, around them, at the ends of the
 accumulators' range and on random ones. Mode 5, the sums that start as floats, among them: within 2^22 its sums are whole floats, beyond
-it only their order counts."""
+it only their order counts. Every scale for which there is a threshold table has at least one form."""
 import os
 import subprocess
 
@@ -139,3 +139,7 @@ def test_every_form_gives_the_reference_s_outputs(result):
     assert result.returncode == 0, result.stdout[-500:] + result.stderr[-500:]
     counts = [int(n) for n in result.stdout.split("modes")[1].split()]
     assert all(n >= 40 for n in counts), result.stdout[-200:]  # (each form met)
+
+
+def test_every_scale_with_a_table_has_a_form(result):
+    assert " ".join(result.stdout.splitlines()[-1].split()[:2]) == "none 0", result.stdout[:500]
