@@ -1,5 +1,7 @@
 """A channel-wise 3x3 convolution and the pointwise 1x1 convolution of its result as one kernel (the model
 runtime's conv_dw_pw), against the oracle's two convolutions run one after the other, bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -178,6 +180,87 @@ def test_the_requantisation_is_switched_between_forwards(graph):
     finally:
         runtime.set_option("noaffine", 0)
         runtime.set_option("no_graph", 0)
+    m.close()
+
+
+class _Pack(C.Structure):
+    _fields_ = [("s1", C.c_float), ("s2", C.c_float), ("c", C.c_float), ("d", C.c_float), ("mode", C.c_int)]
+
+
+def starts_as_floats(act, scales):
+    """whether sums of that layer start as floats (epilogue.h, mode 5): the library's own answer"""
+    f = runtime.lib()._ZN2mg19requant_shifted_forEifff
+    f.argtypes, f.restype = [C.c_int] + [C.c_float] * 3, _Pack
+    return f(act, *scales).mode == 5
+
+
+def swept_biases(channels, values, ratio, lowest):
+    """`values` consecutive sums a channel, from 24 outputs below `lowest` to 24 above 127; the channels at the ends, which
+    saturate, far beyond 2^22 and 2^29"""
+    bias = int(np.floor((lowest - 24) / ratio)) + values * np.arange(channels, dtype=np.int64)
+    bias[[0, -1, -2]] = [-(2 ** 30), 2 ** 30, 2 ** 22 + 3]
+    return bias.astype(np.int32)
+
+
+PASS = (0.5, 1.0, 0.5)  # scales of a layer whose outputs are its sums
+
+
+@pytest.mark.parametrize("noaffine", [0, 1])
+@pytest.mark.parametrize("swept,act", [("dw", A.RELU), ("pw", A.RELU), ("pw", A.IDENTITY)])
+@pytest.mark.parametrize("c", [32, 64, 128, 512])
+def test_every_sum_between_the_lowest_and_the_highest_output(c, swept, act, noaffine):
+    """one layer passes its source on, the other's sums are all whole numbers over the whole range of its outputs: both sides of every
+    step, for sums that start as floats and (noaffine) for those that do not"""
+    values = 256 if swept == "dw" else 128
+    lowest = -128 if act == A.IDENTITY and swept == "pw" else 0
+    ratio = (127 - lowest + 48) / (c * values)
+    scales = (0.0131, 0.0097, 0.0131 * 0.0097 / ratio)
+    if swept == "pw":
+        scales = (PASS[2], 0.0097, PASS[2] * 0.0097 / ratio)
+    dw = ConvCase(A.FMT_NCHW44, A.GROUP, 1, c, 16, values // 16, c, 3, 1, 1, A.RELU, scales=scales if swept == "dw" else PASS)
+    s2 = scales if swept == "pw" else (scales[2], 1.0, scales[2])
+    pw = ConvCase(A.FMT_NCHW44, A.DENSE, 1, c, 16, values // 16, c, 1, 1, 0, act, scales=s2)
+    assert starts_as_floats(act if swept == "pw" else A.RELU, scales)
+    a0, a1 = dw.gen(1), pw.gen(2)
+    x = np.arange(values) - (128 if swept == "dw" else 0)
+    a0["src"] = np.broadcast_to(x.astype(np.int8).reshape(1, 1, 16, values // 16, 1), a0["src"].shape).copy()
+    a0["flt"][...] = 0
+    a0["flt"].reshape(c // 4, 9, 4)[:, 4] = 1
+    a1["flt"][...] = 0
+    w = a1["flt"].reshape(c // 4, c // 4, 4, 4)  # [output group][input group][input][output]
+    for k in range(4):
+        w[np.arange(c // 4), np.arange(c // 4), k, k] = 1
+    for arrays, mine in ((a0, swept == "dw"), (a1, swept == "pw")):
+        arrays["bias"].reshape(-1)[...] = swept_biases(c, values, ratio, lowest) if mine else 0
+    a1["src"] = dw.run_port(a0)
+    want = pw.run_port(a1)
+    assert set(np.unique(want)) == set(range(lowest, 128))
+    bias_scale = lambda k: float(np.float32(k.scales[0]) * np.float32(k.scales[1]))
+    m = runtime.Model()
+    t = x = m.tensor("x", dw.src_shape(), abi.QINT8, dw.scales[0])
+    m.mark_input(x)
+    for k, case, arrays in (("dw", dw, a0), ("pw", pw, a1)):
+        y = m.tensor(k, case.dst_shape(), abi.QINT8, case.scales[2])
+        m.opr(case.symbol(), [t, m.weight(k + ".w", arrays["flt"], abi.QINT8, case.scales[1]),
+                              m.weight(k + ".b", arrays["bias"], abi.QINT32, bias_scale(case))], [y])
+        t = y
+    m.mark_output(t)
+    runtime.set_option("fusedwpw", 1)
+    try:
+        m.finalize()
+    finally:
+        runtime.set_option("fusedwpw", 0)
+    assert m.nr_kernel == 1
+    m.set_input(x, a0["src"])
+    runtime.set_option("noaffine", noaffine)
+    try:
+        m.forward()
+    finally:
+        runtime.set_option("noaffine", 0)
+    got = m.get(t)
+    assert runtime.last_kernel().startswith("conv_dw_pw")
+    bad = np.argwhere(got != want)
+    assert bad.size == 0, "%d differ, first at %s: %d, expected %d" % (len(bad), bad[0], got[tuple(bad[0])], want[tuple(bad[0])])
     m.close()
 
 

@@ -9,6 +9,7 @@ import pytest
 
 from cases import ConvCase
 from megcc_amd import abi, runtime
+from test_dw_pw import starts_as_floats, swept_biases
 
 CALIBRATED, TIES = (1.0 / 127, 0.0051, 0.037, 0.0047, 0.021, 0.0049, 0.043), (1.0 / 127, 0.01, 0.02, 0.01, 0.02, 0.01, 0.05)
 
@@ -74,6 +75,73 @@ def test_head_of_a_network_as_one_kernel(n, oh, ow, oc, act, bias, s):
     for k in range(m.nr_opr):  # operators one by one find their tensors
         m.run_opr(k)
     assert np.array_equal(m.get(ids[-1]), x)
+    m.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("noaffine", [0, 1])
+@pytest.mark.parametrize("swept,act", [("first", abi.RELU), ("dw", abi.RELU), ("pw", abi.RELU), ("pw", abi.IDENTITY)])
+def test_every_sum_between_the_lowest_and_the_highest_output(swept, act, noaffine):
+    """two of the three layers pass their source on, the third one's sums are all whole numbers over the whole range of its outputs, for
+    sums that start as floats (epilogue.h, mode 5) and, noaffine, for those that do not"""
+    oc = 64
+    channels, values = (oc, 128) if swept == "pw" else (32, 256 if swept == "first" else 128)
+    lowest = -128 if act == abi.IDENTITY else 0
+    ratio = (127 - lowest + 48) / (channels * values)
+    unit = 0.5
+    s = [unit, 1.0, unit, 1.0, unit, 1.0, unit]  # (source, filter, result = next source, ...) of layers whose outputs are their sums
+    layer = ["first", "dw", "pw"].index(swept)
+    s[2 * layer + 1] = 0.0097
+    out = float(np.float32(unit) * np.float32(0.0097)) / ratio
+    s[2 * layer + 2:] = [out if k % 2 == 0 else 1.0 for k in range(2 * layer + 2, 7)]
+    layers = _layers(1, 16, 16, oc, act, True, s)
+    assert starts_as_floats(layers[layer].act, layers[layer].scales)
+    q = np.zeros((1, 3, 32, 32), np.int8)
+    x = np.arange(256) - 128 if swept == "first" else np.arange(256) % 128
+    q[:, :, ::2, ::2] = x.reshape(16, 16).astype(np.int8)  # (the pixels under the filters' centres)
+    image = q.astype(np.float32) * np.float32(unit)
+    m = runtime.Model()
+    ids = [m.tensor("image", image.shape, abi.FLOAT), m.tensor("q", image.shape, abi.QINT8, unit)]
+    m.mark_input(ids[0])
+    m.opr("GI_kernel_typecvt_f32qsi8", [ids[0]], [ids[1]])
+    want = q
+    for k, case in enumerate(layers):
+        arrays = case.gen(seed=k)
+        arrays["src"] = want
+        f = arrays["flt"]
+        f[...] = 0
+        if k == 0:
+            f[:, 1, 1, 0, :] = 1
+        elif k == 1:
+            f.reshape(8, 9, 4)[:, 4] = 1
+        else:
+            for o in range(oc // 4):
+                for i in range(4):
+                    f[o, o % 8, 0, 0, i, i] = 1
+        arrays["bias"].reshape(-1)[...] = swept_biases(channels, values, ratio, lowest) if k == layer else 0
+        want = case.run_port(arrays)
+        weights = [m.weight("w%d" % k, f, abi.QINT8, case.scales[1]),
+                   m.weight("b%d" % k, arrays["bias"], abi.QINT32, float(np.float32(case.scales[0]) * np.float32(case.scales[1])))]
+        ids.append(m.tensor("y%d" % k, case.dst_shape(), abi.QINT8, case.scales[2]))
+        m.opr(case.symbol(), [ids[-2]] + weights, [ids[-1]])
+    assert set(np.unique(want)) == set(range(lowest, 128))
+    m.mark_output(ids[-1])
+    runtime.set_option("fusestem", 1)
+    try:
+        m.finalize()
+    finally:
+        runtime.set_option("fusestem", 0)
+    assert m.nr_kernel == 1
+    m.set_input(ids[0], image)
+    runtime.set_option("noaffine", noaffine)
+    try:
+        m.forward()
+    finally:
+        runtime.set_option("noaffine", 0)
+    got = m.get(ids[-1])
+    assert runtime.last_kernel().startswith("conv_stem"), runtime.last_kernel()
+    bad = np.argwhere(got != want)
+    assert bad.size == 0, "%d differ, first at %s: %d, expected %d" % (len(bad), bad[0], got[tuple(bad[0])], want[tuple(bad[0])])
     m.close()
 
 
