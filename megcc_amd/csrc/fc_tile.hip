@@ -401,11 +401,7 @@ TinyNNStatus fc_tile_launch(const ConvGeom& g, const void* src, const void* pack
 #undef MG_FCA
     const dim3 grid((g.oc + part - 1) / part, (g.n + part - 1) / part);
     q.xo = options().no_xcdorder ? XcdOrder{0} : make_xcd_order((int)grid.x, (int)grid.y, (long)(q.M + q.OC) * q.K);
-    // noted: the largest square that fills the chip (else 64) and how many ways the work on a square could be shared before the
-    // chip is full or its blocks of K run out; the part and the groups of waves that share K in it
-    const int square = big >= num_cus() ? 128 : 64;
-    const int share = square == 128 || squares >= 2L * num_cus() || q.nblk < 2 ? 1 : squares >= num_cus() || q.nblk < 4 ? 2 : 4;
-    note_kernel(q.xo.w ? "fc_tile_xo" : "fc_tile", square, share, part, groups);
+    note_kernel(q.xo.w ? "fc_tile_xo" : "fc_tile", part, groups);  // (the part's side, the groups of waves that share K in it)
     note_requant_affine(q.rq.affine());
     hipLaunchKernelGGL(kern, grid, dim3(part == 32 ? 256 : 256 * groups), 0, stream(), q);
     return check_launch("fc_tile");
