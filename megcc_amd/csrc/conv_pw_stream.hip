@@ -372,12 +372,13 @@ TinyNNStatus conv_pw_stream_launch(
     q.rq = requant_pack_pick(g.act, g.s_src, g.s_flt, g.s_dst);
     const int act = q.rq.mode ? g.act : -1;
 
-    const void* kern = nullptr;
+    typedef void (*Kernel)(PwParams);
+    Kernel kern = nullptr;
 #define MG_PW_PICK_ST(KC_, MT_, RG_, ST_)                                                                      \
-    (act == MEGCC_NONLINE_IDENTITY ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_IDENTITY, RG_, ST_> \
-     : act == MEGCC_NONLINE_RELU   ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_RELU, RG_, ST_>     \
-     : act == MEGCC_NONLINE_H_SWISH ? (const void*)conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_H_SWISH, RG_, ST_> \
-                                   : (const void*)conv_pw_stream_kernel<KC_, MT_, -1, RG_, ST_>)
+    (act == MEGCC_NONLINE_IDENTITY ? conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_IDENTITY, RG_, ST_> \
+     : act == MEGCC_NONLINE_RELU   ? conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_RELU, RG_, ST_>     \
+     : act == MEGCC_NONLINE_H_SWISH ? conv_pw_stream_kernel<KC_, MT_, MEGCC_NONLINE_H_SWISH, RG_, ST_> \
+                                   : conv_pw_stream_kernel<KC_, MT_, -1, RG_, ST_>)
 #define MG_PW_PICK_RG(KC_, MT_, RG_) (strided ? MG_PW_PICK_ST(KC_, MT_, RG_, true) : MG_PW_PICK_ST(KC_, MT_, RG_, false))
 #define MG_PW_PICK(KC_, MT_) (ragged ? MG_PW_PICK_RG(KC_, MT_, true) : MG_PW_PICK_RG(KC_, MT_, false))
     switch (kc) {
@@ -395,27 +396,25 @@ TinyNNStatus conv_pw_stream_launch(
     // 512 input channels and more tiles than resident waves: the workgroup-shared form
     if ((g.ic == 512 || g.ic == 1024) && !ragged && (q.groups & 3) == 0 && !options().no_pwshare) {
 #define MG_PWS_PICK_ST(KC_, ST_)                                                                          \
-    (act == MEGCC_NONLINE_IDENTITY ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_IDENTITY, ST_>    \
-     : act == MEGCC_NONLINE_RELU   ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_RELU, ST_>        \
-     : act == MEGCC_NONLINE_H_SWISH ? (const void*)conv_pw_share_kernel<KC_, MEGCC_NONLINE_H_SWISH, ST_>    \
-                                   : (const void*)conv_pw_share_kernel<KC_, -1, ST_>)
+    (act == MEGCC_NONLINE_IDENTITY ? conv_pw_share_kernel<KC_, MEGCC_NONLINE_IDENTITY, ST_>    \
+     : act == MEGCC_NONLINE_RELU   ? conv_pw_share_kernel<KC_, MEGCC_NONLINE_RELU, ST_>        \
+     : act == MEGCC_NONLINE_H_SWISH ? conv_pw_share_kernel<KC_, MEGCC_NONLINE_H_SWISH, ST_>    \
+                                   : conv_pw_share_kernel<KC_, -1, ST_>)
 #define MG_PWS_PICK(KC_) (strided ? MG_PWS_PICK_ST(KC_, true) : MG_PWS_PICK_ST(KC_, false))
-        const void* sk = g.ic == 512 ? MG_PWS_PICK(16) : MG_PWS_PICK(32);
+        const Kernel sk = g.ic == 512 ? MG_PWS_PICK(16) : MG_PWS_PICK(32);
 #undef MG_PWS_PICK
 #undef MG_PWS_PICK_ST
         const long gblocks = q.groups / 4;
-        const long capb = (long)num_cus() * pw_resident_blocks(sk);
+        const long capb = (long)num_cus() * pw_resident_blocks((const void*)sk);
         if ((long)q.tiles * gblocks >= capb / 2) {
             long runs = capb / gblocks;
             if (runs > q.tiles)
                 runs = q.tiles;
             if (runs < 1)
                 runs = 1;
-            void* sargs[] = {&q};
             note_kernel("conv_pw_share", g.ic / 32);
             note_requant_affine(q.rq.affine());
-            hipError_t e = hipLaunchKernel(sk, dim3((unsigned)(runs * gblocks)), dim3(PW_THREADS), sargs, 0, stream());
-            MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_pw_share: %s", hipGetErrorString(e));
+            hipLaunchKernelGGL(sk, dim3((unsigned)(runs * gblocks)), dim3(PW_THREADS), 0, stream(), q);
             return check_launch("conv_pw_share");
         }
     }
@@ -426,7 +425,7 @@ TinyNNStatus conv_pw_stream_launch(
     // (256 input channels: two workgroups a CU of the three that fit - each wave fetches 16 KB of filter rows before its first tile. us with
     // three / two: 16 x 200 -> 300 56 x 56 12.0 / 11.4, 32 x 256 -> 256 28 x 28 7.1 / 6.7, 32 x 256 -> 512 56 x 56 stride 2 18.7 / 17.1; one 15.8 on
     // that, 13.7 on the first. 128: 9.2 / 8.9 and 18.5 / 19.6)
-    const long resident = pw_resident_blocks(kern);
+    const long resident = pw_resident_blocks((const void*)kern);
     const long cap = (long)num_cus() * 4 * (kc == 8 && resident > 2 ? 2 : resident);
     long waves = items < cap ? items : cap;
     long gcd = q.groups, rest = 4;  // unit = lcm(groups, waves per workgroup)
@@ -441,9 +440,7 @@ TinyNNStatus conv_pw_stream_launch(
 
     note_kernel("conv_pw_stream", kc, ragged);
     note_requant_affine(q.rq.affine());
-    void* args[] = {&q};
-    hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(PW_THREADS), args, 0, stream());
-    MG_REQUIRE(e == hipSuccess, TinyNN_ERROR_RUNTIME, "conv_pw_stream: %s", hipGetErrorString(e));
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(PW_THREADS), 0, stream(), q);
     return check_launch("conv_pw_stream");
 }
 

@@ -7,7 +7,7 @@
 // ends the process with SIGSEGV instead of reading a stray value. Nothing here restates an index
 // formula: the addresses dereferenced are the ones the kernels compute.
 //
-// stdin: one case per line, stdout: "ok <line>" per case; exit status 0 when all of them ran.
+// stdin: one case per line, stdout: "ok <line> -> <kernel noted>" per case; exit status 0 when all of them ran.
 //   mm     M K N ta tb lda_pad ldb_pad ws     f32 MatMul through megcc_gfx950_matmul (gemm / gevm); ws = 1: with split-K room
 //   conv   n ic ih iw oc k s p d bias ws      f32 NCHW convolution through the implicit GEMM
 //   small  n ic ih iw oc k s p d bias         f32 NCHW convolution through conv_f32_small (k = 1 or 3)
@@ -15,11 +15,13 @@
 //   first  n ic ih iw oc k s p bias           f32 first layer, NCHW source -> NCHW44 result
 //   fcone  M K OC packed_bytes bias           qsi8 FullyConnected, M <= 64, one launch
 //   fcgevm M K OC packed_bytes bias           qsi8 FullyConnected, M <= 4
-//   fctile M K OC packed_bytes bias           qsi8 FullyConnected, any M and K
+//   fctile M K OC packed_bytes bias cus       qsi8 FullyConnected, any M and K, on a chip of that many CUs
 //   ks     M K N ta tb lda_pad ldb_pad        f32 MatMul whose waves share K (whatever the dispatch would choose)
 //   split  M K N ta tb lda_pad ldb_pad        f32 MatMul on the bf16 instructions, K >= 32 (likewise)
 //   gather n ic ih iw oc k s p d bias packed_bytes       qsi8 dense NCHW44 convolution without staging
 //   dwpw   n c oc h w stride bias packed_bytes           qsi8 channel-wise 3x3 + pointwise 1x1 in one kernel
+//   pw     n ic ih iw oc stride bias packed_bytes cus    qsi8 pointwise NCHW44 layer, streaming, on a chip of that many CUs
+//   stem   n oh ow oc act bias packed_bytes cus          f32 image -> qsi8 -> first convolution -> channel-wise -> pointwise in one kernel
 #include <hip/hip_runtime.h>
 #include <signal.h>
 #include <stdarg.h>
@@ -42,7 +44,8 @@
 namespace mg {
 // what the kernel sources expect from the rest of the library
 hipStream_t stream() { return nullptr; }
-int num_cus() { return 256; }
+static int g_cus = 256;
+int num_cus() { return g_cus; }
 TinyNNStatus fail(TinyNNStatus st, const char* fmt, ...) {
     va_list ap;
     va_start(ap, fmt);
@@ -55,7 +58,8 @@ Options& options() {
     static Options o = {};
     return o;
 }
-void note_kernel(const char*, int, int, int, int, int) {}
+static std::string g_noted;
+void note_kernel(const char* name, int a, int b, int, int, int) { g_noted = std::string(name) + ":" + std::to_string(a) + "," + std::to_string(b); }
 void note_requant_affine(bool) {}
 // (of the case at hand: the library's own figure, which the test passes in)
 static size_t g_packed_bytes = 0;
@@ -91,6 +95,13 @@ bool fc_tile_supported(const ConvGeom& g);
 TinyNNStatus fc_tile_launch(const ConvGeom&, const void*, const void*, const void*, void*);
 bool conv_gather_i8_supported(const ConvGeom& g);
 TinyNNStatus conv_gather_i8_launch(const ConvGeom&, const void*, const void*, const void*, void*);
+bool conv_pw_stream_supported(const ConvGeom& g);
+bool conv_pw_stream_takes_stride(const ConvGeom& g);
+TinyNNStatus conv_pw_stream_launch(const ConvGeom&, const void*, const void*, const void*, void*);
+bool conv_stem_supported(const ConvGeom&, const ConvGeom&, const ConvGeom&, const void*, const void*);
+TinyNNStatus conv_stem_launch(
+        const ConvGeom&, const ConvGeom&, const ConvGeom&, const void*, const void*, const void*, const void*, const void*, const void*,
+        const void*, void*, bool);
 bool conv_dw_pw_supported(const ConvGeom& dw, const ConvGeom& pw, const void* src, const void* dst);
 TinyNNStatus conv_dw_pw_launch(
         const ConvGeom&, const ConvGeom&, const void*, const void*, const void*, const void*, const void*, void*, DwPwBlock*, bool);
@@ -158,6 +169,7 @@ static bool run_case(const std::string& line, bool at_end) {
     std::stringstream ss(line);
     std::string kind;
     ss >> kind;
+    g_cus = 256;
     if (kind == "mm") {
         int M, K, N, ta, tb, pa, pb, ws;
         ss >> M >> K >> N >> ta >> tb >> pa >> pb >> ws;
@@ -227,6 +239,45 @@ static bool run_case(const std::string& line, bool at_end) {
         return conv_dw_pw_launch(dw, pw, src.ptr, df.ptr, bias ? db.ptr : nullptr, wp.ptr, bias ? pb.ptr : nullptr, dst.ptr, nullptr,
                                  false) == TinyNN_SUCCESS;
     }
+    if (kind == "pw") {
+        ConvGeom g;
+        memset(&g, 0, sizeof(g));
+        int s, bias;
+        ss >> g.n >> g.ic >> g.ih >> g.iw >> g.oc >> s >> bias >> g_packed_bytes >> g_cus;
+        g.fh = g.fw = g.dh = g.dw = 1, g.sh = g.sw = s;
+        g.oh = (g.ih - 1) / s + 1, g.ow = (g.iw - 1) / s + 1;
+        g.groups = 1, g.fmt = MEGCC_FMT_NCHW44, g.act = MEGCC_NONLINE_RELU, g.has_bias = bias;
+        g.s_src = g.s_flt = 0.01f, g.s_dst = 0.1f;
+        Fenced src((size_t)g.n * g.ic * g.ih * g.iw, at_end, 4), wp(g_packed_bytes, at_end, 16), b((size_t)g.oc * 4, at_end, 4),
+                dst((size_t)g.n * g.oc * g.oh * g.ow, at_end, 4);
+        if (!(s == 1 ? conv_pw_stream_supported(g) : conv_pw_stream_takes_stride(g))) {
+            fprintf(stderr, "not a conv_pw_stream layer: %s\n", line.c_str());
+            return false;
+        }
+        return conv_pw_stream_launch(g, src.ptr, wp.ptr, bias ? b.ptr : nullptr, dst.ptr) == TinyNN_SUCCESS;
+    }
+    if (kind == "stem") {
+        ConvGeom c0, dw, pw;
+        memset(&c0, 0, sizeof(c0));
+        int oc, act, bias;
+        ss >> c0.n >> c0.oh >> c0.ow >> oc >> act >> bias >> g_packed_bytes >> g_cus;
+        c0.ic = 3, c0.oc = 32, c0.ih = 2 * c0.oh, c0.iw = 2 * c0.ow, c0.fh = c0.fw = 3, c0.sh = c0.sw = 2;
+        c0.ph = c0.pw = c0.dh = c0.dw = c0.groups = 1, c0.fmt = MEGCC_FMT_NCHW_NCHW44, c0.act = MEGCC_NONLINE_RELU, c0.has_bias = bias;
+        c0.s_src = 1.f / 127, c0.s_flt = 0.0051f, c0.s_dst = 0.037f;
+        dw = c0;
+        dw.ic = dw.oc = dw.groups = 32, dw.ih = c0.oh, dw.iw = c0.ow, dw.sh = dw.sw = 1, dw.fmt = MEGCC_FMT_NCHW44;
+        pw = dw;
+        pw.oc = oc, pw.groups = pw.fh = pw.fw = 1, pw.ph = pw.pw = 0, pw.act = act ? MEGCC_NONLINE_RELU : MEGCC_NONLINE_IDENTITY;
+        Fenced image((size_t)c0.n * 3 * c0.ih * c0.iw * 4, at_end, 4), f0(8 * 27 * 4, at_end, 1), b0(32 * 4, at_end, 4), df(32 * 9, at_end, 4),
+                db(32 * 4, at_end, 4), wp(g_packed_bytes, at_end, 16), pb((size_t)oc * 4, at_end, 4),
+                dst((size_t)c0.n * oc * c0.oh * c0.ow, at_end, 4);
+        if (!conv_stem_supported(c0, dw, pw, image.ptr, dst.ptr)) {
+            fprintf(stderr, "not a conv_stem chain: %s\n", line.c_str());
+            return false;
+        }
+        return conv_stem_launch(c0, dw, pw, image.ptr, f0.ptr, bias ? b0.ptr : nullptr, df.ptr, bias ? db.ptr : nullptr, wp.ptr,
+                                bias ? pb.ptr : nullptr, dst.ptr, true) == TinyNN_SUCCESS;
+    }
     if (kind == "conv" || kind == "small") {
         ConvGeom g;
         memset(&g, 0, sizeof(g));
@@ -290,6 +341,8 @@ static bool run_case(const std::string& line, bool at_end) {
         long packed;
         int bias;
         ss >> g.n >> g.ic >> g.oc >> packed >> bias;
+        if (kind == "fctile")
+            ss >> g_cus;
         g.ih = g.iw = g.oh = g.ow = g.fh = g.fw = g.sh = g.sw = g.dh = g.dw = 1;
         g.groups = 1, g.fmt = MEGCC_FMT_NCHW, g.act = MEGCC_NONLINE_RELU, g.has_bias = bias;
         g.s_src = g.s_flt = 0.01f, g.s_dst = 0.1f;
@@ -341,7 +394,7 @@ int main() {
                 return 1;
             }
         }
-        printf("ok %s\n", line.c_str());
+        printf("ok %s -> %s\n", line.c_str(), mg::g_noted.c_str());
         fflush(stdout);
         ++n;
     }

@@ -110,16 +110,19 @@ inline unsigned __umulhi(unsigned a, unsigned b) { return (unsigned)(((unsigned 
 
 #define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)
-#define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) (c)
-#define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) (c)
-#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) (c)
-#define __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, x, y, z) (c)
-#define __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, x, y, z) (c)
-#define __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, c, x, y, z) (c)
+template <typename A, typename B, typename C>
+inline C audit_sums(const A&, const B&, const C& c, int, int, int) { return c; }
+#define __builtin_amdgcn_mfma_f32_32x32x2f32(...) audit_sums(__VA_ARGS__)
+#define __builtin_amdgcn_mfma_f32_16x16x4f32(...) audit_sums(__VA_ARGS__)
+#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(...) audit_sums(__VA_ARGS__)
+#define __builtin_amdgcn_mfma_i32_32x32x32_i8(...) audit_sums(__VA_ARGS__)
+#define __builtin_amdgcn_mfma_i32_16x16x64_i8(...) audit_sums(__VA_ARGS__)
+#define __builtin_amdgcn_mfma_i32_16x16x32_i8(...) audit_sums(__VA_ARGS__)
 #define __builtin_amdgcn_sdot4(a, b, c, clamp) (c)
 #define __builtin_amdgcn_fmed3f(x, lo, hi) (lo)
 #define __builtin_amdgcn_cvt_pk_u8_f32(x, i, r) (r)
 #define __builtin_amdgcn_perm(a, b, sel) ((a) ^ (b) ^ (sel))
+#define __builtin_amdgcn_alignbyte(hi, lo, n) ((hi) ^ (lo) ^ (n))
 #define __builtin_amdgcn_s_barrier() ((void)0)
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)
 #define __builtin_amdgcn_fence(...) ((void)0)

@@ -1,8 +1,8 @@
 """Host-side bounds audit of the kernels that issue their loads unconditionally from clamped
 indices or through range-checked buffers (gemm_f32: all four transpositions and the implicit-GEMM gather; gemm_f32_ks and
 gemm_f32_split: all four transpositions; gevm_f32; conv_f32_small; the f32 NCHW44 channel-wise and first-layer kernels;
-fc_one32 / fc_one; fc_tile; fc_gevm_q8; conv_gather_i8; conv_dw_pw). Not gemm_f32_ks's convolution, whose addresses come
-through LDS from other threads. tests/host_audit/audit.cpp links the library's own kernel sources,
+fc_one32 / fc_one; every part of fc_tile; fc_gevm_q8; conv_gather_i8; conv_pw_stream / conv_pw_share with and without a stride; conv_dw_pw;
+conv_stem). Not gemm_f32_ks's convolution, whose addresses come through LDS from other threads. tests/host_audit/audit.cpp links the library's own kernel sources,
 compiled as host C++ against a stand-in HIP header that runs every thread of every workgroup on
 the CPU, and fences each operand buffer with inaccessible pages: one element outside a tensor ends
 the run. No GPU involved; the shapes are every case of the GPU sweeps plus a seeded sweep of ragged
@@ -23,7 +23,7 @@ AUDIT_DIR = os.path.join(HERE, "host_audit")
 CSRC = os.path.join(os.path.dirname(HERE), "megcc_amd", "csrc")
 CLANG = "/opt/rocm/llvm/bin/clang++"
 SOURCES = ["gemm_f32", "gevm_f32", "conv_f32_small", "conv_f32_nchw44", "fc_stream", "fc_gevm_q8", "fc_tile", "gemm_f32_ks",
-           "gemm_f32_split", "conv_gather_i8", "conv_dw_pw", "requant_table"]
+           "gemm_f32_split", "conv_gather_i8", "conv_pw_stream", "conv_dw_pw", "conv_stem", "requant_table"]
 
 pytestmark = pytest.mark.skipif(not os.path.exists(CLANG), reason="needs ROCm's clang++ for the kernels' vector types")
 
@@ -44,7 +44,7 @@ def compile_audit(out_dir, replace=None, have=None):
             objs.append(os.path.join(have, name + ".o"))
             continue
         objs.append(obj)
-        last = ["-O0", "-g0"] if name == "conv_dw_pw" else []  # (128 instances: half a minute with the optimiser)
+        last = ["-O0", "-g0"] if name in ("conv_dw_pw", "conv_pw_stream") else []  # (some 100 instances: half a minute with the optimiser)
         jobs.append(subprocess.Popen([CLANG] + flags + last + ["-c", src, "-o", obj], stderr=subprocess.PIPE, text=True))
     for j in jobs:
         err = j.communicate()[1]
@@ -89,6 +89,9 @@ def line_of(case, with_ws=1):
                                                        case.sh, case.ph, case.dh, int(case.bias), tail)
     kind = "fcgevm" if case.n <= 4 else "fcone"
     return "%s %d %d %d %d %d" % (kind, case.n, case.ic, case.oc, packed_bytes(case), int(case.bias))
+
+
+FC_TILE_PARTS = [(130, 65, 150), (131, 260, 149), (129, 127, 193), (100, 2049, 101), (128, 2052, 98), (130, 2049, 129), (200, 1924, 130)]
 
 
 def audit_lines():
@@ -167,7 +170,11 @@ def audit_lines():
     for m, k, oc in ((65, 5, 9), (64, 1, 3), (16, 1, 1), (65, 129, 67), (70, 295, 70), (225, 515, 361), (66, 128, 64), (130, 260, 257),
                      (100, 1123, 65), (65, 127, 129), (300, 33, 31)):
         case = ConvCase(abi.FMT_NCHW, abi.DENSE, m, k, 1, 1, oc, 1, 1, 0, abi.RELU, scales=(0.01, 0.01, 0.1))
-        lines.append("fctile %d %d %d %d %d" % (m, k, oc, packed_bytes(case), i & 1))
+        lines.append("fctile %d %d %d %d %d 256" % (m, k, oc, packed_bytes(case), i & 1))
+    # ... and each part at its smallest, on a chip of four CUs: 64 x 64 alone, with four groups, 128 x 128; rows at odd bytes and on words
+    for m, k, oc in FC_TILE_PARTS:
+        case = ConvCase(abi.FMT_NCHW, abi.DENSE, m, k, 1, 1, oc, 1, 1, 0, abi.RELU, scales=(0.01, 0.01, 0.1))
+        lines.append("fctile %d %d %d %d %d 4" % (m, k, oc, packed_bytes(case), k & 1))
     # qsi8 layers without staging, and channel-wise + pointwise pairs: the shapes of their GPU tests
     for case in gp.GATHER:
         if case.n * case.oh * case.ow <= 6000:
@@ -179,6 +186,22 @@ def audit_lines():
         if n * c * h * w <= 1 << 19:
             pw = ConvCase(abi.FMT_NCHW44, abi.DENSE, n, c, (h - 1) // s + 1, (w - 1) // s + 1, oc, 1, 1, 0, act, scales=(0.01, 0.01, 0.1))
             lines.append("dwpw %d %d %d %d %d %d %d %d" % (n, c, oc, h, w, s, (h + w) & 1, packed_bytes(pw)))
+    # pointwise layers, on a chip small enough that the shared form and several tiles a wave are among them; with a stride the shapes
+    # of their GPU test with fewer images, without one channels and pixels off every tile
+    for case in gp.STRIDED_1X1_IN_PLACE:
+        n = min(case.n, 8)
+        if n * case.oh * case.ow >= 32 and case.ic * case.ih * case.iw <= 1 << 18:
+            lines.append("pw %d %d %d %d %d %d %d %d 8" % (n, case.ic, case.ih, case.iw, case.oc, case.sh, int(case.bias), packed_bytes(case)))
+    for n, ic, h, w, oc in ((1, 32, 6, 7, 64), (2, 20, 13, 5, 36), (1, 68, 8, 4, 100), (3, 256, 7, 7, 64), (1, 512, 9, 9, 32), (2, 1024, 5, 4, 64), (1, 136, 9, 7, 44),
+                            (4, 512, 11, 7, 128)):
+        case = ConvCase(abi.FMT_NCHW44, abi.DENSE, n, ic, h, w, oc, 1, 1, 0, abi.RELU, scales=(0.01, 0.01, 0.1))
+        lines.append("pw %d %d %d %d %d 1 %d %d 4" % (n, ic, h, w, oc, h & 1, packed_bytes(case)))
+    # the head of a network in one kernel: the shapes of its GPU test, as one strip an image and as several
+    import test_stem
+    for n, oh, ow, oc, act, bias, _ in test_stem.CASES:
+        pw = ConvCase(abi.FMT_NCHW44, abi.DENSE, min(n, 3), 32, oh, ow, oc, 1, 1, 0, act, scales=(0.01, 0.01, 0.1))
+        for cus in (1, 16):
+            lines.append("stem %d %d %d %d %d %d %d %d" % (min(n, 3), oh, ow, oc, int(act == abi.RELU), int(bias), packed_bytes(pw), cus))
     # qsi8 FullyConnected: 1..64 rows, K = 1..32 blocks of 128 (and beyond 4096), channel counts off every tile size
     for i in range(24):
         m = int(r.choice([1, 2, 3, 4, 5, 31, 32, 33, 63, 64]))
@@ -196,6 +219,10 @@ def test_every_load_and_store_of_the_clamped_kernels_stays_inside_its_tensor(aud
     r = subprocess.run([audit_exe], input="\n".join(lines) + "\n", capture_output=True, text=True, timeout=1500)
     assert r.returncode == 0, "bounds audit failed:\n%s\n%s" % (r.stdout[-1500:], r.stderr[-3000:])
     assert "audited %d cases" % len(lines) in r.stdout
+    ran = {line.split(" -> ")[1] for line in r.stdout.splitlines() if " -> " in line}
+    for kernel in ("fc_tile:32,4", "fc_tile:64,1", "fc_tile:64,4", "fc_tile:128,1", "conv_pw_share:16,-1", "conv_pw_stream:1,0",
+                   "conv_pw_stream:8,1", "conv_pw_stream:32,0", "conv_stem:64,1", "conv_stem:32,1", "conv_stem:64,14"):
+        assert kernel in ran, (kernel, sorted(ran))
 
 
 def test_the_audit_sees_the_out_of_bounds_read_a_missing_clamp_causes(audit_exe, tmp_path):
@@ -211,13 +238,36 @@ def test_the_audit_sees_the_out_of_bounds_read_a_missing_clamp_causes(audit_exe,
     assert r.returncode == 3 and "OUT OF BOUNDS" in r.stderr, (r.returncode, r.stderr[-500:])
 
 
-def test_the_audit_sees_a_row_read_past_the_end_of_its_tensor(audit_exe, tmp_path):
-    """likewise for loads at any byte: without the step back to the tensor's last 16 bytes"""
-    src = open(os.path.join(CSRC, "fc_tile.hip")).read()
-    clamp = "min(roff[i] + b, q.last16)"
-    assert src.count(clamp) == 1
-    mutated = tmp_path / "fc_tile.hip"
-    mutated.write_text(src.replace(clamp, "(roff[i] + b)"))
-    exe = compile_audit(str(tmp_path / "build"), replace={"fc_tile": str(mutated)}, have=os.path.dirname(audit_exe))
-    r = subprocess.run([exe], input="fctile 65 129 67 65536 0\n", capture_output=True, text=True, timeout=300)
+@pytest.mark.parametrize("line", ["fctile 65 129 67 65536 0 256", "fctile 130 65 150 65536 0 4", "fctile 100 2049 101 1048576 1 4",
+                                  "fctile 130 2049 129 1048576 1 4"])
+def test_the_audit_sees_a_row_read_past_the_end_of_its_tensor(audit_exe, tmp_path_factory, line):
+    """likewise for loads at any byte, in every part: without the step back to the tensor's last 16 bytes"""
+    if not _no_clamp:
+        src = open(os.path.join(CSRC, "fc_tile.hip")).read()
+        clamp = "min(roff[i] + b, q.last16)"
+        assert src.count(clamp) == 1
+        folder = tmp_path_factory.mktemp("no_clamp")
+        mutated = folder / "fc_tile.hip"
+        mutated.write_text(src.replace(clamp, "(roff[i] + b)"))
+        _no_clamp.append(compile_audit(str(folder / "build"), replace={"fc_tile": str(mutated)}, have=os.path.dirname(audit_exe)))
+    r = subprocess.run([_no_clamp[0]], input=line + "\n", capture_output=True, text=True, timeout=300)
     assert r.returncode == 3 and "OUT OF BOUNDS" in r.stderr, (r.returncode, r.stderr[-500:])
+
+
+@pytest.mark.parametrize("source,was,by,line", [
+    # pixels beyond the last one; the result's rows below an odd last one (both also without the buffer's own range check)
+    ("conv_pw_stream", "return tile < tend && p < q.P", "return true || (tile < tend && p < q.P)", "pw 3 20 13 11 36 2 0 65536 8"),
+    ("conv_stem", "there && 2 * t + row < q.oh ?", "there ?", "stem 1 7 12 32 0 0 32768 1"),
+])
+def test_the_audit_sees_a_missing_range_test(audit_exe, tmp_path, source, was, by, line):
+    src = open(os.path.join(CSRC, source + ".hip")).read()
+    assert was in src
+    mutated = tmp_path / (source + ".hip")
+    mutated.write_text(src.replace(was, by).replace("make_buffer_rsrc((void*)q.src, 0, q.src_bytes", "make_buffer_rsrc((void*)q.src, 0, 0x7fffffff")
+                       .replace("make_buffer_rsrc((void*)q.dst, 0, q.dst_bytes", "make_buffer_rsrc((void*)q.dst, 0, 0x7fffffff"))
+    exe = compile_audit(str(tmp_path / "build"), replace={source: str(mutated)}, have=os.path.dirname(audit_exe))
+    r = subprocess.run([exe], input=line + "\n", capture_output=True, text=True, timeout=300)
+    assert r.returncode == 3 and "OUT OF BOUNDS" in r.stderr, (r.returncode, r.stderr[-500:])
+
+
+_no_clamp = []
