@@ -216,10 +216,6 @@ RequantAffine requant_affine_for(int act, float s_src, float s_flt, float s_dst)
 RequantAffine requant_affine_pick(bool table, int act, float s_src, float s_flt, float s_dst);
 
 template <int ACT>
-__host__ __device__ __forceinline__ int requant_affine_lo() {
-    return ACT == MEGCC_NONLINE_RELU ? 0 : -128;
-}
-template <int ACT>
 __device__ __forceinline__ int requant_conv_affine(int acc, float c, float d) {
     constexpr int LO = ACT == MEGCC_NONLINE_RELU ? 0 : -128;
     const int m = cvt_floor_i32(__builtin_fmaf((float)acc, c, d));  // saturating conversion
@@ -231,6 +227,30 @@ __device__ __forceinline__ uint32_t pack4_perm(int a, int b, int c, int d) {
     const uint32_t lo = __builtin_amdgcn_perm((uint32_t)b, (uint32_t)a, 0x0c0c0400u);
     const uint32_t hi = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)c, 0x0c0c0400u);
     return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
+// bytes 1 and 3 of two pairs of 16-bit values -> one dword: their floor by 256
+__device__ __forceinline__ uint32_t pack4_high(uint32_t ab, uint32_t cd) {
+    return __builtin_amdgcn_perm(cd, ab, 0x07050301u);
+}
+// two ints saturated to 16 bits
+__device__ __forceinline__ uint32_t pack2_sat(int a, int b) {
+#ifndef MG_HOST_AUDIT
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pk_i16(a, b));
+#else
+    return (uint32_t)(a ^ b);
+#endif
+}
+// IDENTITY's clamp and the packing of whole outputs: times 256 with saturation two by two, of which the upper bytes are the outputs. 5
+// instructions for four of them; the clamp of every one by itself and pack4_perm took 7 (us, 16 x 128 -> 256 28 x 28 3x3 10.22 / 10.13, 34 x 44 ->
+// 60 67 x 67 16.17 / 16.07; with mode 4 15 for 19, 32 x 64 -> 64 56 x 56 pointwise 5.71 / 5.35).
+__device__ __forceinline__ uint32_t pack4_clamp(int a, int b, int c, int d) {
+    uint32_t ab = pack2_sat(a, b), cd = pack2_sat(c, d);
+#ifndef MG_HOST_AUDIT
+    asm("v_pk_mad_i16 %0, %0, %1, 0 clamp" : "+v"(ab) : "s"(0x01000100));
+    asm("v_pk_mad_i16 %0, %0, %1, 0 clamp" : "+v"(cd) : "s"(0x01000100));
+#endif
+    return pack4_high(ab, cd);
 }
 
 // ---- four outputs at a time, without a table ------------------------------------------------------
@@ -258,7 +278,7 @@ __device__ __forceinline__ uint32_t pack4_perm(int a, int b, int c, int d) {
 // those of the float 1.5 * 2^23 + a + m as long as |a + m| < 2^22, where all steps lie (it is asked for), and beyond
 // that floats that still grow with a. d is about 10^4 / c of its last bit there, too coarse to put it between the
 // steps; the whole number m, a few hundred at most, shifts them until a float falls there.
-// Vector instructions for four outputs: 10 (mode 5), 14, 18 - 22, 19, 31 (mode 6), and mode 3 30 (RELU), 39 (IDENTITY), 46 (H_SWISH); the
+// Vector instructions for four outputs: 10 (mode 5), 14, 18 - 22, 15 (mode 4), 29 (mode 6), and mode 3 30 (RELU), 37 (IDENTITY), 46 (H_SWISH); the
 // threshold table's look-ups took 35 (H_SWISH 51) and four gathers from LDS, and its 1 KB among a launch's
 // arguments 0.7 us of the host's time.
 // (mode 0: none of these was proven; s1, s2, c are then the reference's three scales, for requant_conv)
@@ -297,8 +317,7 @@ __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3
             const float x = (float)a[i] * q.s1 * q.s2;
             float v = __builtin_fmaf(x, q.c, x * q.d);  // (RELU: twice the quotient)
             if (ACT == MEGCC_NONLINE_IDENTITY) {
-                const int t = cvt_i32(v + __builtin_copysignf(HALF, v));
-                o[i] = t > 127 ? 127 : (t < -128 ? -128 : t);
+                o[i] = cvt_i32(v + __builtin_copysignf(HALF, v));
                 continue;
             }
             if (ACT == MEGCC_NONLINE_H_SWISH)
@@ -306,23 +325,24 @@ __device__ __forceinline__ uint32_t requant_pack4(int a0, int a1, int a2, int a3
             r = __builtin_amdgcn_cvt_pk_u8_f32(v + HALF, i, r);
         }
         if (ACT == MEGCC_NONLINE_IDENTITY)
-            return pack4_perm(o[0], o[1], o[2], o[3]);
+            return pack4_clamp(o[0], o[1], o[2], o[3]);
         return (r >> 1) & 0x7f7f7f7fu;
     } else if constexpr (MODE == 6) {
         int o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float x = (float)a[i] * q.s1 * q.s2;
-            const int t = cvt_i32(__builtin_fmaf(x, q.c, __builtin_copysignf(q.d, x)));
-            o[i] = t > 127 ? 127 : (t < -128 ? -128 : t);
+            o[i] = cvt_i32(__builtin_fmaf(x, q.c, __builtin_copysignf(q.d, x)));
         }
-        return pack4_perm(o[0], o[1], o[2], o[3]);
+        return pack4_clamp(o[0], o[1], o[2], o[3]);
     } else if constexpr (MODE == 4) {
+        // (256 times the value, which changes no rounding: the floor of its floor by 256, and saturation at 16 bits is the clamp)
+        const float c = q.c * 256.f, d = q.d * 256.f;
         int o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            o[i] = requant_conv_affine<ACT>(a[i], q.c, q.d);
-        return pack4_perm(o[0], o[1], o[2], o[3]);
+            o[i] = cvt_floor_i32(__builtin_fmaf((float)a[i], c, d));
+        return pack4_high(pack2_sat(o[0], o[1]), pack2_sat(o[2], o[3]));
     } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
