@@ -471,7 +471,6 @@ MG_INLINE static RequantPack pack_exact(int act, float s_src, float s_flt, float
 MG_INLINE static RequantPack pack_shifted(int act, float s_src, float s_flt, float s_dst, const RequantSteps& pts) {
     const RequantPack none = {s_src, s_flt, s_dst, 0.f, 0};
     const bool relu = act == MEGCC_NONLINE_RELU;
-    const int lowest = relu ? 0 : -128;
     RequantBounds<true> from;
     RequantBounds<false> to;
     for (int i = 2; i < pts.n; ++i) {
