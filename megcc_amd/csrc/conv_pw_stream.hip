@@ -14,6 +14,8 @@
 //     tile's MFMAs;
 //   * results leave like in the tiled kernels: 4 consecutive accumulator registers are the 4
 //     channels of one NCHW44 dword, 32 lanes store 128 contiguous bytes.
+// Instances of 1, 2, 4, 8, 12 and 16 chunks: a layer between two computes the larger one's products with zeros (12 for 257 .. 384
+// channels, us with 16 / 12: 16 x 300 -> 300 56 x 56 RELU 20.2 / 18.1, IDENTITY 23.0 / 20.2, 11 x 296 -> 208 90 x 90 24.4 / 21.9, 25.5 / 22.7).
 // Waves never synchronise after the set-up (bias to LDS), so any number of
 // them can be resident and the memory latency is hidden by occupancy.
 //
@@ -97,7 +99,7 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
     // positions ahead of their MFMA in the sequence (tile, chunk) -> tile * KC + chunk: four tiles
     // ahead with 32 input channels, half a tile with 512. The loop is unrolled over U tiles so that
     // every ring slot and every "which tile, which chunk" below is a compile-time constant.
-    constexpr int RING = KC == 1 ? 4 : KC == 2 ? 6 : KC >= 16 ? 16 : 8;
+    constexpr int RING = KC == 1 ? 4 : KC == 2 ? 6 : KC == 12 ? 12 : KC >= 16 ? 16 : 8;
     constexpr int U = RING > KC ? RING / KC : 1;           // tiles per unrolled step
     constexpr int AHEAD = (RING + KC - 1) / KC;            // tiles a request can be ahead
     static_assert(RING % KC == 0 || KC % RING == 0, "slots repeat every U tiles");
@@ -122,6 +124,10 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
         }
     };
 
+    // The sums' start of a tile, the bias, is kept in registers where it made a tile shorter (us from LDS / kept): 256 channels, with the
+    // one branch a tile below, 32 x 256 -> 256 56 x 56 17.8 / 17.2 (IDENTITY), 16.3 / 15.9 (RELU); 512, whose other activations lose by it,
+    // 16 x 400 -> 400 40 x 40 23.3 / 23.0 (RELU 22.0 / 22.1, 16 x 300 -> 300 56 x 56 with 16 chunks 20.2 / 20.5)
+    constexpr bool KEEP = KC == 8 || (KC == 16 && ACT == MEGCC_NONLINE_IDENTITY);
     v4i ring[RING];
     static_for<RING>([&](auto sc) {
         constexpr int s = decltype(sc)::value;
@@ -132,6 +138,21 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
     for (int i = tid; i < (RG ? q.groups * (32 * MT) : q.OC); i += PW_THREADS)
         bias_lds[i] = q.bias && i < q.OC ? q.bias[i] : 0;
     __syncthreads();
+    // register e of a tile: channel 8 * (e / 4) + 4 * kg + e % 4
+    auto starts = [&](v16i (&acc)[MT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                const v4i bv = *(const v4i*)(bias_lds + og * (32 * MT) + mi * 32 + e4 * 8 + kg * 4);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    acc[mi][e4 * 4 + k] = bv[k];
+            }
+    };
+    v16i bias[MT];
+    if constexpr (KEEP)
+        starts(bias);
 
     for (; t < tend; t += U) {
         unsigned base[U + AHEAD];  // of tiles t, t + 1, ...: the targets of this step's requests
@@ -144,17 +165,12 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
             const int tile = t + u;
             if (tile < tend) {
                 v16i acc[MT];
+                if constexpr (KEEP)
 #pragma unroll
-                for (int mi = 0; mi < MT; ++mi) {
-                    // register e of a tile: channel 8 * (e / 4) + 4 * kg + e % 4
-#pragma unroll
-                    for (int e4 = 0; e4 < 4; ++e4) {
-                        const v4i bv = *(const v4i*)(bias_lds + og * (32 * MT) + mi * 32 + e4 * 8 + kg * 4);
-#pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            acc[mi][e4 * 4 + k] = bv[k];
-                    }
-                }
+                    for (int mi = 0; mi < MT; ++mi)
+                        acc[mi] = bias[mi];
+                else
+                    starts(acc);
                 static_for<KC>([&](auto cc) {
                     constexpr int c = decltype(cc)::value;
                     constexpr int s = u * KC + c, slot = s % RING;
@@ -169,20 +185,21 @@ __global__ void __launch_bounds__(PW_THREADS) conv_pw_stream_kernel(PwParams q) 
                 const bool ok = p < q.P;
                 const int n = fdiv(p, q.dOHW);
                 const int obase = n * (q.OC >> 2) * q.OHW + (p - n * q.OHW);
+                constexpr int PART = RG ? 1 : MT;  // row tiles requantised in one branch (in one each 32 x 256 -> 256 56 x 56 18.6 us, IDENTITY; now 17.8)
 #pragma unroll
-                for (int mi = 0; mi < MT; ++mi) {
-                    if (RG && (og * MT + mi) * 32 >= q.OC)  // (wave-uniform: a tile of surplus channels)
+                for (int m0 = 0; m0 < MT; m0 += PART) {
+                    if (RG && (og * MT + m0) * 32 >= q.OC)  // (wave-uniform: a tile of surplus channels)
                         continue;
-                    int a[16];
+                    int a[16 * PART];
 #pragma unroll
-                    for (int e = 0; e < 16; ++e)
-                        a[e] = acc[mi][e];
-                    uint32_t d[4];
+                    for (int e = 0; e < 16 * PART; ++e)
+                        a[e] = acc[m0 + e / 16][e % 16];
+                    uint32_t d[4 * PART];
                     requant_dwords<ACT>(a, d, q.rq, q.act);
                     if (ok) {
 #pragma unroll
-                        for (int e4 = 0; e4 < 4; ++e4) {
-                            const int oc4 = og * (8 * MT) + mi * 8 + e4 * 2 + kg;
+                        for (int e4 = 0; e4 < 4 * PART; ++e4) {
+                            const int oc4 = og * (8 * MT) + m0 * 8 + e4 * 2 + kg;
                             if (!RG || oc4 * 4 < q.OC)
                                 q.dst[obase + oc4 * q.OHW] = d[e4];
                         }
@@ -355,10 +372,10 @@ TinyNNStatus conv_pw_stream_launch(
     q.OCP = (g.oc + OC_PAD - 1) / OC_PAD * OC_PAD;
     q.tiles = (q.P + 31) / 32;
     q.IC4 = g.ic >> 2;
-    // (ragged channel counts: IC below the next power of two of 32-channel chunks, OC no multiple of
+    // (ragged channel counts: IC below the chunks of an instance, OC no multiple of
     //  a wave's 64 / 32 channels)
     const int chunks = (g.ic + 31) / 32;
-    const int kc = chunks <= 1 ? 1 : chunks <= 2 ? 2 : chunks <= 4 ? 4 : chunks <= 8 ? 8 : chunks <= 16 ? 16 : 32;
+    const int kc = chunks <= 1 ? 1 : chunks <= 2 ? 2 : chunks <= 4 ? 4 : chunks <= 8 ? 8 : chunks <= 12 ? 12 : chunks <= 16 ? 16 : 32;
     const int per_wave = kc > 8 ? 32 : 64;
     const bool ragged = g.ic != kc * 32 || g.oc % per_wave != 0;
     q.groups = (g.oc + per_wave - 1) / per_wave;
@@ -386,6 +403,7 @@ TinyNNStatus conv_pw_stream_launch(
         case 2: kern = MG_PW_PICK(2, 2); break;
         case 4: kern = MG_PW_PICK(4, 2); break;
         case 8: kern = MG_PW_PICK(8, 2); break;
+        case 12: kern = MG_PW_PICK(12, 1); break;
         case 16: kern = MG_PW_PICK(16, 1); break;  // 512 input channels: 32 output channels per wave
         default: kern = MG_PW_PICK_RG(32, 1, false); break;  // 1024: the filter rows fill half the registers
     }

@@ -193,7 +193,7 @@ def audit_lines():
         if n * case.oh * case.ow >= 32 and case.ic * case.ih * case.iw <= 1 << 18:
             lines.append("pw %d %d %d %d %d %d %d %d 8" % (n, case.ic, case.ih, case.iw, case.oc, case.sh, int(case.bias), packed_bytes(case)))
     for n, ic, h, w, oc in ((1, 32, 6, 7, 64), (2, 20, 13, 5, 36), (1, 68, 8, 4, 100), (3, 256, 7, 7, 64), (1, 512, 9, 9, 32), (2, 1024, 5, 4, 64), (1, 136, 9, 7, 44),
-                            (4, 512, 11, 7, 128)):
+                            (4, 512, 11, 7, 128), (1, 384, 9, 7, 64), (3, 260, 8, 5, 36)):
         case = ConvCase(abi.FMT_NCHW44, abi.DENSE, n, ic, h, w, oc, 1, 1, 0, abi.RELU, scales=(0.01, 0.01, 0.1))
         lines.append("pw %d %d %d %d %d 1 %d %d 4" % (n, ic, h, w, oc, h & 1, packed_bytes(case)))
     # the head of a network in one kernel: the shapes of its GPU test, as one strip an image and as several
@@ -221,7 +221,7 @@ def test_every_load_and_store_of_the_clamped_kernels_stays_inside_its_tensor(aud
     assert "audited %d cases" % len(lines) in r.stdout
     ran = {line.split(" -> ")[1] for line in r.stdout.splitlines() if " -> " in line}
     for kernel in ("fc_tile:32,4", "fc_tile:64,1", "fc_tile:64,4", "fc_tile:128,1", "conv_pw_share:16,-1", "conv_pw_stream:1,0",
-                   "conv_pw_stream:8,1", "conv_pw_stream:32,0", "conv_stem:64,1", "conv_stem:32,1", "conv_stem:64,14"):
+                   "conv_pw_stream:8,1", "conv_pw_stream:12,0", "conv_pw_stream:12,1", "conv_pw_stream:32,0", "conv_stem:64,1", "conv_stem:32,1", "conv_stem:64,14"):
         assert kernel in ran, (kernel, sorted(ran))
 
 

@@ -797,6 +797,20 @@ def test_strided_pointwise_in_place(case):
     compare(run_gpu(case, arrays), case.run_port(arrays), repr(case))
 
 
+# nine to twelve K chunks, the borders either side, whole and ragged channels, several tiles a wave, pixels read with a stride
+@pytest.mark.parametrize("act", [A.IDENTITY, A.RELU, A.H_SWISH, A.SIGMOID])
+@pytest.mark.parametrize("n,ic,ih,iw,oc,s,kernel", [
+    (1, 256, 9, 8, 64, 1, "8,0"), (1, 260, 9, 8, 64, 1, "12,1"), (3, 288, 7, 9, 36, 1, "12,1"), (9, 384, 56, 56, 96, 1, "12,0"),
+    (40, 356, 33, 31, 100, 1, "12,1"), (2, 384, 15, 11, 32, 2, "12,0"), (3, 300, 12, 13, 44, 3, "12,1"), (1, 388, 9, 8, 32, 1, "16,1")])
+def test_pointwise_layers_of_twelve_chunks(n, ic, ih, iw, oc, s, kernel, act):
+    port.set_threads(8)
+    case = ConvCase(A.FMT_NCHW44, A.DENSE, n, ic, ih, iw, oc, 1, s, 0, act, scales=(0.02, 0.01, unsat(ic)))
+    arrays = case.gen(seed=60)
+    got = run_gpu(case, arrays)
+    assert runtime.last_kernel().split("+")[0] == "conv_pw_stream:" + kernel, runtime.last_kernel()
+    compare(got, case.run_port(arrays), repr(case))
+
+
 DOT4 = [
     # dense NCHW44 layers the matrix-core kernels do not take (more than 9 taps): the dot-product
     # kernel; both channel-group widths, an odd number of channel groups, stride, dilation,
