@@ -261,20 +261,20 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
     // Epilogue of one 32 oc x 32 pixel MFMA tile (16 outputs per lane = 4 NCHW44 dwords), written
     // as one straight-line block. ob: dword index in dst of this lane's pixel in oc-group 0 (-1: lane beyond the
     // sub-tile, -2: whole 32-pixel column beyond it, wave-uniform).
-    // the 16 requantised outputs of this lane in tile (mi, ni): 4 channels a dword
-    auto requant_tile = [&](auto mic, auto nic, uint32_t (&w)[4]) __attribute__((always_inline)) {
-        constexpr int mi = decltype(mic)::value, ni = decltype(nic)::value;
+    // the 16 requantised outputs of this lane in tile (mi, ni): 4 channels a dword. form: four sums -> one dword.
+    // With four tiles and more a wave the form is chosen once for all of them, not in front of each (us, IDENTITY: 16 x 256 -> 128 28 x 28 5x5
+    // 37.3 / 36.5, 16 x 128 -> 256 28 x 28 10.24 / 10.11, RELU 10.15 / 9.87, 32 x 256 -> 256 56 x 56 59.6 / 58.3; two tiles, 10 x 452 -> 108 40 x 40
+    // 5x5, 51.3 / 51.95).
+    constexpr bool ONE_FORM = MT * NT >= 4 || ACT == ACT_RT;
+    auto requant_tile = [&](auto mic, auto nic, const auto& form, uint32_t (&w)[4]) __attribute__((always_inline)) {
         int a[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-            a[e] = acc[mi][ni][e];
-        if constexpr (ACT == ACT_RT) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                a[e] = requant_conv_rt(q.act, a[e], q.s_src, q.s_flt, q.s_dst);
+            a[e] = acc[decltype(mic)::value][decltype(nic)::value][e];
+        if constexpr (ONE_FORM) {
 #pragma unroll
             for (int e4 = 0; e4 < 4; ++e4)
-                w[e4] = pack4_perm(a[e4 * 4], a[e4 * 4 + 1], a[e4 * 4 + 2], a[e4 * 4 + 3]);
+                w[e4] = form(a[e4 * 4], a[e4 * 4 + 1], a[e4 * 4 + 2], a[e4 * 4 + 3]);
         } else {
             requant_dwords<ACT>(a, w, q.rq);
         }
@@ -283,15 +283,15 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
     // the lane's column. A lane's four dwords are channels 8 e4 + 4 kg .. + 3, so lanes l and l + 32
     // (same row, the two K-halves) together own 32 consecutive bytes; two v_permlane32_swap give the
     // lower lane the first 16 of them and the upper lane the rest.
-    auto fc_piece = [&](auto mic, auto nic) __attribute__((always_inline)) -> v4u {
+    auto fc_piece = [&](auto mic, auto nic, const auto& form) __attribute__((always_inline)) -> v4u {
         typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
         uint32_t w[4];
-        requant_tile(mic, nic, w);
+        requant_tile(mic, nic, form, w);
         const v2u_t s02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
         const v2u_t s13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
         return v4u{s02[0], s02[1], s13[0], s13[1]};
     };
-    auto emit_tile = [&](auto mic, auto nic, const int ob) __attribute__((always_inline)) {
+    auto emit_tile = [&](auto mic, auto nic, const auto& form, const int ob) __attribute__((always_inline)) {
         constexpr int mi = decltype(mic)::value;
         if (ob < -1)
             return;
@@ -301,14 +301,14 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
             // store per lane instead of four dword stores 4096 bytes apart from their neighbours' (the
             // dword stores were half of the 4096 x 4096 x 4096 layer's time).
             if (q.dst_fc >= 2) {  // (uniform)
-                const v4u px = fc_piece(mic, nic);
+                const v4u px = fc_piece(mic, nic, form);
                 if (ob >= 0 && oc0 + (wm * MT + mi) * 32 < q.OC)  // (whole tiles: OC is a multiple of 32)
                     *(v4u*)(q.dst + (size_t)ob * q.OC + oc0 + (wm * MT + mi) * 32 + kg * 16) = px;
                 return;
             }
         }
         uint32_t d[4];
-        requant_tile(mic, nic, d);
+        requant_tile(mic, nic, form, d);
         if (ob >= 0) {
 #pragma unroll
             for (int e4 = 0; e4 < 4; ++e4) {
@@ -452,40 +452,51 @@ __global__ void __launch_bounds__(256 * WGM, BPC) conv_mfma_i8_dma_kernel(MfmaPa
                 run_stages(cc);
         });
 
-        if constexpr (FCB && MT == 4) {  // (the 256-channel tile: its two stage buffers leave room for the staging area)
-            // dst_fc == 3: the rows leave through a staging area in LDS (this wave's own 32 rows x 64
-            // bytes, rows 80 bytes apart): the lanes park the 16-byte pieces of two neighbouring tiles
-            // and read them back four lanes to a row, so that a store instruction writes 64 contiguous
-            // bytes of each of 16 rows instead of 32 bytes of each of 32.
-            if (q.dst_fc == 3) {  // (uniform)
-                int8_t* const stage = (int8_t*)(bias_lds + (DM_BM > 128 ? DM_BM : 128)) + wave * FC_STAGE_BYTES;
-                static_for<NT>([&](auto nic) {
-                    constexpr int ni = decltype(nic)::value;
-                    if (cur_o[ni] < -1)
-                        return;
-                    const int row0 = p0 + (ni * WGN + wn) * 32;  // first row of this 32-row column
-                    static_for<MT / 2>([&](auto hc) {
-                        constexpr int h = decltype(hc)::value;
-                        const v4u pa = fc_piece(std::integral_constant<int, 2 * h>{}, nic);
-                        const v4u pb = fc_piece(std::integral_constant<int, 2 * h + 1>{}, nic);
-                        *(v4u*)(stage + (lane & 31) * FC_STAGE_ROW + kg * 16) = pa;
-                        *(v4u*)(stage + (lane & 31) * FC_STAGE_ROW + 32 + kg * 16) = pb;
-                        const int ocb = oc0 + (wm * MT + 2 * h) * 32;  // (64 channels from here on)
+        auto emit = [&](const auto& form) __attribute__((always_inline)) {
+            if constexpr (FCB && MT == 4) {  // (the 256-channel tile: its two stage buffers leave room for the staging area)
+                // dst_fc == 3: the rows leave through a staging area in LDS (this wave's own 32 rows x 64
+                // bytes, rows 80 bytes apart): the lanes park the 16-byte pieces of two neighbouring tiles
+                // and read them back four lanes to a row, so that a store instruction writes 64 contiguous
+                // bytes of each of 16 rows instead of 32 bytes of each of 32.
+                if (q.dst_fc == 3) {  // (uniform)
+                    int8_t* const stage = (int8_t*)(bias_lds + (DM_BM > 128 ? DM_BM : 128)) + wave * FC_STAGE_BYTES;
+                    static_for<NT>([&](auto nic) {
+                        constexpr int ni = decltype(nic)::value;
+                        if (cur_o[ni] < -1)
+                            return;
+                        const int row0 = p0 + (ni * WGN + wn) * 32;  // first row of this 32-row column
+                        static_for<MT / 2>([&](auto hc) {
+                            constexpr int h = decltype(hc)::value;
+                            const v4u pa = fc_piece(std::integral_constant<int, 2 * h>{}, nic, form);
+                            const v4u pb = fc_piece(std::integral_constant<int, 2 * h + 1>{}, nic, form);
+                            *(v4u*)(stage + (lane & 31) * FC_STAGE_ROW + kg * 16) = pa;
+                            *(v4u*)(stage + (lane & 31) * FC_STAGE_ROW + 32 + kg * 16) = pb;
+                            const int ocb = oc0 + (wm * MT + 2 * h) * 32;  // (64 channels from here on)
 #pragma unroll
-                        for (int it = 0; it < 2; ++it) {
-                            const int rr = (lane >> 2) + 16 * it, piece = lane & 3;
-                            const v4u v = *(const v4u*)(stage + rr * FC_STAGE_ROW + piece * 16);
-                            if (row0 + rr <= plast && ocb + piece * 16 < q.OC)
-                                *(v4u*)(q.dst + (size_t)(row0 + rr) * q.OC + ocb + piece * 16) = v;
-                        }
+                            for (int it = 0; it < 2; ++it) {
+                                const int rr = (lane >> 2) + 16 * it, piece = lane & 3;
+                                const v4u v = *(const v4u*)(stage + rr * FC_STAGE_ROW + piece * 16);
+                                if (row0 + rr <= plast && ocb + piece * 16 < q.OC)
+                                    *(v4u*)(q.dst + (size_t)(row0 + rr) * q.OC + ocb + piece * 16) = v;
+                            }
+                        });
                     });
-                });
-                continue;
+                    return;
+                }
             }
-        }
-        static_for<MT>([&](auto mic) {
-            static_for<NT>([&](auto nic) { emit_tile(mic, nic, cur_o[decltype(nic)::value]); });
-        });
+            static_for<MT>([&](auto mic) {
+                static_for<NT>([&](auto nic) { emit_tile(mic, nic, form, cur_o[decltype(nic)::value]); });
+            });
+        };
+        if constexpr (ACT == ACT_RT)
+            emit([&](int a0, int a1, int a2, int a3) __attribute__((always_inline)) {
+                auto one = [&](int v) __attribute__((always_inline)) { return requant_conv_rt(q.act, v, q.s_src, q.s_flt, q.s_dst); };
+                return pack4_perm(one(a0), one(a1), one(a2), one(a3));
+            });
+        else if constexpr (ONE_FORM)
+            requant_by_form<ACT>(q.rq, q.act, emit);
+        else
+            emit(0);
     }
 }
 
