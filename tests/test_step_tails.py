@@ -52,7 +52,10 @@ def test_layers_on_both_sides_of_the_staging_border(n, ic, ih, iw, oc, k, stride
     (36, 60, 28, 30, 36, 3, 2, "32,32,4"), (70, 60, 29, 30, 64, 3, 2, "32,32,2"), (130, 60, 29, 30, 64, 3, 2, "32,32,1"),
     (80, 20, 29, 30, 100, 3, 2, "64,32,2"), (80, 80, 29, 30, 100, 3, 2, "64,32,4"), (100, 68, 29, 30, 100, 3, 2, "64,32,2"),
     (28, 56, 41, 59, 16, 3, 1, "32,64,2"), (24, 40, 56, 55, 16, 5, 1, "32,64,4"),
-    (150, 20, 29, 30, 100, 3, 2, "64,64,1"), (150, 100, 29, 30, 100, 3, 2, "64,64,2")])
+    (150, 20, 29, 30, 100, 3, 2, "64,64,1"), (150, 100, 29, 30, 100, 3, 2, "64,64,2"),
+    # one tile a workgroup, its size by what its operands cost: from 25 steps on two channel tiles, from 80 on pixels too
+    (16, 60, 29, 30, 100, 3, 2, "32,32,4"), (16, 20, 29, 30, 100, 5, 2, "64,32,4"), (20, 256, 29, 30, 100, 3, 2, "64,32,4"),
+    (20, 260, 29, 30, 100, 3, 2, "64,64,4"), (40, 256, 29, 30, 28, 3, 2, "32,32,4"), (40, 260, 29, 30, 28, 3, 2, "32,64,4")])
 def test_groups_that_share_k(n, ic, ih, iw, oc, k, stride, kernel):
     port.set_threads(8)
     case = ConvCase(A.FMT_NCHW44, A.DENSE, n, ic, ih, iw, oc, k, stride, k // 2, A.RELU, scales=(0.02, 0.01, unsat(ic * k * k)))
