@@ -119,12 +119,12 @@ struct Model {
     hipStream_t tail_stream = nullptr;
     hipEvent_t ev_head = nullptr, ev_tail = nullptr;
     bool tail_pending = false, tail_reads_input = false;
+    HostStage* stage = nullptr;  // get_output's, where an output is small enough for it
     // The host's waits when the last forward had been launched (the library stream's: when it had been ordered behind that forward).
     // Where the host has waited since, by whichever call of the library - a blocking read, megcc_gfx950_wait() after a forward or
     // an asynchronous read -, nothing is left that the next forward's head could overlap, and on one stream it is over sooner, with
     // no event between head and tail (MobileNetV1, each forward waited for, us on two streams / one: batch 1 123 / 109, 4 139 /
     // 125, 8 145 / 129; with image in and result out, batch 1: 184 - 187 and unsteady / 171 - 173).
-    HostStage* stage = nullptr;  // get_output's, where an output is small enough for it
     HostWaits waits = {0, 0};
     int launched_tail = 0;  // entries of the last forward that went to the tail stream
     std::vector<char> waits_tail;
