@@ -176,7 +176,7 @@ def make_workload(name):
         return case, "qsi8 conv3x3 s1 p1 NCHW44 N=32 Cin=Cout=256 56x56 +bias +ReLU requant", "mfma"
     if name == "conv_cal":
         # The default scales (0.02 * 0.01 / 0.05 = 1 / 250) make every 125th accumulator an exact tie, the
-        # worst case for the requantisation (threshold table). Scales without ties, as a calibrated
+        # worst case for the requantisation (the reference's own sequence). Scales without ties, as a calibrated
         # network has them, requantise by one multiply-add; the output then also uses the whole range.
         return (headline_case(scales=(0.0213, 0.0097, 0.517)),
                 "qsi8 conv3x3 s1 p1 NCHW44 N=32 Cin=Cout=256 56x56 +bias +ReLU requant, scales without exact ties", "mfma")

@@ -578,7 +578,7 @@ const char* megcc_gfx950_last_error(void);
  * which kernel variant the calling thread's most recent operator call selected, as
  * "<kernel>[:n,n,...]" (e.g. "conv_mfma_i8_dma:3,128,512,1024" = variant, oc tile, pixel
  * sub-tile, patch slots); "+affine" at the end: the kernel requantised by the one fused multiply-add
- * the host proved exact for the layer's scales instead of the threshold table. The text lives until
+ * the host proved exact for the layer's scales instead of the reference's own sequence or the threshold table. The text lives until
  * the thread's next call of this function. */
 const char* megcc_gfx950_last_kernel(void);
 /* Diagnostics (no counterpart in the reference): the constants of the one-multiply-add
@@ -586,7 +586,7 @@ const char* megcc_gfx950_last_kernel(void);
  * out = clamp(floor(fma((float)acc, *c, *d)), activation's lowest output, 127) equals the
  * reference's fp32_to_int8(act(acc * s_src * s_flt / s_dst)) (BareMetal/Activation.cpp:47-56,
  * 105-114) for EVERY int32 accumulator. Returns 1 and the pair when the host search finds one
- * (IDENTITY / RELU only), else 0 - such layers requantise by threshold table. Host arithmetic only:
+ * (IDENTITY / RELU only), else 0 - such layers requantise by the reference's own sequence or by threshold table. Host arithmetic only:
  * needs no device. */
 int megcc_gfx950_requant_affine(int nonline_mode, float s_src, float s_flt, float s_dst, float* c, float* d);
 /* Kernel-selection overrides, for regression tests of kernels that un-switched shapes only reach

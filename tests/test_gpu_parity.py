@@ -184,7 +184,7 @@ LIVE = [
     ConvCase(A.FMT_NCHW44, A.DENSE, 5, 32, 31, 33, 36, 5, 1, 4, A.SIGMOID, scales=(0.02, 0.01, unsat(800) * 40), dilate=2),
     ConvCase(A.FMT_NCHW44, A.DENSE, 3, 8, 40, 300, 32, 5, 1, 2, A.IDENTITY, scales=(0.02, 0.01, unsat(200))),
     ConvCase(A.FMT_NCHW44, A.DENSE, 17, 32, 28, 28, 64, 5, 1, 0, A.RELU, scales=(0.02, 0.01, unsat(800))),
-    # H_SWISH through the threshold table in the pointwise kernels (streaming: 64 and 256 input
+    # H_SWISH (the reference's own sequence, its division as two multiply-adds) in the pointwise kernels (streaming: 64 and 256 input
     # channels; workgroup-shared: 512) and the plane-major 3x3 kernel
     ConvCase(A.FMT_NCHW44, A.DENSE, 3, 64, 28, 28, 128, 1, 1, 0, A.H_SWISH, scales=(0.02, 0.01, unsat(64))),
     ConvCase(A.FMT_NCHW44, A.DENSE, 2, 256, 14, 14, 64, 1, 1, 0, A.H_SWISH, scales=(0.02, 0.01, unsat(256))),
@@ -942,7 +942,7 @@ OLDER = [
     ("noxcdorder", MatMulCase(1030, 24, 1024, trans_a=True, trans_b=True)),
     ("noxcdorder", ConvCase(A.FMT_NCHW, A.DENSE, 2048, 128, 1, 1, 2040, 1, 1, 0, A.IDENTITY,
                             scales=(0.02, 0.01, unsat(128)))),
-    # the threshold table where the default is the one-multiply-add requantisation the host proved
+    # the reference's own sequence or the threshold table where the default is the multiply-add that the host proved
     # exact for the layer's scales (scales without exact ties; "+affine" in the kernel's name):
     # pointwise streaming and workgroup-shared kernels, depthwise on the matrix cores and by v_dot4,
     # the matrix-core first layer, the LDS-direct 3x3 kernel with 256- and 512-pixel sub-tiles
@@ -1110,7 +1110,7 @@ def _new_kernel_sweep():
     """seeded random layers for the pointwise kernel with any channel counts, the depthwise 5x5 / 7x7
     kernels and the dense 5x5 / 7x7 layers with one filter row per stage: random image sizes (rows
     that are no multiple of 4 or 8 pixels), strides, batches, channel counts, the three activations
-    that go through the threshold table and SIGMOID"""
+    whose outputs are a step function of the sum and SIGMOID"""
     r = np.random.Generator(np.random.PCG64(77))
     acts = [A.RELU, A.IDENTITY, A.H_SWISH, A.SIGMOID]
     out = []
@@ -1372,7 +1372,7 @@ def _chain_cases(n, c, ih, iw, stride, act, mode, bias):
     s_src, s_flt = 0.02, 0.01
     if n % 2 == 0:
         # scales without exact ties: IDENTITY / RELU then requantise by the proven multiply-add, the
-        # odd batches (0.02 * 0.01 / ...: ties at every 125th accumulator or so) by threshold table
+        # odd batches (0.02 * 0.01 / ...: ties at every 125th accumulator or so) by the reference's own sequence or the table
         s_src, s_flt, sc = 0.0213, 0.0097, sc * 1.0371
     dw = ConvCase(A.FMT_NCHW44, A.GROUP, n, c, ih, iw, c, 3, stride, 1, act, scales=(s_src, s_flt, sc), bias=bias)
     pool = PoolCase(A.FMT_NCHW44, A.POOL_MAX, n, c, dw.oh, dw.ow, 2, 2, 0, scale=sc)

@@ -91,8 +91,8 @@ def test_random_scales_either_have_an_exact_pair_or_none(act):
 
 def test_scales_with_exact_ties_on_both_sides_have_no_pair():
     """0.02 * 0.01 / 0.05: every 125th accumulator is an exact tie and the reference's three roundings
-    send some of them up and some down, which no single multiply-add reproduces: such layers keep the
-    threshold table. The other activations never get a pair."""
+    send some of them up and some down, which no single multiply-add reproduces: such layers run the
+    reference's own sequence or the threshold table. The other activations never get a pair."""
     assert runtime.requant_affine(abi.RELU, 0.02, 0.01, 0.05) is None
     assert runtime.requant_affine(abi.IDENTITY, 0.02, 0.01, 0.05) is None
     assert runtime.requant_affine(abi.H_SWISH, 0.0123, 0.0045, 0.0317) is None
