@@ -575,15 +575,18 @@ extern "C" TinyNNStatus megcc_gfx950_matmul(
     q.is_conv = 0;
     if (q.M == 0 || q.N == 0)
         return TinyNN_SUCCESS;
-    if (q.M <= 4 && q.K > 0 && !options().no_gevm) {  // the reference's gevm case: one pass over B
-        const GevmArgs v = {q.A, q.B, q.C, q.M, q.N, q.K, q.a_rs, q.a_cs, q.b_rs, q.b_cs, q.ldc};
-        if (gevm_f32_supported(v)) {
-            note_kernel("gevm_f32");
-            return gevm_f32_launch(v);
-        }
+    const GevmArgs ks = {q.A, q.B, q.C, q.M, q.N, q.K, q.a_rs, q.a_cs, q.b_rs, q.b_cs, q.ldc};
+    // the reference's gevm case: one pass over B
+#ifdef MG_HOST_AUDIT
+    const bool gevm = true;
+#else
+    const bool gevm = gevm_f32_wins(ks) || options().no_f32ks || !gemm_f32_ks_supported(ks);
+#endif
+    if (q.M <= 4 && !options().no_gevm && gevm_f32_supported(ks) && gevm) {
+        note_kernel("gevm_f32");
+        return gevm_f32_launch(ks);
     }
 #ifndef MG_HOST_AUDIT
-    const GevmArgs ks = {q.A, q.B, q.C, q.M, q.N, q.K, q.a_rs, q.a_cs, q.b_rs, q.b_cs, q.ldc};
     if (!options().no_f32split && gemm_f32_split_supported(ks))
         return gemm_f32_split_launch(ks, ta, tb);
     if (!options().no_f32ks && gemm_f32_ks_supported(ks))

@@ -13,6 +13,7 @@ struct GevmArgs {
 };
 
 bool gevm_f32_supported(const GevmArgs& q);
+bool gevm_f32_wins(const GevmArgs& q);
 TinyNNStatus gevm_f32_launch(const GevmArgs& q);
 
 }  // namespace mg

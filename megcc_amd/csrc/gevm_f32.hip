@@ -3,11 +3,18 @@
 // The layer is ONE pass over B, a few MB: what counts is that every byte of B is requested at
 // once - the whole matrix is smaller than the bandwidth-latency product of the chip - and that it
 // is one launch. No matrix cores (2 flops per 4 bytes of B).
-//   * B row-major [K,N] (not transposed): a workgroup owns 16 columns, a thread 4 of them (one
-//     16-byte load per row) and the rows k = kg, kg + 64, ...; the 64 partial sums of a column meet
-//     in LDS and are added in a fixed order.
-//   * B transposed [N,K]: a wave owns 4 rows of B (= 4 outputs), a lane 16-byte pieces of them
-//     along K; the lanes' partial sums meet by wavefront shuffles in a fixed order.
+//   * B row-major [K,N] (not transposed): a workgroup owns 16 columns, a lane 4 of them (one
+//     16-byte load per row) and every (16 W)-th row, W the waves of the workgroup: 4 to 16, so that all of a
+//     K up to 2048 is asked for at once. The partial sums of a column meet by shifts within 16 lanes and then in
+//     LDS, in a fixed order. Neighbouring workgroups, which share lines of 128 bytes, run on one XCD.
+//   * B transposed [N,K]: a wave owns 1 or 2 rows of B (= outputs), a lane 16-byte pieces of them
+//     along K, 8 in flight; the lanes' partial sums meet by shifts and wavefront shuffles in a fixed order.
+// A 16-byte load needs 4-byte alignment only. The last columns (the end of K) come from a load that begins up to three
+// places earlier; what another lane counts as well is dropped.
+// Measured (us, before - four waves a workgroup, 16-byte loads only where every row was aligned, a wave four rows - / now):
+// 1 x 1024 x 1000 3.75 / 3.6, 1 x 2346 x 311 12.6 / 4.2, 1 x 4000 x 1000 10.7 / 5.9, 1 x 4000 x 3530 27 / 11.5 (4.9 TB/s),
+// 4 x 544 x 311 6.2 / 4.0; B transposed 1 x 1024 x 1000 4.3 / 3.6, 1 x 2346 x 311 12.9 / 3.6, 1 x 4000 x 1000 8.6 / 4.9,
+// 3 x 544 x 1000 8.3 / 3.8, 4 x 4000 x 311 21.4 / 7.7.
 // The order of the additions differs from the reference's ascending k; f32 results are held to the
 // 1e-4 tolerance like the tiled GEMM, not to bit equality.
 #include "common.h"
@@ -16,177 +23,194 @@
 namespace mg {
 namespace {
 
-constexpr int GV_UNROLL = 8;  // rows (or 16-byte pieces) requested before the first one is used
+constexpr int GV_UNROLL = 8;  // 16-byte loads requested before the first one is used
 
-// B[k, n] at B + k * b_rs + n (rows contiguous). VEC: 16-byte loads are possible (base, row stride
-// and N allow it); otherwise the 4 columns are read one by one and checked against N.
-template <int M, bool VEC>
-__global__ void __launch_bounds__(256) gevm_f32_cols_kernel(GevmArgs q) {
-    __shared__ float red[64][M][17];
-    const int tid = threadIdx.x, cg = tid & 3, kg = tid >> 2;
-    const int n0 = blockIdx.x * 16 + cg * 4;
+typedef float gv_v4f __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ void gv_load(const float* p, float (&v)[4]) {
+    const gv_v4f t = *(const gv_v4f*)p;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        v[j] = t[j];
+}
+
+// lane i of every 16 gets what lane i + BY of them holds (0 beyond them)
+template <int BY>
+__device__ __forceinline__ float gv_shift(float v) {
+#ifdef MG_HOST_AUDIT
+    return v;
+#else
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 | BY, 0xf, 0xf, true));
+#endif
+}
+
+// B[k, n] at B + k * b_rs + n (rows contiguous), N >= 4; waves: up to 16
+template <int M>
+__global__ void __launch_bounds__(1024) gevm_f32_cols_kernel(GevmArgs q, int waves, int per_xcd) {
+    __shared__ float red[64][M][16];
+    const int tid = threadIdx.x, cg = tid & 3, kg = tid >> 2, rows = 16 * waves;
+    const int block = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    const int n0 = block * 16 + cg * 4;
+    if (block * 16 >= q.N)  // (the whole workgroup)
+        return;
+    const int first = min(n0, q.N - 4);
     float acc[M][4];
 #pragma unroll
     for (int m = 0; m < M; ++m)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             acc[m][j] = 0.f;
-    if (n0 < q.N) {
-        for (int k0 = kg; k0 < q.K; k0 += 64 * GV_UNROLL) {
-            // No load stands under a condition (the compiler would wait for every outstanding
-            // load at each join, one round trip per row): rows beyond K read row K - 1, columns
-            // beyond N column N - 1, and their products are replaced by 0.
-            float b[GV_UNROLL][4], a[GV_UNROLL][M];
+    for (int k0 = kg; k0 < q.K; k0 += rows * GV_UNROLL) {
+        // No load stands under a condition (the compiler would wait for every outstanding
+        // load at each join, one round trip per row): rows beyond K read row K - 1, and their products are replaced by 0.
+        float b[GV_UNROLL][4], a[GV_UNROLL][M];
 #pragma unroll
-            for (int u = 0; u < GV_UNROLL; ++u) {
-                const int k = min(k0 + u * 64, q.K - 1);
-                const float* p = q.B + (size_t)k * q.b_rs + n0;
-                if (VEC) {
-                    const float4 v = *(const float4*)p;
-                    b[u][0] = v.x; b[u][1] = v.y; b[u][2] = v.z; b[u][3] = v.w;
-                } else {
+        for (int u = 0; u < GV_UNROLL; ++u) {
+            const int k = min(k0 + u * rows, q.K - 1);
+            gv_load(q.B + (size_t)k * q.b_rs + first, b[u]);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        b[u][j] = p[min(j, q.N - 1 - n0)];
-                }
+            for (int m = 0; m < M; ++m)
+                a[u][m] = q.A[(size_t)m * q.a_rs + (size_t)k * q.a_cs];
+        }
 #pragma unroll
-                for (int m = 0; m < M; ++m)
-                    a[u][m] = q.A[(size_t)m * q.a_rs + (size_t)k * q.a_cs];
-            }
+        for (int u = 0; u < GV_UNROLL; ++u) {
+            const bool ok = k0 + u * rows < q.K;
 #pragma unroll
-            for (int u = 0; u < GV_UNROLL; ++u) {
-                const bool ok = k0 + u * 64 < q.K;
+            for (int m = 0; m < M; ++m)
 #pragma unroll
-                for (int m = 0; m < M; ++m)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[m][j] += ok ? a[u][m] * b[u][j] : 0.f;
-            }
+                for (int j = 0; j < 4; ++j)
+                    acc[m][j] += ok ? a[u][m] * b[u][j] : 0.f;
         }
     }
+    // the four of 16 lanes that hold a column, then (m, column) adds those of the workgroup in ascending order
 #pragma unroll
     for (int m = 0; m < M; ++m)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            red[kg][m][cg * 4 + j] = acc[m][j];
+        for (int j = 0; j < 4; ++j) {
+            float s = acc[m][j];
+            s += gv_shift<8>(s);
+            s += gv_shift<4>(s);
+            if ((tid & 15) < 4 && first + j >= n0)  // (the columns in front of n0 are another lane's, or another workgroup's)
+                red[tid >> 4][m][first + j - block * 16] = s;
+        }
     __syncthreads();
-    // thread (m, column) adds the 64 partial sums in ascending kg
     if (tid < M * 16) {
-        const int m = tid >> 4, c = tid & 15, n = blockIdx.x * 16 + c;
+        const int m = tid >> 4, c = tid & 15, n = block * 16 + c;
         if (n < q.N) {
             float s = 0.f;
-#pragma unroll 8
-            for (int g = 0; g < 64; ++g)
-                s += red[g][m][c];
+            for (int w = 0; w < 4 * waves; w += 4) {  // (four in flight)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    s += red[w + i][m][c];
+            }
             q.C[(size_t)m * q.ldc + n] = s;
         }
     }
 }
 
-// B[k, n] at B + n * b_cs + k (B stored transposed, rows of K contiguous)
-template <int M, bool VEC>
+// B[k, n] at B + n * b_cs + k (B stored transposed, rows of K contiguous), A's rows contiguous too, K >= 4
+template <int M, int R>
 __global__ void __launch_bounds__(256) gevm_f32_rows_kernel(GevmArgs q) {
+    constexpr int U = GV_UNROLL / R;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n0 = (blockIdx.x * 4 + wave) * 4;  // this wave's 4 outputs
+    const int n0 = (blockIdx.x * 4 + wave) * R;  // this wave's outputs
     if (n0 >= q.N)
         return;
-    float acc[M][4];
+    float acc[M][R];
 #pragma unroll
     for (int m = 0; m < M; ++m)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < R; ++r)
             acc[m][r] = 0.f;
-    for (int k0 = lane * 4; k0 < q.K; k0 += 256 * 2) {
-        // (no load under a condition, as above: rows beyond N read row N - 1, elements beyond K
-        //  element K - 1, and their products are replaced by 0)
-        float b[2][4][4], a[2][M][4];
+    for (int k0 = lane * 4; k0 < q.K; k0 += 256 * U) {
+        // (no load under a condition, as above: rows beyond N read row N - 1, pieces beyond K the last one)
+        float b[U][R][4], a[U][M][4];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int k = k0 + u * 256;
+        for (int u = 0; u < U; ++u) {
+            const int k = min(k0 + u * 256, q.K - 4);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float* row = q.B + (size_t)min(n0 + r, q.N - 1) * q.b_cs;
-                if (VEC) {  // K % 4 == 0: a piece is whole or beyond K
-                    const float4 v = *(const float4*)(row + min(k, q.K - 4));
-                    b[u][r][0] = v.x; b[u][r][1] = v.y; b[u][r][2] = v.z; b[u][r][3] = v.w;
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        b[u][r][j] = row[min(k + j, q.K - 1)];
-                }
-            }
+            for (int r = 0; r < R; ++r)
+                gv_load(q.B + (size_t)min(n0 + r, q.N - 1) * q.b_cs + k, b[u][r]);
 #pragma unroll
             for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    a[u][m][j] = q.A[(size_t)m * q.a_rs + (size_t)min(k + j, q.K - 1) * q.a_cs];
+                gv_load(q.A + (size_t)m * q.a_rs + k, a[u][m]);
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int k = k0 + u * 256;
+        for (int u = 0; u < U; ++u) {
+            const int own = k0 + u * 256 - min(k0 + u * 256, q.K - 4);  // (elements in front of it are another lane's)
 #pragma unroll
             for (int m = 0; m < M; ++m)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
+                for (int r = 0; r < R; ++r)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        acc[m][r] += k + j < q.K ? a[u][m][j] * b[u][r][j] : 0.f;
+                        acc[m][r] += j >= own ? a[u][m][j] * b[u][r][j] : 0.f;
         }
     }
 #pragma unroll
     for (int m = 0; m < M; ++m)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < R; ++r) {
             float s = acc[m][r];
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1)
-                s += __shfl_down(s, off, 64);
+            s += gv_shift<8>(s);
+            s += gv_shift<4>(s);
+            s += gv_shift<2>(s);
+            s += gv_shift<1>(s);
+            s += __shfl_down(s, 16, 64);
+            s += __shfl_down(s, 32, 64);
             if (lane == 0 && n0 + r < q.N)
                 q.C[(size_t)m * q.ldc + n0 + r] = s;
         }
 }
 
-template <bool VEC>
+template <int M>
 void launch_cols(const GevmArgs& q) {
-    const dim3 grid((q.N + 15) / 16);
-    switch (q.M) {
-        case 1: hipLaunchKernelGGL((gevm_f32_cols_kernel<1, VEC>), grid, dim3(256), 0, stream(), q); break;
-        case 2: hipLaunchKernelGGL((gevm_f32_cols_kernel<2, VEC>), grid, dim3(256), 0, stream(), q); break;
-        case 3: hipLaunchKernelGGL((gevm_f32_cols_kernel<3, VEC>), grid, dim3(256), 0, stream(), q); break;
-        default: hipLaunchKernelGGL((gevm_f32_cols_kernel<4, VEC>), grid, dim3(256), 0, stream(), q); break;
-    }
+    const int blocks = (q.N + 15) / 16, per_xcd = (blocks + 7) / 8;
+    // waves: K dealt evenly to the fewest rounds of 16 of them
+    const int per_wave = 16 * GV_UNROLL, rounds = (int)((q.K + 16L * per_wave - 1) / (16 * per_wave));
+    int waves = (int)((q.K + (long)rounds * per_wave - 1) / ((long)rounds * per_wave));
+    waves = waves < 4 ? 4 : waves;
+    hipLaunchKernelGGL((gevm_f32_cols_kernel<M>), dim3(8 * per_xcd), dim3(64 * waves), 0, stream(), q, waves, per_xcd);
 }
 
-template <bool VEC>
+template <int M>
 void launch_rows(const GevmArgs& q) {
-    const dim3 grid((q.N + 15) / 16);
-    switch (q.M) {
-        case 1: hipLaunchKernelGGL((gevm_f32_rows_kernel<1, VEC>), grid, dim3(256), 0, stream(), q); break;
-        case 2: hipLaunchKernelGGL((gevm_f32_rows_kernel<2, VEC>), grid, dim3(256), 0, stream(), q); break;
-        case 3: hipLaunchKernelGGL((gevm_f32_rows_kernel<3, VEC>), grid, dim3(256), 0, stream(), q); break;
-        default: hipLaunchKernelGGL((gevm_f32_rows_kernel<4, VEC>), grid, dim3(256), 0, stream(), q); break;
-    }
+    if (M == 1 && q.N <= 2048)
+        hipLaunchKernelGGL((gevm_f32_rows_kernel<M, 1>), dim3((q.N + 3) / 4), dim3(256), 0, stream(), q);
+    else
+        hipLaunchKernelGGL((gevm_f32_rows_kernel<M, 2>), dim3((q.N + 7) / 8), dim3(256), 0, stream(), q);
 }
 
 }  // namespace
 
+static bool by_columns(const GevmArgs& q) {
+    return q.b_cs == 1 && q.N >= 4;
+}
+
 bool gevm_f32_supported(const GevmArgs& q) {
-    return q.M >= 1 && q.M <= 4 && q.N >= 1 && q.K >= 1 && (q.b_cs == 1 || q.b_rs == 1);
+    return q.M >= 1 && q.M <= 4 && q.N >= 1 && q.K >= 1 && (by_columns(q) || (q.b_rs == 1 && q.K >= 4 && q.a_cs == 1));
+}
+
+// Against the matrix cores (gemm_f32_ks.hip), whose tiles have 16 rows whatever M is: they win where this kernel's loads of A,
+// M to one of B, are what a CU is busy with (us, here / there: 4 x 2346 x 311 7.0 / 5.9, 4 x 1024 x 311 4.2 / 4.1, 4 x 4000 x 1000
+// 9.2 / 10.6, 3 x 2346 x 1000 6.1 / 6.8; 3 x 1024 x 3530 4.9 / 4.4, 2 x 1024 x 3530 4.6 / 4.4, 3 x 203 x 3530 3.6 / 4.0; B transposed
+// 4 x 544 x 3530 4.7 / 4.2, 4 x 1024 x 3530 4.7 / 5.0, 4 x 544 x 1000 3.9 / 4.0, 3 x 544 x 3530 4.2 / 4.2).
+bool gevm_f32_wins(const GevmArgs& q) {
+    if (by_columns(q))
+        return !(q.M == 4 && q.K > 1536) && !(q.M >= 3 && q.N > 2048 && q.K > 512);
+    return !(q.M == 4 && q.N > 2048 && q.K < 1024);
 }
 
 TinyNNStatus gevm_f32_launch(const GevmArgs& q) {
-    const bool aligned = ((uintptr_t)q.B & 15) == 0;
-    if (q.b_cs == 1) {  // rows of B run along n
-        if (aligned && (q.b_rs & 3) == 0 && (q.N & 3) == 0)
-            launch_cols<true>(q);
-        else
-            launch_cols<false>(q);
-    } else {  // rows of B run along k
-        if (aligned && (q.b_cs & 3) == 0 && (q.K & 3) == 0)
-            launch_rows<true>(q);
-        else
-            launch_rows<false>(q);
+    const bool cols = by_columns(q);
+#define MG_GEVM(M_) (cols ? launch_cols<M_>(q) : launch_rows<M_>(q))
+    switch (q.M) {
+        case 1: MG_GEVM(1); break;
+        case 2: MG_GEVM(2); break;
+        case 3: MG_GEVM(3); break;
+        default: MG_GEVM(4); break;
     }
+#undef MG_GEVM
     return check_launch("gevm_f32");
 }
 
