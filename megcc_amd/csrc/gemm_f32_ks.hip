@@ -34,6 +34,8 @@
 
 namespace mg {
 
+bool conv_f32_small_supported(const ConvGeom& g);
+
 typedef float ks_v16f __attribute__((ext_vector_type(16)));
 typedef float ks_v4f __attribute__((ext_vector_type(4)));
 // the sums of an R x R tile and its product with K = 64 / R
@@ -536,11 +538,14 @@ TinyNNStatus gemm_f32_ks_launch(const GevmArgs& v, int ta, int tb) {
                : (tb ? ks_launch<KS_STRIDED, KS_CONTIG>(q, p, "gemm_f32_ks") : ks_launch<KS_STRIDED, KS_STRIDED>(q, p, "gemm_f32_ks"));
 }
 
+// Where the tiled kernel would be faster by ks_wins, conv_f32_small.hip stands in front of it for layers under 2^27 multiply-adds:
+// those run here (1x1 and 3x3 layers of many pixels and few channels; us, there / here: 13 x 12->34 100^2 1x1 37.6 / 19.0, 16 x
+// 10->99 79 x 77 1x1 80 / 25.7, 4 x 4->10 94^2 1x1 4.85 / 4.05; 7 x 82->121 89^2 1x1 - not under 2^27 - 35.3 here, 34.0 tiled).
 bool conv_f32_ks_supported(const ConvGeom& g) {
     const long P = (long)g.n * g.oh * g.ow, K = (long)g.ic * g.fh * g.fw;
     return g.fmt == MEGCC_FMT_NCHW && g.groups == 1 && g.fh * g.fw <= 31 && K >= 1 && K <= KS_MAX_CONV_K && P >= 1 &&
            P < (1L << 30) && (long)g.n * g.ic * g.ih * g.iw < (1L << 29) - 65536 && (long)g.oc * K < (1L << 29) - 65536 &&
-           P * g.oc < (1L << 31) && g.fh * g.fw >= 1 && ks_wins(g.oc, P, K, true, conv_plan(g));
+           P * g.oc < (1L << 31) && g.fh * g.fw >= 1 && (conv_f32_small_supported(g) || ks_wins(g.oc, P, K, true, conv_plan(g)));
 }
 
 TinyNNStatus conv_f32_ks_launch(const ConvGeom& g, const void* src, const void* flt, const void* bias, void* dst) {
