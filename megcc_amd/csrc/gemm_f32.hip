@@ -475,6 +475,20 @@ static void gemm_launch_reduce(const GemmArgs& q) {
         hipLaunchKernelGGL(gemm_f32_reduce_kernel<1>, dim3(blocks), dim3(256), 0, stream(), q);
 }
 
+#ifndef MG_HOST_AUDIT
+void gemm_f32_add_slices(const float* partial, int slices, int M, int N, float* C, long ldc) {
+    GemmArgs q = {};
+    q.partial = (float*)partial;
+    q.split = slices;
+    q.M = M;
+    q.N = N;
+    q.C = C;
+    q.ldc = ldc;
+    q.g.oh = q.g.ow = 1;
+    gemm_launch_reduce(q);
+}
+#endif
+
 bool conv_f32_gemm_supported(const ConvGeom& g) {
     long P = (long)g.n * g.oh * g.ow;
     return g.fmt == MEGCC_FMT_NCHW && g.groups == 1 && P < (1L << 31) &&
@@ -589,6 +603,8 @@ extern "C" TinyNNStatus megcc_gfx950_matmul(
 #ifndef MG_HOST_AUDIT
     if (!options().no_f32split && gemm_f32_split_supported(ks))
         return gemm_f32_split_launch(ks, ta, tb);
+    if (!options().no_f32split && !options().no_f32ks && gemm_f32_ks_split(ks, ta, tb, ws, &st))
+        return st;
     if (!options().no_f32ks && gemm_f32_ks_supported(ks))
         return gemm_f32_ks_launch(ks, ta, tb);
 #endif

@@ -13,4 +13,10 @@ TinyNNStatus gemm_f32_ks_launch(const GevmArgs& v, int ta, int tb);
 bool conv_f32_ks_supported(const ConvGeom& g);
 TinyNNStatus conv_f32_ks_launch(const ConvGeom& g, const void* src, const void* flt, const void* bias, void* dst);
 
+// 64 x 64 ... 256 tiles on the bf16 instructions, slices of K in the workspace where it has room for them (gemm_f32_ks_split.hip);
+// false: not where this product is faster
+bool gemm_f32_ks_split(const GevmArgs& v, int ta, int tb, const Workspace* ws, TinyNNStatus* status);
+// C = the sum of partial[slices][M][N], in order (gemm_f32.hip)
+void gemm_f32_add_slices(const float* partial, int slices, int M, int N, float* C, long ldc);
+
 }  // namespace mg

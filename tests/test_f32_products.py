@@ -61,3 +61,86 @@ def test_layers_of_many_pixels_and_few_channels(n, ic, h, w, oc, k):
     got, want = run(case, arrays), case.run_port(arrays)
     assert runtime.last_kernel().startswith("conv_f32_gemm_ks"), runtime.last_kernel()
     assert np.abs(got - want).max() <= 1e-4 * max(1.0, np.abs(want).max())
+
+
+def product64(case, arrays):
+    a, b = arrays["a"].astype(np.float64), arrays["b"].astype(np.float64)
+    return (a.T if case.trans_a else a) @ (b.T if case.trans_b else b)
+
+
+# products of middle size on the bf16 parts, a workgroup's waves sharing K: either operand staged, one wave, two and four to a
+# stage's K, with and without slices of K; K with and without a rest of a stage, rows and columns beyond whole tiles
+MIDDLE = [(512, 4096, 4096), (1912, 1206, 1078), (83, 2794, 3689), (947, 2247, 657), (1381, 2795, 925), (3713, 2717, 528), (320, 4095, 1100),
+          (2500, 1216, 400), (1290, 1088, 1290)]
+
+
+@pytest.mark.parametrize("m,k,n", MIDDLE)
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_products_of_middle_size(m, k, n, ta, tb):
+    case = MatMulCase(m, k, n, ta, tb)
+    arrays = case.gen(seed=71)
+    got, want = run(case, arrays), product64(case, arrays)
+    kernel = runtime.last_kernel()
+    print(kernel)
+    # each of the k products and sums is rounded once, in whatever order
+    bound = product64(case, {x: np.abs(v) for x, v in arrays.items()}) * (k * 2.0 ** -24)
+    assert np.all(np.abs(got - want) <= bound)
+    if kernel.startswith("gemm_f32_ks_split"):
+        runtime.set_option("nof32split", 1)
+        try:
+            in_f32 = run(case, arrays)
+            assert runtime.last_kernel().startswith("gemm_f32_ks:"), runtime.last_kernel()
+        finally:
+            runtime.set_option("nof32split", 0)
+        assert np.linalg.norm(got - want) <= np.linalg.norm(in_f32 - want)
+        # whole numbers whose sums fit 24 bits: no rounding is due
+        whole = {x: np.round(8 * v) for x, v in arrays.items()}
+        assert np.array_equal(run(case, whole), product64(case, whole))
+
+
+def test_products_of_middle_size_reach_every_form():
+    seen = set()
+    for m, k, n in MIDDLE:
+        case = MatMulCase(m, k, n, False, True)
+        run(case, case.gen(seed=72))
+        if runtime.last_kernel().startswith("gemm_f32_ks_split"):
+            tile, slices, swap = runtime.last_kernel().split(":")[1].split(",")[1:4]
+            seen |= {"tile " + tile, "swap " + swap, "sliced" if slices != "1" else "whole"}
+    assert seen == {"tile 64", "tile 128", "tile 256", "swap 0", "swap 1", "sliced", "whole"}, seen
+
+
+@pytest.mark.parametrize("m,k,n,tb", [(1912, 1206, 1078, False), (947, 2247, 657, True), (83, 2794, 3689, True), (512, 4096, 4096, False)])
+@pytest.mark.parametrize("value", [2.0 ** -120, 2.0 ** 70, np.inf, np.nan])
+def test_products_of_middle_size_that_meet_a_value_the_parts_cannot_hold(m, k, n, tb, value):
+    """one value at step `at` of K, of either operand: what its tile had summed before must neither be lost nor counted
+    twice, and an infinity must not have been in the bf16 product"""
+    case = MatMulCase(m, k, n, False, tb)
+    arrays = case.gen(seed=73)
+    for name in "ab":
+        arrays[name] = np.where(arrays[name] == 0, np.float32(1), arrays[name])
+    want0, mag0 = product64(case, arrays), product64(case, {x: np.abs(v) for x, v in arrays.items()})
+    a, b = arrays["a"], arrays["b"].T if tb else arrays["b"]
+    for at in (0, 63, 64, 255, 256, 511, 704, k // 2, k - 65, k - 1):
+        for side in "ab":
+            changed = dict(arrays)
+            changed[side] = arrays[side].copy()
+            row = 70
+            (changed["a"] if side == "a" else (changed["b"].T if tb else changed["b"]).T)[row, at] = value
+            got = run(case, changed)
+            assert runtime.last_kernel().startswith("gemm_f32_ks_split"), runtime.last_kernel()
+            want, mag = want0.copy(), mag0.copy()
+            with np.errstate(invalid="ignore"):
+                if side == "a":
+                    want[row] += (value - np.float64(a[row, at])) * b[at].astype(np.float64)
+                    mag[row] += abs(value) * np.abs(b[at])
+                    line = (row, slice(None))
+                else:
+                    want[:, row] += (value - np.float64(b[at, row])) * a[:, at].astype(np.float64)
+                    mag[:, row] += abs(value) * np.abs(a[:, at])
+                    line = (slice(None), row)
+                if not np.isfinite(value):
+                    assert np.array_equal(np.isnan(got[line]), np.isnan(want[line]))
+                    assert np.array_equal(got[line][np.isinf(want[line])], want[line][np.isinf(want[line])])
+                    got[line] = want[line] = mag[line] = 0
+            assert np.all(np.abs(got - want) <= mag * ((k + 2) * 2.0 ** -24)), (side, at)
