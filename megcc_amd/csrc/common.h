@@ -81,7 +81,7 @@ __device__ __forceinline__ void xcd_tile(XcdOrder o, int bx, int by, int gx, int
 // environment (MEGCC_NOPWS=1, ...) ONCE, when the library first consults them; later changes go
 // through megcc_gfx950_set_option(). Nothing on a launch path scans the environment.
 struct Options {
-    bool no_pws, no_gevm, no_fcb, no_small, no_pm768, no_pm, no_dma512, no_pm256, no_dma, no_fcs, no_pwshare, no_hybrid, no_dot4, no_f32small, dw_generic, no_dwmfma, no_dwnchw, no_fuse_softmax, no_graph, no_poolrows, no_firstmfma, no_rowsplit, no_fuse_chain, no_fuse_pwdw, fuse_pwdw, no_fcone, no_xcdorder, no_affine, no_pipeline, no_fuse_dwpw, fuse_dwpw, no_fuse_stem, fuse_stem, no_f32split, no_f32ks;
+    bool no_pws, no_gevm, no_fcb, no_small, no_pm768, no_pm, no_dma512, no_pm256, no_dma, no_fcs, no_pwshare, no_hybrid, no_dot4, no_f32small, dw_generic, no_dwmfma, no_dwnchw, no_fuse_softmax, no_graph, no_poolrows, no_firstmfma, no_rowsplit, no_fuse_chain, no_fuse_pwdw, fuse_pwdw, no_fcone, no_xcdorder, no_affine, no_pipeline, no_fuse_dwpw, fuse_dwpw, no_fuse_stem, fuse_stem, no_f32split, no_f32ks, no_fuse_blocks, fuse_blocks;
 };
 Options& options();
 
@@ -106,6 +106,12 @@ void dw_pw_block_destroy(DwPwBlock* block);
 enum class DwPw { CHECK, PREPARE, RUN };
 TinyNNStatus dw_pw_run(
         const MegccPwDwAttr* attr, Tensor** inputs, int nr_input, Tensor** outputs, int nr_output, DwPwBlock* block, DwPw what);
+// conv_blocks.hip: consecutive prepared pairs as one kernel, where it takes them (else NULL). What a launch needs is kept with it.
+struct BlocksRun;
+bool conv_blocks_takes(const Tensor& x);  // of these channels, rows and columns
+BlocksRun* conv_blocks_create(const DwPwBlock* const* blocks, int count);
+void conv_blocks_destroy(BlocksRun* run);
+TinyNNStatus conv_blocks_launch(const BlocksRun* run);
 // whether it could take the pair, before memory is planned and the pointwise filter packed
 bool dw_pw_takes(
         const MegccConvAttr* dw_attr, const MegccConvAttr* pw_attr, const Tensor* src, const Tensor* dw_flt, const Tensor* mid,

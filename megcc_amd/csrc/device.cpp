@@ -35,7 +35,7 @@ const OptionName kOptions[] = {
         {"nodot4", &Options::no_dot4},       {"nof32small", &Options::no_f32small},
         {"dw_generic", &Options::dw_generic}, {"no_graph", &Options::no_graph},
         {"nodwmfma", &Options::no_dwmfma},   {"nodwnchw", &Options::no_dwnchw},
-        {"nofusesoftmax", &Options::no_fuse_softmax}, {"nopoolrows", &Options::no_poolrows}, {"nofirstmfma", &Options::no_firstmfma}, {"norowsplit", &Options::no_rowsplit}, {"nofusechain", &Options::no_fuse_chain}, {"nofusepwdw", &Options::no_fuse_pwdw}, {"fusepwdw", &Options::fuse_pwdw}, {"nofcone", &Options::no_fcone}, {"noxcdorder", &Options::no_xcdorder}, {"noaffine", &Options::no_affine}, {"nopipeline", &Options::no_pipeline}, {"nofusedwpw", &Options::no_fuse_dwpw}, {"fusedwpw", &Options::fuse_dwpw}, {"nofusestem", &Options::no_fuse_stem}, {"fusestem", &Options::fuse_stem}, {"nof32split", &Options::no_f32split}, {"nof32ks", &Options::no_f32ks},
+        {"nofusesoftmax", &Options::no_fuse_softmax}, {"nopoolrows", &Options::no_poolrows}, {"nofirstmfma", &Options::no_firstmfma}, {"norowsplit", &Options::no_rowsplit}, {"nofusechain", &Options::no_fuse_chain}, {"nofusepwdw", &Options::no_fuse_pwdw}, {"fusepwdw", &Options::fuse_pwdw}, {"nofcone", &Options::no_fcone}, {"noxcdorder", &Options::no_xcdorder}, {"noaffine", &Options::no_affine}, {"nopipeline", &Options::no_pipeline}, {"nofusedwpw", &Options::no_fuse_dwpw}, {"fusedwpw", &Options::fuse_dwpw}, {"nofusestem", &Options::no_fuse_stem}, {"fusestem", &Options::fuse_stem}, {"nof32split", &Options::no_f32split}, {"nof32ks", &Options::no_f32ks}, {"nofuseblocks", &Options::no_fuse_blocks}, {"fuseblocks", &Options::fuse_blocks},
 };
 struct KernelNote {
     const char* name;

@@ -445,6 +445,28 @@ __device__ __forceinline__ void requant_by_form(const RequantPack& q, int act, F
     }
 }
 
+// The same for kernels whose sums started from requant_start(), RELU.
+template <typename F>
+__device__ __forceinline__ void requant_by_started_form(const RequantPack& q, F f) {
+    constexpr int RELU = MEGCC_NONLINE_RELU;
+    RequantPack p = q;
+    auto here = [&]() __attribute__((always_inline)) {
+#ifndef MG_HOST_AUDIT
+        asm volatile("" : "+s"(p.s1), "+s"(p.s2), "+s"(p.c), "+s"(p.d));  // (as in requant_dwords)
+#endif
+    };
+    if (q.mode == 5) {  // (uniform)
+        here();
+        f(RequantForm<5, RELU>{p, RELU});
+    } else if (q.mode == 2) {
+        here();
+        f(RequantForm<2, RELU>{p, RELU});
+    } else {
+        here();
+        f(RequantForm<3, RELU>{p, RELU});
+    }
+}
+
 // fp32_to_int8(sum * sdiv) (RELU: of max(sum, 0) * sdiv) of 4 N sums, QADD's and QFUSE_ADD_RELU's last step (elemwise.hip). RELU's
 // is never negative where sdiv is not, and the conversion above serves: 3 vector instructions a value for 6.
 template <bool RELU, int N>

@@ -57,9 +57,15 @@ struct ModelOpr {
     // the image's conversion, the first convolution and the pair behind it as one kernel; operator of that pair, -1: another kernel
     StemAttr stem;
     int stem_pair = -1;
+    // consecutive channel-wise + pointwise pairs as one kernel (NULL: another kernel), and the operators that begin them
+    BlocksRun* blocks = nullptr;
+    std::vector<int> pairs;
     ModelOpr() = default;
     ModelOpr(const ModelOpr&) = delete;
-    ~ModelOpr() { dw_pw_block_destroy(block); }
+    ~ModelOpr() {
+        dw_pw_block_destroy(block);
+        conv_blocks_destroy(blocks);
+    }
 };
 
 struct Model {
@@ -77,11 +83,14 @@ struct Model {
         bool known = false, faster = false;
         double gain_us = 0;
     };
-    std::vector<PairTime> dw_pw_time, pw_dw_time, stem_time;
+    std::vector<PairTime> dw_pw_time, pw_dw_time, stem_time, blocks_time;
     double schedule_us = 0;
     // per operator: the channel-wise -> pointwise pair that begins there may run as one kernel, so the memory plan keeps
     // the channel-wise layer's source until the pointwise layer is through
     std::vector<char> dw_pw_may;
+    // per operator: the last operator of the run of such pairs that begins there and may run as one kernel (conv_blocks.hip), which
+    // reads the first one's source while it writes the last one's result; -1: none
+    std::vector<int> blocks_may;
     void* arena = nullptr;
     size_t arena_bytes = 0;
     // one scratch buffer shared by all operators (they run one after the other on one stream),
@@ -217,6 +226,8 @@ bool plan_memory(Model* m) {
         // The same for a channel-wise layer in front of a pointwise one (conv_dw_pw.hip).
         if (i < m->dw_pw_may.size() && m->dw_pw_may[i])
             keep_until[root_of(m, o0->in[0])] = (int)i + 1;
+        if (i < m->blocks_may.size() && m->blocks_may[i] >= 0)
+            keep_until[root_of(m, o0->in[0])] = m->blocks_may[i];
         if (!options().no_fuse_pwdw && a.format == MEGCC_FMT_NCHW44 && a.sparse == MEGCC_SPARSE_DENSE && a.kernel_h == 1 && a.kernel_w == 1 &&
             a.stride_h == 1 && a.stride_w == 1 && a.pad_h == 0 && a.pad_w == 0 && b.format == MEGCC_FMT_NCHW44 &&
             b.sparse == MEGCC_SPARSE_GROUP && b.kernel_h == 3 && b.kernel_w == 3 && b.pad_h == 1 && b.pad_w == 1) {
@@ -285,9 +296,15 @@ static bool chain_only(const Model* m, const std::vector<int>& readers, int id, 
     return t->alias_of < 0 && !t->is_input && !t->is_output && !t->is_weight && readers[id] == nr;
 }
 
-// Fills dw_pw_may before the memory plan. Not under "nopipeline", which keeps the plan to the operators as they are.
+// of a pair's source and result
+static bool same_map(const Tensor& a, const Tensor& b) {
+    return a.layout.nr_dim == b.layout.nr_dim && std::equal(a.layout.dims, a.layout.dims + a.layout.nr_dim, b.layout.dims);
+}
+
+// Fills dw_pw_may and blocks_may before the memory plan. Not under "nopipeline", which keeps the plan to the operators as they are.
 static void find_dw_pw(Model* m) {
     m->dw_pw_may.assign(m->oprs.size(), 0);
+    m->blocks_may.assign(m->oprs.size(), -1);
     if (m->preplanned || options().no_fuse_dwpw || options().no_pipeline)
         return;
     const std::vector<int> readers = count_readers(m);
@@ -298,6 +315,23 @@ static void find_dw_pw(Model* m) {
             continue;
         m->dw_pw_may[i] = dw_pw_takes(&o0->desc.attr.conv, &o1->desc.attr.conv, &m->tensors[o0->in[0]]->t, &m->tensors[o0->in[1]]->t,
                                       &m->tensors[o0->out[0]]->t, &m->tensors[o1->in[1]]->t, &m->tensors[o1->out[0]]->t);
+    }
+    if (options().no_fuse_blocks)
+        return;
+    auto block = [&](size_t i) {
+        if (i + 1 >= m->oprs.size() || !m->dw_pw_may[i])
+            return false;
+        const Tensor &x = m->tensors[m->oprs[i]->in[0]]->t, &y = m->tensors[m->oprs[i + 1]->out[0]]->t;
+        return same_map(x, y) && conv_blocks_takes(x);
+    };
+    for (size_t i = 0; i < m->oprs.size(); ++i) {
+        size_t end = i;
+        while (block(end) && (end == i || (m->oprs[end]->in[0] == m->oprs[end - 1]->out[0] && chain_only(m, readers, m->oprs[end]->in[0], 1))))
+            end += 2;
+        if (end >= i + 4)
+            m->blocks_may[i] = (int)end - 1;
+        if (end > i)
+            i = end - 1;
     }
 }
 
@@ -324,6 +358,8 @@ static bool shares_bytes(const Tensor& a, const Tensor& b) {
 }
 // one entry of the schedule
 static TinyNNStatus call_opr(Model* m, ModelOpr* o) {
+    if (o->blocks)
+        return conv_blocks_launch(o->blocks);
     if (o->stem_pair >= 0)
         return stem_run(o->stem, o->in_ptrs.data(), (int)o->in_ptrs.size(), o->out_ptrs.data(), (int)o->out_ptrs.size(), true);
     if (o->dw_pw)
@@ -386,7 +422,7 @@ static bool faster_as_one(Model* m, std::vector<Model::PairTime>& times, int at,
 
 // Which pairs a schedule may contain (a pair that may not, or measured slower, stays two kernels).
 struct Pairs {
-    bool dw_pw, pw_dw;
+    bool dw_pw, pw_dw, blocks;
 };
 
 // The f32 image's conversion to qsi8 and the first convolution, the last two entries of the schedule, with the pair `pair` behind
@@ -439,6 +475,48 @@ static bool stem_taken(Model* m, const std::vector<int>& readers, ModelOpr* pair
     m->schedule.push_back(f);
     m->fused.push_back(f);
     return true;
+}
+
+// Runs of consecutive pairs in the schedule as one kernel each (conv_blocks.hip), where nothing else reads the tensors between them and
+// it measures faster than the pairs: a workgroup has an image for the whole run, so with few images most CUs have none.
+static void join_blocks(Model* m, const std::vector<int>& readers) {
+    if (options().no_fuse_blocks || (options().fuse_dwpw && !options().fuse_blocks))
+        return;
+    for (size_t i = 0; i < m->schedule.size(); ++i) {
+        size_t end = i;
+        while (end < m->schedule.size() && m->schedule[end]->dw_pw &&
+               same_map(*m->schedule[end]->in_ptrs[0], *m->schedule[end]->out_ptrs[0]) && conv_blocks_takes(*m->schedule[end]->in_ptrs[0]) &&
+               (end == i || (m->schedule[end]->in[0] == m->schedule[end - 1]->out[0] && chain_only(m, readers, m->schedule[end]->in[0], 1))))
+            ++end;
+        if (end < i + 2 || shares_bytes(*m->schedule[i]->in_ptrs[0], *m->schedule[end - 1]->out_ptrs[0]))
+            continue;
+        const std::vector<ModelOpr*> run(m->schedule.begin() + (long)i, m->schedule.begin() + (long)end);
+        std::vector<const DwPwBlock*> blocks;
+        ModelOpr* f = new ModelOpr();
+        f->first_index = run[0]->first_index;
+        memset(&f->desc, 0, sizeof(f->desc));
+        memset(&f->ws, 0, sizeof(f->ws));
+        f->symbol = "blocks of depthwise 3x3 + pointwise 1x1 (fused)";
+        for (const ModelOpr* o : run) {
+            blocks.push_back(o->block);
+            f->pairs.push_back(o->first_index);
+            for (size_t k = o == run[0] ? 0 : 1; k < o->in.size(); ++k) {
+                f->in.push_back(o->in[k]);
+                f->in_ptrs.push_back(o->in_ptrs[k]);
+            }
+        }
+        f->out = run.back()->out;
+        f->out_ptrs = run.back()->out_ptrs;
+        f->blocks = conv_blocks_create(blocks.data(), (int)blocks.size());
+        if (f->blocks && (options().fuse_blocks || faster_as_one(m, m->blocks_time, f->first_index, f, run))) {
+            m->fused.push_back(f);
+            m->schedule.erase(m->schedule.begin() + (long)i + 1, m->schedule.begin() + (long)end);
+            m->schedule[i] = f;
+        } else {
+            delete f;
+            i = end - 1;
+        }
+    }
 }
 
 static void build_schedule(Model* m, Pairs allow) {
@@ -666,6 +744,8 @@ static void build_schedule(Model* m, Pairs allow) {
         }
         m->schedule.push_back(o0);
     }
+    if (allow.blocks)
+        join_blocks(m, readers);
 }
 
 // The tail stream, its events and workspace, and which head entries must wait for the previous
@@ -877,11 +957,11 @@ struct Choice {
     int tail_begin;  // where the second stream takes over, -1: it does not
 };
 static Choice choose_schedule(Model* m) {
-    Pairs best = {true, true};
+    Pairs best = {true, true, true};
     build_schedule(m, best);
     setup_tail(m);
     int tail_begin = m->tail_begin;
-    bool dw_pw = false, pw_dw = false;
+    bool dw_pw = false, pw_dw = false, blocks = false;
     double gain = 0;
     for (const ModelOpr* o : m->schedule) {
         pw_dw = pw_dw || o->desc.kind == MEGCC_KERN_PW_DW;
@@ -889,12 +969,18 @@ static Choice choose_schedule(Model* m) {
         dw_pw = dw_pw || pair >= 0;
         if (pair >= 0 && (size_t)pair < m->dw_pw_time.size())
             gain += m->dw_pw_time[(size_t)pair].gain_us;
+        dw_pw = dw_pw || o->blocks;
+        blocks = blocks || o->blocks;
+        for (int p : o->pairs)
+            gain += (size_t)p < m->dw_pw_time.size() ? m->dw_pw_time[(size_t)p].gain_us : 0;
+        if (o->blocks && (size_t)o->first_index < m->blocks_time.size())
+            gain += m->blocks_time[(size_t)o->first_index].gain_us;
     }
     const bool doubt = dw_pw && gain < 0.1 * (m->schedule_us + gain);
     // (kernels of under 8 us: two-stream forwards still vary by a quarter from run to run, and one in three comparisons
     //  at batch 8 and 10 ended with no pairs, 135 us for 129)
-    if (tail_begin < 0 || m->schedule_us < 8.0 * (double)m->schedule.size() || (!doubt && !pw_dw) || options().fuse_dwpw ||
-        options().fuse_pwdw || options().fuse_stem)
+    if (tail_begin < 0 || m->schedule_us < 8.0 * (double)m->schedule.size() || (!doubt && !pw_dw && !blocks) || options().fuse_dwpw ||
+        options().fuse_pwdw || options().fuse_stem || options().fuse_blocks)
         return {best, tail_begin};
     // a forward with these pairs, at the boundary that balances the kernels' times
     auto time_pairs = [&](Pairs p) {
@@ -903,16 +989,32 @@ static Choice choose_schedule(Model* m) {
         setup_tail(m);
         return time_forwards(m, 1);
     };
-    const float first = time_forwards(m, 1);
+    float first = time_forwards(m, 1);
+    // A run of blocks has a CU an image, and what the others do beside it is the other stream's: only where whole forwards are faster
+    // by 2 % (us with MobileNetV1's five blocks as one kernel / without: batch 80 195 / 192, 96 203 / 199, 112 221 / 241, 128 235 / 257).
+    if (blocks) {
+        const Pairs without = {true, true, false};
+        const float as_pairs = time_pairs(without), with = std::min(first, time_pairs(best));
+        if (as_pairs > 0.f && !(with > 0.f && with < 0.98f * std::min(as_pairs, time_pairs(without)))) {
+            best = without;
+            reset_tail(m);
+            build_schedule(m, best);
+            setup_tail(m);
+            tail_begin = m->tail_begin;
+        }
+        first = time_pairs(best);
+        if (!pw_dw && !doubt)
+            return {best, tail_begin};
+    }
     float cost = first;
     Pairs winner = best;
     std::vector<Pairs> others;
     if (pw_dw)
-        others.push_back({true, false});
+        others.push_back({true, false, best.blocks});
     if (doubt)
-        others.push_back({false, true});  // (other pairs become possible without the channel-wise -> pointwise ones)
+        others.push_back({false, true, best.blocks});  // (other pairs become possible without the channel-wise -> pointwise ones)
     if (pw_dw && doubt)
-        others.push_back({false, false});
+        others.push_back({false, false, best.blocks});
     for (const Pairs& p : others) {
         const float t = time_pairs(p);
         if (t > 0.f && t < cost) {
@@ -1014,9 +1116,15 @@ static TinyNNStatus plan_again(Model* m, const Choice& chosen) {
         return TinyNN_SUCCESS;
     reset_tail(m);
     std::vector<char> one(m->oprs.size(), 0);
-    for (const ModelOpr* o : m->schedule)
+    m->blocks_may.assign(m->oprs.size(), -1);
+    for (const ModelOpr* o : m->schedule) {
         if (o->dw_pw || o->stem_pair >= 0)
             one[(size_t)(o->dw_pw ? o->first_index : o->stem_pair)] = 1;
+        for (int p : o->pairs)
+            one[(size_t)p] = 1;
+        if (o->blocks)
+            m->blocks_may[(size_t)o->first_index] = o->pairs.back() + 1;
+    }
     m->dw_pw_may = one;
     for (size_t i = 0; i < one.size(); ++i)
         if (one[i])
