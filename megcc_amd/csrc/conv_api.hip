@@ -585,6 +585,8 @@ static TinyNNStatus conv2d_run(
         nchw44_views(g.n, g.oc, g.oh, g.ow, &view, &dense);
         return strided_copy(dst_nchw, view, dst->ptr, dense, 4, "conv2d (f32 NCHW -> NCHW44)");
     }
+    if (f32 && !options().no_f32small && !options().no_f32ks && conv_f32_wide_supported(g))
+        return conv_f32_wide_launch(g, src->ptr, flt->ptr, b, dst->ptr);  // (notes its own variant)
     if (f32 && !options().no_f32small && !options().no_f32ks && conv_f32_ks_supported(g))
         return conv_f32_ks_launch(g, src->ptr, flt->ptr, b, dst->ptr);  // (notes its own variant)
     if (f32 && conv_f32_small_supported(g) && !options().no_f32small) {

@@ -16,15 +16,6 @@
 
 namespace mg {
 
-static __device__ __forceinline__ float f32_act(int act, float x) {
-    switch (act) {
-        case MEGCC_NONLINE_RELU: return act_apply<MEGCC_NONLINE_RELU>(x);
-        case MEGCC_NONLINE_H_SWISH: return act_apply<MEGCC_NONLINE_H_SWISH>(x);
-        case MEGCC_NONLINE_SIGMOID: return act_apply<MEGCC_NONLINE_SIGMOID>(x);
-        default: return x;
-    }
-}
-
 // ---- channel-wise ------------------------------------------------------------------------------
 // A workgroup makes DW_TH x DW_TW output pixels of one (image, channel group) plane. The input
 // pixels under them - ((DW_TH - 1) S + K) x ((DW_TW - 1) S + K) float4 - are staged in LDS with

@@ -513,4 +513,14 @@ __device__ __forceinline__ int sbyte(uint32_t w, int i) {
     return (int)(int8_t)(w >> (8 * i));
 }
 
+// an f32 layer's activation
+__device__ __forceinline__ float f32_act(int act, float x) {
+    switch (act) {
+        case MEGCC_NONLINE_RELU: return act_apply<MEGCC_NONLINE_RELU>(x);
+        case MEGCC_NONLINE_H_SWISH: return act_apply<MEGCC_NONLINE_H_SWISH>(x);
+        case MEGCC_NONLINE_SIGMOID: return act_apply<MEGCC_NONLINE_SIGMOID>(x);
+        default: return x;
+    }
+}
+
 }  // namespace mg

@@ -19,4 +19,8 @@ bool gemm_f32_ks_split(const GevmArgs& v, int ta, int tb, const Workspace* ws, T
 // C = the sum of partial[slices][M][N], in order (gemm_f32.hip)
 void gemm_f32_add_slices(const float* partial, int slices, int M, int N, float* C, long ldc);
 
+// f32 convolutions of many pixels: a wave has its pixels for the whole of K (conv_f32_wide.hip)
+bool conv_f32_wide_supported(const ConvGeom& g);
+TinyNNStatus conv_f32_wide_launch(const ConvGeom& g, const void* src, const void* flt, const void* bias, void* dst);
+
 }  // namespace mg

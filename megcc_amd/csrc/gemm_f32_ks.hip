@@ -85,15 +85,6 @@ __device__ __forceinline__ void ks_begin(const KsParams& q) {
 #endif
 }
 
-__device__ __forceinline__ float ks_act(int act, float x) {
-    switch (act) {
-        case MEGCC_NONLINE_RELU: return act_apply<MEGCC_NONLINE_RELU>(x);
-        case MEGCC_NONLINE_H_SWISH: return act_apply<MEGCC_NONLINE_H_SWISH>(x);
-        case MEGCC_NONLINE_SIGMOID: return act_apply<MEGCC_NONLINE_SIGMOID>(x);
-        default: return x;
-    }
-}
-
 static constexpr int KS_MAX_WAVES = 8;
 static constexpr int KS_MAX_CONV_K = 4096;  // table entries (8 bytes each)
 static constexpr int KS_SHORT = 28;         // steps of a short K: up to seven for each of four waves
@@ -380,7 +371,7 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
         if (m >= q.M || n >= q.N)
             continue;
         if (CONV) {
-            q.C[((size_t)img * q.M + m) * q.ohw + rem] = ks_act(q.act, v + (R == 16 ? bias : q.bias ? q.bias[m] : 0.f));
+            q.C[((size_t)img * q.M + m) * q.ohw + rem] = f32_act(q.act, v + (R == 16 ? bias : q.bias ? q.bias[m] : 0.f));
         } else {
             q.C[(size_t)m * q.ldc + n] = v;
         }

@@ -63,6 +63,52 @@ def test_layers_of_many_pixels_and_few_channels(n, ic, h, w, oc, k):
     assert np.abs(got - want).max() <= 1e-4 * max(1.0, np.abs(want).max())
 
 
+def convolution64(case, arrays, mag=False):
+    import torch
+    f = np.abs if mag else np.array
+    flt, src = (torch.from_numpy(f(arrays[x]).astype(np.float64)) for x in ("flt", "src"))
+    bias = torch.from_numpy(f(arrays["bias"]).astype(np.float64).reshape(-1)) if case.bias else None
+    return torch.nn.functional.conv2d(src, flt, bias, stride=(case.sh, case.sw), padding=(case.ph, case.pw)).numpy()
+
+
+# a wave has its pixels for the whole of K: tiles of 16, 32 and 64 channels, full and with one channel more or less; K of less
+# than a step, of whole steps and turns of four and with a rest; as few pixels as it takes, and waves without any; taps outside
+WIDE = [("32,32", 1, 17, 96, 96, 128, 1, 1), ("32,32", 2, 9, 31, 90, 113, 1, 1), ("32,32", 6, 8, 30, 71, 83, 3, 1), ("32,32", 13, 15, 81, 83, 83, 3, 1),
+        ("32,32", 4, 31, 64, 67, 67, 1, 1), ("32,32", 8, 12, 33, 41, 41, 3, 1), ("32,32", 4, 32, 32, 112, 112, 3, 1), ("32,32", 10, 86, 19, 63, 86, 1, 1), ("16,32", 7, 6, 12, 77, 77, 3, 1), ("16,32", 14, 45, 9, 91, 15, 3, 1),
+        ("16,32", 16, 3, 8, 112, 112, 3, 1), ("16,32", 9, 16, 16, 111, 111, 3, 2), ("16,32", 14, 51, 35, 95, 49, 1, 2), ("64,32", 8, 64, 64, 56, 56, 3, 1),
+        ("64,32", 7, 52, 121, 42, 42, 3, 1), ("64,32", 4, 25, 60, 79, 79, 5, 1)]
+
+
+@pytest.mark.parametrize("tile,n,ic,oc,h,w,k,stride", WIDE)
+@pytest.mark.parametrize("act,bias", [(A.RELU, True), (A.IDENTITY, False)])
+def test_layers_of_many_pixels(tile, n, ic, oc, h, w, k, stride, act, bias):
+    case = ConvCase(A.FMT_NCHW, A.DENSE, n, ic, h, w, oc, k, stride, k // 2, act, dtype="f32", bias=bias)
+    arrays = case.gen(seed=64)
+    got = run(case, arrays)
+    assert runtime.last_kernel().startswith("conv_f32_gemm_ks_wide"), runtime.last_kernel()
+    want = convolution64(case, arrays)
+    # each of the products and sums (and the bias's) is rounded once, in whatever order
+    bound = (ic * k * k + 2) * 2.0 ** -24 * convolution64(case, arrays, mag=True)
+    assert np.all(np.abs(got - (np.maximum(want, 0) if act == A.RELU else want)) <= bound)
+    # an Inf stays where it belongs: in a channel's filter (the last value, beside the next channel's), in a pixel
+    arrays["flt"][oc // 2, -1, -1, -1] = np.inf
+    assert np.isfinite(np.delete(run(case, arrays), oc // 2, axis=1)).all()
+    arrays = case.gen(seed=64)
+    arrays["src"][n - 1, ic - 1, h - 1, w - 1] = np.inf
+    got = run(case, arrays)
+    assert np.isfinite(got[:n - 1]).all() and np.isfinite(got[n - 1, :, :(h - k) // stride - 1]).all()
+
+
+def test_layers_of_many_pixels_reach_every_tile():
+    for tile, n, ic, oc, h, w, k, stride in WIDE:
+        case = ConvCase(A.FMT_NCHW, A.DENSE, n, ic, h, w, oc, k, stride, k // 2, A.SIGMOID, dtype="f32")
+        arrays = case.gen(seed=65)
+        got = run(case, arrays)
+        assert runtime.last_kernel() == "conv_f32_gemm_ks_wide:" + tile, runtime.last_kernel()
+        want = convolution64(case, arrays)
+        assert np.abs(got - 1 / (1 + np.exp(-want))).max() <= 1e-5
+
+
 def product64(case, arrays):
     a, b = arrays["a"].astype(np.float64), arrays["b"].astype(np.float64)
     return (a.T if case.trans_a else a) @ (b.T if case.trans_b else b)
