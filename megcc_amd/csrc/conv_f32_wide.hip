@@ -279,18 +279,20 @@ struct CwPlan {
 };
 
 // A workgroup puts one wave on each SIMD of a CU: its MFMAs (the matrix units are busy 0.7 - 0.8 of the time), 0.45 - 1 us for the
-// prologue and end of every set of 256 workgroups, 4 for launch and first operands. Rows of 16 cost a fifth more than rows of
-// 32, 64 a twentieth less. Estimated / measured us: 96 -> 11 77 x 77 N=9 in rows of 16, 32, 64 23 / 26, 36 / 40, 65 / 63; 15 -> 81 83 x 83 N=13 36 / 43, 30 / 35, 37 / 43;
-// 64 -> 64 112 x 112 N=16 166 / 188, 144 / 154, 149 / 151; 6 -> 104 76 x 79 1x1 N=6 9.4 / 7.8, 6.8 / 6.8, 7.4 / 7.5. (64 pixels a wave for 32: 64 ->
+// prologue and end of every set of 256 workgroups, 4 for launch and first operands; pixels that do not
+// follow one another cost the loads' way 1.8 times (108 -> 9 87 x 69 stride 2 N=11 23.3 / 23.7, 27 -> 38 86 x 86 stride 2 N=9 14.4 / 14.7). Rows of 16 cost a third more than rows of
+// 32, 64 a twentieth less. Estimated / measured us: 96 -> 11 77 x 77 N=9 in rows of 16, 32, 64 26 / 28, 36 / 40, 65 / 63; 15 -> 81 83 x 83 N=13 41 / 43, 30 / 35, 37 / 43;
+// 64 -> 64 112 x 112 N=16 188 / 188, 144 / 154, 149 / 151; 6 -> 104 76 x 79 1x1 N=6 7.5 / 7.8, 6.8 / 6.8, 7.4 / 7.5. (64 pixels a wave for 32: 64 ->
 // 64 162, 96 -> 11 49; 64 x 64 outputs 174, 74.)
 static CwPlan cw_plan(const ConvGeom& g) {
     static const CwPlan kPlans[] = {{32, 1, 1, 640, 0}, {32, 2, 1, 960, 0}, {16, 1, 2, 1152, 0}};
     const long N = (long)g.n * g.oh * g.ow, K = (long)g.ic * g.fh * g.fw;
     CwPlan best = {0, 0, 0, 0, 1e30};
+    const double each = g.sw > 1 && g.fw > 1 ? 1e-3 : 0.56e-3;
     for (CwPlan p : kPlans) {
         const long wgs = ((g.oc + p.r * p.mt - 1) / (p.r * p.mt)) * ((N + CW_WAVES * 32 - 1) / (CW_WAVES * 32));
         const double sets = (double)((wgs + num_cus() - 1) / num_cus());
-        p.us = 4.0 + sets * ((p.r == 16 ? 0.5 : p.mt == 1 ? 0.45 : 1.0) + 0.56e-3 * (double)K * (p.r == 16 ? 19.2 : p.mt == 1 ? 32.0 : 61.0));
+        p.us = 4.0 + sets * ((p.r == 16 ? 0.5 : p.mt == 1 ? 0.45 : 1.0) + each * (double)K * (p.r == 16 ? 22.0 : p.mt == 1 ? 32.0 : 61.0));
         if (K <= p.longest && p.us < best.us)
             best = p;
     }
@@ -300,15 +302,17 @@ static CwPlan cw_plan(const ConvGeom& g) {
 // Fewer pixels than this leave SIMDs without a wave, unless the waves of a workgroup share K (gemm_f32_ks.hip).
 static constexpr long CW_MIN_PIXELS = 12288;
 
-// What gemm_f32_ks.hip takes with 32 x 32 tiles, or the tiled kernel of gemm_f32.hip where that is the quicker one, in us. Here, there;
+// What gemm_f32_ks.hip takes, or the tiled kernel of gemm_f32.hip where that is the quicker one, in us. Here, there;
 // estimated / measured: 128 -> 128 56 x 56 N=16 165 / 165, 162 / 153 (stays there), 64 -> 64 112 x 112 N=16 144 / 154, 169 / 165; 24 -> 18 68 x 68
 // N=3 6.7 / 7.8, 6.4 / 5.6 (stays); 64 -> 64 56 x 56 N=8 24.6 / 26.5, 29 / 28; 7 -> 118 83 x 24 N=8 6.5 / 8.6, 10 / 13.0; 13 -> 11 82 x 82
-// stride 2 N=9 5.6 / 6.4, 5.4 / 5.4 (stays). The 0.93 where it is used: what both estimates are off by.
+// stride 2 N=9 7 / 6.4, 5.4 / 5.4 (stays). The 0.93 where it is used: what both estimates are off by.
 static double cw_others(const ConvGeom& g) {
     const long N = (long)g.n * g.oh * g.ow, K = (long)g.ic * g.fh * g.fw;
     const double tiles = (double)((((long)g.oc + 31) / 32 * ((N + 31) / 32) + num_cus() - 1) / num_cus());
     const long big = ((long)g.oc + 127) / 128 * ((N + 127) / 128), per_cu = (big + num_cus() - 1) / num_cus();
-    const double ks = tiles * (double)K * 11.8 + 1000.0 * (tiles + (tiles < 7.0 ? tiles : 7.0));
+    // (up to 16 channels and a long K: its 16 x 16 tiles)
+    const double ks = g.oc <= 16 && K >= 250 ? (double)(((N + 15) / 16 + num_cus() - 1) / num_cus()) * ((double)K * 6.2 + 1000.0)
+                                             : tiles * (double)K * 11.8 + 1000.0 * (tiles + (tiles < 7.0 ? tiles : 7.0) - 2.0);
     const double tiled = big < 192 ? 1e30 : (double)K * 128.0 * (per_cu == 1 ? 1.55 : 1.14 * (double)per_cu) * 1.7 + 16000.0 * (double)per_cu;
     return 2.5 + (ks < tiled ? ks : tiled) / 2330.0;
 }

@@ -418,6 +418,13 @@ static KsPlan ks_plan(long M, long N, long K, bool a_contig, bool b_contig, bool
     const bool one_row = ((M > 16 && M <= 32) || (N > 16 && N <= 32)) && K * (M > N ? M : N) > (1L << 22);
     if (small <= num_cus() || (small <= 2L * num_cus() && !one_row))
         best = {16, 1, 1, small <= num_cus() && K >= 16 * (KS_SHORT + 1) ? 8 : 4, (double)K * 4.75 * (small <= num_cus() ? 1.0 : 2.0) + 3000.0};
+    // A convolution of up to 16 channels and a long K in rows of 16 however many there are: half of a 32 x 32 tile's products are for
+    // channels that are not there (us, 32 x 32 / 16 x 16: 114 -> 11 46 x 57 stride 2 N=13 18.1 / 15.4, 95 -> 12 58 x 58 N=3 13.8 / 9.7, 33 -> 12
+    // 83 x 17 N=6 7.7 / 6.0, 32 -> 8 69 x 18 N=13 6.9 / 5.7, 30 -> 9 33 x 33 N=8 7.0 / 5.2; with eight waves 15.6, 11.4, 8.5, -, 7.6). Below, a tile's
+    // set-up is what counts (12 -> 11 57 x 108 N=2 4.6 / 5.2, 8 -> 14 41 x 84 N=5 4.6 / 6.5); from 17 channels on 32 x 32 is mostly the
+    // quicker one (19 -> 17 65 x 65 stride 2 N=6 4.9 / 6.9, 100 -> 37 34 x 34 N=7 14.5 / 16.0).
+    else if (conv && M <= 16 && K >= 250)
+        best = {16, 1, 1, 4, (double)((small + num_cus() - 1) / num_cus()) * ((double)K * 6.2 + 1000.0)};
     return best;
 }
 

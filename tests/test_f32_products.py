@@ -73,9 +73,9 @@ def convolution64(case, arrays, mag=False):
 
 # a wave has its pixels for the whole of K: tiles of 16, 32 and 64 channels, full and with one channel more or less; K of less
 # than a step, of whole steps and turns of four and with a rest; as few pixels as it takes, and waves without any; taps outside
-WIDE = [("32,32", 1, 17, 96, 96, 128, 1, 1), ("32,32", 2, 9, 31, 90, 113, 1, 1), ("32,32", 6, 8, 30, 71, 83, 3, 1), ("32,32", 13, 15, 81, 83, 83, 3, 1),
-        ("32,32", 4, 31, 64, 67, 67, 1, 1), ("32,32", 8, 12, 33, 41, 41, 3, 1), ("32,32", 4, 32, 32, 112, 112, 3, 1), ("32,32", 10, 86, 19, 63, 86, 1, 1), ("16,32", 7, 6, 12, 77, 77, 3, 1), ("16,32", 14, 45, 9, 91, 15, 3, 1),
-        ("16,32", 16, 3, 8, 112, 112, 3, 1), ("16,32", 9, 16, 16, 111, 111, 3, 2), ("16,32", 14, 51, 35, 95, 49, 1, 2), ("64,32", 8, 64, 64, 56, 56, 3, 1),
+WIDE = [("32,32", 1, 17, 96, 96, 128, 1, 1), ("32,32", 11, 18, 97, 68, 68, 1, 2), ("32,32", 11, 5, 22, 63, 63, 3, 1), ("32,32", 13, 15, 81, 83, 83, 3, 1),
+        ("32,32", 4, 31, 64, 67, 67, 1, 1), ("32,32", 8, 12, 33, 41, 41, 3, 1), ("32,32", 4, 32, 32, 112, 112, 3, 1), ("32,32", 10, 86, 19, 63, 86, 1, 1), ("16,32", 7, 6, 12, 77, 77, 3, 1), ("16,32", 16, 89, 15, 101, 16, 3, 1),
+        ("16,32", 16, 3, 8, 112, 112, 3, 1), ("16,32", 16, 3, 16, 112, 112, 3, 2), ("16,32", 14, 51, 35, 95, 49, 1, 2), ("64,32", 8, 64, 64, 56, 56, 3, 1),
         ("64,32", 7, 52, 121, 42, 42, 3, 1), ("64,32", 4, 25, 60, 79, 79, 5, 1)]
 
 
@@ -97,6 +97,17 @@ def test_layers_of_many_pixels(tile, n, ic, oc, h, w, k, stride, act, bias):
     arrays["src"][n - 1, ic - 1, h - 1, w - 1] = np.inf
     got = run(case, arrays)
     assert np.isfinite(got[:n - 1]).all() and np.isfinite(got[n - 1, :, :(h - k) // stride - 1]).all()
+
+
+# up to 16 channels and a long K on fewer pixels, or more than it takes: 16 x 16 tiles with four waves sharing K
+@pytest.mark.parametrize("n,ic,oc,h,w,k,stride", [(8, 28, 16, 33, 33, 3, 1), (3, 250, 16, 53, 52, 1, 1), (13, 114, 11, 46, 57, 3, 2), (3, 95, 1, 65, 65, 3, 1)])
+def test_layers_of_few_channels_and_a_long_k(n, ic, oc, h, w, k, stride):
+    case = ConvCase(A.FMT_NCHW, A.DENSE, n, ic, h, w, oc, k, stride, k // 2, A.IDENTITY, dtype="f32")
+    arrays = case.gen(seed=66)
+    got = run(case, arrays)
+    assert runtime.last_kernel().startswith("conv_f32_gemm_ks:16,16,4"), runtime.last_kernel()
+    bound = (ic * k * k + 2) * 2.0 ** -24 * convolution64(case, arrays, mag=True)
+    assert np.all(np.abs(got - convolution64(case, arrays)) <= bound)
 
 
 def test_layers_of_many_pixels_reach_every_tile():
