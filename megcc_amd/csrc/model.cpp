@@ -992,17 +992,20 @@ static Choice choose_schedule(Model* m) {
     float first = time_forwards(m, 1);
     // A run of blocks has a CU an image, and what the others do beside it is the other stream's: only where whole forwards are faster
     // by 2 % (us with MobileNetV1's five blocks as one kernel / without: batch 80 195 / 192, 96 203 / 199, 112 221 / 241, 128 235 / 257).
+    // (The first forwards were timed while the clocks went up: a lead of 5 % is then one, and is not asked for twice. Preparing MobileNetV1
+    // batch 256 133 ms with every comparison made twice, 115 so, 96 without runs.)
     if (blocks) {
         const Pairs without = {true, true, false};
-        const float as_pairs = time_pairs(without), with = std::min(first, time_pairs(best));
-        if (as_pairs > 0.f && !(with > 0.f && with < 0.98f * std::min(as_pairs, time_pairs(without)))) {
-            best = without;
-            reset_tail(m);
-            build_schedule(m, best);
-            setup_tail(m);
-            tail_begin = m->tail_begin;
+        const float as_pairs = time_pairs(without);
+        bool keep = as_pairs <= 0.f || (first > 0.f && first < 0.95f * as_pairs);
+        if (!keep) {
+            const float with = std::min(first, time_pairs(best));
+            keep = with > 0.f && with < 0.98f * as_pairs && with < 0.98f * time_pairs(without);
         }
+        if (!keep)
+            best = without;
         first = time_pairs(best);
+        tail_begin = m->tail_begin;
         if (!pw_dw && !doubt)
             return {best, tail_begin};
     }
