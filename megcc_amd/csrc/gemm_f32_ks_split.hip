@@ -26,6 +26,7 @@
 // Fp32MatMulM4N12.cpp:9-158 is the loop replaced.
 #include "common.h"
 #include "conv_mfma_i8.h"
+#include "f32_parts.h"
 #include "gemm_f32_ks.h"
 #include "gemm_f32_split.h"
 
@@ -35,7 +36,6 @@ typedef float kp_v16f __attribute__((ext_vector_type(16)));
 typedef float kp_v4f __attribute__((ext_vector_type(4)));
 typedef float kp_v2f __attribute__((ext_vector_type(2)));
 typedef unsigned kp_v4u __attribute__((ext_vector_type(4)));
-typedef unsigned short kp_v2s __attribute__((ext_vector_type(2)));
 typedef __bf16 kp_v2b __attribute__((ext_vector_type(2)));
 typedef __bf16 kp_v8b __attribute__((ext_vector_type(8)));
 
@@ -62,32 +62,25 @@ static constexpr int KP_L = 64, KP_K = 64, KP_STEP = 16;
 static constexpr int KP_PIECE = KP_L * 16 + 16;
 static constexpr int KP_STAGE = 24 * KP_PIECE;  // [part][octet of the 64 steps][row]
 static constexpr int KP_RING = 4;               // steps of R in flight
-static constexpr unsigned KP_LOW = 2 * (25u << 7) - 1;  // of 2^-102, as `least` is counted
-static constexpr float KP_HIGH = 0x1p60f;
 
-// Splits 8 values into three parts each. most: the largest magnitude (a NaN is none, and stays one in the parts), least: the
-// smallest of the upper 16 bits of twice the magnitude, less one (zero counts as the largest there).
+// Splits 8 values into three parts each, and looks at them.
 // `ones`: -1 in the lower half, in the upper half of a register: the rest behind a part is one v_dot2 (exact) instead of a
 // shift or a mask and a subtraction. (As constants the compiler gives the instruction its inline -1.0, whose lower half is 0.)
 struct KpSplit {
-    unsigned ones[2], two, minus;
-    float most;
-    kp_v2s least;
+    unsigned ones[2];
+    PartsRange range;
     __device__ __forceinline__ void begin() {
-        ones[0] = 0x0000bf80u, ones[1] = 0xbf800000u, two = 0x00020002u, minus = ~0u;
+        ones[0] = 0x0000bf80u, ones[1] = 0xbf800000u;
 #ifndef MG_HOST_AUDIT
-        asm volatile("" : "+v"(ones[0]), "+v"(ones[1]), "+v"(two), "+v"(minus));
+        asm volatile("" : "+v"(ones[0]), "+v"(ones[1]));
 #endif
-        most = 0.f;
-        least = 0xffff;
+        range.begin();
     }
     __device__ __forceinline__ void split(const float (&v)[8], kp_v4u (&part)[3]) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             kp_v2f x = {v[2 * i], v[2 * i + 1]};
-#ifndef MG_HOST_AUDIT
-            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(x[0]), "v"(x[1]));
-#endif
+            range.look(x[0], x[1]);
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
                 const kp_v2b b = __builtin_convertvector(x, kp_v2b);
@@ -97,14 +90,8 @@ struct KpSplit {
                     x[1] = __builtin_amdgcn_fdot2_f32_bf16(b, __builtin_bit_cast(kp_v2b, ones[1]), x[1], false);
                 }
             }
-            unsigned d = part[0][i];
-#ifndef MG_HOST_AUDIT
-            asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(d) : "v"(part[0][i]), "v"(two), "v"(minus));
-#endif
-            least = __builtin_elementwise_min(least, __builtin_bit_cast(kp_v2s, d));
         }
     }
-    __device__ __forceinline__ bool beyond() const { return most >= KP_HIGH || min(least[0], least[1]) < KP_LOW; }
 };
 
 // what a lane reads of an operand: 8 steps of K, an octet, of one row
@@ -245,7 +232,7 @@ __global__ void __launch_bounds__(512, 2) gemm_f32_ks_split_kernel(KpParams q) {
     // Whether a thread has met such a value: report(), a barrier, reported(). Every thread then reads the same, since
     // at least one more barrier (a stage's) lies in front of the next report().
     auto report = [&]() __attribute__((always_inline)) {
-        if (sp.beyond())
+        if (sp.range.beyond())
             beyond = 1;
     };
     auto reported = [&]() __attribute__((always_inline)) {

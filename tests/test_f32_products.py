@@ -201,3 +201,30 @@ def test_products_of_middle_size_that_meet_a_value_the_parts_cannot_hold(m, k, n
                     assert np.array_equal(got[line][np.isinf(want[line])], want[line][np.isinf(want[line])])
                     got[line] = want[line] = mag[line] = 0
             assert np.all(np.abs(got - want) <= mag * ((k + 2) * 2.0 ** -24)), (side, at)
+
+
+# (the last two: products of many tiles)
+@pytest.mark.parametrize("m,k,n,tb", [(1912, 1206, 1078, False), (947, 2247, 657, True), (83, 2794, 3689, True), (512, 4096, 4096, False)])
+@pytest.mark.parametrize("value", [2.0 ** -133, 2.0 ** -134, 2.0 ** -140, 2.0 ** -149])
+@pytest.mark.parametrize("side", ["a", "b"])
+def test_products_of_middle_size_of_values_below_every_bf16(m, k, n, tb, value, side):
+    """a row of them times values near 2^58 is made of ordinary numbers: none of them may go for a zero, and a zero is none of them"""
+    case = MatMulCase(m, k, n, False, tb)
+    check_tiny_values(case, "gemm_f32_ks_split", value, side)
+
+
+def check_tiny_values(case, kernel, value, side):
+    arrays = case.gen(seed=74)
+    rng = np.random.default_rng(75)
+    tiny, other = (arrays["a"], arrays["b"].T if case.trans_b else arrays["b"]) if side == "a" else \
+        ((arrays["b"].T if case.trans_b else arrays["b"]).T, arrays["a"].T)
+    row, at = 70, rng.choice(case.k, 9, replace=False)
+    other[:] = (other * 2.0 ** 57).astype(np.float32)
+    tiny[row] = 0
+    tiny[row, at] = (value * rng.choice([-1, 1], 9)).astype(np.float32)
+    got, want = run(case, arrays), product64(case, arrays)
+    assert runtime.last_kernel().startswith(kernel), runtime.last_kernel()
+    mag = product64(case, {x: np.abs(v) for x, v in arrays.items()})
+    line = (row, slice(None)) if side == "a" else (slice(None), row)
+    assert mag[line].min() > 2.0 ** -100
+    assert np.all(np.abs(got - want) <= mag * ((case.k + 1) * 2.0 ** -24))
