@@ -31,6 +31,7 @@
 // Fp32MatMulM4N12.cpp:9-158 is the loop replaced.
 #include "common.h"
 #include "conv_mfma_i8.h"
+#include "f32_parts.h"
 #include "gemm_f32_ks.h"
 #include "gemm_f32_split.h"
 
@@ -40,7 +41,6 @@ typedef float sp_v16f __attribute__((ext_vector_type(16)));
 typedef float sp_v4f __attribute__((ext_vector_type(4)));
 typedef float sp_v2f __attribute__((ext_vector_type(2)));
 typedef unsigned sp_v4u __attribute__((ext_vector_type(4)));
-typedef unsigned short sp_v2s __attribute__((ext_vector_type(2)));
 typedef __bf16 sp_v2b __attribute__((ext_vector_type(2)));
 typedef __bf16 sp_v8b __attribute__((ext_vector_type(8)));
 
@@ -62,7 +62,6 @@ static constexpr int SP_SHORT_K = 512;  // up to here the five small products ha
 // neighbouring threads write, on different banks
 static constexpr int SP_PIECE = SP_T * 16 + 64;
 static constexpr int SP_OPERAND = 6 * SP_PIECE;  // [part][half of the 16 steps][row]
-static constexpr unsigned SP_LOW = 25u << 7, SP_HIGH = 187u << 7;  // 2^-102, 2^60 as bf16
 
 // one operand's part of a thread: 8 steps of K of one row
 template <bool KFAST>
@@ -103,12 +102,13 @@ struct SplitSide {
             v[i] = k < K ? t : 0.f;
         }
     }
-    // splits the 8 values into LDS; most / least - 1: of the magnitudes' bits (zero counts as the largest there)
-    __device__ __forceinline__ void store(char* lds, const float (&v)[8], sp_v2s& most, sp_v2s& least) const {
+    // splits the 8 values into LDS
+    __device__ __forceinline__ void store(char* lds, const float (&v)[8], PartsRange& range) const {
         sp_v4u part[3];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             sp_v2f x = {v[2 * i], v[2 * i + 1]};
+            range.look(x[0], x[1]);
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
                 const unsigned b = __builtin_bit_cast(unsigned, __builtin_convertvector(x, sp_v2b));
@@ -116,9 +116,6 @@ struct SplitSide {
                 x[0] -= __uint_as_float(b << 16);
                 x[1] -= __uint_as_float(b & 0xffff0000u);
             }
-            const sp_v2s u = __builtin_bit_cast(sp_v2s, part[0][i] & 0x7fff7fffu);
-            most = __builtin_elementwise_max(most, u);
-            least = __builtin_elementwise_min(least, (sp_v2s)(u - (unsigned short)1));
         }
 #pragma unroll
         for (int p = 0; p < 3; ++p)
@@ -196,15 +193,16 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_split_kernel(SplitParams q) {
 #undef MG_SP_MUL
     };
     float va[8], vb[8];
-    sp_v2s most = 0, least = 0xffff;
+    PartsRange range;
+    range.begin();
     auto split = [&](int buf) __attribute__((always_inline)) {
-        sa.store(&lds[buf][0], va, most, least);
-        sb.store(&lds[buf][SP_OPERAND], vb, most, least);
+        sa.store(&lds[buf][0], va, range);
+        sb.store(&lds[buf][SP_OPERAND], vb, range);
     };
     // Whether a thread has met such a value: report(), a barrier, reported(). Every thread then reads the same, since
     // at least one more barrier (a stage's) lies in front of the next report().
     auto report = [&]() __attribute__((always_inline)) {
-        if (max(most[0], most[1]) >= SP_HIGH || min(least[0], least[1]) < SP_LOW - 1)
+        if (range.beyond())
             beyond = 1;
     };
     auto reported = [&]() __attribute__((always_inline)) {

@@ -99,6 +99,12 @@ inline float __uint_as_float(unsigned u) {
     return f;
 }
 
+inline unsigned __float_as_uint(float f) {
+    unsigned u;
+    memcpy(&u, &f, 4);
+    return u;
+}
+
 inline void __syncthreads() {}
 template <typename T>
 inline T __shfl_down(T v, int, int = 64) { return v; }

@@ -203,7 +203,6 @@ def test_products_of_middle_size_that_meet_a_value_the_parts_cannot_hold(m, k, n
             assert np.all(np.abs(got - want) <= mag * ((k + 2) * 2.0 ** -24)), (side, at)
 
 
-# (the last two: products of many tiles)
 @pytest.mark.parametrize("m,k,n,tb", [(1912, 1206, 1078, False), (947, 2247, 657, True), (83, 2794, 3689, True), (512, 4096, 4096, False)])
 @pytest.mark.parametrize("value", [2.0 ** -133, 2.0 ** -134, 2.0 ** -140, 2.0 ** -149])
 @pytest.mark.parametrize("side", ["a", "b"])
@@ -216,8 +215,8 @@ def test_products_of_middle_size_of_values_below_every_bf16(m, k, n, tb, value, 
 def check_tiny_values(case, kernel, value, side):
     arrays = case.gen(seed=74)
     rng = np.random.default_rng(75)
-    tiny, other = (arrays["a"], arrays["b"].T if case.trans_b else arrays["b"]) if side == "a" else \
-        ((arrays["b"].T if case.trans_b else arrays["b"]).T, arrays["a"].T)
+    a, b = arrays["a"].T if case.trans_a else arrays["a"], arrays["b"].T if case.trans_b else arrays["b"]
+    tiny, other = (a, b) if side == "a" else (b.T, a.T)  # (views)
     row, at = 70, rng.choice(case.k, 9, replace=False)
     other[:] = (other * 2.0 ** 57).astype(np.float32)
     tiny[row] = 0
@@ -228,3 +227,10 @@ def check_tiny_values(case, kernel, value, side):
     line = (row, slice(None)) if side == "a" else (slice(None), row)
     assert mag[line].min() > 2.0 ** -100
     assert np.all(np.abs(got - want) <= mag * ((case.k + 1) * 2.0 ** -24))
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb", [(2040, 512, 1999, False, False), (1930, 531, 1925, True, True), (2900, 145, 3001, False, True)])
+@pytest.mark.parametrize("value", [2.0 ** -133, 2.0 ** -134, 2.0 ** -149])
+@pytest.mark.parametrize("side", ["a", "b"])
+def test_products_of_many_tiles_of_values_below_every_bf16(m, k, n, ta, tb, value, side):
+    check_tiny_values(MatMulCase(m, k, n, ta, tb), "gemm_f32_split", value, side)
