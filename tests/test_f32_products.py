@@ -40,6 +40,23 @@ def test_few_rows(m, k, n, ta, tb):
     check_product(MatMulCase(m, k, n, ta, tb), 61)
 
 
+# either side of every line between the kernel for few rows and the matrix cores, and the shapes whose times the lines follow from
+GEVM, KS = "gevm_f32", "gemm_f32_ks:"
+
+
+@pytest.mark.parametrize("m,k,n,tb,own", [
+    (4, 1024, 1000, False, GEVM), (4, 1025, 1000, False, KS), (4, 1100, 1000, False, KS), (4, 2346, 311, False, KS), (4, 4096, 1300, False, KS),
+    (4, 2799, 650, False, KS), (4, 2800, 650, False, GEVM), (4, 4000, 576, False, KS), (4, 4000, 577, False, GEVM), (4, 4000, 1000, False, GEVM),
+    (4, 4000, 1008, False, GEVM), (4, 4000, 1009, False, KS), (3, 1024, 3530, False, GEVM), (3, 1025, 2048, False, GEVM), (3, 1025, 2049, False, KS),
+    (3, 2560, 1281, False, GEVM), (3, 2561, 1281, False, KS), (3, 4096, 1280, False, GEVM), (3, 4096, 1300, False, KS), (2, 4000, 1400, False, GEVM),
+    (4, 544, 3530, True, GEVM), (4, 1024, 3530, True, GEVM), (4, 4000, 311, True, GEVM), (3, 4096, 4096, True, GEVM)])
+def test_which_kernel_few_rows_run_on(m, k, n, tb, own):
+    case = MatMulCase(m, k, n, False, tb)
+    check_product(case, 67, own)
+    if own == GEVM:
+        assert runtime.last_kernel() == GEVM
+
+
 def test_few_rows_of_values_that_are_not_finite():
     """a row or column beyond the operands (the clamped loads repeat the last one) leaves no trace, an Inf inside does"""
     case = MatMulCase(2, 515, 18)
