@@ -394,7 +394,7 @@ __global__ void __launch_bounds__(512, 2) gemm_f32_ks_split_kernel(KpParams q) {
 // ---- choice ---------------------------------------------------------------------------------------------
 struct KpPlan {
     int kg, slices;
-    bool swap;
+    bool swap;  // (with four groups of waves both operands have 64 rows: never)
 };
 
 // Estimated cycles of the busiest CU, on the scale of gemm_f32_ks.hip (2.33 GHz): 16 steps of K of the 8 waves of a workgroup, one a
@@ -422,7 +422,7 @@ static bool kp_plan(const GevmArgs& v, size_t room, KpPlan* plan) {
     plan->kg = 0;
     const long most = (long)(room / ((size_t)M * N * 4));
     for (int kg = 1; kg <= 4; kg *= 2)
-        for (int swap = 0; swap < 2; ++swap)
+        for (int swap = 0; swap < (kg == 4 ? 1 : 2); ++swap)
             for (int s = 1; s == 1 || (s <= 16 && s <= most && s * 128L <= K); ++s) {
                 const double cost = kp_cost(M, N, K, kg, s, swap != 0);
                 if (cost < best) {
@@ -451,7 +451,7 @@ static TinyNNStatus kp_launch(KpParams& q, const KpPlan& p, const Workspace* ws)
     if (q.sliced)
         q.C = (float*)ws->ptr;
     note_kernel("gemm_f32_ks_split", KP_L, wide, slices, SWAP);
-    void (*kern)(KpParams) = p.kg == 1 ? gemm_f32_ks_split_kernel<LM, RM, 1, SWAP> : p.kg == 2 ? gemm_f32_ks_split_kernel<LM, RM, 2, SWAP> : gemm_f32_ks_split_kernel<LM, RM, 4, SWAP>;
+    void (*kern)(KpParams) = p.kg == 1 ? gemm_f32_ks_split_kernel<LM, RM, 1, SWAP> : p.kg == 2 ? gemm_f32_ks_split_kernel<LM, RM, 2, SWAP> : gemm_f32_ks_split_kernel<LM, RM, 4, false>;
     hipLaunchKernelGGL(kern, dim3(8 * q.per_xcd), dim3(512), 0, stream(), q);
     if (q.sliced)
         gemm_f32_add_slices(q.C, slices, q.M, q.N, C, q.ldc);
