@@ -360,7 +360,7 @@ TinyNNStatus conv_f32_wide_launch(const ConvGeom& g, const void* src, const void
     const bool tail = q.K % ks != 0;
     void (*const kern)(CwParams) = p.r == 16 ? cw_kernel<16, 1, 2>(gather, tail) : p.mt == 1 ? cw_kernel<32, 1, 1>(gather, tail) : cw_kernel<32, 2, 1>(gather, tail);
     const size_t lds = (gather ? (size_t)(q.K + ks - 1) / ks * ks * 8 : 0) + (size_t)p.r * p.mt * 4;
-    note_kernel("conv_f32_gemm_ks_wide", p.r * p.mt, p.r * p.nt);
+    note_kernel("conv_f32_wide", p.r * p.mt, p.r * p.nt);
     hipLaunchKernelGGL(kern, dim3((unsigned)(8 * q.per_xcd)), dim3(CW_THREADS), lds, stream(), q);
     return check_launch("conv_f32_wide");
 }

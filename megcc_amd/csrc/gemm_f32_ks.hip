@@ -537,8 +537,8 @@ TinyNNStatus gemm_f32_ks_launch(const GevmArgs& v, int ta, int tb) {
 }
 
 // Where the tiled kernel would be faster by ks_wins, conv_f32_small.hip stands in front of it for layers under 2^27 multiply-adds:
-// those run here (1x1 and 3x3 layers of many pixels and few channels; us, there / here: 13 x 12->34 100^2 1x1 37.6 / 19.0, 16 x
-// 10->99 79 x 77 1x1 80 / 25.7, 4 x 4->10 94^2 1x1 4.85 / 4.05; 7 x 82->121 89^2 1x1 - not under 2^27 - 35.3 here, 34.0 tiled).
+// those run here. Few are left of them behind conv_f32_wide.hip, 50 of 200000 drawn layers under 2^27 (us, there / here: 9 x 1->23 62 x 44 3x3 9.4 /
+// 4.5, 8 x 10->183 9 x 169 1x1 20.9 / 9.3, 3 x 2->188 240 x 17 3x3 37.3 / 10.7, 5 x 7->9 63 x 78 1x1 4.2 / 3.7, 2 x 7->2 240 x 204 1x1 stride 2 3.4 / 3.5).
 bool conv_f32_ks_supported(const ConvGeom& g) {
     const long P = (long)g.n * g.oh * g.ow, K = (long)g.ic * g.fh * g.fw;
     return g.fmt == MEGCC_FMT_NCHW && g.groups == 1 && g.fh * g.fw <= 31 && K >= 1 && K <= KS_MAX_CONV_K && P >= 1 &&

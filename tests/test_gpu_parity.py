@@ -422,8 +422,12 @@ F32_SHARED_K = [
 def test_f32_products_whose_waves_share_k(case):
     port.set_threads(8)
     arrays = case.gen(seed=19)
-    got = run_gpu(case, arrays)
-    assert "gemm_ks" in runtime.last_kernel() or runtime.last_kernel().startswith("gemm_f32_ks"), runtime.last_kernel()
+    runtime.set_option("nof32split", 1)  # (the products of middle size among them)
+    try:
+        got = run_gpu(case, arrays)
+    finally:
+        runtime.set_option("nof32split", 0)
+    assert runtime.last_kernel().startswith(("conv_f32_gemm_ks:", "gemm_f32_ks:")), runtime.last_kernel()
     compare(got, case.run_port(arrays), repr(case))
 
 

@@ -95,7 +95,7 @@ def test_f32_products_of_few_tiles(m, k, n, ta, tb):
     case = MatMulCase(m, k, n, trans_a=ta, trans_b=tb)
     arrays = case.gen(seed=43)
     got = run_gpu(case, arrays)
-    assert runtime.last_kernel().startswith("gemm_f32_ks"), runtime.last_kernel()
+    assert runtime.last_kernel().startswith("gemm_f32_ks:"), runtime.last_kernel()
     # each of the k products and sums is rounded once, in whatever order
     bound = _product(case, {x: np.abs(v) for x, v in arrays.items()}) * (k * 2.0 ** -24)
     assert np.all(np.abs(got - _product(case, arrays)) <= bound)
