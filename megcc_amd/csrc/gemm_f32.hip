@@ -475,7 +475,6 @@ static void gemm_launch_reduce(const GemmArgs& q) {
         hipLaunchKernelGGL(gemm_f32_reduce_kernel<1>, dim3(blocks), dim3(256), 0, stream(), q);
 }
 
-#ifndef MG_HOST_AUDIT
 void gemm_f32_add_slices(const float* partial, int slices, int M, int N, float* C, long ldc) {
     GemmArgs q = {};
     q.partial = (float*)partial;
@@ -487,7 +486,6 @@ void gemm_f32_add_slices(const float* partial, int slices, int M, int N, float* 
     q.g.oh = q.g.ow = 1;
     gemm_launch_reduce(q);
 }
-#endif
 
 bool conv_f32_gemm_supported(const ConvGeom& g) {
     long P = (long)g.n * g.oh * g.ow;

@@ -392,11 +392,6 @@ __global__ void __launch_bounds__(512, 2) gemm_f32_ks_split_kernel(KpParams q) {
 }
 
 // ---- choice ---------------------------------------------------------------------------------------------
-struct KpPlan {
-    int kg, slices;
-    bool swap;  // (with four groups of waves both operands have 64 rows: never)
-};
-
 // Estimated cycles of the busiest CU, on the scale of gemm_f32_ks.hip (2.33 GHz): 16 steps of K of the 8 waves of a workgroup, one a
 // CU, 2250 (2100 with two groups of waves, 1720 where every wave has its own rows of R: L is split less often), 4500 for the
 // first operands and the end of each and 4000 for a rest of K; for slices of K a second launch and their way out and back in at 5
@@ -433,6 +428,10 @@ static bool kp_plan(const GevmArgs& v, size_t room, KpPlan* plan) {
     return plan->kg != 0;
 }
 
+static long side_bytes(long rows, long row, long steps, long k) {
+    return 4 * ((rows - 1) * row + (steps - 1) * k + 1);
+}
+
 template <int LM, int RM, bool SWAP>
 static TinyNNStatus kp_launch(KpParams& q, const KpPlan& p, const Workspace* ws) {
     const int wide = 256 / p.kg;
@@ -458,17 +457,10 @@ static TinyNNStatus kp_launch(KpParams& q, const KpPlan& p, const Workspace* ws)
     return check_launch("gemm_f32_ks_split");
 }
 
-bool gemm_f32_ks_split(const GevmArgs& v, int ta, int tb, const Workspace* ws, TinyNNStatus* status) {
-    const long limit = (1L << 31) - 65536;
-    const long as = 4 * ((long)(v.M - 1) * v.a_rs + (long)(v.K - 1) * v.a_cs + 1);
-    const long bs = 4 * ((long)(v.K - 1) * v.b_rs + (long)(v.N - 1) * v.b_cs + 1);
-    KpPlan p;
-    if ((double)v.M * v.N * v.K < 4e8 || v.K < KP_K || as >= limit || bs >= limit || !(v.a_cs == 1 || v.a_rs == 1) || !(v.b_cs == 1 || v.b_rs == 1) ||
-        (long)v.M * v.N >= (1L << 31) || !kp_plan(v, ws && ws->ptr && ((uintptr_t)ws->ptr & 3) == 0 ? ws->size : 0, &p))
-        return false;
+TinyNNStatus gemm_f32_ks_split_launch(const GevmArgs& v, int ta, int tb, const KpPlan& p, const Workspace* ws) {
     KpParams q = {};
-    const KpSide a = {v.A, (unsigned)as, (unsigned)v.a_rs * 4u, (unsigned)v.a_cs * 4u, v.M};
-    const KpSide b = {v.B, (unsigned)bs, (unsigned)v.b_cs * 4u, (unsigned)v.b_rs * 4u, v.N};
+    const KpSide a = {v.A, (unsigned)side_bytes(v.M, v.a_rs, v.K, v.a_cs), (unsigned)v.a_rs * 4u, (unsigned)v.a_cs * 4u, v.M};
+    const KpSide b = {v.B, (unsigned)side_bytes(v.N, v.b_cs, v.K, v.b_rs), (unsigned)v.b_cs * 4u, (unsigned)v.b_rs * 4u, v.N};
     q.C = v.C;
     q.M = v.M;
     q.N = v.N;
@@ -478,8 +470,18 @@ bool gemm_f32_ks_split(const GevmArgs& v, int ta, int tb, const Workspace* ws, T
     q.r = p.swap ? a : b;
     const bool lk = p.swap ? tb : !ta, rk = p.swap ? !ta : tb;  // contiguous along K
 #define MG_KP(L_, R_) (p.swap ? kp_launch<L_, R_, true>(q, p, ws) : kp_launch<L_, R_, false>(q, p, ws))
-    *status = lk ? (rk ? MG_KP(KP_CONTIG, KP_CONTIG) : MG_KP(KP_CONTIG, KP_STRIDED)) : (rk ? MG_KP(KP_STRIDED, KP_CONTIG) : MG_KP(KP_STRIDED, KP_STRIDED));
+    return lk ? (rk ? MG_KP(KP_CONTIG, KP_CONTIG) : MG_KP(KP_CONTIG, KP_STRIDED)) : (rk ? MG_KP(KP_STRIDED, KP_CONTIG) : MG_KP(KP_STRIDED, KP_STRIDED));
 #undef MG_KP
+}
+
+bool gemm_f32_ks_split(const GevmArgs& v, int ta, int tb, const Workspace* ws, TinyNNStatus* status) {
+    const long limit = (1L << 31) - 65536;
+    KpPlan p;
+    if ((double)v.M * v.N * v.K < 4e8 || v.K < KP_K || side_bytes(v.M, v.a_rs, v.K, v.a_cs) >= limit || side_bytes(v.N, v.b_cs, v.K, v.b_rs) >= limit ||
+        !(v.a_cs == 1 || v.a_rs == 1) || !(v.b_cs == 1 || v.b_rs == 1) || (long)v.M * v.N >= (1L << 31) ||
+        !kp_plan(v, ws && ws->ptr && ((uintptr_t)ws->ptr & 3) == 0 ? ws->size : 0, &p))
+        return false;
+    *status = gemm_f32_ks_split_launch(v, ta, tb, p, ws);
     return true;
 }
 

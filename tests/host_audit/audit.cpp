@@ -21,8 +21,12 @@
 //   gather n ic ih iw oc k s p d bias packed_bytes       qsi8 dense NCHW44 convolution without staging
 //   dwpw   n c oc h w stride bias packed_bytes           qsi8 channel-wise 3x3 + pointwise 1x1 in one kernel
 //   pw     n ic ih iw oc stride bias packed_bytes cus    qsi8 pointwise NCHW44 layer, streaming, on a chip of that many CUs
+//   ksplit M K N ta tb lda_pad ldb_pad ldc_pad kg slices swap   f32 MatMul of middle size on the bf16 instructions, by that plan
+//   wide   n ic ih iw oc k s p d bias cus                f32 NCHW convolution of many pixels, on a chip of that many CUs
+//   blocks n c h w count bias                            qsi8 run of channel-wise 3x3 + pointwise 1x1 blocks in one kernel
 //   stem   n oh ow oc act bias packed_bytes cus          f32 image -> qsi8 -> first convolution -> channel-wise -> pointwise in one kernel
 #include <hip/hip_runtime.h>
+#include <sanitizer/asan_interface.h>
 #include <signal.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -35,6 +39,7 @@
 #include <vector>
 
 #include "common.h"
+#include "conv_dw_pw.h"
 #include "conv_geom.h"
 #include "epilogue.h"
 #include "gemm_f32_ks.h"
@@ -78,6 +83,10 @@ __attribute__((aligned(16))) float ks_lds[40 * 1024];
 __attribute__((aligned(16))) int gather_lds[40 * 1024];
 __attribute__((aligned(16))) int8_t dp_lds_mem[160 * 1024];
 
+// ... of conv_f32_wide.hip and conv_blocks.hip, where what lies behind a launch's size is out of bounds too
+__attribute__((aligned(16))) float cw_lds[40 * 1024];
+__attribute__((aligned(16))) int8_t cb_lds[160 * 1024];
+
 size_t gemm_f32_workspace_bytes(long M, long N, long K, bool conv);
 size_t conv_f32_gemm_workspace_bytes(const ConvGeom& g);
 TinyNNStatus conv_f32_gemm_launch(const ConvGeom&, const void*, const void*, const void*, void*, const Workspace*);
@@ -107,6 +116,20 @@ TinyNNStatus conv_dw_pw_launch(
         const ConvGeom&, const ConvGeom&, const void*, const void*, const void*, const void*, const void*, void*, DwPwBlock*, bool);
 }  // namespace mg
 
+void* megcc_gfx950_malloc(size_t n) { return malloc(n); }
+void megcc_gfx950_free(void* p) { free(p); }
+TinyNNStatus megcc_gfx950_memcpy_h2d(void* dst, const void* src, size_t n) { return memcpy(dst, src, n), TinyNN_SUCCESS; }
+
+bool audit_strict = false;
+void audit_dynamic_lds(size_t bytes) {
+    using namespace mg;
+    for (auto lds : {std::make_pair((char*)cw_lds, sizeof(cw_lds)), std::make_pair((char*)cb_lds, sizeof(cb_lds))}) {
+        __asan_unpoison_memory_region(lds.first, lds.second);
+        if (bytes < lds.second)
+            __asan_poison_memory_region(lds.first + bytes, lds.second - bytes);
+    }
+}
+
 // the bf16 conversion of the compiler's vector types (its value does not matter here)
 extern "C" __bf16 __truncsfbf2(float) { return __builtin_bit_cast(__bf16, (unsigned short)0); }
 
@@ -114,6 +137,10 @@ extern "C" TinyNNStatus megcc_gfx950_matmul(
         const MegccMatMulAttr*, Tensor**, int, Tensor**, int, const Workspace*, const RuntimeOpt*);
 
 static std::string g_case;
+void audit_beyond(const char* what, unsigned off, unsigned soff, unsigned bytes) {
+    fprintf(stderr, "OUT OF BOUNDS: %s at %u + %u of %u bytes while running: %s\n", what, off, soff, bytes, g_case.c_str());
+    _exit(3);
+}
 static void on_fault(int, siginfo_t* info, void*) {
     char buf[512];
     int n = snprintf(buf, sizeof(buf), "OUT OF BOUNDS: access at %p while running: %s\n", info->si_addr,
@@ -170,6 +197,10 @@ static bool run_case(const std::string& line, bool at_end) {
     std::string kind;
     ss >> kind;
     g_cus = 256;
+    audit_dynamic_lds(sizeof(cb_lds));  // (all of either)
+    memset(cw_lds, 0, sizeof(cw_lds));
+    memset(cb_lds, 0, sizeof(cb_lds));
+    audit_strict = kind == "ksplit" || kind == "wide" || kind == "blocks";
     if (kind == "mm") {
         int M, K, N, ta, tb, pa, pb, ws;
         ss >> M >> K >> N >> ta >> tb >> pa >> pb >> ws;
@@ -199,6 +230,66 @@ static bool run_case(const std::string& line, bool at_end) {
         const GevmArgs v = {(const float*)A.ptr, (const float*)B.ptr, (float*)Cm.ptr, M, N, K, ta ? 1 : lda, ta ? lda : 1,
                             tb ? 1 : ldb, tb ? ldb : 1, N};
         return (kind == "ks" ? gemm_f32_ks_launch(v, ta, tb) : gemm_f32_split_launch(v, ta, tb)) == TinyNN_SUCCESS;
+    }
+    if (kind == "ksplit") {
+        int M, K, N, ta, tb, pa, pb, pc;
+        KpPlan plan;
+        ss >> M >> K >> N >> ta >> tb >> pa >> pb >> pc >> plan.kg >> plan.slices >> plan.swap;
+        const int ar = ta ? K : M, ac = ta ? M : K, br = tb ? N : K, bc = tb ? K : N;
+        const long lda = ac + pa, ldb = bc + pb, ldc = N + pc;
+        Fenced A(((size_t)(ar - 1) * lda + ac) * 4, at_end, 4), B(((size_t)(br - 1) * ldb + bc) * 4, at_end, 4),
+                Cm(((size_t)(M - 1) * ldc + N) * 4, at_end, 4), W((size_t)plan.slices * M * N * 4, at_end, 4);
+        const GevmArgs v = {(const float*)A.ptr, (const float*)B.ptr, (float*)Cm.ptr, M, N, K, ta ? 1 : lda, ta ? lda : 1,
+                            tb ? 1 : ldb, tb ? ldb : 1, ldc};
+        const Workspace w = {plan.slices > 1 ? W.ptr : nullptr, plan.slices > 1 ? (size_t)plan.slices * M * N * 4 : 0, 0};
+        return gemm_f32_ks_split_launch(v, ta, tb, plan, &w) == TinyNN_SUCCESS;
+    }
+    if (kind == "wide") {
+        ConvGeom g;
+        memset(&g, 0, sizeof(g));
+        int k, s, p, d, bias;
+        ss >> g.n >> g.ic >> g.ih >> g.iw >> g.oc >> k >> s >> p >> d >> bias >> g_cus;
+        g.fh = g.fw = k, g.sh = g.sw = s, g.ph = g.pw = p, g.dh = g.dw = d;
+        g.oh = (g.ih + 2 * p - (d * (k - 1) + 1)) / s + 1;
+        g.ow = (g.iw + 2 * p - (d * (k - 1) + 1)) / s + 1;
+        g.groups = 1, g.fmt = MEGCC_FMT_NCHW, g.act = MEGCC_NONLINE_RELU, g.has_bias = bias;
+        Fenced src((size_t)g.n * g.ic * g.ih * g.iw * 4, at_end, 4), flt((size_t)g.oc * g.ic * k * k * 4, at_end, 4), b((size_t)g.oc * 4, at_end, 4),
+                dst((size_t)g.n * g.oc * g.oh * g.ow * 4, at_end, 4);
+        // (the second time every thread finds the whole table, which the threads of a workgroup write one after the other here)
+        return conv_f32_wide_launch(g, src.ptr, flt.ptr, bias ? b.ptr : nullptr, dst.ptr) == TinyNN_SUCCESS &&
+               conv_f32_wide_launch(g, src.ptr, flt.ptr, bias ? b.ptr : nullptr, dst.ptr) == TinyNN_SUCCESS;
+    }
+    if (kind == "blocks") {
+        int n, c, h, w, count, bias;
+        ss >> n >> c >> h >> w >> count >> bias;
+        const size_t image = (size_t)n * c * h * w;
+        Fenced src(image, at_end, 4), dst(image, at_end, 4), df((size_t)c * 9, at_end, 4), db((size_t)c * 4, at_end, 4), wp((size_t)c * c, at_end, 16),
+                pb((size_t)c * 4, at_end, 4);
+        std::vector<DwPwBlock> blocks((size_t)count);
+        std::vector<const DwPwBlock*> run;
+        for (int i = 0; i < count; ++i) {
+            DwPwArgs a;
+            memset(&a, 0, sizeof(a));
+            // (what lies between two blocks is neither read nor written)
+            a.src = i ? blocks[(size_t)i - 1].host[0].a.dst : (const uint32_t*)src.ptr;
+            a.dst = i + 1 < count ? (uint32_t*)(uintptr_t)(64 * (i + 1)) : (uint32_t*)dst.ptr;
+            a.dflt = (const uint32_t*)df.ptr, a.wp = (const int8_t*)wp.ptr;
+            a.dbias = bias ? (const int32_t*)db.ptr : nullptr, a.pbias = bias ? (const int32_t*)pb.ptr : nullptr;
+            a.src_bytes = a.dst_bytes = (int)image;
+            a.ih = a.oh = h, a.iw = a.ow = w, a.OC = a.OCP = c;
+            a.dq.mode = a.pq.mode = 2;
+            blocks[(size_t)i].host[0].a = blocks[(size_t)i].host[1].a = a;
+            blocks[(size_t)i].act = MEGCC_NONLINE_RELU;
+            run.push_back(&blocks[(size_t)i]);
+        }
+        BlocksRun* r = conv_blocks_create(run.data(), count);
+        if (!r) {
+            fprintf(stderr, "not a conv_blocks run: %s\n", line.c_str());
+            return false;
+        }
+        const TinyNNStatus st = conv_blocks_launch(r);
+        conv_blocks_destroy(r);
+        return st == TinyNN_SUCCESS;
     }
     if (kind == "gather") {
         ConvGeom g;

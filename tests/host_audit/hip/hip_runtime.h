@@ -64,6 +64,7 @@ enum { hipSuccess = 0, hipFuncAttributeMaxDynamicSharedMemorySize = 8 };
 inline const char* hipGetErrorString(hipError_t) { return "host audit"; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipFuncSetAttribute(const void*, int, int) { return hipSuccess; }
+inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 
 inline hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) { return *n = 1, hipSuccess; }
 
@@ -74,17 +75,25 @@ struct audit_rsrc {
     unsigned bytes;
 };
 typedef unsigned audit_v4u __attribute__((ext_vector_type(4)));
-inline unsigned audit_load(audit_rsrc r, unsigned off, unsigned soff) {
-    unsigned v = 0;
+// Most kernels lean on that here and there. Where `audit_strict` is set only offsets with the top bit, which is how a kernel says
+// that it means none, and buffers of no bytes may lie beyond: anything else ends the run as an access out of bounds.
+extern bool audit_strict;
+void audit_beyond(const char* what, unsigned off, unsigned soff, unsigned bytes);
+inline bool audit_inside(audit_rsrc r, unsigned off, unsigned soff, const char* what) {
     if ((unsigned long long)off + soff < r.bytes)
-        v = *(volatile unsigned*)(r.p + off + soff);
-    return v;
+        return true;
+    if (audit_strict && r.bytes && !(off >> 31))
+        audit_beyond(what, off, soff, r.bytes);
+    return false;
+}
+inline unsigned audit_load(audit_rsrc r, unsigned off, unsigned soff) {
+    return audit_inside(r, off, soff, "load") ? *(volatile unsigned*)(r.p + off + soff) : 0;
 }
 inline audit_v4u audit_load4(audit_rsrc r, unsigned off, unsigned soff) {
     return audit_v4u{audit_load(r, off, soff), audit_load(r, off + 4, soff), audit_load(r, off + 8, soff), audit_load(r, off + 12, soff)};
 }
 inline void audit_store(unsigned v, audit_rsrc r, unsigned off, unsigned soff) {
-    if ((unsigned long long)off + soff < r.bytes)
+    if (audit_inside(r, off, soff, "store"))
         *(volatile unsigned*)(r.p + off + soff) = v;
 }
 #define __amdgpu_buffer_rsrc_t audit_rsrc
@@ -124,6 +133,12 @@ inline C audit_sums(const A&, const B&, const C& c, int, int, int) { return c; }
 #define __builtin_amdgcn_mfma_i32_32x32x32_i8(...) audit_sums(__VA_ARGS__)
 #define __builtin_amdgcn_mfma_i32_16x16x64_i8(...) audit_sums(__VA_ARGS__)
 #define __builtin_amdgcn_mfma_i32_16x16x32_i8(...) audit_sums(__VA_ARGS__)
+#define __builtin_amdgcn_fdot2_f32_bf16(a, b, c, clamp) (c)
+struct audit_pair {
+    unsigned v[2];
+    unsigned operator[](int i) const { return v[i]; }
+};
+#define __builtin_amdgcn_permlane32_swap(a, b, x, y) (audit_pair{{(unsigned)(a), (unsigned)(b)}})
 #define __builtin_amdgcn_sdot4(a, b, c, clamp) (c)
 #define __builtin_amdgcn_fmed3f(x, lo, hi) (lo)
 #define __builtin_amdgcn_cvt_pk_u8_f32(x, i, r) (r)
@@ -135,8 +150,10 @@ inline C audit_sums(const A&, const B&, const C& c, int, int, int) { return c; }
 #define __builtin_amdgcn_kernarg_segment_ptr() ((const char*)0)
 
 // every block, every thread, one after the other
+void audit_dynamic_lds(size_t bytes);
 template <typename K, typename... Args>
-inline void host_audit_launch(K kernel, dim3 grid, dim3 block, Args... args) {
+inline void host_audit_launch(K kernel, dim3 grid, dim3 block, size_t lds_bytes, Args... args) {
+    audit_dynamic_lds(lds_bytes);
     gridDim = grid;
     blockDim = block;
     for (unsigned bz = 0; bz < grid.z; ++bz)
@@ -152,4 +169,4 @@ inline void host_audit_launch(K kernel, dim3 grid, dim3 block, Args... args) {
             }
 }
 #define hipLaunchKernelGGL(kernel, grid, block, lds_bytes, strm, ...) \
-    host_audit_launch(kernel, dim3(grid), dim3(block), __VA_ARGS__)
+    host_audit_launch(kernel, dim3(grid), dim3(block), (size_t)(lds_bytes), __VA_ARGS__)

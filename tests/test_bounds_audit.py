@@ -1,6 +1,6 @@
 """Host-side bounds audit of the kernels that issue their loads unconditionally from clamped
-indices or through range-checked buffers (gemm_f32: all four transpositions and the implicit-GEMM gather; gemm_f32_ks and
-gemm_f32_split: all four transpositions; gevm_f32; conv_f32_small; the f32 NCHW44 channel-wise and first-layer kernels;
+indices or through range-checked buffers (gemm_f32: all four transpositions and the implicit-GEMM gather; gemm_f32_ks,
+gemm_f32_split and gemm_f32_ks_split: all four transpositions; conv_f32_wide; conv_blocks; gevm_f32; conv_f32_small; the f32 NCHW44 channel-wise and first-layer kernels;
 fc_one32 / fc_one; every part of fc_tile; fc_gevm_q8; conv_gather_i8; conv_pw_stream / conv_pw_share with and without a stride; conv_dw_pw;
 conv_stem). Not gemm_f32_ks's convolution, whose addresses come through LDS from other threads. tests/host_audit/audit.cpp links the library's own kernel sources,
 compiled as host C++ against a stand-in HIP header that runs every thread of every workgroup on
@@ -24,6 +24,8 @@ CSRC = os.path.join(os.path.dirname(HERE), "megcc_amd", "csrc")
 CLANG = "/opt/rocm/llvm/bin/clang++"
 SOURCES = ["gemm_f32", "gevm_f32", "conv_f32_small", "conv_f32_nchw44", "fc_stream", "fc_gevm_q8", "fc_tile", "gemm_f32_ks",
            "gemm_f32_split", "conv_gather_i8", "conv_pw_stream", "conv_dw_pw", "conv_stem", "requant_table"]
+# compiled with the address sanitizer (host code, like all of it), so that an access beyond a workgroup's LDS ends the run as well
+CHECKED = ["gemm_f32_ks_split", "conv_f32_wide", "conv_blocks"]
 
 pytestmark = pytest.mark.skipif(not os.path.exists(CLANG), reason="needs ROCm's clang++ for the kernels' vector types")
 
@@ -35,7 +37,7 @@ def compile_audit(out_dir, replace=None, have=None):
              "-I" + os.path.join(os.path.dirname(HERE), "include"), "-ffp-contract=off", "-Wno-unknown-attributes"]
     objs = []
     jobs = []
-    for name in SOURCES + ["audit"]:
+    for name in SOURCES + CHECKED + ["audit"]:
         src = os.path.join(AUDIT_DIR, "audit.cpp") if name == "audit" else os.path.join(CSRC, name + ".hip")
         if replace and name in replace:
             src = replace[name]
@@ -45,12 +47,14 @@ def compile_audit(out_dir, replace=None, have=None):
             continue
         objs.append(obj)
         last = ["-O0", "-g0"] if name in ("conv_dw_pw", "conv_pw_stream") else []  # (some 100 instances: half a minute with the optimiser)
+        # (without the optimiser, which leaves out loads that only the stood-in instructions use)
+        last += ["-O0", "-g0", "-fsanitize=address"] if name in CHECKED else []
         jobs.append(subprocess.Popen([CLANG] + flags + last + ["-c", src, "-o", obj], stderr=subprocess.PIPE, text=True))
     for j in jobs:
         err = j.communicate()[1]
         assert j.returncode == 0, err[-4000:]
     exe = os.path.join(out_dir, "audit")
-    subprocess.check_call([CLANG, "-o", exe] + objs)
+    subprocess.check_call([CLANG, "-fsanitize=address", "-o", exe] + objs)
     return exe
 
 
@@ -166,6 +170,28 @@ def audit_lines():
     for m, k, n in ((15, 17, 16), (17, 15, 33), (100, 33, 300), (357, 16, 301), (40, 300, 1700), (513, 9, 530), (600, 31, 700)):
         for t in range(4):
             lines.append("ks %d %d %d %d %d 0 0" % (m, k, n, t & 1, t >> 1))
+    # ... those of middle size, by every plan: rows and columns beyond tiles of 64, 128 and 256; K of less than a stage of 64, of stages and chains with
+    # and without a rest; slices, the last one of less than a stage; padded rows of all three
+    plans = [(kg, slices, swap) for kg in (1, 2, 4) for slices in (1, 2, 3) for swap in (0, 1) if not (kg == 4 and swap)]
+    for t in range(4):
+        for i, plan in enumerate(plans):
+            for k in ((64, 65, 191), (128, 577, 63), (66, 260, 1))[i % 3]:
+                m, n = (int(r.choice([1, 31, 64, 65, 100, 129])) for _ in range(2))
+                lines.append("ksplit %d %d %d %d %d %d %d %d %d %d %d" % ((m, k, n, t & 1, t >> 1) + tuple(int(r.choice([0, 1, 4, 7])) for _ in range(3)) + plan))
+    for plan in plans:
+        lines.append("ksplit 70 1100 270 %d %d 0 3 5 %d %d %d" % ((plan[0] & 1, plan[2]) + plan))
+    # convolutions of many pixels, tiles of 16, 32 and 64 channels: K below a step, of steps, of turns of four and with a rest, taps outside,
+    # a stride, a dilation, pixels beyond the last wave
+    for n, ic, ih, iw, oc, k, st, p, d in (
+            (1, 1, 1, 1, 1, 1, 1, 0, 1), (3, 1, 5, 9, 7, 1, 1, 0, 1), (1, 7, 11, 12, 16, 1, 1, 0, 1), (2, 8, 8, 8, 17, 1, 1, 0, 1), (2, 9, 9, 15, 31, 1, 2, 0, 1), (1, 33, 12, 11, 33, 1, 1, 0, 1),
+            (1, 64, 16, 16, 64, 1, 1, 0, 1), (1, 65, 13, 10, 65, 1, 1, 0, 1), (2, 130, 9, 9, 130, 1, 1, 0, 1), (1, 1, 9, 17, 12, 3, 1, 1, 1), (3, 2, 7, 7, 9, 3, 2, 1, 1), (2, 5, 10, 14, 40, 5, 1, 2, 1),
+            (1, 9, 16, 15, 15, 3, 1, 2, 2), (1, 16, 13, 11, 70, 3, 1, 1, 1), (2, 3, 21, 23, 24, 5, 2, 2, 1), (1, 40, 12, 13, 64, 3, 1, 0, 1), (2, 128, 8, 9, 11, 3, 1, 1, 1), (1, 100, 9, 9, 128, 3, 1, 1, 1),
+            (1, 17, 3, 90, 18, 1, 1, 1, 1), (1, 70, 12, 12, 8, 3, 1, 1, 1), (1, 96, 10, 13, 80, 3, 2, 1, 1)):
+        lines.append("wide %d %d %d %d %d %d %d %d %d %d %d" % (n, ic, ih, iw, oc, k, st, p, d, oc & 1, 1 + 7 * (ic & 1)))
+    # runs of blocks: every kind of map, both numbers of channels
+    for n, h, w, count in ((1, 1, 1, 3), (2, 1, 15, 2), (1, 2, 3, 2), (1, 14, 1, 2), (2, 3, 5, 2), (1, 7, 7, 3), (1, 9, 11, 2), (1, 13, 15, 2), (2, 14, 14, 5), (2, 14, 15, 2)):
+        for c in (256, 512):
+            lines.append("blocks %d %d %d %d %d %d" % (n, c, h, w, count, (h + w + c // 256) & 1))
     # FullyConnected of any K on tiles: rows at any byte, the tensor's last 16 bytes anywhere in a piece
     for m, k, oc in ((65, 5, 9), (64, 1, 3), (16, 1, 1), (65, 129, 67), (70, 295, 70), (225, 515, 361), (66, 128, 64), (130, 260, 257),
                      (100, 1123, 65), (65, 127, 129), (300, 33, 31)):
@@ -221,7 +247,8 @@ def test_every_load_and_store_of_the_clamped_kernels_stays_inside_its_tensor(aud
     assert "audited %d cases" % len(lines) in r.stdout
     ran = {line.split(" -> ")[1] for line in r.stdout.splitlines() if " -> " in line}
     for kernel in ("fc_tile:32,4", "fc_tile:64,1", "fc_tile:64,4", "fc_tile:128,1", "conv_pw_share:16,-1", "conv_pw_stream:1,0",
-                   "conv_pw_stream:8,1", "conv_pw_stream:12,0", "conv_pw_stream:12,1", "conv_pw_stream:32,0", "conv_stem:64,1", "conv_stem:32,1", "conv_stem:64,14"):
+                   "gemm_f32_ks_split:64,256", "gemm_f32_ks_split:64,128", "gemm_f32_ks_split:64,64", "conv_f32_wide:16,32", "conv_f32_wide:32,32",
+                   "conv_f32_wide:64,32", "conv_blocks:256,3", "conv_blocks:512,5", "conv_pw_stream:8,1", "conv_pw_stream:12,0", "conv_pw_stream:12,1", "conv_pw_stream:32,0", "conv_stem:64,1", "conv_stem:32,1", "conv_stem:64,14"):
         assert kernel in ran, (kernel, sorted(ran))
 
 
@@ -268,6 +295,25 @@ def test_the_audit_sees_a_missing_range_test(audit_exe, tmp_path, source, was, b
     exe = compile_audit(str(tmp_path / "build"), replace={source: str(mutated)}, have=os.path.dirname(audit_exe))
     r = subprocess.run([exe], input=line + "\n", capture_output=True, text=True, timeout=300)
     assert r.returncode == 3 and "OUT OF BOUNDS" in r.stderr, (r.returncode, r.stderr[-500:])
+
+
+@pytest.mark.parametrize("source,was,by,line,what", [
+    # a row behind the operand's last; a channel behind the last, stored and of the filter; one value more of a stage in LDS than there is room for; a
+    # layer's last parameter behind the LDS that was asked for
+    ("gemm_f32_ks_split", "min(r, s.rows - 1)", "r", "ksplit 70 128 130 0 0 0 0 0 1 1 0", "OUT OF BOUNDS: load"),
+    ("conv_f32_wide", "if (there && m0 + row + e < q.M)", "if (there)", "wide 1 4 5 7 3 1 1 0 1 1 1", "OUT OF BOUNDS: access"),
+    ("conv_f32_wide", "min(m0 + i * R + c, q.M - 1)", "(m0 + i * R + c)", "wide 1 16 5 7 3 1 1 0 1 1 1", "OUT OF BOUNDS: load"),
+    ("gemm_f32_ks_split", "lds[4 * KP_STAGE > MEET ? 4 * KP_STAGE : MEET]", "lds[4 * KP_STAGE - 32]", "ksplit 64 256 64 0 1 0 0 0 1 1 0", "AddressSanitizer"),
+    ("conv_blocks", "BYTES = MAP + 2 * LAYER * 4;", "BYTES = MAP + 2 * LAYER * 4 - 4;", "blocks 1 256 3 5 2 1", "AddressSanitizer"),
+])
+def test_the_audit_sees_an_access_beyond_a_buffer_or_the_lds(audit_exe, tmp_path, source, was, by, line, what):
+    src = open(os.path.join(CSRC, source + ".hip")).read()
+    assert src.count(was) == 1
+    mutated = tmp_path / (source + ".hip")
+    mutated.write_text(src.replace(was, by))
+    exe = compile_audit(str(tmp_path / "build"), replace={source: str(mutated)}, have=os.path.dirname(audit_exe))
+    r = subprocess.run([exe], input=line + "\n", capture_output=True, text=True, timeout=300)
+    assert r.returncode != 0 and what in r.stderr, (r.returncode, r.stderr[-500:])
 
 
 _no_clamp = []
