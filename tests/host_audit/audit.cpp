@@ -149,6 +149,10 @@ static void on_fault(int, siginfo_t* info, void*) {
     _exit(3);
 }
 
+// what operands hold. As floats: 2.4e-38, which the bf16 parts of f32 products cannot hold, and 0.75
+static const int kFills[] = {0x01, 0x3f};
+static int g_fill = kFills[0];
+
 // `bytes` usable bytes whose end (at_end) or start touches an inaccessible page
 struct Fenced {
     void* map = nullptr;
@@ -173,7 +177,7 @@ struct Fenced {
         } else {
             ptr = base + page;
         }
-        memset(ptr, 1, bytes);
+        memset(ptr, g_fill, bytes);
     }
     ~Fenced() { munmap(map, map_bytes); }
 };
@@ -478,13 +482,20 @@ int main() {
             line.pop_back();
         if (line.empty() || line[0] == '#')
             continue;
-        for (int at_end = 1; at_end >= 0; --at_end) {
-            g_case = line + (at_end ? "  [buffers end at a fence]" : "  [buffers start at a fence]");
-            if (!run_case(line, at_end != 0)) {
-                fprintf(stderr, "FAILED: %s\n", g_case.c_str());
-                return 1;
+        const bool parts = line.rfind("split ", 0) == 0 || line.rfind("ksplit ", 0) == 0;
+        for (int fill : kFills) {
+            if (fill != kFills[0] && !parts)
+                continue;
+            g_fill = fill;
+            for (int at_end = 1; at_end >= 0; --at_end) {
+                g_case = line + (at_end ? "  [buffers end at a fence]" : "  [buffers start at a fence]");
+                if (!run_case(line, at_end != 0)) {
+                    fprintf(stderr, "FAILED: %s\n", g_case.c_str());
+                    return 1;
+                }
             }
         }
+        g_fill = kFills[0];
         printf("ok %s -> %s\n", line.c_str(), mg::g_noted.c_str());
         fflush(stdout);
         ++n;

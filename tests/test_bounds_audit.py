@@ -304,7 +304,7 @@ def test_the_audit_sees_a_missing_range_test(audit_exe, tmp_path, source, was, b
     ("conv_f32_wide", "if (there && m0 + row + e < q.M)", "if (there)", "wide 1 4 5 7 3 1 1 0 1 1 1", "OUT OF BOUNDS: access"),
     ("conv_f32_wide", "min(m0 + i * R + c, q.M - 1)", "(m0 + i * R + c)", "wide 1 16 5 7 3 1 1 0 1 1 1", "OUT OF BOUNDS: load"),
     ("gemm_f32_ks_split", "lds[4 * KP_STAGE > MEET ? 4 * KP_STAGE : MEET]", "lds[4 * KP_STAGE - 32]", "ksplit 64 256 64 0 1 0 0 0 1 1 0", "AddressSanitizer"),
-    ("conv_blocks", "BYTES = MAP + 2 * LAYER * 4;", "BYTES = MAP + 2 * LAYER * 4 - 4;", "blocks 1 256 3 5 2 1", "AddressSanitizer"),
+    ("conv_blocks", "BYTES = MAP + 2 * LAYER * 4;", "BYTES = MAP + 2 * LAYER * 4 - 16;", "blocks 1 256 3 5 2 1", "AddressSanitizer"),
 ])
 def test_the_audit_sees_an_access_beyond_a_buffer_or_the_lds(audit_exe, tmp_path, source, was, by, line, what):
     src = open(os.path.join(CSRC, source + ".hip")).read()
