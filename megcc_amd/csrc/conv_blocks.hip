@@ -328,11 +328,13 @@ static int cb_lds_bytes(int mt) {
     return mt == 2 ? CbLds<2>::BYTES : CbLds<1>::BYTES;
 }
 
-// Fewer images than a fifth of the CUs are not even timed (five blocks of 512 channels N=64, 59 us pair by pair, take 90, which is one image's
-// time): preparing MobileNetV1 batch 1 took 20.5 ms for 17.1 with the question asked.
+// A workgroup an image, two a CU with 256 channels: where fewer images leave CUs without one, runs are not even timed (us, pair by pair / as one
+// kernel: five blocks of 512 channels N=64 58 / 76, 96 76 / 76, 104 78 / 77, 128 83 / 77; of 256 N=32 26 / 36, 52 42 / 36, 64 34 / 36, 80 47 / 36). A tie
+// alone loses beside the other stream: MobileNetV1 batch 88 191 / 198, 96 199 / 206, but 104 229 / 224, 112 243 / 222.
 bool conv_blocks_takes(const Tensor& x) {
     const uint32_t* d = x.layout.dims;
-    return x.layout.nr_dim == 5 && (options().fuse_blocks || 5L * d[0] >= num_cus()) && (d[1] == 64 || d[1] == 128) && d[2] <= 2 * CB_PARTS && d[3] <= CB_COLS;
+    return x.layout.nr_dim == 5 && (d[1] == 64 || d[1] == 128) && (options().fuse_blocks || 5L * d[0] >= (d[1] == 128 ? 2L : 1L) * num_cus()) &&
+           d[2] <= 2 * CB_PARTS && d[3] <= CB_COLS;
 }
 
 void conv_blocks_destroy(BlocksRun* run) {

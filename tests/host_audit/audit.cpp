@@ -24,6 +24,7 @@
 //   ksplit M K N ta tb lda_pad ldb_pad ldc_pad kg slices swap   f32 MatMul of middle size on the bf16 instructions, by that plan
 //   wide   n ic ih iw oc k s p d bias cus                f32 NCHW convolution of many pixels, on a chip of that many CUs
 //   blocks n c h w count bias                            qsi8 run of channel-wise 3x3 + pointwise 1x1 blocks in one kernel
+//   asked  n c h w cus                                   whether that one would be timed, noted as "conv_blocks_takes:1,0" or 0
 //   stem   n oh ow oc act bias packed_bytes cus          f32 image -> qsi8 -> first convolution -> channel-wise -> pointwise in one kernel
 #include <hip/hip_runtime.h>
 #include <sanitizer/asan_interface.h>
@@ -294,6 +295,16 @@ static bool run_case(const std::string& line, bool at_end) {
         const TinyNNStatus st = conv_blocks_launch(r);
         conv_blocks_destroy(r);
         return st == TinyNN_SUCCESS;
+    }
+    if (kind == "asked") {
+        int n, c, h, w;
+        ss >> n >> c >> h >> w >> g_cus;
+        Tensor x = tensor2d(nullptr, 1, 1, 1);
+        const uint32_t dims[5] = {(uint32_t)n, (uint32_t)c / 4, (uint32_t)h, (uint32_t)w, 4};
+        x.layout.nr_dim = 5;
+        std::copy(dims, dims + 5, x.layout.dims);
+        note_kernel("conv_blocks_takes", conv_blocks_takes(x), 0, 0, 0, 0);
+        return true;
     }
     if (kind == "gather") {
         ConvGeom g;

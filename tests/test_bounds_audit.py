@@ -252,6 +252,15 @@ def test_every_load_and_store_of_the_clamped_kernels_stays_inside_its_tensor(aud
         assert kernel in ran, (kernel, sorted(ran))
 
 
+def test_which_runs_of_blocks_are_asked_for(audit_exe):
+    """images for two fifths of the CUs with 512 channels, a fifth with 256 (host code of the library)"""
+    ask = {"102 512 14 14 256": 0, "103 512 14 14 256": 1, "103 512 14 15 256": 1, "103 512 15 14 256": 0, "103 512 14 16 256": 0, "51 256 14 14 256": 0,
+           "52 256 14 14 256": 1, "52 512 14 14 256": 0, "200 384 14 14 256": 0, "200 128 14 14 256": 0, "52 512 7 7 128": 1, "1 256 1 1 5": 1, "1 512 1 1 5": 0}
+    r = subprocess.run([audit_exe], input="".join("asked %s\n" % a for a in ask), capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr[-500:]
+    assert r.stdout.splitlines()[:-1] == ["ok asked %s -> conv_blocks_takes:%d,0" % a for a in ask.items()]
+
+
 def test_the_audit_sees_the_out_of_bounds_read_a_missing_clamp_causes(audit_exe, tmp_path):
     """the audit itself, pinned by a mutation: without the clamp of the gather's column the surplus
     columns of a ragged last pixel tile read up to one image past the tensor; the audit must die on it"""
