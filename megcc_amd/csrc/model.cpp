@@ -490,6 +490,11 @@ static void join_blocks(Model* m, const std::vector<int>& readers) {
             ++end;
         if (end < i + 2 || shares_bytes(*m->schedule[i]->in_ptrs[0], *m->schedule[end - 1]->out_ptrs[0]))
             continue;
+        const size_t at = (size_t)m->schedule[i]->first_index;
+        if (!options().fuse_blocks && at < m->blocks_time.size() && m->blocks_time[at].known && !m->blocks_time[at].faster) {
+            i = end - 1;
+            continue;
+        }
         const std::vector<ModelOpr*> run(m->schedule.begin() + (long)i, m->schedule.begin() + (long)end);
         std::vector<const DwPwBlock*> blocks;
         ModelOpr* f = new ModelOpr();
@@ -991,23 +996,34 @@ static Choice choose_schedule(Model* m) {
     };
     float first = time_forwards(m, 1);
     // A run of blocks has a CU an image, and what the others do beside it is the other stream's: only where whole forwards are faster
-    // by 2 % (us with MobileNetV1's five blocks as one kernel / without: batch 80 195 / 192, 96 203 / 199, 112 221 / 241, 128 235 / 257).
-    // (The first forwards were timed while the clocks went up: a lead of 5 % is then one, and is not asked for twice. Preparing MobileNetV1
-    // batch 256 133 ms with every comparison made twice, 115 so, 96 without runs.)
+    // by 2 %. (The first forwards were timed while the clocks went up: a lead of 5 % is then one, and is not asked for twice.)
     if (blocks) {
         const Pairs without = {true, true, false};
+        const double us = m->schedule_us;
         const float as_pairs = time_pairs(without);
+        const int tail_pairs = m->tail_begin;
         bool keep = as_pairs <= 0.f || (first > 0.f && first < 0.95f * as_pairs);
         if (!keep) {
             const float with = std::min(first, time_pairs(best));
             keep = with > 0.f && with < 0.98f * as_pairs && with < 0.98f * time_pairs(without);
         }
-        if (!keep)
+        if (!keep) {
             best = without;
+            tail_begin = tail_pairs;
+        }
+        if (!pw_dw && !doubt) {
+            // (Nothing more to ask, and what these take is known. Preparing MobileNetV1 batch 256: 105 ms, with the kernels and the forwards timed
+            // once more 114, without runs 96.)
+            reset_tail(m);
+            build_schedule(m, best);
+            if (tail_begin >= 0)
+                setup_tail(m, tail_begin);
+            if (keep)
+                m->schedule_us = us;
+            return {best, m->tail_begin};
+        }
         first = time_pairs(best);
         tail_begin = m->tail_begin;
-        if (!pw_dw && !doubt)
-            return {best, tail_begin};
     }
     float cost = first;
     Pairs winner = best;
