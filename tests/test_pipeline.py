@@ -204,6 +204,45 @@ def test_two_hundred_overlapped_forwards(planned):
     serial.close()
 
 
+@pytest.mark.parametrize("batch,forced,planned", [(32, True, False), (32, True, True), (112, False, False)],
+                         ids=["32_forced_own_plan", "32_forced_reference_plan", "112_as_chosen"])
+def test_forwards_with_a_run_of_blocks_as_one_kernel(batch, forced, planned):
+    """the five blocks of 512 channels as one kernel among the others, on either stream and at the boundary between them: forwards back to
+    back, a graph, the operators one by one. At 112 images whole forwards choose it, and memory is planned again without the run's tensors"""
+    net = mobilenet.Net(batch)
+    images = [mobilenet.draw_input(batch, seed=s) for s in (41, 42, 43)]
+    serial, sids = build(net, False, no_graph=1, nopipeline=1)
+    want = []
+    for img in images:
+        serial.set_input(sids["image"], img)
+        serial.forward()
+        want.append(serial.get(sids["softmax"]).copy())
+    serial.close()
+    assert not np.array_equal(want[0], want[1])
+    for options in (dict(no_graph=1), {}):
+        pipe, ids = build(net, planned, fuseblocks=int(forced), **options)
+        without, _ = build(net, planned, nofuseblocks=1, no_graph=1)
+        print(batch, "kernels", pipe.nr_kernel, "on the second stream", pipe.nr_tail_kernel, "without", without.nr_kernel)
+        if not planned:
+            assert pipe.nr_kernel <= without.nr_kernel - 4
+        without.close()
+        outs = [np.zeros((batch, 1000), np.float32) for _ in range(30)]
+        for k, out in enumerate(outs):
+            pipe.set_input(ids["image"], images[k % 3])
+            pipe.forward()
+            pipe.get_async(ids["softmax"], out)
+        runtime.wait()
+        bad = [k for k, out in enumerate(outs) if not np.array_equal(out, want[k % 3])]
+        assert not bad, bad
+        pipe.set_input(ids["image"], images[1])
+        for i in range(pipe.nr_opr):
+            pipe.run_opr(i)
+        np.testing.assert_array_equal(pipe.get(ids["softmax"]), want[1])
+        pipe.forward()
+        np.testing.assert_array_equal(pipe.get(ids["softmax"]), want[1])
+        pipe.close()
+
+
 def test_a_forward_behind_a_wait_runs_on_one_stream():
     """whichever way the host has waited for the last forward - a blocking read, wait() after it, an asynchronous read and
     wait(), wait() and join() in either order with the next input in between -, the next one finds nothing to overlap; without a
