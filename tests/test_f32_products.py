@@ -143,29 +143,42 @@ def product64(case, arrays):
     return (a.T if case.trans_a else a) @ (b.T if case.trans_b else b)
 
 
-# products of middle size on the bf16 parts, a workgroup's waves sharing K: either operand staged, one wave, two and four to a
-# stage's K, with and without slices of K; K with and without a rest of a stage, rows and columns beyond whole tiles
-MIDDLE = [(512, 4096, 4096), (1912, 1206, 1078), (83, 2794, 3689), (947, 2247, 657), (1381, 2795, 925), (3713, 2717, 528), (320, 4095, 1100),
-          (2500, 1216, 400), (1290, 1088, 1290)]
+# products of middle size on the bf16 parts, a workgroup's waves sharing K, and the plan each is to have (rows of either operand, slices of K, which
+# one is staged; None: not there): every transposition with either operand staged, one wave, two and four to a stage's K, whole and in slices; K with and
+# without a rest of a stage, rows and columns beyond whole tiles
+MIDDLE = [(512, 4096, 4096, "nn", "64,256,2,0"), (512, 4096, 4096, "nt", "64,256,2,0"), (512, 4096, 4096, "tn", "64,256,2,0"),
+          (512, 4096, 4096, "tt", "64,256,2,0"), (1912, 1206, 1078, "nn", "64,128,1,1"), (1912, 1206, 1078, "nt", "64,128,1,1"),
+          (1912, 1206, 1078, "tn", None), (1912, 1206, 1078, "tt", "64,128,1,1"), (83, 2794, 3689, "nn", None), (83, 2794, 3689, "nt", "64,256,8,0"),
+          (83, 2794, 3689, "tn", None), (83, 2794, 3689, "tt", None), (947, 2247, 657, "nn", "64,64,3,0"), (947, 2247, 657, "nt", "64,64,3,0"),
+          (947, 2247, 657, "tn", None), (947, 2247, 657, "tt", "64,64,3,0"), (1381, 2795, 925, "nn", "64,128,3,1"),
+          (1381, 2795, 925, "nt", "64,128,3,1"), (1381, 2795, 925, "tn", None), (1381, 2795, 925, "tt", "64,128,3,1"),
+          (3713, 2717, 528, "nn", "64,256,3,1"), (3713, 2717, 528, "nt", "64,256,3,1"), (3713, 2717, 528, "tn", None), (3713, 2717, 528, "tt", None),
+          (320, 4095, 1100, "nn", "64,128,5,0"), (320, 4095, 1100, "nt", "64,128,5,0"), (320, 4095, 1100, "tn", "64,128,5,0"),
+          (320, 4095, 1100, "tt", "64,128,5,0"), (2500, 1216, 400, "nn", None), (2500, 1216, 400, "nt", "64,256,3,0"), (2500, 1216, 400, "tn", None),
+          (2500, 1216, 400, "tt", None), (1290, 1088, 1290, "nn", "64,128,1,0"), (1290, 1088, 1290, "nt", "64,128,1,0"),
+          (1290, 1088, 1290, "tn", "64,128,1,0"), (1290, 1088, 1290, "tt", "64,128,1,0"), (1741, 1791, 471, "nn", "64,64,1,0"),
+          (1026, 226, 3702, "nn", "64,256,1,0"), (2464, 223, 1597, "nn", "64,256,1,1"), (2942, 1274, 259, "nt", "64,64,1,0"),
+          (1044, 211, 3628, "nt", "64,256,1,0"), (3660, 204, 1047, "nt", "64,256,1,1"), (1545, 3559, 605, "tn", "64,64,1,0"),
+          (40, 3715, 2862, "tn", "64,64,5,0"), (3366, 1021, 563, "tn", "64,128,1,1"), (2927, 4073, 34, "tn", "64,128,11,1"),
+          (3249, 237, 1222, "tn", "64,256,1,0"), (3620, 331, 1047, "tn", "64,256,1,1"), (2831, 2293, 70, "tn", "64,256,9,1"),
+          (1152, 1791, 679, "tt", "64,64,1,0"), (1551, 246, 2436, "tt", "64,256,1,0"), (2466, 218, 1537, "tt", "64,256,1,1"),
+          (1641, 3724, 66, "tt", "64,256,15,1")]
 
 
-@pytest.mark.parametrize("m,k,n", MIDDLE)
-@pytest.mark.parametrize("ta", [False, True])
-@pytest.mark.parametrize("tb", [False, True])
-def test_products_of_middle_size(m, k, n, ta, tb):
-    case = MatMulCase(m, k, n, ta, tb)
+@pytest.mark.parametrize("m,k,n,t,plan", MIDDLE)
+def test_products_of_middle_size(m, k, n, t, plan):
+    case = MatMulCase(m, k, n, t[0] == "t", t[1] == "t")
     arrays = case.gen(seed=71)
     got, want = run(case, arrays), product64(case, arrays)
-    kernel = runtime.last_kernel()
-    print(kernel)
+    assert runtime.last_kernel().startswith("gemm_f32_ks_split:" + plan if plan else KS), runtime.last_kernel()
     # each of the k products and sums is rounded once, in whatever order
     bound = product64(case, {x: np.abs(v) for x, v in arrays.items()}) * (k * 2.0 ** -24)
     assert np.all(np.abs(got - want) <= bound)
-    if kernel.startswith("gemm_f32_ks_split"):
+    if plan:
         runtime.set_option("nof32split", 1)
         try:
             in_f32 = run(case, arrays)
-            assert runtime.last_kernel().startswith("gemm_f32_ks:"), runtime.last_kernel()
+            assert runtime.last_kernel().startswith(("gemm_f32_ks:", "gemm_f32:")), runtime.last_kernel()
         finally:
             runtime.set_option("nof32split", 0)
         assert np.linalg.norm(got - want) <= np.linalg.norm(in_f32 - want)
@@ -174,15 +187,11 @@ def test_products_of_middle_size(m, k, n, ta, tb):
         assert np.array_equal(run(case, whole), product64(case, whole))
 
 
-def test_products_of_middle_size_reach_every_form():
-    seen = set()
-    for m, k, n in MIDDLE:
-        case = MatMulCase(m, k, n, False, True)
-        run(case, case.gen(seed=72))
-        if runtime.last_kernel().startswith("gemm_f32_ks_split"):
-            tile, slices, swap = runtime.last_kernel().split(":")[1].split(",")[1:4]
-            seen |= {"tile " + tile, "swap " + swap, "sliced" if slices != "1" else "whole"}
-    assert seen == {"tile 64", "tile 128", "tile 256", "swap 0", "swap 1", "sliced", "whole"}, seen
+def test_products_of_middle_size_are_of_every_form():
+    seen = {(t,) + tuple(plan.split(",")[1:2]) + (plan.split(",")[3], plan.split(",")[2] != "1") for _, _, _, t, plan in MIDDLE if plan}
+    every = {(t, tile, swap, sliced) for t in ("nn", "nt", "tn", "tt") for tile in ("64", "128", "256") for swap in ("0", "1") for sliced in (False, True)
+             if not (tile == "64" and swap == "1")}  # (64 rows of either: never swapped)
+    assert seen == every, every - seen
 
 
 @pytest.mark.parametrize("m,k,n,tb", [(1912, 1206, 1078, False), (947, 2247, 657, True), (83, 2794, 3689, True), (512, 4096, 4096, False)])
@@ -252,3 +261,60 @@ def check_tiny_values(case, kernel, value, side):
 @pytest.mark.parametrize("side", ["a", "b"])
 def test_products_of_many_tiles_of_values_below_every_bf16(m, k, n, ta, tb, value, side):
     check_tiny_values(MatMulCase(m, k, n, ta, tb), "gemm_f32_split", value, side)
+
+
+def padded(arrays, case, pads):
+    """the operands and the result with rows longer than they are wide, what lies between filled with NaN"""
+    ins, outs = case.specs(arrays)
+    for s, pad in zip(ins + outs, pads):
+        rows, cols = s.shape
+        s.strides = (cols + pad, 1)
+        if s in ins:
+            wide = np.full((rows, cols + pad), np.nan, np.float32)
+            wide[:, :cols] = s.array
+            s.array = wide
+    outs[0].storage = (case.m, case.n + pads[2])
+    return ins, outs
+
+
+# ... with room for all of the slices, for two of them, for less, none, and a workspace that floats cannot be stored to
+@pytest.mark.parametrize("m,k,n,t,plan", [p for p in MIDDLE if p[4] and p[4].split(",")[2] != "1"][::4])
+def test_products_of_middle_size_with_less_workspace(m, k, n, t, plan):
+    case = MatMulCase(m, k, n, t[0] == "t", t[1] == "t")
+    arrays = case.gen(seed=76)
+    want = product64(case, arrays)
+    bound = product64(case, {x: np.abs(v) for x, v in arrays.items()}) * (k * 2.0 ** -24)
+    op = runtime.PreparedOp(runtime.parse_symbol(case.symbol()), *case.specs(arrays))
+    size, ptr = op.ws.size, op.ws.ptr
+    slices = int(plan.split(",")[2])
+    assert size >= slices * m * n * 4
+    for room, at, most in ((slices * m * n * 4, ptr, slices), (2 * m * n * 4, ptr, 2), (2 * m * n * 4 - 1, ptr, 1), (0, None, 1), (size - 1, ptr + 1, 1)):
+        op.ws.size, op.ws.ptr = room, at
+        op.poison_outputs()
+        op.launch()
+        kernel = runtime.last_kernel()
+        if kernel.startswith("gemm_f32_ks_split"):
+            assert int(kernel.split(",")[2]) <= most, (kernel, room)
+        else:
+            assert kernel.startswith(("gemm_f32_ks:", "gemm_f32:")) and most < slices, (kernel, room)
+        assert np.all(np.abs(op.result() - want) <= bound), (kernel, room)
+
+
+PADDED = [(512, 1219, 640, "nn"), (83, 2794, 3689, "nt"), (1290, 1088, 1290, "tt"), (2927, 4073, 34, "tn"), (1, 700, 333, "nn"), (3, 513, 130, "nt"), (4, 2900, 700, "nn"),
+          (2, 260, 75, "tn"), (70, 90, 66, "nn"), (2040, 145, 1999, "tn")]
+
+
+@pytest.mark.parametrize("m,k,n,t", PADDED)
+@pytest.mark.parametrize("pads", [(3, 0, 0), (0, 1, 0), (0, 0, 5), (4, 8, 12), (1, 3, 7)])
+def test_products_of_padded_rows(m, k, n, t, pads):
+    """whichever kernel takes them, nothing between the rows is read into a sum or written"""
+    case = MatMulCase(m, k, n, t[0] == "t", t[1] == "t")
+    arrays = case.gen(seed=77)
+    op = runtime.PreparedOp(runtime.parse_symbol(case.symbol()), *padded(arrays, case, pads))
+    before = op.result()
+    op.launch()
+    print("GPU case:", repr(case), pads, runtime.last_kernel(), flush=True)
+    got = op.result()
+    bound = product64(case, {x: np.abs(v) for x, v in arrays.items()}) * ((k + 1) * 2.0 ** -24)
+    assert np.all(np.abs(got[:, :n] - product64(case, arrays)) <= bound)
+    assert got[:, n:].tobytes() == before[:, n:].tobytes()
