@@ -117,6 +117,21 @@ def test_layers_of_many_pixels(tile, n, ic, oc, h, w, k, stride, act, bias):
     assert np.isfinite(got[:n - 1]).all() and np.isfinite(got[n - 1, :, :(h - k) // stride - 1]).all()
 
 
+# other windows' places: a dilation, no padding and more than half a window, strides of two and three
+@pytest.mark.parametrize("n,ic,oc,h,w,k,stride,pad,dilate", [(12, 8, 30, 71, 83, 3, 1, 2, 2), (10, 12, 20, 60, 75, 3, 1, 0, 1), (18, 3, 16, 98, 90, 5, 2, 4, 1), (6, 10, 40, 60, 70, 1, 1, 1, 1),
+                                                             (42, 6, 62, 103, 101, 3, 3, 1, 1), (4, 5, 70, 66, 61, 5, 1, 4, 2)])
+def test_layers_of_many_pixels_of_other_windows(n, ic, oc, h, w, k, stride, pad, dilate):
+    import torch
+    case = ConvCase(A.FMT_NCHW, A.DENSE, n, ic, h, w, oc, k, stride, pad, A.IDENTITY, dtype="f32", dilate=dilate)
+    arrays = case.gen(seed=68)
+    got = run(case, arrays)
+    assert runtime.last_kernel().startswith("conv_f32_wide:"), runtime.last_kernel()
+    want, mag = (torch.nn.functional.conv2d(*(torch.from_numpy(f(arrays[x]).astype(np.float64)) for x in ("src", "flt")),
+                                            torch.from_numpy(f(arrays["bias"]).astype(np.float64).reshape(-1)), stride=stride, padding=pad,
+                                            dilation=dilate).numpy() for f in (np.array, np.abs))
+    assert np.all(np.abs(got - want) <= (ic * k * k + 2) * 2.0 ** -24 * mag)
+
+
 # up to 16 channels and a long K on fewer pixels, or more than it takes: 16 x 16 tiles with four waves sharing K
 @pytest.mark.parametrize("n,ic,oc,h,w,k,stride", [(8, 28, 16, 33, 33, 3, 1), (3, 250, 16, 53, 52, 1, 1), (13, 114, 11, 46, 57, 3, 2), (3, 95, 1, 65, 65, 3, 1)])
 def test_layers_of_few_channels_and_a_long_k(n, ic, oc, h, w, k, stride):
