@@ -1,6 +1,6 @@
 // A run of blocks - channel-wise 3x3 (pad 1, stride 1, RELU), then the pointwise 1x1 convolution of its result back to the same
 // number of channels (RELU) - as ONE kernel, qsi8 NCHW44, 256 or 512 channels on maps of up to 14 x 15 pixels: the middle of a
-// MobileNet (five blocks of 512 channels at 14 x 14). One workgroup holds one image for the whole run: 100 KB of LDS, which
+// MobileNet (five blocks of 512 channels at 14 x 14). One workgroup holds one image for the whole run in LDS (146 KB with 512 channels, 74 with 256), which
 // every layer overwrites in place. As one kernel a block (conv_dw_pw.hip) a workgroup's tile of 64 pixels waits for its pixels
 // from HBM in every one of its four channel-wise jobs, takes the whole filter (256 KB) for every tile, and each block
 // begins when the last tile of the one before is done.
@@ -15,10 +15,10 @@
 //   wave of a SIMD multiplies while the other requantises. When all waves are through, the results take the pixels' place. The
 //   filter is streamed, four chunks of 32 channels ahead, across the parts and the layers: 512 KB a layer and image.
 // Two barriers a layer. Both requantisations are the exact ones of epilogue.h: bit for bit the layers one by one.
-// Bound: the matrix cores (19700 of a layer's 33000 cycles) and the vector ALU's issue (4200 instructions a SIMD, 3.3 to 5 cycles each with two
-// waves), which overlap in the pointwise half only.
-// Measured (five blocks of 512 channels 14 x 14, us, pair by pair / as one kernel): N=64 59 / 90, 128 84 / 90, 256 142 / 92, 512 246 / 180; 256
-// channels N=128 53 / 44, 256 72 / 45; MobileNetV1 batch 256 490 / 450. With the requantisation behind the barrier, where no wave
+// Bound: the matrix cores (19700 of a layer's 35400 cycles) and the vector ALU's issue (4000 instructions a SIMD with the products, 3.3 to 5 cycles each
+// with two waves), which overlap in the pointwise half only. Counters: profiles/conv_blocks__5_blocks_14x14.txt.
+// Measured (five blocks of 512 channels 14 x 14, us, pair by pair / as one kernel): N=64 60 / 76, 128 88 / 78, 256 146 / 94, 512 264 / 170; 256
+// channels N=128 55 / 38, 256 76 / 43; MobileNetV1 batch 256 495 / 444. With the requantisation behind the barrier, where no wave
 // multiplies, 96.8 for 91.5; operands moved by a lane (DPP) instead of three taps of a product 106; one channel group at a time 96.8 for 94.5.
 #include <cstring>
 #include <vector>
@@ -329,7 +329,7 @@ static int cb_lds_bytes(int mt) {
 }
 
 // A workgroup an image, two a CU with 256 channels: where fewer images leave CUs without one, runs are not even timed (us, pair by pair / as one
-// kernel: five blocks of 512 channels N=64 58 / 76, 96 76 / 76, 104 78 / 77, 128 83 / 77; of 256 N=32 26 / 36, 52 42 / 36, 64 34 / 36, 80 47 / 36). A tie
+// kernel: five blocks of 512 channels N=64 60 / 76, 96 78 / 77, 104 81 / 77, 128 88 / 78; of 256 N=32 26 / 36, 52 45 / 36, 80 48 / 37). A tie
 // alone loses beside the other stream: MobileNetV1 batch 88 191 / 198, 96 199 / 206, but 104 229 / 224, 112 243 / 222.
 bool conv_blocks_takes(const Tensor& x) {
     const uint32_t* d = x.layout.dims;

@@ -15,7 +15,8 @@
 //   * Running sums are closed every 16 or 32 values of K. Relative error against 64 bits, gemm_f32_ks.hip / here: 8 -> 9 3x3 0.93e-7 / 0.89e-7,
 //     126 -> 74 1x1 1.13e-7 / 0.99e-7, 32 -> 32 3x3 1.59e-7 / 1.12e-7, 96 -> 11 3x3 1.53e-7 / 1.28e-7, 100 -> 128 3x3 1.52e-7 / 1.47e-7; it grows with
 //     the number of closings, up to CwPlan's longest K (128 -> 96 3x3 1.55e-7 / 1.74e-7, which is why it stays there).
-// Bound: f32 MFMA (0.7 - 0.8 of the time with two waves a SIMD), launch and a wave's prologue for short K. Eight steps in flight: no
+// Bound: f32 MFMA (by counter 0.43 - 0.67 of the cycles a CU is busy: 96 -> 11 and 64 -> 64 below; profiles/conv_f32_wide__drawn_layers.txt), launch and a wave's prologue for
+// short K. Eight steps in flight: no
 // faster (96 -> 11 39.7 for 40.0). Fp32Im2col.cpp:88-218 is the loop replaced.
 // Measured (us, gemm_f32_ks.hip / here): 3x3 96 -> 11 77 x 77 N=9 39.0 / 29.2, 15 -> 81 83 x 83 N=13 44 / 35, 3 -> 8 112 x 112 N=16 15.4 / 11.4, 7 -> 118
 // 83 x 24 N=8 13.0 / 8.6, 64 -> 64 112 x 112 N=16 164 / 154, 52 -> 121 42 x 42 N=7 26 / 23.6; 1x1 126 -> 74 97 x 87 N=5 25.8 / 15.9,
@@ -278,7 +279,7 @@ struct CwPlan {
     double us;  // estimated
 };
 
-// A workgroup puts one wave on each SIMD of a CU: its MFMAs (the matrix units are busy 0.7 - 0.8 of the time), 0.45 - 1 us for the
+// A workgroup puts one wave on each SIMD of a CU: its MFMAs, 0.45 - 1 us for the
 // prologue and end of every set of 256 workgroups, 4 for launch and first operands; pixels that do not
 // follow one another cost the loads' way 1.8 times (108 -> 9 87 x 69 stride 2 N=11 23.3 / 23.7, 27 -> 38 86 x 86 stride 2 N=9 14.4 / 14.7). Rows of 16 cost a third more than rows of
 // 32, 64 a twentieth less. Estimated / measured us: 96 -> 11 77 x 77 N=9 in rows of 16, 32, 64 26 / 28, 36 / 40, 65 / 63; 15 -> 81 83 x 83 N=13 41 / 43, 30 / 35, 37 / 43;

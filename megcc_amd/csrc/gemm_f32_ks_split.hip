@@ -22,7 +22,8 @@
 // Measured (us, gemm_f32_ks.hip / here): 512 x 4096 x 4096 154 / 109 (158 TFLOP/s of the product), 1912 x 1206 x 1078 58 / 41, 83 x 2794 x 3689
 // nt 41 / 28.5, 1381 x 2795 x 925 nt 92 / 71, 3713 x 2717 x 528 138 / 110, 947 x 2247 x 657 nt 47 / 38. A wave's 16 steps take 0.74 - 0.9 us
 // beside a second wave's, the products alone 0.4 (at 1.85 GHz): with half of the products left out 0.75 of the time, without R's
-// split 0.83, every stage read from one place the same, so no one of them bounds it.
+// split 0.83, every stage read from one place the same, so no one of them bounds it: by counter the matrix units are busy 0.47 of
+// a CU's cycles at 512 x 4096 x 4096, 0.42 - 0.26 for the others (profiles/f32_products__few_rows_and_middle_size.txt).
 // Fp32MatMulM4N12.cpp:9-158 is the loop replaced.
 #include "common.h"
 #include "conv_mfma_i8.h"
