@@ -12,7 +12,7 @@
 //     beyond the operand, which reads zero and touches nothing. Left to itself the compiler puts the four steps' loads
 //     behind their products (64 -> 64 112 x 112 N=16 160 us for 151 with 64 channels).
 //   * The last K % 8 (16) values are one more step, masked on both sides (a row's neighbour may hold anything, Inf included).
-//   * Running sums are closed every 16 or 32 values of K. Relative error against 64 bits, gemm_f32_ks.hip / here: 8 -> 9 3x3 0.93e-7 / 0.89e-7,
+//   * Running sums are closed every 8 (K up to 63), 16 or 32 values of K. Relative error against 64 bits, gemm_f32_ks.hip / here: 8 -> 9 3x3 0.93e-7 / 0.89e-7,
 //     126 -> 74 1x1 1.13e-7 / 0.99e-7, 32 -> 32 3x3 1.59e-7 / 1.12e-7, 96 -> 11 3x3 1.53e-7 / 1.28e-7, 100 -> 128 3x3 1.52e-7 / 1.47e-7; it grows with
 //     the number of closings, up to CwPlan's longest K (128 -> 96 3x3 1.55e-7 / 1.74e-7, which is why it stays there).
 // Bound: f32 MFMA (by counter 0.43 - 0.67 of the cycles a CU is busy: 96 -> 11 and 64 -> 64 below; profiles/conv_f32_wide__drawn_layers.txt), launch and a wave's prologue for
@@ -58,8 +58,8 @@ struct CwParams {
 };
 
 // R: side of an output tile; MT, NT: tiles of a wave along the channels, along the pixels; GATHER: a filter of more than 1 x 1 or
-// padding; TAIL: K is no whole number of steps
-template <int R, int MT, int NT, bool GATHER, bool TAIL>
+// padding; TAIL: K is no whole number of steps; SHORT: sums are closed after every step (MT = 1)
+template <int R, int MT, int NT, bool GATHER, bool TAIL, bool SHORT>
 __global__ void __launch_bounds__(CW_THREADS, 3) conv_f32_wide_kernel(CwParams q) {
     constexpr int RING = 4;  // steps in flight
     constexpr int H = 64 / R, KS = 4 * H, SUMS = R * R / 64;  // groups of lanes along K, values of K a step, sums of a tile per lane
@@ -152,10 +152,10 @@ __global__ void __launch_bounds__(CW_THREADS, 3) conv_f32_wide_kernel(CwParams q
                 v[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, (int)off, GATHER ? 0 : (int)((unsigned)(s * KS + e) * q.plane), 0));
             }
     };
-    // Running sums, closed into `sum`: with 16 and 32 channels every two steps, while the products go to the other set of registers, so that
+    // Running sums, closed into `sum`: with 16 and 32 channels every two steps (SHORT: every step), while the products go to the other set of registers, so that
     // the additions stand between them; with 64 every four (a second set would leave two waves a SIMD for three). 16 channels have
-    // two chains a tile, so no chain is longer than 16 or 32 values.
-    constexpr int SETS = MT == 1 ? 2 : 1, GROUP = MT == 1 ? 2 : RING, CHAINS = R == 16 ? 2 : 1;
+    // two chains a tile, so no chain is longer than 16 (8) or 32 values.
+    constexpr int SETS = MT == 1 ? 2 : 1, GROUP = MT == 1 ? (SHORT ? 1 : 2) : RING, CHAINS = R == 16 ? 2 : 1;
     Sums acc[SETS][CHAINS][MT][NT], sum[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -245,10 +245,13 @@ __global__ void __launch_bounds__(CW_THREADS, 3) conv_f32_wide_kernel(CwParams q
     const bool rest = s < full;
     static_for<RING - 1>([&](auto rc) __attribute__((always_inline)) {
         constexpr int r = decltype(rc)::value;
-        if (s + r < full)
-            multiply(av[r], bv[r], 0, r == 0);
+        if (s + r < full) {
+            multiply(av[r], bv[r], 0, SHORT || r == 0);
+            if (SHORT)  // (not from the other set's registers: with those in use to the end four waves a SIMD are left for five)
+                close(0);
+        }
     });
-    if (rest)
+    if (!SHORT && rest)
         close(0);
     if (TAIL) {
         multiply(at, bt, 0, true);
@@ -275,9 +278,15 @@ __global__ void __launch_bounds__(CW_THREADS, 3) conv_f32_wide_kernel(CwParams q
 
 struct CwPlan {
     int r, mt, nt;
-    long longest;  // K
-    double us;  // estimated
+    long shortest, longest;  // K
+    double us;               // estimated
 };
+
+// Up to this K sums are closed after every step, and rows of 64 begin behind the other: longer chains' error would be larger than that of the four
+// waves' shorter ones in gemm_f32_ks.hip, which had these layers before (relative error there / with chains of 16 / here: 32 channels K = 24 0.69e-7 / 0.94e-7 /
+// 0.69e-7, 48 0.84 / 0.86 / 0.77, 63 0.88 / 0.92 / 0.82, 12 channels K = 48 0.84 / 0.96 / 0.75, 100 channels K = 72 in rows of 64 0.93 / 1.08, of 32 / 0.90). Such layers
+// take up to 4 % longer for it, 40 channels of K = 63, for two tiles of 32 in place of one of 64, 9 (15 x 7 -> 40 62 x 62 11.1 / 12.2 us; 15.6 there).
+static constexpr long CW_SHORT_K = 63, CW_LONG_CHAINS = 129;
 
 // A workgroup puts one wave on each SIMD of a CU: its MFMAs, 0.45 - 1 us for the
 // prologue and end of every set of 256 workgroups, 4 for launch and first operands; pixels that do not
@@ -286,15 +295,15 @@ struct CwPlan {
 // 64 -> 64 112 x 112 N=16 188 / 188, 144 / 154, 149 / 151; 6 -> 104 76 x 79 1x1 N=6 7.5 / 7.8, 6.8 / 6.8, 7.4 / 7.5. (64 pixels a wave for 32: 64 ->
 // 64 162, 96 -> 11 49; 64 x 64 outputs 174, 74.)
 static CwPlan cw_plan(const ConvGeom& g) {
-    static const CwPlan kPlans[] = {{32, 1, 1, 640, 0}, {32, 2, 1, 960, 0}, {16, 1, 2, 1152, 0}};
+    static const CwPlan kPlans[] = {{32, 1, 1, 1, 640, 0}, {32, 2, 1, CW_LONG_CHAINS, 960, 0}, {16, 1, 2, 1, 1152, 0}};
     const long N = (long)g.n * g.oh * g.ow, K = (long)g.ic * g.fh * g.fw;
-    CwPlan best = {0, 0, 0, 0, 1e30};
+    CwPlan best = {0, 0, 0, 0, 0, 1e30};
     const double each = g.sw > 1 && g.fw > 1 ? 1e-3 : 0.56e-3;
     for (CwPlan p : kPlans) {
         const long wgs = ((g.oc + p.r * p.mt - 1) / (p.r * p.mt)) * ((N + CW_WAVES * 32 - 1) / (CW_WAVES * 32));
         const double sets = (double)((wgs + num_cus() - 1) / num_cus());
         p.us = 4.0 + sets * ((p.r == 16 ? 0.5 : p.mt == 1 ? 0.45 : 1.0) + each * (double)K * (p.r == 16 ? 22.0 : p.mt == 1 ? 32.0 : 61.0));
-        if (K <= p.longest && p.us < best.us)
+        if (K >= p.shortest && K <= p.longest && p.us < best.us)
             best = p;
     }
     return best;
@@ -325,10 +334,10 @@ bool conv_f32_wide_supported(const ConvGeom& g) {
            cw_plan(g).us < 0.93 * cw_others(g);
 }
 
-template <int R, int MT, int NT>
+template <int R, int MT, int NT, bool SHORT>
 static void (*cw_kernel(bool gather, bool tail))(CwParams) {
-    return gather ? (tail ? conv_f32_wide_kernel<R, MT, NT, true, true> : conv_f32_wide_kernel<R, MT, NT, true, false>)
-                  : (tail ? conv_f32_wide_kernel<R, MT, NT, false, true> : conv_f32_wide_kernel<R, MT, NT, false, false>);
+    return gather ? (tail ? conv_f32_wide_kernel<R, MT, NT, true, true, SHORT> : conv_f32_wide_kernel<R, MT, NT, true, false, SHORT>)
+                  : (tail ? conv_f32_wide_kernel<R, MT, NT, false, true, SHORT> : conv_f32_wide_kernel<R, MT, NT, false, false, SHORT>);
 }
 
 TinyNNStatus conv_f32_wide_launch(const ConvGeom& g, const void* src, const void* flt, const void* bias, void* dst) {
@@ -359,7 +368,10 @@ TinyNNStatus conv_f32_wide_launch(const ConvGeom& g, const void* src, const void
     const bool gather = !(g.fh == 1 && g.fw == 1 && g.ph == 0 && g.pw == 0);
     const int ks = p.r == 32 ? 8 : 16;
     const bool tail = q.K % ks != 0;
-    void (*const kern)(CwParams) = p.r == 16 ? cw_kernel<16, 1, 2>(gather, tail) : p.mt == 1 ? cw_kernel<32, 1, 1>(gather, tail) : cw_kernel<32, 2, 1>(gather, tail);
+    const bool brief = q.K <= CW_SHORT_K && q.K >= 2 * ks;  // (below two steps there is one chain and the rest)
+    void (*const kern)(CwParams) = p.r == 16   ? (brief ? cw_kernel<16, 1, 2, true>(gather, tail) : cw_kernel<16, 1, 2, false>(gather, tail))
+                                   : p.mt == 1 ? (brief ? cw_kernel<32, 1, 1, true>(gather, tail) : cw_kernel<32, 1, 1, false>(gather, tail))
+                                               : cw_kernel<32, 2, 1, false>(gather, tail);
     const size_t lds = (gather ? (size_t)(q.K + ks - 1) / ks * ks * 8 : 0) + (size_t)p.r * p.mt * 4;
     note_kernel("conv_f32_wide", p.r * p.mt, p.r * p.nt);
     hipLaunchKernelGGL(kern, dim3((unsigned)(8 * q.per_xcd)), dim3(CW_THREADS), lds, stream(), q);

@@ -143,6 +143,31 @@ def test_layers_of_few_channels_and_a_long_k(n, ic, oc, h, w, k, stride):
     assert np.all(np.abs(got - convolution64(case, arrays)) <= bound)
 
 
+@pytest.mark.parametrize("oc", [12, 32, 40])
+@pytest.mark.parametrize("ic,k", [(16, 1), (24, 1), (3, 3), (32, 1), (39, 1), (48, 1), (7, 3), (63, 1)])
+def test_layers_of_many_pixels_and_short_k_are_as_precise_as_sums_of_eight(oc, ic, k):
+    """as the kernel that shares K among waves had them: no chain of a short K is longer than the eight values of a step"""
+    case = ConvCase(A.FMT_NCHW, A.DENSE, 7, ic, 96, 96, oc, k, 1, k // 2, A.IDENTITY, dtype="f32", bias=False)
+    arrays = case.gen(seed=69)
+    got = run(case, arrays)[:2]
+    assert runtime.last_kernel().startswith("conv_f32_wide:"), runtime.last_kernel()
+    flt = arrays["flt"].reshape(oc, -1)
+    src = np.pad(arrays["src"][:2], ((0, 0), (0, 0), (k // 2, k // 2), (k // 2, k // 2)))
+    cols = np.stack([src[:, c, y:y + 96, x:x + 96] for c in range(ic) for y in range(k) for x in range(k)])  # [K][image][row][column]
+    exact = np.tensordot(flt.astype(np.float64), cols.astype(np.float64), 1)
+    total = np.float32(0)
+    for k0 in range(0, len(cols), 8):
+        chain = np.zeros(exact.shape, np.float32)
+        for j in range(k0, min(k0 + 8, len(cols))):  # (a product is exact in 64 bits, and one rounding to 32 follows the addition)
+            chain = (chain + flt[:, j, None, None, None].astype(np.float64) * cols[j].astype(np.float64)).astype(np.float32)
+        total = total + chain
+    exact, total = exact.swapaxes(0, 1), total.swapaxes(0, 1)
+    error, of_eight = np.linalg.norm(got - exact), np.linalg.norm(total - exact)
+    print("relative error", error / np.linalg.norm(exact), "of sums of eight", of_eight / np.linalg.norm(exact))
+    # (the same sums in another order: some 200000 roundings of each kind, whose norms differ by less than 1 %, and instructions of two products)
+    assert error <= 1.03 * of_eight
+
+
 def test_layers_of_many_pixels_reach_every_tile():
     for tile, n, ic, oc, h, w, k, stride in WIDE:
         case = ConvCase(A.FMT_NCHW, A.DENSE, n, ic, h, w, oc, k, stride, k // 2, A.SIGMOID, dtype="f32")
