@@ -57,6 +57,25 @@ def test_which_kernel_few_rows_run_on(m, k, n, tb, own):
         assert runtime.last_kernel() == GEVM
 
 
+@pytest.mark.parametrize("m,k,n", [(4, 64, 1500), (4, 256, 1500), (3, 300, 2000), (2, 500, 3000), (4, 600, 1500), (2, 200, 9000), (4, 330, 9000), (4, 1000, 9000), (4, 16, 30000)])
+def test_few_rows_of_two_transposed_operands_are_as_precise_as_a_tree_of_sums(m, k, n):
+    """as one pass over B had them: four rounded products a lane, and another four every 256, then a tree over 64 lanes"""
+    case = MatMulCase(m, k, n, True, True)
+    arrays = case.gen(seed=78)
+    got, exact = run(case, arrays), product64(case, arrays)
+    assert runtime.last_kernel().startswith(KS + "16,16"), runtime.last_kernel()
+    a, b = arrays["a"], np.ascontiguousarray(arrays["b"].T)  # [k][m], [k][n]
+    lanes = np.zeros((64, m, n), np.float32)
+    for at in range(k):
+        lanes[at // 4 % 64] += a[at][:, None] * b[at]
+    while len(lanes) > 1:
+        lanes = lanes[:len(lanes) // 2] + lanes[len(lanes) // 2:]
+    error, tree = np.linalg.norm(got - exact), np.linalg.norm(lanes[0] - exact)
+    print("relative error", error / np.linalg.norm(exact), "of the tree", tree / np.linalg.norm(exact))
+    # (6000 outputs and more: the ratio of the norms of two such sets of errors spreads by some 1.3 %)
+    assert error <= 1.05 * tree
+
+
 def test_few_rows_of_values_that_are_not_finite():
     """a row or column beyond the operands (the clamped loads repeat the last one) leaves no trace, an Inf inside does"""
     case = MatMulCase(2, 515, 18)
