@@ -193,7 +193,7 @@ bool gevm_f32_supported(const GevmArgs& q) {
 
 // Against the matrix cores (gemm_f32_ks.hip), whose tiles have 16 rows whatever M is. They win where this kernel's loads of A,
 // M to one of B, are what a CU is busy with: four rows of a long K (us, here / there: 4 x 1000 x 1000 4.6 / 4.7, 4 x
-// 1300 x 1000 5.4 / 5.0, which stays, 4 x 1537 x 1000 6.0 / 5.5, 4 x 2346 x 311 7.2 / 6.5, 4 x 4096 x 1300 11.2 / 10.3), and three where there are
+// 1300 x 1000 5.4 / 5.0, which stays, 4 x 1500 x 3000 5.5 / 5.2, 4 x 1537 x 1000 6.0 / 5.5, 4 x 2346 x 311 7.2 / 6.5, 4 x 4096 x 1300 11.2 / 10.3), and three where there are
 // many columns as well (3 x 1000 x 3530 5.1 / 5.3, 3 x 1024 x 3530 5.0 / 4.6, 3 x 4096 x 1300 11.3 / 10.0; 3 x 2048 x 1300 5.6 / 5.5, 3 x 4096 x
 // 1024 7.7 / 8.2). Below 64 of their tiles two XCDs fetch each line of B (xcd_strip): a long K of four rows and 37 tiles
 // or more stays here (4 x 3000 x 650 7.5 / 9.3, 4 x 4000 x 1000 9.3 / 10.7; 4 x 4000 x 400 8.7 / 8.1, 4 x 4000 x 1010 9.3 / 8.5, 4 x 2600 x 580
@@ -204,7 +204,7 @@ bool gevm_f32_wins(const GevmArgs& q) {
     if (!by_columns(q) || q.M <= 2 || q.K <= 1024)
         return true;
     if (q.M == 4)
-        return q.K <= 1536 || (q.K >= 2800 && q.N > 36 * 16 && q.N <= 63 * 16);
+        return (q.K <= 1536 && q.N <= 2048) || (q.K >= 2800 && q.N > 36 * 16 && q.N <= 63 * 16);
     return q.N <= 1280 || (q.N <= 2048 && q.K <= 2560);
 }
 
