@@ -186,7 +186,8 @@ def audit_lines():
             (1, 1, 1, 1, 1, 1, 1, 0, 1), (3, 1, 5, 9, 7, 1, 1, 0, 1), (1, 7, 11, 12, 16, 1, 1, 0, 1), (2, 8, 8, 8, 17, 1, 1, 0, 1), (2, 9, 9, 15, 31, 1, 2, 0, 1), (1, 33, 12, 11, 33, 1, 1, 0, 1),
             (1, 64, 16, 16, 64, 1, 1, 0, 1), (1, 65, 13, 10, 65, 1, 1, 0, 1), (2, 130, 9, 9, 130, 1, 1, 0, 1), (1, 1, 9, 17, 12, 3, 1, 1, 1), (3, 2, 7, 7, 9, 3, 2, 1, 1), (2, 5, 10, 14, 40, 5, 1, 2, 1),
             (1, 9, 16, 15, 15, 3, 1, 2, 2), (1, 16, 13, 11, 70, 3, 1, 1, 1), (2, 3, 21, 23, 24, 5, 2, 2, 1), (1, 40, 12, 13, 64, 3, 1, 0, 1), (2, 128, 8, 9, 11, 3, 1, 1, 1), (1, 100, 9, 9, 128, 3, 1, 1, 1),
-            (1, 17, 3, 90, 18, 1, 1, 1, 1), (1, 70, 12, 12, 8, 3, 1, 1, 1), (1, 96, 10, 13, 80, 3, 2, 1, 1)):
+            (1, 17, 3, 90, 18, 1, 1, 1, 1), (1, 70, 12, 12, 8, 3, 1, 1, 1), (1, 96, 10, 13, 80, 3, 2, 1, 1),
+            (1, 5, 12, 13, 11, 3, 1, 1, 1), (1, 48, 9, 10, 10, 1, 1, 0, 1), (1, 63, 9, 9, 14, 1, 2, 0, 1), (2, 6, 11, 9, 40, 3, 1, 1, 1), (1, 16, 9, 9, 20, 1, 1, 0, 1)):  # (short K)
         lines.append("wide %d %d %d %d %d %d %d %d %d %d %d" % (n, ic, ih, iw, oc, k, st, p, d, oc & 1, 1 + 7 * (ic & 1)))
     # runs of blocks: every kind of map, both numbers of channels
     for n, h, w, count in ((1, 1, 1, 3), (2, 1, 15, 2), (1, 2, 3, 2), (1, 14, 1, 2), (2, 3, 5, 2), (1, 7, 7, 3), (1, 9, 11, 2), (1, 13, 15, 2), (2, 14, 14, 5), (2, 14, 15, 2)):
