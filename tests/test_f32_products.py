@@ -187,6 +187,26 @@ def test_layers_of_many_pixels_and_short_k_are_as_precise_as_sums_of_eight(oc, i
     assert error <= 1.03 * of_eight
 
 
+@pytest.mark.parametrize("ic", [33, 34, 41])
+def test_layers_of_many_pixels_and_a_short_k_with_a_rest(ic):
+    """a rest behind the steps of eight is no further rounding of the whole sum: as precise as where a chain of eight goes on with it"""
+    case = ConvCase(A.FMT_NCHW, A.DENSE, 7, ic, 50, 50, 85, 1, 1, 0, A.IDENTITY, dtype="f32", bias=False)
+    arrays = case.gen(seed=70)
+    got = run(case, arrays)
+    assert runtime.last_kernel().startswith("conv_f32_wide:"), runtime.last_kernel()
+    flt, cols = arrays["flt"].reshape(85, ic).astype(np.float64), arrays["src"].swapaxes(0, 1).astype(np.float64)
+    exact = np.tensordot(flt, cols, 1)
+    total, chain = np.zeros(exact.shape, np.float32), np.zeros(exact.shape, np.float32)
+    for j in range(ic):
+        chain = (chain + flt[:, j, None, None, None] * cols[j]).astype(np.float32)
+        if (j % 8 == 7 and j < ic // 8 * 8 - 1) or j == ic - 1:
+            total, chain = total + chain, np.zeros(exact.shape, np.float32)
+    exact, total = exact.swapaxes(0, 1), total.swapaxes(0, 1)
+    error, of_chains = np.linalg.norm(got - exact), np.linalg.norm(total - exact)
+    print("relative error", error / np.linalg.norm(exact), "of the chains", of_chains / np.linalg.norm(exact))
+    assert error <= 1.02 * of_chains
+
+
 def test_layers_of_many_pixels_reach_every_tile():
     for tile, n, ic, oc, h, w, k, stride in WIDE:
         case = ConvCase(A.FMT_NCHW, A.DENSE, n, ic, h, w, oc, k, stride, k // 2, A.SIGMOID, dtype="f32")
