@@ -8,13 +8,13 @@
 //     K up to 2048 is asked for at once. The partial sums of a column meet by shifts within 16 lanes and then in
 //     LDS, in a fixed order. Neighbouring workgroups, which share lines of 128 bytes, run on one XCD.
 //   * B transposed [N,K]: a wave owns 1 or 2 rows of B (= outputs), a lane 16-byte pieces of them
-//     along K, 8 in flight; the lanes' partial sums meet by shifts and wavefront shuffles in a fixed order.
+//     along K, 8 in flight; the lanes' partial sums meet by swaps of half waves and rows and by shifts, in a fixed order.
 // A 16-byte load needs 4-byte alignment only. The last columns (the end of K) come from a load that begins up to three
 // places earlier; what another lane counts as well is dropped.
 // Measured (us, before - four waves a workgroup, 16-byte loads only where every row was aligned, a wave four rows - / now):
 // 1 x 1024 x 1000 3.75 / 3.6, 1 x 2346 x 311 12.6 / 4.2, 1 x 4000 x 1000 10.7 / 5.9, 1 x 4000 x 3530 27 / 11.5 (4.9 TB/s),
-// 4 x 544 x 311 6.2 / 4.0; B transposed 1 x 1024 x 1000 4.3 / 3.6, 1 x 2346 x 311 12.9 / 3.6, 1 x 4000 x 1000 8.6 / 4.9,
-// 3 x 544 x 1000 8.3 / 3.8, 4 x 4000 x 311 21.4 / 7.7.
+// 4 x 544 x 311 6.2 / 4.0; B transposed 1 x 1024 x 1000 4.3 / 3.2, 1 x 2346 x 311 12.9 / 3.5, 1 x 4000 x 1000 8.6 / 3.8,
+// 3 x 544 x 1000 8.3 / 3.2, 4 x 4000 x 311 21.4 / 7.4.
 // The order of the additions differs from the reference's ascending k; f32 results are held to the
 // 1e-4 tolerance like the tiled GEMM, not to bit equality.
 #include "common.h"
@@ -41,6 +41,18 @@ __device__ __forceinline__ float gv_shift(float v) {
     return v;
 #else
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 | BY, 0xf, 0xf, true));
+#endif
+}
+
+// lanes 0 - 31 (of 32: 0 - 15) get their own and what the other 32 (16) hold
+template <int BY>
+__device__ __forceinline__ float gv_fold(float v) {
+#ifdef MG_HOST_AUDIT
+    return v;
+#else
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto p = BY == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
 #endif
 }
 
@@ -152,12 +164,13 @@ __global__ void __launch_bounds__(256) gevm_f32_rows_kernel(GevmArgs q) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             float s = acc[m][r];
+            // (halves first: behind the shifts the few values of a K just over 64 are one more rounding of the whole sum, K = 66 0.76e-7 for 0.73e-7)
+            s = gv_fold<32>(s);
+            s = gv_fold<16>(s);
             s += gv_shift<8>(s);
             s += gv_shift<4>(s);
             s += gv_shift<2>(s);
             s += gv_shift<1>(s);
-            s += __shfl_down(s, 16, 64);
-            s += __shfl_down(s, 32, 64);
             if (lane == 0 && n0 + r < q.N)
                 q.C[(size_t)m * q.ldc + n0 + r] = s;
         }
@@ -198,8 +211,8 @@ bool gevm_f32_supported(const GevmArgs& q) {
 // 1024 7.7 / 8.2). Below 64 of their tiles two XCDs fetch each line of B (xcd_strip): a long K of four rows and 37 tiles
 // or more stays here (4 x 3000 x 650 7.5 / 9.3, 4 x 4000 x 1000 9.3 / 10.7; 4 x 4000 x 400 8.7 / 8.1, 4 x 4000 x 1010 9.3 / 8.5, 4 x 2600 x 580
 // 7.3 / 6.5). Two rows stay: mostly faster, 7 % slower at worst but for 4096 x 4096 (2 x 4000 x 1400 9.6 / 9.0, 2 x 4096 x 4096 16.0 / 13.9). B transposed all stay (4 x 544 x
-// 3530 4.8 / 4.8, 4 x 1024 x 3530 4.8 / 5.5, 4 x 4000 x 311 7.8 / 11.9, 4 x 4096 x 4096 14.1 / 13.4), though a K just beyond the first round of
-// four rows' loads would be better off there (4 x 1100 x 1000 5.3 / 5.7, 4 x 1200 x 1000 5.3 / 4.7).
+// 3530 4.3 / 3.9, 4 x 1000 x 3530 4.3 / 5.3, 4 x 4000 x 311 7.4 / 11.9, 4 x 4096 x 4096 13.9 / 13.4), though a K just beyond the first round of
+// four rows' loads would be better off there (4 x 1200 x 1000 4.9 / 4.7).
 bool gevm_f32_wins(const GevmArgs& q) {
     if (!by_columns(q) || q.M <= 2 || q.K <= 1024)
         return true;
