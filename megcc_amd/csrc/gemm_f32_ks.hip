@@ -298,10 +298,10 @@ __global__ void __launch_bounds__(64 * KS_MAX_WAVES) gemm_f32_ks_kernel(KsParams
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 bt[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, (int)(boff[j] + (unsigned)tail_k(e) * q.b_k), 0, 0));
-    // Few rows of two transposed operands, which gevm_f32.hip had before: the last runs of a wave are closed after two steps, not four, else the error is up to
+    // Few rows of a transposed B, which gevm_f32.hip had before: the last runs of a wave are closed after two steps, not four, else the error is up to
     // 1.13 times as large as there (relative error there / after four / two: K = 256 0.82e-7 / 0.93e-7 / 0.82e-7, 500 0.91 / 1.01 / 0.91, 1000 1.04 /
-    // 1.04 / 1.00). 0 - 4 % longer (2 x 300 x 1000 3.63 / 3.66 us, 2 x 700 x 1000 4.36 / 4.54).
-    const bool few = R == 16 && AM == KS_STRIDED && BMODE == KS_CONTIG && q.M <= 4;
+    // 1.04 / 1.00; after one, more roundings of the whole sum: K = 544 0.92 / 1.02 / 0.93 / 0.96). 0 - 4 % longer (2 x 300 x 1000 tt 3.63 / 3.66 us, 2 x 700 x 1000 4.36 / 4.54).
+    const bool few = R == 16 && BMODE == KS_CONTIG && q.M <= 4;
     if (nj > 0) {
         static_for<RING>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
@@ -424,10 +424,10 @@ static KsPlan ks_plan(long M, long N, long K, bool a_contig, bool b_contig, bool
     const bool one_row = ((M > 16 && M <= 32) || (N > 16 && N <= 32)) && K * (M > N ? M : N) > (1L << 22);
     if (small <= num_cus() || (small <= 2L * num_cus() && !one_row))
         best = {16, 1, 1, small <= num_cus() && K >= 16 * (KS_SHORT + 1) ? 8 : 4, (double)K * 4.75 * (small <= num_cus() ? 1.0 : 2.0) + 3000.0};
-    // Few rows of two transposed operands in 16 x 16 tiles however many there are: 32 x 64 ones, whose waves add up to 64 values in a row, had up to 1.96 times
+    // Few rows of a transposed B in 16 x 16 tiles however many there are: 32 x 64 ones, whose waves add up to 64 values in a row, had up to 1.96 times
     // the error of gevm_f32.hip, which took them before (2 x 330 x 9000 1.69e-7 for 0.86e-7, now 0.85e-7). Us: 2 x 330 x 9000 7.2 / 4.9, 2 x 1000 x 9000 13.4 / 9.3, 2 x
-    // 128 x 30000 5.7 / 6.5 (gevm_f32.hip 13.1).
-    else if (!conv && M <= 4 && !a_contig && b_contig)
+    // 128 x 30000 5.7 / 6.5 (gevm_f32.hip 13.1); A not transposed 4 x 300 x 12000 6.8 / 5.2, 4 x 64 x 20000 4.1 / 5.4 (gevm_f32.hip 9.9).
+    else if (!conv && M <= 4 && b_contig)
         best = {16, 1, 1, 4, (double)((small + num_cus() - 1) / num_cus()) * ((double)K * 4.75 + 1000.0) + 2000.0};
     // A convolution of up to 16 channels and a long K in rows of 16 however many there are: half of a 32 x 32 tile's products are for
     // channels that are not there (us, 32 x 32 / 16 x 16: 114 -> 11 46 x 57 stride 2 N=13 18.1 / 15.4, 95 -> 12 58 x 58 N=3 13.8 / 9.7, 33 -> 12

@@ -210,11 +210,14 @@ bool gevm_f32_supported(const GevmArgs& q) {
 // many columns as well (3 x 1000 x 3530 5.1 / 5.3, 3 x 1024 x 3530 5.0 / 4.6, 3 x 4096 x 1300 11.3 / 10.0; 3 x 2048 x 1300 5.6 / 5.5, 3 x 4096 x
 // 1024 7.7 / 8.2). Below 64 of their tiles two XCDs fetch each line of B (xcd_strip): a long K of four rows and 37 tiles
 // or more stays here (4 x 3000 x 650 7.5 / 9.3, 4 x 4000 x 1000 9.3 / 10.7; 4 x 4000 x 400 8.7 / 8.1, 4 x 4000 x 1010 9.3 / 8.5, 4 x 2600 x 580
-// 7.3 / 6.5). Two rows stay: mostly faster, 7 % slower at worst but for 4096 x 4096 (2 x 4000 x 1400 9.6 / 9.0, 2 x 4096 x 4096 16.0 / 13.9). B transposed all stay (4 x 544 x
-// 3530 4.3 / 3.9, 4 x 1000 x 3530 4.3 / 5.3, 4 x 4000 x 311 7.4 / 11.9, 4 x 4096 x 4096 13.9 / 13.4), though a K just beyond the first round of
+// 7.3 / 6.5). Two rows stay: mostly faster, 7 % slower at worst but for 4096 x 4096 (2 x 4000 x 1400 9.6 / 9.0, 2 x 4096 x 4096 16.0 / 13.9). B transposed
+// stays but for four rows of many columns and a short K (4 x 300 x 3000 4.3 / 3.4, 4 x 544 x 3530 4.3 / 3.9, 4 x 560 x 8192 5.7 / 4.4; 4 x 600 x 3530 4.3 / 4.4,
+// 4 x 1000 x 3530 4.3 / 5.3, 4 x 4000 x 311 7.4 / 11.9, 4 x 4096 x 4096 13.9 / 13.4), though a K just beyond the first round of
 // four rows' loads would be better off there (4 x 1200 x 1000 4.9 / 4.7).
 bool gevm_f32_wins(const GevmArgs& q) {
-    if (!by_columns(q) || q.M <= 2 || q.K <= 1024)
+    if (!by_columns(q))
+        return !(q.M == 4 && q.N > 2048 && q.K <= 560);
+    if (q.M <= 2 || q.K <= 1024)
         return true;
     if (q.M == 4)
         return (q.K <= 1536 && q.N <= 2048) || (q.K >= 2800 && q.N > 36 * 16 && q.N <= 63 * 16);

@@ -49,7 +49,7 @@ GEVM, KS = "gevm_f32", "gemm_f32_ks:"
     (4, 2799, 650, False, KS), (4, 2800, 650, False, GEVM), (4, 4000, 576, False, KS), (4, 4000, 577, False, GEVM), (4, 4000, 1000, False, GEVM),
     (4, 4000, 1008, False, GEVM), (4, 4000, 1009, False, KS), (3, 1024, 3530, False, GEVM), (3, 1025, 2048, False, GEVM), (3, 1025, 2049, False, KS),
     (3, 2560, 1281, False, GEVM), (3, 2561, 1281, False, KS), (3, 4096, 1280, False, GEVM), (3, 4096, 1300, False, KS), (2, 4000, 1400, False, GEVM),
-    (4, 544, 3530, True, GEVM), (4, 1024, 3530, True, GEVM), (4, 4000, 311, True, GEVM), (3, 4096, 4096, True, GEVM)])
+    (4, 560, 2048, True, GEVM), (4, 560, 2049, True, KS), (4, 561, 3530, True, GEVM), (4, 1024, 3530, True, GEVM), (4, 4000, 311, True, GEVM), (3, 4096, 4096, True, GEVM)])
 def test_which_kernel_few_rows_run_on(m, k, n, tb, own):
     case = MatMulCase(m, k, n, False, tb)
     check_product(case, 67, own)
@@ -85,7 +85,7 @@ def test_few_rows_of_a_transposed_b_are_as_precise_as_a_tree_of_sums(m, k, n):
 # (6000 outputs and more: the ratio of the norms of two such sets of errors spreads by some 1.3 %)
 @pytest.mark.parametrize("m,k,n,ta", [
     (4, 64, 1500, True), (4, 256, 1500, True), (3, 300, 2000, True), (2, 500, 3000, True), (4, 600, 1500, True), (2, 200, 9000, True), (4, 330, 9000, True),
-    (4, 1000, 9000, True), (4, 16, 30000, True)])
+    (4, 1000, 9000, True), (4, 16, 30000, True), (4, 64, 2049, False), (4, 256, 3000, False), (4, 464, 3000, False), (4, 560, 9000, False)])
 def test_few_rows_of_a_transposed_b_on_the_matrix_cores_are_as_precise_as_a_tree_of_sums(m, k, n, ta):
     check_against_tree(MatMulCase(m, k, n, ta, True), 78, KS + "16,16", 1.05)
 
