@@ -206,9 +206,9 @@ bool gevm_f32_supported(const GevmArgs& q) {
 
 // Against the matrix cores (gemm_f32_ks.hip), whose tiles have 16 rows whatever M is. They win where this kernel's loads of A,
 // M to one of B, are what a CU is busy with: four rows of a long K (us, here / there: 4 x 1000 x 1000 4.6 / 4.7, 4 x
-// 1300 x 1000 5.4 / 5.0, which stays, 4 x 1500 x 3000 5.5 / 5.2, 4 x 1537 x 1000 6.0 / 5.5, 4 x 2346 x 311 7.2 / 6.5, 4 x 4096 x 1300 11.2 / 10.3), and three where there are
-// many columns as well (3 x 1000 x 3530 5.1 / 5.3, 3 x 1024 x 3530 5.0 / 4.6, 3 x 4096 x 1300 11.3 / 10.0; 3 x 2048 x 1300 5.6 / 5.5, 3 x 4096 x
-// 1024 7.7 / 8.2). Below 64 of their tiles two XCDs fetch each line of B (xcd_strip): a long K of four rows and 37 tiles
+// 1300 x 1000 5.4 / 5.0, which stays, 4 x 1537 x 1000 6.0 / 5.5, 4 x 2346 x 311 7.2 / 6.5, 4 x 4096 x 1300 11.2 / 10.3), three of many columns
+// as well (3 x 4096 x 1300 11.3 / 10.0; 3 x 2048 x 1300 5.6 / 5.5, 3 x 4096 x 1024 7.7 / 8.2), and both above 2048 columns from K = 513 on (4 x 513 x 3530 4.3 / 3.8,
+// 4 x 800 x 2049 4.3 / 3.9, 4 x 1000 x 3530 5.0 / 5.2, 4 x 1500 x 3000 5.5 / 5.2; 3 x 513 x 3530 3.9 / 3.8, 3 x 800 x 3530 4.6 / 4.2, 3 x 1000 x 3530 4.9 / 5.0, 3 x 1024 x 4096 4.3 / 4.0). Below 64 of their tiles two XCDs fetch each line of B (xcd_strip): a long K of four rows and 37 tiles
 // or more stays here (4 x 3000 x 650 7.5 / 9.3, 4 x 4000 x 1000 9.3 / 10.7; 4 x 4000 x 400 8.7 / 8.1, 4 x 4000 x 1010 9.3 / 8.5, 4 x 2600 x 580
 // 7.3 / 6.5). Two rows stay: mostly faster, 7 % slower at worst but for 4096 x 4096 (2 x 4000 x 1400 9.6 / 9.0, 2 x 4096 x 4096 16.0 / 13.9). B transposed
 // stays but for four rows of many columns and a short K (4 x 300 x 3000 4.3 / 3.4, 4 x 544 x 3530 4.3 / 3.9, 4 x 560 x 8192 5.7 / 4.4; 4 x 600 x 3530 4.3 / 4.4,
@@ -217,11 +217,13 @@ bool gevm_f32_supported(const GevmArgs& q) {
 bool gevm_f32_wins(const GevmArgs& q) {
     if (!by_columns(q))
         return !(q.M == 4 && q.N > 2048 && q.K <= 560);
-    if (q.M <= 2 || q.K <= 1024)
+    if (q.M <= 2 || q.K <= 512)
         return true;
+    if (q.N > 2048)
+        return false;
     if (q.M == 4)
-        return (q.K <= 1536 && q.N <= 2048) || (q.K >= 2800 && q.N > 36 * 16 && q.N <= 63 * 16);
-    return q.N <= 1280 || (q.N <= 2048 && q.K <= 2560);
+        return q.K <= 1536 || (q.K >= 2800 && q.N > 36 * 16 && q.N <= 63 * 16);
+    return q.N <= 1280 || q.K <= 2560;
 }
 
 TinyNNStatus gevm_f32_launch(const GevmArgs& q) {

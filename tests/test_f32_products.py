@@ -45,9 +45,9 @@ GEVM, KS = "gevm_f32", "gemm_f32_ks:"
 
 
 @pytest.mark.parametrize("m,k,n,tb,own", [
-    (4, 1024, 1000, False, GEVM), (4, 1536, 1000, False, GEVM), (4, 1536, 2048, False, GEVM), (4, 1100, 2049, False, KS), (4, 1537, 1000, False, KS), (4, 2346, 311, False, KS), (4, 4096, 1300, False, KS),
+    (4, 1024, 1000, False, GEVM), (4, 1536, 1000, False, GEVM), (4, 1536, 2048, False, GEVM), (4, 512, 4096, False, GEVM), (4, 513, 2049, False, KS), (3, 512, 2049, False, GEVM), (3, 513, 2049, False, KS), (4, 1537, 1000, False, KS), (4, 2346, 311, False, KS), (4, 4096, 1300, False, KS),
     (4, 2799, 650, False, KS), (4, 2800, 650, False, GEVM), (4, 4000, 576, False, KS), (4, 4000, 577, False, GEVM), (4, 4000, 1000, False, GEVM),
-    (4, 4000, 1008, False, GEVM), (4, 4000, 1009, False, KS), (3, 1024, 3530, False, GEVM), (3, 1025, 2048, False, GEVM), (3, 1025, 2049, False, KS),
+    (4, 4000, 1008, False, GEVM), (4, 4000, 1009, False, KS), (3, 1024, 3530, False, KS), (3, 1025, 2048, False, GEVM), (3, 1025, 2049, False, KS), (2, 1024, 3530, False, GEVM),
     (3, 2560, 1281, False, GEVM), (3, 2561, 1281, False, KS), (3, 4096, 1280, False, GEVM), (3, 4096, 1300, False, KS), (2, 4000, 1400, False, GEVM),
     (4, 560, 2048, True, GEVM), (4, 560, 2049, True, KS), (4, 561, 3530, True, GEVM), (4, 1024, 3530, True, GEVM), (4, 4000, 311, True, GEVM), (3, 4096, 4096, True, GEVM)])
 def test_which_kernel_few_rows_run_on(m, k, n, tb, own):
