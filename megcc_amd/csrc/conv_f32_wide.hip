@@ -288,6 +288,7 @@ struct CwPlan {
 // waves' shorter ones in gemm_f32_ks.hip, which had these layers before (relative error there / with chains of 16 / here: 32 channels K = 24 0.69e-7 / 0.94e-7 /
 // 0.69e-7, 48 0.84 / 0.86 / 0.77, 63 0.88 / 0.92 / 0.82, 12 channels K = 48 0.84 / 0.96 / 0.75, 100 channels K = 72 in rows of 64 0.93 / 1.08, of 32 / 0.90). Such layers
 // take up to 4 % longer for it, 40 channels of K = 63, for two tiles of 32 in place of one of 64, 9 (15 x 7 -> 40 62 x 62 11.1 / 12.2 us; 15.6 there).
+// (K = 9 of a 1x1 filter alone is left with more than in conv_f32_small.hip, whose waves add two or three values each: 0.63e-7 for 0.61e-7.)
 static constexpr long CW_SHORT_K = 63, CW_LONG_CHAINS = 129;
 
 // A workgroup puts one wave on each SIMD of a CU: its MFMAs, 0.45 - 1 us for the
